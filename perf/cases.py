@@ -57,29 +57,29 @@ def _requests(width, layers, rows, tokens, steps, dtype="bf16"):
 def listed():
     return [
         # a small assistant's answer to a short question: every launch is small
-        dict(_decode("llama-1b", 16, 1, 128), name="decode 1b, 1 row"),
+        dict(_decode("llama-1b", 16, 1, 128), name="decode 1b 1 row"),
         # one user's chat with the 8B model, sampled as requests are by default
-        dict(_decode("llama-8b", 8, 1, 2048, sampler="draw"), name="decode 8b, 1 row"),
+        dict(_decode("llama-8b", 8, 1, 2048, sampler="draw"), name="decode 8b 1 row"),
         # the same model serving eight requests
-        dict(_decode("llama-8b", 8, 8, 2050), name="decode 8b, 8 rows"),
+        dict(_decode("llama-8b", 8, 8, 2050), name="decode 8b 8 rows"),
         # a full batch of long documents on a shard in the middle of a pipeline
-        dict(_decode("llama-8b", 4, 16, 12289, part="middle"), name="decode 8b, 16 long rows"),
+        dict(_decode("llama-8b", 4, 16, 12289, part="middle"), name="decode 8b 16 long rows"),
         # a mixture of experts serving a few requests
-        dict(_decode("qwen-30b", 6, 4, 1024, sampler="draw"), name="decode 30b, 4 rows"),
+        dict(_decode("qwen-30b", 6, 4, 1024, sampler="draw"), name="decode 30b 4 rows"),
         # one request on a pipeline shard of the large mixture of experts, 8-bit weights
-        dict(_decode("qwen-235b", 3, 1, 4096, bits=8, part="middle"), name="decode 235b 8-bit, 1 row"),
+        dict(_decode("qwen-235b", 3, 1, 4096, bits=8, part="middle"), name="decode 235b 8-bit 1 row"),
         # the usual prompt with its documents
-        dict(_prompt("llama-8b", 4, 2047), name="prompt 8b, 2047"),
+        dict(_prompt("llama-8b", 4, 2047), name="prompt 8b 2047"),
         # a chat message of a few sentences
-        dict(_prompt("llama-8b", 8, 61), name="prompt 8b, 61"),
+        dict(_prompt("llama-8b", 8, 61), name="prompt 8b 61"),
         # a prompt to the mixture of experts
-        dict(_prompt("qwen-30b", 4, 1023), name="prompt 30b, 1023"),
+        dict(_prompt("qwen-30b", 4, 1023), name="prompt 30b 1023"),
         # a late portion of a long document, 8-bit weights, on a shard in the middle of a pipeline
-        dict(_prompt("llama-8b", 2, 4096, past=12288, bits=8, part="middle"), name="prompt 8b 8-bit, 4096 late"),
+        dict(_prompt("llama-8b", 2, 4096, past=12288, bits=8, part="middle"), name="prompt 8b 8-bit 4096 late"),
         # a batch of requests to a layer-list decoder, from prompts to a few tokens
-        dict(_requests(2048, 6, 4, 700, 8), name="requests 2k, 4 rows"),
+        dict(_requests(2048, 6, 4, 700, 8), name="requests 2k 4 rows"),
         # short requests to a small one in 32-bit mode
-        dict(_requests(1024, 6, 2, 40, 16, "f32"), name="requests 1k f32, 2 rows"),
+        dict(_requests(1024, 6, 2, 40, 16, "f32"), name="requests 1k f32 2 rows"),
     ]
 
 
