@@ -24,6 +24,15 @@
 //  * grouped mode (MoE prefill): blockIdx.y is a tile of one expert's sorted rows.
 //  * 128-row tiles over K ranges of 768 or more: weights and activation chunks of four K
 //    steps in flight in registers (DEEP, below) instead of one step.
+//  * inputs that fill the chip with them: a 256x256 tile per CU, four waves side by side, 256 x 64 per
+//    wave.  Nothing is dequantised twice and half as much per product as on the 128-row tile,
+//    and with one wave per SIMD the products of a K step are kept fed by that wave alone:
+//    the operands of the next product block, one dequantised register's half and every other slot an LDS
+//    read, ride between two MFMAs, across the barrier too (see multiply_on).  4096x14336 8-bit
+//    under 4096 rows 474 -> 407 us (1182 TFLOP/s), pair of 14336x4096 968 -> 824; 4-bit pair
+//    under 2047 rows 451 -> 420.  What bounds it: the matrix cores are busy 56 % of the
+//    cycles; 20 % go into the wait for the tile requested a step ahead and the barrier, the rest
+//    into slots with more vector work than an MFMA covers.
 //  * up to 128 rows and few column tiles: blockIdx.z splits K; float32 partial tiles and a
 //    small reduce launch.
 //  * up to 32 rows (64 on matrices of 8192 rows or more): the four waves sit side by side on
@@ -186,10 +195,52 @@ __device__ __forceinline__ uint32_t dequant_piece(uint32_t lo, uint32_t hi, floa
 // accumulators pass through LDS and are added to the first's, which writes the tile out.  A
 // launch of one such tile per CU has two waves per SIMD where four-wave workgroups would leave
 // one, without partial tiles in memory.
+// Tile `t` of a grid of gx column tiles by gy row tiles, in an order that walks GM row tiles by one
+// column tile after the other: neighbours in it share their activation rows or weight rows.
+template <int GM>
+__device__ __forceinline__ void tile_at(int t, int gx, int gy, int& x, int& y) {
+  const int g = t / (GM * gx), in = t - g * (GM * gx), rows = min(GM, gy - g * GM);
+  x = in / rows;
+  y = g * GM + (in - x * rows);
+}
+
+// Workgroups go round robin over the eight XCDs, each with an L2 of its own.  An XCD takes a
+// contiguous run of the tiles in that order, so that the 32 or 64 that it works on at a time
+// share rows (pair of 14336x4096 8-bit under 4096 rows, 256-row tile: 857 -> 821 us).
+__device__ __forceinline__ int xcd_run(int l, int n) {
+  const int xcd = l & 7, q = n >> 3, r = n & 7;
+  return xcd * q + min(xcd, r) + (l >> 3);
+}
+
+template <int GM>
+__device__ __forceinline__ void tile_of_block(int& x, int& y) {
+  const int gx = gridDim.x, gy = gridDim.y, n = gx * gy;
+  if (gridDim.z > 1 && (n & 7)) return;  // (the planes of a split would start on different XCDs)
+  tile_at<GM>(xcd_run(y * gx + x, n), gx, gy, x, y);
+}
+
+// The 256 x 256 tile, one workgroup per CU: whole tiles first, and where the last round would leave half
+// of the CUs idle, its tiles as two halves of 128 rows each.
+constexpr int kCUs = 256;
+__host__ __device__ inline int big_halved(int tiles) { return tiles % kCUs <= kCUs / 2 ? tiles % kCUs : 0; }
+
+__device__ __forceinline__ void big_tile_of_block(const QmmParams& p, int bn, int& x, int& y, int& half) {
+  const int gx = (p.N + bn - 1) / bn, gy = (p.M + 255) / 256, n = gx * gy, h = big_halved(n), l = blockIdx.x;
+  int t;
+  if (l < n - h) {
+    t = xcd_run(l, n - h);
+  } else {
+    const int e = xcd_run(l - (n - h), 2 * h);
+    t = n - h + (e >> 1);
+    half = e & 1;
+  }
+  tile_at<4>(t, gx, gy, x, y);
+}
+
 template <int BITS, int MI, bool GROUPED = false, bool SB4 = false, bool PAIR = false,
           bool WIDE = false, bool DEEP = false, bool KH = false>
-__global__ __launch_bounds__(KH ? 512 : 256, KH ? 1 : 2) void qmm_kernel(const QmmParams p) {
-  static_assert(!WIDE || GROUPED || !PAIR || MI == 4, "the wide pair tile has 128 rows");
+__global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_kernel(const QmmParams p) {
+  static_assert(!WIDE || GROUPED || !PAIR || MI >= 4, "the wide pair tile has 128 or 256 rows");
   static_assert(!DEEP || (SB4 && ((MI == 2 && !WIDE) || (WIDE && MI < 4))),
                 "the deep pipeline is for 128-row tiles; on the 32- and 64-row wide tiles the flag "
                 "selects the ring (K ranges long enough to fill it)");
@@ -209,11 +260,21 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH ? 1 : 2) void qmm_kernel(const Q
   const int tid = threadIdx.x & (kThreads - 1), lane = tid & 63;  // within the team
   const int team = KH ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8) : 0;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int n0 = blockIdx.x * BN;
+  int tile_x = blockIdx.x, tile_y = blockIdx.y, half = -1;
+  if (MI == 8 && WIDE)
+    big_tile_of_block(p, BN, tile_x, tile_y, half);
+  else if (!GROUPED)
+    tile_of_block<BM >= 256 ? 4 : 8>(tile_x, tile_y);
+  const int n0 = tile_x * BN;
   const int wm = WIDE ? 0 : (wave >> 1) * (32 * MI), wn = WIDE ? wave * WN : (wave & 1) * WN;
   const int G = p.K >> 6;
   const int wpr = p.K * BITS / 32;
-  int m0 = blockIdx.y * BM, m_end = p.M;
+  int m0 = tile_y * BM, m_end = p.M;
+  if (MI == 8 && WIDE) {
+    if (half >= 0) m0 += half * (BM / 2);
+    if (m0 >= m_end) return;  // whole workgroup: the second half of a tile that has none
+    m_end = min(m_end, m0 + (half >= 0 ? BM / 2 : BM));
+  }
   size_t w_off = 0, s_off = 0;
   __shared__ int row_pair[GROUPED ? BM : 1];  // pair index of every row of the tile
   if (GROUPED) {
@@ -272,7 +333,7 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH ? 1 : 2) void qmm_kernel(const Q
     // that activation row: rows are 128 bytes apart without padding (the loads write LDS in
     // lane order), and the XOR keeps the operand reads of 16 rows off each other's banks
     const int id = tid + kThreads * r;
-    const int trow = id >> 3, kp = (id & 7) ^ (trow & 7);
+    const int trow = id >> 3, kp = (id & 7) ^ ((trow >> 1) & 7);
     const int row = min(trow, m_end - 1 - m0);
     const uint32_t src = GROUPED ? (uint32_t)(row_pair[row] / p.x_div) : (uint32_t)(m0 + row);
     xoff[r] = (src * (uint32_t)p.K + kp * 8) * 2;  // bytes
@@ -288,9 +349,9 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH ? 1 : 2) void qmm_kernel(const Q
   constexpr int TILE_BYTES = BM * 128;
   // (a team's tiles: two, or the four of the ring)
   char* const tiles = reinterpret_cast<char*>(&xs[0][0]) + team * ((KH && WIDE ? 4 : SLOTS) * TILE_BYTES);
-  auto load_x = [&](int buf, int k0) {
+  auto load_x = [&](int buf, int k0, int n) {
 #pragma unroll
-    for (int r = 0; r < XR; ++r)
+    for (int r = 0; r < n; ++r)
       load_to_lds16(rx, tiles + buf * TILE_BYTES + (wave * 64 + kThreads * r) * 16, xoff[r], k0 * 2);
   };
   // s_waitcnt vmcnt(n) alone (the other counters at "no wait")
@@ -330,7 +391,7 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH ? 1 : 2) void qmm_kernel(const Q
   // byte offset of this lane's operand chunk of MFMA step t inside its tile row
   int aoff[4];
 #pragma unroll
-  for (int t = 0; t < 4; ++t) aoff[t] = ((kq * 4 + t) ^ (frow & 7)) * 16;
+  for (int t = 0; t < 4; ++t) aoff[t] = ((kq * 4 + t) ^ ((frow >> 1) & 7)) * 16;
 
   floatx16 acc[MI][2];
 #pragma unroll
@@ -355,7 +416,7 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH ? 1 : 2) void qmm_kernel(const Q
     // seven vector instructions of the same wave.  The order is pinned slot by slot (one
     // MFMA, one register of the next B operand, one LDS read) with scheduling barriers;
     // left alone, the compiler clumps the MFMAs behind all the vector work.
-    static_assert(MI == 2 || MI == 4 || (WIDE && MI == 1),
+    static_assert(MI == 2 || MI == 4 || MI == 8 || (WIDE && MI == 1),
                   "eight operand registers are spread over 2*MI slots");
     const char* arow = tiles + buf * TILE_BYTES + (wm + frow) * 128;
     bf16x8_t a[2][MI];
@@ -380,7 +441,7 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH ? 1 : 2) void qmm_kernel(const Q
             a[cur][i], __builtin_bit_cast(bf16x8_t, bq[cur][j]), acc[i][j], 0, 0, 0);
         if (t < 3) {
           // 8 registers of the next B operands over the 2*MI slots
-          constexpr int PER = 8 / (2 * MI);
+          constexpr int PER = MI > 4 ? 1 : 8 / (2 * MI);  // (the 256-row wide tile runs the ring's multiply)
 #pragma unroll
           for (int u = 0; u < PER; ++u) {
             const int r8 = m * PER + u, jj = r8 >> 2;
@@ -395,6 +456,91 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH ? 1 : 2) void qmm_kernel(const Q
           if (m < MI)
             a[nxt][m] = *reinterpret_cast<const bf16x8_t*>(arow + m * 32 * 128 + aoff[t + 1]);
         }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+
+  // The ring's multiply: the operands of a step's first products are produced during the last
+  // products of the step before it (`a` and `bq` live across steps), so that a wave's matrix
+  // core has work from the first cycle behind the barrier.  Tile `bn` is in LDS by then: the
+  // barrier in front of this step waited for it.
+  bf16x8_t a[2][MI];
+  uint4 bq[2][2];
+  auto scales_of = [&](const SBlock& sb, int e, float (&sc)[2], float (&bi)[2]) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      sc[j] = w_ok[j] ? pick(sb.s[j], e) : 0.f;
+      bi[j] = w_ok[j] ? pick(sb.b[j], e) : 0.f;
+    }
+  };
+  auto read_first = [&](auto ni, const WStage& st, int buf, const SBlock& sb, int e) {
+    constexpr int NI = decltype(ni)::value;
+    float sc[2], bi[2];
+    scales_of(sb, e, sc, bi);
+    const char* arow = tiles + buf * TILE_BYTES + (wm + frow) * 128;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) a[0][i] = *reinterpret_cast<const bf16x8_t*>(arow + i * 32 * 128 + aoff[0]);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) bq[0][j] = __builtin_bit_cast(uint4, dequant8<BITS>(st.w[j], 0, sc[j], bi[j]));
+  };
+  auto multiply_on = [&](auto ni, const WStage& st, const WStage& sn, int buf, int bn, const SBlock& sb, int e, const SBlock& nb, int ne) {
+    constexpr int NI = decltype(ni)::value;  // row blocks of 32 in use
+    float sc[2], bi[2], scn[2], bin[2];
+    scales_of(sb, e, sc, bi);
+    scales_of(nb, ne, scn, bin);
+    const char* arow = tiles + buf * TILE_BYTES + (wm + frow) * 128;
+    const char* anext = tiles + bn * TILE_BYTES + (wm + frow) * 128;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int cur = t & 1, nxt = cur ^ 1, tn = (t + 1) & 3;
+      const char* src = t < 3 ? arow : anext;
+      uint32_t lo = 0, hi = 0;
+      float f[2][2];
+      // register r8 of the next B operands in two parts that go into different slots: its two codes as
+      // floats, and their scaled values as two bf16
+      auto part_a = [&](int r8) {
+        if ((r8 & 3) == 0) dequant_words<BITS>(t < 3 ? st.w[r8 >> 2] : sn.w[r8 >> 2], tn, lo, hi);
+        float(&o)[2] = f[r8 & 1];
+        const uint32_t v = BITS == 4 ? lo : (r8 & 2) ? hi : lo;
+        if (BITS == 4) {
+          switch (r8 & 3) {
+            case 0: o[0] = ubyte_f<0>(lo), o[1] = ubyte_f<0>(hi); break;
+            case 1: o[0] = ubyte_f<1>(lo), o[1] = ubyte_f<1>(hi); break;
+            case 2: o[0] = ubyte_f<2>(lo), o[1] = ubyte_f<2>(hi); break;
+            default: o[0] = ubyte_f<3>(lo), o[1] = ubyte_f<3>(hi); break;
+          }
+        } else if (r8 & 1) {
+          o[0] = ubyte_f<2>(v), o[1] = ubyte_f<3>(v);
+        } else {
+          o[0] = ubyte_f<0>(v), o[1] = ubyte_f<1>(v);
+        }
+      };
+      auto part_b = [&](int r8) {
+        const int jj = r8 >> 2;
+        const float s1 = t < 3 ? sc[jj] : scn[jj], b1 = t < 3 ? bi[jj] : bin[jj];
+        const float(&o)[2] = f[r8 & 1];
+        reinterpret_cast<uint32_t*>(&bq[nxt][jj])[r8 & 3] = pack_bf2(fmaf(s1, o[0], b1), fmaf(s1, o[1], b1));
+      };
+#pragma unroll
+      for (int m = 0; m < 2 * NI; ++m) {
+        const int i = m >> 1, j = m & 1;
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            a[cur][i], __builtin_bit_cast(bf16x8_t, bq[cur][j]), acc[i][j], 0, 0, 0);
+        if (NI == 8) {  // one part per slot
+          if (m & 1) part_b(m >> 1); else part_a(m >> 1);
+        } else if (NI == 4) {  // the first part of one register, the second of the one before
+          part_a(m);
+          if (m) part_b(m - 1);
+          if (m == 7) part_b(7);
+        } else {
+#pragma unroll
+          for (int r8 = m * 4 / NI; r8 < (m + 1) * 4 / NI; ++r8) {
+            part_a(r8);
+            part_b(r8);
+          }
+        }
+        if (m & 1) a[nxt][i] = *reinterpret_cast<const bf16x8_t*>(src + i * 32 * 128 + aoff[tn]);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -470,11 +616,12 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH ? 1 : 2) void qmm_kernel(const Q
   // (past the end of K the last step again, never multiplied) and the loop body is four steps
   // long with static stage indices, so that the wait at the end of a step is an exact count:
   // the two youngest steps' requests may still be out.
-  constexpr bool RING = WIDE && SB4 && (BITS == 4 || kRing8) && (MI == 4 || DEEP);
+  constexpr bool RING = WIDE && SB4 && (BITS == 4 || kRing8) && (MI >= 4 || DEEP);
   // (8-bit: two steps ahead - three live stages of 16 registers; four spill)
   constexpr int AHEAD = BITS == 4 ? 3 : 2;
   static_assert(RING || !(WIDE && DEEP), "a wide tile with the pipeline flag runs the ring");
-  if (RING) {
+  auto ring = [&](auto ni) {
+    constexpr int NI = decltype(ni)::value;
     constexpr int NW = 2 * (BITS / 4);  // weight requests per step
     WStage wq[4];
     SBlock sbc, sbn;
@@ -482,26 +629,44 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH ? 1 : 2) void qmm_kernel(const Q
     load_sb(sbn, kb >> 8);
 #pragma unroll
     for (int u = 0; u < AHEAD; ++u) {
-      load_x(u, min(kb + u * BK, last));
+      load_x(u, min(kb + u * BK, last), NI);
       load_w(wq[u], min(kb + u * BK, last));
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
     __syncthreads();
+    read_first(ni, wq[0], 0, sbn, 0);
     for (int k0 = kb; k0 < ke; k0 += 4 * BK) {
       sbc = sbn;  // this block's scales: requested a block ago (the first: above)
       load_sb(sbn, min((k0 >> 8) + 1, (ke >> 8) - 1));
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const int kn = min(k0 + (u + AHEAD) * BK, last);
-        load_x((u + AHEAD) & 3, kn);
+        load_x((u + AHEAD) & 3, kn, NI);
         load_w(wq[(u + AHEAD) & 3], kn);
-        multiply(wq[u], u, sbc, u);
-        wait_vm(std::integral_constant<int, (AHEAD - 1) * (XR + NW)>{});
+        multiply_on(ni, wq[u], wq[(u + 1) & 3], u, (u + 1) & 3, sbc, u, u < 3 ? sbc : sbn, (u + 1) & 3);
+        wait_vm(std::integral_constant<int, (AHEAD - 1) * (NI + NW)>{});
         __syncthreads();
       }
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);  // the repeats requested past the end: landed before
-  }                                      // the staging below reuses this memory
+  };                                     // the staging below reuses this memory
+  if constexpr (RING) {
+    // a tile with fewer rows multiplies only the row blocks that it has
+    const int rows = m_end - m0;
+    if constexpr (MI == 8) {
+      if (rows > 192) ring(std::integral_constant<int, 8>{});
+      else if (rows > 128) ring(std::integral_constant<int, 6>{});
+      else if (rows > 64) ring(std::integral_constant<int, 4>{});
+      else ring(std::integral_constant<int, 2>{});
+    } else if constexpr (GROUPED) {
+      if (rows > 96) ring(std::integral_constant<int, 4>{});
+      else if (rows > 64) ring(std::integral_constant<int, 3>{});
+      else if (rows > 32) ring(std::integral_constant<int, 2>{});
+      else ring(std::integral_constant<int, 1>{});
+    } else {
+      ring(std::integral_constant<int, MI>{});
+    }
+  }
   WStage w0, w1;
   SBlock sb0, sb1;  // current block of four K steps, next block
   if (SB4 && !DEEP && !RING) {
@@ -509,7 +674,7 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH ? 1 : 2) void qmm_kernel(const Q
     sb1 = sb0;
   }
   if (!DEEP && !RING) {
-    load_x(0, kb);
+    load_x(0, kb, XR);
     if (!idle) load_w(w0, kb);
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the tile is in LDS
@@ -525,7 +690,7 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH ? 1 : 2) void qmm_kernel(const Q
       if (k0 + 4 * BK < ke) load_sb(sb1, (ks >> 2) + 1);
     }
     if (k0 + BK < ke) {
-      load_x(buf ^ 1, k0 + BK);
+      load_x(buf ^ 1, k0 + BK, XR);
       if (!idle) load_w(w1, k0 + BK);
     }
     if (!idle) multiply(w0, buf, sb0, ks & 3);
@@ -670,6 +835,21 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH ? 1 : 2) void qmm_kernel(const Q
       }
     }
   }
+}
+
+inline unsigned big_grid(int tiles) { return (unsigned)(tiles + big_halved(tiles)); }
+
+// Whether a launch is faster in tiles of 256 x 256 (one workgroup per CU) than in ones of 128 x 256 (two per
+// CU).  In units of a full round of the large tile: a full round of the small one - the same area - takes 1.1
+// (4096x14336 8-bit under 4096 rows, exactly one round: 407 us against 455), a last round of at most one
+// small tile per CU 0.62, and so do the halves of the large one (its last round otherwise 1).  14336x4096 pair
+// under 2047 rows, 3.5 rounds: 420 us against 436; 128256x2048 under 777 rows, 8 rounds against
+// 6.85 since the fourth row tile holds 9 rows: 579 us against 463.
+bool prefer_big(int64_t big, int64_t small) {
+  const int64_t rb = big % kCUs, rs = small % (2 * kCUs);
+  const double tb = big / kCUs + (rb == 0 ? 0. : 2 * rb <= kCUs ? 0.62 : 1.);
+  const double ts = 1.1 * (small / (2 * kCUs)) + (rs == 0 ? 0. : rs <= kCUs ? 0.62 : 1.1);
+  return tb <= ts && big < (1 << 30);
 }
 
 constexpr int kQmmMaxSplit = 16;  // K ranges the reduce kernel adds
@@ -920,6 +1100,8 @@ void launch_qmm(const QmmParams& p, hipStream_t st) {
     // more wide tiles than CUs: the wide tile with the ring, four waves (6144x4096 under 2046
     // rows 144 -> 126 us, 4096x14336 under 4094 rows 523 -> 472, 8192x8192 under 2046 rows
     // 292 -> 270)
+    else if (sb4 && prefer_big((int64_t)gw.x * g4.y, (int64_t)gw.x * gw.y))
+      exo_note_variant("qmm_kernel<%d, 4, false, true, false, true>", BITS), qmm_kernel<BITS, 8, false, true, false, true><<<dim3(big_grid(exo_ceil_div(N, 256) * g4.y)), 256, 0, st>>>(p);
     else if (sb4 && (BITS == 4 || kRing8) && (int64_t)gw.x * gw.y >= kWideRingMinTiles && weights_stay_cached(N, p.K, BITS))
       exo_note_variant("qmm_kernel<%d, 4, false, true, false, true>", BITS), qmm_kernel<BITS, 4, false, true, false, true><<<gw, 256, 0, st>>>(p);
     else if (sb4)
@@ -1179,6 +1361,9 @@ void launch_pair(const QmmParams& p, hipStream_t st) {
     // (up to one tall tile per CU: eight waves per tile, as in launch_qmm)
     if (sb4 && (int64_t)g4.x * g4.y <= 256 && p.K % 512 == 0 && p.K >= 1024)
       exo_note_variant("qmm_kernel<%d, 4, false, true, true, false, false, true>", BITS), qmm_kernel<BITS, 4, false, true, true, false, false, true><<<g4, 512, 0, st>>>(p);
+    else if (sb4 && prefer_big((int64_t)exo_ceil_div(p.N, 128) * exo_ceil_div(p.M, 256), (int64_t)exo_ceil_div(p.N, 128) * exo_ceil_div(p.M, 128)))
+      // (noted as what it is an instance of: the wide tile with the ring)
+      exo_note_variant("qmm_kernel<%d, 4, false, true, true, true>", BITS), qmm_kernel<BITS, 8, false, true, true, true><<<dim3(big_grid(exo_ceil_div(p.N, 128) * exo_ceil_div(p.M, 256))), 256, 0, st>>>(p);
     else if (sb4 && p.M >= kPairWideMinM && weights_stay_cached(2 * (int64_t)p.N, p.K, BITS))
       exo_note_variant("qmm_kernel<%d, 4, false, true, true, true>", BITS), qmm_kernel<BITS, 4, false, true, true, true><<<dim3(exo_ceil_div(p.N, 128), exo_ceil_div(p.M, 128)), 256, 0, st>>>(p);
     else if (sb4)

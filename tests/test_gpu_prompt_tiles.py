@@ -1,0 +1,79 @@
+"""The matrix-core GEMM's tiles for prompts, at the sizes where a tile ends: against float64 products of the
+weights as the kernel forms them (scale * code + bias, rounded to bf16 once)."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+if not torch.cuda.is_available():
+    pytest.skip("needs a GPU", allow_module_level=True)
+
+from exo_amd import ops  # noqa: E402
+from exo_amd.ops import QuantizedWeight  # noqa: E402
+
+
+def packed(N, K, bits, seed, device):
+    g = torch.Generator(device=device).manual_seed(seed)
+    w = torch.randint(-2**31, 2**31 - 1, (N, K * bits // 32), dtype=torch.int32, device=device, generator=g)
+    top = float(2**bits - 1)
+    s = (torch.rand(N, K // 64, device=device, generator=g) * 0.1 + 0.05) / top
+    return QuantizedWeight(w, s.bfloat16(), (-s * top * 0.5).bfloat16(), bits)
+
+
+def weights64(q: QuantizedWeight):
+    codes = ops.unpack_codes(q.weight, q.bits).double().view(q.N, -1, 64)
+    return (codes * q.scales.double()[..., None] + q.biases.double()[..., None]).float().bfloat16().double().view(q.N, -1)
+
+
+def check(got, x, w, residual=None, what=""):
+    """One bf16 rounding of the sum (and one more of the sum with the residual), float32 sums over K terms in any
+    order: K * 2^-24 of the sum of their magnitudes."""
+    want = x.double() @ w.T
+    slack = x.shape[1] * 2.0**-24 * (x.double().abs() @ w.abs().T)
+    size = want.abs()
+    if residual is not None:
+        want = want + residual.double()
+        size = size + want.abs()
+    bad = (got.double() - want).abs() > 2.0**-8 * size + slack + 1e-30
+    assert not bad.any(), f"{what}: {int(bad.sum())} of {bad.numel()} outputs, first at {bad.nonzero()[0].tolist()}"
+
+
+# tiles of 256 x 256 with 6, 134 and 192 rows in the last one (two, six and six blocks of 32), whole rounds of
+# them and a last round in halves, the second of which holds no row; ragged columns
+@pytest.mark.parametrize("M,N,K,bits", [(1030, 16400, 256, 4), (1030, 16397, 512, 8), (902, 16640, 256, 4),
+                                        (960, 16400, 256, 8), (2048, 8192, 256, 4), (513, 32776, 256, 4)])
+def test_prompt_gemm_at_tile_edges(device, M, N, K, bits):
+    q = packed(N, K, bits, M + N, device)
+    g = torch.Generator(device=device).manual_seed(M)
+    x = torch.randn(M, K, device=device, generator=g).bfloat16()
+    r = torch.randn(M, N, device=device, generator=g).bfloat16()
+    check(ops.quantized_matmul(x, q), x, weights64(q), what=f"{M}x{N}x{K}")
+    check(ops.quantized_matmul(x, q, residual=r), x, weights64(q), r, what=f"{M}x{N}x{K} with residual")
+
+
+@pytest.mark.parametrize("M,N,K,bits", [(1030, 8200, 256, 4), (300, 14336, 512, 8), (700, 8197, 256, 4)])
+def test_prompt_pair_gemm_at_tile_edges(device, M, N, K, bits):
+    """The gate and up projections in one launch have the bits of two launches and the SwiGLU kernel."""
+    gate, up = packed(N, K, bits, M, device), packed(N, K, bits, N, device)
+    x = torch.randn(M, K, device=device, generator=torch.Generator(device=device).manual_seed(K)).bfloat16()
+    want = ops.swiglu(ops.qmm(x, gate), ops.qmm(x, up))
+    assert torch.equal(ops.qmm_swiglu(x, gate, up).view(torch.int16), want.view(torch.int16))
+    check(ops.qmm(x, gate), x, weights64(gate), what=f"gate {M}x{N}x{K}")
+
+
+@pytest.mark.parametrize("rows", [1, 32, 33, 64, 65, 96, 97, 128, 129])
+def test_grouped_gemm_multiplies_the_rows_of_its_tile(device, rows):
+    """Experts of 1 to 129 rows beside an empty one: a tile multiplies only the blocks of 32 rows that it has."""
+    E, K, N = 4, 256, 264
+    qs = [packed(N, K, 4, e, device) for e in range(E)]
+    q = QuantizedWeight(torch.stack([t.weight for t in qs]), torch.stack([t.scales for t in qs]),
+                        torch.stack([t.biases for t in qs]), 4)
+    idx = torch.cat([torch.full((rows,), 2), torch.full((40,), 0), torch.full((3,), 3)]).to(torch.int32).to(device)[:, None].contiguous()
+    T = idx.shape[0]
+    x = torch.randn(T, 1, K, device=device, generator=torch.Generator(device=device).manual_seed(rows)).bfloat16()
+    y = ops.grouped_qmm(x, q, ops.moe_group(idx, E), 1)
+    for e in (0, 2, 3):
+        sel = (idx[:, 0] == e).nonzero()[:, 0]
+        check(y[sel, 0], x[sel, 0], weights64(qs[e]), what=f"expert {e} of {len(sel)} rows")
