@@ -8,15 +8,21 @@
 // The D-operand layout of the first product puts, in lane (query, half), registers that
 // are 8 consecutive keys per 16-key step once the K rows are fed in a permuted order;
 // they are rounded to bf16 and used as the B operand of the second product without any
-// data movement.  V is transposed on its way into LDS (2-byte stores), K goes in as is.  (A
-// row-major V tile read back through ds_read_b64_tr_b16 was measured and is slower here:
-// 2046 tokens 100 -> 164 us.)
+// data movement; the V^T operand comes out of the row-major V tile through the transposing LDS read.
 //
 // Work split: a wave owns 32 query tokens of ONE query head; the four waves of a
 // workgroup take four consecutive (token tile, head) units of one kv head, so with GQA
 // (4, 8, 16 query heads per kv head) they share every K/V tile they stage.  Key tiles of
-// 64 in two LDS buffers: while a tile is computed, the next one goes from registers into the
-// other buffer and the one after that is on its way from memory; one barrier per tile.
+// 64, straight from the cache into LDS, two buffers each for K and V; one barrier per tile.
+//
+// What bounds it: a tile is 32 matrix instructions (1024 cycles) and about as many cycles of vector work
+// for its 32 weights per lane (each a multiply-add, a power at a quarter of the rate, a sum, half a
+// rounding and half a maximum).  So the two are written into each other: a wave multiplies the NEXT
+// tile's scores between this tile's weights, and takes the next scores' maxima between this
+// tile's V products; what rescaled the output for every tile runs only when a maximum has moved
+// by more than a factor of 2^8.  32 / 8 heads of 128, 4096 tokens behind 12288: 1212 -> 868 us (1108
+// TFLOP/s), 2047 tokens 76 -> 50 us, 4096 behind 4096 with heads of 64 398 -> 254 us.  (Without the
+// interleaving 1061, 63 and 303 us.)
 //
 // SPLIT (launches of at most one workgroup per CU, i.e. prompts of about a thousand tokens):
 // eight waves, two teams of four that take the first and the second half of the
@@ -32,7 +38,7 @@ namespace {
 
 constexpr int kBN = 64;   // keys per tile
 constexpr int kBM = 32;   // query tokens per wave
-constexpr int kPadK = 8;  // bf16 of padding per K row / V^T row in LDS
+constexpr float kSlack = 8.f;  // see the online softmax
 
 struct FaParams {
   const bf16_t* q;    // [B*T, Hq*D] (already rotated)
@@ -40,30 +46,56 @@ struct FaParams {
   const bf16_t* v;
   const int32_t* pos;  // [B] tokens in the cache before this chunk
   bf16_t* out;         // [B*T, Hq*D]
-  float scale_log2e;
+  float scale_log2e, slack;  // > 0 (a negative scale is in q_sign); kSlack as a difference of scores
+  uint32_t q_sign;           // flips the queries of a negative scale
   int T, Hq, Hkv, S_max, G, units;  // units = token tiles * G
 };
 
 template <int D>
 constexpr int fa_lds_bytes() {
-  return 2 * (kBN * (D + kPadK) + D * (kBN + kPadK)) * 2;
+  return 4 * kBN * D * 2;  // two K tiles, two V tiles
+}
+
+typedef short short4_t __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) char* lds_char;
+typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
+
+// ds_read_b64_tr_b16: four consecutive rows of one column out of a row-major bf16 tile
+__device__ __forceinline__ uint2 read_tr16(lds_char at) {
+  const short4_t v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((short4_t __attribute__((address_space(3)))*)at);
+  return __builtin_bit_cast(uint2, v);
+}
+
+// keeps the computation of a value in the slot where it is written
+template <typename T>
+__device__ __forceinline__ void hold(T& v) {
+  asm volatile("" : "+v"(v));
+}
+
+// 16 bytes per lane from a buffer into LDS at `to` + 16 * lane.  Written as the instruction (it has no register
+// result): the compiler makes every transposing LDS read wait for all such loads that it knows
+// of; here the wait and the barrier at the end of a tile are theirs.
+__device__ __forceinline__ void load_to_lds16(u32x4 rsrc, lds_char to, uint32_t voffset, uint32_t soffset) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               :
+               : "s"((uint32_t)(uintptr_t)to), "v"(voffset), "s"(rsrc), "s"(soffset)
+               : "memory");
 }
 
 template <int D, bool SPLIT>
 __global__ __launch_bounds__(SPLIT ? 512 : 256, SPLIT ? 1 : 2) void fa_prefill_kernel(const FaParams p) {
   constexpr int STEPS = D / 16;  // MFMA steps over d for S^T
   constexpr int DT = D / 32;     // 32-row tiles of O^T
-  constexpr int KS = D + kPadK;  // LDS row stride of K (bf16)
-  constexpr int VS = kBN + kPadK;  // LDS row stride of V^T (bf16)
-  constexpr int VEC = D / 8;     // 16-byte vectors per K/V row
+  constexpr int ROW = D * 2;     // bytes of a K or V row in LDS
+  constexpr int TILE = kBN * ROW;
+  constexpr int VEC = D / 8;     // 16-byte chunks of a row
   constexpr int LOADS = kBN * VEC / 256;
-  constexpr int BUF = kBN * KS + D * VS;  // bf16 elements of one (K, V^T) tile pair
-  extern __shared__ __attribute__((aligned(16))) bf16_t fa_lds[];  // [2][BUF] per team
+  extern __shared__ __attribute__((aligned(16))) char fa_lds[];  // per team: K tiles 0, 1, V tiles 0, 1
 
   const int tid = threadIdx.x & 255, lane = tid & 63;  // within the team
   const int team = SPLIT ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8) : 0;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  bf16_t* const lds = fa_lds + team * (2 * BUF);
+  const lds_char lds = (lds_char)fa_lds + team * (4 * TILE);
   const int n = lane & 31, kq = lane >> 5;
   const int kvh = blockIdx.y, b = blockIdx.z;
   // Heavy (late) token tiles first - but a launch of up to two workgroups per CU is one round
@@ -98,43 +130,42 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, SPLIT ? 1 : 2) void fa_prefill_k
   {
     const bf16_t* qp = p.q + ((size_t)b * p.T + t_lane) * ((size_t)p.Hq * D) + (size_t)hq * D + kq * 8;
 #pragma unroll
-    for (int s = 0; s < STEPS; ++s) qreg[s] = *reinterpret_cast<const uint4*>(qp + s * 16);
+    for (int s = 0; s < STEPS; ++s) {
+      qreg[s] = *reinterpret_cast<const uint4*>(qp + s * 16);
+      qreg[s].x ^= p.q_sign;
+      qreg[s].y ^= p.q_sign;
+      qreg[s].z ^= p.q_sign;
+      qreg[s].w ^= p.q_sign;
+    }
   }
 
-  // K/V tiles come through buffer loads: one descriptor per (sequence, kv head) that ends
-  // with the cache (rows past it read as zero; they are masked), a lane offset that never
-  // changes and the tile as the scalar offset - no 64-bit address per load in registers.
-  // A K tile is one contiguous block (16 bytes per thread and load); a V load takes key
-  // tid % 64, chunk tid / 64 + 4 i, so that a thread's stores into V^T are 8 rows of one key.
+  // K and V tiles go from the cache straight into LDS, row by row as they are: one descriptor per
+  // (sequence, kv head), a lane offset that never changes and the tile as the scalar offset.  A wave's
+  // load writes its 64 chunks of 16 bytes in lane order, so the order of the chunks inside a row is
+  // chosen by what a lane requests: chunk c of K row r sits at c ^ (r % 16) (128-byte rows: c ^ (r / 2 % 8)),
+  // so that the 16 rows of an operand read touch all 64 banks; chunk c of V row r at c ^ (4 * (r % 4))
+  // (c ^ (4 * (r / 2 % 2))), so that the four rows of a transposing read do.
   const size_t head_off = ((size_t)b * p.Hkv + kvh) * (size_t)p.S_max * D;
-  const uint32_t head_bytes = (uint32_t)p.S_max * D * 2;
-  const __amdgpu_buffer_rsrc_t rk =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(p.k + head_off), 0, head_bytes, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rv =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(p.v + head_off), 0, head_bytes, 0x00020000);
-  const uint32_t koff = tid * 16, voff = (tid & (kBN - 1)) * (D * 2) + (tid / kBN) * 16;
-  uint4 kreg[LOADS], vreg[LOADS];
-  auto load_tile = [&](int kt) {
-    const uint32_t tile = (uint32_t)(t_first + kt) * (kBN * D * 2);
-#pragma unroll
-    for (int i = 0; i < LOADS; ++i) {
-      kreg[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rk, koff, tile + i * 4096, 0));
-      vreg[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rv, voff + i * 64, tile, 0));
-    }
+  auto rsrc = [&](const bf16_t* base) {
+    const uint64_t at = (uint64_t)base;
+    return u32x4{(uint32_t)__builtin_amdgcn_readfirstlane((int)at), (uint32_t)__builtin_amdgcn_readfirstlane((int)(at >> 32)) & 0xffffu,
+                 0xffffffffu, 0x00020000u};
   };
-  auto store_tile = [&](int buf) {
-    bf16_t* kl = lds + buf * BUF;
-    bf16_t* vl = kl + kBN * KS;
+  const u32x4 rk = rsrc(p.k + head_off), rv = rsrc(p.v + head_off);
+  const int lrow = tid / VEC, lslot = tid % VEC;  // (row of load i: lrow + i * 256 / VEC, a multiple of 16 further)
+  const uint32_t koff = lrow * ROW + (lslot ^ (D == 128 ? lrow & 15 : (lrow >> 1) & 7)) * 16;
+  const uint32_t voff = lrow * ROW + (lslot ^ (D == 128 ? (lrow & 3) << 2 : ((lrow >> 1) & 1) << 2)) * 16;
+  auto load_tile = [&](u32x4 r, uint32_t off, int tile, int kt) {
+    const int row0 = (t_first + kt) * kBN;
+    const lds_char to = lds + tile * TILE + wave * 1024;
+    if (row0 + kBN <= p.S_max) {
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) {
-      const int vi = tid + i * 256;
-      *reinterpret_cast<uint4*>(&kl[(vi / VEC) * KS + (vi % VEC) * 8]) = kreg[i];
-      const int key = vi & (kBN - 1), c = vi / kBN;
-      const uint32_t w[4] = {vreg[i].x, vreg[i].y, vreg[i].z, vreg[i].w};
+      for (int i = 0; i < LOADS; ++i) load_to_lds16(r, to + i * 4096, off, row0 * ROW + i * 4096);
+    } else {  // rows past the end of the cache: its last row again (they are masked)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        vl[(c * 8 + 2 * j) * VS + key] = (bf16_t)(w[j] & 0xFFFFu);
-        vl[(c * 8 + 2 * j + 1) * VS + key] = (bf16_t)(w[j] >> 16);
+      for (int i = 0; i < LOADS; ++i) {
+        const int row = lrow + i * (256 / VEC), over = max(0, row0 + row - (p.S_max - 1));
+        load_to_lds16(r, to + i * 4096, off + (row0 + i * (256 / VEC) - over) * ROW, 0);
       }
     }
   };
@@ -143,111 +174,174 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, SPLIT ? 1 : 2) void fa_prefill_k
   // of lane half kq are keys 16s + 8kq .. +8
   const int jr = n >> 3;
   const int key_of_row = 16 * (jr >> 1) + 8 * ((n >> 2) & 1) + 4 * (jr & 1) + (n & 3);
+  const int k_at = key_of_row * ROW, k_x = kq ^ (D == 128 ? key_of_row & 15 : (key_of_row >> 1) & 7);
+  // V^T operand: lane (d = 32*dt + n, half kq) takes keys 16*st + 8*kq .. +8 of that d, four at
+  // a time: a block of 16 lanes whose lane r points at V[key0 + r/4][d0 + 4*(r%4) ..+4] gets
+  // V[key0 .. key0+4][d0 + i] in lane i
+  const int v_row = kq * 8 + ((lane & 15) >> 2);
+  const int v_at = v_row * ROW + ((lane >> 4) & 1) * 32 + (lane & 3) * 8;
+  const int v_x = D == 128 ? v_row & 3 : (v_row >> 1) & 1;  // (the same for every key block: they are 4 rows apart)
 
   floatx16 o[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
     for (int e = 0; e < 16; ++e) o[dt][e] = 0.f;
-  float m_run = -INFINITY, l_run = 0.f;
+  // maximum that the weights refer to, the same scaled, the score at which it moves; this half's sums
+  float m_run = -INFINITY, m_ref = 0.f, m_lim = -INFINITY, l0 = 0.f, l1 = 0.f;
 
-  if (!SPLIT || n_tiles > 0) {
-    load_tile(0);
-    store_tile(0);
-  }
-  // Every load so far (the Q operand among them) has landed before the loop is entered: left
-  // to itself the compiler requests Q last and then waits, in EVERY iteration, for as many
-  // loads as were issued after each Q register - which in the loop are the tile loads just
-  // requested, so the prefetch would be waited for on the spot.
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-  if (n_tiles > 1) load_tile(1);
-  for (int kt = 0; kt < n_iter; ++kt) {
-    // tile kt is complete in its buffer, and every wave is done reading the other buffer
-    __syncthreads();
-    if (SPLIT && kt >= n_tiles) continue;  // (team 0 when the tile count is odd)
-    if (kt + 1 < n_tiles) {
-      store_tile((kt + 1) & 1);
-      if (kt + 2 < n_tiles) load_tile(kt + 2);
-    }
+  auto read_k = [&](lds_char tile, int slot) {  // operand of product `slot` of S^T: step slot / 2, sub-tile slot % 2
+    return *reinterpret_cast<__attribute__((address_space(3))) const u32x4*>(
+        tile + (slot & 1) * (32 * ROW) + k_at + (((slot >> 1) * 2) ^ k_x) * 16);
+  };
+  auto read_v = [&](lds_char tile, int slot) {  // of O^T: 16 keys slot / DT, columns slot % DT
+    const lds_char at = tile + (slot / DT) * (16 * ROW) + v_at + ((slot % DT) ^ v_x) * 64;
+    const uint2 lo = read_tr16(at), hi = read_tr16(at + 4 * ROW);
+    return u32x4{lo.x, lo.y, hi.x, hi.y};
+  };
+  // what the scores of tile kt need before they become weights: the causal edge
+  auto mask = [&](floatx16(&s)[2], int kt) {
     const int key0 = (t_first + kt) * kBN;
-    if (key0 > last_w) continue;  // wave-uniform: nothing visible to this wave's rows
-    const bf16_t* k_lds = lds + (kt & 1) * BUF;
-    const bf16_t* v_lds = k_lds + kBN * KS;
-
-    // ---- S^T = K Q^T for the two 32-key sub-tiles
-    floatx16 s[2];
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-#pragma unroll
-      for (int e = 0; e < 16; ++e) s[ks][e] = 0.f;
-      const bf16_t* kr = &k_lds[(ks * 32 + key_of_row) * KS + kq * 8];
-#pragma unroll
-      for (int st = 0; st < STEPS; ++st) {
-        const uint4 a = *reinterpret_cast<const uint4*>(kr + st * 16);
-        s[ks] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a),
-                                                        __builtin_bit_cast(bf16x8_t, qreg[st]),
-                                                        s[ks], 0, 0, 0);
-      }
-    }
-    // ---- online softmax over this lane's 32 keys (+ the partner half's 32)
-    const bool diag = key0 + kBN - 1 > pos + tt * kBM;  // some (query, key) pair is masked
-    const int vis = pos + t_lane - key0;                  // keys 0..vis of the tile are visible
-    float mx = -INFINITY;
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        float x = s[ks][e] * p.scale_log2e;
-        if (diag) {
-          const int key = ks * 32 + 16 * (e >> 3) + 8 * kq + (e & 7);
-          if (key > vis) x = -INFINITY;
-        }
-        s[ks][e] = x;
-        mx = fmaxf(mx, x);
-      }
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float m_new = fmaxf(m_run, mx);
-    // m_new is finite: key 0 is visible to every query, and tiles come in key order
-    const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-    float sum = 0.f;
-    uint4 pb[2][2];
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      float pr[16];
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        pr[e] = __builtin_amdgcn_exp2f(s[ks][e] - m_new);
-        sum += pr[e];
-      }
-#pragma unroll
-      for (int st = 0; st < 2; ++st) {
-        pb[ks][st].x = pack_bf2(pr[8 * st + 0], pr[8 * st + 1]);
-        pb[ks][st].y = pack_bf2(pr[8 * st + 2], pr[8 * st + 3]);
-        pb[ks][st].z = pack_bf2(pr[8 * st + 4], pr[8 * st + 5]);
-        pb[ks][st].w = pack_bf2(pr[8 * st + 6], pr[8 * st + 7]);
-      }
-    }
-    sum += __shfl_xor(sum, 32, 64);
-    l_run = l_run * alpha + sum;
-    m_run = m_new;
-    // ---- O^T = alpha * O^T + V^T P^T
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
-#pragma unroll
-      for (int e = 0; e < 16; ++e) o[dt][e] *= alpha;
-      const bf16_t* vr = &v_lds[(dt * 32 + n) * VS + kq * 8];
+    if (key0 + kBN - 1 > pos + tt * kBM) {  // some (query, key) pair of the wave is masked
+      const int vis = pos + t_lane - key0;  // keys 0..vis of the tile are visible
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-        for (int st = 0; st < 2; ++st) {
-          const uint4 a = *reinterpret_cast<const uint4*>(vr + ks * 32 + st * 16);
-          o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a),
-                                                          __builtin_bit_cast(bf16x8_t, pb[ks][st]),
-                                                          o[dt], 0, 0, 0);
-        }
+        for (int e = 0; e < 16; ++e)
+          if (ks * 32 + 16 * (e >> 3) + 8 * kq + (e & 7) > vis) s[ks][e] = -INFINITY;
     }
-  }
+  };
+  // The reference point m_run moves only when some score lies more than kSlack (in powers of
+  // two) above it: weights up to 2^kSlack are as exact in bf16 and float32 as ones up to 1, and
+  // the rescaling - and the exchange between the halves of a query - is left out otherwise.
+  auto settle = [&](float mx) {
+    if (__builtin_amdgcn_ballot_w64(mx > m_lim) == 0) return;  // (at the first tile: -infinity)
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    const float m_new = fmaxf(m_run, mx);
+    // (a query that has seen no key yet keeps -infinity as its maximum and 0 as its reference)
+    const float ref = m_new == -INFINITY ? 0.f : m_new * p.scale_log2e;
+    const float alpha = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_ref - ref);
+    l0 *= alpha;
+    l1 *= alpha;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) o[dt][e] *= alpha;
+    m_run = m_new;
+    m_ref = ref;
+    m_lim = m_new + p.slack;
+  };
+  constexpr int AHEAD = 3;  // operands in flight from LDS
 
+  // One tile: the products of the NEXT tile's scores, the weights of this one between them; then
+  // this tile's V products, the next scores' maximum between them.  Tile kt's scores are in `s`
+  // (masked, the maximum settled), K of kt + 1 and V of kt in LDS.
+  auto tile_step = [&](floatx16(&s)[2], floatx16(&sn)[2], int kt, int par) {
+    const lds_char kt_lds = lds + (par ^ 1) * TILE, vt_lds = lds + (2 + par) * TILE;
+    u32x4 a[4];
+    float x[32], w[32];
+    uint32_t pb[16];
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) a[i] = read_k(kt_lds, i);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) sn[ks][e] = 0.f;
+    // weights in three stages, a stage per slot: exponent; power; sum and rounding
+    constexpr int PER = 32 / (2 * STEPS);  // scores per slot
+    auto stage = [&](int i) {
+#pragma unroll
+      for (int e = i * PER; e < (i + 1) * PER; ++e)
+        if (e < 32) {
+          x[e] = fmaf(s[e >> 4][e & 15], p.scale_log2e, -m_ref);
+          hold(x[e]);
+        }
+#pragma unroll
+      for (int e = (i - 1) * PER; e < i * PER; ++e)
+        if (e >= 0 && e < 32) {
+          w[e] = __builtin_amdgcn_exp2f(x[e]);
+          hold(w[e]);
+        }
+#pragma unroll
+      for (int e = (i - 2) * PER; e < (i - 1) * PER; e += 2)
+        if (e >= 0 && e < 32) {
+          l0 += w[e];
+          l1 += w[e + 1];
+          pb[e >> 1] = pack_bf2(w[e], w[e + 1]);
+          hold(pb[e >> 1]);
+          hold(l0);
+          hold(l1);
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < 2 * STEPS; ++i) {
+      sn[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a[i & 3]),
+                                                          __builtin_bit_cast(bf16x8_t, qreg[i >> 1]), sn[i & 1], 0, 0, 0);
+      a[(i + AHEAD) & 3] = i + AHEAD < 2 * STEPS ? read_k(kt_lds, i + AHEAD) : read_v(vt_lds, i + AHEAD - 2 * STEPS);
+      stage(i);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    stage(2 * STEPS);
+    stage(2 * STEPS + 1);
+    mask(sn, kt + 1);
+    float mx = fmaxf(sn[0][0], sn[1][0]);
+    constexpr int VS = 4 * DT, MPER = 16 / VS;  // V products; pairs of scores per slot
+#pragma unroll
+    for (int i = 0; i < VS; ++i) {
+      const int g = i / DT, dt = i % DT;  // 16 keys: registers 4g .. 4g+3 of the weights
+      const uint4 bw = make_uint4(pb[4 * g], pb[4 * g + 1], pb[4 * g + 2], pb[4 * g + 3]);
+      o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a[(i + 2 * STEPS) & 3]),
+                                                      __builtin_bit_cast(bf16x8_t, bw), o[dt], 0, 0, 0);
+      if (i + AHEAD < VS) a[(i + AHEAD + 2 * STEPS) & 3] = read_v(vt_lds, i + AHEAD);
+#pragma unroll
+      for (int e = i * MPER; e < (i + 1) * MPER; ++e) mx = fmaxf(fmaxf(mx, sn[0][e]), sn[1][e]);
+      hold(mx);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (kt + 1 < n_tiles) settle(mx);
+  };
+
+  const int n_mine = last_w / kBN + 1 - t_first;  // tiles that this wave's rows see (<= 0: none)
+  load_tile(rk, koff, 0, 0);
+  load_tile(rv, voff, 2, 0);
+  load_tile(rk, koff, 1, 1);
+  // Every load so far (the Q operand among them) has landed before the loop is entered: left
+  // to itself the compiler waits, in EVERY iteration, for as many loads as were issued after Q.
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+  __syncthreads();
+  floatx16 s0[2], s1[2];
+  if (n_mine > 0) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) s0[ks][e] = 0.f;
+#pragma unroll
+    for (int i = 0; i < 2 * STEPS; ++i)
+      s0[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, read_k(lds, i)),
+                                                          __builtin_bit_cast(bf16x8_t, qreg[i >> 1]), s0[i & 1], 0, 0, 0);
+    mask(s0, 0);
+    float mx = fmaxf(s0[0][0], s0[1][0]);
+#pragma unroll
+    for (int e = 1; e < 16; ++e) mx = fmaxf(fmaxf(mx, s0[0][e]), s0[1][e]);
+    settle(mx);
+  }
+  // K of tile kt + 2 goes where K of kt was, V of kt + 1 where V of kt - 1 was: both last read before the barrier
+  // that ended the previous tile, both complete at the one that ends this tile.  (A step past the wave's
+  // or the workgroup's last tile multiplies what lies in LDS and uses none of it.)
+  for (int kt = 0; kt < n_iter; kt += 2) {
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+    __syncthreads();
+    if (kt + 2 < n_tiles) load_tile(rk, koff, 0, kt + 2);
+    if (kt + 1 < n_tiles) load_tile(rv, voff, 3, kt + 1);
+    if (kt < n_mine && kt < n_tiles) tile_step(s0, s1, kt, 0);
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+    __syncthreads();
+    if (kt + 3 < n_tiles) load_tile(rk, koff, 1, kt + 3);
+    if (kt + 2 < n_tiles) load_tile(rv, voff, 2, kt + 2);
+    if (kt + 1 < n_mine && kt + 1 < n_tiles) tile_step(s1, s0, kt + 1, 1);
+  }
+  float l_run = l0 + l1;
+  l_run += __shfl_xor(l_run, 32, 64);
   if (SPLIT) {
     // the second team's sums: through LDS (lane-contiguous floats per register), merged into
     // the first team's, which goes on alone
@@ -265,8 +359,8 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, SPLIT ? 1 : 2) void fa_prefill_k
     if (team == 1) return;  // (no workgroup barrier after this point)
     const float m1 = ex[(DT * 16) * 64 + lane], l1 = ex[(DT * 16 + 1) * 64 + lane];
     const float m = fmaxf(m_run, m1);  // finite: key 0 is visible to one of the teams
-    const float a0 = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run - m);
-    const float a1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m1 - m);
+    const float a0 = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m_run - m) * p.scale_log2e);
+    const float a1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m1 - m) * p.scale_log2e);
     l_run = l_run * a0 + l1 * a1;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
@@ -300,7 +394,10 @@ int exo_sdpa_prefill_mfma(const bf16_t* q, const bf16_t* k_cache, const bf16_t* 
   p.v = v_cache;
   p.pos = pos;
   p.out = out;
-  p.scale_log2e = scale * 1.4426950408889634f;
+  // (a scale of zero: one that rounds every score to zero, so that masked ones stay minus infinity)
+  p.scale_log2e = fmaxf(fabsf(scale) * 1.4426950408889634f, 1e-30f);
+  p.slack = kSlack / p.scale_log2e;
+  p.q_sign = scale < 0.f ? 0x80008000u : 0u;
   p.T = T;
   p.Hq = Hq;
   p.Hkv = Hkv;

@@ -77,3 +77,34 @@ def test_grouped_gemm_multiplies_the_rows_of_its_tile(device, rows):
     for e in (0, 2, 3):
         sel = (idx[:, 0] == e).nonzero()[:, 0]
         check(y[sel, 0], x[sel, 0], weights64(qs[e]), what=f"expert {e} of {len(sel)} rows")
+
+
+# prompts whose last key tile ends with the cache or inside it, queries that see none of a workgroup's later
+# tiles (300 behind 40: the second half of a split starts past the first queries), one and several heads
+# per kv head, both head sizes, a scale of either sign, scores that reach far above the first tile's
+@pytest.mark.parametrize("T,past,Hq,Hkv,D,spare,scale", [
+    (300, 40, 32, 8, 128, 0, 1.0), (300, 40, 4, 4, 128, 7, 1.0), (9, 0, 4, 4, 64, 0, 1.0), (33, 30, 4, 1, 128, 1, -1.0),
+    (257, 61, 8, 1, 64, 0, 1.0), (130, 5, 6, 2, 128, 70, 0.3), (1000, 0, 8, 2, 128, 24, 6.0), (64, 0, 8, 8, 64, 0, 6.0),
+    (2100, 100, 16, 2, 128, 0, 1.0), (520, 1000, 8, 8, 64, 3, -6.0), (128, 64, 4, 2, 64, 0, 0.0)])
+def test_prompt_attention_at_tile_edges(device, T, past, Hq, Hkv, D, spare, scale):
+    g = torch.Generator(device=device).manual_seed(T + past)
+    B, S = 2, past + T + spare
+    q = torch.randn(B * T, Hq * D, device=device, generator=g).bfloat16()
+    k = torch.randn(B, Hkv, S, D, device=device, generator=g)
+    k = (k * torch.linspace(0.2, 1.5, S, device=device)[:, None]).bfloat16()  # later keys score higher
+    v = torch.randn(B, Hkv, S, D, device=device, generator=g).bfloat16()
+    pos = torch.full((B,), past, dtype=torch.int32, device=device)
+    out = torch.empty_like(q)
+    sc = scale * D**-0.5
+    ops.sdpa_prefill(q, k, v, pos, out, sc, B, T, Hq, Hkv, D)
+    keep = torch.arange(S, device=device) <= torch.arange(T, device=device)[:, None] + past
+    for b in range(B):
+        for h in range(Hq):
+            kk, vv = k[b, h * Hkv // Hq].double(), v[b, h * Hkv // Hq].double()
+            s = ((q.view(B, T, Hq, D)[b, :, h].double() @ kk.T) * sc).masked_fill(~keep, float("-inf"))
+            w = s.softmax(-1)
+            want = w @ vv
+            # weights and the result rounded to bf16 once each (2^-9), float32 scores and sums
+            slack = 2.0**-8 * (w @ vv.abs()) + 1e-5
+            bad = (out.view(B, T, Hq, D)[b, :, h].double() - want).abs() > slack + 2.0**-8 * want.abs()
+            assert not bad.any(), f"sequence {b} head {h}: {int(bad.sum())} outputs, first at {bad.nonzero()[0].tolist()}"
