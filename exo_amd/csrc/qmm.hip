@@ -49,6 +49,8 @@
 //    of eight register stages nothing, four K steps per barrier nothing: none was kept.
 #include "../../include/exo_mi355x.h"
 #include "common.h"
+#include "dequant.h"
+#include "qmm_short.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -89,18 +91,6 @@ struct QmmParams {
   const bf16_t* b2 = nullptr;
 };
 
-// byte I of v as float.  Written as the instruction: the compiler otherwise extracts
-// bytes 1 and 2 with a v_bfe_u32 first.
-template <int I>
-__device__ __forceinline__ float ubyte_f(uint32_t v) {
-  float f;
-  if (I == 0) asm("v_cvt_f32_ubyte0 %0, %1" : "=v"(f) : "v"(v));
-  if (I == 1) asm("v_cvt_f32_ubyte1 %0, %1" : "=v"(f) : "v"(v));
-  if (I == 2) asm("v_cvt_f32_ubyte2 %0, %1" : "=v"(f) : "v"(v));
-  if (I == 3) asm("v_cvt_f32_ubyte3 %0, %1" : "=v"(f) : "v"(v));
-  return f;
-}
-
 // buffer descriptor over memory that starts at `base`: raw (stride 0) 32-bit data, no
 // range check (every offset the kernel forms is in range by construction)
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base) {
@@ -130,23 +120,8 @@ struct WRaw {
 // 8 codes -> the bf16x8 B operand of one MFMA step
 template <int BITS>
 __device__ __forceinline__ bf16x8_t dequant8(const WRaw<BITS>& r, int t, float s, float b) {
-  uint4 o;
-  if (BITS == 4) {
-    const uint32_t v = reinterpret_cast<const uint32_t*>(&r.q[0])[t];
-    const uint32_t ev = v & 0x0f0f0f0fu, od = (v >> 4) & 0x0f0f0f0fu;
-    o.x = pack_bf2(fmaf(s, ubyte_f<0>(ev), b), fmaf(s, ubyte_f<0>(od), b));
-    o.y = pack_bf2(fmaf(s, ubyte_f<1>(ev), b), fmaf(s, ubyte_f<1>(od), b));
-    o.z = pack_bf2(fmaf(s, ubyte_f<2>(ev), b), fmaf(s, ubyte_f<2>(od), b));
-    o.w = pack_bf2(fmaf(s, ubyte_f<3>(ev), b), fmaf(s, ubyte_f<3>(od), b));
-  } else {
-    const uint32_t v0 = reinterpret_cast<const uint32_t*>(&r.q[0])[2 * t];
-    const uint32_t v1 = reinterpret_cast<const uint32_t*>(&r.q[0])[2 * t + 1];
-    o.x = pack_bf2(fmaf(s, ubyte_f<0>(v0), b), fmaf(s, ubyte_f<1>(v0), b));
-    o.y = pack_bf2(fmaf(s, ubyte_f<2>(v0), b), fmaf(s, ubyte_f<3>(v0), b));
-    o.z = pack_bf2(fmaf(s, ubyte_f<0>(v1), b), fmaf(s, ubyte_f<1>(v1), b));
-    o.w = pack_bf2(fmaf(s, ubyte_f<2>(v1), b), fmaf(s, ubyte_f<3>(v1), b));
-  }
-  return __builtin_bit_cast(bf16x8_t, o);
+  const uint32_t* w = reinterpret_cast<const uint32_t*>(&r.q[0]);
+  return BITS == 4 ? dequant_words8<4>(w[t], 0, s, b) : dequant_words8<8>(w[(2 * t) & 7], w[(2 * t + 1) & 7], s, b);
 }
 
 // One 32-bit register (two bf16) of that operand: piece P = 0..3.  `lo`, `hi` are the two
@@ -908,6 +883,13 @@ __global__ __launch_bounds__(256) void qmm_reduce_kernel(const float* __restrict
   }
 }
 
+void reduce_parts(const float* part, const bf16_t* residual, bf16_t* y, int M, int N, int parts, hipStream_t st) {
+  const int64_t total = (int64_t)M * N;
+  const int vec_ok = (((uintptr_t)y | (uintptr_t)residual) & 7) == 0;
+  qmm_reduce_kernel<<<dim3(exo_ceil_div(exo_ceil_div(total, 4), 256)), 256, 0, st>>>(
+      part, residual, y, total, (int64_t)part_stride(M, N), parts, vec_ok);
+}
+
 // Pair mode: sums of the gate and of the up partials, each rounded to bf16 as the projections
 // of two GEMMs would be, then SwiGLU.  `stride` floats between K ranges, `half` between the
 // gate and the up partials of one range.
@@ -1044,10 +1026,7 @@ void launch_qmm(const QmmParams& p, hipStream_t st) {
       exo_note_variant("qmm_kernel<%d, 2, false, true, false, true, true>", BITS), qmm_kernel<BITS, 2, false, true, false, true, true><<<g, 256, 0, st>>>(p);
     else
       exo_note_variant("qmm_kernel<%d, 2, false, true, false, true>", BITS), qmm_kernel<BITS, 2, false, true, false, true><<<g, 256, 0, st>>>(p);
-    const int64_t total = (int64_t)M * N;
-    const int vec_ok = (((uintptr_t)p.y | (uintptr_t)p.residual) & 7) == 0;
-    qmm_reduce_kernel<<<dim3(exo_ceil_div(exo_ceil_div(total, 4), 256)), 256, 0, st>>>(
-        p.part, p.residual, p.y, total, (int64_t)part_stride(M, N), p.ksplit, vec_ok);
+    reduce_parts(p.part, p.residual, p.y, M, N, p.ksplit, st);
     return;
   }
   // taller inputs: 256-row tiles halve the dequantisation work and the LDS reads per output
@@ -1075,12 +1054,7 @@ void launch_qmm(const QmmParams& p, hipStream_t st) {
       exo_note_variant("qmm_kernel<%d, 2, false, true>", BITS), qmm_kernel<BITS, 2, false, true><<<g2, 256, 0, st>>>(p);
     else
       exo_note_variant("qmm_kernel<%d, 2, false, false>", BITS), qmm_kernel<BITS, 2, false, false><<<g2, 256, 0, st>>>(p);
-    if (p.ksplit > 1) {
-      const int64_t total = (int64_t)M * N;
-      const int vec_ok = (((uintptr_t)p.y | (uintptr_t)p.residual) & 7) == 0;
-      qmm_reduce_kernel<<<dim3(exo_ceil_div(exo_ceil_div(total, 4), 256)), 256, 0, st>>>(
-          p.part, p.residual, p.y, total, (int64_t)part_stride(M, N), p.ksplit, vec_ok);
-    }
+    if (p.ksplit > 1) reduce_parts(p.part, p.residual, p.y, M, N, p.ksplit, st);
   } else {
     // up to one tall tile per CU: eight waves per tile, K in two halves (four-wave workgroups
     // leave one wave per SIMD there).  4096x4096 under 2046 rows, 256 tiles: 95.0 -> 89.7 us,
@@ -1400,6 +1374,12 @@ extern "C" int exo_qmm_swiglu_ws(const uint16_t* x, const uint32_t* w_gate,
                              ((uintptr_t)workspace & 255) == 0),
               "exo_qmm_swiglu_ws: workspace of %lld bytes, need %lld (256-byte aligned)",
               (long long)workspace_bytes, (long long)exo_qmm_swiglu_workspace(M, N));
+  if (exo_qmm_short_fits(M, K)) {
+    exo_qmm_short(x, w_gate, s_gate, b_gate, w_up, s_up, b_up, nullptr, y, M, N, K, bits, 1, nullptr, 0,
+                  (hipStream_t)stream);
+    EXO_CHECK_LAUNCH("exo_qmm_swiglu");
+    return EXO_OK;
+  }
   QmmParams p{x, w_gate, s_gate, b_gate, nullptr, y, M, N, K};
   p.sorted = nullptr;
   p.tiles = nullptr;
@@ -1462,6 +1442,17 @@ extern "C" int exo_qmm_ws(const uint16_t* x, const uint32_t* w, const uint16_t* 
                              ((uintptr_t)workspace & 255) == 0),
               "exo_qmm_ws: workspace of %lld bytes, need %lld (256-byte aligned)",
               (long long)workspace_bytes, (long long)exo_qmm_workspace(M, N));
+  EXO_REQUIRE((int64_t)M * K < (1ll << 31), "exo_qmm: M*K=%lld exceeds 32-bit byte offsets",
+              (long long)M * K);
+  if (exo_qmm_short_fits(M, K)) {
+    const int parts = workspace ? exo_qmm_short_parts(N, K) : 1;
+    float* const part = reinterpret_cast<float*>(workspace);
+    exo_qmm_short(x, w, scales, biases, nullptr, nullptr, nullptr, residual, y, M, N, K, bits, parts, part,
+                  part_stride(M, N), (hipStream_t)stream);
+    if (parts > 1) reduce_parts(part, residual, y, M, N, parts, (hipStream_t)stream);
+    EXO_CHECK_LAUNCH("exo_qmm");
+    return EXO_OK;
+  }
   QmmParams p{x, w, scales, biases, residual, y, M, N, K};
   p.sorted = nullptr;
   p.tiles = nullptr;
@@ -1471,8 +1462,6 @@ extern "C" int exo_qmm_ws(const uint16_t* x, const uint32_t* w, const uint16_t* 
   if (!p.wide) plan_split(M, N, K, workspace != nullptr, &p.ksplit, &p.kc);
   p.part = reinterpret_cast<float*>(workspace);
   EXO_REQUIRE(exo_ceil_div(M, 128) <= 65535, "exo_qmm: M=%d too large", M);
-  EXO_REQUIRE((int64_t)M * K < (1ll << 31), "exo_qmm: M*K=%lld exceeds 32-bit byte offsets",
-              (long long)M * K);
   if (bits == 4)
     launch_qmm<4>(p, (hipStream_t)stream);
   else

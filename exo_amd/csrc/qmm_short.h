@@ -1,0 +1,19 @@
+// The quantised GEMM of short prompts (qmm_short.hip).
+#pragma once
+#include "common.h"
+
+// Inputs that it takes: 17 to kQmmShortMaxRows rows (fewer: the GEMV family), rows of whole groups whose
+// scales fit beside the activations in LDS.
+// (two blocks of 64 rows would read the weights twice: pair of 14336x4096 under 126 rows 61 us against 54)
+constexpr int kQmmShortMaxRows = 64;
+constexpr int kQmmShortMaxK = 32768;
+inline bool exo_qmm_short_fits(int M, int K) { return M > 16 && M <= kQmmShortMaxRows && K % 64 == 0 && K <= kQmmShortMaxK; }
+
+// parts of K that a launch without a second matrix is best split into
+int exo_qmm_short_parts(int N, int K);
+
+// y[M,N] = x w^T (+ residual), or with a second matrix silu(x w^T) * (x w2^T); with several parts of K only their
+// float32 sums, to part[parts][part_stride]
+void exo_qmm_short(const bf16_t* x, const uint32_t* w, const bf16_t* s, const bf16_t* b, const uint32_t* w2,
+                   const bf16_t* s2, const bf16_t* b2, const bf16_t* residual, bf16_t* y, int M, int N, int K, int bits,
+                   int parts, float* part, size_t part_stride, hipStream_t stream);

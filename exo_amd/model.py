@@ -138,10 +138,8 @@ class _Buffers:
             self.router_logits = torch.empty(R, c.num_experts, **bf)
             self.act = torch.empty(R, k, Ie, **bf)
             self.expert_out = torch.empty(R, k, c.hidden_size, **bf)
-            self.gate = self.up = None
         else:
             self.act = torch.empty(R, c.intermediate_size, **bf)
-            self.gate = self.up = None
         self.sdpa_ws = ops.sdpa_decode_workspace(B, Hq, D, device)
         # sampling outputs (last shard)
         self.logits = None
@@ -309,17 +307,8 @@ class ShardModel(DecoderShard):
             if gemv:  # post-attention norm and SwiGLU fused into the gate/up GEMV pair
                 ops.qmv_swiglu(bf.h, L.gate, L.up, out=bf.act, norm_weight=L.post_norm,
                                eps=c.rms_norm_eps)
-            elif R >= 64:  # one GEMM launch for both projections, SwiGLU in its epilogue
+            else:  # both projections and the SwiGLU in one GEMM launch
                 ops.qmm_swiglu(bf.n, L.gate, L.up, out=bf.act)
-            else:  # up to 63 rows: the 256-column split-K GEMM per projection is faster
-                #   (8192x2048 at 126 rows: pair 27 us, two GEMMs + SwiGLU 44 us; at 32 rows 28 / 29
-                #   us; 14336x4096 at 32 rows 58 / 46 us, at 64 rows 57 / 59 us)
-                if bf.gate is None:
-                    bf.gate = torch.empty_like(bf.act)
-                    bf.up = torch.empty_like(bf.act)
-                ops.quantized_matmul(bf.n, L.gate, out=bf.gate)
-                ops.quantized_matmul(bf.n, L.up, out=bf.up)
-                ops.swiglu(bf.gate, bf.up, out=bf.act)
             ops.quantized_matmul(bf.act, L.down, residual=bf.h, out=bf.h)
             return
         if gemv:  # decode: the post-attention norm is fused into both consumers of it

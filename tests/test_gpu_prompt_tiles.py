@@ -108,3 +108,28 @@ def test_prompt_attention_at_tile_edges(device, T, past, Hq, Hkv, D, spare, scal
             slack = 2.0**-8 * (w @ vv.abs()) + 1e-5
             bad = (out.view(B, T, Hq, D)[b, :, h].double() - want).abs() > slack + 2.0**-8 * want.abs()
             assert not bad.any(), f"sequence {b} head {h}: {int(bad.sum())} outputs, first at {bad.nonzero()[0].tolist()}"
+
+
+# 17 to 64 rows: both sizes of the row tile, a step count below, at and above the eight waves, rows of scales that are no
+# whole 16-byte pieces (K of 64, 192, 832), one to seven column tiles per workgroup, K in four parts, ragged columns
+@pytest.mark.parametrize("M,N,K,bits", [(17, 4096, 64, 4), (32, 264, 192, 8), (33, 4099, 832, 4), (64, 12290, 512, 4),
+                                        (61, 8200, 1024, 8), (18, 16400, 512, 4), (48, 28680, 512, 4), (63, 4096, 8192, 4),
+                                        (31, 1030, 14336, 8), (64, 40, 8192, 4), (40, 128, 2048, 8), (20, 32, 32768, 4)])
+def test_short_prompt_gemm(device, M, N, K, bits):
+    q = packed(N, K, bits, M + N, device)
+    g = torch.Generator(device=device).manual_seed(M)
+    x = torch.randn(M, K, device=device, generator=g).bfloat16()
+    r = torch.randn(M, N, device=device, generator=g).bfloat16()
+    w = weights64(q)
+    check(ops.quantized_matmul(x, q), x, w, what=f"{M}x{N}x{K}")
+    check(ops.quantized_matmul(x, q, residual=r), x, w, r, what=f"{M}x{N}x{K} with residual")
+    check(ops.qmm(x, q), x, w, what=f"{M}x{N}x{K} without workspace")
+
+
+@pytest.mark.parametrize("M,N,K,bits", [(17, 40, 64, 4), (33, 4100, 832, 8), (64, 14336, 512, 4), (50, 8192, 1024, 4), (24, 2050, 2048, 8)])
+def test_short_prompt_pair_gemm(device, M, N, K, bits):
+    """The pair in one launch has the bits of two launches and the SwiGLU kernel."""
+    gate, up = packed(N, K, bits, M, device), packed(N, K, bits, N, device)
+    x = torch.randn(M, K, device=device, generator=torch.Generator(device=device).manual_seed(K)).bfloat16()
+    want = ops.swiglu(ops.qmm(x, gate), ops.qmm(x, up))
+    assert torch.equal(ops.qmm_swiglu(x, gate, up).view(torch.int16), want.view(torch.int16))
