@@ -492,6 +492,19 @@ __global__ __launch_bounds__(256) void sample_fine_kernel(
   RowWs* w = row_ws(ws, row);
   Tables* T = row_tables(ws, row);
   const Wanted q = wanted_of(p, want_top != 0);
+  // the slice's values and the row's partials first: their way from L2 is the scan's
+  const SliceGeom g = slice_geom(logits, V, blockIdx.x);
+  for (int i = threadIdx.x; i < kTargets * kFine; i += 256) {
+    (&hm[0][0])[i] = 0;
+    (&hc[0][0])[i] = 0;
+  }
+  stage_edits(w, g, ed);
+  float xv[16];
+  int i0[2];
+  load_share(logits + (size_t)row * V, g, ed, xv, i0);
+  float mx, lse;
+  int mi;
+  merge_stats(w, mx, mi, lse);
   // every wave finds the target buckets for itself (512 entries, L2 resident)
   int bkt[kTargets];
   unsigned int ac[kTargets];
@@ -511,18 +524,6 @@ __global__ __launch_bounds__(256) void sample_fine_kernel(
     }
   }
   if (bkt[0] < 0 && bkt[1] < 0 && bkt[2] < 0) return;  // (uniform over the workgroup)
-  const SliceGeom g = slice_geom(logits, V, blockIdx.x);
-  for (int i = threadIdx.x; i < kTargets * kFine; i += 256) {
-    (&hm[0][0])[i] = 0;
-    (&hc[0][0])[i] = 0;
-  }
-  stage_edits(w, g, ed);
-  float mx, lse;
-  int mi;
-  merge_stats(w, mx, mi, lse);
-  float xv[16];
-  int i0[2];
-  load_share(logits + (size_t)row * V, g, ed, xv, i0);
 #pragma unroll
   for (int u = 0; u < 2; ++u)
 #pragma unroll
@@ -550,16 +551,14 @@ __global__ __launch_bounds__(256) void sample_fine_kernel(
   }
 }
 
-// The exact keys from the fine tables (one wave; the same values in every lane): the value
-// threshold of top-k / top-p (-inf: none) and the key of the 20th largest value (0: none).
-__device__ __forceinline__ void fine_thresholds(const RowWs* w, const Tables* T, const Wanted& q,
-                                                float& thr, int& key_top) {
-  thr = -INFINITY;
-  key_top = 0;
-#pragma unroll
-  for (int j = 0; j < kTargets; ++j) {
-    const int b = w->bkt[j];
-    if (b < 0) continue;  // fewer than k (20) tokens in all, or the mass never reaches top_p
+// The exact keys from the fine tables, a target per wave (left in `keys`; the caller's barrier): the keys of
+// the k-th largest value, of the nucleus edge and of the 20th largest value, -1 for none.
+__device__ __forceinline__ void fine_keys(const RowWs* w, const Tables* T, const Wanted& q, int (&keys)[kTargets]) {
+  const int j = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  if (j >= kTargets) return;
+  const int b = w->bkt[j];  // (-1: fewer than k (20) tokens in all, or the mass never reaches top_p)
+  int key = -1;
+  if (b >= 0) {
     const unsigned int c0[kTargets] = {w->above_c[j], w->above_c[j], w->above_c[j]};
     const unsigned long long m0[kTargets] = {w->above_m[j], w->above_m[j], w->above_m[j]};
     const bool active[kTargets] = {j == 0, j == 1, j == 2};
@@ -567,14 +566,10 @@ __device__ __forceinline__ void fine_thresholds(const RowWs* w, const Tables* T,
     unsigned int fc[kTargets];
     unsigned long long fm[kTargets];
     scan_down<kFine / 64>(T->fm[j], T->fc[j], q, c0, m0, active, f, fc, fm);
-    if (f[j] >= 0) {
-      const int key = (b << 7) | f[j];
-      if (j == 2)
-        key_top = key;
-      else
-        thr = fmaxf(thr, value_of(key));
-    }
+    const int at = j == 0 ? f[0] : j == 1 ? f[1] : f[2];
+    if (at >= 0) key = (b << 7) | at;
   }
+  if ((threadIdx.x & 63) == 0) keys[j] = key;
 }
 
 // ---- weights ------------------------------------------------------------------
@@ -595,14 +590,27 @@ __global__ __launch_bounds__(256) void sample_weights_kernel(
   const bool sampling = p.temperature != 0.f;
   if (!sampling && !want_top) return;
   RowWs* w = row_ws(ws, row);
-  // the exact keys of this step from the fine tables (every wave for itself); the first
-  // workgroup leaves them for the select launch and clears the bucket table, whose last
-  // reader was the previous launch
+  // the slice's values and the row's partials first: their way from L2 is the scans'
+  const SliceGeom g = slice_geom(logits, V, blockIdx.x);
+  stage_edits(w, g, ed);
+  float xv[16];
+  int i0[2];
+  load_share(logits + (size_t)row * V, g, ed, xv, i0);
+  float mx, lse;
+  int mi;
+  merge_stats(w, mx, mi, lse);
+  // the exact keys of this step from the fine tables; the first workgroup leaves them for the select
+  // launch and clears the bucket table, whose last reader was the previous launch
   float table_thr = -INFINITY;
   int kt = 0;
-  if (row_needs_table(p, want_top != 0)) {
+  if (row_needs_table(p, want_top != 0)) {  // (uniform over the workgroup)
+    __shared__ int s_keys[kTargets];
     Tables* T = row_tables(ws, row);
-    fine_thresholds(w, T, wanted_of(p, want_top != 0), table_thr, kt);
+    fine_keys(w, T, wanted_of(p, want_top != 0), s_keys);
+    __syncthreads();
+    if (s_keys[0] >= 0) table_thr = value_of(s_keys[0]);
+    if (s_keys[1] >= 0) table_thr = fmaxf(table_thr, value_of(s_keys[1]));
+    if (s_keys[2] >= 0) kt = s_keys[2];
     if (blockIdx.x == 0) {
       if (threadIdx.x == 0) {
         w->thr = table_thr;
@@ -614,14 +622,6 @@ __global__ __launch_bounds__(256) void sample_weights_kernel(
       }
     }
   }
-  const SliceGeom g = slice_geom(logits, V, blockIdx.x);
-  stage_edits(w, g, ed);
-  float mx, lse;
-  int mi;
-  merge_stats(w, mx, mi, lse);
-  float xv[16];
-  int i0[2];
-  load_share(logits + (size_t)row * V, g, ed, xv, i0);
   if (want_top) {
     // strictly above the 20th largest value: at most 19 tokens in the whole row, any order
     // (the select launch ranks them); equal to it: this slice's first kTop in vocabulary
@@ -726,37 +726,29 @@ __global__ __launch_bounds__(256) void sample_select_kernel(
   int tok = mi;
   float x_tok = mx;
   if (p.temperature != 0.f) {
-    if (tid == 0) {
-      // the slice in which the running sum of kept weights crosses u * total (slices in
-      // order, sums in float32, the same order every time)
-      float total = 0.f;
-      for (int b = 0; b < kBlocks; ++b) total += w->part[b][3];
+    if (wave == 0) {
+      // the slice in which the running sum of kept weights crosses u * total (slices in order, sums in float32,
+      // the same order every time): a lane holds its slice's sum and what runs up to it
+      const float wb = w->part[lane][3];
+      float total = 0.f, run = 0.f;
+#pragma unroll
+      for (int b = 0; b < kBlocks; ++b) {
+        if (lane == b) run = total;
+        total += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wb), b));
+      }
       uint32_t c[4] = {draws[row], 0u, 0u, 0u};
       philox4x32_10(c, p.seed_lo, p.seed_hi);
       const float u = (float)(c[0] >> 8) * 0x1p-24f;
       const float target = u * total;
-      float run = 0.f;
-      int blk = -1, last = 0;
-      float rem = 0.f;
-      for (int b = 0; b < kBlocks; ++b) {
-        const float wb = w->part[b][3];
-        if (wb > 0.f) {
-          last = b;
-          if (blk < 0 && run + wb > target) {
-            blk = b;
-            rem = target - run;
-          }
-        }
-        run += wb;
+      const unsigned long long kept = __ballot(wb > 0.f), hit = __ballot(wb > 0.f && run + wb > target);
+      // (no slice: rounding at the very end of the distribution)
+      const int blk = hit ? __ffsll((long long)hit) - 1 : kept ? 63 - __clzll((long long)kept) : 0;
+      if (lane == blk) {
+        s_block = blk;
+        s_rem = hit ? target - run : INFINITY;
+        s_tok = -1;
+        s_last_kept = -1;
       }
-      if (blk < 0) {  // rounding at the very end of the distribution
-        blk = last;
-        rem = INFINITY;
-      }
-      s_block = blk;
-      s_rem = rem;
-      s_tok = -1;
-      s_last_kept = -1;
     }
     __syncthreads();
     const SliceGeom g = slice_geom(logits, V, s_block);
@@ -843,29 +835,40 @@ __global__ __launch_bounds__(256) void sample_select_kernel(
     // the tokens strictly above the 20th largest value, ranked: higher key first, lower index
     // first among equals; then the tokens equal to it, lowest ids first (slices in order)
     const int n = min(w->cand_n, kTop - 1);
-    for (int c = tid; c < n; c += 256) {
-      const unsigned long long me = w->cand[c];
+    if (wave == 0) {
+      const unsigned long long me = lane < n ? w->cand[lane] : 0ull;
       const unsigned int mk = (unsigned int)(me >> 32), mi2 = (unsigned int)me;
       int rank = 0;
-      for (int o = 0; o < n; ++o) {
-        const unsigned long long ot = w->cand[o];
-        const unsigned int ok = (unsigned int)(ot >> 32), oi = (unsigned int)ot;
-        rank += (ok > mk || (ok == mk && oi < mi2)) ? 1 : 0;
+#pragma unroll
+      for (int o = 0; o < kTop - 1; ++o) {
+        const unsigned int ok = (unsigned int)__builtin_amdgcn_readlane((int)mk, o);
+        const unsigned int oi = (unsigned int)__builtin_amdgcn_readlane((int)mi2, o);
+        rank += o < n && (ok > mk || (ok == mk && oi < mi2)) ? 1 : 0;
       }
-      top_idx[(size_t)row * kTop + rank] = (int)mi2;
-      top_val[(size_t)row * kTop + rank] = value_of((int)mk) - lse;
+      if (lane < n) {
+        top_idx[(size_t)row * kTop + rank] = (int)mi2;
+        top_val[(size_t)row * kTop + rank] = value_of((int)mk) - lse;
+      }
     }
-    if (tid == 0) {
-      int at = n;
+    if (wave == 1) {  // a lane per slice: its ties go behind those of the slices before it
+      const int mine = w->tie_n[lane];
+      int inc = mine;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int up = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += up;
+      }
       const float tv = value_of(w->key_top) - lse;
-      for (int b = 0; b < kBlocks && at < kTop; ++b)
-        for (int j = 0; j < w->tie_n[b] && at < kTop; ++j, ++at) {
-          top_idx[(size_t)row * kTop + at] = w->tie_idx[b][j];
-          top_val[(size_t)row * kTop + at] = tv;
-        }
-      for (; at < kTop; ++at) {  // vocabularies of fewer than 20 tokens
-        top_idx[(size_t)row * kTop + at] = -1;
-        top_val[(size_t)row * kTop + at] = -INFINITY;
+      const int first = n + inc - mine;
+      for (int j = 0; j < mine && first + j < kTop; ++j) {
+        top_idx[(size_t)row * kTop + first + j] = w->tie_idx[lane][j];
+        top_val[(size_t)row * kTop + first + j] = tv;
+      }
+      // vocabularies of fewer than 20 tokens
+      const int all = n + __shfl(inc, 63, 64);
+      if (lane >= all && lane < kTop) {
+        top_idx[(size_t)row * kTop + lane] = -1;
+        top_val[(size_t)row * kTop + lane] = -INFINITY;
       }
     }
   }
