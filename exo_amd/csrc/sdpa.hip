@@ -37,9 +37,12 @@ constexpr int kBlk = 4;  // keys per lane group per step
 #define EXO_SDPA_TILES_IN_FLIGHT 2
 #endif
 constexpr int kTilesInFlight = EXO_SDPA_TILES_IN_FLIGHT;  // key tiles a wave keeps in flight
-#ifndef EXO_SDPA_ABL
-#define EXO_SDPA_ABL 0  // timing-only ablations (wrong results)
-#endif
+// Contexts of one workgroup: two rounds of four waves' requests (256 keys of 128, 512 of 64).  The hand-over of
+// the splits costs 2.2 us, a round about 0.8.  One sequence, 32 / 8 heads of 128: 60 keys 5.9 -> 3.9 us, 130 keys 5.9
+// -> 4.9, 250 keys 5.9 -> 5.2 (400 keys level); of 64, 130 keys 6.2 -> 4.9, 500 keys 6.3 -> 6.0 (900 keys 6.8 -> 8.1)
+constexpr int kSoloTiles = 2 * 4 * 2;
+constexpr int kSoloMfma = 256;  // the matrix-core kernel: 8 sequences, 130 keys 10.8 -> 8.7 us, 250 keys 11.9 -> 10.6
+                                // (500 keys 12.6 -> 13.8); 4 of 32 / 4 heads, 130 keys 12.1 -> 7.9
 #ifndef EXO_SDPA_TILES_WAVES
 #define EXO_SDPA_TILES_WAVES 4
 #endif
@@ -477,7 +480,11 @@ __global__ __launch_bounds__(64 * NW) void sdpa_tiles_kernel(const SdpaParams p)
   const int b = blockIdx.z;
   const int kvh = (int)blockIdx.y / p.hgroups, hg = (int)blockIdx.y % p.hgroups;
   const int h0 = kvh * (G * p.hgroups) + hg * G;  // first query head of this workgroup
-  const int nwv = p.splits * NW;
+  const int len = min(p.pos[b] + 1, p.S_max);  // keys visible to the query
+  // A short context is left to the first workgroup: the others are gone at once, and nothing is handed over
+  const bool solo = len <= kSoloTiles * STEP;
+  if (solo && blockIdx.x != 0) return;
+  const int nwv = solo ? NW : p.splits * NW;
   const int gwv = (int)blockIdx.x * NW + wave;
 
   const size_t head_base = ((size_t)b * p.Hkv + kvh) * p.S_max * D;
@@ -493,7 +500,6 @@ __global__ __launch_bounds__(64 * NW) void sdpa_tiles_kernel(const SdpaParams p)
       tl.v[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rv, lane_ofs + i * (KPI * D * 2), tb, 0));
     }
   };
-  const int len = min(p.pos[b] + 1, p.S_max);  // keys visible to the query
   const int n_keys = FUSED ? len - 1 : len;     // of which the cache holds these
   const bool own_new = FUSED && ((n_keys / STEP) % nwv) == gwv;  // this wave adds the new token
   const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
@@ -695,10 +701,10 @@ __global__ __launch_bounds__(64 * NW) void sdpa_tiles_kernel(const SdpaParams p)
       acc += red[w][g][e] * sc;
       lsum += red[w][g][D + 1] * sc;
     }
-#if (EXO_SDPA_ABL & 1)  // timing only: no hand-over, every split writes its own result
-    p.out[qrow + (size_t)(h0 + g) * D + e] = f2bf(acc / lsum);
-    continue;
-#endif
+    if (solo) {
+      p.out[qrow + (size_t)(h0 + g) * D + e] = f2bf(acc / lsum);
+      continue;
+    }
     float* dst = p.ws + ((size_t)(b * p.Hq + h0 + g) * p.splits + blockIdx.x) * (D + 2);
     st_dev(dst + e, acc);
     if (e == 0) {
@@ -706,9 +712,7 @@ __global__ __launch_bounds__(64 * NW) void sdpa_tiles_kernel(const SdpaParams p)
       st_dev(dst + D + 1, lsum);
     }
   }
-#if (EXO_SDPA_ABL & 1)
-  return;
-#endif
+  if (solo) return;
   // the last workgroup of this (sequence, kv head, head group) to finish merges the splits
   // (see sdpa_kernel); the counter returns to zero
   wait_own_stores_done();
@@ -779,6 +783,9 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_decode_mfma_kernel(const Sdp
   // the cache holds keys [0, len-1); key len-1 comes from the qkv row
   int chunk = (len + p.splits - 1) / p.splits;
   chunk = (chunk + TK * kWaves - 1) / (TK * kWaves) * (TK * kWaves);
+  if (len <= kSoloMfma) chunk = kSoloMfma;
+  const int used = (len + chunk - 1) / chunk;  // splits that have keys; the others are gone at once
+  if ((int)blockIdx.x >= used) return;
   const bool own_new = (len - 1) / chunk == (int)blockIdx.x;
   const int k_begin = min(min((int)blockIdx.x * chunk, len), len - 1);
   const int k_end = min(min((int)blockIdx.x * chunk + chunk, len), len - 1);
@@ -833,9 +840,6 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_decode_mfma_kernel(const Sdp
       for (int e = 0; e < 8; ++e) sincosf(fpos * p.inv_freq[(sl * 8 + e) % (D / 2)], &sn[e], &cs[e]);
     }
     const bf16_t* row = p.qkv + (size_t)b * (p.Hq + 2 * p.Hkv) * D;
-#if (EXO_SDPA_ABL & 8)  // timing only: no table, no rotation
-    for (int e = 0; e < 8; ++e) cs[e] = 1.f, sn[e] = 0.f;
-#endif
     for (int g = wave * 4 + sub; g < G; g += 4 * kWaves)  // a 16-lane group per head
       *reinterpret_cast<uint4*>(&q_lds[g * D + sl * 8]) =
           head_slice<D, true>(row + (size_t)(h0 + g) * D, sl, p.qn, p.eps, cs, sn);
@@ -877,10 +881,6 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_decode_mfma_kernel(const Sdp
     __builtin_amdgcn_wave_barrier();
     EXO_LOAD_TILE(k0 + TK)
 
-#if (EXO_SDPA_ABL & 4)  // timing only: tiles travel to LDS, nothing is computed
-    o[0][0] += bf2f(k_t[lane]) + bf2f(v_t[lane]);
-    continue;
-#endif
     floatx16 sc;
 #pragma unroll
     for (int e = 0; e < 16; ++e) sc[e] = 0.f;
@@ -1008,10 +1008,10 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_decode_mfma_kernel(const Sdp
       acc += red[w][g][e] * scw;
       lsum += red[w][g][D + 1] * scw;
     }
-#if (EXO_SDPA_ABL & 2)  // timing only: no hand-over, every split writes its own result
-    p.out[qrow + (size_t)(h0 + g) * D + e] = f2bf(acc / lsum);
-    continue;
-#endif
+    if (used == 1) {  // (nothing to hand over)
+      p.out[qrow + (size_t)(h0 + g) * D + e] = f2bf(acc / lsum);
+      continue;
+    }
     float* dst = p.ws + ((size_t)(b * p.Hq + h0 + g) * p.splits + blockIdx.x) * (D + 2);
     st_dev(dst + e, acc);
     if (e == 0) {
@@ -1019,16 +1019,14 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_decode_mfma_kernel(const Sdp
       st_dev(dst + D + 1, lsum);
     }
   }
-#if (EXO_SDPA_ABL & 2)
-  return;
-#endif
+  if (used == 1) return;
   // the last workgroup of this (sequence, kv head) merges the splits (see sdpa_kernel)
   wait_own_stores_done();
   __syncthreads();
   if (threadIdx.x == 0) {
     int* cnt = &p.counters[b * p.Hkv + blockIdx.y];
     const int old = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    s_last = (old == p.splits - 1);
+    s_last = (old == used - 1);
     if (s_last) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   __syncthreads();
@@ -1037,7 +1035,7 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_decode_mfma_kernel(const Sdp
     const int g = idx / D, e = idx % D;
     const int h = h0 + g;
     const float* src = p.ws + (size_t)(b * p.Hq + h) * p.splits * (D + 2);
-    p.out[qrow + (size_t)h * D + e] = f2bf(merge_splits<D>(src, p.splits, e));
+    p.out[qrow + (size_t)h * D + e] = f2bf(merge_splits<D>(src, used, e));
   }
 }
 
