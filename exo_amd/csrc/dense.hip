@@ -12,9 +12,11 @@
 //  * dense_gemm_kernel, any number of rows: a (64 MI) x (64 NJ) tile per workgroup of four waves
 //    (2 x 2, each (32 MI) x (32 NJ) in 32x32 products), K steps of 128 bytes per row through two
 //    LDS buffers, the next two steps' vectors in registers meanwhile; one barrier per step.  A row's
-//    eight 16-byte chunks sit at slot chunk ^ (row % 8), so operand reads of 32 rows meet no bank
-//    twice.  PAIR: the weight tile holds rows of a gate and an up matrix, 32 and 32, so that a
-//    wave's column tiles are (gate, up) of the same outputs and the gated unit is its epilogue.
+//    eight 16-byte chunks sit at slot chunk ^ (row / 2 % 8): the 16 rows of an operand read meet no
+//    bank of the 64 twice (chunk ^ (row % 8): half of the LDS cycles were conflicts; 2048x6912
+//    under 1004 rows 62.0 -> 58.2 us, pair of 6912x2048 80.1 -> 78.2).  PAIR: the weight tile holds
+//    rows of a gate and an up matrix, 32 and 32, so that a wave's column tiles are (gate, up) of the
+//    same outputs and the gated unit is its epilogue.
 //    GROUPED: the rows are one expert's (token, slot) pairs, from exo_moe_group's tile list.
 // Either may send its last output columns to a second, float32 buffer: inputs of 32-bit arithmetic
 // (step sizes, gates, decays) are rows of the same weight matrix as the bf16 projections.
@@ -386,12 +388,12 @@ __global__ __launch_bounds__(256, 2) void dense_gemm_kernel(const GemmParams p) 
 #pragma unroll
     for (int i = 0; i < XV; ++i) {
       const int id = tid + 256 * i, tr = id >> 3, c = id & 7;
-      *reinterpret_cast<uint4*>(xl + tr * 128 + ((c ^ (tr & 7)) << 4)) = x[i];
+      *reinterpret_cast<uint4*>(xl + tr * 128 + ((c ^ ((tr >> 1) & 7)) << 4)) = x[i];
     }
 #pragma unroll
     for (int i = 0; i < WV; ++i) {
       const int id = tid + 256 * i, tr = id >> 3, c = id & 7;
-      *reinterpret_cast<uint4*>(wl + tr * 128 + ((c ^ (tr & 7)) << 4)) = w[i];
+      *reinterpret_cast<uint4*>(wl + tr * 128 + ((c ^ ((tr >> 1) & 7)) << 4)) = w[i];
     }
   };
   const int frow = lane & 31, half = lane >> 5;
@@ -421,7 +423,7 @@ __global__ __launch_bounds__(256, 2) void dense_gemm_kernel(const GemmParams p) 
       const char* wl = lds + (s & 1) * BUF + (BM + wn + frow) * 128;
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        const int slot = ((2 * t + half) ^ (frow & 7)) << 4;
+        const int slot = ((2 * t + half) ^ ((frow >> 1) & 7)) << 4;
         uint4 a[MI], b[NJ];
 #pragma unroll
         for (int i = 0; i < MI; ++i) a[i] = *reinterpret_cast<const uint4*>(xl + i * 4096 + slot);
