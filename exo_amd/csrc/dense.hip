@@ -8,7 +8,11 @@
 //    wave is in flight before anything is waited for.  Range-checked loads stand in for every
 //    tail: rows past N, x rows past M and steps past a wave's range read as zero.  PAIR: a gate and
 //    an up matrix, the gated unit as epilogue.  DUAL: two products with nothing in common but the
-//    number of rows share the launch.
+//    number of rows share the launch.  Few columns under few rows: Q = 2 or 4 parts of K side by
+//    side in the product - A's 16 rows are 16 / Q weight rows times Q parts, B's 16 columns 16 / Q
+//    rows of x times Q parts; of the products of every part with every other the Q of equal parts
+//    count - so that a workgroup has 16 / Q columns and the launch Q times the workgroups: a CU
+//    takes no more than about 25 GB/s from memory, so 6.4 TB/s need all 256.
 //  * dense_gemm_kernel, any number of rows: a (64 MI) x (64 NJ) tile per workgroup of four waves
 //    (2 x 2, each (32 MI) x (32 NJ) in 32x32 products), K steps of 128 bytes per row through two
 //    LDS buffers, the next two steps' vectors in registers meanwhile; one barrier per step.  A row's
@@ -104,30 +108,33 @@ __device__ __forceinline__ floatx4 row4(const float* p, int c, int H, bool on, b
 
 // PP: float4 of a row per lane in front of the product (0: nothing there); NORMED: branches that are normed (0: one
 // that is added as it is)
-template <typename T, int NW, int PP, int NORMED, bool PAIR, bool DUAL>
+template <typename T, int NW, int PP, int NORMED, bool PAIR, bool DUAL, int Q = 1, int STEPS = kBatch>
 __global__ __launch_bounds__(64 * NW) void dense_gemv_kernel(const GemvParams p0, const GemvParams p1, const PostNorm q) {
   constexpr bool POST = PP > 0, TWO = NORMED == 2;
   constexpr int NP = POST ? PP : 1, NU = TWO ? NP : 1;
   constexpr int NM = PAIR ? 2 : 1;
-  constexpr int BATCH = PAIR ? kBatch / 2 : kBatch;
+  static_assert(Q == 1 || PP == 0, "parts of K side by side: plain products");
+  constexpr int R = 16 / Q;  // weight rows, and rows of x
+  constexpr int BATCH = PAIR ? STEPS / 2 : STEPS;
   __shared__ float red[NM][NW][256];
   __shared__ float part[2][NW];
   extern __shared__ __attribute__((aligned(16))) char xs[];  // POST: [M][ldx * sizeof(T) + 16]
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int r = lane & 15, g = lane >> 4;
-  const int tiles0 = (p0.N + 15) / 16;
+  const int tiles0 = (p0.N + R - 1) / R;
   const bool second = DUAL && (int)blockIdx.x >= tiles0;
   const GemvParams& p = second ? p1 : p0;
-  const int n0 = ((int)blockIdx.x - (second ? tiles0 : 0)) * 16, rows = min(16, p.N - n0);
+  const int n0 = ((int)blockIdx.x - (second ? tiles0 : 0)) * R, rows = min(R, p.N - n0);
   const uint32_t wrow = (uint32_t)p.ldw * sizeof(T), xrow = (uint32_t)p.ldx * sizeof(T);
-  const int steps = (int)(wrow >> 6);
+  const int steps = (int)(wrow >> 6) / Q;  // (rows are multiples of 128 or 256 bytes)
+  const uint32_t part_at = Q > 1 ? r / R * steps * 64 : 0;
   const int per = (steps + NW - 1) / NW, s0 = min(steps, wave * per), s1 = min(steps, s0 + per);
   const __amdgpu_buffer_rsrc_t rw =
       buf_of(reinterpret_cast<const char*>(p.w) + (size_t)n0 * wrow, (uint32_t)rows * wrow);
   const __amdgpu_buffer_rsrc_t ru =
       buf_of(reinterpret_cast<const char*>(PAIR ? p.w2 : p.w) + (size_t)n0 * wrow, (uint32_t)rows * wrow);
   const __amdgpu_buffer_rsrc_t rx = buf_of(p.x, (uint32_t)p.M * xrow);
-  const uint32_t woff = r * wrow + g * 16;
+  const uint32_t woff = r % R * wrow + part_at + g * 16;
   uint4 wv[NM][BATCH];
   auto load_w = [&](int s) {
 #pragma unroll
@@ -252,7 +259,7 @@ __global__ __launch_bounds__(64 * NW) void dense_gemv_kernel(const GemvParams p0
       if (POST)  // (steps past the range: any finite values, their weights are zero)
         xv[i] = *reinterpret_cast<const uint4*>(xs + min(r, p.M - 1) * (xrow + 16) + g * 16 + min(s + i, s1 - 1) * 64);
       else
-        xv[i] = buf_load16(rx, s + i < s1 ? r * xrow + g * 16 + (s + i) * 64 : kPastEnd, 0);
+        xv[i] = buf_load16(rx, s + i < s1 ? r % R * xrow + part_at + g * 16 + (s + i) * 64 : kPastEnd, 0);
     }
 #pragma unroll
     for (int i = 0; i < BATCH; ++i)
@@ -265,15 +272,18 @@ __global__ __launch_bounds__(64 * NW) void dense_gemv_kernel(const GemvParams p0
 #pragma unroll
     for (int e = 0; e < 4; ++e) red[k][wave][r * 16 + 4 * g + e] = acc[k][e];  // [m][n]
   __syncthreads();
-  for (int o = threadIdx.x; o < 16 * p.M; o += 64 * NW) {
-    const int m = o >> 4, n = o & 15;
+  for (int o = threadIdx.x; o < R * p.M; o += 64 * NW) {
+    const int m = o / R, n = o % R;
     if (n >= rows) continue;
     float v = 0.f, u = 0.f;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      v += red[0][w][o];
-      if (PAIR) u += red[NM - 1][w][o];
-    }
+    for (int w = 0; w < NW; ++w)
+#pragma unroll
+      for (int k = 0; k < Q; ++k) {
+        const int at = (k * R + m) * 16 + k * R + n;
+        v += red[0][w][at];
+        if (PAIR) u += red[NM - 1][w][at];
+      }
     if (PAIR) {
       store_out<T>(p.y, (size_t)m * p.ldy + n0 + n, clamped_glu(v, u, p.glu), p.y_f32);
       continue;
@@ -648,8 +658,45 @@ void launch_gemv_nw(const GemvParams& p, const GemvParams* p1, const PostNorm* q
   else
     dense_gemv_kernel<T, NW, 0, 0, false, false><<<tiles, 64 * NW, 0, st>>>(p, p, none);
 }
+// Parts of K side by side where 16 columns per workgroup leave CUs without work, as many rows of x as the
+// product then holds, and rows of whole parts.  One part -> these, us: N = 2048 (128 workgroups -> 256) under
+// 4 rows, bf16: K = 4096 8.0 -> 6.9, K = 6912 11.8 -> 9.1 (8 rows: 12.8 -> 9.8); N = 1024 (64 -> 256) under
+// 2 rows, f32: K = 1024 6.5 -> 4.2, K = 2560 11.0 -> 5.7.  Four parts at N = 2048 give no more than two (6.8, 9.8).
+// Single products of 144 workgroups still gain (6.0 -> 5.4); a pair reads two matrices per workgroup: 160
+// of K = 1024, f32, would lose (7.8 -> 8.1).  16 waves instead of 8: 7.4 and 8.7 in place of 6.9 and 9.1, f32 6.9
+// in place of 5.7.
+int gemv_parts(const GemvParams& p, const GemvParams* p1, int elem) {
+  const int tiles = exo_ceil_div(p.N, 16) + (p1 ? exo_ceil_div(p1->N, 16) : 0);
+  const int rows = p.ldw * elem | (p1 ? p1->ldw * elem : 0);
+  if (tiles <= 96 && p.M <= 4 && rows % 256 == 0) return 4;
+  return tiles < (p.w2 ? 160 : 192) && p.M <= 8 && rows % 128 == 0 ? 2 : 1;
+}
+template <typename T, bool PAIR, bool DUAL, int Q>
+void launch_gemv_parts(const GemvParams& p, const GemvParams* p1, hipStream_t st) {
+  const int tiles = exo_ceil_div(p.N, 16 / Q) + (DUAL ? exo_ceil_div(p1->N, 16 / Q) : 0);
+  const PostNorm none{};
+  // (half the requests at once where a wave's share of a part is no more: requests past it cost time as well)
+  const int ldw = DUAL && p1->ldw > p.ldw ? p1->ldw : p.ldw;
+  if (exo_ceil_div((int)((int64_t)ldw * sizeof(T) / 64) / Q, 8) <= (PAIR ? kBatch / 4 : kBatch / 2))
+    dense_gemv_kernel<T, 8, 0, 0, PAIR, DUAL, Q, kBatch / 2><<<tiles, 512, 0, st>>>(p, DUAL ? *p1 : p, none);
+  else
+    dense_gemv_kernel<T, 8, 0, 0, PAIR, DUAL, Q><<<tiles, 512, 0, st>>>(p, DUAL ? *p1 : p, none);
+}
 template <typename T>
 int launch_gemv(const GemvParams& p, const GemvParams* p1, const PostNorm* q, hipStream_t st) {
+  const int parts = q ? 1 : gemv_parts(p, p1, (int)sizeof(T));
+  if (parts > 1) {
+    exo_note_variant("dense_gemv<%s,8,plain,%s> M=%d N=%d parts=%d", sizeof(T) == 2 ? "bf16" : "f32",
+                     p1 ? "dual" : p.w2 ? "pair" : "single", p.M, p.N, parts);
+    const auto launch = parts == 4 ? p1     ? launch_gemv_parts<T, false, true, 4>
+                                     : p.w2 ? launch_gemv_parts<T, true, false, 4>
+                                            : launch_gemv_parts<T, false, false, 4>
+                        : p1       ? launch_gemv_parts<T, false, true, 2>
+                        : p.w2     ? launch_gemv_parts<T, true, false, 2>
+                                   : launch_gemv_parts<T, false, false, 2>;
+    launch(p, p1, st);
+    return EXO_OK;
+  }
   const int nw = gemv_waves(p.N + (p1 ? p1->N : 0));
   exo_note_variant("dense_gemv<%s,%d,%s,%s> M=%d N=%d", sizeof(T) == 2 ? "bf16" : "f32", nw, q ? "post" : "plain",
                    p1 ? "dual" : p.w2 ? "pair" : "single", p.M, p.N);

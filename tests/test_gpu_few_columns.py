@@ -1,0 +1,73 @@
+"""Products of few rows with few columns, whose parts of K lie side by side in one launch, against float64."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+if not torch.cuda.is_available():
+    pytest.skip("needs a GPU", allow_module_level=True)
+
+from exo_amd import dense_ops as D, native  # noqa: E402
+
+
+def check(got, x, w, bias=0.0):
+    """A sum of K products in float32, in any order: at most K roundings of 2^-24 of the sum of their sizes."""
+    x, w = x.double(), w.double()
+    want, size = x @ w.T + bias, x.abs() @ w.abs().T
+    bound = (x.shape[1] + 1) * 2.0**-24 * (size + abs(bias))
+    if got.dtype == torch.bfloat16:
+        bound = bound + 2.0**-8 * want.abs()
+    assert bool(((got.double() - want).abs() <= bound).all())
+
+
+# four parts: up to 4 rows, up to 96 x 16 columns; two: up to 8 rows, below 192 x 16; columns and rows that do
+# not fill a workgroup's, steps of K that do not fill its waves, as few as one for all of them
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,N,K,parts", [(1, 1, 128, 4), (4, 1536, 640, 4), (3, 130, 1920, 4), (4, 1537, 128, 2), (5, 97, 64, 2),
+                                         (8, 3055, 192, 2), (2, 2049, 2112, 2), (7, 1000, 7040, 2), (8, 3057, 128, 1),
+                                         (9, 40, 256, 1)])
+def test_parts_of_k(device, dtype, M, N, K, parts):
+    g = torch.Generator(device=device).manual_seed(M * N + K)
+    x, w = (torch.randn(n, K, device=device, generator=g).to(dtype) for n in (M, N))
+    b = torch.randn(N, device=device, generator=g)
+    out = torch.full((M + 1, N + 3), 7.0, dtype=dtype, device=device)  # (a row and columns past the result stay)
+    tail = min(3, N - 1)
+    t = torch.zeros(M, max(tail, 1), device=device)
+    D.linear(x, w, out, M, bias=b, tail=(t, tail) if tail else None)
+    label = native.last_variant()
+    assert ("parts=%d" % parts in label) if parts > 1 else ("dense_gemv" in label and "parts" not in label), label
+    check(out[:M, : N - tail], x, w[: N - tail], b[: N - tail].double())
+    if tail:
+        check(t, x, w[N - tail :], b[N - tail :].double())
+    assert bool((out[M:] == 7).all()) and bool((out[:, N:] == 7).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,N,K", [(1, 70, 128), (4, 1530, 896), (8, 2500, 192), (6, 2545, 320)])
+def test_gated_pair_and_two_products(device, dtype, M, N, K):
+    g = torch.Generator(device=device).manual_seed(M + N + K)
+    x, x2, gate, up = (torch.randn(n, K, device=device, generator=g).to(dtype) * (1 if n == M else K**-0.5) for n in (M, M, N, N))
+
+    class Plain:
+        limit, alpha, shift, cubic = float("inf"), 1.0, 0.0, 0.0
+
+    out = torch.zeros(M, N, dtype=torch.float32, device=device).to(dtype)
+    D.glu(x, gate, up, out, M, Plain)
+    assert "pair" in native.last_variant() and ("parts" in native.last_variant()) == (N <= 2544)
+    a, c = x.double() @ gate.double().T, x.double() @ up.double().T
+    want = a * torch.sigmoid(a) * c
+    # (silu's slope stays below 1.1 and it below |a|; the two sums' errors as above, the gate's own work 2^-20)
+    size_a, size_c = x.double().abs() @ gate.double().abs().T, x.double().abs() @ up.double().abs().T
+    bound = (K + 1) * 2.0**-24 * (1.1 * size_a * c.abs() + size_c * a.abs()) * 1.01 + 2.0**-20 * want.abs()
+    if dtype == torch.bfloat16:
+        bound = bound + 2.0**-8 * want.abs()
+    assert bool(((out.double() - want).abs() <= bound + 1e-12).all())
+
+    n0 = N // 3
+    y0, y1 = torch.zeros(M, n0, dtype=dtype, device=device), torch.zeros(M, N, dtype=torch.float32, device=device)
+    D.linear_pair(x, gate[:n0].contiguous(), y0, x2, up, y1, M)
+    assert "dual" in native.last_variant()
+    check(y0, x, gate[:n0])
+    check(y1, x2, up)
