@@ -105,6 +105,20 @@ __device__ __forceinline__ void load_to_lds16(__amdgpu_buffer_rsrc_t rsrc, void*
       rsrc, (__attribute__((address_space(3))) void*)lds_base, 16, voffset, soffset, 0, 0);
 }
 
+typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
+
+// The same, written as the instruction (it has no register result): the compiler makes the first LDS read
+// behind such a request wait for it, although it fills a tile that is read steps later, which a step of an expert's
+// few rows does not cover (pair of 768x2048 under 8184 pairs of 128 experts 113 -> 99 us, 2048x768 62.5 -> 58.5; the
+// 256-row tile, whose step does, 409 -> 421).  The waits are the caller's.
+__device__ __forceinline__ void load_to_lds16(u32x4 rsrc, void* lds_base, uint32_t voffset, uint32_t soffset) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               :
+               : "s"((uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds_base), "v"(voffset),
+                 "s"(rsrc), "s"(soffset)
+               : "memory");
+}
+
 // elements between the partial tiles of consecutive K ranges (16-byte aligned rows of 4)
 __host__ __device__ inline size_t part_stride(int M, int N) {
   return ((size_t)M * N + 3) / 4 * 4;
@@ -232,6 +246,9 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
   constexpr int XS_ROWS = WIDE ? 2 * BM : BM;  // (wide: room for the ring's four tiles)
   __shared__ __attribute__((aligned(16))) bf16_t xs[KH ? 2 * SLOTS : SLOTS][XS_ROWS * LDS_STRIDE];
 
+  // (a ring of four activation tiles: below)
+  constexpr bool RING = WIDE && SB4 && (BITS == 4 || kRing8) && (MI >= 4 || DEEP);
+
   const int tid = threadIdx.x & (kThreads - 1), lane = tid & 63;  // within the team
   const int team = KH ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8) : 0;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -290,6 +307,8 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
   // (pair mode: a second set of descriptors for the up matrix, column tile 1)
   constexpr int ND = PAIR ? 2 : 1;
   const __amdgpu_buffer_rsrc_t rx = make_rsrc(p.x);
+  const u32x4 rx4 = {(uint32_t)__builtin_amdgcn_readfirstlane((int)(uintptr_t)p.x),
+                     (uint32_t)__builtin_amdgcn_readfirstlane((int)((uintptr_t)p.x >> 32)) & 0xffffu, ~0u, 0x00020000u};
   __amdgpu_buffer_rsrc_t rw[ND], rs[ND], rb[ND];
   rw[0] = make_rsrc(wbase);
   rs[0] = make_rsrc(sbase);
@@ -326,8 +345,13 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
   char* const tiles = reinterpret_cast<char*>(&xs[0][0]) + team * ((KH && WIDE ? 4 : SLOTS) * TILE_BYTES);
   auto load_x = [&](int buf, int k0, int n) {
 #pragma unroll
-    for (int r = 0; r < n; ++r)
-      load_to_lds16(rx, tiles + buf * TILE_BYTES + (wave * 64 + kThreads * r) * 16, xoff[r], k0 * 2);
+    for (int r = 0; r < n; ++r) {
+      char* const to = tiles + buf * TILE_BYTES + (wave * 64 + kThreads * r) * 16;
+      if constexpr (RING && GROUPED)
+        load_to_lds16(rx4, to, xoff[r], k0 * 2);
+      else
+        load_to_lds16(rx, to, xoff[r], k0 * 2);
+    }
   };
   // s_waitcnt vmcnt(n) alone (the other counters at "no wait")
   auto wait_vm = [](auto n) {
@@ -591,7 +615,6 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
   // (past the end of K the last step again, never multiplied) and the loop body is four steps
   // long with static stage indices, so that the wait at the end of a step is an exact count:
   // the two youngest steps' requests may still be out.
-  constexpr bool RING = WIDE && SB4 && (BITS == 4 || kRing8) && (MI >= 4 || DEEP);
   // (8-bit: two steps ahead - three live stages of 16 registers; four spill)
   constexpr int AHEAD = BITS == 4 ? 3 : 2;
   static_assert(RING || !(WIDE && DEEP), "a wide tile with the pipeline flag runs the ring");
@@ -602,11 +625,11 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
     SBlock sbc, sbn;
     const int last = ke - BK;
     load_sb(sbn, kb >> 8);
+    constexpr int XAHEAD = GROUPED ? 3 : AHEAD;
 #pragma unroll
-    for (int u = 0; u < AHEAD; ++u) {
-      load_x(u, min(kb + u * BK, last), NI);
-      load_w(wq[u], min(kb + u * BK, last));
-    }
+    for (int u = 0; u < AHEAD; ++u) load_w(wq[u], min(kb + u * BK, last));
+#pragma unroll
+    for (int u = 0; u < XAHEAD; ++u) load_x(u, min(kb + u * BK, last), NI);
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
     __syncthreads();
     read_first(ni, wq[0], 0, sbn, 0);
@@ -616,10 +639,14 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const int kn = min(k0 + (u + AHEAD) * BK, last);
-        load_x((u + AHEAD) & 3, kn, NI);
+        // (the compiler's own wait for the weights of a step counts weights alone: with the activations
+        // behind them it leaves four of the youngest out, before them none)
+        if (!GROUPED) load_x((u + XAHEAD) & 3, min(k0 + (u + XAHEAD) * BK, last), NI);
         load_w(wq[(u + AHEAD) & 3], kn);
+        if (GROUPED) load_x((u + XAHEAD) & 3, min(k0 + (u + XAHEAD) * BK, last), NI);
         multiply_on(ni, wq[u], wq[(u + 1) & 3], u, (u + 1) & 3, sbc, u, u < 3 ? sbc : sbn, (u + 1) & 3);
-        wait_vm(std::integral_constant<int, (AHEAD - 1) * (NI + NW)>{});
+        // tile k+2 is in LDS behind the barrier: the next step's last products read its first operands
+        wait_vm(std::integral_constant<int, GROUPED ? NI + NW : (AHEAD - 2) * (NI + NW) + NW>{});
         __syncthreads();
       }
     }

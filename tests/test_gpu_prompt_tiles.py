@@ -64,12 +64,13 @@ def test_prompt_pair_gemm_at_tile_edges(device, M, N, K, bits):
 
 
 @pytest.mark.parametrize("rows", [1, 32, 33, 64, 65, 96, 97, 128, 129])
-def test_grouped_gemm_multiplies_the_rows_of_its_tile(device, rows):
+@pytest.mark.parametrize("K,bits", [(256, 4), (1280, 4), (256, 8), (1536, 8)])
+def test_grouped_gemm_multiplies_the_rows_of_its_tile(device, rows, K, bits):
     """Experts of 1 to 129 rows beside an empty one: a tile multiplies only the blocks of 32 rows that it has."""
-    E, K, N = 4, 256, 264
-    qs = [packed(N, K, 4, e, device) for e in range(E)]
+    E, N = 4, 264
+    qs = [packed(N, K, bits, e, device) for e in range(E)]
     q = QuantizedWeight(torch.stack([t.weight for t in qs]), torch.stack([t.scales for t in qs]),
-                        torch.stack([t.biases for t in qs]), 4)
+                        torch.stack([t.biases for t in qs]), bits)
     idx = torch.cat([torch.full((rows,), 2), torch.full((40,), 0), torch.full((3,), 3)]).to(torch.int32).to(device)[:, None].contiguous()
     T = idx.shape[0]
     x = torch.randn(T, 1, K, device=device, generator=torch.Generator(device=device).manual_seed(rows)).bfloat16()
