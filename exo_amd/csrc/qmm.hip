@@ -33,20 +33,10 @@
 //    under 2047 rows 451 -> 420.  What bounds it: the matrix cores are busy 56 % of the
 //    cycles; 20 % go into the wait for the tile requested a step ahead and the barrier, the rest
 //    into slots with more vector work than an MFMA covers.
-//  * up to 128 rows and few column tiles: blockIdx.z splits K; float32 partial tiles and a
-//    small reduce launch.
-//  * up to 32 rows (64 on matrices of 8192 rows or more): the four waves sit side by side on
-//    a (32 or 64) x 256 tile, so no weight row is dequantised twice, and K is split until the
-//    launch has up to two workgroups per CU (14336x4096 4-bit at 32 rows: 31 -> 21 us,
-//    4096x14336: 32.5 -> 23 us; at 96 rows and more the 128-row tile is level or faster).
-//    Where that launch's time goes (14336x4096 4-bit, 32 rows, 22 us with the reduce launch):
-//    the weights alone, requested as they are, take 10 us (what the one-row GEMV takes for the
-//    same matrix); the dequantisation and products add 5 us that do not overlap (all
-//    workgroups run in step: one round of 448 workgroups, two K ranges of loads each); the
-//    float32 partial tiles 3.4 us to store and 4 us to reduce; the activation tiles 1 us.
-//    Requesting the weights as whole 128-byte lines (8 rows x 128 B per wave instruction
-//    instead of 32 rows x 32 B) gained 8 %, re-reading one weight block from L2 nothing, a ring
-//    of eight register stages nothing, four K steps per barrier nothing: none was kept.
+//  * few output tiles: blockIdx.z splits K; float32 partial tiles and a small reduce launch.
+//  * 17 to 64 rows belong to qmm_short.hip (K up to 32768).  Up to 16 rows that the GEMVs do not take, and up
+//    to 32 beyond that K: the four waves side by side on a 32 x 256 tile, so no weight row is
+//    dequantised twice, and K split until the launch has up to two workgroups per CU.
 #include "../../include/exo_mi355x.h"
 #include "common.h"
 #include "dequant.h"
@@ -167,8 +157,8 @@ __device__ __forceinline__ uint32_t dequant_piece(uint32_t lo, uint32_t hi, floa
 // of the up matrix - a wave's two column tiles are (gate, up) of the same 32 output columns,
 // so the SwiGLU happens in the epilogue and neither projection is written to memory.
 // WIDE: the four waves sit side by side - the workgroup tile is (32*MI) x 256 weight rows,
-// every wave owns 64 of them, so nothing is dequantised twice.  Plain GEMM (inputs of up to
-// 64 rows): blockIdx.z always owns a K range and the tile leaves as a float32 partial.
+// every wave owns 64 of them, so nothing is dequantised twice.  Plain GEMM of up to
+// 32 rows: blockIdx.z always owns a K range and the tile leaves as a float32 partial.
 // Grouped GEMM (MI = 4: the expert's 128-row tile against 256 weight rows, the wave tile of
 // the 256-row kernel): whole K, the usual epilogue.  The same tile for the plain (gate, up)
 // pair of a long input: per product it stages half the activation bytes of the 256 x 64 tile
@@ -231,7 +221,7 @@ template <int BITS, int MI, bool GROUPED = false, bool SB4 = false, bool PAIR = 
 __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_kernel(const QmmParams p) {
   static_assert(!WIDE || GROUPED || !PAIR || MI >= 4, "the wide pair tile has 128 or 256 rows");
   static_assert(!DEEP || (SB4 && ((MI == 2 && !WIDE) || (WIDE && MI < 4))),
-                "the deep pipeline is for 128-row tiles; on the 32- and 64-row wide tiles the flag "
+                "the deep pipeline is for 128-row tiles; on the 32-row wide tile the flag "
                 "selects the ring (K ranges long enough to fill it)");
   static_assert(!KH || (MI == 4 && SB4 && !GROUPED && !DEEP && !(WIDE && PAIR)),
                 "two K halves per workgroup: the 256-row tile of the plain and the pair GEMM, "
@@ -990,7 +980,7 @@ int wide_max_split(int N) {
 }
 
 bool plan_wide(int M, int N, int K, const QmmParams& p, bool have_ws, int* ksplit, int* kc) {
-  if (!have_ws || M > 64 || (M > 32 && N < 8192) || N > kQmmWideMaxN || K % 256 != 0) return false;
+  if (!have_ws || M > 32 || N > kQmmWideMaxN || K % 256 != 0) return false;
   if ((((uintptr_t)p.s | (uintptr_t)p.b) & 7) != 0) return false;
   const int cap = wide_max_split(N);
   int ks = 1;
@@ -1045,14 +1035,10 @@ void launch_qmm(const QmmParams& p, hipStream_t st) {
     // K ranges of twelve steps or more fill the ring (4096x14336 4-bit at 17 rows 22.3 -> 19.3
     // us); on short ranges its start-up costs more than it returns (14336x4096: 20.5 -> 21.4)
     const bool ring = p.kc >= kWideRingMinK;
-    if (M <= 32 && ring)
+    if (ring)
       exo_note_variant("qmm_kernel<%d, 1, false, true, false, true, true>", BITS), qmm_kernel<BITS, 1, false, true, false, true, true><<<g, 256, 0, st>>>(p);
-    else if (M <= 32)
-      exo_note_variant("qmm_kernel<%d, 1, false, true, false, true>", BITS), qmm_kernel<BITS, 1, false, true, false, true><<<g, 256, 0, st>>>(p);
-    else if (ring)
-      exo_note_variant("qmm_kernel<%d, 2, false, true, false, true, true>", BITS), qmm_kernel<BITS, 2, false, true, false, true, true><<<g, 256, 0, st>>>(p);
     else
-      exo_note_variant("qmm_kernel<%d, 2, false, true, false, true>", BITS), qmm_kernel<BITS, 2, false, true, false, true><<<g, 256, 0, st>>>(p);
+      exo_note_variant("qmm_kernel<%d, 1, false, true, false, true>", BITS), qmm_kernel<BITS, 1, false, true, false, true><<<g, 256, 0, st>>>(p);
     reduce_parts(p.part, p.residual, p.y, M, N, p.ksplit, st);
     return;
   }
