@@ -448,20 +448,23 @@ __global__ __launch_bounds__(256, 2) void dense_gemm_kernel(const GemmParams p) 
   }
 
   // ---- epilogue: element e of tile (i, j): row wm + 32 i + 8 (e / 4) + 4 half + e % 4, column lane
-  // One plain output, or a partial one: every store at 32-bit offsets from the tile's first row, rows past
-  // the end dropped by the buffer's range, columns past N by an offset beyond it.  (The whole offset is in
-  // the vector register: the scalar one takes no part in the range check.)
-  if (!GROUPED && !PAIR && (p.ksplit > 1 || (p.n1 == p.N && !p.ep.mul))) {
+  // One plain output (its last columns may go to the float32 buffer), or a partial one: every store at 32-bit
+  // offsets from the tile's first row, rows past the end dropped by the buffer's range, columns of the other
+  // buffer and past N by an offset beyond it.  (The whole offset is in the vector register: the scalar one takes
+  // no part in the range check.)  Element by element, as in the loop at the end, 13664 columns of K = 2048 with
+  // 96 in the second buffer under 1004 rows took 108 us, here 78; 6208 columns 52.5, here 38.
+  if (!GROUPED && !PAIR && (p.ksplit > 1 || (!p.ep.mul && (p.n1 == p.N || p.ldy2 < 1 << 22)))) {
     const bool part = p.ksplit > 1, f32 = part || p.y_f32 || sizeof(T) == 4;
     const uint32_t ld = part ? (uint32_t)p.N : (uint32_t)p.ldy, size = f32 ? 4 : 2;
+    const int n1 = part ? p.N : p.n1, held = min(m_end - m0, BM);
     char* base = part ? reinterpret_cast<char*>(p.part + ((size_t)blockIdx.z * p.M + m0) * p.N)
                       : reinterpret_cast<char*>(p.y) + (size_t)m0 * ld * size;
-    const __amdgpu_buffer_rsrc_t ry = buf_of(base, (uint32_t)min(m_end - m0, BM) * ld * size);
-    uint32_t voff[NJ];
+    const __amdgpu_buffer_rsrc_t ry = buf_of(base, (uint32_t)held * ld * size);
+    const uint32_t ld2 = n1 < p.N ? (uint32_t)p.ldy2 : 0;
+    const __amdgpu_buffer_rsrc_t ry2 = buf_of(p.y2 + (size_t)m0 * ld2, (uint32_t)held * ld2 * 4);
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
-      const int n = n0 + wn + 32 * j + frow;
-      voff[j] = n < p.N ? ((uint32_t)(wm + 4 * half) * ld + n) * size : kPastEnd;
+      const int c0 = n0 + wn + 32 * j, n = c0 + frow;
       if (!part && p.bias) {
         const float b = n < p.N ? p.bias[n] : 0.f;
 #pragma unroll
@@ -469,29 +472,33 @@ __global__ __launch_bounds__(256, 2) void dense_gemm_kernel(const GemmParams p) 
 #pragma unroll
           for (int e = 0; e < 16; ++e) acc[i][j][e] += b;
       }
-    }
-    if (!part && p.ep.act) {
+      auto store = [&](uint32_t voff, uint32_t row_bytes, auto put) __attribute__((always_inline)) {
 #pragma unroll
-      for (int i = 0; i < MI; ++i)
+        for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < NJ; ++j)
+          for (int e = 0; e < 16; ++e) put(acc[i][j][e], voff + (uint32_t)(32 * i + 8 * (e >> 2) + (e & 3)) * row_bytes);
+      };
+      auto put32 = [](const __amdgpu_buffer_rsrc_t& to, float v, uint32_t at) __attribute__((always_inline)) {
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), to, at, 0, 0);
+      };
+      if (c0 + 32 > n1 && n1 < p.N)  // (uniform)
+        store(n >= n1 && n < p.N ? ((uint32_t)(wm + 4 * half) * ld2 + (n - n1)) * 4 : kPastEnd, ld2 * 4,
+              [&](float v, uint32_t at) __attribute__((always_inline)) { put32(ry2, v, at); });
+      if (c0 >= n1) continue;
+      if (!part && p.ep.act) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
 #pragma unroll
           for (int e = 0; e < 16; ++e) acc[i][j][e] = activated(acc[i][j][e], p.ep.act, p.ep.cap);
+      }
+      const uint32_t voff = n < n1 ? ((uint32_t)(wm + 4 * half) * ld + n) * size : kPastEnd;
+      if (f32)
+        store(voff, ld * size, [&](float v, uint32_t at) __attribute__((always_inline)) { put32(ry, v, at); });
+      else
+        store(voff, ld * size, [&](float v, uint32_t at) __attribute__((always_inline)) {
+          __builtin_amdgcn_raw_buffer_store_b16(f2bf(v), ry, at, 0, 0);
+        });
     }
-    auto store = [&](auto put) __attribute__((always_inline)) {
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const uint32_t roff = (uint32_t)(32 * i + 8 * (e >> 2) + (e & 3)) * ld * size;
-#pragma unroll
-          for (int j = 0; j < NJ; ++j) put(acc[i][j][e], voff[j] + roff);
-        }
-    };
-    if (f32)
-      store([&](float v, uint32_t at) { __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), ry, at, 0, 0); });
-    else
-      store([&](float v, uint32_t at) { __builtin_amdgcn_raw_buffer_store_b16(f2bf(v), ry, at, 0, 0); });
     return;
   }
   // Gated pairs and an expert's rows, in the element type: the same with a row's offset from the list of

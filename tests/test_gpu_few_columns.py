@@ -71,3 +71,20 @@ def test_gated_pair_and_two_products(device, dtype, M, N, K):
     assert "dual" in native.last_variant()
     check(y0, x, gate[:n0])
     check(y1, x2, up)
+
+
+# the last columns of a GEMM of many rows in their float32 buffer: a whole block of 32 columns, part of one, none of
+# the first buffer's block; rows that do not fill a tile
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,N,n1", [(17, 300, 256), (64, 300, 250), (65, 4100, 4000), (1000, 3300, 3232), (1000, 3300, 31), (770, 4097, 4096)])
+def test_last_columns_of_a_gemm(device, dtype, M, N, n1):
+    K = 128
+    g = torch.Generator(device=device).manual_seed(M + N)
+    x, w = torch.randn(M, K, device=device, generator=g).to(dtype), (torch.randn(N, K, device=device, generator=g) / 8).to(dtype)
+    b = torch.randn(N, device=device, generator=g)
+    out = torch.full((M + 1, n1 + 5), 7.0, dtype=dtype, device=device)
+    t = torch.full((M + 1, N - n1 + 2), 7.0, device=device)
+    D.linear(x, w, out, M, bias=b, tail=(t, N - n1))
+    check(t[:M, : N - n1], x, w[n1:], b[n1:].double())
+    check(out[:M, :n1], x, w[:n1], b[:n1].double())
+    assert bool((out[M:] == 7).all()) and bool((out[:, n1:] == 7).all()) and bool((t[M:] == 7).all()) and bool((t[:, N - n1 :] == 7).all())
