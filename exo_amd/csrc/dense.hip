@@ -607,10 +607,17 @@ int launch_plain(GemmParams p, int64_t ws_floats, hipStream_t st) {
   p.ksteps = steps;
   const int64_t t2 = (int64_t)cols * exo_ceil_div(p.M, 128), t1 = (int64_t)cols * exo_ceil_div(p.M, 64);
   const bool tall = p.M > 64 && t2 >= 192;
-  if (!PAIR && p.part) {  // few tiles: split K until the chip has about one workgroup per CU
+  // Few tiles: split K until the chip has about one workgroup per CU, and on long ranges of K two, which wait for
+  // different loads: 24 steps where some CUs have none yet, 48 where each has one (2048 columns, bf16, us: 300 rows
+  // of K = 6912, 160 -> 320 workgroups 32.9 -> 28.2; 700 rows 176 -> 352 53.6 -> 46.8; 1004 rows 256 -> 512 56.9 -> 51.6, but of
+  // K = 4096, ranges of 32 steps, 34.8 -> 35.6; tall tiles lose, 2000 rows 78.9 -> 83.1).
+  if (!PAIR && p.part) {
     const int64_t tiles = tall ? t2 : t1;
     int ks = 1;
-    while (ks < 16 && tiles * ks * 2 <= 256 && steps / (ks * 2) >= 4) ks *= 2;
+    auto more = [&](int64_t wgs, int range) {
+      return wgs * 2 <= 256 ? range >= 4 : !tall && wgs * 2 <= 512 && range >= (wgs <= 192 ? 24 : 48);
+    };
+    while (ks < 16 && more(tiles * ks, steps / (ks * 2))) ks *= 2;
     while (ks > 1 && (int64_t)ks * p.M * p.N > ws_floats) ks /= 2;
     if (ks > 1) {
       p.ksteps = exo_ceil_div(steps, ks);

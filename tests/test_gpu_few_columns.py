@@ -88,3 +88,14 @@ def test_last_columns_of_a_gemm(device, dtype, M, N, n1):
     check(t[:M, : N - n1], x, w[n1:], b[n1:].double())
     check(out[:M, :n1], x, w[:n1], b[:n1].double())
     assert bool((out[M:] == 7).all()) and bool((out[:, n1:] == 7).all()) and bool((t[M:] == 7).all()) and bool((t[:, N - n1 :] == 7).all())
+
+
+# K split over two workgroups per CU: from 24 steps of 64 per range where CUs are left over, from 48 where none is
+@pytest.mark.parametrize("M,N,K,split", [(300, 2040, 6912, 4), (300, 2040, 5952, 2), (1000, 2048, 6144, 2), (1000, 2048, 6080, 1), (700, 2048, 3136, 2)])
+def test_long_ranges_of_k(device, M, N, K, split):
+    g = torch.Generator(device=device).manual_seed(K)
+    x, w = (torch.randn(n, K, device=device, generator=g).bfloat16() for n in (M, N))
+    out = torch.zeros(M, N, device=device)
+    D.linear(x, w, out, M)
+    assert native.last_variant().endswith("x%d" % split), native.last_variant()
+    check(out, x, w)
