@@ -47,3 +47,31 @@ def test_decode_attention_around_the_first_split(device, Hq, Hkv, D, S, lens):
                 slack = 2.0**-6 * (w @ vv.abs()) + 2.0**-8 * want.abs() + 1e-5
                 assert ((got - want).abs() <= slack).all(), f"sequence {b} of {n} keys, head {h}"
         assert not ws[: 4 * B * Hkv].view(torch.int32)[: B * Hkv].any()
+
+
+# the launch is laid out for more keys than the rows hold: splits without a tile of 32 keys (four to a split) leave the
+# merge to the others, down to one that writes the result itself; rows of one launch differ, a second launch
+# finds the counters as the first left them
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T,last,window,keep", [(700, [699, 128, 0], None, 0), (700, [127, 255, 256], None, 0), (600, [599, 300, 31], 100, 40)])
+def test_paged_rows_with_idle_splits(device, dtype, T, last, window, keep):
+    from exo_amd import dense_ops as D
+    from exo_amd.paged_cache import PagedKVCache
+    from tests import test_gpu_gekazen as G
+    from tests.stack_util import TOL, close, host
+
+    spec = G.make_spec(8, 2, 64, 64, window, keep)
+    rows = torch.randn(T, (8 + 2 * 2) * 64, generator=torch.Generator().manual_seed(T)).numpy()
+    cache = PagedKVCache([(2, 64, 64)], 3, 2048, "cuda", dtype)
+    att = D.PagedAttention(spec, torch.tensor(spec.slopes, dtype=torch.float32, device=device), 0, cache, 1e-6)
+    qkv = torch.tensor(rows, device=device).to(dtype)
+    held = qkv.float().cpu().numpy().reshape(T, 12, 64)
+    i32 = dict(dtype=torch.int32, device=device)
+    cache.reserve([1], T)
+    att.append(qkv, torch.full((T,), 1, **i32), torch.arange(T, **i32), T)
+    want = G.attn_oracle(spec, (held[:, :8], held[:, 8:10], held[:, 10:]), 1e-6, dtype)
+    part, out = qkv[last].contiguous(), torch.zeros(len(last), 512, dtype=dtype, device=device)
+    for keys in (2000, T, 2000):
+        out.zero_()
+        att.rows(part, out, torch.full((len(last),), 1, **i32), torch.tensor(last, **i32), len(last), keys, append=False)
+        close(host(out).reshape(len(last), 8, 64), want[last], 3 * TOL[dtype], f"{keys} keys allowed for")
