@@ -19,10 +19,9 @@
 // for its 32 weights per lane (each a multiply-add, a power at a quarter of the rate, a sum, half a
 // rounding and half a maximum).  So the two are written into each other: a wave multiplies the NEXT
 // tile's scores between this tile's weights, and takes the next scores' maxima between this
-// tile's V products; what rescaled the output for every tile runs only when a maximum has moved
-// by more than a factor of 2^8.  32 / 8 heads of 128, 4096 tokens behind 12288: 1212 -> 868 us (1108
-// TFLOP/s), 2047 tokens 76 -> 50 us, 4096 behind 4096 with heads of 64 398 -> 254 us.  (Without the
-// interleaving 1061, 63 and 303 us.)
+// tile's V products; the output is rescaled only where some query of the wave has a new maximum.
+// 32 / 8 heads of 128, 4096 tokens behind 12288: 1230 -> 935 us (1029 TFLOP/s), 2047 tokens 67 -> 49 us,
+// 4096 behind 12288 with heads of 64 807 -> 580 us.
 //
 // SPLIT (launches of at most one workgroup per CU, i.e. prompts of about a thousand tokens):
 // eight waves, two teams of four that take the first and the second half of the
@@ -38,7 +37,6 @@ namespace {
 
 constexpr int kBN = 64;   // keys per tile
 constexpr int kBM = 32;   // query tokens per wave
-constexpr float kSlack = 8.f;  // see the online softmax
 
 struct FaParams {
   const bf16_t* q;    // [B*T, Hq*D] (already rotated)
@@ -46,8 +44,8 @@ struct FaParams {
   const bf16_t* v;
   const int32_t* pos;  // [B] tokens in the cache before this chunk
   bf16_t* out;         // [B*T, Hq*D]
-  float scale_log2e, slack;  // > 0 (a negative scale is in q_sign); kSlack as a difference of scores
-  uint32_t q_sign;           // flips the queries of a negative scale
+  float scale_log2e;  // > 0 (a negative scale is in q_sign)
+  uint32_t q_sign;    // flips the queries of a negative scale
   int T, Hq, Hkv, S_max, G, units;  // units = token tiles * G
 };
 
@@ -187,8 +185,8 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, SPLIT ? 1 : 2) void fa_prefill_k
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
     for (int e = 0; e < 16; ++e) o[dt][e] = 0.f;
-  // maximum that the weights refer to, the same scaled, the score at which it moves; this half's sums
-  float m_run = -INFINITY, m_ref = 0.f, m_lim = -INFINITY, l0 = 0.f, l1 = 0.f;
+  // running maximum, the same scaled; this half's sums
+  float m_run = -INFINITY, m_ref = 0.f, l0 = 0.f, l1 = 0.f;
 
   auto read_k = [&](lds_char tile, int slot) {  // operand of product `slot` of S^T: step slot / 2, sub-tile slot % 2
     return *reinterpret_cast<__attribute__((address_space(3))) const u32x4*>(
@@ -211,11 +209,12 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, SPLIT ? 1 : 2) void fa_prefill_k
           if (ks * 32 + 16 * (e >> 3) + 8 * kq + (e & 7) > vis) s[ks][e] = -INFINITY;
     }
   };
-  // The reference point m_run moves only when some score lies more than kSlack (in powers of
-  // two) above it: weights up to 2^kSlack are as exact in bf16 and float32 as ones up to 1, and
-  // the rescaling - and the exchange between the halves of a query - is left out otherwise.
+  // The rescaling, and the exchange between the halves of a query, is left out where no query of the wave
+  // has a new maximum.  The weights refer to the maximum itself: the largest is 1, which bf16 holds.  (Left
+  // behind until a score lay 2^8 above it, the largest weight was rounded while its sum was not:
+  // error 2.2e-3 -> 2.35e-3 under scores of unit width, 1.9e-3 -> 2.4e-3 under twice that.)
   auto settle = [&](float mx) {
-    if (__builtin_amdgcn_ballot_w64(mx > m_lim) == 0) return;  // (at the first tile: -infinity)
+    if (__builtin_amdgcn_ballot_w64(mx > m_run) == 0) return;  // (at the first tile: -infinity)
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
     const float m_new = fmaxf(m_run, mx);
     // (a query that has seen no key yet keeps -infinity as its maximum and 0 as its reference)
@@ -229,7 +228,6 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, SPLIT ? 1 : 2) void fa_prefill_k
       for (int e = 0; e < 16; ++e) o[dt][e] *= alpha;
     m_run = m_new;
     m_ref = ref;
-    m_lim = m_new + p.slack;
   };
   constexpr int AHEAD = 3;  // operands in flight from LDS
 
@@ -396,7 +394,6 @@ int exo_sdpa_prefill_mfma(const bf16_t* q, const bf16_t* k_cache, const bf16_t* 
   p.out = out;
   // (a scale of zero: one that rounds every score to zero, so that masked ones stay minus infinity)
   p.scale_log2e = fmaxf(fabsf(scale) * 1.4426950408889634f, 1e-30f);
-  p.slack = kSlack / p.scale_log2e;
   p.q_sign = scale < 0.f ? 0x80008000u : 0u;
   p.T = T;
   p.Hq = Hq;

@@ -3,6 +3,8 @@ weights as the kernel forms them (scale * code + bias, rounded to bf16 once)."""
 
 from __future__ import annotations
 
+import math
+
 import pytest
 import torch
 
@@ -109,6 +111,28 @@ def test_prompt_attention_at_tile_edges(device, T, past, Hq, Hkv, D, spare, scal
             slack = 2.0**-8 * (w @ vv.abs()) + 1e-5
             bad = (out.view(B, T, Hq, D)[b, :, h].double() - want).abs() > slack + 2.0**-8 * want.abs()
             assert not bad.any(), f"sequence {b} head {h}: {int(bad.sum())} outputs, first at {bad.nonzero()[0].tolist()}"
+
+
+@pytest.mark.parametrize("T,D", [(64, 64), (64, 128), (300, 64), (300, 128)])  # (300: the keys of a workgroup in two halves)
+def test_prompt_attention_weighs_the_largest_score_with_one(device, T, D):
+    """Two keys count, of the same value row: one in the first tile, weight 1, one in the second, weight 2^a (0 < a < 8).
+    The larger one's weight is 1 by the time it is rounded to bf16, and the other's share of the sum, at most 1/2, was exact when
+    it was: the result is that row.  A weight of 2^a itself is off by up to 2^-8 and the row's elements by half a step or more."""
+    Hq, Hkv, past = 4, 2, 128
+    g = torch.Generator(device=device).manual_seed(T)
+    a = torch.rand(T, Hq, device=device, generator=g).mul(7.8).add(0.1).bfloat16()
+    q = torch.zeros(T, Hq, D, device=device, dtype=torch.bfloat16)
+    q[..., 0], q[..., 1] = a, 1
+    k = torch.zeros(1, Hkv, past + T, D, device=device, dtype=torch.bfloat16)
+    k[..., 1] = -100  # weight 2^-100
+    k[:, :, 3] = 0
+    k[:, :, 70, 0], k[:, :, 70, 1] = 1, 0
+    row = (2 - torch.randint(1, 33, (D,), device=device, generator=g) / 128).bfloat16()  # (bf16 steps of 1/128, values near 2)
+    v = row.expand(1, Hkv, past + T, D).contiguous()
+    out = torch.empty(T, Hq * D, device=device, dtype=torch.bfloat16)
+    ops.sdpa_prefill(q.view(T, -1), k, v, torch.tensor([past], dtype=torch.int32, device=device), out, math.log(2.0), 1, T, Hq, Hkv, D)
+    bad = out.view(T, Hq, D) != row
+    assert not bad.any(), f"{int(bad.any(-1).sum())} of {T * Hq} queries"
 
 
 # 17 to 64 rows: both sizes of the row tile, a step count below, at and above the eight waves, rows of scales that are no
