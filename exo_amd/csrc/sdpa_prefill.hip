@@ -392,8 +392,10 @@ int exo_sdpa_prefill_mfma(const bf16_t* q, const bf16_t* k_cache, const bf16_t* 
   p.v = v_cache;
   p.pos = pos;
   p.out = out;
-  // (a scale of zero: one that rounds every score to zero, so that masked ones stay minus infinity)
-  p.scale_log2e = fmaxf(fabsf(scale) * 1.4426950408889634f, 1e-30f);
+  // (a scale of zero: one that rounds every score to zero, so that masked ones stay minus infinity; not fmaxf,
+  // which would make a number of NaN)
+  p.scale_log2e = fabsf(scale) * 1.4426950408889634f;
+  if (p.scale_log2e < 1e-30f) p.scale_log2e = 1e-30f;
   p.q_sign = scale < 0.f ? 0x80008000u : 0u;
   p.T = T;
   p.Hq = Hq;

@@ -135,6 +135,16 @@ def test_prompt_attention_weighs_the_largest_score_with_one(device, T, D):
     assert not bad.any(), f"{int(bad.any(-1).sum())} of {T * Hq} queries"
 
 
+@pytest.mark.parametrize("T", [20, 300])
+def test_prompt_attention_with_a_scale_of_nan_is_nan(device, T):
+    g = torch.Generator(device=device).manual_seed(T)
+    q, k, v = (torch.randn(1, 4, T, 64, device=device, generator=g).bfloat16() for _ in range(3))
+    out = torch.zeros(T, 4 * 64, device=device, dtype=torch.bfloat16)
+    pos = torch.zeros(1, dtype=torch.int32, device=device)
+    ops.sdpa_prefill(q.transpose(1, 2).reshape(T, -1).contiguous(), k, v, pos, out, float("nan"), 1, T, 4, 4, 64)
+    assert out.isnan().all()
+
+
 # 17 to 64 rows: both sizes of the row tile, a step count below, at and above the eight waves, rows of scales that are no
 # whole 16-byte pieces (K of 64, 192, 832), one to seven column tiles per workgroup, K in four parts, ragged columns
 @pytest.mark.parametrize("M,N,K,bits", [(17, 4096, 64, 4), (32, 264, 192, 8), (33, 4099, 832, 4), (64, 12290, 512, 4),
