@@ -299,10 +299,14 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, SPLIT ? 1 : 2) void fa_prefill_k
     if (kt + 1 < n_tiles) settle(mx);
   };
 
+  // A context of one tile (prompts of up to 64 tokens) has nothing to be written into each other: no second K
+  // tile, no next scores, no barriers of the loop (61 tokens, 32 / 8 heads of 128: 7.4 -> 6.5 us, of 64 5.4 -> 4.5;
+  // plain tiles without the interleaving 6.6 and 5.0)
+  const bool one_tile = !SPLIT && n_all == 1;
   const int n_mine = last_w / kBN + 1 - t_first;  // tiles that this wave's rows see (<= 0: none)
   load_tile(rk, koff, 0, 0);
   load_tile(rv, voff, 2, 0);
-  load_tile(rk, koff, 1, 1);
+  if (!one_tile) load_tile(rk, koff, 1, 1);
   // Every load so far (the Q operand among them) has landed before the loop is entered: left
   // to itself the compiler waits, in EVERY iteration, for as many loads as were issued after Q.
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
@@ -323,10 +327,29 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, SPLIT ? 1 : 2) void fa_prefill_k
     for (int e = 1; e < 16; ++e) mx = fmaxf(fmaxf(mx, s0[0][e]), s0[1][e]);
     settle(mx);
   }
+  if (one_tile) {
+    const lds_char vt_lds = lds + 2 * TILE;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {  // 16 keys
+      uint32_t pb[4];
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) {
+        const float w0 = __builtin_amdgcn_exp2f(fmaf(s0[g >> 1][(g & 1) * 8 + e], p.scale_log2e, -m_ref));
+        const float w1 = __builtin_amdgcn_exp2f(fmaf(s0[g >> 1][(g & 1) * 8 + e + 1], p.scale_log2e, -m_ref));
+        l0 += w0;
+        l1 += w1;
+        pb[e >> 1] = pack_bf2(w0, w1);
+      }
+      const bf16x8_t bw = __builtin_bit_cast(bf16x8_t, make_uint4(pb[0], pb[1], pb[2], pb[3]));
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, read_v(vt_lds, g * DT + dt)), bw, o[dt], 0, 0, 0);
+    }
+  }
   // K of tile kt + 2 goes where K of kt was, V of kt + 1 where V of kt - 1 was: both last read before the barrier
   // that ended the previous tile, both complete at the one that ends this tile.  (A step past the wave's
   // or the workgroup's last tile multiplies what lies in LDS and uses none of it.)
-  for (int kt = 0; kt < n_iter; kt += 2) {
+  for (int kt = 0; !one_tile && kt < n_iter; kt += 2) {
     __builtin_amdgcn_s_waitcnt(0x0F70);
     __syncthreads();
     if (kt + 2 < n_tiles) load_tile(rk, koff, 0, kt + 2);

@@ -88,7 +88,9 @@ def test_grouped_gemm_multiplies_the_rows_of_its_tile(device, rows, K, bits):
 @pytest.mark.parametrize("T,past,Hq,Hkv,D,spare,scale", [
     (300, 40, 32, 8, 128, 0, 1.0), (300, 40, 4, 4, 128, 7, 1.0), (9, 0, 4, 4, 64, 0, 1.0), (33, 30, 4, 1, 128, 1, -1.0),
     (257, 61, 8, 1, 64, 0, 1.0), (130, 5, 6, 2, 128, 70, 0.3), (1000, 0, 8, 2, 128, 24, 6.0), (64, 0, 8, 8, 64, 0, 6.0),
-    (2100, 100, 16, 2, 128, 0, 1.0), (520, 1000, 8, 8, 64, 3, -6.0), (128, 64, 4, 2, 64, 0, 0.0)])
+    (2100, 100, 16, 2, 128, 0, 1.0), (520, 1000, 8, 8, 64, 3, -6.0), (128, 64, 4, 2, 64, 0, 0.0),
+    # contexts of one tile, its last key the cache's last and not, and one key past it
+    (64, 0, 4, 4, 128, 0, 3.0), (17, 47, 8, 2, 64, 9, 1.0), (63, 1, 4, 1, 128, 5, -2.0), (1, 0, 4, 1, 64, 0, 1.0), (65, 0, 8, 1, 64, 0, 1.0)])
 def test_prompt_attention_at_tile_edges(device, T, past, Hq, Hkv, D, spare, scale):
     g = torch.Generator(device=device).manual_seed(T + past)
     B, S = 2, past + T + spare
