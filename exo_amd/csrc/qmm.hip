@@ -34,9 +34,10 @@
 //    cycles; 20 % go into the wait for the tile requested a step ahead and the barrier, the rest
 //    into slots with more vector work than an MFMA covers.
 //  * few output tiles: blockIdx.z splits K; float32 partial tiles and a small reduce launch.
-//  * 17 to 64 rows belong to qmm_short.hip (K up to 32768).  Up to 16 rows that the GEMVs do not take, and up
-//    to 32 beyond that K: the four waves side by side on a 32 x 256 tile, so no weight row is
-//    dequantised twice, and K split until the launch has up to two workgroups per CU.
+//  * 17 to 64 rows belong to qmm_short.hip where its launch is one round of workgroups over a K that is not
+//    long (exo_qmm_short_beats_split).  Otherwise up to 32 rows (64 on matrices of 8192 rows or more) have the
+//    four waves side by side on a (32 or 64) x 256 tile, so that no weight row is dequantised twice, and K
+//    split until the launch has up to two workgroups per CU.
 #include "../../include/exo_mi355x.h"
 #include "common.h"
 #include "dequant.h"
@@ -158,7 +159,7 @@ __device__ __forceinline__ uint32_t dequant_piece(uint32_t lo, uint32_t hi, floa
 // so the SwiGLU happens in the epilogue and neither projection is written to memory.
 // WIDE: the four waves sit side by side - the workgroup tile is (32*MI) x 256 weight rows,
 // every wave owns 64 of them, so nothing is dequantised twice.  Plain GEMM of up to
-// 32 rows: blockIdx.z always owns a K range and the tile leaves as a float32 partial.
+// 64 rows: blockIdx.z always owns a K range and the tile leaves as a float32 partial.
 // Grouped GEMM (MI = 4: the expert's 128-row tile against 256 weight rows, the wave tile of
 // the 256-row kernel): whole K, the usual epilogue.  The same tile for the plain (gate, up)
 // pair of a long input: per product it stages half the activation bytes of the 256 x 64 tile
@@ -221,7 +222,7 @@ template <int BITS, int MI, bool GROUPED = false, bool SB4 = false, bool PAIR = 
 __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_kernel(const QmmParams p) {
   static_assert(!WIDE || GROUPED || !PAIR || MI >= 4, "the wide pair tile has 128 or 256 rows");
   static_assert(!DEEP || (SB4 && ((MI == 2 && !WIDE) || (WIDE && MI < 4))),
-                "the deep pipeline is for 128-row tiles; on the 32-row wide tile the flag "
+                "the deep pipeline is for 128-row tiles; on the 32- and 64-row wide tiles the flag "
                 "selects the ring (K ranges long enough to fill it)");
   static_assert(!KH || (MI == 4 && SB4 && !GROUPED && !DEEP && !(WIDE && PAIR)),
                 "two K halves per workgroup: the 256-row tile of the plain and the pair GEMM, "
@@ -980,7 +981,7 @@ int wide_max_split(int N) {
 }
 
 bool plan_wide(int M, int N, int K, const QmmParams& p, bool have_ws, int* ksplit, int* kc) {
-  if (!have_ws || M > 32 || N > kQmmWideMaxN || K % 256 != 0) return false;
+  if (!have_ws || M > 64 || (M > 32 && N < 8192) || N > kQmmWideMaxN || K % 256 != 0) return false;
   if ((((uintptr_t)p.s | (uintptr_t)p.b) & 7) != 0) return false;
   const int cap = wide_max_split(N);
   int ks = 1;
@@ -1035,10 +1036,14 @@ void launch_qmm(const QmmParams& p, hipStream_t st) {
     // K ranges of twelve steps or more fill the ring (4096x14336 4-bit at 17 rows 22.3 -> 19.3
     // us); on short ranges its start-up costs more than it returns (14336x4096: 20.5 -> 21.4)
     const bool ring = p.kc >= kWideRingMinK;
-    if (ring)
+    if (M <= 32 && ring)
       exo_note_variant("qmm_kernel<%d, 1, false, true, false, true, true>", BITS), qmm_kernel<BITS, 1, false, true, false, true, true><<<g, 256, 0, st>>>(p);
-    else
+    else if (M <= 32)
       exo_note_variant("qmm_kernel<%d, 1, false, true, false, true>", BITS), qmm_kernel<BITS, 1, false, true, false, true><<<g, 256, 0, st>>>(p);
+    else if (ring)
+      exo_note_variant("qmm_kernel<%d, 2, false, true, false, true, true>", BITS), qmm_kernel<BITS, 2, false, true, false, true, true><<<g, 256, 0, st>>>(p);
+    else
+      exo_note_variant("qmm_kernel<%d, 2, false, true, false, true>", BITS), qmm_kernel<BITS, 2, false, true, false, true><<<g, 256, 0, st>>>(p);
     reduce_parts(p.part, p.residual, p.y, M, N, p.ksplit, st);
     return;
   }
@@ -1387,7 +1392,7 @@ extern "C" int exo_qmm_swiglu_ws(const uint16_t* x, const uint32_t* w_gate,
                              ((uintptr_t)workspace & 255) == 0),
               "exo_qmm_swiglu_ws: workspace of %lld bytes, need %lld (256-byte aligned)",
               (long long)workspace_bytes, (long long)exo_qmm_swiglu_workspace(M, N));
-  if (exo_qmm_short_fits(M, K)) {
+  if (exo_qmm_short_fits(M, N, K, bits)) {
     exo_qmm_short(x, w_gate, s_gate, b_gate, w_up, s_up, b_up, nullptr, y, M, N, K, bits, 1, nullptr, 0,
                   (hipStream_t)stream);
     EXO_CHECK_LAUNCH("exo_qmm_swiglu");
@@ -1457,8 +1462,11 @@ extern "C" int exo_qmm_ws(const uint16_t* x, const uint32_t* w, const uint16_t* 
               (long long)workspace_bytes, (long long)exo_qmm_workspace(M, N));
   EXO_REQUIRE((int64_t)M * K < (1ll << 31), "exo_qmm: M*K=%lld exceeds 32-bit byte offsets",
               (long long)M * K);
-  if (exo_qmm_short_fits(M, K)) {
-    const int parts = workspace ? exo_qmm_short_parts(N, K) : 1;
+  // (with a workspace the other choice is a tile that splits K, on whole blocks of four steps)
+  const bool can_split = K % 256 == 0 && (((uintptr_t)scales | (uintptr_t)biases) & 7) == 0;
+  if (workspace ? exo_qmm_short_can(M, K) && (exo_qmm_short_beats_split(M, N, K) || (!can_split && exo_qmm_short_fits(M, N, K, bits)))
+                : exo_qmm_short_fits(M, N, K, bits)) {
+    const int parts = workspace ? exo_qmm_short_parts(M, N, K) : 1;
     float* const part = reinterpret_cast<float*>(workspace);
     exo_qmm_short(x, w, scales, biases, nullptr, nullptr, nullptr, residual, y, M, N, K, bits, parts, part,
                   part_stride(M, N), (hipStream_t)stream);

@@ -2,15 +2,22 @@
 #pragma once
 #include "common.h"
 
-// Inputs that it takes: 17 to kQmmShortMaxRows rows (fewer: the GEMV family), rows of whole groups whose
+// Inputs that it can take: 17 to kQmmShortMaxRows rows (fewer: the GEMV family), rows of whole groups whose
 // scales fit beside the activations in LDS.
 // (two blocks of 64 rows would read the weights twice: pair of 14336x4096 under 126 rows 61 us against 54)
 constexpr int kQmmShortMaxRows = 64;
 constexpr int kQmmShortMaxK = 32768;
-inline bool exo_qmm_short_fits(int M, int K) { return M > 16 && M <= kQmmShortMaxRows && K % 64 == 0 && K <= kQmmShortMaxK; }
+inline bool exo_qmm_short_can(int M, int K) { return M > 16 && M <= kQmmShortMaxRows && K % 64 == 0 && K <= kQmmShortMaxK; }
 
-// parts of K that a launch without a second matrix is best split into
-int exo_qmm_short_parts(int N, int K);
+// whether the pair is faster here than on the 128-row tile.  A product without room to split K answers alike,
+// so that the pair keeps the bits of two such products.
+bool exo_qmm_short_fits(int M, int N, int K, int bits);
+
+// parts of K that a launch without a second matrix is best split into, where it has room for their sums
+int exo_qmm_short_parts(int M, int N, int K);
+
+// whether such a launch is faster than the tiles that split K over workgroups (qmm.hip), where those can be had
+bool exo_qmm_short_beats_split(int M, int N, int K);
 
 // y[M,N] = x w^T (+ residual), or with a second matrix silu(x w^T) * (x w2^T); with several parts of K only their
 // float32 sums, to part[parts][part_stride]

@@ -308,21 +308,23 @@ void launch_tiles(const ShortParams& p, int parts, hipStream_t st) {
   qmm_short_kernel<BITS, PAIR, MT, NT><<<dim3(exo_ceil_div(p.tiles, NT), parts), 64 * kWaves, 0, st>>>(p);
 }
 
-// one workgroup per CU, as many tiles each as that takes - as far as their scales fit into LDS
+// Tiles per workgroup: one workgroup per CU, as many tiles each as that takes - as far as the scales of K elements
+// per row fit into LDS.  (Five and six run as seven, on fewer CUs: pair of K = 4096 under 33 rows, 10240 columns
+// 30.7 us, 12288 32.1, 14336 33.4.)
+int tiles_per_wg(int wanted, int K) {
+  const int fit = kQmmShortMaxK / K, nt = std::min(wanted, fit);
+  return nt >= 5 && fit >= 7 ? 7 : nt >= 4 ? 4 : std::max(nt, 1);
+}
+
 template <int BITS, bool PAIR, int MT>
 void launch(const ShortParams& p, int parts, hipStream_t st) {
-  const int fit = kQmmShortMaxK / (p.groups * 64);
-  const int nt = std::min(parts > 1 ? parts : exo_ceil_div(p.tiles, kCUs), fit);
-  if (nt >= 5 && fit >= 7)  // (five tiles and more)
-    launch_tiles<BITS, PAIR, MT, 7>(p, parts, st);
-  else if (nt >= 4)
-    launch_tiles<BITS, PAIR, MT, 4>(p, parts, st);
-  else if (nt == 3)
-    launch_tiles<BITS, PAIR, MT, 3>(p, parts, st);
-  else if (nt >= 2)
-    launch_tiles<BITS, PAIR, MT, 2>(p, parts, st);
-  else
-    launch_tiles<BITS, PAIR, MT, 1>(p, parts, st);
+  switch (tiles_per_wg(parts > 1 ? parts : exo_ceil_div(p.tiles, kCUs), p.groups * 64)) {
+    case 7: return launch_tiles<BITS, PAIR, MT, 7>(p, parts, st);
+    case 4: return launch_tiles<BITS, PAIR, MT, 4>(p, parts, st);
+    case 3: return launch_tiles<BITS, PAIR, MT, 3>(p, parts, st);
+    case 2: return launch_tiles<BITS, PAIR, MT, 2>(p, parts, st);
+    default: return launch_tiles<BITS, PAIR, MT, 1>(p, parts, st);
+  }
 }
 
 template <int BITS, bool PAIR>
@@ -337,8 +339,42 @@ void launch_rows(const ShortParams& p, int parts, hipStream_t st) {
 
 // Four quarters of K where one tile per CU would make every CU read 1 MB of activations and more: 4096x14336 4-bit
 // under 61 rows 37 -> 25 us, 2048x8192 16.8 -> 15.8 (4096x4096, whole: 11 us).
-int exo_qmm_short_parts(int N, int K) {
-  return exo_ceil_div(N, 16) <= kCUs && K >= 8192 && K % (4 * 512) == 0 ? 4 : 1;
+// (Under up to 32 rows the tile that splits K is ahead beyond K = 16384, 4096x28672 28.3 us against 29.6, and
+// on narrow matrices, 128x8192 10.7 against 11.6, 1024x12288 0.92 of its speed.)
+int exo_qmm_short_parts(int M, int N, int K) {
+  return exo_ceil_div(N, 16) <= kCUs && K >= 8192 && (M > 32 || (N >= 2048 && K <= 16384)) && K % (4 * 512) == 0 ? 4 : 1;
+}
+
+// Up to 8192 rows of weights a CU has four tiles at most, and the 128-row tile half of the chip: ahead by a third and
+// more, until K is so long that the activations of every workgroup outweigh it (8192x11008 under 64 rows 0.88 of the
+// other's speed, under 32 rows 1.13).  Beyond that the two are rounds of workgroups against rounds of workgroups,
+// and the times below (us) hold within 7 % (here) and 12 % over 512 <= K <= 28672 and up to 53248 rows.  Pairs, 4-bit,
+// us, 128-row tile -> here: 14336x4096 33 rows 51 -> 33, 16384x2048 (a round against two) 33 rows 0.69 of
+// the speed, 16384x8192 1.33, 28672x1024 17 rows 1.03, 64 rows 0.78, 14336x768 17 rows 1.05, 64 rows 0.80.
+// Products of more than 32768 rows are the matrices of a vocabulary, alone: 65536x4096 17 rows 82 -> 74, 33
+// rows 82 -> 91; 128256x4096 17 rows 161 -> 126, 64 rows 171 -> 170; 128256x2048 17 rows 79 -> 83, 64 rows 85 -> 113.
+bool exo_qmm_short_fits(int M, int N, int K, int bits) {
+  if (!exo_qmm_short_can(M, K)) return false;
+  if (N <= 8192) return K <= 8192 || (M <= 32 && K <= 16384);
+  if (N > 32768 && (M > 32 || K < 3072)) return false;
+  const int tiles = exo_ceil_div(N, 8), nt = tiles_per_wg(exo_ceil_div(tiles, kCUs), K);
+  const int rounds = exo_ceil_div(exo_ceil_div(tiles, nt), kCUs), rounds128 = exo_ceil_div(exo_ceil_div(N, 64), kCUs);
+  const double k = K / 1000., per_tile = bits == 4 ? 0.58 : 0.85;
+  const double whole = M <= 32 ? 7.3 + k * (per_tile * nt + 0.4) : 10.5 + k * (per_tile * nt + 0.9);
+  const double here = K % 512 == 0 ? whole : 1.2 * whole;  // (scales that are no whole 16-byte pieces)
+  const double other = bits == 4 ? 3.7 + 9.75 * k : 2.6 + 12 * k;
+  return rounds * here <= (M > 32 && K > 8192 ? 0.9 : 0.95) * (rounds128 * other);
+}
+
+// One round of workgroups, each with the whole of a K of up to 8192 or with a quarter of it.  A second round does not
+// overlap the first one's end, and every workgroup reads all activations, which over a long K is more than its
+// weights.  4-bit under 64 rows, us, split tile -> here: 16384x8192 (four tiles each) 47 -> 42, 24576x8192 (two
+// rounds) 64 -> 78, 8192x14336 41 -> 48, 8192x28672 66 -> 139, 4096x11008 27 -> 32, 32768x2048 (two rounds) 29 -> 45;
+// under 17 rows 24576x8192 52.5 -> 54, 8192x28672 53 -> 73, 32768x768 14.5 -> 23.
+bool exo_qmm_short_beats_split(int M, int N, int K) {
+  if (exo_qmm_short_parts(M, N, K) > 1) return true;
+  const int tiles = exo_ceil_div(N, 16);
+  return K <= (tiles <= kCUs ? 8191 : 8192) && exo_ceil_div(tiles, tiles_per_wg(exo_ceil_div(tiles, kCUs), K)) <= kCUs;
 }
 
 void exo_qmm_short(const bf16_t* x, const uint32_t* w, const bf16_t* s, const bf16_t* b, const uint32_t* w2,

@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 if not torch.cuda.is_available():
     pytest.skip("needs a GPU", allow_module_level=True)
 
-from exo_amd import ops  # noqa: E402
+from exo_amd import native, ops  # noqa: E402
 from exo_amd.ops import QuantizedWeight  # noqa: E402
 
 
@@ -170,3 +170,41 @@ def test_short_prompt_pair_gemm(device, M, N, K, bits):
     x = torch.randn(M, K, device=device, generator=torch.Generator(device=device).manual_seed(K)).bfloat16()
     want = ops.swiglu(ops.qmm(x, gate), ops.qmm(x, up))
     assert torch.equal(ops.qmm_swiglu(x, gate, up).view(torch.int16), want.view(torch.int16))
+
+
+# where the launch would be more than one round of workgroups, or its K is long, the tiles that split K stay: both sizes of
+# the row tile, with and without enough steps for the ring, more rows of weights than they take, the edges of the rule
+@pytest.mark.parametrize("M,N,K,bits,variant", [
+    (64, 8192, 12288, 4, "qmm_kernel<4, 2, false, true, false, true, true>"), (33, 8200, 8448, 8, "qmm_kernel<8, 2, false, true, false, true, true>"),
+    (64, 32768, 768, 4, "qmm_kernel<4, 2, false, true, false, true>"), (17, 30000, 512, 8, "qmm_kernel<8, 1, false, true, false, true>"),
+    (32, 4100, 28672, 4, "qmm_kernel<4, 1, false, true, false, true, true>"), (40, 1000, 33024, 4, "qmm_kernel<4, 2, false, true, false, false, true>"),
+    (33, 32776, 3072, 4, "qmm_kernel<4, 2, false, true, false, false, true>"), (17, 32776, 2048, 4, "qmm_kernel<4, 2, false, true, false, false, true>"),
+    (32, 32776, 3072, 4, "qmm_short<4,one,2,7>"), (64, 16384, 8192, 4, "qmm_short<4,one,4,4>"), (64, 28672, 512, 8, "qmm_short<8,one,4,7>")])
+def test_short_prompts_take_the_faster_tile(device, M, N, K, bits, variant):
+    q = packed(N, K, bits, M + N, device)
+    x = torch.randn(M, K, device=device, generator=torch.Generator(device=device).manual_seed(M)).bfloat16()
+    got = ops.quantized_matmul(x, q)
+    assert native.last_variant().split(" parts")[0] == variant, native.last_variant()
+    check(got, x, weights64(q), what=f"{M}x{N}x{K}")
+
+
+@pytest.mark.parametrize("M,N,K,bits", [(33, 32776, 512, 4), (20, 32776, 3072, 4)])
+def test_wide_pair_has_the_bits_of_two_products(device, M, N, K, bits):
+    """More rows of weights than one round of workgroups holds: the pair and the products alone take the same tile."""
+    gate, up = packed(N, K, bits, M, device), packed(N, K, bits, N, device)
+    x = torch.randn(M, K, device=device, generator=torch.Generator(device=device).manual_seed(K)).bfloat16()
+    want = ops.swiglu(ops.qmm(x, gate), ops.qmm(x, up))
+    assert torch.equal(ops.qmm_swiglu(x, gate, up, split_k=False).view(torch.int16), want.view(torch.int16))
+
+
+# a short launch of one round against one round, two against one, two against two; up to 8192 rows of weights; a long K
+@pytest.mark.parametrize("M,N,K,bits,short", [(33, 8200, 2048, 4, True), (33, 14336, 768, 8, False), (64, 16384, 1024, 4, False),
+                                              (20, 20480, 2048, 4, True), (64, 20480, 1024, 4, False), (64, 8192, 512, 4, True),
+                                              (64, 1024, 12288, 4, False), (20, 1024, 12288, 4, True)])
+def test_short_prompt_pair_takes_the_faster_tile(device, M, N, K, bits, short):
+    gate, up = packed(N, K, bits, M, device), packed(N, K, bits, N, device)
+    x = torch.randn(M, K, device=device, generator=torch.Generator(device=device).manual_seed(K)).bfloat16()
+    want = ops.swiglu(ops.qmm(x, gate), ops.qmm(x, up))
+    got = ops.qmm_swiglu(x, gate, up, split_k=False)
+    assert native.last_variant().startswith(f"qmm_short<{bits},pair" if short else f"qmm_kernel<{bits}, 2"), native.last_variant()
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
