@@ -34,7 +34,7 @@
 //    cycles; 20 % go into the wait for the tile requested a step ahead and the barrier, the rest
 //    into slots with more vector work than an MFMA covers.
 //  * few output tiles: blockIdx.z splits K; float32 partial tiles and a small reduce launch.
-//  * 17 to 64 rows belong to qmm_short.hip where its launch is one round of workgroups over a K that is not
+//  * 9 to 64 rows belong to qmm_short.hip where its launch is one round of workgroups over a K that is not
 //    long (exo_qmm_short_beats_split).  Otherwise up to 32 rows (64 on matrices of 8192 rows or more) have the
 //    four waves side by side on a (32 or 64) x 256 tile, so that no weight row is dequantised twice, and K
 //    split until the launch has up to two workgroups per CU.

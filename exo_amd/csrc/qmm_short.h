@@ -1,13 +1,17 @@
-// The quantised GEMM of short prompts (qmm_short.hip).
+// The quantised GEMM of 9 to 64 rows (qmm_short.hip).
 #pragma once
 #include "common.h"
 
-// Inputs that it can take: 17 to kQmmShortMaxRows rows (fewer: the GEMV family), rows of whole groups whose
-// scales fit beside the activations in LDS.
+// Inputs that it can take: kQmmShortMinRows (fewer: the GEMV family) to kQmmShortMaxRows rows, K of whole groups
+// whose scales fit beside the activations in LDS.  9 to 16 rows are those of 8-bit models, which leave the GEMVs
+// at 8: pair of 14336x4096 under 12 rows 35 us (128-row tile 55, two products that split K and the SwiGLU 49),
+// of 8192x2048 13 (20, 27); 4096x14336 20.7 (25), 6144x4096 12.8 (16.5).
 // (two blocks of 64 rows would read the weights twice: pair of 14336x4096 under 126 rows 61 us against 54)
-constexpr int kQmmShortMaxRows = 64;
+constexpr int kQmmShortMinRows = 9, kQmmShortMaxRows = 64;
 constexpr int kQmmShortMaxK = 32768;
-inline bool exo_qmm_short_can(int M, int K) { return M > 16 && M <= kQmmShortMaxRows && K % 64 == 0 && K <= kQmmShortMaxK; }
+inline bool exo_qmm_short_can(int M, int K) {
+  return M >= kQmmShortMinRows && M <= kQmmShortMaxRows && K % 64 == 0 && K <= kQmmShortMaxK;
+}
 
 // whether the pair is faster here than on the 128-row tile.  A product without room to split K answers alike,
 // so that the pair keeps the bits of two such products.

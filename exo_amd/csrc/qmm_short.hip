@@ -1,4 +1,4 @@
-// Quantised matmul for short prompts (17 to 128 rows): y[M,N] = x[M,K] @ dq(W)[N,K]^T, or the gate / up pair
+// Quantised matmul of 9 to 64 rows (short prompts, batches of an 8-bit model): y[M,N] = x[M,K] @ dq(W)[N,K]^T, or the gate / up pair
 // with its SwiGLU.
 //
 // A launch of so few rows streams its weights once and has little arithmetic per weight, so what

@@ -214,8 +214,8 @@ def quantized_matmul(
         out = torch.empty(M, qw.N, dtype=torch.bfloat16, device=x.device)
     if norm_weight is not None and M > QMV_MAX_M:
         raise ValueError("fused rms_norm is only available on the GEMV path (M <= 16)")
-    # 9..16 rows: the matrix-core GEMV needs its 16-row variant there, which the split-K
-    # GEMM matches or beats for 8-bit weights (measured on the Llama-8B shapes)
+    # 9..16 rows: the matrix-core GEMV needs its 16-row variant there, which the short
+    # GEMM beats for 8-bit weights (measured on the Llama-8B shapes)
     gemm_rows = M > 8 and norm_weight is None and qw.bits == 8
     # a matrix of up to 1 MiB without a residual (a MoE router): the library runs its
     # single-row kernel once per row in one launch, whatever the bit width

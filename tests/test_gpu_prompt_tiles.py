@@ -208,3 +208,21 @@ def test_short_prompt_pair_takes_the_faster_tile(device, M, N, K, bits, short):
     got = ops.qmm_swiglu(x, gate, up, split_k=False)
     assert native.last_variant().startswith(f"qmm_short<{bits},pair" if short else f"qmm_kernel<{bits}, 2"), native.last_variant()
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("M,N,K,bits", [(9, 14336, 2048, 8), (16, 14336, 1024, 8), (12, 8192, 2048, 8), (9, 40, 64, 8), (16, 2050, 832, 4)])
+def test_nine_to_sixteen_rows(device, M, N, K, bits):
+    """Batches of an 8-bit model past the GEMV: the pair, and its products alone."""
+    gate, up = packed(N, K, bits, M, device), packed(N, K, bits, N, device)
+    x = torch.randn(M, K, device=device, generator=torch.Generator(device=device).manual_seed(K)).bfloat16()
+    got = ops.qmm_swiglu(x, gate, up)
+    assert native.last_variant().startswith(f"qmm_short<{bits},pair,2,"), native.last_variant()
+    a, b = ops.qmm(x, gate), ops.qmm(x, up)
+    check(a, x, weights64(gate), what=f"gate {M}x{N}x{K}")
+    assert torch.equal(got.view(torch.int16), ops.swiglu(a, b).view(torch.int16))
+    r = torch.randn(M, N, device=device, generator=torch.Generator(device=device).manual_seed(N)).bfloat16()
+    y = torch.empty_like(r)
+    ws = ops.qmm_workspace(M, N, device)  # (the product as the engine calls it past the GEMV's rows)
+    native.check(native.load().exo_qmm_ws(x.data_ptr(), gate.weight.data_ptr(), gate.scales.data_ptr(), gate.biases.data_ptr(), r.data_ptr(),
+                                          y.data_ptr(), ws.data_ptr(), ws.numel(), M, N, K, bits, 64, torch.cuda.current_stream().cuda_stream), "qmm")
+    check(y, x, weights64(gate), r, what=f"{M}x{N}x{K} with residual")
