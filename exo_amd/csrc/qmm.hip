@@ -195,7 +195,10 @@ __device__ __forceinline__ int xcd_run(int l, int n) {
 template <int GM>
 __device__ __forceinline__ void tile_of_block(int& x, int& y) {
   const int gx = gridDim.x, gy = gridDim.y, n = gx * gy;
-  if (gridDim.z > 1 && (n & 7)) return;  // (the planes of a split would start on different XCDs)
+  // A launch that splits K is one round of short workgroups: the divisions and the order itself cost more than the
+  // shared rows return (300x6144x4096 8-bit, three row tiles: 53 us in launch order, 59 in this one; 200x9216x4096 59, 64;
+  // 100x4096x4096 4-bit 20.6, 21.7).  One row of tiles has only activations to share (32768x1024 17.4, 19.6).
+  if (gridDim.z > 1 || gy == 1) return;
   tile_at<GM>(xcd_run(y * gx + x, n), gx, gy, x, y);
 }
 
