@@ -1096,7 +1096,7 @@ void launch_qmm(const QmmParams& p, hipStream_t st) {
     // rows 144 -> 126 us, 4096x14336 under 4094 rows 523 -> 472, 8192x8192 under 2046 rows
     // 292 -> 270)
     else if (sb4 && prefer_big((int64_t)gw.x * g4.y, (int64_t)gw.x * gw.y))
-      exo_note_variant("qmm_kernel<%d, 4, false, true, false, true>", BITS), qmm_kernel<BITS, 8, false, true, false, true><<<dim3(big_grid(exo_ceil_div(N, 256) * g4.y)), 256, 0, st>>>(p);
+      exo_note_variant("qmm_kernel<%d, 8, false, true, false, true>", BITS), qmm_kernel<BITS, 8, false, true, false, true><<<dim3(big_grid(exo_ceil_div(N, 256) * g4.y)), 256, 0, st>>>(p);
     else if (sb4 && (BITS == 4 || kRing8) && (int64_t)gw.x * gw.y >= kWideRingMinTiles && weights_stay_cached(N, p.K, BITS))
       exo_note_variant("qmm_kernel<%d, 4, false, true, false, true>", BITS), qmm_kernel<BITS, 4, false, true, false, true><<<gw, 256, 0, st>>>(p);
     else if (sb4)
@@ -1357,8 +1357,7 @@ void launch_pair(const QmmParams& p, hipStream_t st) {
     if (sb4 && (int64_t)g4.x * g4.y <= 256 && p.K % 512 == 0 && p.K >= 1024)
       exo_note_variant("qmm_kernel<%d, 4, false, true, true, false, false, true>", BITS), qmm_kernel<BITS, 4, false, true, true, false, false, true><<<g4, 512, 0, st>>>(p);
     else if (sb4 && prefer_big((int64_t)exo_ceil_div(p.N, 128) * exo_ceil_div(p.M, 256), (int64_t)exo_ceil_div(p.N, 128) * exo_ceil_div(p.M, 128)))
-      // (noted as what it is an instance of: the wide tile with the ring)
-      exo_note_variant("qmm_kernel<%d, 4, false, true, true, true>", BITS), qmm_kernel<BITS, 8, false, true, true, true><<<dim3(big_grid(exo_ceil_div(p.N, 128) * exo_ceil_div(p.M, 256))), 256, 0, st>>>(p);
+      exo_note_variant("qmm_kernel<%d, 8, false, true, true, true>", BITS), qmm_kernel<BITS, 8, false, true, true, true><<<dim3(big_grid(exo_ceil_div(p.N, 128) * exo_ceil_div(p.M, 256))), 256, 0, st>>>(p);
     else if (sb4 && p.M >= kPairWideMinM && weights_stay_cached(2 * (int64_t)p.N, p.K, BITS))
       exo_note_variant("qmm_kernel<%d, 4, false, true, true, true>", BITS), qmm_kernel<BITS, 4, false, true, true, true><<<dim3(exo_ceil_div(p.N, 128), exo_ceil_div(p.M, 128)), 256, 0, st>>>(p);
     else if (sb4)

@@ -102,12 +102,13 @@ def test_llama_8b_decode_step_at_bench_context(device):
 
 
 @pytest.mark.parametrize("M,N,K,bits,variant", [
-    (2046, 14336, 4096, 4, "qmm_kernel<4, 4, false, true, true, true>"),   # Llama-3.1-8B prompt chunk
-    (2046, 12288, 4096, 8, "qmm_kernel<8, 4, false, true, true, true>"),   # an 8-bit MLP of that size
+    (2046, 14336, 4096, 4, "qmm_kernel<4, 8, false, true, true, true>"),   # Llama-3.1-8B prompt chunk: 256-row tiles
+    (2046, 12288, 4096, 8, "qmm_kernel<8, 8, false, true, true, true>"),   # an 8-bit MLP of that size
+    (1030, 14336, 4096, 4, "qmm_kernel<4, 4, false, true, true, true>"),   # 128-row tiles, whose rounds fit this length better
 ])
 def test_gate_up_pair_gemm_at_prompt_size(device, M, N, K, bits, variant):
     """The (gate, up) pair GEMM with the SwiGLU epilogue under a 2046-row chunk - 44 % of the 8B
-    prompt's time - on the wide tile with the ring: bit-equal to the two single GEMMs followed
+    prompt's time - on the wide tiles with the ring: bit-equal to the two single GEMMs followed
     by the SwiGLU kernel; a sample of outputs against the oracle (weights rounded to bf16, as
     the matrix-core operand is), all outputs of both projections against dequantize + float32
     matmul."""
