@@ -841,11 +841,16 @@ inline unsigned big_grid(int tiles) { return (unsigned)(tiles + big_halved(tiles
 // small tile per CU 0.62, and so do the halves of the large one (its last round otherwise 1).  14336x4096 pair
 // under 2047 rows, 3.5 rounds: 420 us against 436; 128256x2048 under 777 rows, 8 rounds against
 // 6.85 since the fourth row tile holds 9 rows: 579 us against 463.
-bool prefer_big(int64_t big, int64_t small) {
+// That holds where K is long: one workgroup per CU has nothing to hide its start and its epilogue behind, two have each
+// other.  Of the small tile's time, over 27 shapes each: products of K = 1024 1.07 to 1.32, 2048 0.96 to
+// 1.15, 3072 0.93 to 1.07, 4096 0.88 to 1.0; pairs of 1024 0.99 to 1.14, 2048 0.90 to 0.97 where the rounds alone
+// give 0.93 and less, otherwise up to 1.04, 3072 0.90 to 0.99.
+bool prefer_big(int64_t big, int64_t small, int K, bool pair) {
+  if (K < (pair ? 2048 : 4096)) return false;
   const int64_t rb = big % kCUs, rs = small % (2 * kCUs);
   const double tb = big / kCUs + (rb == 0 ? 0. : 2 * rb <= kCUs ? 0.62 : 1.);
   const double ts = 1.1 * (small / (2 * kCUs)) + (rs == 0 ? 0. : rs <= kCUs ? 0.62 : 1.1);
-  return tb <= ts && big < (1 << 30);
+  return tb <= (K < 3072 ? 0.93 : 1.) * ts && big < (1 << 30);
 }
 
 constexpr int kQmmMaxSplit = 16;  // K ranges the reduce kernel adds
@@ -1095,7 +1100,7 @@ void launch_qmm(const QmmParams& p, hipStream_t st) {
     // more wide tiles than CUs: the wide tile with the ring, four waves (6144x4096 under 2046
     // rows 144 -> 126 us, 4096x14336 under 4094 rows 523 -> 472, 8192x8192 under 2046 rows
     // 292 -> 270)
-    else if (sb4 && prefer_big((int64_t)gw.x * g4.y, (int64_t)gw.x * gw.y))
+    else if (sb4 && prefer_big((int64_t)gw.x * g4.y, (int64_t)gw.x * gw.y, p.K, false))
       exo_note_variant("qmm_kernel<%d, 8, false, true, false, true>", BITS), qmm_kernel<BITS, 8, false, true, false, true><<<dim3(big_grid(exo_ceil_div(N, 256) * g4.y)), 256, 0, st>>>(p);
     else if (sb4 && (BITS == 4 || kRing8) && (int64_t)gw.x * gw.y >= kWideRingMinTiles && weights_stay_cached(N, p.K, BITS))
       exo_note_variant("qmm_kernel<%d, 4, false, true, false, true>", BITS), qmm_kernel<BITS, 4, false, true, false, true><<<gw, 256, 0, st>>>(p);
@@ -1356,7 +1361,7 @@ void launch_pair(const QmmParams& p, hipStream_t st) {
     // (up to one tall tile per CU: eight waves per tile, as in launch_qmm)
     if (sb4 && (int64_t)g4.x * g4.y <= 256 && p.K % 512 == 0 && p.K >= 1024)
       exo_note_variant("qmm_kernel<%d, 4, false, true, true, false, false, true>", BITS), qmm_kernel<BITS, 4, false, true, true, false, false, true><<<g4, 512, 0, st>>>(p);
-    else if (sb4 && prefer_big((int64_t)exo_ceil_div(p.N, 128) * exo_ceil_div(p.M, 256), (int64_t)exo_ceil_div(p.N, 128) * exo_ceil_div(p.M, 128)))
+    else if (sb4 && prefer_big((int64_t)exo_ceil_div(p.N, 128) * exo_ceil_div(p.M, 256), (int64_t)exo_ceil_div(p.N, 128) * exo_ceil_div(p.M, 128), p.K, true))
       exo_note_variant("qmm_kernel<%d, 8, false, true, true, true>", BITS), qmm_kernel<BITS, 8, false, true, true, true><<<dim3(big_grid(exo_ceil_div(p.N, 128) * exo_ceil_div(p.M, 256))), 256, 0, st>>>(p);
     else if (sb4 && p.M >= kPairWideMinM && weights_stay_cached(2 * (int64_t)p.N, p.K, BITS))
       exo_note_variant("qmm_kernel<%d, 4, false, true, true, true>", BITS), qmm_kernel<BITS, 4, false, true, true, true><<<dim3(exo_ceil_div(p.N, 128), exo_ceil_div(p.M, 128)), 256, 0, st>>>(p);

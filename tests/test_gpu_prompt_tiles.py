@@ -65,6 +65,40 @@ def test_prompt_pair_gemm_at_tile_edges(device, M, N, K, bits):
     check(ops.qmm(x, gate), x, weights64(gate), what=f"gate {M}x{N}x{K}")
 
 
+# the same edges where K is long enough for the 256 x 256 tile: two, four, six and eight blocks of 32 rows in the last
+# tile of a column, a last round in halves, the second of which holds no row, ragged columns
+@pytest.mark.parametrize("M,N,K,bits,pair", [(1030, 12288, 4096, 4, False), (900, 16397, 4352, 8, False), (960, 16640, 4096, 4, False), (1024, 8264, 4096, 8, False),
+                                             (600, 14336, 4096, 4, True), (1000, 8200, 3072, 8, True), (300, 14330, 3328, 4, True), (513, 14336, 4352, 8, True)])
+def test_large_tile_at_tile_edges(device, M, N, K, bits, pair):
+    gate = packed(N, K, bits, M, device)
+    x = torch.randn(M, K, device=device, generator=torch.Generator(device=device).manual_seed(K)).bfloat16()
+    name = f"qmm_kernel<{bits}, 8, false, true, {str(pair).lower()}, true>"
+    if pair:
+        up = packed(N, K, bits, N, device)
+        got = ops.qmm_swiglu(x, gate, up)
+        assert native.last_variant() == name, native.last_variant()
+        a, b = ops.qmm(x, gate), ops.qmm(x, up)
+        check(a, x, weights64(gate), what=f"gate {M}x{N}x{K}")
+        assert torch.equal(got.view(torch.int16), ops.swiglu(a, b).view(torch.int16))
+        return
+    r = torch.randn(M, N, device=device, generator=torch.Generator(device=device).manual_seed(M)).bfloat16()
+    got = ops.quantized_matmul(x, gate)
+    assert native.last_variant() == name, native.last_variant()
+    check(got, x, weights64(gate), what=f"{M}x{N}x{K}")
+    check(ops.quantized_matmul(x, gate, residual=r), x, weights64(gate), r, what=f"{M}x{N}x{K} with residual")
+
+
+@pytest.mark.parametrize("M,N,K,bits,pair", [(4096, 5120, 2048, 4, False), (1030, 16400, 512, 4, False), (1500, 8192, 2048, 4, True), (1000, 8200, 1024, 4, True)])
+def test_short_ranges_of_k_take_the_small_tile(device, M, N, K, bits, pair):
+    gate = packed(N, K, bits, M, device)
+    x = torch.randn(M, K, device=device, generator=torch.Generator(device=device).manual_seed(K)).bfloat16()
+    got = ops.qmm_swiglu(x, gate, gate) if pair else ops.quantized_matmul(x, gate)
+    assert native.last_variant() == f"qmm_kernel<{bits}, 4, false, true, {str(pair).lower()}, true>", native.last_variant()
+    y = ops.qmm(x, gate)
+    check(y, x, weights64(gate), what=f"{M}x{N}x{K}")
+    assert torch.equal(got.view(torch.int16), (ops.swiglu(y, y) if pair else y).view(torch.int16))
+
+
 @pytest.mark.parametrize("rows", [1, 32, 33, 64, 65, 96, 97, 128, 129])
 @pytest.mark.parametrize("K,bits", [(256, 4), (1280, 4), (256, 8), (1536, 8)])
 def test_grouped_gemm_multiplies_the_rows_of_its_tile(device, rows, K, bits):
