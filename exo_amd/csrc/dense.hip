@@ -27,6 +27,8 @@
 #include "../../include/exo_mi355x.h"
 #include "dense.h"
 
+#include <algorithm>
+
 namespace {
 
 // ------------------------------------------------------------------------------ GEMV
@@ -676,13 +678,16 @@ void launch_gemv_nw(const GemvParams& p, const GemvParams* p1, const PostNorm* q
 // product then holds, and rows of whole parts.  One part -> these, us: N = 2048 (128 workgroups -> 256) under
 // 4 rows, bf16: K = 4096 8.0 -> 6.9, K = 6912 11.8 -> 9.1 (8 rows: 12.8 -> 9.8); N = 1024 (64 -> 256) under
 // 2 rows, f32: K = 1024 6.5 -> 4.2, K = 2560 11.0 -> 5.7.  Four parts at N = 2048 give no more than two (6.8, 9.8).
-// Single products of 144 workgroups still gain (6.0 -> 5.4); a pair reads two matrices per workgroup: 160
-// of K = 1024, f32, would lose (7.8 -> 8.1).  16 waves instead of 8: 7.4 and 8.7 in place of 6.9 and 9.1, f32 6.9
-// in place of 5.7.
+// Where the two parts are more than 256 workgroups - a second round of them - only short rows still gain (one part ->
+// two, us: N = 2304 of 2 rows, bf16, K = 1024 1.15 and K = 2048 1.09 times as fast, 2176 0.94, 4096 0.87; f32 1024 1.19,
+// 2048 8.5 -> 9.3, 8 rows 9.0 -> 10.9); a pair reads two matrices per workgroup (N = 2304, bf16 1024 1.07,
+// 2048 0.95; f32 1024 0.95).  16 waves instead of 8: 7.4 and 8.7 in place of 6.9 and 9.1, f32 6.9 in place of 5.7.
 int gemv_parts(const GemvParams& p, const GemvParams* p1, int elem) {
   const int tiles = exo_ceil_div(p.N, 16) + (p1 ? exo_ceil_div(p1->N, 16) : 0);
   const int rows = p.ldw * elem | (p1 ? p1->ldw * elem : 0);
   if (tiles <= 96 && p.M <= 4 && rows % 256 == 0) return 4;
+  const int longest = std::max(p.ldw, p1 ? p1->ldw : 0) * elem;
+  if (tiles > 128 && longest > (p.w2 ? 2048 : 4096)) return 1;
   return tiles < (p.w2 ? 160 : 192) && p.M <= 8 && rows % 128 == 0 ? 2 : 1;
 }
 template <typename T, bool PAIR, bool DUAL, int Q>

@@ -26,7 +26,7 @@ def check(got, x, w, bias=0.0):
 # not fill a workgroup's, steps of K that do not fill its waves, as few as one for all of them
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("M,N,K,parts", [(1, 1, 128, 4), (4, 1536, 640, 4), (3, 130, 1920, 4), (4, 1537, 128, 2), (5, 97, 64, 2),
-                                         (8, 3055, 192, 2), (2, 2049, 2112, 2), (7, 1000, 7040, 2), (8, 3057, 128, 1),
+                                         (8, 3055, 192, 2), (2, 2049, 2112, 2), (2, 2048, 2112, 2), (2, 2049, 1984, 2), (7, 1000, 7040, 2), (8, 3057, 128, 1),
                                          (9, 40, 256, 1)])
 def test_parts_of_k(device, dtype, M, N, K, parts):
     g = torch.Generator(device=device).manual_seed(M * N + K)
@@ -36,6 +36,8 @@ def test_parts_of_k(device, dtype, M, N, K, parts):
     tail = min(3, N - 1)
     t = torch.zeros(M, max(tail, 1), device=device)
     D.linear(x, w, out, M, bias=b, tail=(t, tail) if tail else None)
+    if N > 2048 and K * out.element_size() > 4096:  # (a second round of workgroups over long rows)
+        parts = 1
     label = native.last_variant()
     assert ("parts=%d" % parts in label) if parts > 1 else ("dense_gemv" in label and "parts" not in label), label
     check(out[:M, : N - tail], x, w[: N - tail], b[: N - tail].double())
