@@ -37,10 +37,14 @@ constexpr int kBlk = 4;  // keys per lane group per step
 #define EXO_SDPA_TILES_IN_FLIGHT 2
 #endif
 constexpr int kTilesInFlight = EXO_SDPA_TILES_IN_FLIGHT;  // key tiles a wave keeps in flight
-// Contexts of one workgroup: two rounds of four waves' requests (256 keys of 128, 512 of 64).  The hand-over of
-// the splits costs 2.2 us, a round about 0.8.  One sequence, 32 / 8 heads of 128: 60 keys 5.9 -> 3.9 us, 130 keys 5.9
-// -> 4.9, 250 keys 5.9 -> 5.2 (400 keys level); of 64, 130 keys 6.2 -> 4.9, 500 keys 6.3 -> 6.0 (900 keys 6.8 -> 8.1)
-constexpr int kSoloTiles = 2 * 4 * 2;
+// Contexts of one workgroup, in tiles (16 keys of 128, 32 of 64): two rounds of four waves' requests, less where a
+// tile is worked on for several heads and where heads of 64 make its work longer.  The hand-over of
+// the splits costs 2.2 us, a round about 0.8 and more per head.  One sequence, 32 / 8 heads of 128: 60 keys 5.9 -> 3.9 us,
+// 130 keys 5.9 -> 4.9, 250 keys 5.9 -> 5.2 (400 keys level); of 64, 130 keys 6.2 -> 4.9, 440 keys 1.0 to 1.3 times as
+// fast, 512 keys 0.95 to 1.3.  Heads of 64, two per workgroup (4 sequences): 256 keys 1.13, 384 1.01, 440 0.97; four (8
+// sequences): 256 keys 10.0 -> 9.3, 264 9.6 -> 10.8, 440 9.9 -> 12.0.
+template <int D, int G>
+constexpr int kSoloTiles = D >= 128 ? 16 : G == 1 ? 14 : G == 2 ? 12 : 8;
 constexpr int kSoloMfma = 256;  // the matrix-core kernel: 8 sequences, 130 keys 10.8 -> 8.7 us, 250 keys 11.9 -> 10.6
                                 // (500 keys 12.6 -> 13.8); 4 of 32 / 4 heads, 130 keys 12.1 -> 7.9
 #ifndef EXO_SDPA_TILES_WAVES
@@ -455,11 +459,11 @@ __global__ __launch_bounds__(kThreads) void sdpa_kernel(const SdpaParams p) {
 // ---------------------------------------------------------------- decode, interleaved tiles
 // Decode attention with the key tiles dealt out round robin: the NWV = splits * 4 waves
 // that serve one (sequence, kv head, head group) take the tiles of STEP keys in turn (wave w:
-// tiles w, w + NWV, w + 2 NWV ...).  Which tile a wave starts with does not depend on the
-// sequence's length, so its first two tiles are requested before the position has even been
-// read - their latency runs beside the position -> rope table -> q rotation chain instead of
-// behind it - and every wave gets the same number of tiles to within one, whatever the length
-// (contiguous ranges rounded to whole steps left the last splits of a 2050-key context idle).
+// tiles w, w + NWV, w + 2 NWV ...; the four waves of the first workgroup all of them where the
+// context is short).  The first two tiles are requested as soon as the position is known, beside the
+// rope table's row and ahead of the q rotation, and every wave gets the same number of tiles to
+// within one, whatever the length (contiguous ranges rounded to whole steps left the last splits of
+// a 2050-key context idle).
 // Tiles come through buffer loads whose range ends at the last cached key: a refill past the
 // end moves no data and returns zeros, so every refill is issued unconditionally and the
 // number of loads in flight at each wait is a compile-time constant.
@@ -481,9 +485,9 @@ __global__ __launch_bounds__(64 * NW) void sdpa_tiles_kernel(const SdpaParams p)
   const int kvh = (int)blockIdx.y / p.hgroups, hg = (int)blockIdx.y % p.hgroups;
   const int h0 = kvh * (G * p.hgroups) + hg * G;  // first query head of this workgroup
   const int len = min(p.pos[b] + 1, p.S_max);  // keys visible to the query
-  // A short context is left to the first workgroup: the others are gone at once, and nothing is handed over
-  const bool solo = len <= kSoloTiles * STEP;
-  if (solo && blockIdx.x != 0) return;
+  // A short context is left to the first workgroup: the others are gone ahead of the tiles (not here: the requests
+  // for q would wait for the position too, 257 to 400 keys 1 % slower), and nothing is handed over
+  const bool solo = len <= kSoloTiles<D, G> * STEP;
   const int nwv = solo ? NW : p.splits * NW;
   const int gwv = (int)blockIdx.x * NW + wave;
 
@@ -537,6 +541,7 @@ __global__ __launch_bounds__(64 * NW) void sdpa_tiles_kernel(const SdpaParams p)
     for (int g = 0; g < G; ++g)
       qv[g] = *reinterpret_cast<const uint4*>(p.q + qrow + (size_t)(h0 + g) * D + sl * 8);
   }
+  if (solo && blockIdx.x != 0) return;
   Tile tl[NT];
 #pragma unroll
   for (int n = 0; n < NT; ++n) load_tile(tl[n], rk, rv, gwv + n * nwv);

@@ -18,10 +18,11 @@ def rotated(x, pos, inv):
     return torch.cat([lo * a.cos() - hi * a.sin(), hi * a.cos() + lo * a.sin()], -1).float().bfloat16().double()
 
 
-# one workgroup up to 256 keys of 128 or 512 of 64 (the matrix-core kernel, 16 and more pairs of 128: 256), several
+# one workgroup up to 256 keys of 128, or of 64 up to 448, 384 and 256 with one, two and four heads in it (the matrix-core kernel, 16 and more pairs of 128: 256), several
 # beyond; lengths differ inside a batch, and a second call finds the hand-over's counters as the first left them
 @pytest.mark.parametrize("Hq,Hkv,D,S,lens", [
     (32, 8, 128, 4096, [1]), (32, 8, 128, 4096, [256]), (32, 8, 128, 4096, [257]), (32, 8, 64, 600, [512]), (32, 8, 64, 600, [513]),
+    (32, 8, 64, 600, [448]), (32, 8, 64, 600, [449]), (32, 8, 64, 600, [384, 385, 383, 600]), (32, 8, 64, 600, [256, 257, 255, 1, 512, 300, 64, 33]),
     (16, 16, 64, 200, [130, 1]), (64, 4, 128, 1100, [255, 1024]), (32, 8, 128, 1024, [1, 255, 256, 257, 513, 700, 129, 2]),
     (32, 4, 128, 700, [256, 257, 31, 600]), (64, 4, 128, 300, [256, 300, 128, 129])])
 def test_decode_attention_around_the_first_split(device, Hq, Hkv, D, S, lens):
