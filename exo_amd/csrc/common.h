@@ -10,7 +10,20 @@ typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
 
+typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
+typedef __attribute__((address_space(3))) char* lds_char;
+
 #define EXO_WAVE 64
+
+// 16 bytes per lane from a buffer into LDS at `to` + 16 * lane, counted by vmcnt.  Written as the instruction (it
+// has no register result): the compiler makes the first LDS read behind such a request of its own wait for
+// it, whichever tile it fills.  It knows nothing of this one: the waits are the caller's.
+__device__ __forceinline__ void load_to_lds16_untracked(u32x4 rsrc, lds_char to, uint32_t voffset, uint32_t soffset) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               :
+               : "s"((uint32_t)(uintptr_t)to), "v"(voffset), "s"(rsrc), "s"(soffset)
+               : "memory", "m0");
+}
 
 __device__ __forceinline__ float bf2f(bf16_t b) {
   return __builtin_bit_cast(float, (uint32_t)b << 16);

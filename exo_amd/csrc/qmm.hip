@@ -96,20 +96,6 @@ __device__ __forceinline__ void load_to_lds16(__amdgpu_buffer_rsrc_t rsrc, void*
       rsrc, (__attribute__((address_space(3))) void*)lds_base, 16, voffset, soffset, 0, 0);
 }
 
-typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
-
-// The same, written as the instruction (it has no register result): the compiler makes the first LDS read
-// behind such a request wait for it, although it fills a tile that is read steps later, which a step of an expert's
-// few rows does not cover (pair of 768x2048 under 8184 pairs of 128 experts 113 -> 99 us, 2048x768 62.5 -> 58.5; the
-// 256-row tile, whose step does, 409 -> 421).  The waits are the caller's.
-__device__ __forceinline__ void load_to_lds16(u32x4 rsrc, void* lds_base, uint32_t voffset, uint32_t soffset) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-               :
-               : "s"((uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds_base), "v"(voffset),
-                 "s"(rsrc), "s"(soffset)
-               : "memory");
-}
-
 // elements between the partial tiles of consecutive K ranges (16-byte aligned rows of 4)
 __host__ __device__ inline size_t part_stride(int M, int N) {
   return ((size_t)M * N + 3) / 4 * 4;
@@ -341,8 +327,10 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
 #pragma unroll
     for (int r = 0; r < n; ++r) {
       char* const to = tiles + buf * TILE_BYTES + (wave * 64 + kThreads * r) * 16;
+      // (a step of an expert's few rows does not cover the compiler's wait, pair of 768x2048 under 8184 pairs of
+      // 128 experts 113 -> 99 us, 2048x768 62.5 -> 58.5; the 256-row tile's step does, 409 -> 421)
       if constexpr (RING && GROUPED)
-        load_to_lds16(rx4, to, xoff[r], k0 * 2);
+        load_to_lds16_untracked(rx4, (lds_char)to, xoff[r], k0 * 2);
       else
         load_to_lds16(rx, to, xoff[r], k0 * 2);
     }

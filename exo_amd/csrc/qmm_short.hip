@@ -35,8 +35,6 @@ namespace {
 constexpr int kWaves = 8;
 constexpr int kCUs = 256;
 
-typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
-
 struct ShortParams {
   const bf16_t* x;
   const uint32_t *w, *w2;

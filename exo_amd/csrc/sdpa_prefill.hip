@@ -55,8 +55,6 @@ constexpr int fa_lds_bytes() {
 }
 
 typedef short short4_t __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) char* lds_char;
-typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
 
 // ds_read_b64_tr_b16: four consecutive rows of one column out of a row-major bf16 tile
 __device__ __forceinline__ uint2 read_tr16(lds_char at) {
@@ -68,16 +66,6 @@ __device__ __forceinline__ uint2 read_tr16(lds_char at) {
 template <typename T>
 __device__ __forceinline__ void hold(T& v) {
   asm volatile("" : "+v"(v));
-}
-
-// 16 bytes per lane from a buffer into LDS at `to` + 16 * lane.  Written as the instruction (it has no register
-// result): the compiler makes every transposing LDS read wait for all such loads that it knows
-// of; here the wait and the barrier at the end of a tile are theirs.
-__device__ __forceinline__ void load_to_lds16(u32x4 rsrc, lds_char to, uint32_t voffset, uint32_t soffset) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-               :
-               : "s"((uint32_t)(uintptr_t)to), "v"(voffset), "s"(rsrc), "s"(soffset)
-               : "memory");
 }
 
 template <int D, bool SPLIT>
@@ -137,7 +125,9 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, SPLIT ? 1 : 2) void fa_prefill_k
     }
   }
 
-  // K and V tiles go from the cache straight into LDS, row by row as they are: one descriptor per
+  // K and V tiles go from the cache straight into LDS, row by row as they are (by the instruction: the compiler
+  // makes every transposing LDS read wait for all such loads that it knows of; the wait and the barrier
+  // at the end of a tile are theirs): one descriptor per
   // (sequence, kv head), a lane offset that never changes and the tile as the scalar offset.  A wave's
   // load writes its 64 chunks of 16 bytes in lane order, so the order of the chunks inside a row is
   // chosen by what a lane requests: chunk c of K row r sits at c ^ (r % 16) (128-byte rows: c ^ (r / 2 % 8)),
@@ -158,12 +148,12 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, SPLIT ? 1 : 2) void fa_prefill_k
     const lds_char to = lds + tile * TILE + wave * 1024;
     if (row0 + kBN <= p.S_max) {
 #pragma unroll
-      for (int i = 0; i < LOADS; ++i) load_to_lds16(r, to + i * 4096, off, row0 * ROW + i * 4096);
+      for (int i = 0; i < LOADS; ++i) load_to_lds16_untracked(r, to + i * 4096, off, row0 * ROW + i * 4096);
     } else {  // rows past the end of the cache: its last row again (they are masked)
 #pragma unroll
       for (int i = 0; i < LOADS; ++i) {
         const int row = lrow + i * (256 / VEC), over = max(0, row0 + row - (p.S_max - 1));
-        load_to_lds16(r, to + i * 4096, off + (row0 + i * (256 / VEC) - over) * ROW, 0);
+        load_to_lds16_untracked(r, to + i * 4096, off + (row0 + i * (256 / VEC) - over) * ROW, 0);
       }
     }
   };

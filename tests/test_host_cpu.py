@@ -44,6 +44,15 @@ def test_library_exports_every_declared_symbol():
     assert sorted(native.SIGNATURES) == syms  # the ctypes table covers the header one to one
 
 
+def test_assembly_that_writes_m0_says_so():
+    """The compiler keeps values of its own in m0 (the LDS base of its loads): a statement that writes it names it."""
+    sources = sorted((Path(native.__file__).parent / "csrc").glob("*"))
+    found = [(p.name, body) for p in sources for body in re.findall(r"\basm\b(?:\s+volatile)?\s*\((.*?)\);", p.read_text(), re.S)]
+    writers = [(name, body) for name, body in found if re.search(r"\bs_\w+ m0,", body)]
+    assert len(found) > 5 and writers
+    assert [name for name, body in writers if '"m0"' not in body.rsplit(":", 1)[1]] == []
+
+
 def test_argument_errors_without_gpu():
     lib = native.load()
     assert lib.exo_abi_version() == 1
