@@ -150,6 +150,8 @@ __global__ __launch_bounds__(64 * kWaves) void qmm_short_kernel(const ShortParam
     for (int j = 0; j < NT; ++j) load_w(w0, j, k_of(0));
 #pragma unroll
     for (int j = 0; j < XR; ++j) load_x(0, j, k_of(0));
+    // (step 0 waits by count for all but the last XR + NT requests: none of step 1 may be sent ahead of these)
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < NT; ++j) load_w(w1, j, k_of(1));
 #pragma unroll
@@ -178,7 +180,8 @@ __global__ __launch_bounds__(64 * kWaves) void qmm_short_kernel(const ShortParam
       sb[((row >> 4) * G + g) * 16 + (row & 15)] = s | b << 16;
     }
   }
-  // (the barrier's own fence would wait for the activations too)
+  // (No fence.  The first two steps have landed here all the same: the requests stand in branches, across which the
+  // compiler cannot count, so that its waits for the scales are waits for everything.)
   __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
   asm volatile("s_barrier" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
