@@ -96,9 +96,10 @@ __global__ __launch_bounds__(TH) void post_norm_add_kernel(const exo_post_norm q
   const bool vec = H % kCols == 0 && (m.y ? m.ldy % kCols == 0 && m.lds % kCols == 0 : q.ldb % kCols == 0);
   const bool gvec = H % kCols == 0;
   float v[PASSES][kCols], xv[PASSES][kCols];
-  // The gains with the inputs where a row's chain counts and there are registers for them: requested between
-  // one sum and the next they are a memory latency each (4 rows of 2048 columns, 5.6 -> 5.2 us).
-  constexpr bool AHEAD = PASSES <= TH / 512 || PASSES == 1;
+  // The gains with the inputs where a row's chain counts and it pays: requested between one sum and the next
+  // they are a memory latency each (4 rows, one branch / two: 1024 columns 3.35 -> 3.25 / 4.5 -> 4.2 us, 5120 4.4 ->
+  // 4.2 / 6.4 -> 6.4), but 2048 to 4096 columns in one pass of 1024 threads lose or are level (2048 3.57 -> 3.66 / 5.15).
+  constexpr bool AHEAD = TH == 256 ? PASSES == 1 : PASSES == 2;
   float ga[PASSES][kCols], gb[PASSES][kCols], gn[PASSES][kCols], gp[PASSES][kCols];
   auto load_gains = [&](int i, int c, int left, bool branches, bool sum, bool pre) {
     if (q.branch2 && branches) load_cols<float>(q.gain_a + c, ga[i], gvec, left), load_cols<float>(q.gain_b + c, gb[i], gvec, left);
