@@ -29,8 +29,8 @@
 //    and with one wave per SIMD the products of a K step are kept fed by that wave alone:
 //    the operands of the next product block, one dequantised register's half and every other slot an LDS
 //    read, ride between two MFMAs, across the barrier too (see multiply_on).  4096x14336 8-bit
-//    under 4096 rows 474 -> 407 us (1182 TFLOP/s), pair of 14336x4096 968 -> 824; 4-bit pair
-//    under 2047 rows 451 -> 420.  What bounds it: the matrix cores are busy 56 % of the
+//    under 4096 rows 471 -> 402 us (1197 TFLOP/s), pair of 14336x4096 949 -> 814 (1182); 4-bit pair
+//    under 2047 rows 439 -> 411 (1169).  Over a short K it loses (see prefer_big).  What bounds it: the matrix cores are busy 56 % of the
 //    cycles; 20 % go into the wait for the tile requested a step ahead and the barrier, the rest
 //    into slots with more vector work than an MFMA covers.
 //  * few output tiles: blockIdx.z splits K; float32 partial tiles and a small reduce launch.

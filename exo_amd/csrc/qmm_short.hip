@@ -13,16 +13,17 @@
 //  * rows of an activation slot are 128 bytes; chunk c of row r sits at c ^ (r / 2 % 8), so that an
 //    operand read of 16 rows touches all 64 banks.
 //  * the activations of a step are in registers before the products start, so its slot is refilled at once.
-//  * every workgroup reads all activations (64 rows x 4096: 512 KB, as much as 100 rows of weights); where K is
-//    long and the columns are few, one tile of columns per CU, that is most of the launch.  Such
+//  * every workgroup reads all activations (64 rows x 4096: 512 KB, as much as 228 rows of 4-bit weights and
+//    scales); where K is long and the columns are few, one tile of columns per CU, that is most of the launch.  Such
 //    launches give a workgroup four tiles and a quarter of K, and a reduce launch adds the quarters.
 // 4-bit under 61 rows: pair of 14336x4096 52 -> 34 us (two products of 21, their reduce launches and the SwiGLU before:
 // 57), 6144x4096 23 -> 14, 4096x4096 17 -> 11, 4096x14336 30 -> 25; under 20 rows the pair 49 -> 26.
 // What bounds it: the dequantisation alone is 11 us of the pair's vector issue and a plain read of
 // its weights 12; the rest is the start (scales, first steps: two memory latencies), the
-// activations through L2 (7 us at a CU's 64 bytes per cycle) and the sums' way through LDS.
-// It replaces tiles of 32 or 64 x 256 with K split over workgroups, whose partial sums (up to 16 times the
-// output in float32) went to memory and came back through a second launch.
+// activations through L2 (3.4 us at a CU's 64 bytes per cycle) and the sums' way through LDS.
+// Where a launch is one round of such workgroups it replaces tiles of 32 or 64 x 256 with K split over
+// workgroups, whose partial sums (up to 16 times the output in float32) go to memory and come back through a
+// second launch; where not, those stay (exo_qmm_short_beats_split, exo_qmm_short_fits).
 #include "dequant.h"
 #include "qmm_short.h"
 
