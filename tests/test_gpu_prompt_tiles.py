@@ -42,8 +42,8 @@ def check(got, x, w, residual=None, what=""):
     assert not bad.any(), f"{what}: {int(bad.sum())} of {bad.numel()} outputs, first at {bad.nonzero()[0].tolist()}"
 
 
-# tiles of 256 x 256 with 6, 134 and 192 rows in the last one (two, six and six blocks of 32), whole rounds of
-# them and a last round in halves, the second of which holds no row; ragged columns
+# short ranges of K, which leave prompts to the 128-row tiles: 6, 134 and 192 rows in the last 256, whole rounds and
+# a nearly empty last one; ragged columns
 @pytest.mark.parametrize("M,N,K,bits", [(1030, 16400, 256, 4), (1030, 16397, 512, 8), (902, 16640, 256, 4),
                                         (960, 16400, 256, 8), (2048, 8192, 256, 4), (513, 32776, 256, 4)])
 def test_prompt_gemm_at_tile_edges(device, M, N, K, bits):
@@ -182,17 +182,24 @@ def test_prompt_attention_with_a_scale_of_nan_is_nan(device, T):
 
 
 # 17 to 64 rows: both sizes of the row tile, a step count below, at and above the eight waves, rows of scales that are no
-# whole 16-byte pieces (K of 64, 192, 832), one to seven column tiles per workgroup, K in four parts, ragged columns
-@pytest.mark.parametrize("M,N,K,bits", [(17, 4096, 64, 4), (32, 264, 192, 8), (33, 4099, 832, 4), (64, 12290, 512, 4),
-                                        (61, 8200, 1024, 8), (18, 16400, 512, 4), (48, 28680, 512, 4), (63, 4096, 8192, 4),
-                                        (31, 1030, 14336, 8), (64, 40, 8192, 4), (40, 128, 2048, 8), (20, 32, 32768, 4)])
-def test_short_prompt_gemm(device, M, N, K, bits):
+# whole 16-byte pieces (K of 64, 192, 832), one to seven column tiles per workgroup, K in four parts, ragged columns; and
+# where the tiles that split K are faster, those
+@pytest.mark.parametrize("M,N,K,bits,variant", [
+    (17, 4096, 64, 4, "qmm_short<4,one,2,1> parts=1"), (32, 264, 192, 8, "qmm_short<8,one,2,1> parts=1"), (33, 4099, 832, 4, "qmm_short<4,one,4,2> parts=1"),
+    (64, 12290, 512, 4, "qmm_short<4,one,4,4> parts=1"), (61, 8200, 1024, 8, "qmm_short<8,one,4,3> parts=1"), (18, 16400, 512, 4, "qmm_short<4,one,2,7> parts=1"),
+    (48, 28680, 512, 4, "qmm_kernel<4, 2, false, true, false, true>"), (63, 4096, 8192, 4, "qmm_short<4,one,4,4> parts=4"),
+    (31, 1030, 14336, 8, "qmm_kernel<8, 1, false, true, false, true, true>"), (31, 2050, 14336, 8, "qmm_short<8,one,2,4> parts=4"),
+    (64, 40, 8192, 4, "qmm_short<4,one,4,4> parts=4"), (40, 128, 2048, 8, "qmm_short<8,one,4,1> parts=1"),
+    (20, 32, 32768, 4, "qmm_kernel<4, 1, false, true, false, true, true>")])
+def test_short_prompt_gemm(device, M, N, K, bits, variant):
     q = packed(N, K, bits, M + N, device)
     g = torch.Generator(device=device).manual_seed(M)
     x = torch.randn(M, K, device=device, generator=g).bfloat16()
     r = torch.randn(M, N, device=device, generator=g).bfloat16()
     w = weights64(q)
-    check(ops.quantized_matmul(x, q), x, w, what=f"{M}x{N}x{K}")
+    got = ops.quantized_matmul(x, q)
+    assert native.last_variant() == variant, native.last_variant()
+    check(got, x, w, what=f"{M}x{N}x{K}")
     check(ops.quantized_matmul(x, q, residual=r), x, w, r, what=f"{M}x{N}x{K} with residual")
     check(ops.qmm(x, q), x, w, what=f"{M}x{N}x{K} without workspace")
 
@@ -234,7 +241,7 @@ def test_wide_pair_has_the_bits_of_two_products(device, M, N, K, bits):
 # a short launch of one round against one round, two against one, two against two; up to 8192 rows of weights; a long K
 @pytest.mark.parametrize("M,N,K,bits,short", [(33, 8200, 2048, 4, True), (33, 14336, 768, 8, False), (64, 16384, 1024, 4, False),
                                               (20, 20480, 2048, 4, True), (64, 20480, 1024, 4, False), (64, 8192, 512, 4, True),
-                                              (64, 1024, 12288, 4, False), (20, 1024, 12288, 4, True)])
+                                              (64, 1024, 12288, 4, False), (20, 1024, 12288, 4, True), (20, 8200, 32768, 4, True)])
 def test_short_prompt_pair_takes_the_faster_tile(device, M, N, K, bits, short):
     gate, up = packed(N, K, bits, M, device), packed(N, K, bits, N, device)
     x = torch.randn(M, K, device=device, generator=torch.Generator(device=device).manual_seed(K)).bfloat16()
@@ -242,6 +249,7 @@ def test_short_prompt_pair_takes_the_faster_tile(device, M, N, K, bits, short):
     got = ops.qmm_swiglu(x, gate, up, split_k=False)
     assert native.last_variant().startswith(f"qmm_short<{bits},pair" if short else f"qmm_kernel<{bits}, 2"), native.last_variant()
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    check(ops.qmm(x, gate), x, weights64(gate), what=f"gate {M}x{N}x{K}")
 
 
 @pytest.mark.parametrize("M,N,K,bits", [(9, 14336, 2048, 8), (16, 14336, 1024, 8), (12, 8192, 2048, 8), (9, 40, 64, 8), (16, 2050, 832, 4)])
