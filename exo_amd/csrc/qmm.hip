@@ -11,8 +11,7 @@
 //    so the weights do NOT go through LDS:
 //  * every wave loads the packed words of its own 64 weight rows straight into registers
 //    in the MFMA B-operand layout - lane (row, half) takes 16 B (4-bit) or 32 B (8-bit) =
-//    32 consecutive codes - and dequantises them there to bf16(fma(s, q, b)) with
-//    v_cvt_f32_ubyteN.  MFMA step t of a K step then covers k = 32*half + 8*t .. +8, and
+//    32 consecutive codes - and dequantises them there to bf16(fma(s, q, b)) (dequant.h).  MFMA step t of a K step then covers k = 32*half + 8*t .. +8, and
 //    the A operand is read from the activation tile at that same offset.  The two waves
 //    that share weight rows dequantise them twice; in exchange the LDS carries a third less
 //    traffic.
@@ -108,31 +107,16 @@ struct WRaw {
   bf16_t s, b;
 };
 
-// 8 codes -> the bf16x8 B operand of one MFMA step
+// word W of the codes of MFMA step t (8 bits: two of them)
 template <int BITS>
-__device__ __forceinline__ bf16x8_t dequant8(const WRaw<BITS>& r, int t, float s, float b) {
-  const uint32_t* w = reinterpret_cast<const uint32_t*>(&r.q[0]);
-  return BITS == 4 ? dequant_words8<4>(w[t], 0, s, b) : dequant_words8<8>(w[(2 * t) & 7], w[(2 * t + 1) & 7], s, b);
+__device__ __forceinline__ uint32_t code_word(const WRaw<BITS>& r, int t, int w) {
+  return reinterpret_cast<const uint32_t*>(&r.q[0])[BITS == 4 ? t : 2 * t + w];
 }
 
-// One 32-bit register (two bf16) of that operand: piece P = 0..3.  `lo`, `hi` are the two
-// source words prepared by dequant_words().
+// 8 codes -> the bf16x8 B operand of one MFMA step
 template <int BITS>
-__device__ __forceinline__ void dequant_words(const WRaw<BITS>& r, int t, uint32_t& lo, uint32_t& hi) {
-  if (BITS == 4) {
-    const uint32_t v = reinterpret_cast<const uint32_t*>(&r.q[0])[t];
-    lo = v & 0x0f0f0f0fu;         // even codes, one per byte
-    hi = (v >> 4) & 0x0f0f0f0fu;  // odd codes
-  } else {
-    lo = reinterpret_cast<const uint32_t*>(&r.q[0])[2 * t];
-    hi = reinterpret_cast<const uint32_t*>(&r.q[0])[2 * t + 1];
-  }
-}
-template <int BITS, int P>
-__device__ __forceinline__ uint32_t dequant_piece(uint32_t lo, uint32_t hi, float s, float b) {
-  if (BITS == 4) return pack_bf2(fmaf(s, ubyte_f<P>(lo), b), fmaf(s, ubyte_f<P>(hi), b));
-  const uint32_t v = P < 2 ? lo : hi;
-  return pack_bf2(fmaf(s, ubyte_f<(2 * P) & 3>(v), b), fmaf(s, ubyte_f<((2 * P) & 3) + 1>(v), b));
+__device__ __forceinline__ bf16x8_t dequant8(const WRaw<BITS>& r, int t, const GroupScale<BITS>& g) {
+  return dequant_words8<BITS>(code_word(r, t, 0), code_word(r, t, 1), g);
 }
 
 // MI = 32-row MFMA tiles per wave along M: the workgroup tile is (64*MI) x 128.
@@ -273,11 +257,9 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
   const bf16_t* sbase = p.s + s_off + (size_t)n0 * G;
   const bf16_t* bbase = p.b + s_off + (size_t)n0 * G;
   uint32_t woff[2], soff[2];
-  bool w_ok[2];
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     const int n = n0 + wn + (PAIR ? 0 : j * 32) + frow;
-    w_ok[j] = n < p.N;
     const uint32_t rel = (uint32_t)(min(n, p.N - 1) - n0);  // rows past N re-read the last one
     woff[j] = (rel * (uint32_t)wpr + kq * BITS) * 4;  // bytes; 32 codes = BITS words per half K step
     soff[j] = rel * (uint32_t)G * 2;
@@ -384,13 +366,10 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
 
   // multiply tile `buf` by the weights held (packed) in `st`
   auto multiply = [&](const WStage& st, int buf, const SBlock& sb, int e) {
-    float sc[2], bi[2];
+    GroupScale<BITS> gs[2];  // (rows past N: the last row's; their products are never written)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      sc[j] = SB4 ? pick(sb.s[j], e) : bf2f(st.w[j].s);
-      bi[j] = SB4 ? pick(sb.b[j], e) : bf2f(st.w[j].b);
-      if (!w_ok[j]) sc[j] = bi[j] = 0.f;
-    }
+    for (int j = 0; j < 2; ++j)
+      gs[j] = SB4 ? group_scale<BITS>(pick(sb.s[j], e), pick(sb.b[j], e)) : group_scale<BITS>(bf2f(st.w[j].s), bf2f(st.w[j].b));
     // MFMA step t covers k = 32*kq + 8*t .. +8 of the K step.  Software pipeline: the A
     // operands and the dequantised B operands of step t+1 are produced while the products
     // of step t run - a 32x32x16 MFMA occupies the matrix core for 8 passes, time for about
@@ -406,15 +385,11 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
     for (int i = 0; i < MI; ++i)
       a[0][i] = *reinterpret_cast<const bf16x8_t*>(arow + i * 32 * 128 + aoff[0]);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) bq[0][j] = __builtin_bit_cast(uint4, dequant8<BITS>(st.w[j], 0, sc[j], bi[j]));
+    for (int j = 0; j < 2; ++j) bq[0][j] = __builtin_bit_cast(uint4, dequant8<BITS>(st.w[j], 0, gs[j]));
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const int cur = t & 1, nxt = cur ^ 1;
-      uint32_t lo[2], hi[2];
-      if (t < 3) {
-#pragma unroll
-        for (int j = 0; j < 2; ++j) dequant_words<BITS>(st.w[j], t + 1, lo[j], hi[j]);
-      }
+      PieceCodes pc{};
 #pragma unroll
       for (int m = 0; m < 2 * MI; ++m) {
         const int i = m >> 1, j = m & 1;
@@ -426,13 +401,8 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
 #pragma unroll
           for (int u = 0; u < PER; ++u) {
             const int r8 = m * PER + u, jj = r8 >> 2;
-            uint32_t* dst = reinterpret_cast<uint32_t*>(&bq[nxt][jj]);
-            switch (r8 & 3) {
-              case 0: dst[0] = dequant_piece<BITS, 0>(lo[jj], hi[jj], sc[jj], bi[jj]); break;
-              case 1: dst[1] = dequant_piece<BITS, 1>(lo[jj], hi[jj], sc[jj], bi[jj]); break;
-              case 2: dst[2] = dequant_piece<BITS, 2>(lo[jj], hi[jj], sc[jj], bi[jj]); break;
-              default: dst[3] = dequant_piece<BITS, 3>(lo[jj], hi[jj], sc[jj], bi[jj]); break;
-            }
+            piece_codes<BITS>(pc, r8 & 3, code_word(st.w[jj], t + 1, 0), code_word(st.w[jj], t + 1, 1));
+            reinterpret_cast<uint32_t*>(&bq[nxt][jj])[piece_reg<BITS>(r8 & 3)] = piece_value<BITS>(r8 & 3, pc, gs[jj]);
           }
           if (m < MI)
             a[nxt][m] = *reinterpret_cast<const bf16x8_t*>(arow + m * 32 * 128 + aoff[t + 1]);
@@ -448,60 +418,40 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
   // barrier in front of this step waited for it.
   bf16x8_t a[2][MI];
   uint4 bq[2][2];
-  auto scales_of = [&](const SBlock& sb, int e, float (&sc)[2], float (&bi)[2]) {
+  GroupScale<BITS> gs[2];  // of the step whose operands are being made
+  auto scales_of = [&](const SBlock& sb, int e, GroupScale<BITS>(&g)[2]) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      sc[j] = w_ok[j] ? pick(sb.s[j], e) : 0.f;
-      bi[j] = w_ok[j] ? pick(sb.b[j], e) : 0.f;
-    }
+    for (int j = 0; j < 2; ++j) g[j] = group_scale<BITS>(pick(sb.s[j], e), pick(sb.b[j], e));
   };
   auto read_first = [&](auto ni, const WStage& st, int buf, const SBlock& sb, int e) {
     constexpr int NI = decltype(ni)::value;
-    float sc[2], bi[2];
-    scales_of(sb, e, sc, bi);
+    scales_of(sb, e, gs);
     const char* arow = tiles + buf * TILE_BYTES + (wm + frow) * 128;
 #pragma unroll
     for (int i = 0; i < NI; ++i) a[0][i] = *reinterpret_cast<const bf16x8_t*>(arow + i * 32 * 128 + aoff[0]);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) bq[0][j] = __builtin_bit_cast(uint4, dequant8<BITS>(st.w[j], 0, sc[j], bi[j]));
+    for (int j = 0; j < 2; ++j) bq[0][j] = __builtin_bit_cast(uint4, dequant8<BITS>(st.w[j], 0, gs[j]));
   };
-  auto multiply_on = [&](auto ni, const WStage& st, const WStage& sn, int buf, int bn, const SBlock& sb, int e, const SBlock& nb, int ne) {
+  auto multiply_on = [&](auto ni, const WStage& st, const WStage& sn, int buf, int bn, const SBlock& nb, int ne) {
     constexpr int NI = decltype(ni)::value;  // row blocks of 32 in use
-    float sc[2], bi[2], scn[2], bin[2];
-    scales_of(sb, e, sc, bi);
-    scales_of(nb, ne, scn, bin);
+    GroupScale<BITS> gn[2];
+    scales_of(nb, ne, gn);
     const char* arow = tiles + buf * TILE_BYTES + (wm + frow) * 128;
     const char* anext = tiles + bn * TILE_BYTES + (wm + frow) * 128;
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const int cur = t & 1, nxt = cur ^ 1, tn = (t + 1) & 3;
       const char* src = t < 3 ? arow : anext;
-      uint32_t lo = 0, hi = 0;
-      float f[2][2];
-      // register r8 of the next B operands in two parts that go into different slots: its two codes as
-      // floats, and their scaled values as two bf16
+      // the parts of piece r8 of the next B operands go into different slots
+      PieceCodes pc[2];  // (4 bits: of two pieces at a time)
       auto part_a = [&](int r8) {
-        if ((r8 & 3) == 0) dequant_words<BITS>(t < 3 ? st.w[r8 >> 2] : sn.w[r8 >> 2], tn, lo, hi);
-        float(&o)[2] = f[r8 & 1];
-        const uint32_t v = BITS == 4 ? lo : (r8 & 2) ? hi : lo;
-        if (BITS == 4) {
-          switch (r8 & 3) {
-            case 0: o[0] = ubyte_f<0>(lo), o[1] = ubyte_f<0>(hi); break;
-            case 1: o[0] = ubyte_f<1>(lo), o[1] = ubyte_f<1>(hi); break;
-            case 2: o[0] = ubyte_f<2>(lo), o[1] = ubyte_f<2>(hi); break;
-            default: o[0] = ubyte_f<3>(lo), o[1] = ubyte_f<3>(hi); break;
-          }
-        } else if (r8 & 1) {
-          o[0] = ubyte_f<2>(v), o[1] = ubyte_f<3>(v);
-        } else {
-          o[0] = ubyte_f<0>(v), o[1] = ubyte_f<1>(v);
-        }
+        const WRaw<BITS>& w = t < 3 ? st.w[r8 >> 2] : sn.w[r8 >> 2];
+        piece_codes<BITS>(pc[BITS == 4 ? (r8 >> 1) & 1 : r8 & 1], r8 & 3, code_word(w, tn, 0), code_word(w, tn, 1));
       };
       auto part_b = [&](int r8) {
         const int jj = r8 >> 2;
-        const float s1 = t < 3 ? sc[jj] : scn[jj], b1 = t < 3 ? bi[jj] : bin[jj];
-        const float(&o)[2] = f[r8 & 1];
-        reinterpret_cast<uint32_t*>(&bq[nxt][jj])[r8 & 3] = pack_bf2(fmaf(s1, o[0], b1), fmaf(s1, o[1], b1));
+        reinterpret_cast<uint32_t*>(&bq[nxt][jj])[piece_reg<BITS>(r8 & 3)] =
+            piece_value<BITS>(r8 & 3, pc[BITS == 4 ? (r8 >> 1) & 1 : r8 & 1], t < 3 ? gs[jj] : gn[jj]);
       };
 #pragma unroll
       for (int m = 0; m < 2 * NI; ++m) {
@@ -525,6 +475,8 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
         __builtin_amdgcn_sched_barrier(0);
       }
     }
+    gs[0] = gn[0];
+    gs[1] = gn[1];
   };
 
   // At K step k: the x tile of k is in LDS buffer k&1, the x tile of k+1 in registers
@@ -626,7 +578,7 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
         if (!GROUPED) load_x((u + XAHEAD) & 3, min(k0 + (u + XAHEAD) * BK, last), NI);
         load_w(wq[(u + AHEAD) & 3], kn);
         if (GROUPED) load_x((u + XAHEAD) & 3, min(k0 + (u + XAHEAD) * BK, last), NI);
-        multiply_on(ni, wq[u], wq[(u + 1) & 3], u, (u + 1) & 3, sbc, u, u < 3 ? sbc : sbn, (u + 1) & 3);
+        multiply_on(ni, wq[u], wq[(u + 1) & 3], u, (u + 1) & 3, u < 3 ? sbc : sbn, (u + 1) & 3);
         // tile k+2 is in LDS behind the barrier: the next step's last products read its first operands
         wait_vm(std::integral_constant<int, GROUPED ? NI + NW : (AHEAD - 2) * (NI + NW) + NW>{});
         __syncthreads();

@@ -210,23 +210,13 @@ __global__ __launch_bounds__(64 * kWaves) void qmm_short_kernel(const ShortParam
     // a tile its codes of step i + 2 are requested and a share of that step's activations.
     const int kn = k_of(i + 2);
     u32x4 bw[2];
-    uint32_t lo = 0, hi = 0;
-    float s = 0.f, b = 0.f;
+    PieceCodes pc{};
+    GroupScale<BITS> gs{};
     auto piece = [&](int q, int d) {  // two of an operand's eight values
       const int j = q >> 1, t = q & 1;
-      if (d == 0) {
-        if (t == 0) s = bf_lo(sc[j]), b = bf_hi(sc[j]);
-        if (BITS == 4)
-          lo = w[j].q[t] & 0x0f0f0f0fu, hi = (w[j].q[t] >> 4) & 0x0f0f0f0fu;
-        else
-          lo = w[j].q[(2 * t) & (WORDS - 1)], hi = w[j].q[(2 * t + 1) & (WORDS - 1)];
-      }
-      bw[q & 1][d] = BITS == 4 ? (d == 0   ? pack_bf2(fmaf(s, ubyte_f<0>(lo), b), fmaf(s, ubyte_f<0>(hi), b))
-                                  : d == 1 ? pack_bf2(fmaf(s, ubyte_f<1>(lo), b), fmaf(s, ubyte_f<1>(hi), b))
-                                  : d == 2 ? pack_bf2(fmaf(s, ubyte_f<2>(lo), b), fmaf(s, ubyte_f<2>(hi), b))
-                                           : pack_bf2(fmaf(s, ubyte_f<3>(lo), b), fmaf(s, ubyte_f<3>(hi), b)))
-                               : (d & 1) ? pack_bf2(fmaf(s, ubyte_f<2>(d < 2 ? lo : hi), b), fmaf(s, ubyte_f<3>(d < 2 ? lo : hi), b))
-                                         : pack_bf2(fmaf(s, ubyte_f<0>(d < 2 ? lo : hi), b), fmaf(s, ubyte_f<1>(d < 2 ? lo : hi), b));
+      if (d == 0 && t == 0) gs = group_scale<BITS>(bf_lo(sc[j]), bf_hi(sc[j]));
+      piece_codes<BITS>(pc, d, w[j].q[BITS == 4 ? t : (2 * t) & (WORDS - 1)], w[j].q[BITS == 4 ? t : (2 * t + 1) & (WORDS - 1)]);
+      bw[q & 1][piece_reg<BITS>(d)] = piece_value<BITS>(d, pc, gs);
     };
 #pragma unroll
     for (int d = 0; d < 4; ++d) piece(0, d);

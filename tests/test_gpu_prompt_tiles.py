@@ -268,3 +268,24 @@ def test_nine_to_sixteen_rows(device, M, N, K, bits):
     native.check(native.load().exo_qmm_ws(x.data_ptr(), gate.weight.data_ptr(), gate.scales.data_ptr(), gate.biases.data_ptr(), r.data_ptr(),
                                           y.data_ptr(), ws.data_ptr(), ws.numel(), M, N, K, bits, 64, torch.cuda.current_stream().cuda_stream), "qmm")
     check(y, x, weights64(gate), r, what=f"{M}x{N}x{K} with residual")
+
+
+# rows of the short GEMM, of the 128-row and of the 256-row tile; K whose scales come one by one, and in fours
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("M,N,K", [(20, 64, 64), (61, 2048, 256), (100, 200, 192), (200, 264, 256), (300, 8192, 768), (1030, 12288, 4096)])
+def test_products_with_unit_rows_are_the_weights(device, M, N, K, bits):
+    """The operand that a kernel makes of codes is bf16(scale * code + bias) bit for bit, from subnormal scales to
+    those of 2^100: products with rows of one 1 are the weights themselves."""
+    g = torch.Generator(device=device).manual_seed(N + bits)
+    q = packed(N, K, bits, M, device)
+    e = torch.randint(-133, 100, q.scales.shape, device=device, generator=g)
+    e[: N // 2] = torch.randint(-12, 2, q.scales[: N // 2].shape, device=device, generator=g)
+    big = torch.ldexp(torch.rand(q.scales.shape, device=device, generator=g).double() + 0.5, e)
+    s = torch.where(torch.rand(e.shape, device=device, generator=g) < 0.5, -big, big).bfloat16()
+    b = (-big * 2.0 ** (bits - 1)).bfloat16()
+    q = QuantizedWeight(q.weight, s, b, bits)
+    at = torch.randint(0, K, (M,), device=device, generator=g)
+    x = torch.zeros(M, K, device=device, dtype=torch.bfloat16)
+    x[torch.arange(M, device=device), at] = 1
+    # (a sum adds zeros to the weight; +0 where it is -0)
+    assert torch.equal(ops.quantized_matmul(x, q).double(), weights64(q).T[at])
