@@ -27,11 +27,12 @@
 //    wave.  Nothing is dequantised twice and half as much per product as on the 128-row tile,
 //    and with one wave per SIMD the products of a K step are kept fed by that wave alone:
 //    the operands of the next product block, one dequantised register's half and every other slot an LDS
-//    read, ride between two MFMAs, across the barrier too (see multiply_on).  4096x14336 8-bit
-//    under 4096 rows 471 -> 402 us (1197 TFLOP/s), pair of 14336x4096 949 -> 814 (1182); 4-bit pair
-//    under 2047 rows 439 -> 411 (1169).  Over a short K it loses (see prefer_big).  What bounds it: the matrix cores are busy 56 % of the
-//    cycles; 20 % go into the wait for the tile requested a step ahead and the barrier, the rest
-//    into slots with more vector work than an MFMA covers.
+//    read, ride between two MFMAs, across the barrier too (see multiply_on), and so do the step's
+//    requests, one at a time: sent together at its start, 40 KB of them fill the CU's address unit (16 cycles
+//    per KB) and the four waves stood 600 of a step's 3300 cycles.  4096x14336 8-bit under 4096 rows 411 -> 377 us
+//    (1276 TFLOP/s), pair of 14336x4096 844 -> 779 (1235); 4-bit pair under 2047 rows 414 -> 396 (1214).
+//    Over a short K the tile loses (see prefer_big).  What bounds it: the clock, which falls from 2.2 to 1.7 GHz
+//    under the products with their operands' traffic, and slots with more vector work than an MFMA covers.
 //  * few output tiles: blockIdx.z splits K; float32 partial tiles and a small reduce launch.
 //  * 9 to 64 rows belong to qmm_short.hip where its launch is one round of workgroups over a K that is not
 //    long (exo_qmm_short_beats_split).  Otherwise up to 32 rows (64 on matrices of 8192 rows or more) have the
@@ -208,7 +209,11 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
   constexpr int SLOTS = 2;  // activation tiles in LDS
   // (the grouped wide tile leaves through the staging epilogue: four waves x 32*MI rows)
   constexpr int XS_ROWS = WIDE ? 2 * BM : BM;  // (wide: room for the ring's four tiles)
-  __shared__ __attribute__((aligned(16))) bf16_t xs[KH ? 2 * SLOTS : SLOTS][XS_ROWS * LDS_STRIDE];
+  constexpr int XS_BYTES = (KH ? 2 * SLOTS : SLOTS) * XS_ROWS * LDS_STRIDE * 2;
+  // ONE array, the grouped mode's row list behind the tiles: with a second array in LDS the compiler makes each
+  // read of a tile wait for all requests into LDS (pair of 768x2048 under 8184 pairs of 128 experts 95 -> 135 us)
+  __shared__ __attribute__((aligned(16))) char lds[XS_BYTES + (GROUPED ? BM * 4 : 0)];
+  bf16_t* const xs = reinterpret_cast<bf16_t*>(lds);
 
   // (a ring of four activation tiles: below)
   constexpr bool RING = WIDE && SB4 && (BITS == 4 || kRing8) && (MI >= 4 || DEEP);
@@ -232,7 +237,7 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
     m_end = min(m_end, m0 + (half >= 0 ? BM / 2 : BM));
   }
   size_t w_off = 0, s_off = 0;
-  __shared__ int row_pair[GROUPED ? BM : 1];  // pair index of every row of the tile
+  int* const row_pair = reinterpret_cast<int*>(lds + XS_BYTES);  // grouped: pair index of every row of the tile
   if (GROUPED) {
     const int32_t* ti = p.tiles + 3 * (size_t)blockIdx.y;
     const int e = ti[0];
@@ -269,8 +274,6 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
   // (pair mode: a second set of descriptors for the up matrix, column tile 1)
   constexpr int ND = PAIR ? 2 : 1;
   const __amdgpu_buffer_rsrc_t rx = make_rsrc(p.x);
-  const u32x4 rx4 = {(uint32_t)__builtin_amdgcn_readfirstlane((int)(uintptr_t)p.x),
-                     (uint32_t)__builtin_amdgcn_readfirstlane((int)((uintptr_t)p.x >> 32)) & 0xffffu, ~0u, 0x00020000u};
   __amdgpu_buffer_rsrc_t rw[ND], rs[ND], rb[ND];
   rw[0] = make_rsrc(wbase);
   rs[0] = make_rsrc(sbase);
@@ -304,31 +307,29 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
   // order.  Completion is counted by vmcnt.
   constexpr int TILE_BYTES = BM * 128;
   // (a team's tiles: two, or the four of the ring)
-  char* const tiles = reinterpret_cast<char*>(&xs[0][0]) + team * ((KH && WIDE ? 4 : SLOTS) * TILE_BYTES);
+  char* const tiles = lds + team * ((KH && WIDE ? 4 : SLOTS) * TILE_BYTES);
+  auto load_x1 = [&](int buf, int k0, int r) {
+    char* const to = tiles + buf * TILE_BYTES + (wave * 64 + kThreads * r) * 16;
+    load_to_lds16(rx, to, xoff[r], k0 * 2);
+  };
   auto load_x = [&](int buf, int k0, int n) {
 #pragma unroll
-    for (int r = 0; r < n; ++r) {
-      char* const to = tiles + buf * TILE_BYTES + (wave * 64 + kThreads * r) * 16;
-      // (a step of an expert's few rows does not cover the compiler's wait, pair of 768x2048 under 8184 pairs of
-      // 128 experts 113 -> 99 us, 2048x768 62.5 -> 58.5; the 256-row tile's step does, 409 -> 421)
-      if constexpr (RING && GROUPED)
-        load_to_lds16_untracked(rx4, (lds_char)to, xoff[r], k0 * 2);
-      else
-        load_to_lds16(rx, to, xoff[r], k0 * 2);
-    }
+    for (int r = 0; r < n; ++r) load_x1(buf, k0, r);
   };
   // s_waitcnt vmcnt(n) alone (the other counters at "no wait")
   auto wait_vm = [](auto n) {
     constexpr int N = decltype(n)::value;
     __builtin_amdgcn_s_waitcnt((N & 15) | 0x0F70 | ((N >> 4) << 14));
   };
+  auto load_w1 = [&](WStage& st, int k0, int j, int i) {
+    st.w[j].q[i] = __builtin_bit_cast(
+        uint4, __builtin_amdgcn_raw_buffer_load_b128(rw[PAIR ? j : 0], woff[j] + i * 16, k0 * BITS / 8, 0));
+  };
   auto load_w = [&](WStage& st, int k0) {
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
 #pragma unroll
-      for (int i = 0; i < BITS / 4; ++i)
-        st.w[j].q[i] = __builtin_bit_cast(
-            uint4, __builtin_amdgcn_raw_buffer_load_b128(rw[PAIR ? j : 0], woff[j] + i * 16, k0 * BITS / 8, 0));
+      for (int i = 0; i < BITS / 4; ++i) load_w1(st, k0, j, i);
       if (!SB4) {
         st.w[j].s = (bf16_t)__builtin_amdgcn_raw_buffer_load_b16(rs[PAIR ? j : 0], soff[j], (k0 >> 6) * 2, 0);
         st.w[j].b = (bf16_t)__builtin_amdgcn_raw_buffer_load_b16(rb[PAIR ? j : 0], soff[j], (k0 >> 6) * 2, 0);
@@ -432,7 +433,7 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
 #pragma unroll
     for (int j = 0; j < 2; ++j) bq[0][j] = __builtin_bit_cast(uint4, dequant8<BITS>(st.w[j], 0, gs[j]));
   };
-  auto multiply_on = [&](auto ni, const WStage& st, const WStage& sn, int buf, int bn, const SBlock& nb, int ne) {
+  auto multiply_on = [&](auto ni, const WStage& st, const WStage& sn, int buf, int bn, const SBlock& nb, int ne, auto request) {
     constexpr int NI = decltype(ni)::value;  // row blocks of 32 in use
     GroupScale<BITS> gn[2];
     scales_of(nb, ne, gn);
@@ -472,6 +473,7 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
           }
         }
         if (m & 1) a[nxt][i] = *reinterpret_cast<const bf16x8_t*>(src + i * 32 * 128 + aoff[tn]);
+        request(t * 2 * NI + m);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -559,7 +561,7 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
     SBlock sbc, sbn;
     const int last = ke - BK;
     load_sb(sbn, kb >> 8);
-    constexpr int XAHEAD = GROUPED ? 3 : AHEAD;
+    constexpr int XAHEAD = 3;
 #pragma unroll
     for (int u = 0; u < AHEAD; ++u) load_w(wq[u], min(kb + u * BK, last));
 #pragma unroll
@@ -572,16 +574,24 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
       load_sb(sbn, min((k0 >> 8) + 1, (ke >> 8) - 1));
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const int kn = min(k0 + (u + AHEAD) * BK, last);
-        // (the compiler's own wait for the weights of a step counts weights alone: with the activations
-        // behind them it leaves four of the youngest out, before them none)
-        if (!GROUPED) load_x((u + XAHEAD) & 3, min(k0 + (u + XAHEAD) * BK, last), NI);
-        load_w(wq[(u + AHEAD) & 3], kn);
-        if (GROUPED) load_x((u + XAHEAD) & 3, min(k0 + (u + XAHEAD) * BK, last), NI);
-        multiply_on(ni, wq[u], wq[(u + 1) & 3], u, (u + 1) & 3, u < 3 ? sbc : sbn, (u + 1) & 3);
-        // tile k+2 is in LDS behind the barrier: the next step's last products read its first operands
-        wait_vm(std::integral_constant<int, GROUPED ? NI + NW : (AHEAD - 2) * (NI + NW) + NW>{});
-        __syncthreads();
+        const int kw = min(k0 + (u + AHEAD) * BK, last), kx = min(k0 + (u + XAHEAD) * BK, last);
+        multiply_on(ni, wq[u], wq[(u + 1) & 3], u, (u + 1) & 3, u < 3 ? sbc : sbn, (u + 1) & 3, [&](int slot) {
+          // (a whole step's requests at once are more than the address unit takes in: the wave stands until
+          // they have left, and its matrix core with it)
+#pragma unroll
+          for (int r = 0; r < NW; ++r)
+            if (slot == (!GROUPED ? r * (8 * NI) / (NW + NI) : BITS == 4 ? r * (4 * NI) / NW : 0)) load_w1(wq[(u + AHEAD) & 3], kw, r / (NW / 2), r % (NW / 2));
+#pragma unroll
+          for (int r = 0; r < NI; ++r)  // (grouped: behind the last wait for weights, which does not count these)
+            if (slot == (GROUPED ? 7 * NI + r : (NW + r) * (8 * NI) / (NW + NI))) load_x1((u + XAHEAD) & 3, kx, r);
+        });
+        // Tile k+2 is in LDS behind the barrier: the next step's last products read its first operands.  What was
+        // requested in this step may still be out - but the fence of __syncthreads() would wait for every
+        // request into LDS, so that the barrier stands alone.  (Reads of tile k, whose memory the next
+        // step's requests fill, have been multiplied.)
+        wait_vm(std::integral_constant<int, NI + NW>{});
+        asm volatile("s_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);  // the repeats requested past the end: landed before
@@ -639,7 +649,7 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
   if (KH) {
     // the second team's sums: through LDS (lane-contiguous floats per accumulator register),
     // added to the first team's, which goes on alone
-    float* ex = reinterpret_cast<float*>(&xs[0][0]);
+    float* ex = reinterpret_cast<float*>(lds);
     __syncthreads();  // both teams have finished reading their activation tiles
     if (team == 1) {
 #pragma unroll
@@ -695,7 +705,7 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
   // and then copies whole rows out with 16-byte stores (residual added on the way).
   if (!KH) __syncthreads();  // every wave has finished reading the last activation tile
   constexpr int TS = 64 + 8;  // row stride of the staging tile (bf16)
-  bf16_t* stage = &xs[0][0] + (size_t)wave * (32 * MI) * TS;
+  bf16_t* stage = xs + (size_t)wave * (32 * MI) * TS;
   if (PAIR) {
     // SwiGLU of the bf16-rounded projections (the rounding points of two GEMMs followed by
     // the elementwise kernel), then rows of 32 columns out
