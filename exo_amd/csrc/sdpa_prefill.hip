@@ -141,21 +141,18 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, SPLIT ? 1 : 2) void fa_prefill_k
   };
   const u32x4 rk = rsrc(p.k + head_off), rv = rsrc(p.v + head_off);
   const int lrow = tid / VEC, lslot = tid % VEC;  // (row of load i: lrow + i * 256 / VEC, a multiple of 16 further)
-  const uint32_t koff = lrow * ROW + (lslot ^ (D == 128 ? lrow & 15 : (lrow >> 1) & 7)) * 16;
-  const uint32_t voff = lrow * ROW + (lslot ^ (D == 128 ? (lrow & 3) << 2 : ((lrow >> 1) & 1) << 2)) * 16;
+  const uint32_t koff = (lslot ^ (D == 128 ? lrow & 15 : (lrow >> 1) & 7)) * 16;
+  const uint32_t voff = (lslot ^ (D == 128 ? (lrow & 3) << 2 : ((lrow >> 1) & 1) << 2)) * 16;
+  // piece i of a wave's share of key tile kt (past the last one: that one again); rows past the end of the cache: its last
+  // row again (they are masked)
+  auto load_piece = [&](u32x4 r, uint32_t off, int tile, int kt, int i) {
+    const int row0 = (t_first + min(kt, max(n_tiles, 1) - 1)) * kBN;
+    const uint32_t at = min(lrow * ROW, (p.S_max - 1 - row0 - i * (256 / VEC)) * ROW) + off;
+    load_to_lds16_untracked(r, lds + tile * TILE + wave * 1024 + i * 4096, at, row0 * ROW + i * 4096);
+  };
   auto load_tile = [&](u32x4 r, uint32_t off, int tile, int kt) {
-    const int row0 = (t_first + kt) * kBN;
-    const lds_char to = lds + tile * TILE + wave * 1024;
-    if (row0 + kBN <= p.S_max) {
 #pragma unroll
-      for (int i = 0; i < LOADS; ++i) load_to_lds16_untracked(r, to + i * 4096, off, row0 * ROW + i * 4096);
-    } else {  // rows past the end of the cache: its last row again (they are masked)
-#pragma unroll
-      for (int i = 0; i < LOADS; ++i) {
-        const int row = lrow + i * (256 / VEC), over = max(0, row0 + row - (p.S_max - 1));
-        load_to_lds16_untracked(r, to + i * 4096, off + (row0 + i * (256 / VEC) - over) * ROW, 0);
-      }
-    }
+    for (int i = 0; i < LOADS; ++i) load_piece(r, off, tile, kt, i);
   };
 
   // A-operand row r of a 32-key sub-tile holds this key, so that D registers 8s..8s+7
@@ -267,6 +264,11 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, SPLIT ? 1 : 2) void fa_prefill_k
                                                           __builtin_bit_cast(bf16x8_t, qreg[i >> 1]), sn[i & 1], 0, 0, 0);
       a[(i + AHEAD) & 3] = i + AHEAD < 2 * STEPS ? read_k(kt_lds, i + AHEAD) : read_v(vt_lds, i + AHEAD - 2 * STEPS);
       stage(i);
+      if (SPLIT && i % (STEPS / LOADS) == 0) {
+        const int l = i / (STEPS / LOADS);
+        if (l & 1) load_piece(rv, voff, 2 + (par ^ 1), kt + 1, l >> 1);
+        else load_piece(rk, koff, par, kt + 2, l >> 1);
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
     stage(2 * STEPS);
@@ -339,18 +341,25 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, SPLIT ? 1 : 2) void fa_prefill_k
   // K of tile kt + 2 goes where K of kt was, V of kt + 1 where V of kt - 1 was: both last read before the barrier
   // that ended the previous tile, both complete at the one that ends this tile.  (A step past the wave's
   // or the workgroup's last tile multiplies what lies in LDS and uses none of it.)
+  // SPLIT: the requests of a tile stand one by one between its products; together at its start they fill the CU's address
+  // unit (16 cycles per KB) and the wave stands (1023 tokens of 32 / 4 heads 25.3 -> 24.3 us, 300 behind 2000 of 64 / 4
+  // 42.8 -> 40.2, 512 behind 9000 with heads of 64 97.7 -> 90.7).  Of two workgroups per CU one goes on meanwhile: the same
+  // there is 1 to 3 % on some shapes, but 1500 tokens of 64 / 4 heads take 64 -> 66, with two tiles requested past the last.
   for (int kt = 0; !one_tile && kt < n_iter; kt += 2) {
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
-    if (kt + 2 < n_tiles) load_tile(rk, koff, 0, kt + 2);
-    if (kt + 1 < n_tiles) load_tile(rv, voff, 3, kt + 1);
-    if (kt < n_mine && kt < n_tiles) tile_step(s0, s1, kt, 0);
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
-    if (kt + 3 < n_tiles) load_tile(rk, koff, 1, kt + 3);
-    if (kt + 2 < n_tiles) load_tile(rv, voff, 2, kt + 2);
-    if (kt + 1 < n_mine && kt + 1 < n_tiles) tile_step(s1, s0, kt + 1, 1);
+    auto turn = [&](floatx16(&s)[2], floatx16(&sn)[2], int kt, int par) {
+      const bool mine = kt < n_mine && kt < n_tiles;
+      __builtin_amdgcn_s_waitcnt(0x0F70);
+      __syncthreads();
+      if (!SPLIT || !mine) {
+        if (SPLIT || kt + 2 < n_tiles) load_tile(rk, koff, par, kt + 2);
+        if (SPLIT || kt + 1 < n_tiles) load_tile(rv, voff, 2 + (par ^ 1), kt + 1);
+      }
+      if (mine) tile_step(s, sn, kt, par);
+    };
+    turn(s0, s1, kt, 0);
+    turn(s1, s0, kt + 1, 1);
   }
+  if (SPLIT) __builtin_amdgcn_s_waitcnt(0x0F70);  // the repeats requested past the end
   float l_run = l0 + l1;
   l_run += __shfl_xor(l_run, 32, 64);
   if (SPLIT) {
