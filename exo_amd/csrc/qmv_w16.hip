@@ -1,36 +1,43 @@
 // Fused dequant-GEMV for up to 16 activation rows on v_mfma_f32_16x16x32_bf16 (4-bit codes).
 //
 // The instruction multiplies A[16][32] by B[32][16]: lane l holds A[l%16][8*(l/16) .. +8],
-// B[8*(l/16) .. +8][l%16], and D[4*(l/16) + r][l%16] in register r.  Here A is the activations
-// (row = activation row m), B a block of 16 weight rows (column = weight row j), so a lane's
-// four results belong to ONE weight row: scale and bias of a quantisation group are one value
-// per lane.
+// B[8*(l/16) .. +8][l%16], and D[4*(l/16) + r][l%16] in register r.  Here A is the activations,
+// B a block of 16 weight rows (column = weight row j), so a lane's four results belong to ONE
+// weight row: scale and bias of a quantisation group are one value per lane.
 //  * a wave instruction loads 16 rows x 64 contiguous bytes (128 codes = two groups of a row):
 //    lane (lane/4, lane%4) takes 16-byte chunk lane%4 of row lane/4, so that the four lanes of
-//    a quad read 64 contiguous bytes.  A product wants 8 codes (one word) of row j in lane
-//    (j, kg): the words change lanes through the LDS crossbar (ds_bpermute_b32, no LDS memory)
-//    when the block is consumed - two permutes and one select per product, because the four
-//    K slots of a product must come from one group (= two chunks x four words).
+//    a quad read 64 contiguous bytes.  A product wants words of row j in the lanes (j, kg): they
+//    change lanes through 1 KB of the wave's own LDS, one 16-byte write and one or two reads per
+//    lane (chunk c of row r at c ^ r/4 % 4: all 64 banks in each).  (Through the crossbar, two
+//    ds_bpermute_b32 and a select per product, the same took 1.5 us of the pair's 20.)
+//  * more than eight rows (WIDE): lane (j, kg) takes 8 bytes of each of the slice's two groups, so
+//    that a product's four K slots belong to one group.
+//  * up to eight rows: lane (j, kg) takes chunk kg, of whose words K slots 0 and 1 belong to the
+//    first group and 2 and 3 to the second.  The operand A keeps them apart: its rows 0..7 are the
+//    activation rows with zeros in slots 2 and 3, its rows 8..15 the same with zeros in slots 0 and 1.
+//    Lanes kg < 2 get the first group's sums and the others the second's: no lane scales rows that
+//    do not exist.  The halves of the wave are added once per row block.
 //  * a wave owns SL such 64-byte slices of every row block of its workgroup; the matching
-//    activations stay in registers in operand order for the whole launch.  The waves of a
-//    workgroup together cover K; their partial sums meet in LDS once per phase of row blocks.
+//    activations stay in registers in operand order for the whole launch.  They are loaded as
+//    whole runs of a row, normalised there, and change lanes through the same LDS region.  The waves of
+//    a workgroup together cover K; their partial sums meet in LDS once, at the end.
 //  * codes become (128+nibble) bf16 pairs with one v_and_or_b32 each (exact).  Per group:
 //      acc += s * D + (b - 128 s) * Sx        D = sum (128+q) x,  Sx = sum x   (float32)
-//  * DEPTH row blocks of weights are in flight per wave (register buffers in rotation); every
-//    refill is issued whether or not a block is left (past the end it is out of the buffer's
-//    range and moves no data), so that the number of loads in flight at each wait is a constant.
+//    Sx comes out of products with a column of ones, in the lanes and registers of D.
+//  * DEPTH row blocks of weights are in flight per wave (register buffers in rotation), all of
+//    them requested right behind the activations.  Every refill is issued whether or not a block is
+//    left (past the end all lanes read the same 16 bytes), so that the number of loads in flight at
+//    each wait is a constant.
+// At 8 | 16 rows: pair of 14336x4096 20.2 | 22.2 -> 16.4 | 19.4 us (one row: 15.3, a plain read of its weights 12.3),
+// 6144x4096 11.4 | 12.8 -> 8.9 | 11.2, 4096x4096 7.6 | 8.8 -> 6.1 | 7.3, 4096x14336 15.8 | 17.6 -> 13.8 | 16.0,
+// 128256x4096 76 | 91 -> 62 | 79, pair of 8192x2048 at 8 rows 10.1 -> 8.0, 2048x4096 7.2 | 8.3 -> 5.2 | 6.1.
+// What bounds it: the way to the first product (activations, norm, lane changes: 3 us), after which the pair
+// streams at 5 TB/s; with K split, 3 us of hand-over; at 16 rows vector issue (two epilogues per slice).
 #include "../../include/exo_mi355x.h"
 #include "common.h"
 #include "qmv_internal.h"
 
 namespace {
-
-#ifndef EXO_W16_PAIR8
-#define EXO_W16_PAIR8 1  // the (gate, up) pair in blocks of 8 rows of both matrices where that fits
-#endif
-#ifndef EXO_W16_ABL
-#define EXO_W16_ABL 0  // timing-only ablations (wrong results): 1 no products, 2 no lane permutation, 4 no group epilogue, 8 no unpacking
-#endif
 
 struct W16Params {
   const bf16_t* x;       // [M, K]
@@ -44,10 +51,10 @@ struct W16Params {
   int M, N, K;
   int row_bytes;  // K / 2
   int G;          // K / 64
-  int blocks;     // N / 16
-  int ph;         // row blocks per workgroup at most (LDS holds their partial sums)
-  int lw;         // lanes of a wave that hold results: 16 * ceil(M / 4)
-  int red_bytes;  // LDS bytes of the partial sums; the staged scales and biases follow
+  int blocks;     // N / 16 (pair: N / 8)
+  int wave_bytes; // LDS of a wave: lane changes, partial sums
+  int wide_pieces;  // a row's scales are whole pieces of eight groups, else of two
+  int piece_mul;    // 65536 / pieces of a row + 1
   // K split over `kparts` workgroups per group of row blocks (long rows: the activations of
   // a whole row would not fit the registers): workgroup i takes part i % kparts, Gp groups
   // of every row; float32 partial results meet in `part`, the last workgroup of a group to
@@ -56,6 +63,16 @@ struct W16Params {
   float* part;    // [kparts][M][N]
   int* counters;  // [block groups], zero between launches
 };
+
+constexpr int kLdsMax = 160 * 1024 - 2048 - 64;  // (beside the sums of squares)
+constexpr int kRowPad = 16;                      // bytes between rows of staged scales: 16 rows, 64 banks
+
+// bytes through which a wave's chunks change lanes: all slices at once where the LDS allows it
+constexpr int turn_bytes(bool wide, int sl) { return (wide ? 1 : sl) * 1024; }
+// staged activation rows: 16, or eight and one of zeros
+constexpr int x_bytes(bool wide, int sl) { return (wide ? 16 : 9) * (sl * 256); }
+// partial sums of a row block
+constexpr int sum_bytes(bool wide) { return wide ? 1024 : 512; }
 
 __device__ __forceinline__ void st_dev(float* p, float v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -76,63 +93,61 @@ __device__ __forceinline__ void norm8(uint4& xv, const uint4& wv, float inv) {
   xv.w = pack_bf2(bf_lo(xv.w) * inv * bf_lo(wv.w), bf_hi(xv.w) * inv * bf_hi(wv.w));
 }
 // the 8 activations of one packed word in the order of the unpacked nibble pairs:
-// (x0,x4),(x1,x5),(x2,x6),(x3,x7); `sum` = their sum
-__device__ __forceinline__ uint4 pair_order(const uint4& xv, float& sum) {
+// (x0,x4),(x1,x5),(x2,x6),(x3,x7)
+__device__ __forceinline__ uint4 pair_order(const uint4& xv) {
   uint4 o;
   o.x = __builtin_amdgcn_perm(xv.z, xv.x, 0x05040100u);
   o.y = __builtin_amdgcn_perm(xv.z, xv.x, 0x07060302u);
   o.z = __builtin_amdgcn_perm(xv.w, xv.y, 0x05040100u);
   o.w = __builtin_amdgcn_perm(xv.w, xv.y, 0x07060302u);
-  sum = (bf_lo(o.x) + bf_hi(o.x)) + (bf_lo(o.y) + bf_hi(o.y)) + (bf_lo(o.z) + bf_hi(o.z)) +
-        (bf_lo(o.w) + bf_hi(o.w));
   return o;
 }
+__device__ __forceinline__ floatx4 mfma(const uint4& a, const uint4& b, const floatx4& c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+}
+// a of lanes l and l + 32 added in lane l, b of both in lane l + 32
+__device__ __forceinline__ float fold_halves(float a, float b) {
+  const auto t = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
+  const uint32_t lo = t[0], hi = t[1];
+  return __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
+}
+// what the lanes of a wave wrote to LDS is read by others of its lanes behind this (its LDS operations complete in order)
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+// a workgroup's LDS writes before it are visible behind it; requests to memory stay in flight
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+  asm volatile("s_barrier" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
 
-template <int SL>
-struct SbWord;  // (scale or bias) of the 2*SL groups of a wave's slices: SL words of two bf16
-template <>
-struct SbWord<1> {
-  uint32_t v[1];
-  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, int vo, int so) {
-    v[0] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, vo, so, 0);
-  }
-};
-template <>
-struct SbWord<2> {
-  uint32_t v[2];
-  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, int vo, int so) {
-    const auto t = __builtin_amdgcn_raw_buffer_load_b64(r, vo, so, 0);
-    const uint2 u = __builtin_bit_cast(uint2, t);
-    v[0] = u.x;
-    v[1] = u.y;
-  }
-};
-
-// NMAT matrices (2: the (gate, up) pair with SwiGLU), SL 64-byte slices of K per wave, DEPTH
-// row blocks in flight per wave.
-// NORM: fused RMSNorm of the activations.
-// SBLDS: the scales and biases of ALL the workgroup's rows are staged in LDS in front of the
-// loop, with whole-line loads (one 16-byte chunk per thread and array).  Loaded per block by
-// the lanes that need them - 8 bytes each out of 16 different lines per instruction, every
-// line touched again by each of the 16 waves - they cost 4.5 of the 24 us of the 14336x4096
-// pair (measured with the loads taken out).  Needs K a multiple of 512 and LDS for them beside
-// the partial sums (up to 8 activation rows).
+// WIDE: more than eight activation rows.  SL: 64-byte slices of K per wave.  DEPTH: row blocks in
+// flight per wave (1: the launch gives a workgroup no more than one).  NORM: fused RMSNorm of the activations.
 // KSPLIT: K split over several workgroups (single matrix, no fused norm).  An instance of its
 // own: compiled into the others, the hand-over code costs them 0.5 us per launch untaken.
-// P8 (the (gate, up) pair as ONE operand block: NMAT == 1, staged scales): the 16 columns of a
-// product are 8 rows of the gate matrix and the same 8 rows of the up matrix.  A workgroup's
-// share is then counted in blocks of 8 rows of both - 14336 rows are 1792 blocks, seven for each
-// of 256 workgroups, where blocks of 16 rows leave half the workgroups with four and half with
-// three.  Per-lane addresses (two matrices in one load instruction), clamped to the
-// workgroup's last block instead of range-checked.
-template <int NMAT, int SL, int DEPTH, bool NORM, bool SBLDS, bool KSPLIT = false, bool P8 = false>
+// PAIR: a (gate, up) pair with SwiGLU; the 16 columns of a product are 8 rows of the gate matrix and the
+// same 8 rows of the up matrix.  A workgroup's share is then counted in blocks of 8 rows of both -
+// 14336 rows are 1792 blocks, seven for each of 256 workgroups, where blocks of 16 rows leave
+// half the workgroups with four and half with three.
+// The scales and biases of ALL the workgroup's rows are staged in LDS in front of the loop, as pairs
+// and with whole-line loads (one piece per thread and array).  Loaded per block by the lanes
+// that need them - 8 bytes each out of 16 different lines per instruction, every line touched again
+// by each of the 16 waves - they cost 4.5 of 24 us of the 14336x4096 pair (measured with the loads
+// taken out).
+template <bool WIDE, int SL, int DEPTH, bool NORM, bool KSPLIT, bool PAIR>
 __global__ __launch_bounds__(1024) void qmv_w16_kernel(const W16Params p) {
-  static_assert(!P8 || (NMAT == 1 && SBLDS && !KSPLIT), "pair-of-8 mode: one operand block, staged scales");
-  constexpr bool KSPLIT_OK = KSPLIT && NMAT == 1 && !NORM;
-  constexpr int RPB = P8 ? 8 : 16;     // rows of a matrix per block
-  constexpr int NS = P8 ? 2 : NMAT;    // matrices with scales to stage
-  extern __shared__ float red[];  // [ph][NMAT][nw][4][lw]
-  __shared__ float s_part[16][16];
+  static_assert(!KSPLIT || (!NORM && !PAIR), "split K: one matrix, activations as they are");
+  constexpr int RPB = PAIR ? 8 : 16;       // rows of a matrix per block
+  constexpr int TURN = turn_bytes(WIDE, SL), SUMS = sum_bytes(WIDE);
+  constexpr int LPR = 16 * SL;             // lanes that load a wave's run of an activation row
+  constexpr int RPL = 64 / LPR;            // rows of a load
+  constexpr int NX = (WIDE ? 16 : 8) / RPL;
+  constexpr int XROW = SL * 256;
+  constexpr int NG = WIDE ? 2 : 1;         // groups of a slice whose sums a lane holds
+  extern __shared__ __attribute__((aligned(16))) char lds[];  // [nw][wave_bytes], scales [rows][Gp (s, b) pairs + pad]
+  __shared__ __attribute__((aligned(16))) float s_part[16][32];
   __shared__ int s_last;
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -142,346 +157,239 @@ __global__ __launch_bounds__(1024) void qmv_w16_kernel(const W16Params p) {
   const int lr = lane >> 2, lc = lane & 3;  // load layout: row of the block, chunk of the slice
 
   // contiguous, balanced range of row blocks of this workgroup
-  const int kparts = KSPLIT_OK ? p.kparts : 1;
-  const int kpart = (int)blockIdx.x % kparts, bgroup = (int)blockIdx.x / kparts;
-  const int ngroups = (int)gridDim.x / kparts;
+  const int kparts = KSPLIT ? p.kparts : 1;
+  const int kpart = KSPLIT ? (int)blockIdx.x % kparts : 0, bgroup = KSPLIT ? (int)blockIdx.x / kparts : (int)blockIdx.x;
+  const int ngroups = KSPLIT ? (int)gridDim.x / kparts : (int)gridDim.x;
   const int qbase = p.blocks / ngroups, qrem = p.blocks - qbase * ngroups;
   const int q0 = bgroup * qbase + min(bgroup, qrem);
   const int nq = qbase + (bgroup < qrem ? 1 : 0);
   if (nq <= 0) return;
   const int g_first = kpart * p.Gp;  // first quantisation group of this workgroup's part of K
 
-  struct Buf {
-    uint4 w[NMAT][SL];
-    SbWord<SL> s[NMAT], b[NMAT];
-  };
-  // buffer resources over exactly this workgroup's rows (a refill past them returns zeros)
-  __amdgpu_buffer_rsrc_t rw[NMAT], rs[NS], rb[NS];
-#pragma unroll
-  for (int a = 0; a < NMAT; ++a)
-    rw[a] = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<char*>(reinterpret_cast<const char*>(p.w[a]) + (size_t)q0 * RPB * p.row_bytes), 0,
-        nq * RPB * p.row_bytes, 0x00020000);
-#pragma unroll
-  for (int a = 0; a < NS; ++a) {
-    rs[a] = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(p.s[a] + (size_t)q0 * RPB * p.G), 0,
-                                              nq * RPB * p.G * 2, 0x00020000);
-    rb[a] = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(p.b[a] + (size_t)q0 * RPB * p.G), 0,
-                                              nq * RPB * p.G * 2, 0x00020000);
-  }
-  const int wofs = lr * p.row_bytes + g_first * 32 + wave * (SL * 64) + lc * 16;
-  // P8: this lane's row of its matrix (lanes of block rows 0..7: gate, 8..15: up), first block
-  const uint32_t* const w_mine = (P8 && lr >= 8) ? p.w[1] : p.w[0];
-  const char* const w_lane = reinterpret_cast<const char*>(w_mine) +
-                             (size_t)(q0 * RPB + (lr & (RPB - 1))) * p.row_bytes + wave * (SL * 64) + lc * 16;
-  const int sofs = (j * p.G + g_first + wave * (SL * 2)) * 2;  // this lane's weight row, the wave's groups
-  // PIN (the issues in front of the loop): the loads leave in program order - weights, then
-  // scales and biases, buffer by buffer, as in the loop.  The compiler counts the loads still
-  // in flight at each wait; where the order in front of the loop differs from the order in the
-  // loop it has to assume the worse of the two and waits for a whole buffer too many.
-  auto issue_w = [&](Buf& bf, int q, bool pin) {  // q: row block of this workgroup's range (past it: zeros)
-    const int wq = q * 16 * p.row_bytes;  // uniform: scalar offset
-    if (pin) __builtin_amdgcn_sched_barrier(0);
-    if constexpr (P8) {
-      const char* src = w_lane + (size_t)min(q, nq - 1) * (8 * p.row_bytes);
-#pragma unroll
-      for (int sl = 0; sl < SL; ++sl) bf.w[0][sl] = *reinterpret_cast<const uint4*>(src + sl * 64);
-    } else {
-#pragma unroll
-      for (int sl = 0; sl < SL; ++sl)
-#pragma unroll
-        for (int a = 0; a < NMAT; ++a)
-          bf.w[a][sl] = __builtin_bit_cast(
-              uint4, __builtin_amdgcn_raw_buffer_load_b128(rw[a], wofs + sl * 64, wq, 0));
-    }
-    if (pin) __builtin_amdgcn_sched_barrier(0);
-  };
-  auto issue_sb = [&](Buf& bf, int q, bool pin) {
-    const int sq = q * 16 * p.G * 2;
-#if (EXO_W16_ABL & 64)  // timing only: no scale / bias loads
-#pragma unroll
-    for (int a = 0; a < NMAT; ++a)
-#pragma unroll
-      for (int sl = 0; sl < SL; ++sl) bf.s[a].v[sl] = bf.b[a].v[sl] = 0x3c003c00u + sq;
-#else
-#pragma unroll
-    for (int a = 0; a < NMAT; ++a) {
-      bf.s[a].load(rs[a], sofs, sq);
-      bf.b[a].load(rb[a], sofs, sq);
-    }
-#endif
-    if (pin) __builtin_amdgcn_sched_barrier(0);
-  };
-  auto issue = [&](Buf& bf, int q, bool pin) {
-    issue_w(bf, q, pin);
-    if (!SBLDS) issue_sb(bf, q, pin);
-  };
-  // staged scales / biases: array (matrix a, scale|bias) x local row x (G + 4) bf16 (rows
-  // padded by 8 bytes: the 16 rows a wave reads at once then sit in different banks)
-  char* const sb_lds = reinterpret_cast<char*>(red) + p.red_bytes;
-  const int sb_row = p.Gp * 2 + 8, sb_arr = p.ph * RPB * sb_row;
-  char* const nw_lds = sb_lds + (SBLDS ? NS * 2 * sb_arr : 0);  // the norm weights, K bf16
+  char* const mine = lds + wave * p.wave_bytes;
+  char* const red = mine + TURN;  // this wave's partial sums: [block][64 lanes][4 or 2]
+  char* const sb_lds = lds + nw * p.wave_bytes;
+  const int sb_row = p.Gp * 4 + kRowPad;
 
-  // ---- activations: lane (m = j, kg) holds, for product (sl, g, h), the 8 elements of row m
-  // that the weight word of lane (., kg) covers: word 4*(2g + kg%2) + 2h + kg/2 of the slice
-  uint4 xa[SL][2][2];
-  float sx[SL][2][4];  // group sums of the activation rows 4*kg + r of this lane's results
-  Buf buf[DEPTH];
+  // ---- requests: the wave's runs of the activation rows (rows past M: out of range, zeros), norm weights,
+  // this thread's piece of the scales and biases, the first row blocks of weights, in this order
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(p.x), 0, p.M * p.K * 2, 0x00020000);
+  const int run_ofs = g_first * 128 + wave * (SL * 256);  // bytes of activations in front of the wave's
+  const int xrow = lane / LPR, xchunk = lane % LPR;
+  uint4 xr[NX], gain = make_uint4(0, 0, 0, 0);
+#pragma unroll
+  for (int i = 0; i < NX; ++i)
+    xr[i] = __builtin_bit_cast(
+        uint4, __builtin_amdgcn_raw_buffer_load_b128(rx, (i * RPL + xrow) * (p.K * 2) + xchunk * 16, run_ofs, 0));
+  if (NORM) gain = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(p.norm_w) + run_ofs + xchunk * 16);
+  const int ppr = p.wide_pieces ? p.Gp >> 3 : p.Gp >> 1;  // pieces of a row
+  const int prow = (tid * p.piece_mul) >> 16, pcol = tid - prow * ppr;
+  u32x4 ps = {}, pb = {};
   {
-    // range-checked loads: lanes of rows m >= M get zeros
-    const __amdgpu_buffer_rsrc_t rx =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(p.x), 0, p.M * p.K * 2, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rn = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<bf16_t*>(NORM ? p.norm_w : p.x), 0, p.K * 2, 0x00020000);
-    const int lane_word = 4 * (kg & 1) + (kg >> 1);  // + 8g + 2h: the word of product (g, h)
-    const int xofs = (j * p.K + lane_word * 8) * 2, nofs = lane_word * 16;
-    // bytes of activations in front of the wave's slices
-    const int wave_ofs = g_first * 128 + wave * (SL * 256);
-    // staging: chunk tid of each array (past the workgroup's rows: out of range, no traffic)
-    // (the norm weights too: chunk tid; every lane reads its words back after the barrier -
-    // loaded per lane they are 16 times the bytes, one copy per activation row, and their
-    // registers are live across the barrier beside everything else)
-    uint4 nstg = make_uint4(0, 0, 0, 0);
-    if (NORM) nstg = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rn, tid * 16, 0, 0));
-    uint4 stg[NS][2];
-    if (SBLDS) {
-      // thread -> (local row, 16-byte chunk of the row's part); past the rows: out of range
-      const int cpr = p.Gp >> 3, row = tid / cpr, col = tid - row * cpr;
-      const int so = row < nq * RPB ? (row * p.G + g_first) * 2 + col * 16 : 0x7ffffff0;
-#pragma unroll
-      for (int a = 0; a < NS; ++a) {
-        stg[a][0] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs[a], so, 0, 0));
-        stg[a][1] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rb[a], so, 0, 0));
-      }
+    const int row = min(prow, nq * 16 - 1), a = PAIR ? (row >> 3) & 1 : 0;
+    const int r = PAIR ? (row >> 4) * 8 + (row & 7) : row;
+    const size_t at = (size_t)(q0 * RPB + r) * p.G + g_first;
+    const bf16_t *s = (a ? p.s[1] : p.s[0]) + at, *b = (a ? p.b[1] : p.b[0]) + at;
+    if (p.wide_pieces) {
+      ps = *reinterpret_cast<const u32x4*>(s + pcol * 8);
+      pb = *reinterpret_cast<const u32x4*>(b + pcol * 8);
+    } else {
+      ps[0] = *reinterpret_cast<const uint32_t*>(s + pcol * 2);
+      pb[0] = *reinterpret_cast<const uint32_t*>(b + pcol * 2);
     }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  struct Block {
+    u32x4 w[SL];
+  } b0, b1;
+  const uint32_t* const w_mine = (PAIR && lr >= 8) ? p.w[1] : p.w[0];
+  const char* const w_lane = reinterpret_cast<const char*>(w_mine) + (size_t)(q0 * RPB + (lr & (RPB - 1))) * p.row_bytes +
+                             g_first * 32 + wave * (SL * 64) + lc * 16;
+  auto issue = [&](Block& to, int q) {
+    const char* src = q < nq ? w_lane + (size_t)(q * RPB) * p.row_bytes : reinterpret_cast<const char*>(p.w[0]);
 #pragma unroll
-    for (int sl = 0; sl < SL; ++sl)
+    for (int sl = 0; sl < SL; ++sl) to.w[sl] = *reinterpret_cast<const u32x4*>(src + sl * 64);
+  };
+  issue(b0, 0);
+  __builtin_amdgcn_sched_barrier(0);
+  if (DEPTH == 2) issue(b1, 1);
+  __builtin_amdgcn_sched_barrier(0);
+
+  // ---- activations into operand order
+  auto stage_sb = [&]() {
+    if (prow >= nq * 16) return;
+    uint2* to = reinterpret_cast<uint2*>(sb_lds + prow * sb_row + pcol * (p.wide_pieces ? 32 : 8));
 #pragma unroll
-      for (int g = 0; g < 2; ++g)
+    for (int c = 0; c < 4; ++c)
+      if (c == 0 || p.wide_pieces) to[c] = make_uint2((ps[c] & 0xffffu) | pb[c] << 16, ps[c] >> 16 | (pb[c] & 0xffff0000u));
+  };
+  if (NORM) {
+    // sums of squares: of a row by runs of 16 lanes, [row][slice of the row]
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int wo = (sl * 16 + 8 * g + 2 * h) * 16;
-          xa[sl][g][h] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rx, xofs + wo, wave_ofs, 0));
-        }
-    // the activation loads go first (they are waited for first), then the weights - with the
-    // fused norm only the first block: beside the raw words and the staging registers every
-    // buffer at once does not fit, and a spilled value is reloaded behind a wait for ALL
-    // outstanding loads
-#pragma unroll
-    for (int d = 0; d < (NORM ? 1 : DEPTH); ++d) issue(buf[d], d, true);
-    auto stage_sb = [&](const uint4 (&v)[NS][2]) {
-      const int cpr = p.Gp >> 3;  // 16-byte chunks per row
-      const int row = tid / cpr, col = tid - row * cpr;
-      if (row < nq * RPB) {
-#pragma unroll
-        for (int a = 0; a < NS; ++a)
-#pragma unroll
-          for (int t = 0; t < 2; ++t) {
-            uint2* dst = reinterpret_cast<uint2*>(sb_lds + (a * 2 + t) * sb_arr + row * sb_row + col * 16);
-            dst[0] = make_uint2(v[a][t].x, v[a][t].y);
-            dst[1] = make_uint2(v[a][t].z, v[a][t].w);
-          }
-      }
-    };
-    if (SBLDS && !NORM) {
-      stage_sb(stg);
-      __syncthreads();
+    for (int i = 0; i < NX; ++i) {
+      const float ss = run_sum<16>(sumsq8(xr[i]));
+      if ((lane & 15) == 0) s_part[i * RPL + xrow][wave * SL + (xchunk >> 4)] = ss;
     }
-    if (NORM) {
-      // rows past the waves of this workgroup count as zero in the fixed-order sum below
-      if (wave + nw < 16 && lane < 16) {
-        for (int w2 = wave + nw; w2 < 16; w2 += nw) s_part[w2][lane] = 0.f;
-      }
-    }
-    if (NORM) {  // fused RMSNorm: every wave holds its slices of every row
-      float ss = 0.f;
+  }
+  stage_sb();
+  lds_barrier();
+  if (NORM) {
+    // lane (row lane/8, four slices from 4 (lane%8) on); a row's total in each of its eight lanes
+    const int slices = nw * SL, c0 = (lane & 7) * 4;
 #pragma unroll
-      for (int sl = 0; sl < SL; ++sl)
-#pragma unroll
-        for (int g = 0; g < 2; ++g)
-#pragma unroll
-          for (int h = 0; h < 2; ++h) ss += sumsq8(xa[sl][g][h]);
-      ss += __shfl_xor(ss, 16, 64);
-      ss += __shfl_xor(ss, 32, 64);
-      if (lane < 16) s_part[wave][lane] = ss;
-      if (SBLDS) stage_sb(stg);
-      if (tid * 16 < p.K * 2) *reinterpret_cast<uint4*>(nw_lds + tid * 16) = nstg;
-      __syncthreads();
-      // the waves' sums of row m in wave order: lane (m, kg) adds waves kg, kg+4, kg+8, kg+12
-      float t = (s_part[kg][j] + s_part[kg + 4][j]) + (s_part[kg + 8][j] + s_part[kg + 12][j]);
-      t += __shfl_xor(t, 16, 64);
-      t += __shfl_xor(t, 32, 64);
+    for (int h = 0; h < (WIDE ? 2 : 1); ++h) {
+      const floatx4 v = *reinterpret_cast<const floatx4*>(&s_part[h * 8 + (lane >> 3)][c0]);
+      float t = ((c0 < slices ? v[0] : 0.f) + (c0 + 1 < slices ? v[1] : 0.f)) +
+                ((c0 + 2 < slices ? v[2] : 0.f) + (c0 + 3 < slices ? v[3] : 0.f));
+      t = run_sum<8>(t);
       const float inv = rsqrtf(t / (float)p.K + p.eps);
 #pragma unroll
-      for (int sl = 0; sl < SL; ++sl)
-#pragma unroll
-        for (int g = 0; g < 2; ++g)
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            const int wo = (sl * 16 + 8 * g + 2 * h) * 16;
-            norm8(xa[sl][g][h], *reinterpret_cast<const uint4*>(nw_lds + wave_ofs + nofs + wo), inv);
-          }
+      for (int i = 0; i < 8 / RPL; ++i) norm8(xr[h * (8 / RPL) + i], gain, __shfl(inv, (i * RPL + xrow) * 8, 64));
     }
+  }
+  uint4 xa[SL][4];      // operands of the products of a slice
+  floatx4 sx[SL][NG];   // sums over a group, where D has them
+  {
+    // chunk c of row r sits at c ^ r (in 256 bytes): an operand read touches all 64 banks
+#pragma unroll
+    for (int i = 0; i < NX; ++i) {
+      const int r = i * RPL + xrow;
+      *reinterpret_cast<uint4*>(mine + r * XROW + (xchunk ^ r) * 16) = pair_order(xr[i]);
+    }
+    if (!WIDE && lane < LPR) *reinterpret_cast<uint4*>(mine + 8 * XROW + lane * 16) = make_uint4(0, 0, 0, 0);
+    wave_lds_order();
+    // (up to eight rows: row 8 of the staged ones, zeros, in the slots of the other group)
+    const int r = WIDE ? j : (j >> 3) == (kg >> 1) ? j & 7 : 8;
+    const char* from = mine + r * XROW;
+    const uint4 ones = make_uint4(0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u);
 #pragma unroll
     for (int sl = 0; sl < SL; ++sl)
 #pragma unroll
-      for (int g = 0; g < 2; ++g) {
-        float gs = 0.f;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          float s1;
-          xa[sl][g][h] = pair_order(xa[sl][g][h], s1);
-          gs += s1;
-        }
-        gs += __shfl_xor(gs, 16, 64);
-        gs += __shfl_xor(gs, 32, 64);  // every lane (m, .) holds the group sum of row m
-#pragma unroll
-        for (int r = 0; r < 4; ++r) sx[sl][g][r] = __shfl(gs, 4 * kg + r, 64);
+      for (int t = 0; t < 4; ++t) {
+        const int c = WIDE ? (t >> 1) * 8 + kg * 2 + (t & 1) : kg * 4 + t;
+        xa[sl][t] = *reinterpret_cast<const uint4*>(from + sl * 256 + (c ^ r) * 16);
       }
-    if (NORM) {
+    wave_lds_order();
 #pragma unroll
-      for (int d = 1; d < DEPTH; ++d) issue(buf[d], d, true);
-    }
+    for (int sl = 0; sl < SL; ++sl)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        floatx4& to = sx[sl][WIDE ? t >> 1 : 0];
+        if (t % (4 / NG) == 0) to = floatx4{0.f, 0.f, 0.f, 0.f};
+        to = mfma(xa[sl][t], ones, to);
+      }
   }
 
   uint32_t kmask = 0x000F000Fu, kmagic = 0x43004300u;
   asm volatile("" : "+s"(kmask));
   asm volatile("" : "+v"(kmagic));
-  // The lane's coordinates once more, from the hardware lane count: values derived from the
-  // first copy would have to live through the register-tight set-up above, and the compiler
-  // spilled one of them - a spilled value is reloaded behind a wait for ALL outstanding loads.
-  const int lane_l = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-  const int jl = lane_l & 15, kgl = lane_l >> 4;
-  const bool hi_half = kgl >= 2;
-  const int lw = p.lw;
+  char* const turn_to = mine + lr * 64 + ((lc ^ (lr >> 2)) & 3) * 16;
+  const char* const turn_from = mine + j * 64 + (WIDE ? (((kg >> 1) ^ (j >> 2)) & 3) * 16 + (kg & 1) * 8 : ((kg ^ (j >> 2)) & 3) * 16);
+  const int turn_group = (((2 + (kg >> 1)) ^ (j >> 2)) & 3) * 16 - (((kg >> 1) ^ (j >> 2)) & 3) * 16;  // WIDE: to the second group
+  const char* const sb_lane = sb_lds + j * sb_row + (wave * (SL * 2) + (WIDE ? 0 : kg >> 1)) * 4;
 
-  // one row block of this wave's slices; leaves the wave's partial sums in LDS slot `slot`
-  auto consume = [&](const Buf& bf, int slot) {
-    floatx4 acc[NMAT];
+  // one row block of this wave's slices; leaves the wave's partial sums in LDS.  The block's registers are
+  // free, and the next one requested into them, as soon as its words change lanes.
+  auto consume = [&](Block& block, int slot) {
+    uint4 c[SL];
+    uint32_t sb[SL][NG];
 #pragma unroll
-    for (int a = 0; a < NMAT; ++a) acc[a] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int sl = 0; sl < SL; ++sl) {
+      char* const to = turn_to + (WIDE ? 0 : sl * 1024);
+      if (WIDE) wave_lds_order();
+      *reinterpret_cast<u32x4*>(to) = block.w[sl];
+      if (!WIDE) continue;
+      wave_lds_order();
+      const uint2 g0 = *reinterpret_cast<const uint2*>(turn_from), g1 = *reinterpret_cast<const uint2*>(turn_from + turn_group);
+      c[sl] = make_uint4(g0.x, g0.y, g1.x, g1.y);
+    }
+    wave_lds_order();
 #pragma unroll
-    for (int sl = 0; sl < SL; ++sl)
+    for (int sl = 0; sl < SL; ++sl) {
+      if (!WIDE) c[sl] = *reinterpret_cast<const uint4*>(turn_from + sl * 1024);
 #pragma unroll
-      for (int a = 0; a < NMAT; ++a)
+      for (int g = 0; g < NG; ++g) sb[sl][g] = *reinterpret_cast<const uint32_t*>(sb_lane + slot * 16 * sb_row + sl * 8 + g * 4);
+    }
+    wave_lds_order();
+    if (DEPTH == 2) issue(block, slot + 2);
+    __builtin_amdgcn_sched_barrier(0);
+    floatx4 acc = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int g = 0; g < 2; ++g) {
-          // lane (j, kg) takes its words from the lane that loaded chunk 2g + kg%2 of row j
-          const int src = (4 * jl + 2 * g + (kgl & 1)) * 4;
-#if (EXO_W16_ABL & 2)
-          const uint32_t q0w = bf.w[a][sl].x + src, q1w = bf.w[a][sl].y, q2w = bf.w[a][sl].z, q3w = bf.w[a][sl].w;
-#else
-          const uint32_t q0w = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)bf.w[a][sl].x);
-          const uint32_t q1w = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)bf.w[a][sl].y);
-          const uint32_t q2w = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)bf.w[a][sl].z);
-          const uint32_t q3w = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)bf.w[a][sl].w);
-#endif
-          floatx4 dq = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int sl = 0; sl < SL; ++sl) {
+      const uint32_t word[4] = {c[sl].x, c[sl].y, c[sl].z, c[sl].w};
+      floatx4 dq[NG];
 #pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            const uint32_t wd = h == 0 ? (hi_half ? q1w : q0w) : (hi_half ? q3w : q2w);
-            uint4 bw;
-#if (EXO_W16_ABL & 8)
-            bw.x = wd; bw.y = wd ^ kmagic; bw.z = wd | kmagic; bw.w = wd & kmagic;
-#else
-            bw.x = (wd & kmask) | kmagic;
-            bw.y = ((wd >> 4) & kmask) | kmagic;
-            bw.z = ((wd >> 8) & kmask) | kmagic;
-            bw.w = ((wd >> 12) & kmask) | kmagic;
-#endif
-#if (EXO_W16_ABL & 1)
-            dq[0] += __builtin_bit_cast(float, bw.x ^ bw.y ^ bw.z ^ bw.w ^ xa[sl][g][h].x);
-#else
-            dq = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, xa[sl][g][h]),
-                                                        __builtin_bit_cast(bf16x8_t, bw), dq, 0, 0, 0);
-#endif
-          }
-          uint32_t sw, bwd;
-          if (P8) {  // this lane's column: row jl % 8 of the gate (jl < 8) or the up matrix
-            const char* base = sb_lds + (slot * 8 + (jl & 7)) * sb_row + (wave * SL + sl) * 4 + (jl >> 3) * 2 * sb_arr;
-            sw = *reinterpret_cast<const uint32_t*>(base);
-            bwd = *reinterpret_cast<const uint32_t*>(base + sb_arr);
-          } else if (SBLDS) {
-            const char* base = sb_lds + (slot * 16 + jl) * sb_row + (wave * SL + sl) * 4;
-            sw = *reinterpret_cast<const uint32_t*>(base + (a * 2) * sb_arr);
-            bwd = *reinterpret_cast<const uint32_t*>(base + (a * 2 + 1) * sb_arr);
-          } else {
-            sw = bf.s[a].v[sl];
-            bwd = bf.b[a].v[sl];
-          }
-          const float sc = g == 0 ? bf_lo(sw) : bf_hi(sw);
-          const float bi = g == 0 ? bf_lo(bwd) : bf_hi(bwd);
-#if (EXO_W16_ABL & 4)
-          acc[a][0] += dq[0] * sc + dq[1] + dq[2] + dq[3] + bi;
-#else
-          const float t = fmaf(-128.f, sc, bi);
+      for (int t = 0; t < 4; ++t) {
+        uint4 bw;
+        bw.x = (word[t] & kmask) | kmagic;
+        bw.y = ((word[t] >> 4) & kmask) | kmagic;
+        bw.z = ((word[t] >> 8) & kmask) | kmagic;
+        bw.w = ((word[t] >> 12) & kmask) | kmagic;
+        const int g = WIDE ? t >> 1 : 0;
+        dq[g] = mfma(xa[sl][t], bw, t % (4 / NG) == 0 ? floatx4{0.f, 0.f, 0.f, 0.f} : dq[g]);
+      }
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            acc[a][r] = fmaf(sc, dq[r], acc[a][r]);
-            acc[a][r] = fmaf(t, sx[sl][g][r], acc[a][r]);
-          }
-#endif
-        }
-    if (lane_l < lw) {
+      for (int g = 0; g < NG; ++g) {
+        const float sc = bf_lo(sb[sl][g]), tb = fmaf(-128.f, sc, bf_hi(sb[sl][g]));
 #pragma unroll
-      for (int a = 0; a < NMAT; ++a)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          red[((((size_t)slot * NMAT + a) * nw + wave) * 4 + r) * lw + lane_l] = acc[a][r];
+        for (int r = 0; r < 4; ++r) acc[r] = fmaf(tb, sx[sl][g][r], fmaf(sc, dq[g][r], acc[r]));
+      }
+    }
+    if (WIDE) {
+      *reinterpret_cast<floatx4*>(red + slot * SUMS + lane * 16) = acc;
+    } else {
+      // the two groups' halves of the wave: lanes 0..31 get results r = 0 and 2 of rows 4 (kg%2) + r, the others 1 and 3
+      const float2 v = make_float2(fold_halves(acc[0], acc[1]), fold_halves(acc[2], acc[3]));
+      *reinterpret_cast<float2*>(red + slot * SUMS + lane * 8) = v;
     }
   };
 
-  // the phase's results: sum over the waves in a fixed order, epilogue, store
-  auto finish_phase = [&](int q_first, int n, bool res) {
-    __syncthreads();
-    if constexpr (P8) {
-      for (int idx = tid; idx < n * p.M * 8; idx += (int)blockDim.x) {
-        const int jj = idx & 7, m = (idx >> 3) % p.M, slot = (idx >> 3) / p.M;
-        const float* src = &red[(((size_t)slot * nw * 4) + (m & 3)) * lw + (m >> 2) * 16 + jj];
-        float tg = 0.f, tu = 0.f;
-        for (int w = 0; w < nw; ++w) {
-          tg += src[(size_t)w * 4 * lw];
-          tu += src[(size_t)w * 4 * lw + 8];
-        }
-        // SwiGLU on the bf16-rounded projections
-        const float g = bf2f(f2bf(tg)), up = bf2f(f2bf(tu));
-        p.y[(size_t)m * p.N + (q0 + q_first + slot) * 8 + jj] = f2bf(g / (1.f + __expf(-g)) * up);
-      }
-      __syncthreads();
-      return;
-    }
-    for (int idx = tid; idx < n * p.M * 16; idx += (int)blockDim.x) {
-      const int jj = idx & 15, m = (idx >> 4) % p.M, slot = (idx >> 4) / p.M;
-      const int src_lane = (m >> 2) * 16 + jj, r = m & 3;
-      float tot[NMAT];
-#pragma unroll
-      for (int a = 0; a < NMAT; ++a) {
-        const float* src = &red[(((size_t)slot * NMAT + a) * nw * 4 + r) * lw + src_lane];
-        float t = 0.f;
-        for (int w = 0; w < nw; ++w) t += src[(size_t)w * 4 * lw];
-        tot[a] = t;
-      }
-      const int row = (q0 + q_first + slot) * 16 + jj;
-      const size_t o = (size_t)m * p.N + row;
-      if (KSPLIT_OK && p.kparts > 1) {  // (single matrices only) this part's share of the sum
-        st_dev(&p.part[(size_t)kpart * p.M * p.N + o], tot[0]);
-        continue;
-      }
-      float out;
-      if (NMAT == 2) {  // SwiGLU on the bf16-rounded projections
-        const float g = bf2f(f2bf(tot[0])), up = bf2f(f2bf(tot[NMAT - 1]));
-        out = g / (1.f + __expf(-g)) * up;
-      } else {
-        out = tot[0];
-        if (res && p.residual) out = bf2f(f2bf(out)) + bf2f(p.residual[o]);
-      }
-      p.y[o] = f2bf(out);
-    }
-    __syncthreads();
+  if constexpr (DEPTH == 2) {
+    // (a workgroup of one block multiplies what its second request brought as well, for nobody)
+    int q = 0;
+    do {
+      consume(b0, q);
+      consume(b1, q + 1);
+      q += 2;
+    } while (q + 1 < nq);
+    if (q < nq) consume(b0, q);
+  } else {
+    consume(b0, 0);
+  }
+
+  // ---- the workgroup's results: sum over the waves in a fixed order, epilogue, store
+  lds_barrier();
+  // result (column jj, row m) of a block: where consume() has left it
+  auto total = [&](int slot, int jj, int m) {
+    const int at = WIDE ? ((m >> 2) * 16 + jj) * 4 + (m & 3) : ((m & 1) * 32 + (m >> 2) * 16 + jj) * 2 + ((m >> 1) & 1);
+    const char* src = lds + TURN + slot * SUMS + at * 4;
+    float t = 0.f;
+    for (int w = 0; w < nw; ++w) t += *reinterpret_cast<const float*>(src + w * p.wave_bytes);
+    return t;
   };
-  // Split K: the last of a group's workgroups to arrive adds the parts in part order (the result
-  // does not depend on arrival order) and writes y; the counter returns to zero.
-  auto merge_parts = [&](int n) {
+  if constexpr (PAIR) {
+    for (int idx = tid; idx < nq * p.M * 8; idx += (int)blockDim.x) {
+      const int jj = idx & 7, m = (idx >> 3) % p.M, slot = (idx >> 3) / p.M;
+      // SwiGLU on the bf16-rounded projections
+      const float g = bf2f(f2bf(total(slot, jj, m))), up = bf2f(f2bf(total(slot, jj + 8, m)));
+      p.y[(size_t)m * p.N + (q0 + slot) * 8 + jj] = f2bf(g / (1.f + __expf(-g)) * up);
+    }
+    return;
+  }
+  for (int idx = tid; idx < nq * p.M * 16; idx += (int)blockDim.x) {
+    const int jj = idx & 15, m = (idx >> 4) % p.M, slot = (idx >> 4) / p.M;
+    const size_t o = (size_t)m * p.N + (q0 + slot) * 16 + jj;
+    float out = total(slot, jj, m);
+    if (KSPLIT) {  // this part's share of the sum
+      st_dev(&p.part[(size_t)kpart * p.M * p.N + o], out);
+      continue;
+    }
+    if (p.residual) out = bf2f(f2bf(out)) + bf2f(p.residual[o]);
+    p.y[o] = f2bf(out);
+  }
+  if constexpr (KSPLIT) {
+    // The last of a group's workgroups to arrive adds the parts in part order (the result does not
+    // depend on arrival order) and writes y; the counter returns to zero.
     wait_own_stores_done();  // this wave's device-scope partial stores have completed
     __syncthreads();
     if (tid == 0) {
@@ -492,7 +400,7 @@ __global__ __launch_bounds__(1024) void qmv_w16_kernel(const W16Params p) {
     }
     __syncthreads();
     if (!s_last) return;
-    for (int idx = tid; idx < n * p.M * 16; idx += (int)blockDim.x) {
+    for (int idx = tid; idx < nq * p.M * 16; idx += (int)blockDim.x) {
       const int jj = idx & 15, m = (idx >> 4) % p.M, slot = (idx >> 4) / p.M;
       const size_t o = (size_t)m * p.N + (q0 + slot) * 16 + jj;
       float t = 0.f;
@@ -500,106 +408,69 @@ __global__ __launch_bounds__(1024) void qmv_w16_kernel(const W16Params p) {
       if (p.residual) t = bf2f(f2bf(t)) + bf2f(p.residual[o]);
       p.y[o] = f2bf(t);
     }
-  };
-
-  int slot = 0, q_first = 0;
-  for (int base = 0;; base += DEPTH) {
-#pragma unroll
-    for (int d = 0; d < DEPTH; ++d) {
-      if (base + d < nq) {
-        consume(buf[d], slot);
-        ++slot;
-      }
-      issue(buf[d], base + d + DEPTH, false);
-    }
-    if (base + DEPTH >= nq) break;
   }
-  // (One phase: the launcher gives a workgroup no more row blocks than the LDS holds partial
-  // sums for.  A reduction inside the streaming loop - even an empty conditional block that
-  // resets `slot` - makes the compiler wait for a whole buffer too many at the first block of
-  // every round.)
-  finish_phase(q_first, slot, true);
-  if (KSPLIT_OK && p.kparts > 1) merge_parts(slot);
 }
 
-constexpr size_t kLdsBudget = 144 * 1024;  // LDS for partial sums and staged scales (the norm weights: 8 KB more)
-
-template <int NMAT, int SL, int DEPTH, bool NORM, bool SBLDS, bool KSPLIT = false, bool P8 = false>
-int launch_w16s(W16Params p, int nw, hipStream_t st) {
-  auto kern = qmv_w16_kernel<NMAT, SL, DEPTH, NORM, SBLDS, KSPLIT, P8>;
-  constexpr int RPB = P8 ? 8 : 16, NS = P8 ? 2 : NMAT;
-  p.blocks = p.N / RPB;
-  p.lw = 16 * ((p.M + 3) / 4);
-  const size_t per_block = (size_t)NMAT * nw * 4 * p.lw * sizeof(float);
-  const size_t sb_block = SBLDS ? (size_t)NS * 2 * RPB * (p.Gp * 2 + 8) : 0;
-  int ph = (int)(kLdsBudget / (per_block + sb_block));  // row blocks a workgroup can hold
-  // staging: one 16-byte chunk per thread and array
-  const int stage_max = 64 * nw / (RPB * (p.Gp / 8));
-  if (SBLDS && ph > stage_max) ph = stage_max;
-  if (ph < 1) {
-    exo_set_error("exo_qmv: internal: no LDS for one row block (M=%d K=%d)", p.M, p.K);
-    return EXO_ERR_ARG;
-  }
-  // one workgroup per CU (kparts workgroups per group of row blocks); more rounds where a
-  // workgroup's share would not fit the LDS
-  const int round = 256 / p.kparts;
-  int groups = round;
-  while ((p.blocks + groups - 1) / groups > ph) groups += round;
-  if (groups > p.blocks) groups = p.blocks;
-  const int grid = groups * p.kparts;
-  const int nq = (p.blocks + groups - 1) / groups;
-  p.ph = nq;
-  p.red_bytes = (int)(per_block * nq);
-  const size_t lds = (per_block + sb_block) * nq + (NORM ? (size_t)p.K * 2 : 0);
+template <bool WIDE, int SL, int DEPTH, bool NORM, bool KSPLIT, bool PAIR>
+int launch_instance(const W16Params& p, int grid, int nq, int nw, size_t bytes, hipStream_t st) {
+  auto kern = qmv_w16_kernel<WIDE, SL, DEPTH, NORM, KSPLIT, PAIR>;
   static bool attr_done = false;
-  if (!attr_done && lds > 48 * 1024) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, 156 * 1024);
+  if (!attr_done && bytes > 48 * 1024) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMax);
     if (e != hipSuccess) {
       exo_set_error("exo_qmv: cannot raise dynamic LDS limit: %s", hipGetErrorString(e));
       return EXO_ERR_HIP;
     }
     attr_done = true;
   }
-  exo_note_variant("qmv_w16<%d,%d,%d,%s,%s> grid=%d waves=%d blocks=%d kparts=%d", P8 ? 2 : NMAT, SL, DEPTH,
-                   NORM ? "norm" : "plain", P8 ? "pair8" : (SBLDS ? "staged" : "direct"), grid, nw, nq, p.kparts);
-  kern<<<dim3(grid), dim3(64 * nw), lds, st>>>(p);
+  exo_note_variant("qmv_w16<%d,%d,%d,%s,%s> grid=%d waves=%d blocks=%d kparts=%d", PAIR ? 2 : 1, SL, DEPTH,
+                   NORM ? "norm" : "plain", PAIR ? "pair8" : "staged", grid, nw, nq, p.kparts);
+  kern<<<dim3(grid), dim3(64 * nw), bytes, st>>>(p);
   return EXO_OK;
 }
-template <int NMAT, int SL, int DEPTH>
-int launch_w16(const W16Params& p, int nw, hipStream_t st) {
-  // staged scales where they fit the LDS beside the partial sums of one round of 256 workgroups
-  // (the 14336-row pair: up to 12 activation rows) and one chunk per thread covers them
-  const int round = 256 / p.kparts;
-  const int groups1 = p.blocks < round ? p.blocks : round, nq1 = (p.blocks + groups1 - 1) / groups1;
-  const size_t need1 = ((size_t)NMAT * nw * 4 * 16 * ((p.M + 3) / 4) * sizeof(float) +
-                        (size_t)NMAT * 2 * 16 * (p.Gp * 2 + 8)) * nq1;
-  const bool staged = p.Gp % 8 == 0 && need1 <= kLdsBudget && nq1 <= 32 * nw / p.Gp && !(EXO_W16_ABL & 128);
-  if constexpr (NMAT == 2) {
-    // the pair in blocks of 8 rows of both matrices where their share of one round of 256
-    // workgroups fits the LDS with staged scales: 14336 rows are seven such blocks per
-    // workgroup, against four or three blocks of 16 rows (8 activation rows: 20.4 -> us)
-    const int blocks8 = p.N / 8, g8 = blocks8 < 256 ? blocks8 : 256, nq8 = (blocks8 + g8 - 1) / g8;
-    const size_t need8 = ((size_t)nw * 4 * 16 * ((p.M + 3) / 4) * sizeof(float) +
-                          (size_t)2 * 2 * 8 * (p.Gp * 2 + 8)) * nq8;
-    if (p.N % 8 == 0 && p.Gp % 8 == 0 && need8 <= kLdsBudget && nq8 <= 64 * nw / (8 * (p.Gp / 8)) &&
-        EXO_W16_PAIR8) {
-      return p.norm_w ? launch_w16s<1, SL, DEPTH, true, true, false, true>(p, nw, st)
-                      : launch_w16s<1, SL, DEPTH, false, true, false, true>(p, nw, st);
-    }
-  }
-  if (p.kparts > 1) {
-    if constexpr (NMAT == 1)
-      return staged ? launch_w16s<1, SL, DEPTH, false, true, true>(p, nw, st)
-                    : launch_w16s<1, SL, DEPTH, false, false, true>(p, nw, st);
-    exo_set_error("exo_qmv: internal: split K with a matrix pair");
+
+template <bool WIDE, int SL, bool NORM, bool KSPLIT, bool PAIR>
+int launch_w16s(W16Params p, int nw, hipStream_t st) {
+  p.blocks = p.N / (PAIR ? 8 : 16);
+  // a wave's region: its activations on their way into operand order, later the lane changes and the partial sums
+  const int scales = 16 * (p.Gp * 4 + kRowPad);
+  auto wave_bytes = [&](int nq) {
+    const int stream = turn_bytes(WIDE, SL) + nq * sum_bytes(WIDE);
+    return stream > x_bytes(WIDE, SL) ? stream : x_bytes(WIDE, SL);
+  };
+  auto lds_bytes = [&](int nq) { return nw * wave_bytes(nq) + nq * scales; };
+  p.wide_pieces = p.Gp % 8 == 0;
+  const int ppr = p.wide_pieces ? p.Gp / 8 : p.Gp / 2;
+  p.piece_mul = 65536 / ppr + 1;
+  // row blocks that a workgroup can hold: partial sums, scales (one piece per thread and array)
+  auto fits = [&](int nq) { return lds_bytes(nq) <= kLdsMax && nq * 16 * ppr <= 64 * nw; };
+  if (!fits(1)) {
+    exo_set_error("exo_qmv: internal: no LDS for one row block (M=%d K=%d)", p.M, p.K);
     return EXO_ERR_ARG;
   }
-  if (p.norm_w)
-    return staged ? launch_w16s<NMAT, SL, DEPTH, true, true>(p, nw, st)
-                  : launch_w16s<NMAT, SL, DEPTH, true, false>(p, nw, st);
-  return staged ? launch_w16s<NMAT, SL, DEPTH, false, true>(p, nw, st)
-                : launch_w16s<NMAT, SL, DEPTH, false, false>(p, nw, st);
+  // one workgroup per CU (kparts workgroups per group of row blocks); more rounds where a
+  // workgroup's share would not fit
+  const int round = 256 / p.kparts;
+  int groups = round;
+  while (!fits((p.blocks + groups - 1) / groups)) groups += round;
+  if (groups > p.blocks) groups = p.blocks;
+  const int nq = (p.blocks + groups - 1) / groups;
+  p.wave_bytes = wave_bytes(nq);
+  const int grid = groups * p.kparts;
+  const size_t bytes = (size_t)lds_bytes(nq);
+  if (nq == 1) return launch_instance<WIDE, SL, 1, NORM, KSPLIT, PAIR>(p, grid, nq, nw, bytes, st);
+  return launch_instance<WIDE, SL, 2, NORM, KSPLIT, PAIR>(p, grid, nq, nw, bytes, st);
+}
+template <bool WIDE, int SL>
+int launch_w16(const W16Params& p, bool pair, int nw, hipStream_t st) {
+  if (p.kparts > 1) {
+    if (!pair && !p.norm_w) return launch_w16s<WIDE, SL, false, true, false>(p, nw, st);
+    exo_set_error("exo_qmv: internal: split K with a matrix pair or a norm");
+    return EXO_ERR_ARG;
+  }
+  if (pair)
+    return p.norm_w ? launch_w16s<WIDE, SL, true, false, true>(p, nw, st) : launch_w16s<WIDE, SL, false, false, true>(p, nw, st);
+  return p.norm_w ? launch_w16s<WIDE, SL, true, false, false>(p, nw, st) : launch_w16s<WIDE, SL, false, false, false>(p, nw, st);
 }
 
 // 64-byte slices per wave and waves per workgroup for rows of `row_bytes`
@@ -664,9 +535,7 @@ int exo_qmv_w16_launch(const bf16_t* x, const bf16_t* norm_w, float eps, const u
   p.row_bytes = K / 2;
   p.G = K / 64;
   p.blocks = N / 16;  // (the launcher sets the count for its block size)
-  p.ph = 1;
-  p.lw = 64;
-  p.red_bytes = 0;
+  p.wave_bytes = p.wide_pieces = p.piece_mul = 0;
   const bool pair = w2 != nullptr;
   int sl = 0, nw = 0;
   const int kp = exo_qmv_w16_ok(M, N, K, 4, norm_w != nullptr, pair, workspace != nullptr)
@@ -681,9 +550,6 @@ int exo_qmv_w16_launch(const bf16_t* x, const bf16_t* norm_w, float eps, const u
   // the workspace of the split-K GEMV: counters (64 KiB), then the float32 partial results
   p.counters = reinterpret_cast<int*>(workspace);
   p.part = workspace ? reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + 64 * 1024) : nullptr;
-#ifndef EXO_W16_DEPTH
-#define EXO_W16_DEPTH 2
-#endif
-  if (sl == 1) return pair ? launch_w16<2, 1, EXO_W16_DEPTH>(p, nw, st) : launch_w16<1, 1, EXO_W16_DEPTH>(p, nw, st);
-  return pair ? launch_w16<2, 2, 2>(p, nw, st) : launch_w16<1, 2, EXO_W16_DEPTH>(p, nw, st);
+  if (sl == 1) return M > 8 ? launch_w16<true, 1>(p, pair, nw, st) : launch_w16<false, 1>(p, pair, nw, st);
+  return M > 8 ? launch_w16<true, 2>(p, pair, nw, st) : launch_w16<false, 2>(p, pair, nw, st);
 }

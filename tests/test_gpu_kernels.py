@@ -164,6 +164,21 @@ def test_qmv_16x16x32_kernel_shapes(device, N, K, M):
                      what=f"w16 pair {M}x{N}x{K}")
 
 
+@pytest.mark.parametrize("N,K,blocks", [
+    (16, 1024, 1), (8208, 768, 3), (8176, 1152, 2), (69648, 512, 9),  # one block; shares of 2 and 3; of 1 and 2; two rounds
+])
+@pytest.mark.parametrize("M", [6, 8, 9])
+def test_qmv_16x16x32_shares_of_blocks(device, N, K, blocks, M):
+    """The 16x16x32 GEMV where its workgroups' shares of row blocks differ, at both operand layouts (to 8 rows, beyond)
+    and with scales in pieces of eight groups and of two."""
+    trip = rand_quantized(N, K, 4, seed=N + K)
+    x, r = rand_bf16((M, K), seed=M, scale=1.5), rand_bf16((M, N), seed=N)
+    got = ops.quantized_matmul(t_bf16(x, device), t_qw(trip, 4, device), residual=t_bf16(r, device))
+    assert native.last_variant().startswith("qmv_w16<1,1,") and f" blocks={blocks} " in native.last_variant(), native.last_variant()
+    want = affine.bf16_round(affine.bf16_round(affine.qmm(x, *trip, 64, 4)) + r)
+    assert_close(n_f32(got), want, what=f"w16 {M}x{N}x{K}")
+
+
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("M,N,K", [(8, 1000, 4096), (3, 96, 14336), (16, 2080, 2048), (5, 14336, 512)])
 def test_qmv_swiglu_rows_equal_separate_launches(device, bits, M, N, K):
