@@ -14,6 +14,8 @@
 //          launch can be replayed from a HIP graph while the sequence grows.
 // prefill: grid (T, Hkv, B); one workgroup per new token, causal limit pos+t+1,
 //          writes the output directly.
+#include <type_traits>
+
 #include "../../include/exo_mi355x.h"
 #include "common.h"
 #include <mutex>
@@ -45,8 +47,18 @@ constexpr int kTilesInFlight = EXO_SDPA_TILES_IN_FLIGHT;  // key tiles a wave ke
 // sequences): 256 keys 10.0 -> 9.3, 264 9.6 -> 10.8, 440 9.9 -> 12.0.
 template <int D, int G>
 constexpr int kSoloTiles = D >= 128 ? 16 : G == 1 ? 14 : G == 2 ? 12 : 8;
-constexpr int kSoloMfma = 256;  // the matrix-core kernel: 8 sequences, 130 keys 10.8 -> 8.7 us, 250 keys 11.9 -> 10.6
-                                // (500 keys 12.6 -> 13.8); 4 of 32 / 4 heads, 130 keys 12.1 -> 7.9
+// The matrix-core kernel.  Waves of a workgroup: four leave a SIMD one wave, whose loads, LDS round trip and products do not
+// overlap; each wave more is 0.13 us more of start and merge.  32 / 8 heads, 4 | 6 | 8 waves: 8 sequences of 130 keys
+// 8.2 | 6.8 | 7.2 us, 2050 keys 18.5 | 17.9 | 18.1, 16 of 12290 145 | 141 | 139; 4 of 32 / 4 heads, 1030 keys
+// 11.0 | 10.5 | 10.0; 8 of 64 / 4, 1030 keys 15.2 | 13.7 | 13.5.
+template <int G>
+constexpr int kMfmaWaves = G == 4 ? 6 : 8;
+// Contexts left to one workgroup, whose second round of tiles costs less than the hand-over: 8 sequences of 32 / 8 heads,
+// 300 keys 9.9 -> 8.8 us, 500 keys 11.2 -> 13.0.
+constexpr int kSoloMfma = 320;
+// Tiles of a split before another takes part: 500 keys (16 tiles) with two splits 11.9 us, with four 11.2; 600 keys with three 11.4,
+// with four 11.6.
+constexpr int kMfmaSplitTiles = 5;
 #ifndef EXO_SDPA_TILES_WAVES
 #define EXO_SDPA_TILES_WAVES 4
 #endif
@@ -101,48 +113,116 @@ __device__ __forceinline__ float partner_lpk(float v) {
   return __shfl_xor(v, LPK / 2, 64);
 }
 
-__device__ __forceinline__ void st_dev(float* p, float v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// one float, or two in one request
+template <int E>
+struct Run {
+  float v[E];
+};
+template <int E>
+__device__ __forceinline__ void st_dev(float* p, const Run<E>& r) {
+  typedef std::conditional_t<E == 2, uint64_t, uint32_t> bits;
+  __hip_atomic_store(reinterpret_cast<bits*>(p), __builtin_bit_cast(bits, r), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ float ld_dev(const float* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+template <int E>
+__device__ __forceinline__ Run<E> ld_dev(const float* p) {
+  typedef std::conditional_t<E == 2, uint64_t, uint32_t> bits;
+  return __builtin_bit_cast(Run<E>, __hip_atomic_load(reinterpret_cast<const bits*>(p), __ATOMIC_RELAXED,
+                                                      __HIP_MEMORY_SCOPE_AGENT));
+}
+// output elements per thread in the merges below: two where there are more of them than threads
+template <int D, int G, int THREADS>
+constexpr int kMergeRun = G * D > THREADS ? 2 : 1;
+
+template <int E>
+__device__ __forceinline__ void store_out(bf16_t* to, const Run<E>& acc, float lsum) {
+  if constexpr (E == 2) {
+    *reinterpret_cast<uint32_t*>(to) = pack_bf2(acc.v[0] / lsum, acc.v[1] / lsum);
+  } else {
+    *to = f2bf(acc.v[0] / lsum);
+  }
 }
 
-// The last workgroup's merge of the key splits of one output element: partials
-// [splits][D + 2] (D sums, then the split's maximum and its sum of weights), taken sixteen
+// The last workgroup's merge of the key splits of E neighbouring output elements: partials
+// [splits][D + 2] (D sums, then the split's maximum and its sum of weights), taken MS
 // splits at a time - all loads of a batch are issued before any is used (they miss every
 // cache) - and folded into a running (maximum, sum, weighted sum).
-template <int D>
-__device__ __forceinline__ float merge_splits(const float* src, int splits, int e) {
-  constexpr int MS = 16;
-  float mw = -INFINITY, acc = 0.f, lsum = 0.f;
+template <int D, int MS, int E>
+__device__ __forceinline__ void merge_batches(const float* src, int splits, int e, bf16_t* to) {
+  float mw = -INFINITY, lsum = 0.f;
+  Run<E> acc = {};
   for (int s0 = 0; s0 < splits; s0 += MS) {
-    float pm[MS], pl[MS], po[MS];
+    Run<2> ml[MS];
+    Run<E> po[MS];
 #pragma unroll
     for (int sp = 0; sp < MS; ++sp) {
       const int spc = min(s0 + sp, splits - 1);
-      pm[sp] = ld_dev(src + (size_t)spc * (D + 2) + D);
-      pl[sp] = ld_dev(src + (size_t)spc * (D + 2) + D + 1);
-      po[sp] = ld_dev(src + (size_t)spc * (D + 2) + e);
+      ml[sp] = ld_dev<2>(src + (size_t)spc * (D + 2) + D);
+      po[sp] = ld_dev<E>(src + (size_t)spc * (D + 2) + e);
     }
     float mc = mw;
 #pragma unroll
     for (int sp = 0; sp < MS; ++sp)
-      if (s0 + sp < splits) mc = fmaxf(mc, pm[sp]);
+      if (s0 + sp < splits) mc = fmaxf(mc, ml[sp].v[0]);
     if (s0 > 0) {  // earlier batches move to the new maximum
       const float r = (mw == -INFINITY) ? 0.f : __expf(mw - mc);
-      acc *= r;
+#pragma unroll
+      for (int i = 0; i < E; ++i) acc.v[i] *= r;
       lsum *= r;
     }
 #pragma unroll
     for (int sp = 0; sp < MS; ++sp) {
-      const float sc = (s0 + sp >= splits || pm[sp] == -INFINITY) ? 0.f : __expf(pm[sp] - mc);
-      acc += po[sp] * sc;
-      lsum += pl[sp] * sc;
+      const float sc = (s0 + sp >= splits || ml[sp].v[0] == -INFINITY) ? 0.f : __expf(ml[sp].v[0] - mc);
+#pragma unroll
+      for (int i = 0; i < E; ++i) acc.v[i] += po[sp].v[i] * sc;
+      lsum += ml[sp].v[1] * sc;
     }
     mw = mc;
   }
-  return acc / lsum;
+  store_out(to, acc, lsum);
+}
+// The waves of a workgroup have left (sums of weighted values, maximum, sum of weights) of G heads in `red`; they are
+// added up: the result, or this split's partial at device scope (the merging workgroup may run on another XCD,
+// whose L2 is not coherent with this one).  `ws`: the first head's partial of this split, `stride` floats between heads.
+template <int D, int G, int NW, int E = kMergeRun<D, G, 64 * NW>, int RS>
+__device__ __forceinline__ void merge_waves(const float (&red)[NW][G][RS], bool solo, bf16_t* out, float* ws, size_t stride) {
+  for (int idx = threadIdx.x; idx < G * (D / E); idx += 64 * NW) {
+    const int g = idx / (D / E), e = idx % (D / E) * E;
+    float mw = red[0][g][D];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) mw = fmaxf(mw, red[w][g][D]);
+    float lsum = 0.f;
+    Run<E> acc = {};
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float mm = red[w][g][D];
+      const float sc = (mm == -INFINITY) ? 0.f : __expf(mm - mw);
+#pragma unroll
+      for (int i = 0; i < E; ++i) acc.v[i] += red[w][g][e + i] * sc;
+      lsum += red[w][g][D + 1] * sc;
+    }
+    if (solo) {
+      store_out(out + (size_t)g * D + e, acc, lsum);
+      continue;
+    }
+    st_dev(ws + g * stride + e, acc);
+    if (e == 0) st_dev(ws + g * stride + D, Run<2>{mw, lsum});
+  }
+}
+// The last workgroup's merge of the splits of G heads (`ws`: the first split of the first head).  (Sixteen splits at
+// a time whatever their number, one element per thread, maximum and sum loaded apart are 48 loads a thread, most of them of
+// splits that are not there: 8 sequences of 32 / 8 heads, 2050 keys, four splits 18.9 us against 17.8.)
+template <int D, int G, int THREADS, int E = kMergeRun<D, G, THREADS>, bool FOUR = false>
+__device__ __forceinline__ void merge_heads(const float* ws, size_t stride, int splits, bf16_t* out) {
+  for (int idx = threadIdx.x; idx < G * (D / E); idx += THREADS) {
+    const int g = idx / (D / E), e = idx % (D / E) * E;
+    bf16_t* const to = out + (size_t)g * D + e;
+    if (FOUR && splits <= 4)
+      merge_batches<D, 4, E>(ws + g * stride, splits, e, to);
+    else if (splits <= 8)
+      merge_batches<D, 8, E>(ws + g * stride, splits, e, to);
+    else
+      merge_batches<D, 16, E>(ws + g * stride, splits, e, to);
+  }
 }
 
 // One head slice (8 elements of this lane, the head spread over LPK lanes) taken from a
@@ -206,7 +286,7 @@ __global__ __launch_bounds__(kThreads) void sdpa_kernel(const SdpaParams p) {
   constexpr int LPK = D / 8;        // lanes per key
   constexpr int KPI = 64 / LPK;     // keys per wave instruction
   constexpr int STEP = KPI * kBlk;  // keys per wave per step
-  __shared__ float red[kWaves][G][D + 2];
+  __shared__ __attribute__((aligned(16))) float red[kWaves][G][D + 4];
   __shared__ int s_last;
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -403,34 +483,8 @@ __global__ __launch_bounds__(kThreads) void sdpa_kernel(const SdpaParams p) {
   }
   __syncthreads();
 
-  // merge the waves; thread -> (head, element)
-  for (int idx = threadIdx.x; idx < G * D; idx += kThreads) {
-    const int g = idx / D, e = idx % D;
-    float mw = red[0][g][D];
-#pragma unroll
-    for (int w = 1; w < kWaves; ++w) mw = fmaxf(mw, red[w][g][D]);
-    float acc = 0.f, lsum = 0.f;
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) {
-      const float mm = red[w][g][D];
-      const float sc = (mm == -INFINITY) ? 0.f : __expf(mm - mw);
-      acc += red[w][g][e] * sc;
-      lsum += red[w][g][D + 1] * sc;
-    }
-    const int h = h0 + g;
-    if (DECODE) {
-      // device-scope (write-through) stores: the merging workgroup may run on another
-      // XCD, whose L2 is not coherent with this one
-      float* dst = p.ws + ((size_t)(b * p.Hq + h) * p.splits + blockIdx.x) * (D + 2);
-      st_dev(dst + e, acc);
-      if (e == 0) {
-        st_dev(dst + D, mw);
-        st_dev(dst + D + 1, lsum);
-      }
-    } else {
-      p.out[qrow + (size_t)h * D + e] = f2bf(acc / lsum);
-    }
-  }
+  merge_waves<D, G, kWaves>(red, !DECODE, p.out + qrow + (size_t)h0 * D,
+                          p.ws + ((size_t)(b * p.Hq + h0) * p.splits + blockIdx.x) * (D + 2), (size_t)p.splits * (D + 2));
   if (!DECODE) return;
 
   // The last workgroup of this (sequence, kv head) to finish merges the splits.  The
@@ -448,12 +502,8 @@ __global__ __launch_bounds__(kThreads) void sdpa_kernel(const SdpaParams p) {
   }
   __syncthreads();
   if (!s_last) return;
-  for (int idx = threadIdx.x; idx < G * D; idx += kThreads) {
-    const int g = idx / D, e = idx % D;
-    const int h = h0 + g;
-    const float* src = p.ws + (size_t)(b * p.Hq + h) * p.splits * (D + 2);
-    p.out[qrow + (size_t)h * D + e] = f2bf(merge_splits<D>(src, p.splits, e));
-  }
+  merge_heads<D, G, kThreads>(p.ws + (size_t)(b * p.Hq + h0) * p.splits * (D + 2), (size_t)p.splits * (D + 2), p.splits,
+                             p.out + qrow + (size_t)h0 * D);
 }
 
 // ---------------------------------------------------------------- decode, interleaved tiles
@@ -475,7 +525,7 @@ __global__ __launch_bounds__(64 * NW) void sdpa_tiles_kernel(const SdpaParams p)
   constexpr int KPI = 64 / LPK;     // keys per wave instruction
   constexpr int STEP = KPI * kBlk;  // keys per tile
   constexpr int NT = kTilesInFlight;
-  __shared__ float red[NW][G][D + 2];
+  __shared__ __attribute__((aligned(16))) float red[NW][G][D + 4];
   __shared__ int s_last;
 
   const int lane = threadIdx.x & 63;
@@ -691,32 +741,8 @@ __global__ __launch_bounds__(64 * NW) void sdpa_tiles_kernel(const SdpaParams p)
   }
   __syncthreads();
 
-  // merge the waves; thread -> (head, element); partial results at device scope (the merging
-  // workgroup may run on another XCD, whose L2 is not coherent with this one)
-  for (int idx = threadIdx.x; idx < G * D; idx += 64 * NW) {
-    const int g = idx / D, e = idx % D;
-    float mw = red[0][g][D];
-#pragma unroll
-    for (int w = 1; w < NW; ++w) mw = fmaxf(mw, red[w][g][D]);
-    float acc = 0.f, lsum = 0.f;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      const float mm = red[w][g][D];
-      const float sc = (mm == -INFINITY) ? 0.f : __expf(mm - mw);
-      acc += red[w][g][e] * sc;
-      lsum += red[w][g][D + 1] * sc;
-    }
-    if (solo) {
-      p.out[qrow + (size_t)(h0 + g) * D + e] = f2bf(acc / lsum);
-      continue;
-    }
-    float* dst = p.ws + ((size_t)(b * p.Hq + h0 + g) * p.splits + blockIdx.x) * (D + 2);
-    st_dev(dst + e, acc);
-    if (e == 0) {
-      st_dev(dst + D, mw);
-      st_dev(dst + D + 1, lsum);
-    }
-  }
+  merge_waves<D, G, NW>(red, solo, p.out + qrow + (size_t)h0 * D,
+                          p.ws + ((size_t)(b * p.Hq + h0) * p.splits + blockIdx.x) * (D + 2), (size_t)p.splits * (D + 2));
   if (solo) return;
   // the last workgroup of this (sequence, kv head, head group) to finish merges the splits
   // (see sdpa_kernel); the counter returns to zero
@@ -730,12 +756,8 @@ __global__ __launch_bounds__(64 * NW) void sdpa_tiles_kernel(const SdpaParams p)
   }
   __syncthreads();
   if (!s_last) return;
-  for (int idx = threadIdx.x; idx < G * D; idx += 64 * NW) {
-    const int g = idx / D, e = idx % D;
-    const int h = h0 + g;
-    const float* src = p.ws + (size_t)(b * p.Hq + h) * p.splits * (D + 2);
-    p.out[qrow + (size_t)h * D + e] = f2bf(merge_splits<D>(src, p.splits, e));
-  }
+  merge_heads<D, G, 64 * NW>(p.ws + (size_t)(b * p.Hq + h0) * p.splits * (D + 2), (size_t)p.splits * (D + 2), p.splits,
+                             p.out + qrow + (size_t)h0 * D);
 }
 
 typedef short short4_t __attribute__((ext_vector_type(4)));
@@ -757,13 +779,19 @@ __device__ __forceinline__ uint2 lds_read_tr16(const bf16_t* p) {
 //   O^T[d][head]  += V^T . P^T   A = V^T: 8 keys of one d per lane, out of the row-major V
 //                                tile with two transposing LDS reads; B = the S^T registers
 // as in the prefill kernel (same permuted key order, same per-lane softmax state).
-// Work split: grid (splits, Hkv, B); a workgroup's four waves take a quarter of the split's
-// keys each, in tiles of 32 that go global -> registers -> the wave's own LDS region (no
-// block barrier in the loop).  The new token's key and value come from registers / LDS and
-// are added by wave 0 of the split that owns position len-1.  The partial results leave in
-// the layout of the scalar kernel, so the merge of waves and splits is the same code.
+// Work split: grid (splits, Hkv, B); tiles of 32 keys are dealt to the waves of all splits and go
+// global -> registers -> the wave's own LDS region (no block barrier in the loop).  The new token's
+// key and value come from registers / LDS and are added by wave 0 of the last split that takes part.
+// The partial results leave in the layout of the scalar kernel, so the merge of waves and splits is the same code.
+// What bounds it: from thousands of keys the memory (16 sequences of 12290 keys 5.8 TB/s); below, the chain position ->
+// first tile and rope row -> rotation -> products -> merge of the waves (5.4 us with 20 keys) and 3 us of
+// hand-over.  8 sequences of 32 / 8 heads, 2050 keys 20.5 -> 17.9 us (ranges of whole rounds of 128 keys, as they were,
+// gave three of four splits five tiles a wave and the last one), 1030 keys 15.1 -> 13.1, 300 keys 10.5 -> 8.8; 250
+// keys, where two of six waves have a second tile, 8.1 -> 8.4; 4 of 32 / 4 heads, 1030 keys 13.3 -> 10.0; 8 of 64 / 4,
+// 1030 keys 20.9 -> 13.5; one of 64 / 4, 16000 keys 32.3 -> 23.4.
 template <int G>
-__global__ __launch_bounds__(kThreads, 2) void sdpa_decode_mfma_kernel(const SdpaParams p) {
+__global__ __launch_bounds__(64 * kMfmaWaves<G>) void sdpa_decode_mfma_kernel(const SdpaParams p) {
+  constexpr int NW = kMfmaWaves<G>;
   constexpr int D = 128;
   constexpr int TK = 32;          // keys per tile
   constexpr int KS = D + 8;       // LDS row stride (bf16)
@@ -771,8 +799,9 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_decode_mfma_kernel(const Sdp
   constexpr int VS = D + 16;      // V rows: 32 bytes past a multiple of the 256-byte bank span
   constexpr int TILE = TK * KS;   // bf16 elements of a K tile
   constexpr int WAVE_TILES = TK * KS + TK * VS;  // K tile + V tile of one wave
-  constexpr int TILE_BYTES = kWaves * WAVE_TILES * 2;
-  constexpr int RED_BYTES = kWaves * G * (D + 2) * 4;
+  constexpr int TILE_BYTES = NW * WAVE_TILES * 2;
+  constexpr int RS = D + 4;       // floats of a head's partial: whole 16-byte pieces
+  constexpr int RED_BYTES = NW * G * RS * 4;
   constexpr int SMEM = TILE_BYTES > RED_BYTES ? TILE_BYTES : RED_BYTES;
   __shared__ __attribute__((aligned(16))) char smem[SMEM];
   __shared__ __attribute__((aligned(16))) bf16_t q_lds[G * D];
@@ -786,43 +815,45 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_decode_mfma_kernel(const Sdp
   const int h0 = kvh * G;
   const int len = min(p.pos[b] + 1, p.S_max);
   // the cache holds keys [0, len-1); key len-1 comes from the qkv row
-  int chunk = (len + p.splits - 1) / p.splits;
-  chunk = (chunk + TK * kWaves - 1) / (TK * kWaves) * (TK * kWaves);
-  if (len <= kSoloMfma) chunk = kSoloMfma;
-  const int used = (len + chunk - 1) / chunk;  // splits that have keys; the others are gone at once
-  if ((int)blockIdx.x >= used) return;
-  const bool own_new = (len - 1) / chunk == (int)blockIdx.x;
-  const int k_begin = min(min((int)blockIdx.x * chunk, len), len - 1);
-  const int k_end = min(min((int)blockIdx.x * chunk + chunk, len), len - 1);
-  const int per_wave = ((k_end - k_begin + kWaves - 1) / kWaves + TK - 1) / TK * TK;
-  const int w_begin = min(k_begin + wave * per_wave, k_end);
-  const int w_end = min(w_begin + per_wave, k_end);
+  // Tiles of 32 keys are dealt round robin over the waves of all splits that take part, so that every wave has the
+  // same number to within one whatever the length.  A short context is left to one workgroup alone.
+  const int cached = len - 1, tiles = (cached + TK - 1) / TK;
+  const int used = len <= kSoloMfma ? 1 : min(p.splits, (tiles + kMfmaSplitTiles - 1) / kMfmaSplitTiles);
+  if ((int)blockIdx.x >= used) return;  // (splits without work are gone at once)
+  const bool own_new = (int)blockIdx.x == used - 1;
+  const int w_begin = (wave * used + (int)blockIdx.x) * TK, w_step = NW * used * TK;
 
   const size_t head_base = ((size_t)b * p.Hkv + kvh) * p.S_max * D;
   const bf16_t* kb = p.kc + head_base;
   const bf16_t* vb = p.vc + head_base;
   // tile loads: 16-byte chunk vi = lane + 64*i of the tile is (key vi/16, chunk vi%16)
-  // (always executed, with clamped keys, so that the tile registers are plain values: a
-  // conditional refill made the compiler keep them in scratch memory and wait for every
-  // load right after issuing it)
   // (eight named registers each, not arrays: those stayed in scratch memory here)
   uint4 k0r, k1r, k2r, k3r, k4r, k5r, k6r, k7r, v0r, v1r, v2r, v3r, v4r, v5r, v6r, v7r;
-#define EXO_LOAD1(I, K0)                                                                \
+#define EXO_LOAD1(R, P, I, K0)                                                          \
   {                                                                                     \
     const int vi = lane + 64 * I;                                                       \
-    const int key = max(min((K0) + (vi >> 4), w_end - 1), 0); /* past the range: masked */ \
-    k##I##r = *reinterpret_cast<const uint4*>(kb + (size_t)key * D + (vi & 15) * 8);    \
-    v##I##r = *reinterpret_cast<const uint4*>(vb + (size_t)key * D + (vi & 15) * 8);    \
+    const int key = max(min((K0) + (vi >> 4), cached - 1), 0); /* past the range: masked */ \
+    R##I##r = *reinterpret_cast<const uint4*>(P + (size_t)key * D + (vi & 15) * 8);     \
   }
-#define EXO_LOAD_TILE(K0) \
-  EXO_LOAD1(0, K0) EXO_LOAD1(1, K0) EXO_LOAD1(2, K0) EXO_LOAD1(3, K0) EXO_LOAD1(4, K0) EXO_LOAD1(5, K0) EXO_LOAD1(6, K0) EXO_LOAD1(7, K0)
-#define EXO_STORE1(I)                                                                  \
-  {                                                                                    \
-    const int vi = lane + 64 * I;                                                      \
-    *reinterpret_cast<uint4*>(&k_t[(vi >> 4) * KS + (vi & 15) * 8]) = k##I##r;         \
-    *reinterpret_cast<uint4*>(&v_t[(vi >> 4) * VS + (vi & 15) * 8]) = v##I##r;         \
+#define EXO_LOAD_K(K0) \
+  EXO_LOAD1(k, kb, 0, K0) EXO_LOAD1(k, kb, 1, K0) EXO_LOAD1(k, kb, 2, K0) EXO_LOAD1(k, kb, 3, K0) EXO_LOAD1(k, kb, 4, K0) EXO_LOAD1(k, kb, 5, K0) EXO_LOAD1(k, kb, 6, K0) EXO_LOAD1(k, kb, 7, K0)
+#define EXO_LOAD_V(K0) \
+  EXO_LOAD1(v, vb, 0, K0) EXO_LOAD1(v, vb, 1, K0) EXO_LOAD1(v, vb, 2, K0) EXO_LOAD1(v, vb, 3, K0) EXO_LOAD1(v, vb, 4, K0) EXO_LOAD1(v, vb, 5, K0) EXO_LOAD1(v, vb, 6, K0) EXO_LOAD1(v, vb, 7, K0)
+#define EXO_STORE1(R, T, S, I)                                            \
+  {                                                                       \
+    const int vi = lane + 64 * I;                                         \
+    *reinterpret_cast<uint4*>(&T[(vi >> 4) * S + (vi & 15) * 8]) = R##I##r; \
   }
-  EXO_LOAD_TILE(w_begin)  // in flight during the q work
+#define EXO_STORE_K EXO_STORE1(k, k_t, KS, 0) EXO_STORE1(k, k_t, KS, 1) EXO_STORE1(k, k_t, KS, 2) EXO_STORE1(k, k_t, KS, 3) EXO_STORE1(k, k_t, KS, 4) EXO_STORE1(k, k_t, KS, 5) EXO_STORE1(k, k_t, KS, 6) EXO_STORE1(k, k_t, KS, 7)
+#define EXO_STORE_V EXO_STORE1(v, v_t, VS, 0) EXO_STORE1(v, v_t, VS, 1) EXO_STORE1(v, v_t, VS, 2) EXO_STORE1(v, v_t, VS, 3) EXO_STORE1(v, v_t, VS, 4) EXO_STORE1(v, v_t, VS, 5) EXO_STORE1(v, v_t, VS, 6) EXO_STORE1(v, v_t, VS, 7)
+  // in flight during the q work.  (A wave without a tile requests nothing: 64 lanes' 16 bytes occupy the CU's address
+  // unit whatever they hit.)
+  k0r = k1r = k2r = k3r = k4r = k5r = k6r = k7r = v0r = v1r = v2r = v3r = v4r = v5r = v6r = v7r = make_uint4(0, 0, 0, 0);
+  if (w_begin < cached) {
+    EXO_LOAD_K(w_begin)
+    __builtin_amdgcn_sched_barrier(0);
+    EXO_LOAD_V(w_begin)
+  }
 
   // ---- q of the G heads (RoPE, optional head norm) -> LDS; the new token's k and v
   {
@@ -845,10 +876,10 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_decode_mfma_kernel(const Sdp
       for (int e = 0; e < 8; ++e) sincosf(fpos * p.inv_freq[(sl * 8 + e) % (D / 2)], &sn[e], &cs[e]);
     }
     const bf16_t* row = p.qkv + (size_t)b * (p.Hq + 2 * p.Hkv) * D;
-    for (int g = wave * 4 + sub; g < G; g += 4 * kWaves)  // a 16-lane group per head
+    for (int g = wave * 4 + sub; g < G; g += 4 * NW)  // a 16-lane group per head
       *reinterpret_cast<uint4*>(&q_lds[g * D + sl * 8]) =
           head_slice<D, true>(row + (size_t)(h0 + g) * D, sl, p.qn, p.eps, cs, sn);
-    if (own_new && wave == kWaves - 1 && sub < 2) {
+    if (own_new && wave == NW - 1 && sub < 2) {
       const uint4 t = sub == 0 ? head_slice<D, true>(row + (size_t)(p.Hq + kvh) * D, sl, p.kn, p.eps, cs, sn)
                                : head_slice<D, false>(row + (size_t)(p.Hq + p.Hkv + kvh) * D, sl, nullptr, 0.f, cs, sn);
       *reinterpret_cast<uint4*>(&kv_new[sub * D + sl * 8]) = t;
@@ -879,12 +910,15 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_decode_mfma_kernel(const Sdp
     for (int e = 0; e < 16; ++e) o[dt][e] = 0.f;
   float m_run = -INFINITY, l_run = 0.f;  // log2 domain
 
-  for (int k0 = w_begin; k0 < w_end; k0 += TK) {
-    EXO_STORE1(0) EXO_STORE1(1) EXO_STORE1(2) EXO_STORE1(3) EXO_STORE1(4) EXO_STORE1(5) EXO_STORE1(6) EXO_STORE1(7)
-    // the tile is private to the wave: its writes are complete before its reads
+  // the tile is private to the wave: its writes are complete before its reads
+  auto tile_written = [] {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_wave_barrier();
-    EXO_LOAD_TILE(k0 + TK)
+  };
+  for (int k0 = w_begin; k0 < cached; k0 += w_step) {
+    // (keys and values apart: the scores do not wait for the values)
+    EXO_STORE_K
+    tile_written();
 
     floatx16 sc;
 #pragma unroll
@@ -899,7 +933,15 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_decode_mfma_kernel(const Sdp
                                                      __builtin_bit_cast(bf16x8_t, qv), sc, 0, 0, 0);
       }
     }
-    const int vis = w_end - k0;  // keys [0, vis) of the tile are real
+    EXO_STORE_V
+    tile_written();
+    if (k0 + w_step < cached) {
+      EXO_LOAD_K(k0 + w_step)
+      __builtin_amdgcn_sched_barrier(0);
+      EXO_LOAD_V(k0 + w_step)
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const int vis = cached - k0;  // keys [0, vis) of the tile are real
     float mx = -INFINITY;
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
@@ -979,19 +1021,23 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_decode_mfma_kernel(const Sdp
       }
   }
 
-#undef EXO_LOAD_TILE
+#undef EXO_LOAD_K
+#undef EXO_LOAD_V
 #undef EXO_LOAD1
+#undef EXO_STORE_K
+#undef EXO_STORE_V
 #undef EXO_STORE1
   // ---- partial results of the waves, in the scalar kernel's layout: red[wave][head][d],
   // then (max, sum) in natural-log units
   __syncthreads();  // every wave is done with its tiles: the memory changes hands
-  float (*red)[G][D + 2] = reinterpret_cast<float (*)[G][D + 2]>(smem);
+  float (&red)[NW][G][RS] = *reinterpret_cast<float (*)[NW][G][RS]>(smem);
   if (n < G) {
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
-        red[wave][n][dt * 32 + 8 * (r >> 2) + 4 * kq + (r & 3)] = o[dt][r];
+      for (int r = 0; r < 16; r += 4)
+        *reinterpret_cast<float4*>(&red[wave][n][dt * 32 + 2 * r + 4 * kq]) =
+            make_float4(o[dt][r], o[dt][r + 1], o[dt][r + 2], o[dt][r + 3]);
     if (kq == 0) {
       red[wave][n][D] = m_run * 0.6931471805599453f;
       red[wave][n][D + 1] = l_run;
@@ -1000,30 +1046,8 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_decode_mfma_kernel(const Sdp
   __syncthreads();
 
   const size_t qrow = (size_t)b * p.Hq * D;
-  for (int idx = threadIdx.x; idx < G * D; idx += kThreads) {
-    const int g = idx / D, e = idx % D;
-    float mw = red[0][g][D];
-#pragma unroll
-    for (int w = 1; w < kWaves; ++w) mw = fmaxf(mw, red[w][g][D]);
-    float acc = 0.f, lsum = 0.f;
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) {
-      const float mm = red[w][g][D];
-      const float scw = (mm == -INFINITY) ? 0.f : __expf(mm - mw);
-      acc += red[w][g][e] * scw;
-      lsum += red[w][g][D + 1] * scw;
-    }
-    if (used == 1) {  // (nothing to hand over)
-      p.out[qrow + (size_t)(h0 + g) * D + e] = f2bf(acc / lsum);
-      continue;
-    }
-    float* dst = p.ws + ((size_t)(b * p.Hq + h0 + g) * p.splits + blockIdx.x) * (D + 2);
-    st_dev(dst + e, acc);
-    if (e == 0) {
-      st_dev(dst + D, mw);
-      st_dev(dst + D + 1, lsum);
-    }
-  }
+  merge_waves<D, G, NW, 2>(red, used == 1, p.out + qrow + (size_t)h0 * D,
+                          p.ws + ((size_t)(b * p.Hq + h0) * p.splits + blockIdx.x) * (D + 2), (size_t)p.splits * (D + 2));
   if (used == 1) return;
   // the last workgroup of this (sequence, kv head) merges the splits (see sdpa_kernel)
   wait_own_stores_done();
@@ -1036,12 +1060,8 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_decode_mfma_kernel(const Sdp
   }
   __syncthreads();
   if (!s_last) return;
-  for (int idx = threadIdx.x; idx < G * D; idx += kThreads) {
-    const int g = idx / D, e = idx % D;
-    const int h = h0 + g;
-    const float* src = p.ws + (size_t)(b * p.Hq + h) * p.splits * (D + 2);
-    p.out[qrow + (size_t)h * D + e] = f2bf(merge_splits<D>(src, used, e));
-  }
+  merge_heads<D, G, 64 * NW, 2, true>(p.ws + (size_t)(b * p.Hq + h0) * p.splits * (D + 2), (size_t)p.splits * (D + 2), used,
+                             p.out + qrow + (size_t)h0 * D);
 }
 
 // Decode work split.  The G = Hq/Hkv query heads of a kv head are spread over `hgroups`
@@ -1310,11 +1330,11 @@ extern "C" int exo_attn_decode_hint(const uint16_t* qkv, uint16_t* k_cache, uint
     const dim3 grid(p.splits, Hkv, B);
     exo_note_variant("sdpa_decode_mfma<%d> grid=%dx%dx%d", G, (int)grid.x, (int)grid.y, (int)grid.z);
     if (G == 4)
-      sdpa_decode_mfma_kernel<4><<<grid, kThreads, 0, (hipStream_t)stream>>>(p);
+      sdpa_decode_mfma_kernel<4><<<grid, 64 * kMfmaWaves<4>, 0, (hipStream_t)stream>>>(p);
     else if (G == 8)
-      sdpa_decode_mfma_kernel<8><<<grid, kThreads, 0, (hipStream_t)stream>>>(p);
+      sdpa_decode_mfma_kernel<8><<<grid, 64 * kMfmaWaves<8>, 0, (hipStream_t)stream>>>(p);
     else
-      sdpa_decode_mfma_kernel<16><<<grid, kThreads, 0, (hipStream_t)stream>>>(p);
+      sdpa_decode_mfma_kernel<16><<<grid, 64 * kMfmaWaves<16>, 0, (hipStream_t)stream>>>(p);
     EXO_CHECK_LAUNCH("exo_attn_decode");
     return EXO_OK;
   }
