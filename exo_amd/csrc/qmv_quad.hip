@@ -30,9 +30,6 @@ namespace {
 typedef short short4_t __attribute__((ext_vector_type(4)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 
-#ifndef EXO_QUAD_ABL
-#define EXO_QUAD_ABL 0  // timing-only ablations (wrong results): 1 no products, 2 no lane permutation
-#endif
 #ifndef EXO_QMV_QUAD_MAX_DEPTH
 #define EXO_QMV_QUAD_MAX_DEPTH 6
 #endif
@@ -199,13 +196,8 @@ __global__ __launch_bounds__(MSETS == 4 ? 512 : 1024) void qmv_quad_kernel(const
       for (int a = 0; a < NMAT; ++a) {
         bf.w[a][sl] = __builtin_bit_cast(
             uint4, __builtin_amdgcn_raw_buffer_load_b128(rw[a], wofs + sl * 256, wq, 0));
-#if (EXO_QUAD_ABL & 4)
-        bf.s[a][sl] = 0x3c00;
-        bf.b[a][sl] = 0x3c00;
-#else
         bf.s[a][sl] = (bf16_t)__builtin_amdgcn_raw_buffer_load_b16(rs[a], sofs + sl * (16 / CPG) * 2, sq, 0);
         bf.b[a][sl] = (bf16_t)__builtin_amdgcn_raw_buffer_load_b16(rb[a], sofs + sl * (16 / CPG) * 2, sq, 0);
-#endif
         if (pin) __builtin_amdgcn_sched_barrier(0);
       }
   };
@@ -335,10 +327,6 @@ __global__ __launch_bounds__(MSETS == 4 ? 512 : 1024) void qmv_quad_kernel(const
       for (int a = 0; a < NMAT; ++a) {
         // load layout -> operand layout
         uint32_t wd[4];
-#if (EXO_QUAD_ABL & 2)
-        wd[0] = bf.w[a][sl].x; wd[1] = bf.w[a][sl].y; wd[2] = bf.w[a][sl].z; wd[3] = bf.w[a][sl].w;
-        const uint32_t sbw = (uint32_t)bf.s[a][sl] | ((uint32_t)bf.b[a][sl] << 16);
-#else
         wd[0] = (uint32_t)__builtin_amdgcn_ds_bpermute(perm_src, (int)bf.w[a][sl].x);
         wd[1] = (uint32_t)__builtin_amdgcn_ds_bpermute(perm_src, (int)bf.w[a][sl].y);
         wd[2] = (uint32_t)__builtin_amdgcn_ds_bpermute(perm_src, (int)bf.w[a][sl].z);
@@ -350,7 +338,6 @@ __global__ __launch_bounds__(MSETS == 4 ? 512 : 1024) void qmv_quad_kernel(const
         asm volatile("" : "+v"(s_raw), "+v"(b_raw));
         const uint32_t sbw =
             (uint32_t)__builtin_amdgcn_ds_bpermute(perm_src, (int)(s_raw | (b_raw << 16)));
-#endif
         const float sc = bf_lo(sbw), bi = bf_hi(sbw);
         float4_t dq[MSETS];
 #pragma unroll
@@ -362,17 +349,11 @@ __global__ __launch_bounds__(MSETS == 4 ? 512 : 1024) void qmv_quad_kernel(const
           const uint32_t p2 = ((wd[t] >> 8) & kmask) | kmagic;
           const uint32_t p3 = ((wd[t] >> 12) & kmask) | kmagic;
           const short4_t b0 = as_s4(p0, p1), b1 = as_s4(p2, p3);
-#if (EXO_QUAD_ABL & 1)
-          for (int set = 0; set < MSETS; ++set)
-            dq[set][0] += __builtin_bit_cast(float, p0 ^ p1 ^ p2 ^ p3);
-          (void)b0; (void)b1;
-#else
 #pragma unroll
           for (int set = 0; set < MSETS; ++set) {
             dq[set] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(xa[set][sl][t][0], b0, dq[set], 0, 0, 0);
             dq[set] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(xa[set][sl][t][1], b1, dq[set], 0, 0, 0);
           }
-#endif
         }
 #pragma unroll
         for (int set = 0; set < MSETS; ++set)
