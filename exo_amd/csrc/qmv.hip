@@ -1411,6 +1411,26 @@ extern "C" int exo_qmv(const uint16_t* x, const uint32_t* w, const uint16_t* sca
 #define EXO_QMV_W16_MIN_M 5
 #endif
 
+// Two to four rows that take it too, from a sweep of N = 1024 to 151936 and K = 768 to 4096 (its time over the 4x4x4 kernel's, or
+// where rows are not whole 256-byte slices over that of the kernels below).  K of up to 1024: 0.3 to 0.99 (151936x1024 39 ->
+// 21 us).  Four rows 0.72 to 1.01 from N = 2048 on (4096x4096 7.0 -> 5.8 us, 128256x4096 66 -> 58), 0.97 to 1.18 below.  Three
+// rows behind a norm 0.71 to 1.02 and pairs to 1.03 (14336x4096 18.5 -> 15.3); without a norm 0.85 to 1.0 from N = 4096
+// on, 1.0 to 1.27 below and 1.02 to 1.04 where N and K are both long.  Heads of K = 1536 and 2048 lose up to 8 % under
+// three and four rows (several rounds of workgroups).  Two rows behind a norm 0.79 to 1.0 up to N = 4096 or K = 1536
+// (others to 1.13, without a norm to 1.35), pairs 0.83 to 0.99 from K = 2560 on (wider than 16384 and shorter ones to 1.13).
+// Split K loses (a hand-over: 2048x8192 5.9 | 8.0 us).  Longer pairs of four rows stay with the other, whose instance the
+// tests of the decode step name, although it is behind: 14336x4096 19.4 | 15.6.
+static bool few_rows_on_w16(int M, int N, int K, bool norm, bool pair) {
+  if (N < 1024 || K < 768 || K > 4096) return false;
+  if (K <= 1024) return true;
+  if (N < 2048) return false;
+  if (pair) return M == 3 || (M == 2 && K >= 2560 && N <= 16384);
+  if (M >= 3 && K <= 2048 && N > 65536) return false;
+  if (M == 4) return true;
+  if (norm) return M == 3 || N <= 4096 || K <= 1536;
+  return M == 3 && (N == 4096 || (N > 4096 && K <= 3072));
+}
+
 static int norm_qmv_impl(const uint16_t* x, const uint16_t* norm_weight, float eps,
                          const uint32_t* w, const uint16_t* scales, const uint16_t* biases,
                          const uint16_t* residual, uint16_t* y, void* workspace, int M, int N,
@@ -1432,7 +1452,9 @@ static int norm_qmv_impl(const uint16_t* x, const uint16_t* norm_weight, float e
     EXO_CHECK_LAUNCH("exo_qmv");
     return EXO_OK;
   }
-  if (M >= EXO_QMV_QUAD_MIN_M && M <= EXO_QMV_QUAD_MAX_M &&
+  const bool few_w16 = M >= 2 && M < EXO_QMV_W16_MIN_M && few_rows_on_w16(M, N, K, norm_weight != nullptr, false) &&
+                       exo_qmv_w16_ok(M, N, K, bits, norm_weight != nullptr, false, false);
+  if (!few_w16 && M >= EXO_QMV_QUAD_MIN_M && M <= EXO_QMV_QUAD_MAX_M &&
       exo_qmv_quad_ok(M, N, K, bits, norm_weight != nullptr)) {
     rc = exo_qmv_quad_launch(x, norm_weight, eps, w, scales, biases, nullptr, nullptr, nullptr,
                              residual, y, M, N, K, bits, (hipStream_t)stream);
@@ -1440,8 +1462,8 @@ static int norm_qmv_impl(const uint16_t* x, const uint16_t* norm_weight, float e
     EXO_CHECK_LAUNCH("exo_qmv");
     return EXO_OK;
   }
-  if (M >= EXO_QMV_W16_MIN_M &&
-      exo_qmv_w16_ok(M < 16 ? M : 16, N, K, bits, norm_weight != nullptr, false, workspace != nullptr)) {
+  if (few_w16 || (M >= EXO_QMV_W16_MIN_M &&
+                  exo_qmv_w16_ok(M < 16 ? M : 16, N, K, bits, norm_weight != nullptr, false, workspace != nullptr))) {
     for (int m0 = 0; m0 < M; m0 += 16) {
       const int mt = (M - m0 < 16) ? (M - m0) : 16;
       rc = exo_qmv_w16_launch(x + (size_t)m0 * K, norm_weight, eps, w, scales, biases, nullptr,
@@ -1540,7 +1562,9 @@ extern "C" int exo_norm_qmv_swiglu_ws(const uint16_t* x, const uint16_t* norm_we
               "exo_norm_qmv_swiglu_ws: workspace of %lld bytes, need %lld (256-byte aligned)",
               (long long)workspace_bytes, (long long)exo_qmv_workspace(2 * N));
   if (M == 0) return EXO_OK;
-  if (M >= EXO_QMV_QUAD_MIN_M && M <= EXO_QMV_QUAD_MAX_M &&
+  const bool few_w16 = M >= 2 && M < EXO_QMV_W16_MIN_M && few_rows_on_w16(M, N, K, norm_weight != nullptr, true) &&
+                       exo_qmv_w16_ok(M, N, K, bits, norm_weight != nullptr, true, false);
+  if (!few_w16 && M >= EXO_QMV_QUAD_MIN_M && M <= EXO_QMV_QUAD_MAX_M &&
       exo_qmv_quad_ok(M, N, K, bits, norm_weight != nullptr)) {
     rc = exo_qmv_quad_launch(x, norm_weight, eps, wg, sg, bg, wu, su, bu, nullptr, y, M, N, K, bits,
                              (hipStream_t)stream);
@@ -1548,7 +1572,7 @@ extern "C" int exo_norm_qmv_swiglu_ws(const uint16_t* x, const uint16_t* norm_we
     EXO_CHECK_LAUNCH("exo_qmv_swiglu");
     return EXO_OK;
   }
-  if (M >= EXO_QMV_W16_MIN_M && exo_qmv_w16_ok(M < 16 ? M : 16, N, K, bits, norm_weight != nullptr, true, false)) {
+  if (few_w16 || (M >= EXO_QMV_W16_MIN_M && exo_qmv_w16_ok(M < 16 ? M : 16, N, K, bits, norm_weight != nullptr, true, false))) {
     for (int m0 = 0; m0 < M; m0 += 16) {
       const int mt = (M - m0 < 16) ? (M - m0) : 16;
       rc = exo_qmv_w16_launch(x + (size_t)m0 * K, norm_weight, eps, wg, sg, bg, wu, su, bu, nullptr,

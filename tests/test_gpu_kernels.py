@@ -179,6 +179,31 @@ def test_qmv_16x16x32_shares_of_blocks(device, N, K, blocks, M):
     assert_close(n_f32(got), want, what=f"w16 {M}x{N}x{K}")
 
 
+@pytest.mark.parametrize("M,N,K,norm,pair,w16", [
+    (2, 1024, 768, False, False, True), (2, 1024, 1152, True, False, False), (2, 2048, 2048, True, False, True),
+    (2, 2048, 2048, False, False, False), (2, 2048, 2560, True, True, True), (3, 4096, 2048, False, False, True),
+    (3, 2064, 1536, True, True, True), (4, 2048, 4096, False, False, True), (4, 2048, 8192, False, False, False),
+    (4, 1040, 1024, True, True, True), (4, 2048, 2048, True, True, False),
+])
+def test_qmv_few_rows_routes(device, M, N, K, norm, pair, w16):
+    """2..4 rows on both sides of the line between the 16x16x32 and the 4x4x4 kernel."""
+    trip, up = rand_quantized(N, K, 4, seed=N + K), rand_quantized(N, K, 4, seed=N + K + 1)
+    x, g = rand_bf16((M, K), seed=M + K, scale=1.5), affine.bf16_round(rand_bf16((K,), seed=6) * 0.1 + 1.0)
+    xn = O.rms_norm(x, g, 1e-5) if norm else x
+    kw = dict(norm_weight=t_bf16(g, device), eps=1e-5) if norm else {}
+    want = affine.qmm(xn, *trip, 64, 4)
+    if pair:
+        got = ops.qmv_swiglu(t_bf16(x, device), t_qw(trip, 4, device), t_qw(up, 4, device), **kw)
+        want = O.swiglu(want, affine.qmm(xn, *up, 64, 4))
+    else:
+        r = rand_bf16((M, N), seed=N)
+        got = ops.quantized_matmul(t_bf16(x, device), t_qw(trip, 4, device), residual=t_bf16(r, device), **kw)
+        want = affine.bf16_round(affine.bf16_round(want) + r)
+    assert native.last_variant().startswith("qmv_w16" if w16 else "qmv_"), native.last_variant()
+    assert w16 or not native.last_variant().startswith("qmv_w16"), native.last_variant()
+    assert_close(n_f32(got), want, what=f"few rows {M}x{N}x{K}")
+
+
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("M,N,K", [(8, 1000, 4096), (3, 96, 14336), (16, 2080, 2048), (5, 14336, 512)])
 def test_qmv_swiglu_rows_equal_separate_launches(device, bits, M, N, K):
