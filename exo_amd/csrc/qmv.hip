@@ -541,41 +541,26 @@ __global__ __launch_bounds__(kThreads) void qmv_rows_kernel(const QmvParams p) {
   const char* sb[NMAT];
   const char* bb[NMAT];
   // Base pointers of this workgroup's matrices.  Gather modes: the expert of its pair.
-  // Routing mode: wave 0 repeats the routing of the token, the others wait at one barrier;
-  // called once the activation loads are on their way, so that their latency covers it.
-  // In the register-resident layout every wave repeats it from logits it requested first
-  // (route_raw): no barrier at all.
+  // Routing mode: every wave repeats the routing of the token from logits that it requested first
+  // (route_raw), as far as its own slot; called once the activation loads are on their way, so
+  // that their latency covers it.  (All selections in every wave: 32 pairs of 768x2048 16.6 us against 16.0, 8 pairs
+  // 8.25 | 8.08.  In wave 0 with the others at a barrier, 8 pairs of 8-bit 1536x4096 25.7 | 24.0.)
   constexpr bool XR = kRowsXR<MT, ITERS, NMAT, ROUTE>;
-  __shared__ int s_expert;
   uint32_t route_raw[4] = {0, 0, 0, 0};
   auto select_matrices = [&]() {
     size_t ew = 0, eg = 0;
-    if (ROUTE && XR && p.route) {
+    if (ROUTE && p.route) {
       const int t = pair / p.topk, slot = pair - t * p.topk;
       int my_id;
       float my_p, tot;
-      route_topk_regs(route_raw, p.E, p.topk, lane, my_id, my_p, tot);
-      if (blockIdx.x == 0 && slot == 0 && wave == 0 && lane < p.topk) {
+      // (the selections up to its own slot; all of them where the routing is recorded)
+      const bool record = blockIdx.x == 0 && slot == 0 && wave == 0;
+      route_topk_regs(route_raw, p.E, record ? p.topk : slot + 1, lane, my_id, my_p, tot);
+      if (record && lane < p.topk) {
         p.route_idx[(size_t)t * p.topk + lane] = my_id;
         p.route_scores[(size_t)t * p.topk + lane] = route_score(my_p, tot, p.route_renorm);
       }
       const int e = __builtin_amdgcn_readlane(my_id, slot);
-      ew = (size_t)e * p.N * p.wpr;
-      eg = (size_t)e * p.N * G;
-    } else if (ROUTE && p.route) {
-      const int t = pair / p.topk, slot = pair - t * p.topk;
-      if (wave == 0) {
-        int my_id;
-        float my_p, tot;
-        route_topk_wave(p.route + (size_t)t * p.E, p.E, p.topk, lane, my_id, my_p, tot);
-        if (blockIdx.x == 0 && slot == 0 && lane < p.topk) {
-          p.route_idx[(size_t)t * p.topk + lane] = my_id;
-          p.route_scores[(size_t)t * p.topk + lane] = route_score(my_p, tot, p.route_renorm);
-        }
-        if (lane == slot) s_expert = my_id;
-      }
-      __syncthreads();
-      const int e = __builtin_amdgcn_readfirstlane(s_expert);
       ew = (size_t)e * p.N * p.wpr;
       eg = (size_t)e * p.N * G;
     } else if (p.idx) {
@@ -789,6 +774,7 @@ __global__ __launch_bounds__(kThreads) void qmv_rows_kernel(const QmvParams p) {
       if (nrows > b * R) issue(buf[b], r0 + b * R);
   } else {
     XStage<BITS, MT, ITERS> xst;
+    if (ROUTE && p.route) route_load(p.route + (size_t)(pair / p.topk) * p.E, p.E, lane, route_raw);
     stage_x_load<BITS, MT, ITERS>(p, xin, xst);
     select_matrices();
     if (nrows > 0) issue(buf[0], r0);
