@@ -22,6 +22,7 @@
 //    rows of a gate and an up matrix, 32 and 32, so that a wave's column tiles are (gate, up) of the
 //    same outputs and the gated unit is its epilogue.
 //    GROUPED: the rows are one expert's (token, slot) pairs, from exo_moe_group's tile list.
+//  * dense_gemm_wide_kernel: 256 x 256 tiles for bf16 launches of enough of them.
 // Either may send its last output columns to a second, float32 buffer: inputs of 32-bit arithmetic
 // (step sizes, gates, decays) are rows of the same weight matrix as the bf16 projections.
 #include "../../include/exo_mi355x.h"
@@ -319,6 +320,124 @@ struct GemmParams {
   float* part;         // [ksplit][M][N]
 };
 
+// A wave's results, accumulators acc[i][j] of the 32 x 32 tiles at row wm + 32 i, weight row wn + 32 j of the workgroup's tile;
+// wcol: the wave's place among those side by side.
+template <typename T, int MI, int NJ, bool GROUPED, bool PAIR>
+__device__ __forceinline__ void store_tile(const GemmParams& p, floatx16 (&acc)[MI][NJ], int n0, int m0, int m_end, int wm, int wn,
+                                           int wcol, int lane, const int* row_pair) {
+  const int frow = lane & 31, half = lane >> 5;
+  // ---- epilogue: element e of tile (i, j): row wm + 32 i + 8 (e / 4) + 4 half + e % 4, column lane
+  // One plain output (its last columns may go to the float32 buffer), or a partial one: every store at 32-bit
+  // offsets from the tile's first row, rows past the end dropped by the buffer's range, columns of the other
+  // buffer and past N by an offset beyond it.  (The whole offset is in the vector register: the scalar one takes
+  // no part in the range check.)  Element by element, as in the loop at the end, 13664 columns of K = 2048 with
+  // 96 in the second buffer under 1004 rows took 108 us, here 78; 6208 columns 52.5, here 38.
+  if (!GROUPED && !PAIR && (p.ksplit > 1 || (!p.ep.mul && (p.n1 == p.N || p.ldy2 < 1 << 22)))) {
+    const bool part = p.ksplit > 1, f32 = part || p.y_f32 || sizeof(T) == 4;
+    const uint32_t ld = part ? (uint32_t)p.N : (uint32_t)p.ldy, size = f32 ? 4 : 2;
+    const int n1 = part ? p.N : p.n1, held = m_end - m0;
+    char* base = part ? reinterpret_cast<char*>(p.part + ((size_t)blockIdx.z * p.M + m0) * p.N)
+                      : reinterpret_cast<char*>(p.y) + (size_t)m0 * ld * size;
+    const __amdgpu_buffer_rsrc_t ry = buf_of(base, (uint32_t)held * ld * size);
+    const uint32_t ld2 = n1 < p.N ? (uint32_t)p.ldy2 : 0;
+    const __amdgpu_buffer_rsrc_t ry2 = buf_of(p.y2 + (size_t)m0 * ld2, (uint32_t)held * ld2 * 4);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const int c0 = n0 + wn + 32 * j, n = c0 + frow;
+      if (!part && p.bias) {
+        const float b = n < p.N ? p.bias[n] : 0.f;
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) acc[i][j][e] += b;
+      }
+      auto store = [&](uint32_t voff, uint32_t row_bytes, auto put) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) put(acc[i][j][e], voff + (uint32_t)(32 * i + 8 * (e >> 2) + (e & 3)) * row_bytes);
+      };
+      auto put32 = [](const __amdgpu_buffer_rsrc_t& to, float v, uint32_t at) __attribute__((always_inline)) {
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), to, at, 0, 0);
+      };
+      if (c0 + 32 > n1 && n1 < p.N)  // (uniform)
+        store(n >= n1 && n < p.N ? ((uint32_t)(wm + 4 * half) * ld2 + (n - n1)) * 4 : kPastEnd, ld2 * 4,
+              [&](float v, uint32_t at) __attribute__((always_inline)) { put32(ry2, v, at); });
+      if (c0 >= n1) continue;
+      if (!part && p.ep.act) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) acc[i][j][e] = activated(acc[i][j][e], p.ep.act, p.ep.cap);
+      }
+      const uint32_t voff = n < n1 ? ((uint32_t)(wm + 4 * half) * ld + n) * size : kPastEnd;
+      if (f32)
+        store(voff, ld * size, [&](float v, uint32_t at) __attribute__((always_inline)) { put32(ry, v, at); });
+      else
+        store(voff, ld * size, [&](float v, uint32_t at) __attribute__((always_inline)) {
+          __builtin_amdgcn_raw_buffer_store_b16(f2bf(v), ry, at, 0, 0);
+        });
+    }
+    return;
+  }
+  // Gated pairs and an expert's rows, in the element type: the same with a row's offset from the list of
+  // pairs (four consecutive tile rows at a time).
+  if (GROUPED || PAIR) {
+    const uint32_t ld = (uint32_t)p.ldy * sizeof(T);
+    char* base = reinterpret_cast<char*>(p.y) + (GROUPED ? 0 : (size_t)m0 * ld);
+    const __amdgpu_buffer_rsrc_t ry = buf_of(base, GROUPED ? kPastEnd : (uint32_t)(m_end - m0) * ld);
+    constexpr int JS = PAIR ? 2 : 1;  // accumulators per output
+    uint32_t coff[NJ / JS];
+#pragma unroll
+    for (int j = 0; j < NJ / JS; ++j) {
+      const int n = PAIR ? n0 + wcol * (16 * NJ) + j * 32 + frow : n0 + wn + 32 * j + frow;
+      coff[j] = n < p.N ? (uint32_t)n * sizeof(T) : kPastEnd;
+    }
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int t0 = wm + 32 * i + 8 * k + 4 * half;
+        int rows[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) rows[e] = GROUPED ? row_pair[t0 + e] : t0 + e;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const bool in = GROUPED ? t0 + e < m_end : true;  // (not grouped: by the range)
+#pragma unroll
+          for (int j = 0; j < NJ / JS; ++j) {
+            float v = acc[i][JS * j][4 * k + e];
+            if (PAIR) v = gated<T>(v, acc[i][JS * j + JS - 1][4 * k + e], p.glu);
+            const uint32_t off = in && coff[j] != kPastEnd ? (uint32_t)rows[e] * ld + coff[j] : kPastEnd;
+            if (sizeof(T) == 4)
+              __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), ry, off, 0, 0);
+            else
+              __builtin_amdgcn_raw_buffer_store_b16(f2bf(v), ry, off, 0, 0);
+          }
+        }
+      }
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int tr = wm + 32 * i + 8 * (e >> 2) + 4 * half + (e & 3);
+      if (m0 + tr >= m_end) continue;
+      const size_t row = (size_t)(m0 + tr);
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        const int n = n0 + wn + 32 * j + frow;
+        if (n >= p.N) continue;
+        const float v = acc[i][j][e] + (p.bias ? p.bias[n] : 0.f);
+        if (n < p.n1)
+          store_out<T>(p.y, row * p.ldy + n, finish<T>(v, row, n, p.ep), p.y_f32);
+        else
+          p.y2[row * p.ldy2 + n - p.n1] = v;
+      }
+    }
+}
+
 template <typename T, int MI, int NJ, bool GROUPED, bool PAIR>
 __global__ __launch_bounds__(256, 2) void dense_gemm_kernel(const GemmParams p) {
   constexpr int BM = 64 * MI, BW = 64 * NJ;      // tile rows of x, of weights
@@ -449,129 +568,151 @@ __global__ __launch_bounds__(256, 2) void dense_gemm_kernel(const GemmParams p) 
     }
   }
 
-  // ---- epilogue: element e of tile (i, j): row wm + 32 i + 8 (e / 4) + 4 half + e % 4, column lane
-  // One plain output (its last columns may go to the float32 buffer), or a partial one: every store at 32-bit
-  // offsets from the tile's first row, rows past the end dropped by the buffer's range, columns of the other
-  // buffer and past N by an offset beyond it.  (The whole offset is in the vector register: the scalar one takes
-  // no part in the range check.)  Element by element, as in the loop at the end, 13664 columns of K = 2048 with
-  // 96 in the second buffer under 1004 rows took 108 us, here 78; 6208 columns 52.5, here 38.
-  if (!GROUPED && !PAIR && (p.ksplit > 1 || (!p.ep.mul && (p.n1 == p.N || p.ldy2 < 1 << 22)))) {
-    const bool part = p.ksplit > 1, f32 = part || p.y_f32 || sizeof(T) == 4;
-    const uint32_t ld = part ? (uint32_t)p.N : (uint32_t)p.ldy, size = f32 ? 4 : 2;
-    const int n1 = part ? p.N : p.n1, held = min(m_end - m0, BM);
-    char* base = part ? reinterpret_cast<char*>(p.part + ((size_t)blockIdx.z * p.M + m0) * p.N)
-                      : reinterpret_cast<char*>(p.y) + (size_t)m0 * ld * size;
-    const __amdgpu_buffer_rsrc_t ry = buf_of(base, (uint32_t)held * ld * size);
-    const uint32_t ld2 = n1 < p.N ? (uint32_t)p.ldy2 : 0;
-    const __amdgpu_buffer_rsrc_t ry2 = buf_of(p.y2 + (size_t)m0 * ld2, (uint32_t)held * ld2 * 4);
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const int c0 = n0 + wn + 32 * j, n = c0 + frow;
-      if (!part && p.bias) {
-        const float b = n < p.N ? p.bias[n] : 0.f;
-#pragma unroll
-        for (int i = 0; i < MI; ++i)
-#pragma unroll
-          for (int e = 0; e < 16; ++e) acc[i][j][e] += b;
-      }
-      auto store = [&](uint32_t voff, uint32_t row_bytes, auto put) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < MI; ++i)
-#pragma unroll
-          for (int e = 0; e < 16; ++e) put(acc[i][j][e], voff + (uint32_t)(32 * i + 8 * (e >> 2) + (e & 3)) * row_bytes);
-      };
-      auto put32 = [](const __amdgpu_buffer_rsrc_t& to, float v, uint32_t at) __attribute__((always_inline)) {
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), to, at, 0, 0);
-      };
-      if (c0 + 32 > n1 && n1 < p.N)  // (uniform)
-        store(n >= n1 && n < p.N ? ((uint32_t)(wm + 4 * half) * ld2 + (n - n1)) * 4 : kPastEnd, ld2 * 4,
-              [&](float v, uint32_t at) __attribute__((always_inline)) { put32(ry2, v, at); });
-      if (c0 >= n1) continue;
-      if (!part && p.ep.act) {
-#pragma unroll
-        for (int i = 0; i < MI; ++i)
-#pragma unroll
-          for (int e = 0; e < 16; ++e) acc[i][j][e] = activated(acc[i][j][e], p.ep.act, p.ep.cap);
-      }
-      const uint32_t voff = n < n1 ? ((uint32_t)(wm + 4 * half) * ld + n) * size : kPastEnd;
-      if (f32)
-        store(voff, ld * size, [&](float v, uint32_t at) __attribute__((always_inline)) { put32(ry, v, at); });
-      else
-        store(voff, ld * size, [&](float v, uint32_t at) __attribute__((always_inline)) {
-          __builtin_amdgcn_raw_buffer_store_b16(f2bf(v), ry, at, 0, 0);
-        });
-    }
-    return;
+  store_tile<T, MI, NJ, GROUPED, PAIR>(p, acc, n0, m0, GROUPED ? m_end : min(m_end, m0 + BM), wm, wn, wave & 1, lane, row_pair);
+}
+
+// The same product in bf16 on 256 x 256 tiles, one workgroup of eight waves (2 x 4, each 128 x 64) per CU.  On the 128 x 128 tile
+// a wave reads as many bytes of LDS per product as the CU delivers meanwhile (64 x 64: 16 KB per 16 products of 32
+// cycles on each of four SIMDs), and the vectors pass through registers on their way there; here it is three quarters of that.  K steps of 64
+// bytes per row through four LDS buffers, requested into them directly three steps ahead, each request in a slot of its
+// own behind a product; one barrier per step, which drains nothing.  A step's first operands are read in the step before it, so
+// that no wave stands behind the barrier.  A row's four 16-byte chunks sit at chunk ^ (row / 4 % 4): no bank twice in
+// an operand read.
+// Pair of 6912x2048 under 1004 rows 76 -> 59 us (970 TFLOP/s), 4100 rows 292 -> 229, 32768x2048 under 1004 rows 169 -> 129,
+// 4096x13824 in four ranges 153 -> 117.  What bounds it: a round of 256 tiles takes 41 to 57 us of K = 2048 by how many CUs
+// it fills, where the matrix cores are busy for 28; the first tiles' latency, the stores and the step after the barrier.
+// (256 x 128 tiles, four waves of the same size: 1.2 to 1.3 times the time where both fill the chip, 2 to 8 % less than
+// the 128 x 128 tile where few tiles do: not kept.)
+constexpr int kWideStage = 2 * 256 * 64;
+template <bool PAIR>
+__global__ __launch_bounds__(512) void dense_gemm_wide_kernel(const GemmParams p) {
+  typedef bf16_t T;
+  constexpr int MI = 4, NJ = 2, BN = PAIR ? 128 : 256;
+  constexpr int RQ = 4;  // a wave's requests of a step: 2 x 16 rows of x, 2 x 16 weight rows (PAIR: of one matrix)
+  extern __shared__ __attribute__((aligned(1024))) char lds[];  // [4][x 256 rows | weights 256 rows][64]
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int wm = (wave >> 2) * 128, wcol = wave & 3, wn = wcol * 64;
+  int bx, by;  // (tiles by XCD, as above)
+  {
+    const int total = (int)(gridDim.x * gridDim.y), id = (int)(blockIdx.y * gridDim.x + blockIdx.x);
+    const int q = total >> 3, rem = total & 7, xcd = id & 7, k = id >> 3;
+    const int t = xcd * q + min(xcd, rem) + k;
+    by = t % (int)gridDim.y;
+    bx = t / (int)gridDim.y;
   }
-  // Gated pairs and an expert's rows, in the element type: the same with a row's offset from the list of
-  // pairs (four consecutive tile rows at a time).
-  if (GROUPED || PAIR) {
-    const uint32_t ld = (uint32_t)p.ldy * sizeof(T);
-    char* base = reinterpret_cast<char*>(p.y) + (GROUPED ? 0 : (size_t)m0 * ld);
-    const __amdgpu_buffer_rsrc_t ry = buf_of(base, GROUPED ? kPastEnd : (uint32_t)min(m_end - m0, BM) * ld);
-    constexpr int JS = PAIR ? 2 : 1;  // accumulators per output
-    uint32_t coff[NJ / JS];
+  const int n0 = bx * BN, m0 = by * 256;
+  const uint32_t wrow = (uint32_t)p.ldw * sizeof(T), xrow = (uint32_t)p.ldx * sizeof(T);
+  const int all = (int)(wrow >> 6), k0 = p.ksplit > 1 ? (int)blockIdx.z * p.ksteps * 2 : 0;
+  const int steps = (p.ksplit > 1 ? min(all, k0 + p.ksteps * 2) : all) - k0;
+  auto rsrc = [](const void* base) {
+    const uint64_t a = reinterpret_cast<uint64_t>(base);
+    return u32x4{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a), (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)),
+                 0xFFFFFFFFu, 0x00020000u};
+  };
+  // (rows past the end repeat the last one, their results are not stored)
+  const u32x4 rx = rsrc(reinterpret_cast<const char*>(p.x) + (size_t)m0 * xrow);
+  const u32x4 rw = rsrc(reinterpret_cast<const char*>(PAIR && (wave & 1) ? p.w2 : p.w) + (size_t)n0 * wrow);
+  uint32_t xoff[2], woff[2];
 #pragma unroll
-    for (int j = 0; j < NJ / JS; ++j) {
-      const int n = PAIR ? n0 + (wave & 1) * (16 * NJ) + j * 32 + frow : n0 + wn + 32 * j + frow;
-      coff[j] = n < p.N ? (uint32_t)n * sizeof(T) : kPastEnd;
-    }
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const int t0 = wm + 32 * i + 8 * k + 4 * half;
-        int rows[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) rows[e] = GROUPED ? row_pair[t0 + e] : t0 + e;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const bool in = GROUPED ? t0 + e < m_end : true;  // (not grouped: by the range)
-#pragma unroll
-          for (int j = 0; j < NJ / JS; ++j) {
-            float v = acc[i][JS * j][4 * k + e];
-            if (PAIR) v = gated<T>(v, acc[i][JS * j + JS - 1][4 * k + e], p.glu);
-            const uint32_t off = in && coff[j] != kPastEnd ? (uint32_t)rows[e] * ld + coff[j] : kPastEnd;
-            if (sizeof(T) == 4)
-              __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), ry, off, 0, 0);
-            else
-              __builtin_amdgcn_raw_buffer_store_b16(f2bf(v), ry, off, 0, 0);
-          }
-        }
-      }
-    return;
+  for (int i = 0; i < 2; ++i) {
+    const int tr = (wave * 2 + i) * 16 + (lane >> 2), c = (lane & 3) ^ ((tr >> 2) & 3);
+    const int n = PAIR ? (wave >> 1) * 32 + (tr & 31) : tr;
+    xoff[i] = (uint32_t)min(tr, p.M - 1 - m0) * xrow + c * 16;
+    woff[i] = (uint32_t)min(n, p.N - 1 - n0) * wrow + c * 16;
   }
+  auto request = [&](int which, int s) {  // one of the wave's of step s (past the end: of the last)
+    const uint32_t so = (uint32_t)(k0 + min(s, steps - 1)) * 64;
+    const bool x = which < 2;
+    const int i = which & 1;
+    char* to = lds + (s & 3) * kWideStage + (x ? 0 : 256 * 64) + (wave * 2 + i) * 1024;
+    load_to_lds16_untracked(x ? rx : rw, (lds_char)to, x ? xoff[i] : woff[i], so);
+  };
+  const int frow = lane & 31, half = lane >> 5, swz = (frow >> 2) & 3;
+  const char* const xl = lds + (wm + frow) * 64;
+  const char* const wl = lds + 256 * 64 + (wn + frow) * 64;
+  floatx16 acc[MI][NJ];
 #pragma unroll
   for (int i = 0; i < MI; ++i)
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int tr = wm + 32 * i + 8 * (e >> 2) + 4 * half + (e & 3);
-      if (m0 + tr >= m_end) continue;
-      const size_t row = (size_t)(m0 + tr);
+    for (int j = 0; j < NJ; ++j)
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) {
-        const int n = n0 + wn + 32 * j + frow;
-        if (n >= p.N) continue;
-        const float v = acc[i][j][e] + (p.bias ? p.bias[n] : 0.f);
-        if (n < p.n1)
-          store_out<T>(p.y, row * p.ldy + n, finish<T>(v, row, n, p.ep), p.y_f32);
-        else
-          p.y2[row * p.ldy2 + n - p.n1] = v;
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+  uint4 a[2][MI], b[2][NJ];
+  auto read = [&](int which, int s, int t) {  // one of the six operands of half t of step s
+    const int at = (s & 3) * kWideStage + (((2 * t + half) ^ swz) << 4);
+    if (which < NJ)
+      b[t][which] = *reinterpret_cast<const uint4*>(wl + at + which * 32 * 64);
+    else
+      a[t][which - NJ] = *reinterpret_cast<const uint4*>(xl + at + (which - NJ) * 32 * 64);
+  };
+#pragma unroll
+  for (int s = 0; s < 3; ++s)
+#pragma unroll
+    for (int i = 0; i < RQ; ++i) request(i, s);
+  auto landed = [](bool first) {
+    if (first)
+      __builtin_amdgcn_s_waitcnt(0x0F70 | (2 * RQ));  // vmcnt: step 0 is here
+    else
+      __builtin_amdgcn_s_waitcnt(0x0F70 | RQ);  // vmcnt: the next step's tiles are here too
+    asm volatile("s_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  landed(true);
+#pragma unroll
+  for (int i = 0; i < MI + NJ; ++i) read(i, 0, 0);
+  for (int s = 0; s < steps; ++s) {
+    // every wave has read step s - 1: its buffer takes step s + 3
+    landed(false);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int k = 0; k < MI * NJ; ++k) {
+        const int i = k / NJ, j = k % NJ;
+        acc[i][j] = Elem<T>::mma32(a[t][i], b[t][j], acc[i][j]);
+        // (the other half's operands, first the ones that its first products need)
+        if (k < MI + NJ) read(k, t ? s + 1 : s, t ^ 1);
+        if (k >= MI * NJ - RQ / 2) request(t * (RQ / 2) + k - (MI * NJ - RQ / 2), s + 3);
+        __builtin_amdgcn_sched_barrier(0);
       }
-    }
+  }
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // the repeated requests have landed
+  store_tile<T, MI, NJ, false, PAIR>(p, acc, n0, m0, min(p.M, m0 + 256), wm, wn, wcol, lane, nullptr);
 }
 
-// adds the K ranges in their order
-template <typename T>
+// adds the K ranges in their order.  VEC (columns in fours, no activation or factor): four neighbouring columns per thread
+template <typename T, bool VEC>
 __global__ __launch_bounds__(256) void dense_reduce_kernel(const GemmParams p) {
-  const int n = blockIdx.x * 256 + threadIdx.x, m = blockIdx.y;
+  constexpr int C = VEC ? 4 : 1;
+  const int n = (blockIdx.x * 256 + threadIdx.x) * C, m = blockIdx.y;
   if (n >= p.N) return;
-  float v = p.bias ? p.bias[n] : 0.f;
-  for (int z = 0; z < p.ksplit; ++z) v += p.part[((size_t)z * p.M + m) * p.N + n];
-  if (n < p.n1)
-    store_out<T>(p.y, (size_t)m * p.ldy + n, finish<T>(v, m, n, p.ep), p.y_f32);
+  float v[C];
+#pragma unroll
+  for (int e = 0; e < C; ++e) v[e] = p.bias ? p.bias[n + e] : 0.f;
+  for (int z = 0; z < p.ksplit; ++z) {
+    const float* at = p.part + ((size_t)z * p.M + m) * p.N + n;
+    if constexpr (VEC) {
+      const floatx4 u = *reinterpret_cast<const floatx4*>(at);
+#pragma unroll
+      for (int e = 0; e < C; ++e) v[e] += u[e];
+    } else {
+      v[0] += *at;
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < C; ++e) {
+    if (n + e < p.n1)
+      store_out<T>(p.y, (size_t)m * p.ldy + n + e, VEC ? v[e] : finish<T>(v[e], m, n + e, p.ep), p.y_f32);
+    else
+      p.y2[(size_t)m * p.ldy2 + n + e - p.n1] = v[e];
+  }
+}
+template <typename T>
+void launch_reduce(const GemmParams& p, hipStream_t st) {
+  // (from 2 MB of results on; below, one column per thread is as fast or, 130 rows of 2048, 15.9 us of a product against 18.0, faster)
+  if (p.N % 4 == 0 && !p.ep.act && !p.ep.mul && (int64_t)p.M * p.N >= 1 << 19 && ((uintptr_t)p.part & 15) == 0)
+    dense_reduce_kernel<T, true><<<dim3(exo_ceil_div(p.N, 1024), p.M), 256, 0, st>>>(p);
   else
-    p.y2[(size_t)m * p.ldy2 + n - p.n1] = v;
+    dense_reduce_kernel<T, false><<<dim3(exo_ceil_div(p.N, 256), p.M), 256, 0, st>>>(p);
 }
 
 int raise_lds(const void* fn, int bytes, bool* done) {
@@ -600,6 +741,27 @@ int launch_gemm(const GemmParams& p, int row_tiles, hipStream_t st) {
   return EXO_OK;
 }
 
+template <bool PAIR>
+int launch_wide(const GemmParams& p, hipStream_t st) {
+  static bool done = false;
+  const auto fn = dense_gemm_wide_kernel<PAIR>;
+  const int rc = raise_lds(reinterpret_cast<const void*>(fn), 4 * kWideStage, &done);
+  if (rc) return rc;
+  const dim3 grid(exo_ceil_div(p.N, PAIR ? 128 : 256), exo_ceil_div(p.M, 256), p.ksplit);
+  exo_note_variant("dense_gemm_wide<%s> grid=%dx%dx%d", PAIR ? "pair" : "single", (int)grid.x, (int)grid.y, (int)grid.z);
+  fn<<<grid, 512, 4 * kWideStage, st>>>(p);
+  return EXO_OK;
+}
+
+// Whether 256 x 256 tiles are the faster: rounds of 256 of them, the last one by its share, against rounds of 512 of 128 x 128, in
+// units of such a round (37 us of K = 2048).
+bool wide_is_faster(int64_t wide, int64_t narrow) {
+  const int64_t last = wide % 256;
+  const double tw = 1.5 * (wide / 256) + (last ? 1.15 + 0.35 * last / 256 : 0.0);
+  const double tn = narrow <= 512 ? 1.0 : narrow / 512.0 + 0.4;
+  return tw < tn;
+}
+
 // rows per tile: the tallest that still leaves a workgroup per CU, else the shorter ones
 template <typename T, bool PAIR>
 int launch_plain(GemmParams p, int64_t ws_floats, hipStream_t st) {
@@ -609,6 +771,25 @@ int launch_plain(GemmParams p, int64_t ws_floats, hipStream_t st) {
   p.ksteps = steps;
   const int64_t t2 = (int64_t)cols * exo_ceil_div(p.M, 128), t1 = (int64_t)cols * exo_ceil_div(p.M, 64);
   const bool tall = p.M > 64 && t2 >= 192;
+  if constexpr (sizeof(T) == 2) {
+    const int64_t wide = (int64_t)exo_ceil_div(p.N, PAIR ? 128 : 256) * exo_ceil_div(p.M, 256);
+    if (p.M > 128 && wide_is_faster(wide, t2)) return launch_wide<PAIR>(p, st);
+    // ... or of ranges of K, while they are long against the partial sums' way through memory (columns x K, rows, us before | now:
+    // 4096x13824, 300 88 | 66, 700 150 | 105, 2000 271 | 222; 4096x8192, 1004 93 | 85; 3072x6144, 700 65 | 54; 2048x6912, 1500 77 | 66; but
+    // in ranges of 864, 1004 rows 54 | 58, and 4096x4096, 1004 rows 51 | 59)
+    if (!PAIR && p.part && p.M > 256 && steps >= 96) {
+      int ks = 1;
+      while (wide * ks * 2 <= 256 && steps / (ks * 2) >= 16) ks *= 2;
+      while (ks > 1 && (int64_t)ks * p.M * p.N > ws_floats) ks /= 2;
+      if (ks > 1 && wide * ks > 128) {
+        p.ksteps = exo_ceil_div(steps, ks);
+        p.ksplit = exo_ceil_div(steps, p.ksteps);
+        const int rc = launch_wide<PAIR>(p, st);
+        if (rc == EXO_OK) launch_reduce<T>(p, st);
+        return rc;
+      }
+    }
+  }
   // Few tiles: split K until the chip has about one workgroup per CU, and on long ranges of K two, which wait for
   // different loads: 24 steps where some CUs have none yet, 48 where each has one (2048 columns, bf16, us: 300 rows
   // of K = 6912, 160 -> 320 workgroups 32.9 -> 28.2; 700 rows 176 -> 352 53.6 -> 46.8; 1004 rows 256 -> 512 56.9 -> 51.6, but of
@@ -633,7 +814,7 @@ int launch_plain(GemmParams p, int64_t ws_floats, hipStream_t st) {
     rc = launch_gemm<T, 1, 2, false, PAIR>(p, exo_ceil_div(p.M, 64), st);
   if (rc) return rc;
   if (p.ksplit > 1)
-    dense_reduce_kernel<T><<<dim3(exo_ceil_div(p.N, 256), p.M), 256, 0, st>>>(p);
+    launch_reduce<T>(p, st);
   return EXO_OK;
 }
 

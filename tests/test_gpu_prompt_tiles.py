@@ -4,6 +4,7 @@ weights as the kernel forms them (scale * code + bias, rounded to bf16 once)."""
 from __future__ import annotations
 
 import math
+from types import SimpleNamespace
 
 import pytest
 import torch
@@ -12,7 +13,7 @@ pytestmark = pytest.mark.gpu
 if not torch.cuda.is_available():
     pytest.skip("needs a GPU", allow_module_level=True)
 
-from exo_amd import native, ops  # noqa: E402
+from exo_amd import dense_ops, native, ops  # noqa: E402
 from exo_amd.ops import QuantizedWeight  # noqa: E402
 
 
@@ -289,3 +290,38 @@ def test_products_with_unit_rows_are_the_weights(device, M, N, K, bits):
     x[torch.arange(M, device=device), at] = 1
     # (a sum adds zeros to the weight; +0 where it is -0)
     assert torch.equal(ops.quantized_matmul(x, q).double(), weights64(q).T[at])
+
+
+@pytest.mark.parametrize("M,N,K,kind", [
+    (129, 40004, 64, "plain"), (257, 30004, 192, "tail"), (512, 20000, 128, "act"), (300, 13000, 128, "pair"),
+    (257, 4100, 8192, "split"), (600, 3076, 6144, "split"),
+])
+def test_dense_wide_tiles(device, M, N, K, kind):
+    """The 256 x 256 tile of the float products: one row past a tile, ragged columns, two to six steps of K, ranges of K, and
+    each form of the store."""
+    g = torch.Generator().manual_seed(M + N)
+    x, w = torch.randn(M, K, generator=g).bfloat16(), (torch.randn(N, K, generator=g) * K ** -0.5).bfloat16()
+    bias, up = torch.randn(N, generator=g), (torch.randn(N, K, generator=g) * K ** -0.5).bfloat16()
+    xd, wd, bd, ud = x.to(device), w.to(device), bias.to(device), up.to(device)
+    want = x.float() @ w.float().T
+    out = torch.full((M, N), 7.0, dtype=torch.bfloat16, device=device)
+    if kind == "pair":
+        spec = SimpleNamespace(limit=7.0, alpha=1.702, shift=1.0, cubic=0.0)
+        dense_ops.glu(xd, wd, ud, out, M, spec)
+        u = (x.float() @ up.float().T).clamp(-7, 7)
+        want = want.clamp(max=7) * torch.sigmoid(1.702 * want.clamp(max=7)) * (u + 1)
+    elif kind == "tail":  # the last 100 columns in a float32 buffer
+        t = torch.empty(M, 100, device=device)
+        dense_ops.linear(xd, wd, out, M, bias=bd, tail=(t, 100))
+        want = want + bias
+        torch.testing.assert_close(t.cpu(), want[:, -100:], rtol=1e-5, atol=1e-5)
+        assert (out[:, -100:] == 7).all()
+        out, want = out[:, :-100], want[:, :-100]
+    else:
+        after = dense_ops.After("relu2") if kind == "act" else None
+        dense_ops.linear(xd, wd, out, M, after=after)
+        want = want.clamp(min=0).square() if kind == "act" else want
+    assert native.last_variant().startswith("dense_gemm_wide<" + ("pair" if kind == "pair" else "single")), native.last_variant()
+    assert (kind == "split") != native.last_variant().endswith("x1"), native.last_variant()
+    # one rounding to bf16 of a sum of K products in float32
+    torch.testing.assert_close(out.float().cpu(), want, rtol=2.0 ** -8, atol=2e-5 * K ** 0.5)
