@@ -859,17 +859,38 @@ void launch_gemv_nw(const GemvParams& p, const GemvParams* p1, const PostNorm* q
 // product then holds, and rows of whole parts.  One part -> these, us: N = 2048 (128 workgroups -> 256) under
 // 4 rows, bf16: K = 4096 8.0 -> 6.9, K = 6912 11.8 -> 9.1 (8 rows: 12.8 -> 9.8); N = 1024 (64 -> 256) under
 // 2 rows, f32: K = 1024 6.5 -> 4.2, K = 2560 11.0 -> 5.7.  Four parts at N = 2048 give no more than two (6.8, 9.8).
-// Where the two parts are more than 256 workgroups - a second round of them - only short rows still gain (one part ->
-// two, us: N = 2304 of 2 rows, bf16, K = 1024 1.15 and K = 2048 1.09 times as fast, 2176 0.94, 4096 0.87; f32 1024 1.19,
-// 2048 8.5 -> 9.3, 8 rows 9.0 -> 10.9); a pair reads two matrices per workgroup (N = 2304, bf16 1024 1.07,
-// 2048 0.95; f32 1024 0.95).  16 waves instead of 8: 7.4 and 8.7 in place of 6.9 and 9.1, f32 6.9 in place of 5.7.
+// From 128 tiles of 16 columns on - more than 256 workgroups of two parts - the smaller pieces fill the CUs more evenly, but each
+// reads x and adds its sums again; the times of two parts over those of one, from a sweep of 280 shapes of 1, 4 and 8 rows:
+//   rows of 4 KB: 0.78 to 1.01 below 1024 tiles (13664 columns of K = 2048 bf16 under 4 rows 14.9 -> 13.6 us, 5120 8.7 -> 7.5), and
+//     under two rows beyond (65536 of f32 46.9 -> 43.7; 4 and 8 rows 1.01 to 1.16); pairs from 256 tiles on 0.76 to 0.95
+//     (6912 13.8 -> 13.0), below 1.01 to 1.12
+//   2 KB: 0.83 to 0.99 where one part's last round of 256 is not full (w, what a round has over what is in it, from 1.15 on; full 1.0
+//     to 1.09, beyond 1024 tiles 1.24 and more)
+//   longer: 0.78 to 0.94 where one part leaves half a round (w from 1.5 on; w of 1.15 only under one row 0.93 to 0.99), else to 1.3;
+//     of more than 12 KB 0.78 to 1.01 under up to four rows from 256 tiles on, pairs 0.73 to 0.99
+// 16 waves instead of 8: 7.4 and 8.7 in place of 6.9 and 9.1, f32 6.9 in place of 5.7.
 int gemv_parts(const GemvParams& p, const GemvParams* p1, int elem) {
   const int tiles = exo_ceil_div(p.N, 16) + (p1 ? exo_ceil_div(p1->N, 16) : 0);
   const int rows = p.ldw * elem | (p1 ? p1->ldw * elem : 0);
   if (tiles <= 96 && p.M <= 4 && rows % 256 == 0) return 4;
+  if (p.M > 8 || rows % 128) return 1;
+  if (tiles <= 128) return 2;
   const int longest = std::max(p.ldw, p1 ? p1->ldw : 0) * elem;
-  if (tiles > 128 && longest > (p.w2 ? 2048 : 4096)) return 1;
-  return tiles < (p.w2 ? 160 : 192) && p.M <= 8 && rows % 128 == 0 ? 2 : 1;
+  const double w = exo_ceil_div(tiles, 256) * 256.0 / tiles;
+  bool two;
+  if (tiles < (p.w2 ? 160 : 192))  // (one round's worth of CUs; beyond it rows of less than 1 KB have no step for every wave of a part)
+    two = longest <= (p.w2 ? 2048 : 4096);
+  else if (longest < 1024)
+    two = false;
+  else if (longest <= 2048)
+    two = tiles < 1024 && w >= 1.15 && (!p.w2 || (tiles >= 256 && p.M <= 4));
+  else if (longest <= 4096)
+    two = p.w2 ? tiles >= 256 && tiles < 1024 : tiles < 1024 || p.M <= 2;
+  else if (longest <= 12 * 1024)
+    two = tiles >= 256 && tiles < 1024 && ((w >= 1.5 && p.M <= 4) || (!p.w2 && w >= 1.15 && p.M == 1));
+  else
+    two = tiles >= 256 && tiles < 1024 && (p.w2 || p.M <= 4);
+  return two ? 2 : 1;
 }
 template <typename T, bool PAIR, bool DUAL, int Q>
 void launch_gemv_parts(const GemvParams& p, const GemvParams* p1, hipStream_t st) {

@@ -46,6 +46,34 @@ def test_parts_of_k(device, dtype, M, N, K, parts):
     assert bool((out[M:] == 7).all()) and bool((out[:, N:] == 7).all())
 
 
+# beyond one part's 192 x 16 columns: bytes of a row, and how full one part leaves its last round of 256 workgroups
+@pytest.mark.parametrize("M,N,row,pair,parts", [
+    (4, 3072, 1024, False, 2), (4, 4096, 2048, False, 1), (8, 5003, 2048, False, 2), (3, 16390, 2048, False, 1), (4, 8192, 4096, False, 2),
+    (3, 16400, 3072, False, 1), (2, 16400, 3072, False, 2), (4, 5120, 6144, False, 2), (8, 5120, 6144, False, 1), (1, 6148, 8192, False, 2),
+    (4, 4100, 13824, False, 2), (8, 4100, 13824, False, 1), (4, 3072, 3072, True, 1), (8, 4099, 3072, True, 2), (8, 4100, 13824, True, 2),
+])
+def test_parts_of_k_beyond_one_round(device, M, N, row, pair, parts):
+    K = row // 2
+    g = torch.Generator(device=device).manual_seed(M + N + K)
+    x, w, u = (torch.randn(n, K, device=device, generator=g).bfloat16() for n in (M, N, N if pair else 1))
+    out = torch.zeros(M, N, dtype=torch.bfloat16, device=device)
+    if pair:  # (a gate of 1 and no bend: the product of the two)
+        class Ones:
+            limit, alpha, shift, cubic = float("inf"), 0.0, 0.0, 0.0
+
+        D.glu(x, w, u, out, M, Ones)
+    else:
+        D.linear(x, w, out, M)
+    assert ("parts=%d" % parts in native.last_variant()) if parts > 1 else "parts" not in native.last_variant(), native.last_variant()
+    if not pair:
+        check(out, x, w)
+        return
+    a, c = x.double() @ w.double().T, x.double() @ u.double().T  # sigmoid(0) = 1/2
+    size_a, size_c = x.double().abs() @ w.double().abs().T, x.double().abs() @ u.double().abs().T
+    bound = (K + 1) * 2.0**-24 * (size_a * c.abs() + size_c * a.abs()) * 0.51 + 2.0**-8 * (a * c / 2).abs()
+    assert bool(((out.double() - a * c / 2).abs() <= bound + 1e-12).all())
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("M,N,K", [(1, 70, 128), (4, 1530, 896), (8, 2500, 192), (6, 2545, 320)])
 def test_gated_pair_and_two_products(device, dtype, M, N, K):
