@@ -93,6 +93,27 @@ __device__ __forceinline__ float run_sum(float v) {
   return v;
 }
 
+// sum over the wave, in every lane (all 64 active), without the LDS crossbar: rows of 16 by DPP, the four rows by swaps
+__device__ __forceinline__ float wave_total(float v) {
+  v = run_sum<16>(v);
+  const auto a = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, v), __builtin_bit_cast(uint32_t, v), false, false);
+  const uint32_t a0 = a[0], a1 = a[1];
+  v = __builtin_bit_cast(float, a0) + __builtin_bit_cast(float, a1);
+  const auto b = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, v), __builtin_bit_cast(uint32_t, v), false, false);
+  const uint32_t b0 = b[0], b1 = b[1];
+  return __builtin_bit_cast(float, b0) + __builtin_bit_cast(float, b1);
+}
+// sum of the NW values (a power of two up to 16) that a workgroup's waves have left at `part`, in every lane
+template <int NW>
+__device__ __forceinline__ float total_of(const float* part) {
+  float v = part[threadIdx.x & (NW - 1)];
+  if (NW >= 2) v += dpp_get<0xB1, 0xf>(v);
+  if (NW >= 4) v += dpp_get<0x4E, 0xf>(v);
+  if (NW >= 8) v += dpp_get<0x141, 0xf>(v);
+  if (NW >= 16) v += dpp_get<0x140, 0xf>(v);
+  return v;
+}
+
 // Hand-over of results to another workgroup without a device-wide fence: the producer
 // writes its values with device-scope stores, then every storing wave waits here until all
 // of its outstanding vector-memory operations have completed (on gfx9 stores count in

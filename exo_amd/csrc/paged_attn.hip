@@ -153,7 +153,7 @@ __device__ __forceinline__ void unit_row(const T* __restrict__ src, T* dst, int 
     const float v = Elem<T>::load(src[d]);
     ss += v * v;
   }
-  const float inv = unit ? 1.f / sqrtf(wave_sum(ss) / D + eps) : 1.f;
+  const float inv = unit ? 1.f / sqrtf(wave_total(ss) / D + eps) : 1.f;
   for (int d = lane; d < D; d += 64) dst[d] = Elem<T>::make(Elem<T>::load(src[d]) * inv * (gain ? gain[d] : 1.f));
 }
 

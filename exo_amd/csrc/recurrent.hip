@@ -1050,7 +1050,7 @@ __global__ __launch_bounds__(BLOCK) void gated_norm_kernel(const exo_gated_norm 
       ss += v[i][e] * v[i][e];
     }
   }
-  ss = wave_sum(ss);
+  ss = wave_total(ss);
   if (TEAM > 64) {
     if ((tid & 63) == 0) part[tid >> 6] = ss;
     __syncthreads();

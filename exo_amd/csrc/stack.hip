@@ -10,18 +10,16 @@ namespace {
 
 constexpr int kRowThreads = 256;
 
-// sum over a workgroup of TH threads, in every thread
+// sum over a workgroup of TH threads, in every thread.  tmp: 2 x TH / 64 floats; a call leaves its own half alone until the
+// one after the next, so that one barrier is enough (at most 32 waves' worth of sums through the crossbar, two barriers and
+// sixteen dependent additions before: post_norm_add of 4 rows of 2048 columns 3.5 -> 3.1 us, of two branches 4.9 -> 3.9)
 template <int TH = kRowThreads>
-__device__ __forceinline__ float block_sum(float v, float* tmp) {
-  v = wave_sum(v);
-  const int wave = threadIdx.x >> 6;
-  __syncthreads();  // (tmp may still be read from an earlier call)
-  if ((threadIdx.x & 63) == 0) tmp[wave] = v;
+__device__ __forceinline__ float block_sum(float v, float* tmp, int& phase) {
+  v = wave_total(v);
+  float* const mine = tmp + (phase ^= 1) * (TH / 64);
+  if ((threadIdx.x & 63) == 0) mine[threadIdx.x >> 6] = v;
   __syncthreads();
-  float s = 0.f;
-#pragma unroll
-  for (int w = 0; w < TH / 64; ++w) s += tmp[w];
-  return s;
+  return total_of<TH / 64>(mine);
 }
 
 // ------------------------------------------------------------------------------ embedding
@@ -43,15 +41,16 @@ template <typename T, int TH>
 __global__ __launch_bounds__(TH) void norm_rows_kernel(const float* __restrict__ x, const int32_t* __restrict__ rows,
                                                        const float* __restrict__ gain, T* __restrict__ y, int H, int ldx,
                                                        int ldy, float eps, int center) {
-  __shared__ float tmp[TH / 64];
+  __shared__ float tmp[2 * (TH / 64)];
+  int phase = 0;
   const float* xr = x + (size_t)(rows ? rows[blockIdx.x] : (int)blockIdx.x) * ldx;
   float mean = 0.f, ss = 0.f;
   if (center) {
     for (int c = threadIdx.x; c < H; c += TH) mean += xr[c];
-    mean = block_sum<TH>(mean, tmp) / H;
+    mean = block_sum<TH>(mean, tmp, phase) / H;
   }
   for (int c = threadIdx.x; c < H; c += TH) ss += (xr[c] - mean) * (xr[c] - mean);
-  const float inv = 1.f / sqrtf(block_sum<TH>(ss, tmp) / H + eps);
+  const float inv = 1.f / sqrtf(block_sum<TH>(ss, tmp, phase) / H + eps);
   for (int c = threadIdx.x; c < H; c += TH) y[(size_t)blockIdx.x * ldy + c] = Elem<T>::make((xr[c] - mean) * inv * gain[c]);
 }
 
@@ -90,7 +89,8 @@ __device__ __forceinline__ void load_cols(const T* p, float (&f)[kCols], bool ve
 template <typename T, int TH, int PASSES>
 __global__ __launch_bounds__(TH) void post_norm_add_kernel(const exo_post_norm q, const MoeSum m,
                                                                     float* __restrict__ x, T* __restrict__ xb, int ldx) {
-  __shared__ float tmp[TH / 64];
+  __shared__ float tmp[2 * (TH / 64)];
+  int phase = 0;
   const int row = blockIdx.x, H = q.H;
   float* xr = x + (size_t)row * H;
   const bool vec = H % kCols == 0 && (m.y ? m.ldy % kCols == 0 && m.lds % kCols == 0 : q.ldb % kCols == 0);
@@ -157,7 +157,7 @@ __global__ __launch_bounds__(TH) void post_norm_add_kernel(const exo_post_norm q
 #pragma unroll
       for (int e = 0; e < kCols; ++e) su += e < left ? u[i][e] * u[i][e] : 0.f;
     }
-    const float ia = 0.5f / sqrtf(block_sum<TH>(ss, tmp) / H + q.eps), ib = 0.5f / sqrtf(block_sum<TH>(su, tmp) / H + q.eps);
+    const float ia = 0.5f / sqrtf(block_sum<TH>(ss, tmp, phase) / H + q.eps), ib = 0.5f / sqrtf(block_sum<TH>(su, tmp, phase) / H + q.eps);
     ss = 0.f;
 #pragma unroll
     for (int i = 0; i < PASSES; ++i) {
@@ -184,7 +184,7 @@ __global__ __launch_bounds__(TH) void post_norm_add_kernel(const exo_post_norm q
         s += e < left ? v[i][e] : 0.f;
       }
     }
-    const float mean = q.center ? block_sum<TH>(s, tmp) / H : 0.f;
+    const float mean = q.center ? block_sum<TH>(s, tmp, phase) / H : 0.f;
     ss = 0.f;
 #pragma unroll
     for (int i = 0; i < PASSES; ++i) {
@@ -197,7 +197,7 @@ __global__ __launch_bounds__(TH) void post_norm_add_kernel(const exo_post_norm q
       }
     }
   }
-  const float inv = q.gain ? (q.sum ? 1.f : q.mult) / sqrtf(block_sum<TH>(ss, tmp) / H + q.eps) : q.mult;
+  const float inv = q.gain ? (q.sum ? 1.f : q.mult) / sqrtf(block_sum<TH>(ss, tmp, phase) / H + q.eps) : q.mult;
   ss = 0.f;
 #pragma unroll
   for (int i = 0; i < PASSES; ++i) {
@@ -210,7 +210,7 @@ __global__ __launch_bounds__(TH) void post_norm_add_kernel(const exo_post_norm q
       ss += e < left ? xv[i][e] * xv[i][e] : 0.f;
     }
   }
-  const float pinv = q.pre ? 1.f / sqrtf(block_sum<TH>(ss, tmp) / H + q.eps) : 1.f;
+  const float pinv = q.pre ? 1.f / sqrtf(block_sum<TH>(ss, tmp, phase) / H + q.eps) : 1.f;
 #pragma unroll
   for (int i = 0; i < PASSES; ++i) {
     const int c = (threadIdx.x + i * TH) * kCols, left = H - c;
