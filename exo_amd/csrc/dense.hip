@@ -29,6 +29,7 @@
 #include "dense.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace {
 
@@ -82,31 +83,30 @@ __host__ __device__ inline int post_waves_per_row(int M, int NW) {
   return NW > p ? NW / p : 1;
 }
 
-// sums over the wpr waves that share a row
+// what the wpr waves (a power of two) that share a row have left at `part`, added up
 template <int NW>
-__device__ __forceinline__ void row_sums(float& a, float& b, float (&part)[2][NW], int wave, int wpr, int lane) {
-  a = wave_sum(a);
-  b = wave_sum(b);
-  __syncthreads();  // (earlier sums have been read)
-  if (lane == 0) part[0][wave] = a, part[1][wave] = b;
-  __syncthreads();
-  a = b = 0.f;
-  for (int w = 0; w < wpr; ++w) a += part[0][wave / wpr * wpr + w], b += part[1][wave / wpr * wpr + w];
-}
-
-// four columns from c on, zero past H
-__device__ __forceinline__ floatx4 row4(const float* p, int c, int H, bool on, bool vec) {
-  floatx4 v = {0.f, 0.f, 0.f, 0.f};
-  if (on && c < H) {
-    if (vec) {
-      v = *reinterpret_cast<const floatx4*>(p + c);
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (c + e < H) v[e] = p[c + e];
-    }
-  }
+__device__ __forceinline__ float row_total(const float* part, int wave, int wpr, int lane) {
+  float v = part[(wave & ~(wpr - 1)) + (lane & (wpr - 1))];
+  if (wpr >= 2) v += dpp_get<0xB1, 0xf>(v);
+  if (wpr >= 4) v += dpp_get<0x4E, 0xf>(v);
+  if (wpr >= 8) v += dpp_get<0x141, 0xf>(v);
+  if (wpr >= 16) v += dpp_get<0x140, 0xf>(v);
   return v;
+}
+// a workgroup's LDS writes before it are visible behind it; requests to memory stay in flight
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+  asm volatile("s_barrier" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+// sum over those waves.  part: two buffers in turn, so that one barrier is enough
+template <int NW>
+__device__ __forceinline__ float row_sum(float a, float (&part)[4][NW], int& phase, int wave, int wpr, int lane) {
+  a = wave_total(a);
+  phase ^= 1;
+  if (lane == 0) part[phase][wave] = a;
+  lds_barrier();
+  return row_total<NW>(part[phase], wave, wpr, lane);
 }
 
 // PP: float4 of a row per lane in front of the product (0: nothing there); NORMED: branches that are normed (0: one
@@ -120,7 +120,7 @@ __global__ __launch_bounds__(64 * NW) void dense_gemv_kernel(const GemvParams p0
   constexpr int R = 16 / Q;  // weight rows, and rows of x
   constexpr int BATCH = PAIR ? STEPS / 2 : STEPS;
   __shared__ float red[NM][NW][256];
-  __shared__ float part[2][NW];
+  __shared__ float part[4][NW];  // (the last two: sums of two branches)
   extern __shared__ __attribute__((aligned(16))) char xs[];  // POST: [M][ldx * sizeof(T) + 16]
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int r = lane & 15, g = lane >> 4;
@@ -148,36 +148,101 @@ __global__ __launch_bounds__(64 * NW) void dense_gemv_kernel(const GemvParams p0
     }
   };
   if (POST) {
-    // a row's columns over wpr waves; its inputs are requested ahead of the first weights
+    // A row's columns over wpr waves.  Everything that the sums need is requested ahead of the first weights, without a branch
+    // that the compiler could not count across: a wait for a row's inputs or gains then leaves the weights in flight.  (Behind branches
+    // every wait was for all requests: the norm began when the weights were there, and its gains were two more latencies.  2048 -> 6912
+    // columns bf16 with the norms: 1 row 10.5 -> 9.4 us, 4 rows 18.0 -> 14.4; 1024 -> 4384 float, 2 rows 12.0 -> 10.5.)
     const int wpr = post_waves_per_row(p.M, NW), rpi = NW / wpr;  // rows per iteration
     const uint32_t lrow = xrow + 16;
     const bool vec = q.H % 4 == 0 && q.ldb % 4 == 0;
-    for (int m0 = 0; m0 < p.M; m0 += rpi) {
-      const int m = m0 + wave / wpr, c0 = ((wave % wpr) * 64 + lane) * 4, cs = wpr * 256;
-      const bool on = m < p.M;
-      const size_t o = (size_t)m * q.H, ob = (size_t)m * q.ldb;
-      floatx4 v[NP], x[NP], u[NU];
+    const __amdgpu_buffer_rsrc_t rv = buf_of(q.branch, (uint32_t)p.M * q.ldb * 4), rr = buf_of(q.x ? q.x : q.branch, q.x ? (uint32_t)p.M * q.H * 4 : 0),
+                                 r2 = buf_of(TWO ? q.branch2 : q.branch, (uint32_t)p.M * q.ldb * 4);
+    const uint32_t gbytes = (uint32_t)q.H * 4;
+    const __amdgpu_buffer_rsrc_t ra = buf_of(TWO ? q.gain_a : q.branch, TWO ? gbytes : 0), rb = buf_of(TWO ? q.gain_b : q.branch, TWO ? gbytes : 0),
+                                 rg = buf_of(NORMED ? q.gain : q.branch, NORMED ? gbytes : 0), rp = buf_of(q.pre ? q.pre : q.branch, q.pre ? gbytes : 0);
+    floatx4 v[NP], x[NP], u[NU], ga[NU], gb[NU], gn[NP], gp[NP];
+    int phase = 0;
+    const int cfirst = ((wave % wpr) * 64 + lane) * 4, cs = wpr * 256;
+    // four columns from c on of a row that starts at element `at`: zero past H, past the buffer and where `on` is not set
+    auto four = [&](const __amdgpu_buffer_rsrc_t& r, uint32_t at, int c, bool on, auto whole) __attribute__((always_inline)) {
+      if constexpr (decltype(whole)::value) {
+        return __builtin_bit_cast(floatx4, buf_load16(r, on && c < q.H ? (at + c) * 4 : kPastEnd, 0));
+      } else {
+        floatx4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t w = __builtin_amdgcn_raw_buffer_load_b32(r, on && c + e < q.H ? (at + c + e) * 4 : kPastEnd, 0, 0);
+          o[e] = __builtin_bit_cast(float, w);
+        }
+        return o;
+      }
+    };
+    constexpr bool AHEAD = PP * NU <= 2 && PP <= 2;  // (beyond, the gains do not fit beside the weights: requested where they are used)
+    auto branch_gains = [&](auto whole) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < NU; ++i) ga[i] = four(ra, 0, cfirst + i * cs, true, whole), gb[i] = four(rb, 0, cfirst + i * cs, true, whole);
+    };
+    auto gains = [&](auto whole) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < NP; ++i) gn[i] = four(rg, 0, cfirst + i * cs, true, whole);
+    };
+    auto pre_gains = [&](auto whole) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < NP; ++i) gp[i] = four(rp, 0, cfirst + i * cs, true, whole);
+    };
+    auto all_gains = [&](auto whole) __attribute__((always_inline)) {
+      if (TWO) branch_gains(whole);
+      if (NORMED) gains(whole);
+      pre_gains(whole);
+    };
+    auto here = [&](auto f) __attribute__((always_inline)) {  // not ahead
+      if (AHEAD) return;
+      if (vec)
+        f(std::true_type());
+      else
+        f(std::false_type());
+    };
+    auto inputs = [&](int m0, auto whole) __attribute__((always_inline)) {
+      const int m = m0 + wave / wpr;
 #pragma unroll
       for (int i = 0; i < NP; ++i) {
-        v[i] = row4(q.branch + ob, c0 + i * cs, q.H, on, vec);
-        if (TWO) u[TWO ? i : 0] = row4(q.branch2 + ob, c0 + i * cs, q.H, on, vec);
-        x[i] = row4(q.x + o, c0 + i * cs, q.H, on && q.x, vec);
+        const int c = cfirst + i * cs;
+        v[i] = four(rv, (uint32_t)m * q.ldb, c, m < p.M, whole);
+        if (TWO) u[TWO ? i : 0] = four(r2, (uint32_t)m * q.ldb, c, m < p.M, whole);
+        x[i] = four(rr, (uint32_t)m * q.H, c, m < p.M, whole);
       }
-      if (m0 == 0) load_w(s0);
+    };
+    auto request = [&](int m0) __attribute__((always_inline)) {
+      if (vec) {
+        inputs(m0, std::true_type());
+        if (AHEAD && m0 == 0) all_gains(std::true_type());
+      } else {
+        inputs(m0, std::false_type());
+        if (AHEAD && m0 == 0) all_gains(std::false_type());
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto normed = [&](int m0) __attribute__((always_inline)) {
+      const int m = m0 + wave / wpr;
+      const bool on = m < p.M;
+      const size_t o = (size_t)m * q.H;
       float ss = 0.f, su = 0.f;
       if (TWO) {  // half the sum of the two normed branches
 #pragma unroll
         for (int i = 0; i < NP; ++i)
 #pragma unroll
           for (int e = 0; e < 4; ++e) ss += v[i][e] * v[i][e], su += u[TWO ? i : 0][e] * u[TWO ? i : 0][e];
-        row_sums<NW>(ss, su, part, wave, wpr, lane);
+        ss = wave_total(ss), su = wave_total(su);
+        if (lane == 0) part[2][wave] = ss, part[3][wave] = su;
+        lds_barrier();
+        ss = row_total<NW>(part[2], wave, wpr, lane), su = row_total<NW>(part[3], wave, wpr, lane);
         const float ia = 0.5f / sqrtf(ss / q.H + q.eps), ib = 0.5f / sqrtf(su / q.H + q.eps);
+        here(branch_gains);
 #pragma unroll
-        for (int i = 0; i < NP; ++i) {
-          const floatx4 ga = row4(q.gain_a, c0 + i * cs, q.H, on, vec), gb = row4(q.gain_b, c0 + i * cs, q.H, on, vec);
+        for (int i = 0; i < NP; ++i)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) v[i][e] = v[i][e] * ia * ga[e] + u[TWO ? i : 0][e] * ib * gb[e];
-        }
+          for (int e = 0; e < 4; ++e)
+            v[i][e] = v[i][e] * ia * ga[TWO ? i : 0][e] + u[TWO ? i : 0][e] * ib * gb[TWO ? i : 0][e];
         ss = su = 0.f;
       }
       if (NORMED && q.sum) {  // the sum itself is normed
@@ -190,13 +255,12 @@ __global__ __launch_bounds__(64 * NW) void dense_gemv_kernel(const GemvParams p0
             su += v[i][e];
           }
         if (q.center) {
-          row_sums<NW>(ss, su, part, wave, wpr, lane);
-          const float mean = su / q.H;
+          const float mean = row_sum<NW>(su, part, phase, wave, wpr, lane) / q.H;
 #pragma unroll
           for (int i = 0; i < NP; ++i)
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-              if (c0 + i * cs + e < q.H) v[i][e] -= mean;
+              if (cfirst + i * cs + e < q.H) v[i][e] -= mean;
         }
         ss = su = 0.f;
       }
@@ -206,33 +270,32 @@ __global__ __launch_bounds__(64 * NW) void dense_gemv_kernel(const GemvParams p0
         for (int i = 0; i < NP; ++i)
 #pragma unroll
           for (int e = 0; e < 4; ++e) ss += v[i][e] * v[i][e];
-        row_sums<NW>(ss, su, part, wave, wpr, lane);
+        ss = row_sum<NW>(ss, part, phase, wave, wpr, lane);
         inv = (q.sum ? 1.f : q.mult) / sqrtf(ss / q.H + q.eps);
       }
       ss = 0.f;
+      if (NORMED) here(gains);
 #pragma unroll
-      for (int i = 0; i < NP; ++i) {
-        const floatx4 gn = NORMED ? row4(q.gain, c0 + i * cs, q.H, on, vec) : floatx4{1.f, 1.f, 1.f, 1.f};
+      for (int i = 0; i < NP; ++i)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          x[i][e] += v[i][e] * inv * gn[e];  // zero past H
+          x[i][e] += v[i][e] * inv * (NORMED ? gn[i][e] : 1.f);  // zero past H
           ss += x[i][e] * x[i][e];
         }
-      }
       float pinv = 1.f;
       if (q.pre) {
-        row_sums<NW>(ss, su, part, wave, wpr, lane);
+        ss = row_sum<NW>(ss, part, phase, wave, wpr, lane);
         pinv = 1.f / sqrtf(ss / q.H + q.eps);
+        here(pre_gains);
       }
 #pragma unroll
       for (int i = 0; i < NP; ++i) {
-        const int c = c0 + i * cs;
+        const int c = cfirst + i * cs;
         if (!on || c >= p.ldx) continue;
         floatx4 y = x[i];
         if (q.pre) {
-          const floatx4 gp = row4(q.pre, c, q.H, on, vec);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) y[e] = y[e] * pinv * gp[e];
+          for (int e = 0; e < 4; ++e) y[e] = y[e] * pinv * gp[i][e];
         }
         T out[4];
 #pragma unroll
@@ -247,8 +310,16 @@ __global__ __launch_bounds__(64 * NW) void dense_gemv_kernel(const GemvParams p0
 #pragma unroll
         for (int e = 0; e < 4; ++e) dst[e] = out[e];
       }
+    };
+    request(0);
+    load_w(s0);
+    __builtin_amdgcn_sched_barrier(0);
+    normed(0);
+    for (int m0 = rpi; m0 < p.M; m0 += rpi) {
+      request(m0);
+      normed(m0);
     }
-    __syncthreads();
+    lds_barrier();
   } else {
     load_w(s0);
   }
