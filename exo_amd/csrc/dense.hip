@@ -116,7 +116,6 @@ __global__ __launch_bounds__(64 * NW) void dense_gemv_kernel(const GemvParams p0
   constexpr bool POST = PP > 0, TWO = NORMED == 2;
   constexpr int NP = POST ? PP : 1, NU = TWO ? NP : 1;
   constexpr int NM = PAIR ? 2 : 1;
-  static_assert(Q == 1 || PP == 0, "parts of K side by side: plain products");
   constexpr int R = 16 / Q;  // weight rows, and rows of x
   constexpr int BATCH = PAIR ? STEPS / 2 : STEPS;
   __shared__ float red[NM][NW][256];
@@ -331,7 +330,7 @@ __global__ __launch_bounds__(64 * NW) void dense_gemv_kernel(const GemvParams p0
 #pragma unroll
     for (int i = 0; i < BATCH; ++i) {
       if (POST)  // (steps past the range: any finite values, their weights are zero)
-        xv[i] = *reinterpret_cast<const uint4*>(xs + min(r, p.M - 1) * (xrow + 16) + g * 16 + min(s + i, s1 - 1) * 64);
+        xv[i] = *reinterpret_cast<const uint4*>(xs + min(r % R, p.M - 1) * (xrow + 16) + part_at + g * 16 + min(s + i, s1 - 1) * 64);
       else
         xv[i] = buf_load16(rx, s + i < s1 ? r % R * xrow + part_at + g * 16 + (s + i) * 64 : kPastEnd, 0);
     }
@@ -899,12 +898,13 @@ bool post_fits(int M, int N, int H, int ldx, int elem) {
          (int64_t)M * (ldx * elem + 16) <= 40 * 1024;
 }
 
-template <typename T, int NW, int PP>
+template <typename T, int NW, int PP, int Q = 1>
 void launch_gemv_post(const GemvParams& p, const PostNorm& q, hipStream_t st) {
-  const int tiles = exo_ceil_div(p.N, 16), lds = p.M * (p.ldx * (int)sizeof(T) + 16);
-  const auto fn = q.branch2 ? (p.w2 ? dense_gemv_kernel<T, NW, PP, 2, true, false> : dense_gemv_kernel<T, NW, PP, 2, false, false>)
-                  : q.gain  ? (p.w2 ? dense_gemv_kernel<T, NW, PP, 1, true, false> : dense_gemv_kernel<T, NW, PP, 1, false, false>)
-                            : (p.w2 ? dense_gemv_kernel<T, NW, PP, 0, true, false> : dense_gemv_kernel<T, NW, PP, 0, false, false>);
+  constexpr int one = Q > 1 ? kBatch / 2 : kBatch;  // (post_parts: a wave's share of a part; a pair has half of STEPS of each)
+  const int tiles = exo_ceil_div(p.N, 16 / Q), lds = p.M * (p.ldx * (int)sizeof(T) + 16);
+  const auto fn = q.branch2 ? (p.w2 ? dense_gemv_kernel<T, NW, PP, 2, true, false, Q> : dense_gemv_kernel<T, NW, PP, 2, false, false, Q, one>)
+                  : q.gain  ? (p.w2 ? dense_gemv_kernel<T, NW, PP, 1, true, false, Q> : dense_gemv_kernel<T, NW, PP, 1, false, false, Q, one>)
+                            : (p.w2 ? dense_gemv_kernel<T, NW, PP, 0, true, false, Q> : dense_gemv_kernel<T, NW, PP, 0, false, false, Q, one>);
   fn<<<tiles, 64 * NW, lds, st>>>(p, p, q);
 }
 template <typename T, int NW>
@@ -963,6 +963,19 @@ int gemv_parts(const GemvParams& p, const GemvParams* p1, int elem) {
     two = tiles >= 256 && tiles < 1024 && (p.w2 || p.M <= 4);
   return two ? 2 : 1;
 }
+// The same behind norms, which every workgroup repeats: more workgroups than one round cost more of them.  Rows up to 4 KB whose
+// columns are at most two float4 per lane; the times of two parts over those of one, from a sweep of 672 shapes of 1 to 4 rows:
+//   up to 128 tiles of 16 columns 0.60 to 0.85 (1536 columns of K = 512 bf16 5.8 -> 4.3 us, 2048 of K = 1024 float 8.3 -> 5.6)
+//   below 256: one float4 per lane 0.77 to 0.96 (2 rows of 1024 float, 3072 columns 9.0 -> 8.1), two 0.93 to 1.07, pairs 0.90 to 1.18
+//   beyond, rows of 4 KB behind one branch: 0.87 to 0.95 up to 352 tiles, pairs 0.77 to 1.01; 0.92 to 1.33 with more columns,
+//     1.01 to 1.34 for shorter rows, 0.96 to 1.5 behind two branches
+int post_parts(const GemvParams& p, const PostNorm& q, int elem) {
+  const int tiles = exo_ceil_div(p.N, 16), row = p.ldw * elem, passes = exo_ceil_div(p.ldx, post_waves_per_row(p.M, 8) * 256);
+  if (p.M > 8 || row > 4096 || row % 128 || passes > 2) return 1;
+  if (tiles <= 128) return 2;
+  if (tiles < 256) return !p.w2 && passes == 1 ? 2 : 1;
+  return row > 3072 && !q.branch2 && tiles > 256 && tiles < (p.w2 ? 1024 : 352) ? 2 : 1;
+}
 template <typename T, bool PAIR, bool DUAL, int Q>
 void launch_gemv_parts(const GemvParams& p, const GemvParams* p1, hipStream_t st) {
   const int tiles = exo_ceil_div(p.N, 16 / Q) + (DUAL ? exo_ceil_div(p1->N, 16 / Q) : 0);
@@ -976,6 +989,14 @@ void launch_gemv_parts(const GemvParams& p, const GemvParams* p1, hipStream_t st
 }
 template <typename T>
 int launch_gemv(const GemvParams& p, const GemvParams* p1, const PostNorm* q, hipStream_t st) {
+  if (q && post_parts(p, *q, (int)sizeof(T)) == 2) {
+    exo_note_variant("dense_gemv<%s,8,post,%s> M=%d N=%d parts=2", sizeof(T) == 2 ? "bf16" : "f32", p.w2 ? "pair" : "single", p.M, p.N);
+    if (p.ldx <= post_waves_per_row(p.M, 8) * 256)
+      launch_gemv_post<T, 8, 1, 2>(p, *q, st);
+    else
+      launch_gemv_post<T, 8, 2, 2>(p, *q, st);
+    return EXO_OK;
+  }
   const int parts = q ? 1 : gemv_parts(p, p1, (int)sizeof(T));
   if (parts > 1) {
     exo_note_variant("dense_gemv<%s,8,plain,%s> M=%d N=%d parts=%d", sizeof(T) == 2 ? "bf16" : "f32",

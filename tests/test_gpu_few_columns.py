@@ -74,6 +74,46 @@ def test_parts_of_k_beyond_one_round(device, M, N, row, pair, parts):
     assert bool(((out.double() - a * c / 2).abs() <= bound + 1e-12).all())
 
 
+# behind the norms of the residual: up to 128 x 16 columns always, below 256 x 16 with a float4 of a row per lane, beyond for rows of
+# 4 KB; rows that are not whole vectors, columns that do not fill a workgroup's, steps that do not fill its waves
+@pytest.mark.parametrize("dtype,M,N,H,two,pair,parts", [
+    ("bf16", 1, 41, 70, True, False, 2), ("f32", 8, 2041, 250, False, True, 2), ("bf16", 2, 2048, 2000, True, True, 2), ("bf16", 3, 2048, 2000, True, True, 1), ("f32", 4, 2048, 512, False, False, 2),
+    ("f32", 2, 3001, 1000, True, False, 2), ("f32", 2, 3001, 1000, False, True, 1), ("f32", 4, 3001, 1000, False, False, 1), ("bf16", 5, 2501, 320, False, False, 1),
+    ("bf16", 2, 5001, 2048, False, False, 2), ("bf16", 1, 5001, 2048, True, False, 1), ("bf16", 1, 5700, 2048, False, False, 1), ("f32", 2, 9001, 1021, False, True, 2),
+])
+def test_parts_of_k_behind_norms(device, dtype, M, N, H, two, pair, parts):
+    dtype = torch.bfloat16 if dtype == "bf16" else torch.float32
+    g = torch.Generator(device=device).manual_seed(M * N + H)
+    rand = lambda *n: torch.randn(*n, device=device, generator=g)  # noqa: E731
+    x, ld = rand(M, H), D.pad64(H)
+    w, u = (torch.nn.functional.pad(rand(N, H), (0, ld - H)).to(dtype) for _ in range(2))
+    br = D.Branches(rand(M, H), rand(H), 0.5, *((rand(M, H), rand(H), rand(H)) if two else ()))
+    pre, xo, xb, op = rand(H), torch.zeros(M, H, device=device), torch.zeros(M, ld, dtype=dtype, device=device), torch.zeros(M, ld, dtype=dtype, device=device)
+    out = torch.full((M + 1, N + 3), 7.0, dtype=dtype, device=device)
+
+    class Ones:  # (a gate of 1 and no bend: half the product of the two)
+        limit, alpha, shift, cubic = float("inf"), 0.0, 0.0, 0.0
+
+    D.post_linear(x, br, 1e-5, xo, xb, w, out, M, pre=pre, up=u if pair else None, spec=Ones if pair else None)
+    label = native.last_variant()
+    assert "post" in label and ("parts=2" in label) == (parts == 2), label
+    D.post_norm_add(br, 1e-5, x, op, M, pre)
+    # (sums of H squares in another order, up to three norms: less than 2 H roundings each; one more of the element type)
+    near = 6 * H * 2.0**-24
+    assert bool(((xo - x).abs() <= near * (x.abs() + 4)).all())
+    off, size = (xb.float() - op.float()).abs(), op.float().abs()
+    assert bool((off <= near * float(size.max()) + (2.0**-7 * size if dtype == torch.bfloat16 else 0)).all())
+    assert not bool(xb[:, H:].any()) and bool((out[M:] == 7).all()) and bool((out[:, N:] == 7).all())
+    got, w, u = out[:M, :N], w[:, :H], u[:, :H]
+    if not pair:
+        check(got, xb[:, :H], w)
+        return
+    o = xb[:, :H].double()
+    a, c, size_a, size_c = o @ w.double().T, o @ u.double().T, o.abs() @ w.double().abs().T, o.abs() @ u.double().abs().T
+    bound = (H + 1) * 2.0**-24 * (size_a * c.abs() + size_c * a.abs()) * 0.51 + (2.0**-8 if dtype == torch.bfloat16 else 2.0**-22) * (a * c / 2).abs()
+    assert bool(((got.double() - a * c / 2).abs() <= bound + 1e-12).all())
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("M,N,K", [(1, 70, 128), (4, 1530, 896), (8, 2500, 192), (6, 2545, 320)])
 def test_gated_pair_and_two_products(device, dtype, M, N, K):
