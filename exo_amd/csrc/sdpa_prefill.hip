@@ -144,11 +144,13 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, SPLIT ? 1 : 2) void fa_prefill_k
   const uint32_t koff = (lslot ^ (D == 128 ? lrow & 15 : (lrow >> 1) & 7)) * 16;
   const uint32_t voff = (lslot ^ (D == 128 ? (lrow & 3) << 2 : ((lrow >> 1) & 1) << 2)) * 16;
   // piece i of a wave's share of key tile kt (past the last one: that one again); rows past the end of the cache: its last
-  // row again (they are masked)
+  // row again (they are masked).  Rows are clamped before they are multiplied: a piece may begin past the end, and the bytes of a
+  // whole cache need not fit 31 bits; both offsets of the instruction are unsigned.
   auto load_piece = [&](u32x4 r, uint32_t off, int tile, int kt, int i) {
     const int row0 = (t_first + min(kt, max(n_tiles, 1) - 1)) * kBN;
-    const uint32_t at = min(lrow * ROW, (p.S_max - 1 - row0 - i * (256 / VEC)) * ROW) + off;
-    load_to_lds16_untracked(r, lds + tile * TILE + wave * 1024 + i * 4096, at, row0 * ROW + i * 4096);
+    const int first = min(row0 + i * (256 / VEC), p.S_max - 1);
+    const uint32_t at = (uint32_t)min(lrow, p.S_max - 1 - first) * ROW + off;
+    load_to_lds16_untracked(r, lds + tile * TILE + wave * 1024 + i * 4096, at, (uint32_t)first * ROW);
   };
   auto load_tile = [&](u32x4 r, uint32_t off, int tile, int kt) {
 #pragma unroll

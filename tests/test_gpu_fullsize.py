@@ -21,7 +21,7 @@ from tests.util import (assert_close, assert_close_stat, check_tokens, n_bits, n
 
 pytestmark = pytest.mark.gpu
 
-from exo_amd import ops  # noqa: E402
+from exo_amd import native, ops  # noqa: E402
 from exo_amd.config import named_config  # noqa: E402
 from exo_amd.model import ShardModel  # noqa: E402
 from exo_amd.ops import QuantizedWeight  # noqa: E402
@@ -249,6 +249,39 @@ def test_prefill_attention_two_team_layout(device, D, Hq, Hkv, T, pos, S_max):
     ref = _causal_ref(q, k[0], v[0], pos, T, heads, Hq, Hkv, D)
     got = out.view(T, Hq, D).permute(1, 0, 2)
     assert_close(n_f32(got), n_f32(ref), what=f"two-team prefill sdpa T={T} pos={pos} {Hq}/{Hkv} D={D}")
+
+
+@pytest.mark.parametrize("D,Hq,Hkv,T,end,waves", [
+    (128, 8, 2, 300, 577, 8), (128, 16, 2, 256, 273, 8), (128, 4, 4, 257, 305, 8), (64, 8, 2, 320, 385, 8), (64, 4, 1, 256, 337, 8),
+    (64, 16, 2, 300, 305, 8), (128, 8, 2, 40, 65, 4), (128, 8, 2, 100, 145, 4), (64, 8, 2, 40, 81, 4),
+])
+def test_prefill_attention_at_the_end_of_the_cache(device, D, Hq, Hkv, T, end, waves):
+    """A last key tile of 1, 17 or 49 rows, so that whole requests of it begin past the cache: they take its last row again, and
+    nothing behind the cache (NaN here) is read."""
+    g = torch.Generator(device=device).manual_seed(end + D)
+    q = torch.randn(T, Hq * D, device=device, generator=g).bfloat16()
+    k, v = (torch.full((Hkv * end + 64, D), float("nan"), device=device, dtype=torch.bfloat16) for _ in range(2))
+    k, v = (t[: Hkv * end].copy_(torch.randn(Hkv * end, D, device=device, generator=g)).view(1, Hkv, end, D) for t in (k, v))
+    out, pos = torch.empty_like(q), end - T
+    ops.sdpa_prefill(q, k, v, torch.tensor([pos], dtype=torch.int32, device=device), out, D ** -0.5, 1, T, Hq, Hkv, D)
+    assert native.last_variant().startswith(f"fa_prefill<{D},{'true' if waves == 8 else 'false'}>"), native.last_variant()
+    ref = _causal_ref(q, k[0], v[0], pos, T, list(range(Hq)), Hq, Hkv, D)
+    assert_close(n_f32(out.view(T, Hq, D).permute(1, 0, 2)), n_f32(ref), what=f"prefill sdpa T={T} to the end at {end}, D={D}")
+
+
+@pytest.mark.parametrize("T", [40, 300])  # four waves, eight
+def test_prefill_attention_in_a_cache_of_more_than_2_gib(device, T):
+    """A cache whose bytes per head do not fit 31 bits: its first rows are those that are read."""
+    D, Hq, S_max, pos = 128, 4, 8388608 + 100, 60
+    g = torch.Generator(device=device).manual_seed(T)
+    q = torch.randn(T, Hq * D, device=device, generator=g).bfloat16()
+    k, v = (torch.empty(1, 1, S_max, D, device=device, dtype=torch.bfloat16) for _ in range(2))
+    for t in (k, v):
+        t[:, :, :512] = torch.randn(512, D, device=device, generator=g)
+    out = torch.empty_like(q)
+    ops.sdpa_prefill(q, k, v, torch.tensor([pos], dtype=torch.int32, device=device), out, D ** -0.5, 1, T, Hq, 1, D)
+    ref = _causal_ref(q, k[0, :, :512], v[0, :, :512], pos, T, list(range(Hq)), Hq, 1, D)
+    assert_close(n_f32(out.view(T, Hq, D).permute(1, 0, 2)), n_f32(ref), what=f"prefill sdpa T={T} in a long cache")
 
 
 def _fused_decode_case(device, B, Hq, Hkv, lens, S_max, seed, keys_hint=0):
