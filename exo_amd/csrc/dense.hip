@@ -823,6 +823,13 @@ int launch_wide(const GemmParams& p, hipStream_t st) {
   return EXO_OK;
 }
 
+// 256 rows of each output lie below kPastEnd, where store_tile sends what it drops (the checks of the entry points allow
+// for the 128 rows of the other tiles: strides of float32 from 2097152 on stay with those)
+bool wide_fits(const GemmParams& p) {
+  const int64_t row = (int64_t)p.ldy * (p.y_f32 ? 4 : 2), row2 = p.n1 < p.N ? (int64_t)p.ldy2 * 4 : 0;
+  return 256 * std::max(row, row2) < kPastEnd;
+}
+
 // Whether 256 x 256 tiles are the faster: rounds of 256 of them, the last one by its share, against rounds of 512 of 128 x 128, in
 // units of such a round (37 us of K = 2048).
 bool wide_is_faster(int64_t wide, int64_t narrow) {
@@ -843,7 +850,7 @@ int launch_plain(GemmParams p, int64_t ws_floats, hipStream_t st) {
   const bool tall = p.M > 64 && t2 >= 192;
   if constexpr (sizeof(T) == 2) {
     const int64_t wide = (int64_t)exo_ceil_div(p.N, PAIR ? 128 : 256) * exo_ceil_div(p.M, 256);
-    if (p.M > 128 && wide_is_faster(wide, t2)) return launch_wide<PAIR>(p, st);
+    if (p.M > 128 && wide_fits(p) && wide_is_faster(wide, t2)) return launch_wide<PAIR>(p, st);
     // ... or of ranges of K, while they are long against the partial sums' way through memory (columns x K, rows, us before | now:
     // 4096x13824, 300 88 | 66, 700 150 | 105, 2000 271 | 222; 4096x8192, 1004 93 | 85; 3072x6144, 700 65 | 54; 2048x6912, 1500 77 | 66; but
     // in ranges of 864, 1004 rows 54 | 58, and 4096x4096, 1004 rows 51 | 59)

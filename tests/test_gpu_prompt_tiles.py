@@ -325,3 +325,25 @@ def test_dense_wide_tiles(device, M, N, K, kind):
     assert (kind == "split") != native.last_variant().endswith("x1"), native.last_variant()
     # one rounding to bf16 of a sum of K products in float32
     torch.testing.assert_close(out.float().cpu(), want, rtol=2.0 ** -8, atol=2e-5 * K ** 0.5)
+
+
+@pytest.mark.parametrize("tail", [False, True])
+@pytest.mark.parametrize("ld,wide", [(2097136, True), (2097152, False), (2200000, False)])
+def test_dense_float_outputs_of_long_rows(device, ld, wide, tail):
+    """Rows of a float32 output so far apart that 256 of them reach the offset of dropped stores: the 128-row tile, and nothing
+    beside the ragged columns of either output is written."""
+    M, N, K, T = 257, 30005, 64, 117
+    g = torch.Generator().manual_seed(ld)
+    x, w = torch.randn(M, K, generator=g).bfloat16(), torch.randn(N, K, generator=g).bfloat16()
+    far = torch.full((M, ld), 7.0, device=device)
+    if tail:  # the last columns go to the far buffer
+        near = torch.full((M, N), 7.0, dtype=torch.bfloat16, device=device)
+        dense_ops.linear(x.to(device), w.to(device), near, M, tail=(far, T))
+        assert bool((near[:, N - T :] == 7).all())
+        torch.testing.assert_close(near[:, : N - T].float().cpu(), (x.float() @ w.float().T)[:, : N - T], rtol=2.0**-8, atol=1e-5)
+    else:
+        T = N
+        dense_ops.linear(x.to(device), w.to(device), far[:, :N], M)
+    assert native.last_variant().startswith("dense_gemm_wide<" if wide else "dense_gemm<"), native.last_variant()
+    torch.testing.assert_close(far[:, :T].cpu(), (x.float() @ w.float().T)[:, N - T :], rtol=1e-5, atol=1e-5)
+    assert bool((far[:, T:] == 7).all())
