@@ -1089,6 +1089,24 @@ extern "C" int exo_post_linear_fits(int M, int N, int H, int ldx, int dtype) {
   return M > 0 && N > 0 && H > 0 && post_fits(M, N, H, ldx, dtype == 0 ? 2 : 4);
 }
 
+// row m of the launch alone (of its arguments; the branches' row stride then has no use)
+static exo_linear row_of(exo_linear a, int m) {
+  const size_t elem = a.dtype ? 4 : 2;
+  auto at = [](auto* p, size_t bytes) { return p ? reinterpret_cast<decltype(p)>((uintptr_t)p + bytes) : p; };
+  a.y = at(a.y, (size_t)m * a.ldy * (a.y_f32 ? 4 : elem)), a.y2 = at(a.y2, (size_t)m * a.ldy2 * 4);
+  a.mul = at(a.mul, a.mul_rows ? 0 : (size_t)m * a.ldmul * elem), a.mul_rows = at(a.mul_rows, (size_t)m * 4);
+  a.M = 1;
+  return a;
+}
+static exo_post_norm row_of(exo_post_norm q, const exo_linear& a, int m) {
+  auto at = [](auto* p, size_t bytes) { return p ? reinterpret_cast<decltype(p)>((uintptr_t)p + bytes) : p; };
+  q.x = at(q.x, (size_t)m * q.H * 4), q.x_out = at(q.x_out, (size_t)m * q.H * 4);
+  q.branch = at(q.branch, (size_t)m * q.ldb * 4), q.branch2 = at(q.branch2, (size_t)m * q.ldb * 4);
+  q.operand = at(q.operand, (size_t)m * a.ldx * (a.dtype ? 4 : 2));
+  q.ldb = q.H;
+  return q;
+}
+
 extern "C" int exo_post_linear(const exo_post_norm* q, const exo_linear* a, exo_stream_t stream) {
   int rc = linear_check(a, "exo_post_linear");
   if (rc) return rc;
@@ -1100,6 +1118,15 @@ extern "C" int exo_post_linear(const exo_post_norm* q, const exo_linear* a, exo_
   EXO_REQUIRE(!q->branch2 || (q->gain_a && q->gain_b), "exo_post_linear: two branches need a gain each");
   EXO_REQUIRE(post_fits(a->M, a->N, q->H, a->ldx, a->dtype == 0 ? 2 : 4), "exo_post_linear: %d rows of %d columns do not fit one launch",
               a->M, q->H);
+  // (the kernel's offsets into all rows of a branch have 32 bits and stay below kPastEnd; rows further apart one by one)
+  if ((int64_t)a->M * q->ldb * 4 >= kPastEnd && q->ldb > q->H) {
+    for (int m = 0; m < a->M; ++m) {
+      const exo_linear one = row_of(*a, m);
+      const exo_post_norm norms = row_of(*q, *a, m);
+      if ((rc = exo_post_linear(&norms, &one, stream))) return rc;
+    }
+    return EXO_OK;
+  }
   const GemvParams p = gemv_of(a);
   const PostNorm n{q->x, q->branch, q->branch2, q->gain_a, q->gain_b, q->gain, q->pre, q->x_out, q->operand, q->H, q->ldb,
                    q->sum, q->center, q->eps, q->mult, q->keep};

@@ -2,6 +2,8 @@
 
 from __future__ import annotations
 
+from types import SimpleNamespace
+
 import pytest
 import torch
 
@@ -169,3 +171,36 @@ def test_long_ranges_of_k(device, M, N, K, split):
     D.linear(x, w, out, M)
     assert native.last_variant().endswith("x%d" % split), native.last_variant()
     check(out, x, w)
+
+
+@pytest.mark.parametrize("M,ldb,kind", [(4, 1 << 27, "tail"), (16, 1 << 26, "rows"), (4, 1 << 27, "factor"), (8, 3 << 25, "pair")])
+def test_products_behind_branches_of_far_rows(device, M, ldb, kind):
+    """Rows of a branch whose bytes do not fit 31 or 32 bits together: the same as rows that lie close."""
+    H, N, T, two = 200, 96, 20, kind == "factor"
+    g = torch.Generator(device=device).manual_seed(M)
+    rand = lambda *n: torch.randn(*n, device=device, generator=g)  # noqa: E731
+    x, gains, pre, bias, ld = rand(M, H), [rand(H) for _ in range(3)], rand(H), rand(N), D.pad64(H)
+    w, u = (torch.nn.functional.pad(rand(N, H), (0, ld - H)).bfloat16() for _ in range(2))
+    near = [rand(M, H) for _ in range(1 + two)]
+    far = []
+    for t in near:
+        flat = torch.empty((M - 1) * ldb + H, device=device)
+        far.append(flat.as_strided((M, H), (ldb, 1)).copy_(t))
+    factor, rows = rand(M + 3, N).bfloat16(), torch.arange(M + 2, 2, -1, dtype=torch.int32, device=device)
+    spec = SimpleNamespace(limit=7.0, alpha=1.702, shift=1.0, cubic=0.0)
+
+    def run(b):
+        br = D.Branches(b[0], gains[0], 0.5, *((b[1], gains[1], gains[2]) if two else ()))
+        xo, xb = torch.empty(M, H, device=device), torch.zeros(M, ld, dtype=torch.bfloat16, device=device)
+        out, tail = torch.full((M, N + 8), 7.0, dtype=torch.bfloat16, device=device), torch.full((M, T + 4), 7.0, device=device)
+        kw = dict(tail=dict(bias=bias, tail=(tail, T)), rows=dict(after=D.After("relu2", mul=factor, rows=rows)),
+                  factor=dict(after=D.After(mul=factor)), pair=dict(up=u, spec=spec))[kind]
+        D.post_linear(x, br, 1e-5, xo, xb, w, out, M, pre=pre, **kw)
+        return xo, xb.float(), out.float(), tail
+
+    # the sums of a row over another number of waves: 2 H roundings for each of up to three norms; then, where that
+    # turns a rounding to the operand's type, its last bit in some of the H products of a column
+    (xo, *got), (xo_near, *want) = run(far), run(near)
+    assert bool(((xo - xo_near).abs() <= 6 * H * 2.0**-24 * (xo_near.abs() + 4)).all())
+    for a, b in zip(got, want):
+        torch.testing.assert_close(a, b, rtol=2.0**-7, atol=2.0**-9 * float(b.abs().max()))
