@@ -26,10 +26,14 @@ __device__ __forceinline__ float fma_half(float a, uint32_t v, float c) {
 // Scale and bias of a group, as the codes want them.
 //  4 bits: a code that is masked where it stands, in the low eight bits of a half-word, IS the float16
 // q * 2^-24 (bits 0..3) or q * 2^-20 (bits 4..7), a denormal, so that the mixed-precision FMA takes it without
-// a conversion: fma(s * 2^24, q * 2^-24, b) is fma(s, q, b), bit for bit (|s| < 2^104).  Eight codes to
+// a conversion: fma(s * 2^24, q * 2^-24, b) is fma(s, q, b), bit for bit.  Eight codes to
 // bf16 are 4 masks, a shift, 8 FMAs and 4 packs instead of 3 + 8 conversions + 8 + 4, and vector issue is what the
 // GEMMs' loops have too much of: 4-bit pair of 14336x4096 under 2047 rows 425 -> 414 us, under 100 rows 58 -> 52,
 // 6144x4096 under 300 rows 49.7 -> 45.8.
+//  Scales from 2^104 on have no s * 2^24.  With KEEP such a lane keeps s twice (no other but a zero is its own sixteenth), and
+// where a lane of the wave has one, large_scales() makes those lanes' operands once more; otherwise their operands are not
+// right.  (The branch behind each operand costs the short GEMM nothing, the prompt GEMM 2 to 12 %: that one only notes that there
+// are some, and multiplies the wave's tile once more.)
 template <int BITS>
 struct GroupScale {
   float s, b;
@@ -38,16 +42,24 @@ template <>
 struct GroupScale<4> {
   float s24, s20, b;
 };
-template <int BITS>
+template <int BITS, bool KEEP = false>
 __device__ __forceinline__ GroupScale<BITS> group_scale(float s, float b) {
   GroupScale<BITS> g;
-  if constexpr (BITS == 4)
-    g.s24 = s * 0x1p24f, g.s20 = s * 0x1p20f;
-  else
+  if constexpr (BITS == 4) {
+    const bool keep = KEEP && fabsf(s) >= 0x1p104f;
+    g.s24 = s * (keep ? 1.f : 0x1p24f), g.s20 = s * (keep ? 1.f : 0x1p20f);
+  } else {
     g.s = s;
+  }
   g.b = b;
   return g;
 }
+// the largest magnitude so far: one instruction for two scales
+__device__ __forceinline__ void note_scales(float& most, float s0, float s1) {
+  asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(most) : "v"(s0), "v"(s1));
+}
+// whether a lane's scale, or the largest that it has noted, is one of those
+__device__ __forceinline__ bool any_large(float s) { return __builtin_amdgcn_ballot_w64(fabsf(s) >= 0x1p104f) != 0; }
 
 // One MFMA step's B operand - eight codes as bf16(fma(s, q, b)) - is made in four pieces of one
 // register each, in two parts so that a caller can put products between them: piece_codes() masks or converts the
@@ -83,7 +95,24 @@ __device__ __forceinline__ uint32_t piece_value(int i, const PieceCodes& w, cons
   }
 }
 
-// The whole operand at once
+// The operand of lanes whose scale is large, from its codes (4 bits; 8 have no such scales).  any: some lane has one
+template <int BITS, typename V>
+__device__ __forceinline__ void large_scales(V& operand, uint32_t v0, const GroupScale<BITS>& g, bool any) {
+  if constexpr (BITS == 4) {
+    if (!__builtin_expect(any, 0)) return;
+    u32x4 o = __builtin_bit_cast(u32x4, operand);
+    const uint32_t ev = v0 & 0x0f0f0f0fu, od = (v0 >> 4) & 0x0f0f0f0fu;
+    const u32x4 l = {pack_bf2(fmaf(g.s24, ubyte_f<0>(ev), g.b), fmaf(g.s24, ubyte_f<0>(od), g.b)),
+                     pack_bf2(fmaf(g.s24, ubyte_f<1>(ev), g.b), fmaf(g.s24, ubyte_f<1>(od), g.b)),
+                     pack_bf2(fmaf(g.s24, ubyte_f<2>(ev), g.b), fmaf(g.s24, ubyte_f<2>(od), g.b)),
+                     pack_bf2(fmaf(g.s24, ubyte_f<3>(ev), g.b), fmaf(g.s24, ubyte_f<3>(od), g.b))};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = g.s24 == g.s20 ? l[i] : o[i];
+    operand = __builtin_bit_cast(V, o);
+  }
+}
+
+// The whole operand at once (but for large scales)
 template <int BITS>
 __device__ __forceinline__ bf16x8_t dequant_words8(uint32_t v0, uint32_t v1, const GroupScale<BITS>& g) {
   u32x4 o;

@@ -365,12 +365,15 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
+  float most = 0.f;  // 4 bits: the largest scale so far (from 2^104 on the loops do not make operands right)
+
   // multiply tile `buf` by the weights held (packed) in `st`
   auto multiply = [&](const WStage& st, int buf, const SBlock& sb, int e) {
     GroupScale<BITS> gs[2];  // (rows past N: the last row's; their products are never written)
 #pragma unroll
     for (int j = 0; j < 2; ++j)
       gs[j] = SB4 ? group_scale<BITS>(pick(sb.s[j], e), pick(sb.b[j], e)) : group_scale<BITS>(bf2f(st.w[j].s), bf2f(st.w[j].b));
+    if (BITS == 4) note_scales(most, SB4 ? pick(sb.s[0], e) : bf2f(st.w[0].s), SB4 ? pick(sb.s[1], e) : bf2f(st.w[1].s));
     // MFMA step t covers k = 32*kq + 8*t .. +8 of the K step.  Software pipeline: the A
     // operands and the dequantised B operands of step t+1 are produced while the products
     // of step t run - a 32x32x16 MFMA occupies the matrix core for 8 passes, time for about
@@ -423,6 +426,7 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
   auto scales_of = [&](const SBlock& sb, int e, GroupScale<BITS>(&g)[2]) {
 #pragma unroll
     for (int j = 0; j < 2; ++j) g[j] = group_scale<BITS>(pick(sb.s[j], e), pick(sb.b[j], e));
+    if (BITS == 4) note_scales(most, pick(sb.s[0], e), pick(sb.s[1], e));
   };
   auto read_first = [&](auto ni, const WStage& st, int buf, const SBlock& sb, int e) {
     constexpr int NI = decltype(ni)::value;
@@ -644,6 +648,47 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
     __builtin_amdgcn_s_waitcnt(0x0F70);
     __syncthreads();
     buf ^= 1;
+  }
+
+  // Weights of large scales (dequant.h): the wave's sums once more, in the same order, one step at a time and without LDS
+  if constexpr (BITS == 4) {
+    if (__builtin_expect(any_large(most), 0)) {
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+      for (int k0 = kb; k0 < ke; k0 += BK) {
+        WStage st;
+        GroupScale<BITS> g[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          load_w1(st, k0, j, 0);
+          g[j] = group_scale<BITS, true>(bf2f((bf16_t)__builtin_amdgcn_raw_buffer_load_b16(rs[PAIR ? j : 0], soff[j], (k0 >> 6) * 2, 0)),
+                                         bf2f((bf16_t)__builtin_amdgcn_raw_buffer_load_b16(rb[PAIR ? j : 0], soff[j], (k0 >> 6) * 2, 0)));
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          bf16x8_t w[2];
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            w[j] = dequant8<BITS>(st.w[j], t, g[j]);
+            large_scales<BITS>(w[j], code_word(st.w[j], t, 0), g[j], true);
+          }
+#pragma unroll
+          for (int i = 0; i < MI; ++i) {
+            const int row = min(wm + i * 32 + frow, m_end - 1 - m0);
+            const uint32_t src = GROUPED ? (uint32_t)(row_pair[row] / p.x_div) : (uint32_t)(m0 + row);
+            const bf16x8_t x = __builtin_bit_cast(
+                bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(rx, (src * (uint32_t)p.K + kq * 32 + t * 8) * 2, k0 * 2, 0));
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, w[j], acc[i][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);  // (no registers for this)
+          }
+        }
+      }
+    }
   }
 
   if (KH) {

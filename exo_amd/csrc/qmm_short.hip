@@ -212,11 +212,13 @@ __global__ __launch_bounds__(64 * kWaves) void qmm_short_kernel(const ShortParam
     u32x4 bw[2];
     PieceCodes pc{};
     GroupScale<BITS> gs{};
+    bool large = false;
     auto piece = [&](int q, int d) {  // two of an operand's eight values
       const int j = q >> 1, t = q & 1;
-      if (d == 0 && t == 0) gs = group_scale<BITS>(bf_lo(sc[j]), bf_hi(sc[j]));
+      if (d == 0 && t == 0) gs = group_scale<BITS, true>(bf_lo(sc[j]), bf_hi(sc[j])), large = BITS == 4 && any_large(bf_lo(sc[j]));
       piece_codes<BITS>(pc, d, w[j].q[BITS == 4 ? t : (2 * t) & (WORDS - 1)], w[j].q[BITS == 4 ? t : (2 * t + 1) & (WORDS - 1)]);
       bw[q & 1][piece_reg<BITS>(d)] = piece_value<BITS>(d, pc, gs);
+      if (d == 3) large_scales<BITS>(bw[q & 1], w[j].q[t], gs, large);
     };
 #pragma unroll
     for (int d = 0; d < 4; ++d) piece(0, d);

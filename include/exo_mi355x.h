@@ -109,8 +109,6 @@ int exo_norm_qmv_swiglu_ws(const uint16_t* x, const uint16_t* norm_weight, float
 
 /* K2: the same operator for any M (prefill): weights are dequantised to bf16 in
  * registers and multiplied on the matrix cores, float32 accumulation, bf16 out.
- * 4-bit scales are below 2^104 in magnitude here and in the launches that follow (a weight of
- * more is infinite or NaN).
  * (.typings/mlx/core/__init__.pyi:4198-4234) */
 int exo_qmm(const uint16_t* x, const uint32_t* w, const uint16_t* scales,
             const uint16_t* biases, const uint16_t* residual, uint16_t* y, int M, int N,

@@ -292,6 +292,62 @@ def test_products_with_unit_rows_are_the_weights(device, M, N, K, bits):
     assert torch.equal(ops.quantized_matmul(x, q).double(), weights64(q).T[at])
 
 
+@pytest.mark.parametrize("M,N,K", [(20, 64, 64), (61, 2048, 256), (100, 200, 192), (200, 264, 256), (300, 8192, 768), (1030, 12288, 4096)])
+def test_products_with_unit_rows_under_the_largest_scales(device, M, N, K):
+    """4-bit scales up to the largest bf16 holds, in some groups of some rows: the weights bit for bit, there and beside."""
+    g = torch.Generator(device=device).manual_seed(N + K)
+    q = packed(N, K, 4, M, device)
+    rand = lambda: torch.rand(q.scales.shape, device=device, generator=g)  # noqa: E731
+    e = torch.randint(-12, 2, q.scales.shape, device=device, generator=g)
+    e = torch.where(rand() < 0.1, torch.randint(100, 128, e.shape, device=device, generator=g), e)
+    e[:, 0][rand()[:, 0] < 0.1] = 104  # (the first that cannot be multiplied by 2^24)
+    size = torch.ldexp(1 + 0.9 * rand().double(), e)
+    size[e == 104] = 2.0**104
+    s = torch.where(rand() < 0.5, -size, size).bfloat16()
+    far = e > 123
+    s[-1, -1], far[-1, -1] = 2.0**127 * 1.9921875, True
+    b = torch.where(far, -s.float(), torch.where(far, 0, -s.float()) * 8).bfloat16()
+    # (the farthest: codes 0 and 1, so that every weight is a number: -s and 0)
+    codes = q.weight.view(N, K // 64, 8)
+    w = torch.where(far[..., None], codes & 0x11111111, codes).view(N, K // 8).contiguous()
+    q = QuantizedWeight(w, s, b, 4)
+    at = torch.randint(0, K, (M,), device=device, generator=g)
+    x = torch.zeros(M, K, device=device, dtype=torch.bfloat16)
+    x[torch.arange(M, device=device), at] = 1
+    want = weights64(q).T[at]
+    assert bool(want.isfinite().all())
+    assert torch.equal(ops.quantized_matmul(x, q).double(), want)
+
+
+@pytest.mark.parametrize("M,pair", [(100, True), (600, True), (300, False)])
+def test_large_scales_of_pairs_and_experts(device, M, pair):
+    """The same in the gated pair (large scales in some groups of the up matrix) and in the experts' GEMM, whose rows come by a list."""
+    N, K, E, top = 512, 256, 3, 2
+    g = torch.Generator(device=device).manual_seed(M)
+    at = torch.randint(0, K, (M,), device=device, generator=g)
+    x = torch.zeros(M, K, device=device, dtype=torch.bfloat16)
+    x[torch.arange(M, device=device), at] = 1
+
+    def large(n, seed):
+        q = packed(n, K, 4, seed, device)
+        some = torch.rand(q.scales.shape, device=device, generator=g) < 0.1
+        return QuantizedWeight(q.weight, torch.where(some, q.scales.float() * 2.0**115, q.scales.float()).bfloat16(),
+                               torch.where(some, q.biases.float() * 2.0**115, q.biases.float()).bfloat16(), 4)
+
+    if pair:
+        gate, up = packed(N, K, 4, 1, device), large(N, 2)
+        assert bool((up.scales.float() > 2.0**104).any())
+        got, a, u = ops.qmm_swiglu(x, gate, up), weights64(gate).T[at], weights64(up).T[at]
+        torch.testing.assert_close(got.double(), a * torch.sigmoid(a) * u, rtol=2.0**-7, atol=0)
+        return
+    q = large(E * N, 3)
+    w = weights64(q).view(E, N, K)
+    experts = QuantizedWeight(q.weight.view(E, N, -1), q.scales.view(E, N, -1), q.biases.view(E, N, -1), 4)
+    idx = torch.stack([torch.randperm(E, device=device, generator=g)[:top] for _ in range(M)]).int()
+    got = ops.grouped_qmm(x.view(M, 1, K), experts, ops.moe_group(idx, E), top)
+    assert torch.equal(got.view(M, top, N).double(), w[idx.long(), :, at[:, None]])
+
+
 @pytest.mark.parametrize("M,N,K,kind", [
     (129, 40004, 64, "plain"), (257, 30004, 192, "tail"), (512, 20000, 128, "act"), (300, 13000, 128, "pair"),
     (257, 4100, 8192, "split"), (600, 3076, 6144, "split"),
