@@ -35,6 +35,8 @@
 //   one sequence per workgroup sharing page-sized key tiles through LDS (two buffers, the next tile
 //   in registers meanwhile); 32x32 products, transposed like above so that running maximum, sum and
 //   rescale factor are per-lane scalars.
+#include <type_traits>
+
 #include "../../include/exo_mi355x.h"
 #include "dense.h"
 #include "rotary.h"
@@ -101,14 +103,24 @@ __device__ __forceinline__ Params only(Params p) {
 __device__ __forceinline__ void st_dev(float* p, float v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// two floats in one request
-__device__ __forceinline__ void st_dev(float* p, float a, float b) {
-  __hip_atomic_store(reinterpret_cast<uint64_t*>(p), __builtin_bit_cast(uint64_t, make_float2(a, b)), __ATOMIC_RELAXED,
-                     __HIP_MEMORY_SCOPE_AGENT);
+// two floats, where they lie at a multiple of eight bytes in one request
+template <bool EIGHT>
+__device__ __forceinline__ void st_dev2(float* p, float a, float b) {
+  if (EIGHT) {
+    __hip_atomic_store(reinterpret_cast<uint64_t*>(p), __builtin_bit_cast(uint64_t, make_float2(a, b)), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+  } else {
+    st_dev(p, a);
+    st_dev(p + 1, b);
+  }
 }
+template <bool EIGHT>
 __device__ __forceinline__ float2 ld_dev2(const float* p) {
-  return __builtin_bit_cast(float2, __hip_atomic_load(reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED,
-                                                      __HIP_MEMORY_SCOPE_AGENT));
+  if (EIGHT)
+    return __builtin_bit_cast(float2, __hip_atomic_load(reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED,
+                                                        __HIP_MEMORY_SCOPE_AGENT));
+  return make_float2(__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
+                     __hip_atomic_load(p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
 }
 
 // whole blocks that lie before the window of a query at pos
@@ -845,6 +857,8 @@ __global__ __launch_bounds__(64 * kRowWaves) void paged_rows_kernel(const Params
   const size_t wsrow = (size_t)blockIdx.z * p.H;
   // two neighbouring columns per thread (an odd number of them: the last one beside nothing that is stored)
   const int per = (p.E + 1) / 2, stride_ws = p.E + 2;
+  // every pair of floats of the partials at a multiple of 8 bytes
+  const bool eight = (((uint32_t)(uintptr_t)p.ws >> 2 | (uint32_t)p.E) & 1) == 0;
   auto finished = [&](int h, int d, float a, float b) {
     const float hgate = head_gate(p, row, h0 + h);
     out[(h0 + h) * p.E + d] = Elem<T>::make(a * hgate * column_gate<T>(p, row, (h0 + h) * p.E + d));
@@ -865,11 +879,14 @@ __global__ __launch_bounds__(64 * kRowWaves) void paged_rows_kernel(const Params
       finished(h, d, a0 / lw, a1 / lw);
     } else {
       float* dst = p.ws + ((wsrow + h0 + h) * p.nsplit + split) * stride_ws;
-      if (d + 1 < p.E)
-        st_dev(dst + d, a0, a1);
-      else
+      if (__builtin_expect(eight, 1)) {
+        st_dev2<true>(dst + d, a0, a1);
+        if (d == 0) st_dev2<true>(dst + p.E, mm, lw);
+      } else {
         st_dev(dst + d, a0);
-      if (d == 0) st_dev(dst + p.E, mm, lw);
+        if (d + 1 < p.E) st_dev(dst + d + 1, a1);
+        if (d == 0) st_dev2<false>(dst + p.E, mm, lw);
+      }
     }
   }
   if (used == 1) return;
@@ -889,33 +906,40 @@ __global__ __launch_bounds__(64 * kRowWaves) void paged_rows_kernel(const Params
   // A batch of splits at a time, all its requests ahead of their use, in a running (maximum, sum, weighted sum).  (First every
   // split's factor, then sixteen values of one column at a time whatever the number of splits, the waves one column at a
   // time through conflicting banks: 4 rows of 32 / 4 heads, 700 keys 19.8 us against 16.3.)
-  constexpr int MS = 8;
-  for (int i = threadIdx.x; i < gs * per; i += 64 * kRowWaves) {
-    const int h = i / per, d = (i - h * per) * 2;
-    const float* src = p.ws + (wsrow + h0 + h) * p.nsplit * stride_ws;
-    float a0 = 0.f, a1 = 0.f, lsum = 0.f, mw = -INFINITY;
-    for (int s0 = 0; s0 < used; s0 += MS) {
-      float2 ml[MS], v[MS];
+  auto merge = [&](auto pairs) __attribute__((always_inline)) {
+    constexpr bool EIGHT = decltype(pairs)::value;
+    constexpr int MS = 8;
+    for (int i = threadIdx.x; i < gs * per; i += 64 * kRowWaves) {
+      const int h = i / per, d = (i - h * per) * 2;
+      const float* src = p.ws + (wsrow + h0 + h) * p.nsplit * stride_ws;
+      float a0 = 0.f, a1 = 0.f, lsum = 0.f, mw = -INFINITY;
+      for (int s0 = 0; s0 < used; s0 += MS) {
+        float2 ml[MS], v[MS];
 #pragma unroll
-      for (int s = 0; s < MS; ++s) {
-        const float* at = src + (size_t)min(s0 + s, used - 1) * stride_ws;
-        ml[s] = ld_dev2(at + p.E);
-        v[s] = ld_dev2(at + d);
+        for (int s = 0; s < MS; ++s) {
+          const float* at = src + (size_t)min(s0 + s, used - 1) * stride_ws;
+          ml[s] = ld_dev2<EIGHT>(at + p.E);
+          v[s] = ld_dev2<EIGHT>(at + d);
+        }
+        float mc = mw;
+#pragma unroll
+        for (int s = 0; s < MS; ++s) mc = s0 + s < used ? fmaxf(mc, ml[s].x) : mc;
+        const float back = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw - mc);
+        a0 *= back, a1 *= back, lsum *= back;
+#pragma unroll
+        for (int s = 0; s < MS; ++s) {
+          const float w1 = s0 + s >= used || ml[s].x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml[s].x - mc);
+          a0 += v[s].x * w1, a1 += v[s].y * w1, lsum += ml[s].y * w1;
+        }
+        mw = mc;
       }
-      float mc = mw;
-#pragma unroll
-      for (int s = 0; s < MS; ++s) mc = s0 + s < used ? fmaxf(mc, ml[s].x) : mc;
-      const float back = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw - mc);
-      a0 *= back, a1 *= back, lsum *= back;
-#pragma unroll
-      for (int s = 0; s < MS; ++s) {
-        const float w1 = s0 + s >= used || ml[s].x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml[s].x - mc);
-        a0 += v[s].x * w1, a1 += v[s].y * w1, lsum += ml[s].y * w1;
-      }
-      mw = mc;
+      finished(h, d, a0 / lsum, a1 / lsum);
     }
-    finished(h, d, a0 / lsum, a1 / lsum);
-  }
+  };
+  if (__builtin_expect(eight, 1))
+    merge(std::true_type());
+  else
+    merge(std::false_type());
 }
 
 // ------------------------------------------------------------------------------ prompts

@@ -76,3 +76,34 @@ def test_paged_rows_with_idle_splits(device, dtype, T, last, window, keep):
         out.zero_()
         att.rows(part, out, torch.full((len(last),), 1, **i32), torch.tensor(last, **i32), len(last), keys, append=False)
         close(host(out).reshape(len(last), 8, 64), want[last], 3 * TOL[dtype], f"{keys} keys allowed for")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("vdim,offset", [(63, 0), (1, 0), (64, 4), (33, 4)])
+def test_paged_rows_merge_partials_at_any_float(device, monkeypatch, dtype, vdim, offset):
+    """Several splits whose partials do not lie at multiples of eight bytes: an odd value width, a workspace four bytes further."""
+    from exo_amd import dense_ops as D
+    from exo_amd import native
+    from exo_amd.paged_cache import PagedKVCache
+    from tests import test_gpu_gekazen as G
+    from tests.stack_util import TOL, close, host
+
+    T, last, cols = 700, [699, 300, 0], 10 * 64 + 2 * vdim
+    spec = G.make_spec(8, 2, 64, vdim, None, 0)
+    rows = torch.randn(T, cols, generator=torch.Generator().manual_seed(vdim)).to(device).to(dtype)
+    cache = PagedKVCache([(2, 64, vdim)], 3, 2048, "cuda", dtype)
+    att = D.PagedAttention(spec, torch.tensor(spec.slopes, dtype=torch.float32, device=device), 0, cache, 1e-6)
+    held = rows.float().cpu().numpy()
+    i32 = dict(dtype=torch.int32, device=device)
+    cache.reserve([1], T)
+    att.append(rows, torch.full((T,), 1, **i32), torch.arange(T, **i32), T)
+    q, k, v = held[:, :512].reshape(T, 8, 64), held[:, 512:640].reshape(T, 2, 64), held[:, 640:].reshape(T, 2, vdim)
+    want = G.attn_oracle(spec, (q, k, v), 1e-6, dtype)
+    held_ws = torch.zeros(1 << 22, dtype=torch.uint8, device=device)
+    monkeypatch.setattr(D, "attn_workspace", lambda *a: held_ws[offset:])
+    part, out = rows[last].contiguous(), torch.full((len(last), 8 * vdim + 1), 7.0, dtype=dtype, device=device)
+    for _ in range(2):
+        att.rows(part, out, torch.full((len(last),), 1, **i32), torch.tensor(last, **i32), len(last), T, append=False)
+        assert "splits=1 " not in native.last_variant(), native.last_variant()
+        close(host(out[:, : 8 * vdim]).reshape(len(last), 8, vdim), want[last], 3 * TOL[dtype], f"values of {vdim}")
+        assert bool((out[:, 8 * vdim] == 7).all())
