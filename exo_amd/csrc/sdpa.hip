@@ -136,7 +136,8 @@ constexpr int kMergeRun = G * D > THREADS ? 2 : 1;
 template <int E>
 __device__ __forceinline__ void store_out(bf16_t* to, const Run<E>& acc, float lsum) {
   if constexpr (E == 2) {
-    *reinterpret_cast<uint32_t*>(to) = pack_bf2(acc.v[0] / lsum, acc.v[1] / lsum);
+    typedef uint32_t __attribute__((aligned(2))) two_bf16;  // (one store all the same; outputs may begin at any element)
+    *reinterpret_cast<two_bf16*>(to) = pack_bf2(acc.v[0] / lsum, acc.v[1] / lsum);
   } else {
     *to = f2bf(acc.v[0] / lsum);
   }

@@ -50,6 +50,21 @@ def test_decode_attention_around_the_first_split(device, Hq, Hkv, D, S, lens):
         assert not ws[: 4 * B * Hkv].view(torch.int32)[: B * Hkv].any()
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,D,keys", [(1, 32, 8, 128, 40), (1, 32, 4, 128, 700), (8, 32, 8, 128, 700), (2, 8, 2, 64, 300), (8, 32, 4, 128, 100)])
+def test_decode_attention_into_any_element(device, B, Hq, Hkv, D, keys):
+    """An output that begins at an odd element of its buffer: the bits of one that does not, and nothing beside it."""
+    g = torch.Generator(device=device).manual_seed(keys)
+    kc, vc = (torch.randn(B, Hkv, 1024, D, device=device, generator=g).bfloat16() for _ in range(2))
+    qkv = torch.randn(B, (Hq + 2 * Hkv) * D, device=device, generator=g).bfloat16()
+    pos = torch.full((B,), keys - 1, dtype=torch.int32, device=device)
+    inv = 1e4 ** (-torch.arange(0, D, 2, dtype=torch.float32, device=device) / D)
+    ws, n = ops.sdpa_decode_workspace(B, Hq, D, device), B * Hq * D
+    outs = [torch.full((n + 2,), 7.0, dtype=torch.bfloat16, device=device) for _ in range(2)]
+    for at, out in enumerate(outs):
+        ops.attn_decode(qkv, kc, vc, pos, inv, out[at : at + n], ws, D**-0.5, B, Hq, Hkv, D)
+    assert torch.equal(outs[0][:n], outs[1][1 : n + 1]) and bool((outs[0][n:] == 7).all()) and bool((outs[1][:: n + 1] == 7).all())
+
+
 # the launch is laid out for more keys than the rows hold: splits without a tile of 32 keys (four to a split) leave the
 # merge to the others, down to one that writes the result itself; rows of one launch differ, a second launch
 # finds the counters as the first left them
