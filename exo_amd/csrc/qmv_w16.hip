@@ -53,8 +53,9 @@ struct W16Params {
   int G;          // K / 64
   int blocks;     // N / 16 (pair: N / 8)
   int wave_bytes; // LDS of a wave: lane changes, partial sums
-  int wide_pieces;  // a row's scales are whole pieces of eight groups, else of two
-  int piece_mul;    // 65536 / pieces of a row + 1
+  int wide_pieces;  // a row's scales are whole pieces of eight groups, else a piece may begin in one row and end in the next
+  int piece_mul;    // 65536 / pieces of a row + 1, else 2^20 / pairs of groups of a row + 1
+  int pairs_log2;   // else: pairs of groups of a piece: 1, where there are threads for all of them, or 4
   // K split over `kparts` workgroups per group of row blocks (long rows: the activations of
   // a whole row would not fit the registers): workgroup i takes part i % kparts, Gp groups
   // of every row; float32 partial results meet in `part`, the last workgroup of a group to
@@ -64,7 +65,7 @@ struct W16Params {
   int* counters;  // [block groups], zero between launches
 };
 
-constexpr int kLdsMax = 160 * 1024 - 2048 - 64;  // (beside the sums of squares)
+constexpr int kLdsMax = 160 * 1024 - 2048 - 64, kLdsHalf = 80 * 1024 - 2048 - 64;  // (beside the sums of squares)
 constexpr int kRowPad = 16;                      // bytes between rows of staged scales: 16 rows, 64 banks
 
 // bytes through which a wave's chunks change lanes: all slices at once where the LDS allows it
@@ -135,7 +136,9 @@ __device__ __forceinline__ void lds_barrier() {
 // and with whole-line loads (one piece per thread and array).  Loaded per block by the lanes
 // that need them - 8 bytes each out of 16 different lines per instruction, every line touched again
 // by each of the 16 waves - they cost 4.5 of 24 us of the 14336x4096 pair (measured with the loads
-// taken out).
+// taken out).  Rows that are not whole pieces of eight groups follow one another all the same, so that a piece begins in one row
+// and ends in the next; up to four pieces per thread.  (With pieces of two groups, one per thread, a workgroup held two blocks of K = 2304:
+// 8 rows, 9216 columns 9.0 -> 6.6 us, 256000 119 -> 73, pair of 9216 15.9 -> 9.7.)
 template <bool WIDE, int SL, int DEPTH, bool NORM, bool KSPLIT, bool PAIR>
 __global__ __launch_bounds__(1024) void qmv_w16_kernel(const W16Params p) {
   static_assert(!KSPLIT || (!NORM && !PAIR), "split K: one matrix, activations as they are");
@@ -182,21 +185,30 @@ __global__ __launch_bounds__(1024) void qmv_w16_kernel(const W16Params p) {
     xr[i] = __builtin_bit_cast(
         uint4, __builtin_amdgcn_raw_buffer_load_b128(rx, (i * RPL + xrow) * (p.K * 2) + xchunk * 16, run_ofs, 0));
   if (NORM) gain = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(p.norm_w) + run_ofs + xchunk * 16);
-  const int ppr = p.wide_pieces ? p.Gp >> 3 : p.Gp >> 1;  // pieces of a row
-  const int prow = (tid * p.piece_mul) >> 16, pcol = tid - prow * ppr;
+  const int prow = (tid * p.piece_mul) >> 16, pcol = tid - prow * (p.Gp >> 3);  // (whole pieces)
+  const int of_one = nq * RPB * p.Gp >> 1 >> p.pairs_log2;  // (else: pieces of a matrix, whose rows follow one another - K is not split then)
   u32x4 ps = {}, pb = {};
-  {
+  auto piece_of = [&](int e) {  // (a matrix may begin at any row of a larger one)
+    typedef u32x4 __attribute__((aligned(4))) four;
+    const bool a = PAIR && e >= of_one;
+    const size_t at = (size_t)(q0 * RPB) * p.G + ((a ? e - of_one : e) << p.pairs_log2) * 2;
+    const bf16_t *s = (a ? p.s[1] : p.s[0]) + at, *b = (a ? p.b[1] : p.b[0]) + at;
+    if (p.pairs_log2) {
+      ps = *reinterpret_cast<const four*>(s);
+      pb = *reinterpret_cast<const four*>(b);
+    } else {
+      ps[0] = *reinterpret_cast<const uint32_t*>(s);
+      pb[0] = *reinterpret_cast<const uint32_t*>(b);
+    }
+  };
+  if (p.wide_pieces) {
     const int row = min(prow, nq * 16 - 1), a = PAIR ? (row >> 3) & 1 : 0;
     const int r = PAIR ? (row >> 4) * 8 + (row & 7) : row;
-    const size_t at = (size_t)(q0 * RPB + r) * p.G + g_first;
-    const bf16_t *s = (a ? p.s[1] : p.s[0]) + at, *b = (a ? p.b[1] : p.b[0]) + at;
-    if (p.wide_pieces) {
-      ps = *reinterpret_cast<const u32x4*>(s + pcol * 8);
-      pb = *reinterpret_cast<const u32x4*>(b + pcol * 8);
-    } else {
-      ps[0] = *reinterpret_cast<const uint32_t*>(s + pcol * 2);
-      pb[0] = *reinterpret_cast<const uint32_t*>(b + pcol * 2);
-    }
+    const size_t at = (size_t)(q0 * RPB + r) * p.G + g_first + pcol * 8;
+    ps = *reinterpret_cast<const u32x4*>((a ? p.s[1] : p.s[0]) + at);
+    pb = *reinterpret_cast<const u32x4*>((a ? p.b[1] : p.b[0]) + at);
+  } else {
+    piece_of(min(tid, (PAIR ? 2 : 1) * of_one - 1));
   }
   __builtin_amdgcn_sched_barrier(0);
   struct Block {
@@ -217,11 +229,26 @@ __global__ __launch_bounds__(1024) void qmv_w16_kernel(const W16Params p) {
 
   // ---- activations into operand order
   auto stage_sb = [&]() {
-    if (prow >= nq * 16) return;
-    uint2* to = reinterpret_cast<uint2*>(sb_lds + prow * sb_row + pcol * (p.wide_pieces ? 32 : 8));
+    if (p.wide_pieces) {
+      if (prow >= nq * 16) return;
+      uint2* to = reinterpret_cast<uint2*>(sb_lds + prow * sb_row + pcol * 32);
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
-      if (c == 0 || p.wide_pieces) to[c] = make_uint2((ps[c] & 0xffffu) | pb[c] << 16, ps[c] >> 16 | (pb[c] & 0xffff0000u));
+      for (int c = 0; c < 4; ++c) to[c] = make_uint2((ps[c] & 0xffffu) | pb[c] << 16, ps[c] >> 16 | (pb[c] & 0xffff0000u));
+      return;
+    }
+    const int row_pairs = p.Gp >> 1;
+    for (int e = tid; e < (PAIR ? 2 : 1) * of_one; e += (int)blockDim.x) {
+      const int a = PAIR && e >= of_one;
+      if (e != tid) piece_of(e);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {  // two groups of a row at a time
+        if (c > 0 && p.pairs_log2 == 0) break;
+        const uint32_t at = ((e - a * of_one) << p.pairs_log2) + c, r = at * (uint32_t)p.piece_mul >> 20, col = at - r * row_pairs;
+        const uint32_t row = PAIR ? (r >> 3) * 16 + a * 8 + (r & 7) : r;
+        *reinterpret_cast<uint2*>(sb_lds + row * sb_row + col * 8) =
+            make_uint2((ps[c] & 0xffffu) | pb[c] << 16, ps[c] >> 16 | (pb[c] & 0xffff0000u));
+      }
+    }
   };
   if (NORM) {
     // sums of squares: of a row by runs of 16 lanes, [row][slice of the row]
@@ -440,10 +467,10 @@ int launch_w16s(W16Params p, int nw, hipStream_t st) {
   };
   auto lds_bytes = [&](int nq) { return nw * wave_bytes(nq) + nq * scales; };
   p.wide_pieces = p.Gp % 8 == 0;
-  const int ppr = p.wide_pieces ? p.Gp / 8 : p.Gp / 2;
-  p.piece_mul = 65536 / ppr + 1;
-  // row blocks that a workgroup can hold: partial sums, scales (one piece per thread and array)
-  auto fits = [&](int nq) { return lds_bytes(nq) <= kLdsMax && nq * 16 * ppr <= 64 * nw; };
+  p.piece_mul = p.wide_pieces ? 65536 / (p.Gp / 8) + 1 : (1 << 20) / (p.Gp / 2) + 1;
+  // row blocks that a workgroup can hold: partial sums, scales (pieces per thread and array)
+  const int pieces = p.wide_pieces ? 1 : 4;
+  auto fits = [&](int nq) { return lds_bytes(nq) <= kLdsMax && nq * 2 * p.Gp <= 64 * nw * pieces; };
   if (!fits(1)) {
     exo_set_error("exo_qmv: internal: no LDS for one row block (M=%d K=%d)", p.M, p.K);
     return EXO_ERR_ARG;
@@ -452,10 +479,20 @@ int launch_w16s(W16Params p, int nw, hipStream_t st) {
   // workgroup's share would not fit
   const int round = 256 / p.kparts;
   int groups = round;
-  while (!fits((p.blocks + groups - 1) / groups)) groups += round;
+  auto share = [&]() { return (p.blocks + groups - 1) / groups; };
+  while (!fits(share())) groups += round;
+  // Rows of few waves (rows of broken pieces; whole ones have eight waves or sixteen): two workgroups per CU beside each other where one
+  // round of one has up to six waves, or where there are several rounds of up to nine.  Behind a norm, one per CU -> two, 8 | 16 rows, us:
+  // 262144x1152 41 | 50 -> 35 | 54 (without the norm 39 | 46 -> 33 | 39), 151936x896 31 | 32 -> 21 | 27, 40000x640 8.3 | 10.0 -> 7.5 | 9.0; but
+  // of ten waves and more 128000x1280 22.8 | 30.1 -> 22.4 | 38.2, 151936x1664 36 -> 41.
+  if (!p.wide_pieces && ((nw <= 6 && share() > 4) || (nw <= 9 && SL == 1 && groups > round))) {
+    if (groups == round) groups = 2 * round;
+    while (share() > 8 || lds_bytes(share()) > kLdsHalf) groups += round;
+  }
   if (groups > p.blocks) groups = p.blocks;
   const int nq = (p.blocks + groups - 1) / groups;
   p.wave_bytes = wave_bytes(nq);
+  p.pairs_log2 = nq * 8 * p.Gp <= 64 * nw ? 0 : 2;
   const int grid = groups * p.kparts;
   const size_t bytes = (size_t)lds_bytes(nq);
   if (nq == 1) return launch_instance<WIDE, SL, 1, NORM, KSPLIT, PAIR>(p, grid, nq, nw, bytes, st);
@@ -535,7 +572,7 @@ int exo_qmv_w16_launch(const bf16_t* x, const bf16_t* norm_w, float eps, const u
   p.row_bytes = K / 2;
   p.G = K / 64;
   p.blocks = N / 16;  // (the launcher sets the count for its block size)
-  p.wave_bytes = p.wide_pieces = p.piece_mul = 0;
+  p.wave_bytes = p.wide_pieces = p.piece_mul = p.pairs_log2 = 0;
   const bool pair = w2 != nullptr;
   int sl = 0, nw = 0;
   const int kp = exo_qmv_w16_ok(M, N, K, 4, norm_w != nullptr, pair, workspace != nullptr)

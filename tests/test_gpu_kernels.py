@@ -179,6 +179,43 @@ def test_qmv_16x16x32_shares_of_blocks(device, N, K, blocks, M):
     assert_close(n_f32(got), want, what=f"w16 {M}x{N}x{K}")
 
 
+@pytest.mark.parametrize("M,N,K,pair,blocks", [
+    (8, 9216, 2304, False, 3), (16, 9216, 2304, True, 5), (16, 24592, 896, False, 7), (6, 40976, 2304, False, 11), (8, 36880, 2304, True, 19),
+    (16, 69648, 1152, False, 6), (8, 40016, 640, False, 5), (4, 2064, 1920, False, 1), (9, 5136, 640, True, 3),
+])
+def test_qmv_16x16x32_rows_of_broken_pieces(device, M, N, K, pair, blocks):
+    """K that is no multiple of 512: pieces of eight scales that begin in one row and end in the next, more of them than threads,
+    of a matrix that begins anywhere in another; a workgroup's share is what it is for whole pieces."""
+    g = torch.Generator(device=device).manual_seed(N + M)
+
+    def rows():
+        w = torch.randint(-2**31, 2**31 - 1, (N + 1, K // 8), dtype=torch.int32, device=device, generator=g)
+        s, b = (torch.randn(N + 1, K // 64, device=device, generator=g).bfloat16() * f for f in (0.02, 0.1))
+        return ops.QuantizedWeight(w[1:], s[1:], b[1:], 4)
+
+    def product(q):
+        """In float64, and how far a kernel may be off: sums over a slice's 128 and over the slices of |x| (|128 + code| |s| + |b|) in
+        float32, and the rounding to bf16."""
+        s, b = q.scales.double()[..., None], q.biases.double()[..., None]
+        w = (ops.unpack_codes(q.weight, 4).double().view(N, -1, 64) * s + b).view(N, K)
+        size = (143 * s.abs() + b.abs()).expand(N, K // 64, 64).reshape(N, K)
+        y = x.double() @ w.T
+        return y, 2.0**-8 * y.abs() + (128 + K // 64) * 2.0**-24 * (x.double().abs() @ size.T)
+
+    x = torch.randn(M, K, device=device, generator=g).bfloat16()
+    q = rows()
+    want, slack = product(q)
+    if pair:  # (the gate's unit grows by at most 1.1 of what the gate does)
+        up = rows()
+        got, (u, slack_u) = ops.qmv_swiglu(x, q, up), product(up)
+        unit = want * torch.sigmoid(want)
+        want, slack = unit * u, 1.1 * slack * (u.abs() + slack_u) + unit.abs() * slack_u + 2.0**-8 * (unit * u).abs()
+    else:
+        got = ops.quantized_matmul(x, q)
+    assert native.last_variant().startswith("qmv_w16<") and f" blocks={blocks} " in native.last_variant(), native.last_variant()
+    assert bool(((got.double() - want).abs() <= slack).all()), float(((got.double() - want).abs() - slack).max())
+
+
 @pytest.mark.parametrize("M,N,K,norm,pair,w16", [
     (2, 1024, 768, False, False, True), (2, 1024, 1152, True, False, False), (2, 2048, 2048, True, False, True),
     (2, 2048, 2048, False, False, False), (2, 2048, 2560, True, True, True), (3, 4096, 2048, False, False, True),
