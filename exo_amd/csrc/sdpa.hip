@@ -53,9 +53,9 @@ constexpr int kSoloTiles = D >= 128 ? 16 : G == 1 ? 14 : G == 2 ? 12 : 8;
 // 11.0 | 10.5 | 10.0; 8 of 64 / 4, 1030 keys 15.2 | 13.7 | 13.5.
 template <int G>
 constexpr int kMfmaWaves = G == 4 ? 6 : 8;
-// Contexts left to one workgroup, whose second round of tiles costs less than the hand-over: 8 sequences of 32 / 8 heads,
-// 300 keys 9.9 -> 8.8 us, 500 keys 11.2 -> 13.0.
-constexpr int kSoloMfma = 320;
+// A context is left to one workgroup as long as each wave has one tile: a second round of them costs more than the hand-over to a second
+// workgroup.  Two rounds | two workgroups (keys and values of 24 layers in turn): 8 sequences of 32 / 8 heads, 200 keys 9.5 | 8.8 us, 320
+// 10.5 | 9.7; of 32 / 4, 270 keys 10.8 | 9.6, but 200 keys, one round of its eight waves, 8.7 | 8.9.
 // Tiles of a split before another takes part: 500 keys (16 tiles) with two splits 11.9 us, with four 11.2; 600 keys with three 11.4,
 // with four 11.6.
 constexpr int kMfmaSplitTiles = 5;
@@ -787,9 +787,8 @@ __device__ __forceinline__ uint2 lds_read_tr16(const bf16_t* p) {
 // What bounds it: from thousands of keys the memory (16 sequences of 12290 keys 5.8 TB/s); below, the chain position ->
 // first tile and rope row -> rotation -> products -> merge of the waves (5.4 us with 20 keys) and 3 us of
 // hand-over.  8 sequences of 32 / 8 heads, 2050 keys 20.5 -> 17.9 us (ranges of whole rounds of 128 keys, as they were,
-// gave three of four splits five tiles a wave and the last one), 1030 keys 15.1 -> 13.1, 300 keys 10.5 -> 8.8; 250
-// keys, where two of six waves have a second tile, 8.1 -> 8.4; 4 of 32 / 4 heads, 1030 keys 13.3 -> 10.0; 8 of 64 / 4,
-// 1030 keys 20.9 -> 13.5; one of 64 / 4, 16000 keys 32.3 -> 23.4.
+// gave three of four splits five tiles a wave and the last one), 1030 keys 15.1 -> 13.1, 350 keys 9.5 -> 8.0; 4 of 32 / 4 heads, 1030 keys
+// 13.3 -> 10.0; 8 of 64 / 4, 1030 keys 20.9 -> 13.5; one of 64 / 4, 16000 keys 32.3 -> 23.4.
 template <int G>
 __global__ __launch_bounds__(64 * kMfmaWaves<G>) void sdpa_decode_mfma_kernel(const SdpaParams p) {
   constexpr int NW = kMfmaWaves<G>;
@@ -819,7 +818,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves<G>) void sdpa_decode_mfma_kernel(co
   // Tiles of 32 keys are dealt round robin over the waves of all splits that take part, so that every wave has the
   // same number to within one whatever the length.  A short context is left to one workgroup alone.
   const int cached = len - 1, tiles = (cached + TK - 1) / TK;
-  const int used = len <= kSoloMfma ? 1 : min(p.splits, (tiles + kMfmaSplitTiles - 1) / kMfmaSplitTiles);
+  const int used = tiles <= NW ? 1 : min(p.splits, (tiles + kMfmaSplitTiles - 1) / kMfmaSplitTiles);
   if ((int)blockIdx.x >= used) return;  // (splits without work are gone at once)
   const bool own_new = (int)blockIdx.x == used - 1;
   const int w_begin = (wave * used + (int)blockIdx.x) * TK, w_step = NW * used * TK;

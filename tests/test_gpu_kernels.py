@@ -751,7 +751,7 @@ def test_attn_decode_fused(device, D, Hq, Hkv, qk_norm, lens, table):
 
 
 @pytest.mark.parametrize("Hq,Hkv", [(32, 8), (32, 4), (64, 4)])
-@pytest.mark.parametrize("lens", [[1, 32, 33, 34], [192, 193, 194, 257], [319, 320, 321, 322], [481, 482, 641, 1024]])
+@pytest.mark.parametrize("lens", [[1, 32, 33, 34], [192, 193, 194, 257], [319, 320, 321, 322], [481, 482, 641, 1024], [225, 226, 256, 258]])
 def test_attn_decode_matrix_core_edges(device, Hq, Hkv, lens):
     """The matrix-core decode kernel where a tile, a round of its waves, one workgroup's share or a split ends."""
     test_attn_decode_fused(device, 128, Hq, Hkv, False, lens, True)

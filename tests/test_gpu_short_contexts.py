@@ -18,7 +18,7 @@ def rotated(x, pos, inv):
     return torch.cat([lo * a.cos() - hi * a.sin(), hi * a.cos() + lo * a.sin()], -1).float().bfloat16().double()
 
 
-# one workgroup up to 256 keys of 128, or of 64 up to 448, 384 and 256 with one, two and four heads in it (the matrix-core kernel, 16 and more pairs of 128: 256), several
+# one workgroup up to 256 keys of 128, or of 64 up to 448, 384 and 256 with one, two and four heads in it (the matrix-core kernel, 16 and more pairs of 128: a tile of 32 cached keys for each of its six or eight waves), several
 # beyond; lengths differ inside a batch, and a second call finds the hand-over's counters as the first left them
 @pytest.mark.parametrize("Hq,Hkv,D,S,lens", [
     (32, 8, 128, 4096, [1]), (32, 8, 128, 4096, [256]), (32, 8, 128, 4096, [257]), (32, 8, 64, 600, [512]), (32, 8, 64, 600, [513]),
