@@ -938,14 +938,11 @@ void launch_gemv_nw(const GemvParams& p, const GemvParams* p1, const PostNorm* q
 // 4 rows, bf16: K = 4096 8.0 -> 6.9, K = 6912 11.8 -> 9.1 (8 rows: 12.8 -> 9.8); N = 1024 (64 -> 256) under
 // 2 rows, f32: K = 1024 6.5 -> 4.2, K = 2560 11.0 -> 5.7.  Four parts at N = 2048 give no more than two (6.8, 9.8).
 // From 128 tiles of 16 columns on - more than 256 workgroups of two parts - the smaller pieces fill the CUs more evenly, but each
-// reads x and adds its sums again; the times of two parts over those of one, from a sweep of 280 shapes of 1, 4 and 8 rows:
-//   rows of 4 KB: 0.78 to 1.01 below 1024 tiles (13664 columns of K = 2048 bf16 under 4 rows 14.9 -> 13.6 us, 5120 8.7 -> 7.5), and
-//     under two rows beyond (65536 of f32 46.9 -> 43.7; 4 and 8 rows 1.01 to 1.16); pairs from 256 tiles on 0.76 to 0.95
-//     (6912 13.8 -> 13.0), below 1.01 to 1.12
-//   2 KB: 0.83 to 0.99 where one part's last round of 256 is not full (w, what a round has over what is in it, from 1.15 on; full 1.0
-//     to 1.09, beyond 1024 tiles 1.24 and more)
-//   longer: 0.78 to 0.94 where one part leaves half a round (w from 1.5 on; w of 1.15 only under one row 0.93 to 0.99), else to 1.3;
-//     of more than 12 KB 0.78 to 1.01 under up to four rows from 256 tiles on, pairs 0.73 to 0.99
+// reads x and adds its sums again.  `even`: how much less uneven they are (the work of the fullest CU over the average, of one part
+// over that of two); of 24 widths of 2100 to 40000 columns, ten row lengths, 1 to 8 rows, bf16 and f32 (2656 points) two parts take
+//   0.77 to 0.95 of the time of one where even is 1.33, 0.80 to 1.08 at 1.2 and 1.0 to 1.3 at 1.0, the more the more rows of x there are and
+//   the longer they are (4 | 8 rows of 8 KB 1.0 to 1.2 | 1.0 to 1.24); hence the line, which leaves 0.5 % of the points more than 2 % behind one part
+//   rows of 2 to 4 KB under few rows of x at any width below 16384 columns 0.77 to 1.04, short ones where one part leaves CUs idle 0.86 to 1.02
 // 16 waves instead of 8: 7.4 and 8.7 in place of 6.9 and 9.1, f32 6.9 in place of 5.7.
 int gemv_parts(const GemvParams& p, const GemvParams* p1, int elem) {
   const int tiles = exo_ceil_div(p.N, 16) + (p1 ? exo_ceil_div(p1->N, 16) : 0);
@@ -954,20 +951,27 @@ int gemv_parts(const GemvParams& p, const GemvParams* p1, int elem) {
   if (p.M > 8 || rows % 128) return 1;
   if (tiles <= 128) return 2;
   const int longest = std::max(p.ldw, p1 ? p1->ldw : 0) * elem;
-  const double w = exo_ceil_div(tiles, 256) * 256.0 / tiles;
+  const int halves = exo_ceil_div(p.N, 8) + (p1 ? exo_ceil_div(p1->N, 8) : 0);
+  auto fullest = [](int n) { return exo_ceil_div(n, 256) * 256.0 / n; };  // of 256 CUs, over the average
+  const double one = fullest(tiles), even = one / fullest(halves);
+  const bool pair = p.w2, short_rows = longest <= 2048, up_to_4k = longest <= 4096;
   bool two;
-  if (tiles < (p.w2 ? 160 : 192))  // (one round's worth of CUs; beyond it rows of less than 1 KB have no step for every wave of a part)
-    two = longest <= (p.w2 ? 2048 : 4096);
+  if (tiles < (pair ? 160 : 192))  // (one round's worth of CUs; beyond it rows of less than 1 KB have no step for every wave of a part)
+    two = pair ? short_rows : up_to_4k;
   else if (longest < 1024)
     two = false;
-  else if (longest <= 2048)
-    two = tiles < 1024 && w >= 1.15 && (!p.w2 || (tiles >= 256 && p.M <= 4));
-  else if (longest <= 4096)
-    two = p.w2 ? tiles >= 256 && tiles < 1024 : tiles < 1024 || p.M <= 2;
-  else if (longest <= 12 * 1024)
-    two = tiles >= 256 && tiles < 1024 && ((w >= 1.5 && p.M <= 4) || (!p.w2 && w >= 1.15 && p.M == 1));
+  else if (tiles >= 1024)
+    two = !pair && !short_rows && up_to_4k && p.M <= 2;
+  else if (tiles < 256)
+    two = !pair && up_to_4k;
+  else if (!up_to_4k && !pair && p.M > 4)  // (0.9 to 1.3)
+    two = false;
+  else if (short_rows)
+    two = even >= 1.02 + 0.02 * p.M || (!pair && p.M <= 2 && one >= 1.15);
+  else if (up_to_4k)
+    two = longest <= 3072 ? even >= 1.02 + 0.02 * p.M || p.M <= 2 : even >= 1.1 || p.M <= 4;
   else
-    two = tiles >= 256 && tiles < 1024 && (p.w2 || p.M <= 4);
+    two = even >= 1.05 + (pair ? 0.02 : 0.05) * p.M || (!pair && p.M == 1 && longest <= 8192 && one >= 1.15);
   return two ? 2 : 1;
 }
 // The same behind norms, which every workgroup repeats: more workgroups than one round cost more of them.  Rows up to 4 KB whose

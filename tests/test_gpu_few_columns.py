@@ -53,6 +53,7 @@ def test_parts_of_k(device, dtype, M, N, K, parts):
     (4, 3072, 1024, False, 2), (4, 4096, 2048, False, 1), (8, 5003, 2048, False, 2), (3, 16390, 2048, False, 1), (4, 8192, 4096, False, 2),
     (3, 16400, 3072, False, 1), (2, 16400, 3072, False, 2), (4, 5120, 6144, False, 2), (8, 5120, 6144, False, 1), (1, 6148, 8192, False, 2),
     (4, 4100, 13824, False, 2), (8, 4100, 13824, False, 1), (4, 3072, 3072, True, 1), (8, 4099, 3072, True, 2), (8, 4100, 13824, True, 2),
+    (8, 7000, 2048, False, 1), (4, 12288, 16384, False, 1), (4, 5120, 16384, False, 2), (8, 6912, 4096, True, 1), (8, 4700, 4096, True, 2),
 ])
 def test_parts_of_k_beyond_one_round(device, M, N, row, pair, parts):
     K = row // 2
