@@ -831,9 +831,13 @@ bool wide_fits(const GemmParams& p) {
 }
 
 // Whether 256 x 256 tiles are the faster: rounds of 256 of them, the last one by its share, against rounds of 512 of 128 x 128, in
-// units of such a round (37 us of K = 2048).
-bool wide_is_faster(int64_t wide, int64_t narrow) {
+// units of such a round (37 us of K = 2048).  More than one round only from K = 1024 on, or where the output is more than the last cache
+// takes in: there is one workgroup per CU, whose stores nothing covers (widths of 6912 to 65536 under 130 to 2000 rows, of the time of 128 x
+// 128: one round 0.72 to 0.97 at K = 2048, 0.83 to 1.05 at 64 to 192; several 0.74 to 0.98 at 2048, up to 1.05 at 1024, 1.19 at 768 and 1.44 at
+// 192; of 151936 columns of K = 64 under 520 to 1004 rows 0.74 to 0.85).
+bool wide_is_faster(int64_t wide, int64_t narrow, int steps, int64_t out_bytes) {
   const int64_t last = wide % 256;
+  if (wide > 256 && steps < 16 && out_bytes < 1 << 27) return false;
   const double tw = 1.5 * (wide / 256) + (last ? 1.15 + 0.35 * last / 256 : 0.0);
   const double tn = narrow <= 512 ? 1.0 : narrow / 512.0 + 0.4;
   return tw < tn;
@@ -850,7 +854,7 @@ int launch_plain(GemmParams p, int64_t ws_floats, hipStream_t st) {
   const bool tall = p.M > 64 && t2 >= 192;
   if constexpr (sizeof(T) == 2) {
     const int64_t wide = (int64_t)exo_ceil_div(p.N, PAIR ? 128 : 256) * exo_ceil_div(p.M, 256);
-    if (p.M > 128 && wide_fits(p) && wide_is_faster(wide, t2)) return launch_wide<PAIR>(p, st);
+    if (p.M > 128 && wide_fits(p) && wide_is_faster(wide, t2, steps, (int64_t)p.M * p.N * (p.y_f32 ? 4 : 2))) return launch_wide<PAIR>(p, st);
     // ... or of ranges of K, while they are long against the partial sums' way through memory (columns x K, rows, us before | now:
     // 4096x13824, 300 88 | 66, 700 150 | 105, 2000 271 | 222; 4096x8192, 1004 93 | 85; 3072x6144, 700 65 | 54; 2048x6912, 1500 77 | 66; but
     // in ranges of 864, 1004 rows 54 | 58, and 4096x4096, 1004 rows 51 | 59)

@@ -403,3 +403,20 @@ def test_dense_float_outputs_of_long_rows(device, ld, wide, tail):
     assert native.last_variant().startswith("dense_gemm_wide<" if wide else "dense_gemm<"), native.last_variant()
     torch.testing.assert_close(far[:, :T].cpu(), (x.float() @ w.float().T)[:, N - T :], rtol=1e-5, atol=1e-5)
     assert bool((far[:, T:] == 7).all())
+
+
+@pytest.mark.parametrize("M,N,K,pair,wide", [(520, 40001, 960, False, False), (520, 40001, 1024, False, True), (257, 32001, 64, False, True),
+                                             (520, 30002, 192, True, False), (520, 30002, 1024, True, True)])
+def test_dense_wide_tiles_of_short_k(device, M, N, K, pair, wide):
+    """More 256 x 256 tiles than CUs only over K of 1024 and more."""
+    g = torch.Generator(device=device).manual_seed(K)
+    x, w, u = ((torch.randn(n, K, device=device, generator=g) * f).bfloat16() for n, f in ((M, 1), (N, K**-0.5), (N, K**-0.5)))
+    out, want = torch.empty(M, N, dtype=torch.bfloat16, device=device), x.float() @ w.float().T
+    if pair:
+        dense_ops.glu(x, w, u, out, M, SimpleNamespace(limit=7.0, alpha=1.702, shift=1.0, cubic=0.0))
+        want = want.clamp(max=7) * torch.sigmoid(1.702 * want.clamp(max=7)) * ((x.float() @ u.float().T).clamp(-7, 7) + 1)
+    else:
+        dense_ops.linear(x, w, out, M)
+    assert native.last_variant().startswith("dense_gemm_wide<") == wide, native.last_variant()
+    # one rounding to bf16 of a sum of K products in float32
+    torch.testing.assert_close(out.float(), want, rtol=2.0**-8, atol=2e-5 * K**0.5)
