@@ -1397,24 +1397,26 @@ extern "C" int exo_qmv(const uint16_t* x, const uint32_t* w, const uint16_t* sca
 #define EXO_QMV_W16_MIN_M 5
 #endif
 
-// Two to four rows that take it too, from a sweep of N = 1024 to 151936 and K = 768 to 4096 (its time over the 4x4x4 kernel's, or
+// Two to four rows that take it too, from sweeps of N = 1024 to 151936 and K = 768 to 4096 (its time over the 4x4x4 kernel's, or
 // where rows are not whole 256-byte slices over that of the kernels below).  K of up to 1024: 0.3 to 0.99 (151936x1024 39 ->
-// 21 us).  Four rows 0.72 to 1.01 from N = 2048 on (4096x4096 7.0 -> 5.8 us, 128256x4096 66 -> 58), 0.97 to 1.18 below.  Three
-// rows behind a norm 0.71 to 1.02 and pairs to 1.03 (14336x4096 18.5 -> 15.3); without a norm 0.85 to 1.0 from N = 4096
-// on, 1.0 to 1.27 below and 1.02 to 1.04 where N and K are both long.  Heads of K = 1536 and 2048 lose up to 8 % under
-// three and four rows (several rounds of workgroups).  Two rows behind a norm 0.79 to 1.0 up to N = 4096 or K = 1536
-// (others to 1.13, without a norm to 1.35), pairs 0.83 to 0.99 from K = 2560 on (wider than 16384 and shorter ones to 1.13).
-// Split K loses (a hand-over: 2048x8192 5.9 | 8.0 us).  Longer pairs of four rows stay with the other, whose instance the
-// tests of the decode step name, although it is behind: 14336x4096 19.4 | 15.6.
+// 21 us).  Behind a norm four rows 0.72 to 1.01 from N = 2048 on (128256x4096 66 -> 58), three 0.71 to 1.02, two 0.79 to 1.0 up to N = 4096 or
+// K = 1536 (others to 1.13).  Without a norm four and three rows 0.84 to 1.02 where the row blocks are dealt evenly, at most a third
+// over the average on the fullest CU, and 1.02 to 1.09 where they are not (4112x3584 under four 6.2 | 6.7); fewer blocks than CUs 0.9 to 0.95
+// under four and 1.0 to 1.27 under three; three rows of more than 3072 gain with one block per CU alone (0.93 to 0.97, else 1.02 to 1.04).
+// Heads of K = 1536 and 2048 lose up to 8 % under three and four rows (several rounds of workgroups).  Two rows without a norm
+// to 1.35.  Pairs of three rows 0.71 to 0.95 up to N = 16384 or K = 2048 (else to 1.1), of two 0.83 to 0.99 from K = 2560 on
+// (wider than 16384 and shorter ones to 1.13).  Split K loses (a hand-over: 2048x8192 5.9 | 8.0 us).  Longer pairs of four rows stay with the
+// other, whose instance the tests of the decode step name, although it is behind: 14336x4096 19.4 | 15.6.
 static bool few_rows_on_w16(int M, int N, int K, bool norm, bool pair) {
   if (N < 1024 || K < 768 || K > 4096) return false;
   if (K <= 1024) return true;
   if (N < 2048) return false;
-  if (pair) return M == 3 || (M == 2 && K >= 2560 && N <= 16384);
+  if (pair) return N <= 16384 ? M == 3 || (M == 2 && K >= 2560) : M == 3 && K <= 2048;
   if (M >= 3 && K <= 2048 && N > 65536) return false;
-  if (M == 4) return true;
-  if (norm) return M == 3 || N <= 4096 || K <= 1536;
-  return M == 3 && (N == 4096 || (N > 4096 && K <= 3072));
+  if (norm) return M >= 3 || N <= 4096 || K <= 1536;
+  const int share = exo_ceil_div(N, 16 * 256);  // row blocks of the fullest workgroup
+  if (M == 2 || (share > 1 && 3 * share * 4096 > 4 * N)) return false;
+  return M == 4 || (N >= 4096 && (K <= 3072 || share == 1));
 }
 
 static int norm_qmv_impl(const uint16_t* x, const uint16_t* norm_weight, float eps,

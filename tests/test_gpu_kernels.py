@@ -220,7 +220,8 @@ def test_qmv_16x16x32_rows_of_broken_pieces(device, M, N, K, pair, blocks):
     (2, 1024, 768, False, False, True), (2, 1024, 1152, True, False, False), (2, 2048, 2048, True, False, True),
     (2, 2048, 2048, False, False, False), (2, 2048, 2560, True, True, True), (3, 4096, 2048, False, False, True),
     (3, 2064, 1536, True, True, True), (4, 2048, 4096, False, False, True), (4, 2048, 8192, False, False, False),
-    (4, 1040, 1024, True, True, True), (4, 2048, 2048, True, True, False),
+    (4, 1040, 1024, True, True, True), (4, 2048, 2048, True, True, False), (3, 4096, 4096, False, False, True), (3, 4112, 4096, False, False, False),
+    (4, 4112, 2048, False, False, False), (4, 6144, 2048, False, False, True), (3, 16400, 2560, True, True, False),
 ])
 def test_qmv_few_rows_routes(device, M, N, K, norm, pair, w16):
     """2..4 rows on both sides of the line between the 16x16x32 and the 4x4x4 kernel."""
