@@ -543,8 +543,8 @@ __global__ __launch_bounds__(kThreads) void qmv_rows_kernel(const QmvParams p) {
   // Base pointers of this workgroup's matrices.  Gather modes: the expert of its pair.
   // Routing mode: every wave repeats the routing of the token from logits that it requested first
   // (route_raw), as far as its own slot; called once the activation loads are on their way, so
-  // that their latency covers it.  (All selections in every wave: 32 pairs of 768x2048 16.6 us against 16.0, 8 pairs
-  // 8.25 | 8.08.  In wave 0 with the others at a barrier, 8 pairs of 8-bit 1536x4096 25.7 | 24.0.)
+  // that their latency covers it.  (All selections in every wave, other tokens in each launch: 32 pairs of 768x2048 15.3 us against
+  // 15.0, 8 pairs level.  In wave 0 with the others at a barrier, 8 pairs of 8-bit 1536x4096 24.7 | 23.6, 64 139.3 | 138.5.)
   constexpr bool XR = kRowsXR<MT, ITERS, NMAT, ROUTE>;
   uint32_t route_raw[4] = {0, 0, 0, 0};
   auto select_matrices = [&]() {
