@@ -565,7 +565,10 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
     SBlock sbc, sbn;
     const int last = ke - BK;
     load_sb(sbn, kb >> 8);
-    constexpr int XAHEAD = 3;
+    // Two teams of 8-bit codes: activations two steps ahead and in front of the weights (three, and behind them: 4096x14336
+    // under 520 rows 115.7 | 121.5 us, 1500 205 | 211, 6144x4096 under 1023 60.9 | 61.5)
+    constexpr bool X_FIRST = KH && BITS == 8;
+    constexpr int XAHEAD = X_FIRST ? 2 : 3;
 #pragma unroll
     for (int u = 0; u < AHEAD; ++u) load_w(wq[u], min(kb + u * BK, last));
 #pragma unroll
@@ -582,18 +585,19 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
         multiply_on(ni, wq[u], wq[(u + 1) & 3], u, (u + 1) & 3, u < 3 ? sbc : sbn, (u + 1) & 3, [&](int slot) {
           // (a whole step's requests at once are more than the address unit takes in: the wave stands until
           // they have left, and its matrix core with it)
+          constexpr int W0 = X_FIRST ? NI : 0, X0 = X_FIRST ? 0 : NW;
 #pragma unroll
           for (int r = 0; r < NW; ++r)
-            if (slot == (!GROUPED ? r * (8 * NI) / (NW + NI) : BITS == 4 ? r * (4 * NI) / NW : 0)) load_w1(wq[(u + AHEAD) & 3], kw, r / (NW / 2), r % (NW / 2));
+            if (slot == (!GROUPED ? (W0 + r) * (8 * NI) / (NW + NI) : BITS == 4 ? r * (4 * NI) / NW : 0)) load_w1(wq[(u + AHEAD) & 3], kw, r / (NW / 2), r % (NW / 2));
 #pragma unroll
           for (int r = 0; r < NI; ++r)  // (grouped: behind the last wait for weights, which does not count these)
-            if (slot == (GROUPED ? 7 * NI + r : (NW + r) * (8 * NI) / (NW + NI))) load_x1((u + XAHEAD) & 3, kx, r);
+            if (slot == (GROUPED ? 7 * NI + r : (X0 + r) * (8 * NI) / (NW + NI))) load_x1((u + XAHEAD) & 3, kx, r);
         });
         // Tile k+2 is in LDS behind the barrier: the next step's last products read its first operands.  What was
-        // requested in this step may still be out - but the fence of __syncthreads() would wait for every
+        // requested in this step (behind that tile) may still be out - but the fence of __syncthreads() would wait for every
         // request into LDS, so that the barrier stands alone.  (Reads of tile k, whose memory the next
         // step's requests fill, have been multiplied.)
-        wait_vm(std::integral_constant<int, NI + NW>{});
+        wait_vm(std::integral_constant<int, X_FIRST ? NW : NI + NW>{});
         asm volatile("s_barrier" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
       }
