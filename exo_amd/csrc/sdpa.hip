@@ -152,18 +152,19 @@ __device__ __forceinline__ void merge_batches(const float* src, int splits, int 
   float mw = -INFINITY, lsum = 0.f;
   Run<E> acc = {};
   for (int s0 = 0; s0 < splits; s0 += MS) {
-    Run<2> ml[MS];
+    float pm[MS], pl[MS];  // (two requests: all lanes of a head ask for the same eight bytes, and one of eight takes longer)
     Run<E> po[MS];
 #pragma unroll
     for (int sp = 0; sp < MS; ++sp) {
       const int spc = min(s0 + sp, splits - 1);
-      ml[sp] = ld_dev<2>(src + (size_t)spc * (D + 2) + D);
+      pm[sp] = ld_dev<1>(src + (size_t)spc * (D + 2) + D).v[0];
+      pl[sp] = ld_dev<1>(src + (size_t)spc * (D + 2) + D + 1).v[0];
       po[sp] = ld_dev<E>(src + (size_t)spc * (D + 2) + e);
     }
     float mc = mw;
 #pragma unroll
     for (int sp = 0; sp < MS; ++sp)
-      if (s0 + sp < splits) mc = fmaxf(mc, ml[sp].v[0]);
+      if (s0 + sp < splits) mc = fmaxf(mc, pm[sp]);
     if (s0 > 0) {  // earlier batches move to the new maximum
       const float r = (mw == -INFINITY) ? 0.f : __expf(mw - mc);
 #pragma unroll
@@ -172,10 +173,10 @@ __device__ __forceinline__ void merge_batches(const float* src, int splits, int 
     }
 #pragma unroll
     for (int sp = 0; sp < MS; ++sp) {
-      const float sc = (s0 + sp >= splits || ml[sp].v[0] == -INFINITY) ? 0.f : __expf(ml[sp].v[0] - mc);
+      const float sc = (s0 + sp >= splits || pm[sp] == -INFINITY) ? 0.f : __expf(pm[sp] - mc);
 #pragma unroll
       for (int i = 0; i < E; ++i) acc.v[i] += po[sp].v[i] * sc;
-      lsum += ml[sp].v[1] * sc;
+      lsum += pl[sp] * sc;
     }
     mw = mc;
   }
