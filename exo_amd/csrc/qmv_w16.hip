@@ -21,9 +21,11 @@
 //    activations stay in registers in operand order for the whole launch.  They are loaded as
 //    whole runs of a row, normalised there, and change lanes through the same LDS region.  The waves of
 //    a workgroup together cover K; their partial sums meet in LDS once, at the end.
-//  * codes become (128+nibble) bf16 pairs with one v_and_or_b32 each (exact).  Per group:
-//      acc += s * D + (b - 128 s) * Sx        D = sum (128+q) x,  Sx = sum x   (float32)
-//    Sx comes out of products with a column of ones, in the lanes and registers of D.
+//  * codes become (128+nibble) bf16 pairs with one v_and_or_b32 each (exact; up to four rows: 16+nibble).  Per group:
+//      acc += s * D + (b / -128) * C      C = -128 sum x,  D = C + sum (128+q) x   (float32)
+//    C comes out of products with a column of -128, in the lanes and registers of D, and is where D's sum starts: the
+//    offset leaves in the matrix core, not between two scaled sums (s D + (b - 128 s) sum x, D = sum (128+q) x, rounded
+//    the other way than the exact result 1.6 outputs in 1000 of 14336x4096 under 8 rows; now 0.7).
 //  * DEPTH row blocks of weights are in flight per wave (register buffers in rotation), all of
 //    them requested right behind the activations.  Every refill is issued whether or not a block is
 //    left (past the end all lanes read the same 16 bytes), so that the number of loads in flight at
@@ -139,9 +141,16 @@ __device__ __forceinline__ void lds_barrier() {
 // taken out).  Rows that are not whole pieces of eight groups follow one another all the same, so that a piece begins in one row
 // and ends in the next; up to four pieces per thread.  (With pieces of two groups, one per thread, a workgroup held two blocks of K = 2304:
 // 8 rows, 9216 columns 9.0 -> 6.6 us, 256000 119 -> 73, pair of 9216 15.9 -> 9.7.)
-template <bool WIDE, int SL, int DEPTH, bool NORM, bool KSPLIT, bool PAIR>
+// FEW: up to four rows.  A code c goes into the products as 16 + c instead of 128 + c - the sums that the offset leaves behind are
+// an eighth - for one shift more per four words (1 % of a launch where it was taken for 8 rows).  The 4x4x4 kernel, which takes
+// the other launches of up to four rows, rounds 0.4 to 0.5 outputs in 1000 the other way than the exact result, 128 + c 0.6 to 0.7
+// and 16 + c 0.1 to 0.15.
+template <bool WIDE, int SL, int DEPTH, bool NORM, bool KSPLIT, bool PAIR, bool FEW>
 __global__ __launch_bounds__(1024) void qmv_w16_kernel(const W16Params p) {
   static_assert(!KSPLIT || (!NORM && !PAIR), "split K: one matrix, activations as they are");
+  static_assert(!FEW || (!KSPLIT && !WIDE), "up to four rows: K is not split");
+  constexpr uint32_t MINUS_OFFSET = FEW ? 0xC180C180u : 0xC300C300u;
+  constexpr float PER_OFFSET = FEW ? -0x1p-4f : -0x1p-7f;
   constexpr int RPB = PAIR ? 8 : 16;       // rows of a matrix per block
   constexpr int TURN = turn_bytes(WIDE, SL), SUMS = sum_bytes(WIDE);
   constexpr int LPR = 16 * SL;             // lanes that load a wave's run of an activation row
@@ -275,7 +284,7 @@ __global__ __launch_bounds__(1024) void qmv_w16_kernel(const W16Params p) {
     }
   }
   uint4 xa[SL][4];      // operands of the products of a slice
-  floatx4 sx[SL][NG];   // sums over a group, where D has them
+  floatx4 sx[SL][NG];   // - offset * (sum over a group), where D has them
   {
     // chunk c of row r sits at c ^ r (in 256 bytes): an operand read touches all 64 banks
 #pragma unroll
@@ -288,7 +297,7 @@ __global__ __launch_bounds__(1024) void qmv_w16_kernel(const W16Params p) {
     // (up to eight rows: row 8 of the staged ones, zeros, in the slots of the other group)
     const int r = WIDE ? j : (j >> 3) == (kg >> 1) ? j & 7 : 8;
     const char* from = mine + r * XROW;
-    const uint4 ones = make_uint4(0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u);
+    const uint4 offset = make_uint4(MINUS_OFFSET, MINUS_OFFSET, MINUS_OFFSET, MINUS_OFFSET);
 #pragma unroll
     for (int sl = 0; sl < SL; ++sl)
 #pragma unroll
@@ -303,11 +312,11 @@ __global__ __launch_bounds__(1024) void qmv_w16_kernel(const W16Params p) {
       for (int t = 0; t < 4; ++t) {
         floatx4& to = sx[sl][WIDE ? t >> 1 : 0];
         if (t % (4 / NG) == 0) to = floatx4{0.f, 0.f, 0.f, 0.f};
-        to = mfma(xa[sl][t], ones, to);
+        to = mfma(xa[sl][t], offset, to);
       }
   }
 
-  uint32_t kmask = 0x000F000Fu, kmagic = 0x43004300u;
+  uint32_t kmask = FEW ? 0x00780078u : 0x000F000Fu, kmagic = FEW ? 0x41804180u : 0x43004300u;
   asm volatile("" : "+s"(kmask));
   asm volatile("" : "+v"(kmagic));
   char* const turn_to = mine + lr * 64 + ((lc ^ (lr >> 2)) & 3) * 16;
@@ -348,16 +357,16 @@ __global__ __launch_bounds__(1024) void qmv_w16_kernel(const W16Params p) {
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         uint4 bw;
-        bw.x = (word[t] & kmask) | kmagic;
-        bw.y = ((word[t] >> 4) & kmask) | kmagic;
-        bw.z = ((word[t] >> 8) & kmask) | kmagic;
-        bw.w = ((word[t] >> 12) & kmask) | kmagic;
+        bw.x = ((FEW ? word[t] << 3 : word[t]) & kmask) | kmagic;
+        bw.y = ((word[t] >> (FEW ? 1 : 4)) & kmask) | kmagic;
+        bw.z = ((word[t] >> (FEW ? 5 : 8)) & kmask) | kmagic;
+        bw.w = ((word[t] >> (FEW ? 9 : 12)) & kmask) | kmagic;
         const int g = WIDE ? t >> 1 : 0;
-        dq[g] = mfma(xa[sl][t], bw, t % (4 / NG) == 0 ? floatx4{0.f, 0.f, 0.f, 0.f} : dq[g]);
+        dq[g] = mfma(xa[sl][t], bw, t % (4 / NG) == 0 ? sx[sl][g] : dq[g]);
       }
 #pragma unroll
       for (int g = 0; g < NG; ++g) {
-        const float sc = bf_lo(sb[sl][g]), tb = fmaf(-128.f, sc, bf_hi(sb[sl][g]));
+        const float sc = bf_lo(sb[sl][g]), tb = bf_hi(sb[sl][g]) * PER_OFFSET;
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[r] = fmaf(tb, sx[sl][g][r], fmaf(sc, dq[g][r], acc[r]));
       }
@@ -438,9 +447,9 @@ __global__ __launch_bounds__(1024) void qmv_w16_kernel(const W16Params p) {
   }
 }
 
-template <bool WIDE, int SL, int DEPTH, bool NORM, bool KSPLIT, bool PAIR>
+template <bool WIDE, int SL, int DEPTH, bool NORM, bool KSPLIT, bool PAIR, bool FEW>
 int launch_instance(const W16Params& p, int grid, int nq, int nw, size_t bytes, hipStream_t st) {
-  auto kern = qmv_w16_kernel<WIDE, SL, DEPTH, NORM, KSPLIT, PAIR>;
+  auto kern = qmv_w16_kernel<WIDE, SL, DEPTH, NORM, KSPLIT, PAIR, FEW>;
   static bool attr_done = false;
   if (!attr_done && bytes > 48 * 1024) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMax);
@@ -456,8 +465,10 @@ int launch_instance(const W16Params& p, int grid, int nq, int nw, size_t bytes, 
   return EXO_OK;
 }
 
-template <bool WIDE, int SL, bool NORM, bool KSPLIT, bool PAIR>
+template <bool WIDE, int SL, bool NORM, bool KSPLIT, bool PAIR, bool FEW = false>
 int launch_w16s(W16Params p, int nw, hipStream_t st) {
+  if constexpr (!WIDE && !KSPLIT && !FEW)
+    if (p.M <= 4) return launch_w16s<WIDE, SL, NORM, KSPLIT, PAIR, true>(p, nw, st);
   p.blocks = p.N / (PAIR ? 8 : 16);
   // a wave's region: its activations on their way into operand order, later the lane changes and the partial sums
   const int scales = 16 * (p.Gp * 4 + kRowPad);
@@ -495,8 +506,8 @@ int launch_w16s(W16Params p, int nw, hipStream_t st) {
   p.pairs_log2 = nq * 8 * p.Gp <= 64 * nw ? 0 : 2;
   const int grid = groups * p.kparts;
   const size_t bytes = (size_t)lds_bytes(nq);
-  if (nq == 1) return launch_instance<WIDE, SL, 1, NORM, KSPLIT, PAIR>(p, grid, nq, nw, bytes, st);
-  return launch_instance<WIDE, SL, 2, NORM, KSPLIT, PAIR>(p, grid, nq, nw, bytes, st);
+  if (nq == 1) return launch_instance<WIDE, SL, 1, NORM, KSPLIT, PAIR, FEW>(p, grid, nq, nw, bytes, st);
+  return launch_instance<WIDE, SL, 2, NORM, KSPLIT, PAIR, FEW>(p, grid, nq, nw, bytes, st);
 }
 template <bool WIDE, int SL>
 int launch_w16(const W16Params& p, bool pair, int nw, hipStream_t st) {
