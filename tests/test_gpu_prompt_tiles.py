@@ -353,8 +353,7 @@ def test_large_scales_of_pairs_and_experts(device, M, pair):
     (257, 4100, 8192, "split"), (600, 3076, 6144, "split"),
 ])
 def test_dense_wide_tiles(device, M, N, K, kind):
-    """The 256 x 256 tile of the float products: one row past a tile, ragged columns, two to six steps of K, ranges of K, and
-    each form of the store."""
+    """The 256 x 256 tile of the float products: one row past a tile, ragged columns, one to three steps of K, and ranges of K."""
     g = torch.Generator().manual_seed(M + N)
     x, w = torch.randn(M, K, generator=g).bfloat16(), (torch.randn(N, K, generator=g) * K ** -0.5).bfloat16()
     bias, up = torch.randn(N, generator=g), (torch.randn(N, K, generator=g) * K ** -0.5).bfloat16()
@@ -381,6 +380,42 @@ def test_dense_wide_tiles(device, M, N, K, kind):
     assert (kind == "split") != native.last_variant().endswith("x1"), native.last_variant()
     # one rounding to bf16 of a sum of K products in float32
     torch.testing.assert_close(out.float().cpu(), want, rtol=2.0 ** -8, atol=2e-5 * K ** 0.5)
+
+
+@pytest.mark.parametrize("M,N,K,columns,act,mul,f32,bias", [
+    (257, 30004, 192, 0, None, True, False, True), (300, 32003, 64, 0, "gelu_tanh", True, False, False), (257, 30004, 64, 0, "gelu_tanh", False, True, True),
+    (300, 32003, 64, 77, None, False, True, True),
+    # ranges of K: four columns per thread add them up from 2^19 results on, a fourth of them across both outputs; one with a factor, an
+    # activation or 3077 columns
+    (600, 3076, 6144, 77, None, False, False, True), (600, 3076, 6144, 0, None, False, True, False), (600, 3076, 6144, 0, "relu2", True, False, True),
+    (600, 3077, 6144, 77, None, False, False, True),
+])
+def test_dense_wide_tiles_stores(device, M, N, K, columns, act, mul, f32, bias):
+    """Each form of the 256 x 256 tile's store: bias, activation, factor by row number, element type or float32, a second buffer of the
+    last columns that begins anywhere."""
+    g = torch.Generator(device=device).manual_seed(M + N)
+    x, w, factor = (torch.randn(n, k, device=device, generator=g).bfloat16() for n, k in ((M, K), (N, K), (9, N)))
+    w = (w.float() * K**-0.5).bfloat16()
+    rows = torch.randint(0, 9, (M,), dtype=torch.int32, device=device, generator=g)
+    b = torch.randn(N, device=device, generator=g) if bias else None
+    out = torch.full((M, N), 7.0, dtype=torch.float32 if f32 else torch.bfloat16, device=device)
+    last = torch.full((M, 80), 7.0, device=device)
+    dense_ops.linear(x, w, out, M, bias=b, tail=(last, columns) if columns else None,
+                     after=dense_ops.After(act, factor if mul else None, rows if mul else None))
+    assert native.last_variant().startswith("dense_gemm_wide<single"), native.last_variant()
+    assert (K == 6144) != native.last_variant().endswith("x1"), native.last_variant()
+    y = x.float() @ w.float().T + (b if bias else 0)
+    assert bool((out[:, N - columns:] == 7).all()) and bool((last[:, columns:] == 7).all())
+    # the sum of K products and a bias in float32
+    torch.testing.assert_close(last[:, :columns], y[:, N - columns:], rtol=2.0**-20, atol=2e-5)
+    y = y[:, : N - columns]
+    if act:
+        y = torch.nn.functional.gelu(y, approximate="tanh") if act == "gelu_tanh" else y.clamp(min=0).square()
+    if mul:
+        y = y * factor[rows.long(), : N - columns].float()
+    # one rounding to bf16 (none to float32) of sums that are off by 2e-5; squared and times a factor of up to 5, ten times that
+    rtol = (0 if f32 else 2.0**-8) + 2e-5
+    torch.testing.assert_close(out[:, : N - columns].float(), y, rtol=rtol, atol=2e-4)
 
 
 @pytest.mark.parametrize("tail", [False, True])
