@@ -30,10 +30,9 @@ __device__ __forceinline__ float fma_half(float a, uint32_t v, float c) {
 // bf16 are 4 masks, a shift, 8 FMAs and 4 packs instead of 3 + 8 conversions + 8 + 4, and vector issue is what the
 // GEMMs' loops have too much of: 4-bit pair of 14336x4096 under 2047 rows 425 -> 414 us, under 100 rows 58 -> 52,
 // 6144x4096 under 300 rows 49.7 -> 45.8.
-//  Scales from 2^104 on have no s * 2^24.  With KEEP such a lane keeps s twice (no other but a zero is its own sixteenth), and
-// where a lane of the wave has one, large_scales() makes those lanes' operands once more; otherwise their operands are not
-// right.  (The branch behind each operand costs the short GEMM nothing, the prompt GEMM 2 to 12 %: that one only notes that there
-// are some, and multiplies the wave's tile once more.)
+//  Scales from 2^104 on have no s * 2^24: operands made from them are not right until large_scales() has made those of such lanes
+// once more, from the scale itself.  (A branch behind each operand costs the short GEMM 0.6 %, the prompt GEMM 2 to 12: their loops only
+// note that there are some, and the wave's sums are made once more.)
 template <int BITS>
 struct GroupScale {
   float s, b;
@@ -42,15 +41,13 @@ template <>
 struct GroupScale<4> {
   float s24, s20, b;
 };
-template <int BITS, bool KEEP = false>
+template <int BITS>
 __device__ __forceinline__ GroupScale<BITS> group_scale(float s, float b) {
   GroupScale<BITS> g;
-  if constexpr (BITS == 4) {
-    const bool keep = KEEP && fabsf(s) >= 0x1p104f;
-    g.s24 = s * (keep ? 1.f : 0x1p24f), g.s20 = s * (keep ? 1.f : 0x1p20f);
-  } else {
+  if constexpr (BITS == 4)
+    g.s24 = s * 0x1p24f, g.s20 = s * 0x1p20f;
+  else
     g.s = s;
-  }
   g.b = b;
   return g;
 }
@@ -95,19 +92,18 @@ __device__ __forceinline__ uint32_t piece_value(int i, const PieceCodes& w, cons
   }
 }
 
-// The operand of lanes whose scale is large, from its codes (4 bits; 8 have no such scales).  any: some lane has one
+// The operand of lanes whose scale is large, from its codes (4 bits; 8 have no such scales)
 template <int BITS, typename V>
-__device__ __forceinline__ void large_scales(V& operand, uint32_t v0, const GroupScale<BITS>& g, bool any) {
+__device__ __forceinline__ void large_scales(V& operand, uint32_t v0, float s, float b) {
   if constexpr (BITS == 4) {
-    if (!__builtin_expect(any, 0)) return;
     u32x4 o = __builtin_bit_cast(u32x4, operand);
     const uint32_t ev = v0 & 0x0f0f0f0fu, od = (v0 >> 4) & 0x0f0f0f0fu;
-    const u32x4 l = {pack_bf2(fmaf(g.s24, ubyte_f<0>(ev), g.b), fmaf(g.s24, ubyte_f<0>(od), g.b)),
-                     pack_bf2(fmaf(g.s24, ubyte_f<1>(ev), g.b), fmaf(g.s24, ubyte_f<1>(od), g.b)),
-                     pack_bf2(fmaf(g.s24, ubyte_f<2>(ev), g.b), fmaf(g.s24, ubyte_f<2>(od), g.b)),
-                     pack_bf2(fmaf(g.s24, ubyte_f<3>(ev), g.b), fmaf(g.s24, ubyte_f<3>(od), g.b))};
+    const u32x4 l = {pack_bf2(fmaf(s, ubyte_f<0>(ev), b), fmaf(s, ubyte_f<0>(od), b)),
+                     pack_bf2(fmaf(s, ubyte_f<1>(ev), b), fmaf(s, ubyte_f<1>(od), b)),
+                     pack_bf2(fmaf(s, ubyte_f<2>(ev), b), fmaf(s, ubyte_f<2>(od), b)),
+                     pack_bf2(fmaf(s, ubyte_f<3>(ev), b), fmaf(s, ubyte_f<3>(od), b))};
 #pragma unroll
-    for (int i = 0; i < 4; ++i) o[i] = g.s24 == g.s20 ? l[i] : o[i];
+    for (int i = 0; i < 4; ++i) o[i] = fabsf(s) >= 0x1p104f ? l[i] : o[i];
     operand = __builtin_bit_cast(V, o);
   }
 }

@@ -665,12 +665,13 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
           for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
       for (int k0 = kb; k0 < ke; k0 += BK) {
         WStage st;
+        float s[2];
         GroupScale<BITS> g[2];
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
           load_w1(st, k0, j, 0);
-          g[j] = group_scale<BITS, true>(bf2f((bf16_t)__builtin_amdgcn_raw_buffer_load_b16(rs[PAIR ? j : 0], soff[j], (k0 >> 6) * 2, 0)),
-                                         bf2f((bf16_t)__builtin_amdgcn_raw_buffer_load_b16(rb[PAIR ? j : 0], soff[j], (k0 >> 6) * 2, 0)));
+          s[j] = bf2f((bf16_t)__builtin_amdgcn_raw_buffer_load_b16(rs[PAIR ? j : 0], soff[j], (k0 >> 6) * 2, 0));
+          g[j] = group_scale<BITS>(s[j], bf2f((bf16_t)__builtin_amdgcn_raw_buffer_load_b16(rb[PAIR ? j : 0], soff[j], (k0 >> 6) * 2, 0)));
         }
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
@@ -678,7 +679,7 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
 #pragma unroll
           for (int j = 0; j < 2; ++j) {
             w[j] = dequant8<BITS>(st.w[j], t, g[j]);
-            large_scales<BITS>(w[j], code_word(st.w[j], t, 0), g[j], true);
+            large_scales<BITS>(w[j], code_word(st.w[j], t, 0), s[j], g[j].b);
           }
 #pragma unroll
           for (int i = 0; i < MI; ++i) {

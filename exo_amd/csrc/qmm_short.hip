@@ -187,6 +187,7 @@ __global__ __launch_bounds__(64 * kWaves) void qmm_short_kernel(const ShortParam
   asm volatile("s_barrier" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
 
+  float most = 0.f;  // 4 bits: the largest scale so far (from 2^104 on the steps do not make operands right)
   auto step = [&](Codes(&w)[NT], int slot, int i) {
     // x(i) and w(i) are here; those of step i + 1 may still be out
     wait_vm<XR + NT>();
@@ -212,13 +213,15 @@ __global__ __launch_bounds__(64 * kWaves) void qmm_short_kernel(const ShortParam
     u32x4 bw[2];
     PieceCodes pc{};
     GroupScale<BITS> gs{};
-    bool large = false;
+    if (BITS == 4) {
+#pragma unroll
+      for (int j = 0; j < NT; j += 2) note_scales(most, bf_lo(sc[j]), bf_lo(sc[min(j + 1, NT - 1)]));
+    }
     auto piece = [&](int q, int d) {  // two of an operand's eight values
       const int j = q >> 1, t = q & 1;
-      if (d == 0 && t == 0) gs = group_scale<BITS, true>(bf_lo(sc[j]), bf_hi(sc[j])), large = BITS == 4 && any_large(bf_lo(sc[j]));
+      if (d == 0 && t == 0) gs = group_scale<BITS>(bf_lo(sc[j]), bf_hi(sc[j]));
       piece_codes<BITS>(pc, d, w[j].q[BITS == 4 ? t : (2 * t) & (WORDS - 1)], w[j].q[BITS == 4 ? t : (2 * t + 1) & (WORDS - 1)]);
       bw[q & 1][piece_reg<BITS>(d)] = piece_value<BITS>(d, pc, gs);
-      if (d == 3) large_scales<BITS>(bw[q & 1], w[j].q[t], gs, large);
     };
 #pragma unroll
     for (int d = 0; d < 4; ++d) piece(0, d);
@@ -247,6 +250,37 @@ __global__ __launch_bounds__(64 * kWaves) void qmm_short_kernel(const ShortParam
     step(w1, 1, i + 1);
   }
   if (i < steps) step(w0, 0, i);
+
+  // Weights of large scales (dequant.h): the wave's sums once more, in the same order, one step at a time and without the
+  // activations' slots
+  if constexpr (BITS == 4) {
+    if (__builtin_expect(any_large(most), 0)) {
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) acc[j][m] = floatx4{0.f, 0.f, 0.f, 0.f};
+      for (int n = 0; n < steps; ++n) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+          load_w(w0, j, k_of(n));
+          const uint32_t sc = sb[(j * G + wave + kWaves * n) * 16 + n16];
+          const GroupScale<BITS> gs = group_scale<BITS>(bf_lo(sc), bf_hi(sc));
+#pragma unroll
+          for (int t = 0; t < 2; ++t) {
+            bf16x8_t w = dequant_words8<BITS>(w0[j].q[t], 0, gs);
+            large_scales<BITS>(w, w0[j].q[t], bf_lo(sc), gs.b);
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+              const uint32_t at = ((uint32_t)min(m * 16 + n16, p.M - 1) * (uint32_t)p.K + g0 * 64 + (2 * g4 + t) * 8) * 2;
+              const bf16x8_t a = __builtin_bit_cast(bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(rx, at, k_of(n) * 2, 0));
+              acc[j][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, w, acc[j][m], 0, 0, 0);
+              __builtin_amdgcn_sched_barrier(0);  // (no registers for this)
+            }
+          }
+        }
+      }
+    }
+  }
 
   // the waves' sums: four of them through LDS into the other four, then all eight waves add the four
   __builtin_amdgcn_s_waitcnt(0x0F70);  // the repeated requests have landed
