@@ -273,7 +273,7 @@ def test_nine_to_sixteen_rows(device, M, N, K, bits):
 
 # rows of the short GEMM, of the 128-row and of the 256-row tile; K whose scales come one by one, and in fours
 @pytest.mark.parametrize("bits", [4, 8])
-@pytest.mark.parametrize("M,N,K", [(20, 64, 64), (61, 2048, 256), (100, 200, 192), (200, 264, 256), (300, 8192, 768), (1030, 12288, 4096)])
+@pytest.mark.parametrize("M,N,K", [(20, 64, 64), (61, 2048, 256), (33, 12290, 832), (18, 28680, 512), (63, 4096, 8192), (100, 200, 192), (200, 264, 256), (300, 8192, 768), (1030, 12288, 4096)])
 def test_products_with_unit_rows_are_the_weights(device, M, N, K, bits):
     """The operand that a kernel makes of codes is bf16(scale * code + bias) bit for bit, from subnormal scales to
     those of 2^100: products with rows of one 1 are the weights themselves."""
@@ -292,7 +292,7 @@ def test_products_with_unit_rows_are_the_weights(device, M, N, K, bits):
     assert torch.equal(ops.quantized_matmul(x, q).double(), weights64(q).T[at])
 
 
-@pytest.mark.parametrize("M,N,K", [(20, 64, 64), (61, 2048, 256), (100, 200, 192), (200, 264, 256), (300, 8192, 768), (1030, 12288, 4096)])
+@pytest.mark.parametrize("M,N,K", [(20, 64, 64), (61, 2048, 256), (33, 12290, 832), (18, 28680, 512), (63, 4096, 8192), (100, 200, 192), (200, 264, 256), (300, 8192, 768), (1030, 12288, 4096)])
 def test_products_with_unit_rows_under_the_largest_scales(device, M, N, K):
     """4-bit scales up to the largest bf16 holds, in some groups of some rows: the weights bit for bit, there and beside."""
     g = torch.Generator(device=device).manual_seed(N + K)
@@ -319,7 +319,7 @@ def test_products_with_unit_rows_under_the_largest_scales(device, M, N, K):
     assert torch.equal(ops.quantized_matmul(x, q).double(), want)
 
 
-@pytest.mark.parametrize("M,pair", [(100, True), (600, True), (300, False)])
+@pytest.mark.parametrize("M,pair", [(40, True), (100, True), (600, True), (300, False)])
 def test_large_scales_of_pairs_and_experts(device, M, pair):
     """The same in the gated pair (large scales in some groups of the up matrix) and in the experts' GEMM, whose rows come by a list."""
     N, K, E, top = 512, 256, 3, 2
