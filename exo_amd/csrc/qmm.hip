@@ -569,6 +569,10 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
     // under 520 rows 115.7 | 121.5 us, 1500 205 | 211, 6144x4096 under 1023 60.9 | 61.5)
     constexpr bool X_FIRST = KH && BITS == 8;
     constexpr int XAHEAD = X_FIRST ? 2 : 3;
+    // Experts: activations behind the last wait for weights, which does not count them; of up to 64 rows, where the step is too short
+    // for what is requested at its end, right behind the first weights (at the end | so, gate/up of 1536x4096, 128 experts, 8 bits: 80
+    // tokens 468 | 455 us, 600 514 | 503; 768x2048 level; 2048x768 47.6 | 48.5 under 400; of more rows 2047 tokens 885 | 897)
+    constexpr bool LATE = NI > 2;
 #pragma unroll
     for (int u = 0; u < AHEAD; ++u) load_w(wq[u], min(kb + u * BK, last));
 #pragma unroll
@@ -590,8 +594,8 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
           for (int r = 0; r < NW; ++r)
             if (slot == (!GROUPED ? (W0 + r) * (8 * NI) / (NW + NI) : BITS == 4 ? r * (4 * NI) / NW : 0)) load_w1(wq[(u + AHEAD) & 3], kw, r / (NW / 2), r % (NW / 2));
 #pragma unroll
-          for (int r = 0; r < NI; ++r)  // (grouped: behind the last wait for weights, which does not count these)
-            if (slot == (GROUPED ? 7 * NI + r : (X0 + r) * (8 * NI) / (NW + NI))) load_x1((u + XAHEAD) & 3, kx, r);
+          for (int r = 0; r < NI; ++r)
+            if (slot == (GROUPED ? LATE ? 7 * NI + r : 0 : (X0 + r) * (8 * NI) / (NW + NI))) load_x1((u + XAHEAD) & 3, kx, r);
         });
         // Tile k+2 is in LDS behind the barrier: the next step's last products read its first operands.  What was
         // requested in this step (behind that tile) may still be out - but the fence of __syncthreads() would wait for every
