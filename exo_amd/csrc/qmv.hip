@@ -1398,7 +1398,8 @@ extern "C" int exo_qmv(const uint16_t* x, const uint32_t* w, const uint16_t* sca
 #endif
 
 // Two to four rows that take it too, from sweeps of N = 1024 to 151936 and K = 768 to 4096 (its time over the 4x4x4 kernel's, or
-// where rows are not whole 256-byte slices over that of the kernels below).  K of up to 1024: 0.3 to 0.99 (151936x1024 39 ->
+// where rows are not whole 256-byte slices over that of the kernels below; with codes as 128 + c, as they are now 0.01 more).
+// K of up to 1024: 0.3 to 0.99 (151936x1024 39 ->
 // 21 us).  Behind a norm four rows 0.72 to 1.01 from N = 2048 on (128256x4096 66 -> 58), three 0.71 to 1.02, two 0.79 to 1.0 up to N = 4096 or
 // K = 1536 (others to 1.13).  Without a norm four and three rows 0.84 to 1.02 where the row blocks are dealt evenly, at most a third
 // over the average on the fullest CU, and 1.02 to 1.09 where they are not (4112x3584 under four 6.2 | 6.7); fewer blocks than CUs 0.9 to 0.95

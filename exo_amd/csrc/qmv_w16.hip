@@ -30,9 +30,9 @@
 //    them requested right behind the activations.  Every refill is issued whether or not a block is
 //    left (past the end all lanes read the same 16 bytes), so that the number of loads in flight at
 //    each wait is a constant.
-// At 8 | 16 rows: pair of 14336x4096 20.2 | 22.2 -> 16.4 | 19.4 us (one row: 15.3, a plain read of its weights 12.3),
-// 6144x4096 11.4 | 12.8 -> 8.9 | 11.2, 4096x4096 7.6 | 8.8 -> 6.1 | 7.3, 4096x14336 15.8 | 17.6 -> 13.8 | 16.0,
-// 128256x4096 76 | 91 -> 62 | 79, pair of 8192x2048 at 8 rows 10.1 -> 8.0, 2048x4096 7.2 | 8.3 -> 5.2 | 6.1.
+// At 8 | 16 rows, behind a norm, up to 12 matrices in turn, before the operands came this way -> now: pair of 14336x4096 18.5 | 21.0 -> 15.7 | 18.7
+// us, 6144x4096 11.0 | 12.2 -> 8.4 | 10.3, 4096x4096 9.9 | 11.2 -> 6.9 | 8.7, 128256x4096 69 | 83 -> 56 | 73, pair of 8192x2048 9.6 | 10.7 -> 7.8 |
+// 9.0, 2048x4096 9.8 | 11.0 -> 6.4 | 8.1; 4096x14336 without one 15.5 | 17.4 -> 13.4 | 15.5.
 // What bounds it: the way to the first product (activations, norm, lane changes: 3 us), after which the pair
 // streams at 5 TB/s; with K split, 3 us of hand-over; at 16 rows vector issue (two epilogues per slice).
 #include "../../include/exo_mi355x.h"
