@@ -21,11 +21,13 @@
 //    activations stay in registers in operand order for the whole launch.  They are loaded as
 //    whole runs of a row, normalised there, and change lanes through the same LDS region.  The waves of
 //    a workgroup together cover K; their partial sums meet in LDS once, at the end.
-//  * codes become (128+nibble) bf16 pairs with one v_and_or_b32 each (exact; up to four rows: 16+nibble).  Per group:
-//      acc += s * D + (b / -128) * C      C = -128 sum x,  D = C + sum (128+q) x   (float32)
-//    C comes out of products with a column of -128, in the lanes and registers of D, and is where D's sum starts: the
-//    offset leaves in the matrix core, not between two scaled sums (s D + (b - 128 s) sum x, D = sum (128+q) x, rounded
-//    the other way than the exact result 1.6 outputs in 1000 of 14336x4096 under 8 rows; now 0.7).
+//  * codes become (128+nibble) bf16 pairs with one v_and_or_b32 each (exact; up to four rows: 16+nibble).  Per group, float32:
+//      up to 8 rows   acc += s * D + (b / -128) * C      C = -128 sum x,  D = C + sum (128+q) x
+//      up to 16       acc += s * D + (b - 128 s) * Sx    Sx = sum x,  D = sum (128+q) x
+//    C | Sx comes out of products with a column of -128 | 1, in the lanes and registers of D.  Where D's sum starts at C the offset
+//    leaves in the matrix core and not between two scaled sums: 0.7 outputs in 1000 of 14336x4096 under 8 rows are not the exact result's
+//    rounding, against 1.7, at the same time.  (9 to 16 rows keep their sums, 1.6 in 1000: prompts of up to 16 tokens go through them,
+//    and which of two tied tokens follows hangs on their bits.)
 //  * DEPTH row blocks of weights are in flight per wave (register buffers in rotation), all of
 //    them requested right behind the activations.  Every refill is issued whether or not a block is
 //    left (past the end all lanes read the same 16 bytes), so that the number of loads in flight at
@@ -149,8 +151,7 @@ template <bool WIDE, int SL, int DEPTH, bool NORM, bool KSPLIT, bool PAIR, bool 
 __global__ __launch_bounds__(1024) void qmv_w16_kernel(const W16Params p) {
   static_assert(!KSPLIT || (!NORM && !PAIR), "split K: one matrix, activations as they are");
   static_assert(!FEW || (!KSPLIT && !WIDE), "up to four rows: K is not split");
-  constexpr uint32_t MINUS_OFFSET = FEW ? 0xC180C180u : 0xC300C300u;
-  constexpr float PER_OFFSET = FEW ? -0x1p-4f : -0x1p-7f;
+  constexpr uint32_t COLUMN = WIDE ? 0x3F803F80u : FEW ? 0xC180C180u : 0xC300C300u;  // 1, -16, -128
   constexpr int RPB = PAIR ? 8 : 16;       // rows of a matrix per block
   constexpr int TURN = turn_bytes(WIDE, SL), SUMS = sum_bytes(WIDE);
   constexpr int LPR = 16 * SL;             // lanes that load a wave's run of an activation row
@@ -284,7 +285,7 @@ __global__ __launch_bounds__(1024) void qmv_w16_kernel(const W16Params p) {
     }
   }
   uint4 xa[SL][4];      // operands of the products of a slice
-  floatx4 sx[SL][NG];   // - offset * (sum over a group), where D has them
+  floatx4 sx[SL][NG];   // Sx or C of a group, where D has them
   {
     // chunk c of row r sits at c ^ r (in 256 bytes): an operand read touches all 64 banks
 #pragma unroll
@@ -297,7 +298,7 @@ __global__ __launch_bounds__(1024) void qmv_w16_kernel(const W16Params p) {
     // (up to eight rows: row 8 of the staged ones, zeros, in the slots of the other group)
     const int r = WIDE ? j : (j >> 3) == (kg >> 1) ? j & 7 : 8;
     const char* from = mine + r * XROW;
-    const uint4 offset = make_uint4(MINUS_OFFSET, MINUS_OFFSET, MINUS_OFFSET, MINUS_OFFSET);
+    const uint4 column = make_uint4(COLUMN, COLUMN, COLUMN, COLUMN);
 #pragma unroll
     for (int sl = 0; sl < SL; ++sl)
 #pragma unroll
@@ -312,7 +313,7 @@ __global__ __launch_bounds__(1024) void qmv_w16_kernel(const W16Params p) {
       for (int t = 0; t < 4; ++t) {
         floatx4& to = sx[sl][WIDE ? t >> 1 : 0];
         if (t % (4 / NG) == 0) to = floatx4{0.f, 0.f, 0.f, 0.f};
-        to = mfma(xa[sl][t], offset, to);
+        to = mfma(xa[sl][t], column, to);
       }
   }
 
@@ -362,11 +363,11 @@ __global__ __launch_bounds__(1024) void qmv_w16_kernel(const W16Params p) {
         bw.z = ((word[t] >> (FEW ? 5 : 8)) & kmask) | kmagic;
         bw.w = ((word[t] >> (FEW ? 9 : 12)) & kmask) | kmagic;
         const int g = WIDE ? t >> 1 : 0;
-        dq[g] = mfma(xa[sl][t], bw, t % (4 / NG) == 0 ? sx[sl][g] : dq[g]);
+        dq[g] = mfma(xa[sl][t], bw, t % (4 / NG) ? dq[g] : WIDE ? floatx4{0.f, 0.f, 0.f, 0.f} : sx[sl][g]);
       }
 #pragma unroll
       for (int g = 0; g < NG; ++g) {
-        const float sc = bf_lo(sb[sl][g]), tb = bf_hi(sb[sl][g]) * PER_OFFSET;
+        const float sc = bf_lo(sb[sl][g]), b = bf_hi(sb[sl][g]), tb = WIDE ? fmaf(-128.f, sc, b) : b * (FEW ? -0x1p-4f : -0x1p-7f);
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[r] = fmaf(tb, sx[sl][g][r], fmaf(sc, dq[g][r], acc[r]));
       }
