@@ -497,6 +497,7 @@ extern "C" int exo_rope_kv_append_tab(const uint16_t* qkv, uint16_t* q_out, uint
   EXO_REQUIRE(!rope_table || table_rows > 0, "exo_rope_kv_append: table without rows");
   EXO_REQUIRE((int64_t)B * T <= 0x7fffffff / 2, "exo_rope_kv_append: too many tokens");
   const uintptr_t all = (uintptr_t)qkv | (uintptr_t)q_out | (uintptr_t)k_cache | (uintptr_t)v_cache | (uintptr_t)rope_table | (uintptr_t)q_norm_w | (uintptr_t)k_norm_w;
+  if (!rope_table) table_rows = 0;  // (no position is inside it)
   if ((all & 15) == 0) {
     const auto fn = D == 128 ? rope_kv_wide_kernel<128> : rope_kv_wide_kernel<64>;
     fn<<<dim3(B * T, exo_ceil_div(Hq + 2 * Hkv, 2048 / D * kRopeHeadsPerThread)), 256, 0, (hipStream_t)stream>>>(

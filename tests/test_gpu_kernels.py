@@ -780,6 +780,31 @@ def test_rope_kv_append_pieces(device, D, Hq, Hkv, qk_norm):
     assert bool((out[0][1][0, :, T:] == 7).all()) and bool((out[0][2][1, :, :30] == 7).all())
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("at", [0, 4])
+def test_rope_kv_append_rows_without_a_table(device, D, at):
+    """A null table with a number of rows, operands at 16 bytes and not: the angles come from the frequencies for every position, as
+    in the entry point that takes no table."""
+    B, T, Hq, Hkv, S_max = 2, 5, 4, 2, 16
+    g = torch.Generator(device=device).manual_seed(D)
+    n = B * T * (Hq + 2 * Hkv) * D
+    qkv = torch.randn(n + 8, device=device, generator=g).bfloat16()[at : at + n]
+    inv = torch.from_numpy(O.rope_inv_freq(D, 5e5, None)).to(device)
+    pos = torch.tensor([0, 9], dtype=torch.int32, device=device)
+    out = []
+    for rows in (None, 8):
+        kc, vc = (torch.zeros(B, Hkv, S_max, D, device=device).bfloat16() for _ in range(2))
+        q = torch.empty(B * T, Hq * D, device=device).bfloat16()
+        head = [t.data_ptr() for t in (qkv, q, kc, vc, pos, inv)]
+        tail = [None, None, 0.0, B, T, Hq, Hkv, D, S_max, torch.cuda.current_stream().cuda_stream]
+        lib = native.load()
+        rc = lib.exo_rope_kv_append(*head, *tail) if rows is None else lib.exo_rope_kv_append_tab(*head, None, rows, *tail)
+        assert rc == 0
+        out.append((q, kc, vc))
+    for a, b in zip(*out):
+        assert torch.equal(a, b) and bool(a.any())
+
+
 @pytest.mark.parametrize("D,Hq,Hkv", [(64, 32, 8), (128, 32, 8), (128, 32, 4), (128, 64, 4), (128, 4, 4)])
 @pytest.mark.parametrize("lens", [[1, 2], [100, 37], [513, 1024]])
 def test_sdpa_decode(device, D, Hq, Hkv, lens):
