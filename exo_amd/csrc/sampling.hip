@@ -56,10 +56,14 @@ constexpr float kBan = -1e9f;
 typedef unsigned long long u64;
 
 // Count and mass of a table entry in one word, so that one integer addition carries both: the mass in 2^-40 below, the
-// count above.  A row has at most 2^18 tokens and its probabilities sum up to 1 but for rounding, so neither overflows.
-constexpr int kCountShift = 41;
+// count above.  A row has at most 2^18 tokens.  Its probabilities sum up to 1 but for the rounding of the log-normaliser lse = max + log
+// sum: less than 2 where |max| is below 2^23 (lse off by 1/2 at most).  Beyond that the logarithm may be lost whole, each of n equal
+// maxima then has a probability of 1, and masses count in 2^-26 (mass_shift): 2^18 of those still fit below the count.
+constexpr int kCountShift = 45;
 constexpr u64 kMassMask = (1ull << kCountShift) - 1;
 constexpr float kMassOne = 0x1p40f;
+constexpr int kMassShift = 14;
+__device__ __forceinline__ int mass_shift(float mx) { return fabsf(mx) < 0x1p23f ? 0 : kMassShift; }
 
 struct RowWs {
   float part[kBlocks][4];  // max, argmax (int bits), sum exp(x - max), kept weight
@@ -371,14 +375,17 @@ struct Wanted {
   unsigned int kk;  // top-k (0: none)
   bool use_p;       // top-p
   u64 target;       // top_p of the mass, fixed point
+  float one;        // a probability of 1 in the same
   bool top;         // the 20 most likely
 };
-__device__ __forceinline__ Wanted wanted_of(const exo_sampler_params& p, bool want_top) {
+__device__ __forceinline__ Wanted wanted_of(const exo_sampler_params& p, bool want_top, float mx) {
   const bool sampling = p.temperature != 0.f;
   Wanted q;
   q.kk = (sampling && p.top_k > 0) ? (unsigned int)p.top_k : 0u;
   q.use_p = sampling && p.top_p > 0.f && p.top_p < 1.f;
-  q.target = q.use_p ? (u64)((double)p.top_p * (double)kMassOne) : 0ull;
+  const int shift = mass_shift(mx);
+  q.one = shift ? kMassOne / (float)(1 << kMassShift) : kMassOne;
+  q.target = q.use_p ? ((u64)((double)p.top_p * (double)kMassOne) + (1u << shift) - 1) >> shift : 0ull;
   q.top = want_top;
   return q;
 }
@@ -508,7 +515,6 @@ __global__ __launch_bounds__(256) void sample_coarse_kernel(
   const int n_edit = has_edits ? w->n_edit : 0;
   const exo_sampler_params p = params[row];
   if (!row_needs_table(p, want_top != 0)) return;
-  const Wanted q = wanted_of(p, want_top != 0);
   for (int i = threadIdx.x; i < kBuckets * kCopies / 2; i += 256) reinterpret_cast<uint4*>(hist)[i] = make_uint4(0, 0, 0, 0);
   stage_edits(w, g, n_edit, ed);
   float xv[8 * NU];
@@ -516,6 +522,7 @@ __global__ __launch_bounds__(256) void sample_coarse_kernel(
   float mx, lse;
   int mi;
   merge_stats(part, mx, mi, lse);
+  const Wanted q = wanted_of(p, want_top != 0, mx);
   const int lo = smallest_key(p, q, part.mx, mx);
   __syncthreads();
 #pragma unroll
@@ -527,7 +534,7 @@ __global__ __launch_bounds__(256) void sample_coarse_kernel(
         const int key = key_of(x);
         if (sh.i0[u] + k < g.hi && key >= lo) {  // (-inf logits are real values too: key 0x007f)
           u64 v = 1ull << kCountShift;
-          if (q.use_p) v += (u64)(expf(x - lse) * kMassOne);
+          if (q.use_p) v += (u64)(expf(x - lse) * q.one);
           atomicAdd(&hist[(key >> 7) * kCopies + (threadIdx.x & (kCopies - 1))], v);
         }
       }
@@ -562,18 +569,18 @@ __global__ __launch_bounds__(256) void sample_fine_kernel(
   const int n_edit = has_edits ? w->n_edit : 0;
   const exo_sampler_params p = params[row];
   if (!row_needs_table(p, want_top != 0)) return;
-  const Wanted q = wanted_of(p, want_top != 0);
   for (int i = threadIdx.x; i < kTargets * kFine; i += 256) (&hist[0][0])[i] = 0;
   stage_edits(w, g, n_edit, ed);
+  float mx, lse;
+  int mi;
+  merge_stats(part, mx, mi, lse);
+  const Wanted q = wanted_of(p, want_top != 0, mx);
   int bkt[kTargets];
   u64 above[kTargets] = {0ull, 0ull, 0ull};
   {
     const bool active[kTargets] = {q.kk != 0, q.use_p, q.top};
     scan_down(entry, q, active, bkt, above);
   }
-  float mx, lse;
-  int mi;
-  merge_stats(part, mx, mi, lse);
   if (blockIdx.x == 0 && threadIdx.x == 0) {
 #pragma unroll
     for (int j = 0; j < kTargets; ++j) {
@@ -595,7 +602,7 @@ __global__ __launch_bounds__(256) void sample_fine_kernel(
         if (sh.i0[u] + k < g.hi && (b == bkt[0] || b == bkt[1] || b == bkt[2])) {
           const u64 one = 1ull << kCountShift;
           if (b == bkt[0]) atomicAdd(&hist[0][f], one);
-          if (b == bkt[1]) atomicAdd(&hist[1][f], one + (u64)(expf(x - lse) * kMassOne));
+          if (b == bkt[1]) atomicAdd(&hist[1][f], one + (u64)(expf(x - lse) * q.one));
           if (b == bkt[2]) atomicAdd(&hist[2][f], one);
         }
       }
@@ -659,17 +666,17 @@ __global__ __launch_bounds__(256) void sample_weights_kernel(
   float table_thr = -INFINITY;
   int kt = 0;
   const bool table = has_tables && row_needs_table(p, want_top != 0);  // (uniform over the workgroup)
+  float mx, lse;
+  int mi;
+  merge_stats(part, mx, mi, lse);
   if (table) {
-    fine_keys(fine, wanted_of(p, want_top != 0), s_keys);
+    fine_keys(fine, wanted_of(p, want_top != 0, mx), s_keys);
     if (blockIdx.x == 0)
       for (int b = threadIdx.x; b < kBuckets; b += 256) T->coarse[b] = 0;
   }
   stage_edits(w, g, n_edit, ed);
   float xv[8 * NU];
   expand_share(sh, g, n_edit, ed, xv);
-  float mx, lse;
-  int mi;
-  merge_stats(part, mx, mi, lse);
   if (table) {
     __syncthreads();
     if (s_keys[0] >= 0) table_thr = value_of(s_keys[0]);

@@ -140,6 +140,34 @@ def test_sample_counts_only_what_matters(device, V):
         _check_rows(ds, x, settings, [[] for _ in settings], draws, want_top=True)
 
 
+@pytest.mark.parametrize("V", [5000, 262144])
+def test_sample_equal_maxima_that_hide_their_number(device, V):
+    """Equal maxima so large that the log-normaliser cannot be told from them: each has a probability of 1, and the mass that
+    they add up to reaches neither the counts beside it nor the nucleus edge, which is their value (a temperature of the logits'
+    own size would draw the others too)."""
+    rows = [(2.0**24, 2), (2.0**25, 3), (-(2.0**24), 33), (2.0**26, 19), (2.0**30, 20), (2.0**23, 21), (2.0**28, 4999), (-(2.0**40), V)]
+    settings = [SamplerSettings(temperature=abs(m) / 8, min_p=0.0, top_p=p, seed=i) for i, ((m, _), p) in enumerate(zip(rows, [0.5, 0.9, 0.3, 1e-9, 0.3, 0.7, 0.6, 0.95]))]
+    x = np.zeros((len(rows), V), np.float32)
+    r = np.random.default_rng(V)
+    for i, (m, n) in enumerate(rows):
+        x[i] = m - abs(m) * np.linspace(0.25, 0.75, V, dtype=np.float32)
+        x[i, r.permutation(V)[:n]] = m
+    lt = t_bf16(x, device)
+    x = lt.float().cpu().numpy()
+    ds = DeviceSampler(len(rows), V, device)
+    for i, s in enumerate(settings):
+        ds.set_row(i, s, [])
+    for _ in range(6):
+        ds.sample(lt, len(rows), ds.mode(len(rows), want_top=True))
+        torch.cuda.synchronize()
+        lse, tok = ds.lse.cpu().numpy(), ds.token.cpu().numpy()
+        for i in range(len(rows)):
+            ids, _ = S.top_logprobs(x[i], 20)
+            np.testing.assert_array_equal(ds.top_idx[i].cpu().numpy(), ids, err_msg=f"row {i} top ids")
+            np.testing.assert_array_equal(ds.top_val[i].cpu().numpy(), x[i][ids] - lse[i])
+            assert x[i, tok[i]] == x[i].max(), (i, tok[i], x[i, tok[i]])
+
+
 def test_sample_modes_and_reuse(device):
     """Rows that do not ask for a stage pass through it untouched; the key tables are left
     zero (the same launch twice gives the same result); launches of different row counts
