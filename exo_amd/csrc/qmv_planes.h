@@ -2,12 +2,13 @@
 //
 // The dot-product kernel spends 44 vector instructions on 32 codes of a lane, half of them at half rate: masks, shifts and
 // dot products, 70 ns of a SIMD per KiB of 4-bit codes, and 15 to 20 more for scales and the sum over the wave.  Here codes enter
-// v_mfma_i32_16x16x64_i8 as they are (4 bits: two masks and a shift per word; 8 bits: less 128) and the row enters exactly:
-// as 32-bit whole numbers in units of 2^(E-29), E the exponent of the largest element of a wave's share, cut into four
+// v_mfma_i32_16x16x64_i8 as they are (4 bits: two masks and a shift per word; 8 bits: less 128) and the row enters as
+// 32-bit whole numbers in units of 2^(E-29), E the exponent of the largest element of a group of 64, cut into four
 // signed bytes ("planes") that are rows of the A operand.  Products and sums over a group are whole numbers, without
 // rounding; a lane puts a group's four plane sums together (exact but for the conversions), scales them, and adds
-// float32.  An element more than 22 binades below the largest of its share loses its last bits, an error of 2^-29 of that
-// largest.
+// float32.  An element more than 22 binades below the largest of its group is rounded to that unit, which is at most 2^-30 of the
+// largest; float32 sums of products with 128 + c lose 2^-17 of it.  (A unit per group and not per row: an element
+// far larger than all others leaves the other groups as they are.)
 //
 // A workgroup's four waves split K.  A tile is 8 weight rows (a pair: 4 of each matrix): columns 0..7 of the B operand are the
 // first half of a wave's share of K, columns 8..15 the second, and a wave instruction loads 16 x 64 bytes.  The planes of the
@@ -28,8 +29,13 @@ constexpr int kPlaneRows = 8;  // weight rows of a tile
 // A product's planes in LDS: four lanes' 16 codes, four planes, 16 bytes each, and 16 zeros for the operand rows that a lane does
 // not hold
 constexpr int kPlaneBlock = 272;
+// A group of the row beside its planes
+struct GroupSum {
+  float sum;
+  int unit;  // its whole numbers count in 2^unit
+};
 // LDS of a wave: the planes of K / 4 codes and their groups' sums
-__host__ __device__ constexpr int planes_wave_bytes(int K) { return K / 256 * kPlaneBlock + K / 64; }
+__host__ __device__ constexpr int planes_wave_bytes(int K) { return K / 256 * kPlaneBlock + K / 256 * (int)sizeof(GroupSum); }
 
 // What a lane does for its rows of a tile and half of a row's share (see above): the groups' products, from the four accumulator rows
 // that it holds, or the biases.
@@ -59,46 +65,44 @@ __device__ __forceinline__ const char* plane_operand(const char* planes, int lan
   return planes + (mine ? half * (units * (BITS == 4 ? 2 : 1) * kPlaneBlock) + q * 64 + (n & 3) * 16 : 256);
 }
 
-// bound of a run's absolute values, ahead of a norm with weights w
-__device__ __forceinline__ float plane_bound(const uint4& x, const uint4& w, bool norm) {
-  const uint32_t x4[4] = {x.x, x.y, x.z, x.w}, n4[4] = {w.x, w.y, w.z, w.w};
-  float most = 0.f;
-  if (norm) {
-#pragma unroll
-    for (int k = 0; k < 4; ++k) most = fmaxf(most, fmaxf(fabsf(bf_lo(x4[k]) * bf_lo(n4[k])), fabsf(bf_hi(x4[k]) * bf_hi(n4[k]))));
-  } else {
-#pragma unroll
-    for (int k = 0; k < 4; ++k) most = fmaxf(most, fmaxf(fabsf(bf_lo(x4[k])), fabsf(bf_hi(x4[k]))));
-  }
-  return most;
+// the largest of eight lanes' runs, as the bits of its absolute value
+__device__ __forceinline__ uint32_t group_most(const uint4& x) {
+  typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+  auto larger = [](uint32_t a, uint32_t b) {
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b)));
+  };
+  constexpr uint32_t kAbs = 0x7fff7fffu;
+  uint32_t m = larger(larger(x.x & kAbs, x.y & kAbs), larger(x.z & kAbs, x.w & kAbs));
+  m = larger(m, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0xB1, 0xf, 0xf, false));   // quad_perm [1,0,3,2]
+  m = larger(m, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x4E, 0xf, 0xf, false));   // quad_perm [2,3,0,1]
+  m = larger(m, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x141, 0xf, 0xf, false));  // row_half_mirror
+  return max(m & 0xffffu, m >> 16);
 }
 
-// A wave's elements as planes: `runs` runs of 8, lane l holding the runs l, l + 64 ...; `most` bounds their absolute values.
+// A wave's elements as planes: `runs` runs of 8, lane l holding the runs l, l + 64 ...
 // `place`: where the 16-byte pieces of 16 elements begin, their four planes 16 bytes apart.
-// `unit`: what the whole numbers count in; `bad`: an element is infinite or not a number, which makes every result one that is
+// `bad`: an element is infinite or not a number, which makes every result one that is
 // not a number, as its products with 128 + c would.
 template <int BITS, int XS, typename Place>
-__device__ __forceinline__ void store_planes(const uint4 (&xr)[XS], float most, int runs, Place place, float* sums, float& unit, bool& bad) {
+__device__ __forceinline__ void store_planes(const uint4 (&xr)[XS], int runs, Place place, GroupSum* sums, bool& bad) {
   const int lane = threadIdx.x & 63;
-  // |x| * 2^shift < 2^30.  (No more than 2^120: what undoes it stays a normal number.  It is undone ahead of the scales, which
-  // may be as large as their type holds.)
-  const int shift = min(29 - ((int)(__builtin_bit_cast(uint32_t, most) >> 23) - 127), 120);
-  unit = __builtin_ldexpf(1.f, -shift);
-  float all = 0.f;
+  uint32_t largest = 0;
 #pragma unroll
   for (int i = 0; i < XS; ++i) {
     const int run = lane + 64 * i;
     const uint32_t x4[4] = {xr[i].x, xr[i].y, xr[i].z, xr[i].w};
+    const uint32_t most = group_most(xr[i]);
+    largest = max(largest, most);
+    const int shift = 29 + 127 - (int)(most >> 7);  // |x| * 2^shift < 2^30
     uint32_t d[8];
     float gs = 0.f;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       gs += bf_lo(x4[k]) + bf_hi(x4[k]);
       // byte i of X + 0x808080 less 128 (the top one as it is): the signed digits of X
-      d[2 * k] = (uint32_t)(int)__builtin_ldexpf(bf_lo(x4[k]), shift) + 0x00808080u;
-      d[2 * k + 1] = (uint32_t)(int)__builtin_ldexpf(bf_hi(x4[k]), shift) + 0x00808080u;
+      d[2 * k] = (uint32_t)(int)__builtin_rintf(__builtin_ldexpf(bf_lo(x4[k]), shift)) + 0x00808080u;
+      d[2 * k + 1] = (uint32_t)(int)__builtin_rintf(__builtin_ldexpf(bf_hi(x4[k]), shift)) + 0x00808080u;
     }
-    all += gs;
     // operand words: the codes of a word's even places, then of its odd ones (8 bits: as they come)
     uint32_t out[4][2];  // [plane][operand word]
 #pragma unroll
@@ -119,10 +123,10 @@ __device__ __forceinline__ void store_planes(const uint4 (&xr)[XS], float most, 
     if (XS * 64 == runs || run < runs) {
 #pragma unroll
       for (int pl = 0; pl < 4; ++pl) *reinterpret_cast<uint2*>(place(run >> 1) + pl * 16 + (run & 1) * 8) = make_uint2(out[pl][0], out[pl][1]);
-      if ((run & 7) == 0) sums[run >> 3] = gs;
+      if ((run & 7) == 0) sums[run >> 3] = {gs, -shift};
     }
   }
-  bad = __ballot(!(fabsf(all) < INFINITY)) != 0;
+  bad = __ballot(largest >= 0x7f80u) != 0;
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   __builtin_amdgcn_wave_barrier();  // (what a wave reads below it has written itself)
 }
@@ -138,8 +142,8 @@ __device__ __forceinline__ void clear_planes(char* planes, int blocks) {
 
 // acc += a batch's groups: UB units of codes w and their scales s, the operands from a and the groups' sums from sr on
 template <int BITS, int UB, int SW>
-__device__ __forceinline__ void plane_products(const uint4 (&w)[UB], const uint32_t (&s)[SW], const char* a, const float* sr, const PlaneLane& l,
-                                               float unit, uint32_t kmask, float& acc) {
+__device__ __forceinline__ void plane_products(const uint4 (&w)[UB], const uint32_t (&s)[SW], const char* a, const GroupSum* sr, const PlaneLane& l,
+                                               uint32_t kmask, float& acc) {
   constexpr int GU = BITS == 4 ? 2 : 1;
   i32x4 d[UB];
 #pragma unroll
@@ -160,9 +164,11 @@ __device__ __forceinline__ void plane_products(const uint4 (&w)[UB], const uint3
   }
 #pragma unroll
   for (int u = 0; u < UB; ++u) {
-    float f = fmaf((float)((d[u][3] << 8) + d[u][2]), 65536.f * unit, (float)((d[u][1] << 8) + d[u][0]) * unit);
+    const GroupSum g = sr[u * GU];
+    // (the unit is put in ahead of the scales, which may be as large as their type holds)
+    float f = __builtin_ldexpf(fmaf((float)((d[u][3] << 8) + d[u][2]), 65536.f, (float)((d[u][1] << 8) + d[u][0])), g.unit);
     if (!l.products) f = 0.f;  // (the other half's codes)
-    const float v = fmaf(l.offset, sr[u * GU], f);
+    const float v = fmaf(l.offset, g.sum, f);
     float sc;
     if constexpr (BITS == 4)
       sc = l.group ? bf_hi(s[u]) : bf_lo(s[u]);
@@ -205,7 +211,7 @@ __global__ __launch_bounds__(256) void qmv_planes_kernel(const QmvParams p) {
 
   // LDS, of each wave by itself: the planes, the groups' sums; then the tiles' partial sums
   char* const planes = reinterpret_cast<char*>(smem) + wave * planes_wave_bytes(K);
-  float* const sums = reinterpret_cast<float*>(planes + (K / 256) * kPlaneBlock);
+  GroupSum* const sums = reinterpret_cast<GroupSum*>(planes + (K / 256) * kPlaneBlock);
   float (*const red)[4][kPlaneRows] = reinterpret_cast<float (*)[4][kPlaneRows]>(reinterpret_cast<char*>(smem) + 4 * planes_wave_bytes(K));
   __shared__ float s_ss[4];
 
@@ -300,28 +306,22 @@ __global__ __launch_bounds__(256) void qmv_planes_kernel(const QmvParams p) {
   issue(buf[1]);
   __builtin_amdgcn_sched_barrier(0);
 
-  // ---- the row: norm, whole numbers, planes.  The largest element's exponent is bounded ahead of the norm's barrier.
-  float most = 0.f, ss = 0.f;
-#pragma unroll
-  for (int i = 0; i < XS; ++i) {
-    most = fmaxf(most, plane_bound(xr[i], nw[i], p.norm_w != nullptr));
-    if (p.norm_w) ss += sumsq_word<4>(xr[i]);
-  }
-  most = wave_max_f32_uniform(most);
+  // ---- the row: norm, whole numbers, planes
   if (p.norm_w) {
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < XS; ++i) ss += sumsq_word<4>(xr[i]);
     ss = wave_total(ss);
     if (lane == 0) s_ss[wave] = ss;
     __syncthreads();
     const float inv = rsqrtf((s_ss[0] + s_ss[1] + s_ss[2] + s_ss[3]) / (float)K + p.eps);
 #pragma unroll
     for (int i = 0; i < XS; ++i) norm_word<4>(xr[i], nw[i], inv);
-    most *= inv * 1.0625f;  // (the two products' order and the rounding to 8 bits)
   }
-  float unit;
   bool bad;
-  store_planes<BITS, XS>(xr, most, XS * 64, [&](int piece) { return plane_piece<BITS>(planes, piece); }, sums, unit, bad);
+  store_planes<BITS, XS>(xr, XS * 64, [&](int piece) { return plane_piece<BITS>(planes, piece); }, sums, bad);
   const char* const a_row = plane_operand<BITS>(planes, lane, UW);
-  const float* const s_row = sums + l.half * (UW * GU) + l.group;
+  const GroupSum* const s_row = sums + l.half * (UW * GU) + l.group;
   uint32_t kmask = 0x0F0F0F0Fu;
   asm volatile("" : "+s"(kmask));
 
@@ -329,8 +329,8 @@ __global__ __launch_bounds__(256) void qmv_planes_kernel(const QmvParams p) {
   int tile = t0, batch = 0;
   auto compute = [&](const Batch& b) {
     const char* a = a_row + batch * (UB * H * kPlaneBlock);
-    const float* sr = s_row + batch * (UB * GU);
-    plane_products<BITS>(b.w, b.s, a, sr, l, unit, kmask, acc);
+    const GroupSum* sr = s_row + batch * (UB * GU);
+    plane_products<BITS>(b.w, b.s, a, sr, l, kmask, acc);
     if (++batch == ITERS) {  // the tile's row sums of this wave
       batch = 0;
       const float v = plane_row_sum(acc, l);

@@ -23,7 +23,7 @@ template <int TOK>
 constexpr int kRowsTiles = TOK == 4 ? 2 : 1;  // tiles between barriers
 template <int TOK>
 constexpr int rows_lds(int K) {
-  return K / 64 * kPlaneGroup * (TOK / 4) + TOK * (K / 64 + 4) * 4 + 2 * kRowsTiles<TOK> * kRowsWaves * TOK * 16 * 4;
+  return K / 64 * kPlaneGroup * (TOK / 4) + TOK * (K / 64 + 4) * (int)sizeof(GroupSum) + 2 * kRowsTiles<TOK> * kRowsWaves * TOK * 16 * 4;
 }
 
 // K = 2048 * XS; p.slots: tiles of 16 rows (a pair: 8 of each matrix)
@@ -42,9 +42,9 @@ __global__ __launch_bounds__(64 * kRowsWaves) void qmv_planes_rows_kernel(const 
   const int n = lane & 15, q = lane >> 4;
 
   char* const planes = reinterpret_cast<char*>(smem);
-  float* const sums = reinterpret_cast<float*>(planes + SETS * G * kPlaneGroup);  // [TOK][G + 4]
+  GroupSum* const sums = reinterpret_cast<GroupSum*>(planes + SETS * G * kPlaneGroup);  // [TOK][G + 4]
   float (*const red)[C][kRowsWaves][SETS * 64] = reinterpret_cast<float (*)[C][kRowsWaves][SETS * 64]>(sums + TOK * (G + 4));
-  __shared__ float s_ss[kRowsWaves], s_unit[kRowsWaves];
+  __shared__ float s_ss[kRowsWaves];
   __shared__ int s_bad[kRowsWaves];
 
   const int tiles = p.slots;
@@ -110,11 +110,8 @@ __global__ __launch_bounds__(64 * kRowsWaves) void qmv_planes_rows_kernel(const 
     asm volatile("s_barrier" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
   };
-  float most = 0.f, ss = 0.f;
-#pragma unroll
-  for (int i = 0; i < XR; ++i) most = fmaxf(most, plane_bound(xr[i], nw[i], p.norm_w != nullptr));
-  most = wave_max_f32_uniform(most);
   if (p.norm_w) {
+    float ss = 0.f;
 #pragma unroll
     for (int i = 0; i < XR; ++i) ss += sumsq_word<4>(xr[i]);
     ss = wave_total(ss);
@@ -126,33 +123,30 @@ __global__ __launch_bounds__(64 * kRowsWaves) void qmv_planes_rows_kernel(const 
     const float inv = rsqrtf(ss / (float)K + p.eps);
 #pragma unroll
     for (int i = 0; i < XR; ++i) norm_word<4>(xr[i], nw[i], inv);
-    most *= inv * 1.0625f;  // (the two products' order and the rounding to 8 bits)
   }
-  float unit;
   bool bad;
   {
     char* const mine = planes + ((tok >> 2) * G + part * (G / WPT)) * kPlaneGroup + (tok & 3) * 64;
-    float* const ms = sums + tok * (G + 4) + part * (G / WPT);
-    store_planes<BITS, XR>(xr, most, XR * 64, [&](int piece) {
+    GroupSum* const ms = sums + tok * (G + 4) + part * (G / WPT);
+    store_planes<BITS, XR>(xr, XR * 64, [&](int piece) {
       const int pc = piece & 3, slot = BITS == 4 ? (pc & 1) << 1 | pc >> 1 : pc;
       return mine + (piece >> 2) * kPlaneGroup + slot * kPlaneQuarter;
-    }, ms, unit, bad);
+    }, ms, bad);
   }
-  if (lane == 0) s_unit[wave] = unit, s_bad[wave] = bad;
+  if (lane == 0) s_bad[wave] = bad;
   lds_barrier();
 
-  float scale_of[SETS], poison[SETS];
+  float poison[SETS];
 #pragma unroll
   for (int s = 0; s < SETS; ++s) {
     const int t = s * 4 + q;
-    scale_of[s] = s_unit[t + (WPT == 2 ? wave / TOK * TOK : 0)];
     int any = s_bad[t];
 #pragma unroll
     for (int w = 1; w < WPT; ++w) any |= s_bad[t + w * TOK];
     poison[s] = any ? __builtin_nanf("") : 0.f;
   }
   const char* const a_row = planes + wave * GW * kPlaneGroup + q * kPlaneQuarter + n * 16;
-  const float* const s_row = sums + q * (G + 4) + wave * GW;
+  const GroupSum* const s_row = sums + q * (G + 4) + wave * GW;
   uint32_t kmask = 0x0F0F0F0Fu;
   asm volatile("" : "+s"(kmask));
 
@@ -187,7 +181,9 @@ __global__ __launch_bounds__(64 * kRowsWaves) void qmv_planes_rows_kernel(const 
   };
   auto compute = [&](Batch& b) {
     const char* a = a_row + batch * (GB * kPlaneGroup);
-    const float* sr = s_row + batch * GB;
+    int at = batch * GB;
+    if (SETS == 2) asm volatile("" : "+v"(at));  // (eight groups' sums held across tiles would leave one workgroup per CU)
+    const GroupSum* sr = s_row + at;
 #pragma unroll
     for (int j = 0; j < GB; ++j) {
       i32x4 c;
@@ -209,10 +205,10 @@ __global__ __launch_bounds__(64 * kRowsWaves) void qmv_planes_rows_kernel(const 
       for (int s = 0; s < SETS; ++s) {
         const i32x4 zero = {0, 0, 0, 0};
         const i32x4 d = __builtin_amdgcn_mfma_i32_16x16x64_i8(*reinterpret_cast<const i32x4*>(a + (s * G + j) * kPlaneGroup), c, zero, 0, 0, 0);
-        const float x = sr[s * 4 * (G + 4) + j];
-        float f = fmaf((float)((d[3] << 8) + d[2]), 65536.f * scale_of[s], (float)((d[1] << 8) + d[0]) * scale_of[s]);
-        if (BITS == 8) f = fmaf(128.f, x, f);
-        acc[s] = fmaf(bi, x, fmaf(sc, f, acc[s]));
+        const GroupSum x = sr[s * 4 * (G + 4) + j];
+        float f = __builtin_ldexpf(fmaf((float)((d[3] << 8) + d[2]), 65536.f, (float)((d[1] << 8) + d[0])), x.unit);
+        if (BITS == 8) f = fmaf(128.f, x.sum, f);
+        acc[s] = fmaf(bi, x.sum, fmaf(sc, f, acc[s]));
       }
     }
     if (++batch == ITERS) {  // the tile's sums of this wave

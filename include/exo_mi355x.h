@@ -54,6 +54,10 @@ int exo_embed_dequant(const int32_t* ids, const uint32_t* w, const uint16_t* sca
 
 /* K1: mx.quantized_matmul(x, w, scales, biases, transpose=True) for M <= 16 rows of
  * x (decode): y[M,N] = x[M,K] @ dq(w)[N,K]^T, float32 accumulation, bf16 out.
+ * Inside a group of 64 an element of x counts with an error of up to 2^-17 of the group's largest (sums in
+ * float32 of products with 128 + code; 2^-30 and exact sums where whole numbers stand for them); groups do not
+ * affect one another but through the float32 sum of their results.  An element that is infinite or not a number
+ * makes its row's results ones that are not numbers.  All of the GEMV entry points below are alike in this.
  * Optional fused epilogue: if `residual` is non-null, y = bf16(residual + bf16(acc))
  * (the `h + r` of a transformer block).  (.typings/mlx/core/__init__.pyi:4198-4234,
  * reached through nn.QuantizedLinear.__call__ .typings/mlx/nn/layers/quantized.pyi:87-118) */

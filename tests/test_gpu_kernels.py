@@ -164,6 +164,11 @@ def test_qmv_16x16x32_kernel_shapes(device, N, K, M):
                      what=f"w16 pair {M}x{N}x{K}")
 
 
+def most_of_group(xa):
+    """The largest of each element's quantisation group."""
+    return xa.view(xa.shape[0], -1, 64).amax(2).repeat_interleave(64, 1)
+
+
 @pytest.mark.parametrize("bits,N,K,pair", [
     (4, 4099, 2048, False), (4, 16389, 2048, False), (4, 2050, 4096, False), (4, 1371, 6144, False), (4, 1030, 8192, False),
     (8, 2049, 2048, False), (8, 8195, 2048, False), (8, 1025, 4096, False), (8, 687, 6144, False), (8, 521, 8192, False),
@@ -180,14 +185,14 @@ def test_qmv_planes(device, bits, N, K, pair):
         return ops.QuantizedWeight(w, s, b, bits)
 
     def product(x, q):
-        """In float64, and how far the kernel may be off: whole-number sums are exact but for an element's last bits, 2^-28 of the
-        largest; a group's sum is rounded three times and K / 64 of them are added; the rounding to bf16."""
+        """In float64, and how far the kernel may be off: whole-number sums are exact but for an element's last bits, 2^-30 of the
+        largest of its group; a group's sum is rounded three times and K / 64 of them are added; the rounding to bf16."""
         s, b = q.scales.double()[..., None], q.biases.double()[..., None]
         codes = ops.unpack_codes(q.weight, bits).double().view(N, -1, 64)
         w = (codes * s + b).view(N, K)
         size = ((codes + 128 * (bits == 8)) * s.abs() + b.abs()).view(N, K)
         y, xa = x.double() @ w.T, x.double().abs()
-        return y, 2.0**-8 * y.abs() + (4 + K // 64) * 2.0**-24 * ((xa + 2.0**-8 * xa.max()) @ size.T)
+        return y, 2.0**-8 * y.abs() + ((4 + K // 64) * 2.0**-24 * xa + 2.0**-30 * most_of_group(xa)) @ size.T
 
     q = rows()
     up = rows() if pair else None
@@ -251,12 +256,12 @@ def test_qmv_planes_rows(device, bits, M, N, K, pair, norm):
         return ops.QuantizedWeight(w, s, b, bits)
 
     def product(x, q):
-        """As above; the largest element is that of a row (of half of one: no more)."""
+        """As above."""
         s, b = q.scales.double()[..., None], q.biases.double()[..., None]
         codes = ops.unpack_codes(q.weight, bits).double().view(N, -1, 64)
         y, xa = x.double() @ (codes * s + b).view(N, K).T, x.double().abs()
         size = ((codes + 128 * (bits == 8)) * s.abs() + b.abs()).view(N, K)
-        return y, 2.0**-8 * y.abs() + (4 + K // 64) * 2.0**-24 * ((xa + 2.0**-8 * xa.amax(1, keepdim=True)) @ size.T)
+        return y, 2.0**-8 * y.abs() + ((4 + K // 64) * 2.0**-24 * xa + 2.0**-30 * most_of_group(xa)) @ size.T
 
     q, up = rows(), rows() if pair else None
     nw = (torch.randn(K, device=device, generator=g) * 0.1 + 1).bfloat16()
@@ -288,6 +293,38 @@ def test_qmv_planes_rows(device, bits, M, N, K, pair, norm):
     bad[M - 1, K - 1] = float("nan")
     other = run(bad)
     assert bool(other[M - 1].isnan().all()) and torch.equal(other[: M - 1], got[: M - 1])
+
+
+@pytest.mark.parametrize("bits,M,N,K,down", [(4, 1, 8600, 2048, 0), (4, 1, 1960, 8192, 0), (8, 1, 4300, 2048, 0), (8, 1, 1400, 6144, 0), (8, 3, 1600, 2048, 0),
+                                             (8, 8, 4100, 4096, 0), (4, 3, 28700, 8192, 0), (4, 1, 77, 1536, 8), (8, 2, 50, 768, 2)])
+@pytest.mark.parametrize("far", [2.0**40, 2.0**-90])
+def test_qmv_planes_of_far_elements(device, bits, M, N, K, down, far):
+    """An element far larger than all others that meets zero weights, and elements far smaller than that one's type could hold beside
+    it: the other groups' products are what they are without it."""
+    g = torch.Generator(device=device).manual_seed(N + K)
+    w = torch.randint(-2**31, 2**31 - 1, (N, K * bits // 32), dtype=torch.int32, device=device, generator=g)
+    s, b = (torch.randn(N, K // 64, device=device, generator=g).bfloat16() * f for f in (0.02, 0.1))
+    s[:, 3], b[:, 3] = 0, 0
+    x = torch.randn(M, K, device=device, generator=g) * min(far, 1)
+    x[:, 3 * 64 + 5] = max(far, 1)
+    x = x.bfloat16()
+    codes = ops.unpack_codes(w, bits).double().view(N, -1, 64)
+    others = x.double()
+    others[:, 3 * 64 : 4 * 64] = 0
+    y = others @ (codes * s.double()[..., None] + b.double()[..., None]).view(N, K).T
+    size = ((codes + 128 * (bits == 8)) * s.double().abs()[..., None] + b.double().abs()[..., None]).view(N, K)
+    # (rounding to bf16; a group's sum is rounded three times, and K / 64 of them are added; elements to 2^-30 of their group's largest)
+    slack = 2.0**-8 * y.abs() + ((4 + K // 64) * 2.0**-24 * others.abs() + 2.0**-30 * most_of_group(others.abs())) @ size.T
+    if down:  # every slot the same row of x and expert, all but the first with no weight
+        one = lambda t: t[None].contiguous()  # noqa: E731
+        scores = torch.zeros(M, down, dtype=torch.bfloat16, device=device)
+        scores[:, 0] = 1
+        got = ops.gather_qmv_combine(x[:, None].repeat(1, down, 1), ops.QuantizedWeight(one(w), one(s), one(b), bits), torch.zeros(M, down, dtype=torch.int32, device=device),
+                                     scores, scratch=torch.empty(M, down, N, dtype=torch.bfloat16, device=device))
+    else:
+        got = ops.quantized_matmul(x, ops.QuantizedWeight(w, s, b, bits))
+    assert "planes" in native.last_variant(), native.last_variant()
+    assert bool(((got.double() - y).abs() <= slack).all()), float(((got.double() - y).abs() - slack).max())
 
 
 @pytest.mark.parametrize("bits,E,N,K,T,topk", [(4, 16, 5, 2048, 1, 8), (4, 8, 772, 2048, 5, 2), (8, 8, 9, 4096, 3, 4), (4, 4, 130, 8192, 2, 3), (8, 4, 66, 6144, 2, 2)])
