@@ -48,7 +48,52 @@ class LayerKV:
         return self._owner._last_trim
 
 
-class ShardKVCache(list):
+class HostWrites:
+    """What the host changes in a cache (positions, page numbers) reaches the device in launches on the stream that is current, and
+    the call returns before they have run.  Whatever changes the cache next and every model's forward call ``order`` first,
+    which on another stream waits for the last change and all that was in front of it, so ``trim``, ``reserve`` and ``reset`` on
+    one stream and a step on another need no event between them.  Other readers of ``pos`` or of a page table, and
+    steps that run side by side, are ordered by their callers, as on any tensor."""
+
+    pos: torch.Tensor
+    _change: torch.cuda.Event | None = None  # behind the last change (None: on the default stream, which outlives it)
+    _seen: set[int] | None = None            # streams that are behind it (None: no change yet)
+
+    def order(self) -> None:
+        if self._seen is None:
+            return
+        from . import ops
+        device = self.pos.device.index
+        stream = ops.stream_of(device)
+        if stream in self._seen or torch.cuda.is_current_stream_capturing():
+            return
+        if self._change is None:
+            torch.cuda.current_stream(device).wait_stream(torch.cuda.default_stream(device))
+        else:
+            torch.cuda.current_stream(device).wait_event(self._change)
+        self._seen.add(stream)
+
+    def _changed(self) -> None:
+        if not self.pos.is_cuda:
+            return
+        from . import ops
+        device = self.pos.device.index
+        stream = ops.stream_of(device)
+        self._change = None
+        if stream:
+            self._change = torch.cuda.Event()
+            self._change.record(torch.cuda.current_stream(device))
+        self._seen = {stream}
+
+    def sync_pos(self) -> None:
+        """Push the host offsets to the device copy."""
+        from . import ops
+        self.order()
+        ops.put_ints(self.pos, self.offsets)
+        self._changed()
+
+
+class ShardKVCache(HostWrites, list):
     """list[LayerKV] plus the shared storage."""
 
     def __init__(self, n_layers: int, batch: int, n_kv_heads: int, head_dim: int,
@@ -74,11 +119,6 @@ class ShardKVCache(list):
     def advance_host(self, t: int, rows=None) -> None:
         for r in (range(self.batch) if rows is None else rows):
             self.offsets[r] += t
-
-    def sync_pos(self) -> None:
-        """Push the host offsets to the device copy."""
-        from . import ops
-        ops.put_ints(self.pos, self.offsets)
 
     def trim(self, n: int, rows=None) -> int:
         rows = range(self.batch) if rows is None else rows

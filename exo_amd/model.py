@@ -188,6 +188,7 @@ class DecoderShard:
         rsl = slice(row0, row0 + B)
         if row0 < 0 or row0 + B > cache.batch:
             raise ValueError(f"rows [{row0}, {row0 + B}) outside the cache's {cache.batch} rows")
+        cache.order()
         cache.reserve(range(row0, row0 + B), 1)
         if sampler is not None and not self.is_last:
             raise ValueError("sampling needs the shard that holds the lm_head")
@@ -419,6 +420,7 @@ class ShardModel(DecoderShard):
         r0 = rows.start if rows is not None else 0
         if max(cache.offsets[r0 : r0 + B]) + T > cache.max_seq:
             raise ValueError(f"KV cache overflow: {max(cache.offsets[r0:r0 + B])}+{T} > {cache.max_seq}")
+        cache.order()
         bf = self._buffers(B, T)
         if self.is_first:
             bf.tokens.copy_(tokens.reshape(-1).to(torch.int32))

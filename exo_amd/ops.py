@@ -37,9 +37,14 @@ def _stream() -> int:
     raw getter (a fraction of a microsecond) is used where this torch build has it;
     ``torch.cuda.current_stream()`` builds a Stream object and costs about 8 us, most of the
     host time of a launch from Python."""
+    return stream_of(torch.cuda.current_device())
+
+
+def stream_of(device: int) -> int:
+    """The same of a device."""
     if _raw_stream is not None:
-        return _raw_stream(torch.cuda.current_device())
-    return torch.cuda.current_stream().cuda_stream
+        return _raw_stream(device)
+    return torch.cuda.current_stream(device).cuda_stream
 
 
 PUT_INTS_MAX = 4 * 960  # four launches; a longer list goes as a copy

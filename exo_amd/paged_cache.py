@@ -21,7 +21,7 @@ from __future__ import annotations
 import torch
 
 from . import ops
-from .cache import LayerKV
+from .cache import HostWrites, LayerKV
 from .state_pool import StatePool, StateShape
 
 PAGE = 64
@@ -70,7 +70,7 @@ class PageTable:
         self.table[[a, b]] = self.table[[b, a]]
 
 
-class PagedKVCache(list):
+class PagedKVCache(HostWrites, list):
     """list[LayerKV] (one per layer with keys of its own and per recurrent state) plus the pools."""
 
     def __init__(self, layers: list[tuple[int, int, int]], rows: int, max_seq: int, device, dtype=torch.bfloat16,
@@ -133,10 +133,16 @@ class PagedKVCache(list):
             need.append(self._main.missing(r, self.offsets[r] + n))
         if sum(need) > len(self._free):
             raise PoolExhausted(f"{sum(need)} pages of {PAGE} tokens wanted, {len(self._free)} free")
+        self.order()
+        taken = sum(need)
         for (r, n), k in zip(wants, need):
             self._main.take(r, k)
             for p, t in self.means.items():
-                t.take(r, t.missing(r, self._whole(r, n, p)))
+                k = t.missing(r, self._whole(r, n, p))
+                t.take(r, k)
+                taken += k
+        if taken:
+            self._changed()
 
     def _whole(self, row: int, n: int, block: int) -> int:
         """Positions in whole blocks after ``n`` more tokens."""
@@ -151,9 +157,6 @@ class PagedKVCache(list):
     def advance_host(self, t: int, rows=None) -> None:
         for r in (range(self.batch) if rows is None else rows):
             self.offsets[r] += t
-
-    def sync_pos(self) -> None:
-        ops.put_ints(self.pos, self.offsets)
 
     def trim(self, n: int, rows=None) -> int:
         rows = range(self.batch) if rows is None else rows
@@ -230,7 +233,10 @@ class PagedKVCache(list):
         lo, hi, t = start // p, end // p, self.means[self.blocks[layer]]
         if hi <= lo:
             return
-        t.take(row, t.missing(row, hi * p))
+        if missing := t.missing(row, hi * p):
+            self.order()
+            t.take(row, missing)
+            self._changed()
         k, v = (x.float().view(hi - lo, p, *x.shape[1:]).mean(1) for x in self.read_nhd(layer, row, lo * p, (hi - lo) * p))
         at = torch.arange(lo, hi, device=self.pos.device)
         page = torch.tensor(t.pages[row], dtype=torch.int64, device=self.pos.device)[at // PAGE]

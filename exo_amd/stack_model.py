@@ -451,7 +451,7 @@ class StackModel(DecoderShard):
         """One batch: ``entries`` are (cache row, its next tokens, places among them whose logits are
         asked for), each row at most once.  Appends the tokens to the rows' sequences and returns
         the logits [wanted, V] in entry order (None if nothing is wanted).  The result is valid until
-        the next step."""
+        the next step, and on the current stream, as any tensor's contents: the call returns before the launches have run."""
         if not (self.is_first and self.is_last):
             raise ValueError("step() needs a shard that holds the whole model")
         if len({e[0] for e in entries}) != len(entries) or any(not e[1] for e in entries):
@@ -472,6 +472,7 @@ class StackModel(DecoderShard):
         n = sum(c for _, c in counts)
         if n == 0:
             return None
+        cache.order()
         cache.reserve_each(counts)
         bf = self._buffers(1, max(n, 2))
         if tokens is not None:

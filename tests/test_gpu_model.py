@@ -848,3 +848,48 @@ def test_generate_with_persistent_state_equals_fresh_state(ckpt, device):
         it.close()
     with pytest.raises(ValueError):
         list(generate(gm, None, reqs[0][0], list(range(1, 128)), state=st))
+
+
+def _busy(device):
+    """A stream with some tens of milliseconds of work in front of whatever comes next."""
+    a, s = torch.randn(4096, 4096, device=device), torch.cuda.Stream()
+    torch.mm(a, a)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s):
+        for _ in range(40):
+            torch.mm(a, a)
+    return s
+
+
+def test_trim_and_steps_on_streams_of_their_own(ckpt, device):
+    """A cache cut on one stream and used on another without an event between them: the forward, the captured step and a further
+    cut find the positions that were left, whichever stream each runs on."""
+    cfg, gm = ckpt["cfg"], ckpt["model"]
+    toks = torch.from_numpy(rng(21).integers(0, cfg.vocab_size, size=(1, 24)).astype(np.int32))
+    want_cache, cache = gm.make_cache(1, 64), gm.make_cache(1, 64)
+    gm(toks[:, :12], want_cache)
+    want = gm(toks[:, 12:20], want_cache).clone()
+    gm._buffers(1, 1).tokens.copy_(toks[0, 20:21])
+    want_step = gm.decode_step(want_cache, 1).logits.clone()
+    gm(toks[:, :12], cache)
+    gm(toks[:, 12:], cache)
+    gm.decode_step(cache, 1)  # (its capture)
+    torch.cuda.synchronize()
+    first = _busy(device)
+    with torch.cuda.stream(first):
+        cache.trim(10)
+    cache.trim(3)  # 12 left
+    got = gm(toks[:, 12:20], cache)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want) and cache.pos.tolist() == cache.offsets == [20]
+    gm(toks[:, :2], cache)
+    gm._buffers(1, 1).tokens.copy_(toks[0, 20:21])
+    torch.cuda.synchronize()
+    second = _busy(device)
+    with torch.cuda.stream(second):
+        cache.trim(2)
+    third = torch.cuda.Stream()
+    with torch.cuda.stream(third):
+        got = gm.decode_step(cache, 1).logits
+    torch.cuda.synchronize()
+    assert torch.equal(got, want_step) and cache.pos.tolist() == cache.offsets == [21]

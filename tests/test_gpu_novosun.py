@@ -584,3 +584,31 @@ def test_trace_program(built, tmp_path, dtype):
     want = np.stack([built.want["b"][99], built.want["b"][3], built.want["d"][1], built.want["d"][22],
                      built.want["b"][102], built.want["b"][101], built.want["d"][22]])
     assert rel_rms(got, want).max() < LIMIT[dtype]
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_pages_change_hands_on_streams_of_their_own(built, dtype):
+    """Rows given back on one stream, pages taken on a second and stepped on a third, no event between them."""
+    m, a, c = built.models[dtype], built.toks["a"], built.toks["c"]
+    fresh = m.make_cache(2, 512)
+    want = [m.step(fresh, [(0, c[:40], [39]), (1, a[:70], [69])]).clone(), m.step(fresh, [(0, c[40:41], [0]), (1, a[70:71], [0])]).clone()]
+    cache = m.make_cache(2, 512)
+    m.step(cache, [(0, a[:200], []), (1, c[:30], [])])
+    torch.cuda.synchronize()
+    x, busy = torch.randn(4096, 4096, device="cuda"), torch.cuda.Stream()
+    torch.mm(x, x)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(busy):
+        for _ in range(40):
+            torch.mm(x, x)
+        cache.reset()
+    with torch.cuda.stream(torch.cuda.Stream()):
+        cache.reserve([1], 70)
+    third = torch.cuda.Stream()
+    with torch.cuda.stream(third):
+        got = [m.step(cache, [(0, c[:40], [39]), (1, a[:70], [69])]).clone()]
+    got.append(m.step(cache, [(0, c[40:41], [0]), (1, a[70:71], [0])]))
+    torch.cuda.synchronize()
+    for g, w in zip(got, want):
+        assert torch.equal(g, w)
+    assert cache.pos.tolist() == cache.offsets == [41, 71]
