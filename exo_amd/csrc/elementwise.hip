@@ -2,6 +2,7 @@
 // SwiGLU, MoE routing/combination, greedy sampling reductions.
 #include "../../include/exo_mi355x.h"
 #include "common.h"
+#include "dense.h"
 #include "route.h"
 #include <cstring>
 
@@ -33,10 +34,9 @@ __device__ __forceinline__ float block_sum_256(float v, float* sh) {
   return r;
 }
 
-// Row, residual and weights are requested together, without a branch (past the row: its first elements, as zeros): behind branches they were
-// up to nine memory latencies in a chain.  Without | with a residual, us: 61 rows of 2048 3.0 | 3.2 -> 2.8 | 2.9, of 4096 3.4 | 3.7 -> 3.1 | 3.3, of 8192 4.0 | 4.7 ->
-// 3.5 | 3.9; 4096 rows of 2048 6.9 | 12.4 -> 6.4 | 11.4; 1023 of 4096 with a residual 6.2 -> 6.4.
-template <int CHUNKS>
+// TOGETHER: row, residual and weights are requested together, without a branch (past the row: nothing, as zeros); behind branches they are
+// up to nine memory latencies in a chain.  Otherwise piece by piece, weights behind the sum (norm_together: where that is the faster one).
+template <int CHUNKS, bool TOGETHER>
 __global__ __launch_bounds__(kNormThreads) void add_rmsnorm_kernel(
     const bf16_t* __restrict__ x, const bf16_t* __restrict__ res,
     const bf16_t* __restrict__ w, bf16_t* __restrict__ h_out, bf16_t* __restrict__ n_out,
@@ -44,46 +44,76 @@ __global__ __launch_bounds__(kNormThreads) void add_rmsnorm_kernel(
   __shared__ float sh[4];
   const size_t row = (size_t)blockIdx.x * H;
   uint4 a[CHUNKS], r[CHUNKS], wv[CHUNKS];
+  if (TOGETHER) {
+    const uint32_t bytes = (uint32_t)H * 2;
+    const __amdgpu_buffer_rsrc_t rx = buf_of(x + row, bytes), rr = buf_of(res ? res + row : x, res ? bytes : 0), rw = buf_of(w, bytes);
 #pragma unroll
-  for (int i = 0; i < CHUNKS; ++i) {
-    const int e0 = (threadIdx.x + i * kNormThreads) * 8, at = e0 < H ? e0 : 0;
-    a[i] = *reinterpret_cast<const uint4*>(x + row + at);
-    r[i] = *reinterpret_cast<const uint4*>((res ? res : x) + row + at);
-  }
+    for (int i = 0; i < CHUNKS; ++i) {
+      const uint32_t at = (threadIdx.x + i * kNormThreads) * 16;
+      a[i] = buf_load16(rx, at, 0);
+      r[i] = buf_load16(rr, at, 0);
+    }
 #pragma unroll
-  for (int i = 0; i < CHUNKS; ++i) {
-    const int e0 = (threadIdx.x + i * kNormThreads) * 8;
-    wv[i] = *reinterpret_cast<const uint4*>(w + (e0 < H ? e0 : 0));
+    for (int i = 0; i < CHUNKS; ++i) wv[i] = buf_load16(rw, (threadIdx.x + i * kNormThreads) * 16, 0);
+    __builtin_amdgcn_sched_barrier(0);
   }
-  __builtin_amdgcn_sched_barrier(0);
   float v[CHUNKS][8];
   float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < CHUNKS; ++i) {
     const int e0 = (threadIdx.x + i * kNormThreads) * 8;
-    const uint32_t a4[4] = {a[i].x, a[i].y, a[i].z, a[i].w}, r4[4] = {r[i].x, r[i].y, r[i].z, r[i].w};
-    uint32_t o4[4];
+    if (TOGETHER || e0 < H) {
+      if (!TOGETHER) {
+        a[i] = *reinterpret_cast<const uint4*>(x + row + e0);
+        if (res) r[i] = *reinterpret_cast<const uint4*>(res + row + e0);
+      }
+      const uint32_t a4[4] = {a[i].x, a[i].y, a[i].z, a[i].w}, r4[4] = {r[i].x, r[i].y, r[i].z, r[i].w};
+      uint32_t o4[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      o4[e] = res ? pack_bf2(bf_lo(a4[e]) + bf_lo(r4[e]), bf_hi(a4[e]) + bf_hi(r4[e])) : a4[e];
-      v[i][2 * e] = e0 < H ? bf_lo(o4[e]) : 0.f;
-      v[i][2 * e + 1] = e0 < H ? bf_hi(o4[e]) : 0.f;
+      for (int e = 0; e < 4; ++e) {
+        o4[e] = res ? pack_bf2(bf_lo(a4[e]) + bf_lo(r4[e]), bf_hi(a4[e]) + bf_hi(r4[e])) : a4[e];
+        v[i][2 * e] = bf_lo(o4[e]);
+        v[i][2 * e + 1] = bf_hi(o4[e]);
+      }
+      if (h_out && e0 < H) *reinterpret_cast<uint4*>(h_out + row + e0) = make_uint4(o4[0], o4[1], o4[2], o4[3]);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) ss = fmaf(v[i][e], v[i][e], ss);
     }
-    if (h_out && e0 < H) *reinterpret_cast<uint4*>(h_out + row + e0) = make_uint4(o4[0], o4[1], o4[2], o4[3]);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) ss = fmaf(v[i][e], v[i][e], ss);
   }
   ss = block_sum_256(ss, sh);
   const float inv = rsqrtf(ss / (float)H + eps);
 #pragma unroll
   for (int i = 0; i < CHUNKS; ++i) {
     const int e0 = (threadIdx.x + i * kNormThreads) * 8;
-    const uint32_t w4[4] = {wv[i].x, wv[i].y, wv[i].z, wv[i].w};
-    uint32_t o4[4];
+    if (e0 < H) {
+      if (!TOGETHER) wv[i] = *reinterpret_cast<const uint4*>(w + e0);
+      const uint32_t w4[4] = {wv[i].x, wv[i].y, wv[i].z, wv[i].w};
+      uint32_t o4[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) o4[e] = pack_bf2(v[i][2 * e] * inv * bf_lo(w4[e]), v[i][2 * e + 1] * inv * bf_hi(w4[e]));
-    if (e0 < H) *reinterpret_cast<uint4*>(n_out + row + e0) = make_uint4(o4[0], o4[1], o4[2], o4[3]);
+      for (int e = 0; e < 4; ++e) o4[e] = pack_bf2(v[i][2 * e] * inv * bf_lo(w4[e]), v[i][2 * e + 1] * inv * bf_hi(w4[e]));
+      *reinterpret_cast<uint4*>(n_out + row + e0) = make_uint4(o4[0], o4[1], o4[2], o4[3]);
+    }
   }
+}
+// Few rows of two pieces and more wait for their latencies; between 800 and 2000 they keep the memory busier when the requests
+// come one after another; beyond, those without a residual or of two or three pieces are together again the faster.  One piece is one chain either way; with a residual and more
+// than the L2s hold, together (3000 of 2048 8.9 and 9.3).
+// Without | with a residual, us, together and piece by piece: 61 rows of 4096 3.1 | 3.3 and 3.1 | 3.6, of 8192 3.5 | 3.9 and 3.9 | 4.9; 1023 of 3072
+// 4.3 | 5.7 and 4.0 | 5.3, of 4096 4.6 | 6.4 and 4.5 | 6.1, of 8192 6.7 | 11.3 and 6.7 | 12.2; 3000 of 4096 8.7 | 15.8 and 9.6 | 16.4; 4096 of 1024 5.1 | 7.2 and
+// 4.7 | 6.7.
+bool norm_together(int rows, int H, bool residual) {
+  const int chunks = exo_ceil_div(H, kNormThreads * 8);
+  if (chunks == 1) return residual && (int64_t)rows * H >= 5000000;
+  if (rows < 800) return true;
+  if (chunks == 2) return rows >= 2100;
+  return residual ? chunks == 3 || rows < 1800 : rows >= 1600;
+}
+template <bool TOGETHER>
+void launch_add_rmsnorm(const bf16_t* x, const bf16_t* res, const bf16_t* w, bf16_t* h_out, bf16_t* n_out, int rows, int H, float eps, hipStream_t st) {
+  const int chunks = exo_ceil_div(H, kNormThreads * 8);
+  const auto fn = chunks <= 1 ? add_rmsnorm_kernel<1, TOGETHER> : chunks <= 2 ? add_rmsnorm_kernel<2, TOGETHER> :
+                  chunks <= 3 ? add_rmsnorm_kernel<3, TOGETHER> : add_rmsnorm_kernel<kNormMaxChunks, TOGETHER>;
+  fn<<<dim3(rows), kNormThreads, 0, st>>>(x, res, w, h_out, n_out, H, eps);
 }
 
 // ------------------------------------------------------ RoPE + KV append (+ head norm)
@@ -476,9 +506,8 @@ extern "C" int exo_add_rmsnorm(const uint16_t* x, const uint16_t* residual,
               "exo_add_rmsnorm: H=%d must be a multiple of 8 and <= %d", H,
               kNormThreads * 8 * kNormMaxChunks);
   if (rows == 0) return EXO_OK;
-  const int chunks = exo_ceil_div(H, kNormThreads * 8);
-  (chunks <= 1 ? add_rmsnorm_kernel<1> : chunks <= 2 ? add_rmsnorm_kernel<2> : add_rmsnorm_kernel<kNormMaxChunks>)<<<dim3(rows), kNormThreads, 0, (hipStream_t)stream>>>(
-      x, residual, weight, h_out, n_out, H, eps);
+  const auto launch = norm_together(rows, H, residual != nullptr) ? launch_add_rmsnorm<true> : launch_add_rmsnorm<false>;
+  launch(x, residual, weight, h_out, n_out, rows, H, eps, (hipStream_t)stream);
   EXO_CHECK_LAUNCH("exo_add_rmsnorm");
   return EXO_OK;
 }

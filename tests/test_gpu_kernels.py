@@ -776,10 +776,11 @@ def test_rope_kv_append(device, D, Hq, Hkv, qk_norm):
             assert torch.equal(a.view(torch.int16), b_.view(torch.int16))
 
 
-@pytest.mark.parametrize("rows,H", [(1, 8), (3, 2048), (2, 2056), (5, 4096), (2, 4104), (61, 8192)])
+@pytest.mark.parametrize("rows,H", [(1, 8), (3, 2048), (2, 2056), (5, 4096), (2, 4104), (3, 6144), (2, 6152), (61, 8192),
+                                    (800, 2056), (1023, 4096), (2100, 2064), (800, 4104), (1600, 6144), (1800, 8192), (2442, 2048)])
 @pytest.mark.parametrize("residual", [False, True])
 def test_add_rms_norm_chunks(device, rows, H, residual):
-    """One, two and four pieces of a row per thread, full and not; the sum in place of the residual."""
+    """One to four pieces of a row per thread, full and not, requested together and one after another; the sum in place of the residual."""
     g = torch.Generator(device=device).manual_seed(H)
     x, r = (torch.randn(rows, H, device=device, generator=g).bfloat16() for _ in range(2))
     w = (1 + 0.1 * torch.randn(H, device=device, generator=g)).bfloat16()
