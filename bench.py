@@ -111,11 +111,8 @@ def measure_kernels(model, torch, reps: int = 20):
     y_h = torch.empty(1, H, **bf)
     y_i = torch.empty(1, I, **bf)
     y_v = torch.empty(1, c.vocab_size, **bf)
-    def kernel_name(nmat, K):  # of the launch just made
-        if native.last_variant().endswith("planes"):  # template arguments <bits, matrices, K / 2048, self-routing>
-            return "qmv_planes_kernel<%d,%d,%d,false>" % (c.bits, nmat, K // 2048)
-        # template arguments <bits, rows of x, matrices, 1 KiB units per row, self-routing>
-        return "qmv_rows_kernel<%d,1,%d,%d,false>" % (c.bits, nmat, K * c.bits // 8 // 1024)
+    def kernel_name():  # of the launch just made, from the instance that it reports
+        return native.last_variant().split()[0].replace("<", "_kernel<", 1)
 
     nw, eps = torch.ones(H, **bf), c.rms_norm_eps
 
@@ -135,20 +132,19 @@ def measure_kernels(model, torch, reps: int = 20):
 
     groups = {
         "norm_gate_up_swiglu": (lambda L: ops.qmv_swiglu(xh, L.gate, L.up, out=y_i, norm_weight=nw, eps=eps),
-                                2 * qbytes(I, H, c.bits) + 2 * (2 * H + I), (2, H)),
+                                2 * qbytes(I, H, c.bits) + 2 * (2 * H + I)),
         "down_residual": (lambda L: ops.quantized_matmul(xi, L.down, residual=y_h, out=y_h),
-                          qbytes(H, I, c.bits) + 2 * (I + 2 * H), (1, I)),
+                          qbytes(H, I, c.bits) + 2 * (I + 2 * H)),
         "norm_qkv": (lambda L: ops.quantized_matmul(xh, L.qkv, out=y_qkv, norm_weight=nw, eps=eps),
-                     qbytes((Hq + 2 * Hkv) * D, H, c.bits) + 2 * (2 * H + (Hq + 2 * Hkv) * D),
-                     (1, H)),
+                     qbytes((Hq + 2 * Hkv) * D, H, c.bits) + 2 * (2 * H + (Hq + 2 * Hkv) * D)),
         "o_residual": (lambda L: ops.quantized_matmul(xa, L.o, residual=y_h, out=y_h),
-                       qbytes(H, Hq * D, c.bits) + 2 * (Hq * D + 2 * H), (1, Hq * D)),
+                       qbytes(H, Hq * D, c.bits) + 2 * (Hq * D + 2 * H)),
     }
     out = []
-    for name, (fn, nbytes, of) in groups.items():
+    for name, (fn, nbytes) in groups.items():
         for L in model.layers:  # warm-up (also sets kernel attributes outside capture)
             fn(L)
-        kname = kernel_name(*of)
+        kname = kernel_name()
         torch.cuda.synchronize()
         g = torch.cuda.CUDAGraph()
         with capture_graph(g):
@@ -179,7 +175,7 @@ def measure_kernels(model, torch, reps: int = 20):
     us = timed_rounds(g, len(heads))
     del heads
     nbytes = qbytes(c.vocab_size, H, c.bits) + 2 * (2 * H + c.vocab_size)
-    out.append(dict(name="norm_lm_head", kernel=kernel_name(1, H), launches_per_token=1,
+    out.append(dict(name="norm_lm_head", kernel=kernel_name(), launches_per_token=1,
                     bytes_per_launch=nbytes, avg_us=us, GBps=nbytes / us * 1e-3))
     return out
 

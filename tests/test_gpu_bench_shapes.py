@@ -280,40 +280,74 @@ def test_moe_stack_at_real_shape(device, name, layers, T):
 # ------------------------------------------------------------------ which instance runs
 
 
+def _check_product(got, x, q, up=None, norm_weight=None, residual=None):
+    """A launch's result against the product in float64 of the packed weights: the rounding to bf16, K / 64 + 4 float32 roundings of
+    what is added (of products with 128 + code at the most), and behind a norm an element's rounding to bf16 the other way here and there
+    (its sum of squares is in another order): some K 2^-9 of a product each, independent."""
+    xn = x if norm_weight is None else ops.rms_norm(x, norm_weight, 1e-5)
+    K, few = x.shape[1], 8192
+
+    def product(q):
+        y, slack = [], []
+        for a in range(0, q.weight.shape[0], few):
+            s, b = (t[a : a + few].double()[..., None] for t in (q.scales, q.biases))
+            codes = ops.unpack_codes(q.weight[a : a + few].contiguous(), q.bits).double().view(s.shape[0], -1, 64)
+            y.append(xn.double() @ (codes * s + b).view(-1, K).T)
+            slack.append((4 + K // 64) * 2.0**-24 * (xn.double().abs() @ ((codes + 128) * s.abs() + b.abs()).view(-1, K).T))
+        y = torch.cat(y, 1)
+        return y, 2.0**-8 * y.abs() + torch.cat(slack, 1) + (0.0 if norm_weight is None else 2.0**-7 * y.pow(2).mean().sqrt())
+
+    y, slack = product(q)
+    if up is not None:
+        yu, slack_u = product(up)
+        unit = y * torch.sigmoid(y)
+        y, slack = unit * yu, (1.1 * slack + 2.0**-8 * unit.abs()) * yu.abs() + unit.abs() * (slack_u + 2.0**-8 * yu.abs()) + 1.1 * slack * slack_u + 2.0**-8 * (unit * yu).abs() + 1e-30
+    if residual is not None:
+        y, slack = y + residual.double(), slack + 2.0**-8 * (y.abs() + residual.double().abs())
+    off = (got.double() - y).abs() - slack
+    assert float(off.max()) <= 0, (native.last_variant(), float(off.max()), int(off.argmax()))
+
+
 def test_decode_launches_reach_their_instances(device):
-    """The launches of the headline decode step report the instance they are tuned as."""
+    """The launches of the headline decode step report the instance they are tuned as, and their results are the product's.  The
+    gate/up pair of one row and of four may go to the integer matrix cores as well."""
     bits, H, I = 4, 4096, 14336
     x = t_bf16(rand_bf16((1, H), seed=1), device)
     nw = t_bf16(affine.bf16_round(rand_bf16((H,), seed=2) * 0.1 + 1.0), device)
     g, u = _packed(I, H, bits, 1, device), _packed(I, H, bits, 2, device)
-    ops.qmv_swiglu(x, g, u, norm_weight=nw, eps=1e-5)
-    assert native.last_variant() == "qmv_rows<4,1,2,2,false> grid=1792x1", native.last_variant()
-    ops.quantized_matmul(x, _packed(6144, H, bits, 3, device), norm_weight=nw, eps=1e-5)
-    assert native.last_variant().startswith("qmv_rows<4,1,1,2,false>"), native.last_variant()
+
+    def launched(*names):
+        assert native.last_variant().startswith(names), native.last_variant()
+
+    def pair(x, *names):
+        got = ops.qmv_swiglu(x, g, u, norm_weight=nw, eps=1e-5)
+        launched(*names)
+        _check_product(got, x, g, up=u, norm_weight=nw)
+
+    def single(x, q, *names, residual=None, norm_weight=None):
+        got = ops.quantized_matmul(x, q, residual=residual, norm_weight=norm_weight, eps=1e-5)
+        launched(*names)
+        _check_product(got, x, q, norm_weight=norm_weight, residual=residual)
+
+    pair(x, "qmv_rows<4,1,2,2,false> grid=1792x1", "qmv_planes<4,2,2,false> ")
+    qkv = _packed(6144, H, bits, 3, device)
+    single(x, qkv, "qmv_planes<4,1,2,false> ", norm_weight=nw)
     xa = t_bf16(rand_bf16((1, H), seed=6), device)
-    ops.quantized_matmul(xa, _packed(H, H, bits, 5, device), residual=x)
-    assert native.last_variant().startswith("qmv_rows<4,1,1,2,false>"), native.last_variant()
-    ops.quantized_matmul(x, _packed(128256, H, bits, 6, device), norm_weight=nw, eps=1e-5)
-    assert native.last_variant().startswith("qmv_rows<4,1,1,2,false>"), native.last_variant()
+    single(xa, _packed(H, H, bits, 5, device), "qmv_rows<4,1,1,2,false> ", residual=x)
+    single(x, _packed(128256, H, bits, 6, device), "qmv_planes<4,1,2,false> ", norm_weight=nw)
     xi = t_bf16(rand_bf16((1, I), seed=3), device)
-    ops.quantized_matmul(xi, _packed(H, I, bits, 4, device))
-    assert native.last_variant().startswith("qmv_rows<4,1,1,7,false>"), native.last_variant()
+    down = _packed(H, I, bits, 4, device)
+    single(xi, down, "qmv_rows<4,1,1,7,false> ")
     x4 = t_bf16(rand_bf16((4, H), seed=4), device)
-    ops.qmv_swiglu(x4, g, u, norm_weight=nw, eps=1e-5)
-    assert native.last_variant().startswith("qmv_quad<4,2,1,4,1>"), native.last_variant()
+    pair(x4, "qmv_quad<4,2,1,4,1>", "qmv_planes_rows<4,2,2,4> ")
     x8 = t_bf16(rand_bf16((8, H), seed=5), device)
-    ops.qmv_swiglu(x8, g, u, norm_weight=nw, eps=1e-5)
-    assert native.last_variant().startswith("qmv_w16<2,2,2,norm,pair8> grid=256 waves=16 blocks=7"), native.last_variant()
+    pair(x8, "qmv_w16<2,2,2,norm,pair8> grid=256 waves=16 blocks=7")
     x16 = t_bf16(rand_bf16((16, H), seed=7), device)
-    ops.qmv_swiglu(x16, g, u, norm_weight=nw, eps=1e-5)
-    assert native.last_variant().startswith("qmv_w16<2,2,2,norm,pair8> grid=256 waves=16 blocks=7"), native.last_variant()
+    pair(x16, "qmv_w16<2,2,2,norm,pair8> grid=256 waves=16 blocks=7")
     # the down projection under 8 rows: K split over four workgroups per group of row blocks
     xi8 = t_bf16(rand_bf16((8, I), seed=8), device)
-    ops.quantized_matmul(xi8, _packed(H, I, bits, 4, device), residual=x8)
-    assert native.last_variant().startswith("qmv_w16<1,2,2,plain,staged> grid=256 waves=14 blocks=4 kparts=4"), \
-        native.last_variant()
-    ops.quantized_matmul(x8, _packed(6144, H, bits, 3, device), norm_weight=nw, eps=1e-5)
-    assert native.last_variant().startswith("qmv_w16<1,2,2,norm,staged>"), native.last_variant()
+    single(xi8, down, "qmv_w16<1,2,2,plain,staged> grid=256 waves=14 blocks=4 kparts=4", residual=x8)
+    single(x8, qkv, "qmv_w16<1,2,2,norm,staged>", norm_weight=nw)
     # decode attention: one sequence of 32 / 8 heads on the scalar kernel, eight on the matrix cores
     D, Hq, Hkv, S = 128, 32, 8, 2304
     inv = torch.from_numpy(O.rope_inv_freq(D, 5e5, None)).to(device)

@@ -221,14 +221,14 @@ def test_qmv_planes(device, bits, N, K, pair):
         else:
             got = ops.quantized_matmul(x, q)
         if norm:
-            assert native.last_variant().endswith(" planes"), native.last_variant()
+            assert native.last_variant().startswith("qmv_planes<"), native.last_variant()
         off = (got.double() - y).abs() - slack
         assert off.max() <= 0, (what, off.max(), off.argmax())
     if bits == 4 and not pair:  # sums that fit the type under scales that leave no room
         big = ops.QuantizedWeight(q.weight, (q.scales.float() * 2.0**110).bfloat16(), (q.biases.float() * 2.0**110).bfloat16(), bits)
         x = normal.bfloat16()
         got = ops.quantized_matmul(x, big, norm_weight=nw, eps=1e-5)
-        assert native.last_variant().endswith(" planes")
+        assert native.last_variant().startswith("qmv_planes<")
         y, slack = product(ops.rms_norm(x, nw, 1e-5), big)
         assert ((got.double() - y).abs() <= slack + 2.0**-7 * y.pow(2).mean().sqrt()).all()
     for bad in (float("inf"), float("nan")):  # reach every output, whichever wave holds them
@@ -343,7 +343,7 @@ def test_qmv_planes_of_experts(device, bits, E, N, K, T, topk):
     nw = (torch.randn(K, device=device, generator=g) * 0.1 + 1).bfloat16()
     idx = torch.stack([torch.randperm(E, generator=torch.Generator().manual_seed(t))[:topk] for t in range(T)]).int().to(device)
     got = ops.gather_qmv_swiglu(x, gate, up, idx, norm_weight=nw, eps=1e-5)
-    assert native.last_variant().endswith(" planes"), native.last_variant()
+    assert native.last_variant().startswith("qmv_planes<"), native.last_variant()
     one = lambda q, e: ops.QuantizedWeight(q.weight[e].contiguous(), q.scales[e].contiguous(), q.biases[e].contiguous(), bits)  # noqa: E731
     for t in range(T):
         for k in range(topk):
