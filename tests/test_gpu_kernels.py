@@ -169,14 +169,18 @@ def most_of_group(xa):
     return xa.view(xa.shape[0], -1, 64).amax(2).repeat_interleave(64, 1)
 
 
-@pytest.mark.parametrize("bits,N,K,pair", [
-    (4, 4099, 2048, False), (4, 16389, 2048, False), (4, 2050, 4096, False), (4, 1371, 6144, False), (4, 1030, 8192, False),
-    (8, 2049, 2048, False), (8, 8195, 2048, False), (8, 1025, 4096, False), (8, 687, 6144, False), (8, 521, 8192, False),
-    (4, 2051, 2048, True), (4, 8193, 2048, True), (4, 689, 6144, True), (4, 514, 8192, True), (8, 1027, 2048, True), (8, 4097, 4096, True), (8, 259, 8192, True),
+@pytest.mark.parametrize("bits,N,K,pair,plain", [
+    (4, 4099, 2048, False, False), (4, 16389, 2048, False, True), (4, 2050, 4096, False, False), (4, 4301, 4096, False, True), (4, 1371, 6144, False, False),
+    (4, 2611, 6144, False, True), (4, 1030, 8192, False, False), (4, 1957, 8192, False, True),
+    (8, 2049, 2048, False, False), (8, 8195, 2048, False, True), (8, 1025, 4096, False, False), (8, 2001, 4096, False, True), (8, 687, 6144, False, False),
+    (8, 1307, 6144, False, True), (8, 521, 8192, False, False), (8, 979, 8192, False, True),
+    (4, 2051, 2048, True, False), (4, 8193, 2048, True, True), (4, 689, 6144, True, False), (4, 1307, 6144, True, True), (4, 514, 8192, True, False), (4, 979, 8192, True, True),
+    (8, 1027, 2048, True, False), (8, 2151, 2048, True, True), (8, 4097, 4096, True, True), (8, 653, 6144, True, True), (8, 259, 8192, True, False), (8, 491, 8192, True, True),
 ])
-def test_qmv_planes(device, bits, N, K, pair):
-    """One row on the integer matrix cores: last tiles of a few rows, one and several tiles per workgroup, every K;
-    elements of one size, a few far larger, sizes spread over many binades, zeros, the smallest and the largest, and scales of 2^104."""
+def test_qmv_planes(device, bits, N, K, pair, plain):
+    """One row on the integer matrix cores: last tiles of a few rows, one and several tiles per workgroup, every K, behind a norm and (launches that
+    are large enough for it) without one, with a residual and without; elements of one size, a few far larger, sizes spread over many
+    binades, zeros, the smallest and the largest whose results the type holds, and scales of 2^104."""
     g = torch.Generator(device=device).manual_seed(N + K)
 
     def rows():
@@ -201,9 +205,13 @@ def test_qmv_planes(device, bits, N, K, pair):
     normal = torch.randn(1, K, device=device, generator=g)
     few, spread = normal.clone(), normal * torch.exp(4 * torch.randn(1, K, device=device, generator=g))
     few[0, ::977] *= 300
-    for what, x in (("normal", normal), ("few", few), ("spread", spread), ("zero", normal * 0), ("small", normal * 2.0**-80), ("large", normal * 2.0**90)):
+    ends = (2.0**-45, 2.0**45) if pair else (2.0**-115, 2.0**110)  # (of a pair the product of two sums)
+    inputs = [("normal", normal, True, True), ("few", few, True, False)]
+    if plain:
+        inputs += [("normal", normal, False, True), ("few", few, False, False), ("spread", spread, False, True), ("zero", normal * 0, False, False),
+                   ("small", normal * ends[0], False, False), ("large", normal * ends[1], False, False)]
+    for what, x, norm, residual in inputs:
         x = x.bfloat16()
-        norm = what in ("normal", "few")
         xn = ops.rms_norm(x, nw, 1e-5) if norm else x  # (its sum of squares is in another order: a rounding of an element may differ)
         kw = dict(norm_weight=nw, eps=1e-5) if norm else {}
         y, slack = product(xn, q)
@@ -212,18 +220,15 @@ def test_qmv_planes(device, bits, N, K, pair):
             got = ops.qmv_swiglu(x, q, up, **kw)
             yu, slack_u = product(xn, up)
             slack_u = slack_u + (2.0**-7 * yu.pow(2).mean().sqrt() if norm else 0.0)
-            if what in ("small", "large"):
-                continue  # (products of two sums out of the type's range)
             y, slack = y * torch.sigmoid(y) * yu, (1.1 * slack + 2.0**-8 * y.abs()) * yu.abs() + y.abs() * (slack_u + 2.0**-8 * yu.abs()) + 1.1 * slack * slack_u + 1e-30
-        elif norm:
+        elif residual:
             got = ops.quantized_matmul(x, q, residual=res, **kw)
             y, slack = y + res.double(), slack + 2.0**-8 * (y.abs() + res.double().abs())
         else:
-            got = ops.quantized_matmul(x, q)
-        if norm:
-            assert native.last_variant().startswith("qmv_planes<"), native.last_variant()
+            got = ops.quantized_matmul(x, q, **kw)
+        assert native.last_variant().startswith("qmv_planes<%d,%d,%d," % (bits, 1 + pair, K // 2048)), native.last_variant()
         off = (got.double() - y).abs() - slack
-        assert off.max() <= 0, (what, off.max(), off.argmax())
+        assert off.max() <= 0, (what, norm, off.max(), off.argmax())
     if bits == 4 and not pair:  # sums that fit the type under scales that leave no room
         big = ops.QuantizedWeight(q.weight, (q.scales.float() * 2.0**110).bfloat16(), (q.biases.float() * 2.0**110).bfloat16(), bits)
         x = normal.bfloat16()
