@@ -65,6 +65,12 @@ __device__ __forceinline__ const char* plane_operand(const char* planes, int lan
   return planes + (mine ? half * (units * (BITS == 4 ? 2 : 1) * kPlaneBlock) + q * 64 + (n & 3) * 16 : 256);
 }
 
+// to the nearest whole number (of halves the larger)
+__device__ __forceinline__ int nearest(float v) {
+  int r;
+  asm("v_cvt_rpi_i32_f32 %0, %1" : "=v"(r) : "v"(v));
+  return r;
+}
 // the largest of eight lanes' runs, as the bits of its absolute value
 __device__ __forceinline__ uint32_t group_most(const uint4& x) {
   typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
@@ -100,8 +106,8 @@ __device__ __forceinline__ void store_planes(const uint4 (&xr)[XS], int runs, Pl
     for (int k = 0; k < 4; ++k) {
       gs += bf_lo(x4[k]) + bf_hi(x4[k]);
       // byte i of X + 0x808080 less 128 (the top one as it is): the signed digits of X
-      d[2 * k] = (uint32_t)(int)__builtin_rintf(__builtin_ldexpf(bf_lo(x4[k]), shift)) + 0x00808080u;
-      d[2 * k + 1] = (uint32_t)(int)__builtin_rintf(__builtin_ldexpf(bf_hi(x4[k]), shift)) + 0x00808080u;
+      d[2 * k] = (uint32_t)nearest(__builtin_ldexpf(bf_lo(x4[k]), shift)) + 0x00808080u;
+      d[2 * k + 1] = (uint32_t)nearest(__builtin_ldexpf(bf_hi(x4[k]), shift)) + 0x00808080u;
     }
     // operand words: the codes of a word's even places, then of its odd ones (8 bits: as they come)
     uint32_t out[4][2];  // [plane][operand word]
