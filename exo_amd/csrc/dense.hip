@@ -947,7 +947,12 @@ void launch_gemv_post(const GemvParams& p, const PostNorm& q, hipStream_t st) {
 // 15.3, 20000 of 4096 72.7 -> 63.6.  The ring takes 72 registers instead of 51, 6 waves per SIMD instead of 8, which costs where x takes
 // longer than the weights' latency: 16 rows 0.89 to 1.03 of the speed, 6 and 8 rows in the many workgroups of 4 waves 0.96 to 1.03 (20000 of 4096 bf16
 // 8 rows 37.3 -> 39.1; 4 rows 0.98 to 1.09), pairs, whose rings hold two matrices, 0.89 to 1.02.
-bool gemv_ring(const GemvParams& p, int waves) { return p.M <= (waves == 4 ? 4 : 8); }
+// A wave whose steps are one batch has nothing to request again and only fewer neighbours: f32 10822 columns of K = 256 under 6 rows 7.5 | 9.4,
+// 11765 of 384 under 7 8.2 | 10.2, 14550 of 448 under 5 9.4 | 10.3, bf16 22185 of 768 under one 9.5 | 9.9 with it.
+bool gemv_ring(const GemvParams& p, const GemvParams* p1, int waves, int elem) {
+  const int steps = std::max(p.ldw, p1 ? p1->ldw : 0) * elem / 64;
+  return p.M <= (waves == 4 ? 4 : 8) && steps > waves * kBatch;
+}
 template <typename T, int NW>
 void launch_gemv_nw(const GemvParams& p, const GemvParams* p1, const PostNorm* q, hipStream_t st) {
   const int tiles = exo_ceil_div(p.N, 16);
@@ -963,7 +968,7 @@ void launch_gemv_nw(const GemvParams& p, const GemvParams* p1, const PostNorm* q
   } else if (p.w2)
     dense_gemv_kernel<T, NW, 0, 0, true, false><<<tiles, 64 * NW, 0, st>>>(p, p, none);
   else {
-    const bool ring = gemv_ring(p, NW);
+    const bool ring = gemv_ring(p, p1, NW, (int)sizeof(T));
     const auto fn = p1 ? (ring ? dense_gemv_kernel<T, NW, 0, 0, false, true, 1, kBatch, true> : dense_gemv_kernel<T, NW, 0, 0, false, true>)
                        : (ring ? dense_gemv_kernel<T, NW, 0, 0, false, false, 1, kBatch, true> : dense_gemv_kernel<T, NW, 0, 0, false, false>);
     fn<<<tiles + (p1 ? exo_ceil_div(p1->N, 16) : 0), 64 * NW, 0, st>>>(p, p1 ? *p1 : p, none);
