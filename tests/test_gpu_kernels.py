@@ -247,7 +247,7 @@ def test_qmv_planes(device, bits, N, K, pair, plain):
 @pytest.mark.parametrize("bits,M,N,K,pair,norm", [
     (8, 3, 1537, 2048, False, False), (8, 2, 4100, 2048, False, True), (8, 8, 36865, 2048, False, True), (8, 5, 1, 2048, True, True), (8, 7, 17, 4096, True, False),
     (8, 6, 4113, 4096, False, True), (8, 4, 2577, 4096, False, False), (8, 3, 9, 6144, True, True), (8, 2, 35, 8192, False, True), (8, 4, 8200, 4096, True, True),
-    (4, 2, 7, 2048, True, False), (4, 3, 2055, 2048, True, True), (4, 4, 4609, 2048, False, True), (4, 2, 33000, 2048, False, True),
+    (4, 3, 7, 2048, True, False), (4, 2, 1031, 2048, True, False), (4, 3, 2055, 2048, True, True), (4, 4, 4609, 2048, False, True), (4, 2, 33000, 2048, False, True),
     (4, 4, 2100, 4096, True, True), (4, 3, 28677, 8192, False, False), (4, 4, 14341, 8192, True, True),
 ])
 def test_qmv_planes_rows(device, bits, M, N, K, pair, norm):
