@@ -200,14 +200,15 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(
 // token beside one piece of the table's row.  What bounds it is the memory (a token of 32 / 8 heads of 128 is 24 KB in and out, 4.8 TB/s of it from 4096
 // tokens on); the kernel above moves 2 bytes a lane and sums a head's squares over the whole wave.  32 / 8 heads of 128, without | with norms, us: 61 tokens
 // 3.5 | 4.4 -> 3.3 | 3.6, 1023 9.5 | 12.5 -> 7.3 | 7.7, 4096 27.3 | 37.8 -> 20.1 | 20.9; of 64, 1023 tokens 8.7 | 11.8 -> 5.5 | 5.7.
+// Few heads leave most of 256 threads without one: as many threads as heads take (8000 tokens of 1 / 1 heads of 64 12.5 -> 5.8 us, of 5 / 1 13.3 -> 6.6).
 constexpr int kRopeHeadsPerThread = 3;
-template <int D>
-__global__ __launch_bounds__(256) void rope_kv_wide_kernel(
+template <int D, int THREADS>
+__global__ __launch_bounds__(THREADS) void rope_kv_wide_kernel(
     const bf16_t* __restrict__ qkv, bf16_t* __restrict__ q_out, bf16_t* __restrict__ kc,
     bf16_t* __restrict__ vc, const int32_t* __restrict__ pos, const float* __restrict__ inv_freq,
     const float2* __restrict__ tab, int tab_rows, const bf16_t* __restrict__ qn,
     const bf16_t* __restrict__ kn, float eps, int T, int Hq, int Hkv, int S_max) {
-  constexpr int LPH = D / 8, GROUPS = 256 / LPH, U = kRopeHeadsPerThread;
+  constexpr int LPH = D / 8, GROUPS = THREADS / LPH, U = kRopeHeadsPerThread;
   const int tok = blockIdx.x;  // b*T + t
   const int b = tok / T, t = tok - b * T;
   const int sl = threadIdx.x % LPH, h0 = (int)blockIdx.y * GROUPS * U + threadIdx.x / LPH;
@@ -528,8 +529,10 @@ extern "C" int exo_rope_kv_append_tab(const uint16_t* qkv, uint16_t* q_out, uint
   const uintptr_t all = (uintptr_t)qkv | (uintptr_t)q_out | (uintptr_t)k_cache | (uintptr_t)v_cache | (uintptr_t)rope_table | (uintptr_t)q_norm_w | (uintptr_t)k_norm_w;
   if (!rope_table) table_rows = 0;  // (no position is inside it)
   if ((all & 15) == 0) {
-    const auto fn = D == 128 ? rope_kv_wide_kernel<128> : rope_kv_wide_kernel<64>;
-    fn<<<dim3(B * T, exo_ceil_div(Hq + 2 * Hkv, 2048 / D * kRopeHeadsPerThread)), 256, 0, (hipStream_t)stream>>>(
+    const int heads = Hq + 2 * Hkv, lanes = heads * (D / 8), threads = lanes <= 64 ? 64 : lanes <= 128 ? 128 : 256;
+    const auto fn = D == 128 ? (threads == 64 ? rope_kv_wide_kernel<128, 64> : threads == 128 ? rope_kv_wide_kernel<128, 128> : rope_kv_wide_kernel<128, 256>)
+                             : (threads == 64 ? rope_kv_wide_kernel<64, 64> : threads == 128 ? rope_kv_wide_kernel<64, 128> : rope_kv_wide_kernel<64, 256>);
+    fn<<<dim3(B * T, exo_ceil_div(heads, threads / (D / 8) * kRopeHeadsPerThread)), threads, 0, (hipStream_t)stream>>>(
         qkv, q_out, k_cache, v_cache, pos, inv_freq, reinterpret_cast<const float2*>(rope_table), table_rows, q_norm_w, k_norm_w, eps, T, Hq, Hkv, S_max);
     EXO_CHECK_LAUNCH("exo_rope_kv_append");
     return EXO_OK;

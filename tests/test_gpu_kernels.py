@@ -796,7 +796,7 @@ def test_add_rms_norm_chunks(device, rows, H, residual):
     assert bool(((got.double() - want).abs() <= (2.0**-8 + (H / 4 + 10) * 2.0**-24) * want.abs()).all())
 
 
-@pytest.mark.parametrize("D,Hq,Hkv", [(64, 5, 1), (64, 96, 1), (128, 46, 1), (128, 64, 8), (128, 1, 1)])
+@pytest.mark.parametrize("D,Hq,Hkv", [(64, 5, 1), (64, 6, 1), (64, 7, 1), (64, 14, 1), (64, 15, 1), (64, 96, 1), (128, 46, 1), (128, 64, 8), (128, 1, 1), (128, 2, 1), (128, 3, 1), (128, 6, 1), (128, 7, 1)])
 @pytest.mark.parametrize("qk_norm", [False, True])
 def test_rope_kv_append_pieces(device, D, Hq, Hkv, qk_norm):
     """Operands at 16 bytes against ones that are not, which go element by element: the same bits, with head norms but for the order of
