@@ -200,7 +200,7 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(
 // token beside one piece of the table's row.  What bounds it is the memory (a token of 32 / 8 heads of 128 is 24 KB in and out, 4.8 TB/s of it from 4096
 // tokens on); the kernel above moves 2 bytes a lane and sums a head's squares over the whole wave.  32 / 8 heads of 128, without | with norms, us: 61 tokens
 // 3.5 | 4.4 -> 3.3 | 3.6, 1023 9.5 | 12.5 -> 7.3 | 7.7, 4096 27.3 | 37.8 -> 20.1 | 20.9; of 64, 1023 tokens 8.7 | 11.8 -> 5.5 | 5.7.
-// Few heads leave most of 256 threads without one: as many threads as heads take (8000 tokens of 1 / 1 heads of 64 12.5 -> 5.8 us, of 5 / 1 13.3 -> 6.6).
+// Few heads leave most of 256 threads without one: as many threads as heads take (8000 tokens of 1 / 1 heads of 64 12.5 -> 5.8 us, of 5 / 1 13.3 -> 6.8).
 constexpr int kRopeHeadsPerThread = 3;
 template <int D, int THREADS>
 __global__ __launch_bounds__(THREADS) void rope_kv_wide_kernel(
