@@ -112,7 +112,7 @@ __device__ __forceinline__ float row_sum(float a, float (&part)[4][NW], int& pha
 // PP: float4 of a row per lane in front of the product (0: nothing there); NORMED: branches that are normed (0: one
 // that is added as it is).  RING: operands that are used up are requested again at once, for the step a batch ahead, so that requests
 // are in flight throughout (gemv_ring: where that is the faster one)
-template <typename T, int NW, int PP, int NORMED, bool PAIR, bool DUAL, int Q = 1, int STEPS = kBatch, bool RING = Q == 1 && PP == 0 ? false : !PAIR>
+template <typename T, int NW, int PP, int NORMED, bool PAIR, bool DUAL, int Q = 1, int STEPS = kBatch, bool RING = (Q != 1 && !PAIR)>
 __global__ __launch_bounds__(64 * NW) void dense_gemv_kernel(const GemvParams p0, const GemvParams p1, const PostNorm q) {
   constexpr bool POST = PP > 0, TWO = NORMED == 2;
   constexpr int NP = POST ? PP : 1, NU = TWO ? NP : 1;
@@ -932,15 +932,6 @@ bool post_fits(int M, int N, int H, int ldx, int elem) {
          (int64_t)M * (ldx * elem + 16) <= 40 * 1024;
 }
 
-template <typename T, int NW, int PP, int Q = 1>
-void launch_gemv_post(const GemvParams& p, const PostNorm& q, hipStream_t st) {
-  constexpr int one = Q > 1 ? kBatch / 2 : kBatch;  // (post_parts: a wave's share of a part; a pair has half of STEPS of each)
-  const int tiles = exo_ceil_div(p.N, 16 / Q), lds = p.M * (p.ldx * (int)sizeof(T) + 16);
-  const auto fn = q.branch2 ? (p.w2 ? dense_gemv_kernel<T, NW, PP, 2, true, false, Q> : dense_gemv_kernel<T, NW, PP, 2, false, false, Q, one>)
-                  : q.gain  ? (p.w2 ? dense_gemv_kernel<T, NW, PP, 1, true, false, Q> : dense_gemv_kernel<T, NW, PP, 1, false, false, Q, one>)
-                            : (p.w2 ? dense_gemv_kernel<T, NW, PP, 0, true, false, Q> : dense_gemv_kernel<T, NW, PP, 0, false, false, Q, one>);
-  fn<<<tiles, 64 * NW, lds, st>>>(p, p, q);
-}
 // Where a wave has more steps than one batch, the next batch was requested only when the last was used up, one memory latency after another.
 // Requested in a ring, rows of x as well as weights, us: 4096 columns bf16 K = 14336 under 1 | 4 | 8 rows 28.1 | 29.4 | 30.6 -> 24.6 | 25.4 | 27.4, K =
 // 4096 9.1 | 9.7 | 10.2 -> 8.4 | 8.8 | 9.4; 2048 columns of K = 6912 in two parts 8.2 | 9.0 | 9.8 -> 7.7 | 8.5 | 9.4; f32 4096 of 4096 under 2 rows 18.6 ->
@@ -952,6 +943,28 @@ void launch_gemv_post(const GemvParams& p, const PostNorm& q, hipStream_t st) {
 bool gemv_ring(const GemvParams& p, const GemvParams* p1, int waves, int elem) {
   const int steps = std::max(p.ldw, p1 ? p1->ldw : 0) * elem / 64;
   return p.M <= (waves == 4 ? 4 : 8) && steps > waves * kBatch;
+}
+// Behind norms, where the ring's registers come on top of the norms': from two whole batches on (f32, one row of 2048 into 20480 columns 37.6 -> 34.3
+// us, of 4096 81.7 -> 78.0; bf16 level), and not where a wave has one or one and a half (four rows of 1024 into 9216 13.6 | 14.3, one of 2048 into 3072 9.3 | 9.7).
+bool gemv_ring_post(const GemvParams& p, int waves, int elem) { return p.ldw * elem / 64 >= 2 * waves * kBatch; }
+template <typename T, int NW, int PP, int Q, bool RING>
+void launch_gemv_post_as(const GemvParams& p, const PostNorm& q, hipStream_t st) {
+  constexpr int one = Q > 1 ? kBatch / 2 : kBatch;  // (post_parts: a wave's share of a part; a pair has half of STEPS of each)
+  const int tiles = exo_ceil_div(p.N, 16 / Q), lds = p.M * (p.ldx * (int)sizeof(T) + 16);
+  const auto fn = q.branch2 ? dense_gemv_kernel<T, NW, PP, 2, false, false, Q, one, RING> : q.gain ? dense_gemv_kernel<T, NW, PP, 1, false, false, Q, one, RING>
+                                                                                                   : dense_gemv_kernel<T, NW, PP, 0, false, false, Q, one, RING>;
+  fn<<<tiles, 64 * NW, lds, st>>>(p, p, q);
+}
+template <typename T, int NW, int PP, int Q = 1>
+void launch_gemv_post(const GemvParams& p, const PostNorm& q, hipStream_t st) {
+  if (p.w2) {
+    const auto fn = q.branch2 ? dense_gemv_kernel<T, NW, PP, 2, true, false, Q> : q.gain ? dense_gemv_kernel<T, NW, PP, 1, true, false, Q> : dense_gemv_kernel<T, NW, PP, 0, true, false, Q>;
+    fn<<<exo_ceil_div(p.N, 16 / Q), 64 * NW, p.M * (p.ldx * (int)sizeof(T) + 16), st>>>(p, p, q);
+  } else if (Q > 1 || gemv_ring_post(p, NW, (int)sizeof(T))) {
+    launch_gemv_post_as<T, NW, PP, Q, true>(p, q, st);
+  } else if constexpr (Q == 1) {
+    launch_gemv_post_as<T, NW, PP, Q, false>(p, q, st);
+  }
 }
 template <typename T, int NW>
 void launch_gemv_nw(const GemvParams& p, const GemvParams* p1, const PostNorm* q, hipStream_t st) {
