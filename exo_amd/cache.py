@@ -50,10 +50,10 @@ class LayerKV:
 
 class HostWrites:
     """What the host changes in a cache (positions, page numbers) reaches the device in launches on the stream that is current, and
-    the call returns before they have run.  Whatever changes the cache next and every model's forward call ``order`` first,
-    which on another stream waits for the last change and all that was in front of it, so ``trim``, ``reserve`` and ``reset`` on
-    one stream and a step on another need no event between them.  Other readers of ``pos`` or of a page table, and
-    steps that run side by side, are ordered by their callers, as on any tensor."""
+    the call returns before they have run.  Every method that changes or reads a row's contents and every model's forward call
+    ``order`` first, which on another stream waits for the last change and all that was in front of it, so ``trim``, ``reserve``,
+    ``reset`` or ``restore`` on one stream and a step on another need no event between them.  Other readers of the tensors
+    here, and steps that run side by side, are ordered by their callers, as on any tensor."""
 
     pos: torch.Tensor
     _change: torch.cuda.Event | None = None  # behind the last change (None: on the default stream, which outlives it)
@@ -148,19 +148,23 @@ class ShardKVCache(HostWrites, list):
     # -- one row's contents as [n, Hkv, D] tensors (prefix cache, wire)
     def read_nhd(self, layer: int, row: int, start: int, n: int) -> tuple[torch.Tensor, torch.Tensor]:
         from . import ops
+        self.order()
         return (ops.kv_export_nhd(self.k[layer][row], start, n), ops.kv_export_nhd(self.v[layer][row], start, n))
 
     def write_nhd(self, layer: int, row: int, start: int, k: torch.Tensor, v: torch.Tensor) -> None:
         from . import ops
+        self.order()
         ops.kv_import_nhd(k, self.k[layer][row], start)
         ops.kv_import_nhd(v, self.v[layer][row], start)
 
     def snapshot(self, row: int) -> list[torch.Tensor]:
         """Detached copy of the row's positions, per layer [2, Hkv, n, D]."""
         n = self.offsets[row]
+        self.order()
         return [torch.stack((k[row, :, :n], v[row, :, :n])) for k, v in zip(self.k, self.v)]
 
     def restore(self, row: int, layers: list[torch.Tensor], length: int) -> None:
+        self.order()
         for kv, k, v in zip(layers, self.k, self.v):
             k[row, :, :length].copy_(kv[0, :, :length])
             v[row, :, :length].copy_(kv[1, :, :length])
@@ -170,6 +174,7 @@ class ShardKVCache(HostWrites, list):
     def copy_row(self, src: int, dst: int) -> None:
         """Move one sequence's cache to another batch row (slot compaction)."""
         n = self.offsets[src]
+        self.order()
         for k, v in zip(self.k, self.v):
             k[dst, :, :n].copy_(k[src, :, :n])
             v[dst, :, :n].copy_(v[src, :, :n])

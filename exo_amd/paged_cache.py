@@ -110,9 +110,11 @@ class PagedKVCache(HostWrites, list):
         return not len(self.states)
 
     def save_states(self, rows) -> list[torch.Tensor]:
+        self.order()
         return self.states.read(rows)
 
     def load_states(self, rows, saved: list[torch.Tensor]) -> None:
+        self.order()
         self.states.write(rows, saved)
 
     # -- pages
@@ -182,6 +184,7 @@ class PagedKVCache(HostWrites, list):
     def copy_row(self, src: int, dst: int) -> None:
         """Move one sequence to another row (slot compaction): pages and state slot change hands,
         no key or state moves."""
+        self.order()
         for t in (self._main, *self.means.values()):
             t.move(src, dst)
         self.offsets[dst], self.offsets[src] = self.offsets[src], 0
@@ -191,6 +194,7 @@ class PagedKVCache(HostWrites, list):
     def swap_rows(self, a: int, b: int) -> None:
         if a == b:
             return
+        self.order()
         for t in (self._main, *self.means.values()):
             t.swap(a, b)
         self.offsets[a], self.offsets[b] = self.offsets[b], self.offsets[a]
@@ -206,6 +210,7 @@ class PagedKVCache(HostWrites, list):
 
     def read_nhd(self, layer: int, row: int, start: int, n: int) -> tuple[torch.Tensor, torch.Tensor]:
         """Keys [n, G, D] and values [n, G, E] of positions [start, start + n)."""
+        self.order()
         g, d, e = self.shapes[layer]
         idx, off = self._row_pages(row, start, start + n), start % PAGE
         rows = len(idx) * PAGE
@@ -220,6 +225,7 @@ class PagedKVCache(HostWrites, list):
         g, d, e = self.shapes[layer]
         if tuple(k.shape[1:]) != (g, d) or tuple(v.shape) != (n, g, e):
             raise ValueError(f"keys {tuple(k.shape)} / values {tuple(v.shape)} do not fit layer {layer} ({g}, {d}, {e})")
+        self.order()
         at = torch.arange(start, start + n, device=self.pos.device)
         page = self._row_pages(row, 0, start + n)[at // PAGE]
         self.k[layer][page, :, at % PAGE, :d] = k.to(self.k[layer].dtype)
@@ -246,6 +252,7 @@ class PagedKVCache(HostWrites, list):
     def snapshot(self, row: int) -> list[tuple[torch.Tensor, torch.Tensor]]:
         """Detached copy of the row's positions, per layer (keys, values), then the recurrent
         states (one entry of all of them, if there are any)."""
+        self.order()
         kv = [self.read_nhd(i, row, 0, self.offsets[row]) for i in range(len(self.k))]
         return kv + ([tuple(self.states.read([row]))] if len(self.states) else [])
 

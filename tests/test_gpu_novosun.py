@@ -612,3 +612,35 @@ def test_pages_change_hands_on_streams_of_their_own(built, dtype):
     for g, w in zip(got, want):
         assert torch.equal(g, w)
     assert cache.pos.tolist() == cache.offsets == [41, 71]
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_rows_move_and_are_read_on_streams_of_their_own(built, dtype):
+    """A step behind other work on one stream, rows swapped and moved on a second, read on a third and stepped on a fourth, no
+    event between them."""
+    m, a, c = built.models[dtype], built.toks["a"], built.toks["c"]
+    quiet, cache = m.make_cache(3, 512), m.make_cache(3, 512)
+    x = torch.randn(4096, 4096, device="cuda")
+    torch.mm(x, x)
+    torch.cuda.synchronize()
+    m.step(quiet, [(0, a[:100], []), (1, c[:30], [])])
+    quiet.swap_rows(0, 1)
+    quiet.copy_row(1, 2)
+    want = quiet.snapshot(2) + [m.step(quiet, [(0, c[30:31], [0]), (2, a[100:101], [0])]).clone()]
+    torch.cuda.synchronize()
+    with torch.cuda.stream(torch.cuda.Stream()):
+        for _ in range(40):
+            torch.mm(x, x)
+        m.step(cache, [(0, a[:100], []), (1, c[:30], [])])
+    with torch.cuda.stream(torch.cuda.Stream()):
+        cache.swap_rows(0, 1)
+        cache.copy_row(1, 2)
+    with torch.cuda.stream(torch.cuda.Stream()):
+        got = cache.snapshot(2)
+    with torch.cuda.stream(torch.cuda.Stream()):
+        got.append(m.step(cache, [(0, c[30:31], [0]), (2, a[100:101], [0])]).clone())
+    torch.cuda.synchronize()
+    for g, w in zip(got, want):
+        for g1, w1 in zip(*((v if isinstance(v, (tuple, list)) else (v,)) for v in (g, w))):
+            assert torch.equal(g1, w1)
+    assert cache.pos.tolist() == cache.offsets
