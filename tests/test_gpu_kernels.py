@@ -332,10 +332,12 @@ def test_qmv_planes_of_far_elements(device, bits, M, N, K, down, far):
     assert bool(((got.double() - y).abs() <= slack).all()), float(((got.double() - y).abs() - slack).max())
 
 
-@pytest.mark.parametrize("bits,E,N,K,T,topk", [(4, 16, 5, 2048, 1, 8), (4, 8, 772, 2048, 5, 2), (8, 8, 9, 4096, 3, 4), (4, 4, 130, 8192, 2, 3), (8, 4, 66, 6144, 2, 2)])
+@pytest.mark.parametrize("bits,E,N,K,T,topk", [(4, 16, 5, 2048, 1, 8), (4, 8, 772, 2048, 5, 2), (8, 8, 9, 4096, 3, 4), (4, 4, 130, 8192, 2, 3), (8, 4, 66, 6144, 2, 2),
+                                                   (4, 8, 24, 2048, 12, 4), (8, 4, 9, 4096, 6, 2), (8, 4, 9, 4096, 5, 2), (4, 2, 30, 4096, 6, 2), (4, 2, 30, 4096, 5, 2)])
 def test_qmv_planes_of_experts(device, bits, E, N, K, T, topk):
     """The routed pair on the integer matrix cores: each (token, slot) has the outputs of its expert's own launch or, where that is
-    too small for it, those of the dot products to the last place or so."""
+    too small for it, those of the dot products to the last place or so; just below and at the pairs an expert from which K = 4096 stays with
+    the dot products."""
     g = torch.Generator(device=device).manual_seed(E + N)
 
     def experts():
@@ -348,7 +350,8 @@ def test_qmv_planes_of_experts(device, bits, E, N, K, T, topk):
     nw = (torch.randn(K, device=device, generator=g) * 0.1 + 1).bfloat16()
     idx = torch.stack([torch.randperm(E, generator=torch.Generator().manual_seed(t))[:topk] for t in range(T)]).int().to(device)
     got = ops.gather_qmv_swiglu(x, gate, up, idx, norm_weight=nw, eps=1e-5)
-    assert native.last_variant().startswith("qmv_planes<"), native.last_variant()
+    dots = K == 4096 and T * topk >= (3 if bits == 8 else 6) * E
+    assert native.last_variant().startswith("qmv_rows<" if dots else "qmv_planes<"), native.last_variant()
     one = lambda q, e: ops.QuantizedWeight(q.weight[e].contiguous(), q.scales[e].contiguous(), q.biases[e].contiguous(), bits)  # noqa: E731
     for t in range(T):
         for k in range(topk):
