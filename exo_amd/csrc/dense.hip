@@ -44,6 +44,7 @@ struct GemvParams {
   void* y;
   float* y2;       // columns from n1 on
   int M, N, n1, ldx, ldw, ldy, ldy2, y_f32;
+  int cols;        // weight rows of a workgroup, at most 16 / Q
   GluConst glu;
   Epilogue ep;
 };
@@ -124,10 +125,10 @@ __global__ __launch_bounds__(64 * NW) void dense_gemv_kernel(const GemvParams p0
   extern __shared__ __attribute__((aligned(16))) char xs[];  // POST: [M][ldx * sizeof(T) + 16]
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int r = lane & 15, g = lane >> 4;
-  const int tiles0 = (p0.N + R - 1) / R;
+  const int tiles0 = (p0.N + p0.cols - 1) / p0.cols;
   const bool second = DUAL && (int)blockIdx.x >= tiles0;
   const GemvParams& p = second ? p1 : p0;
-  const int n0 = ((int)blockIdx.x - (second ? tiles0 : 0)) * R, rows = min(R, p.N - n0);
+  const int n0 = ((int)blockIdx.x - (second ? tiles0 : 0)) * p.cols, rows = min(p.cols, p.N - n0);
   const uint32_t wrow = (uint32_t)p.ldw * sizeof(T), xrow = (uint32_t)p.ldx * sizeof(T);
   const int steps = (int)(wrow >> 6) / Q;  // (rows are multiples of 128 or 256 bytes)
   const uint32_t part_at = Q > 1 ? r / R * steps * 64 : 0;
@@ -950,7 +951,7 @@ bool gemv_ring_post(const GemvParams& p, int waves, int elem) { return p.ldw * e
 template <typename T, int NW, int PP, int Q, bool RING>
 void launch_gemv_post_as(const GemvParams& p, const PostNorm& q, hipStream_t st) {
   constexpr int one = Q > 1 ? kBatch / 2 : kBatch;  // (post_parts: a wave's share of a part; a pair has half of STEPS of each)
-  const int tiles = exo_ceil_div(p.N, 16 / Q), lds = p.M * (p.ldx * (int)sizeof(T) + 16);
+  const int tiles = exo_ceil_div(p.N, p.cols), lds = p.M * (p.ldx * (int)sizeof(T) + 16);
   const auto fn = q.branch2 ? dense_gemv_kernel<T, NW, PP, 2, false, false, Q, one, RING> : q.gain ? dense_gemv_kernel<T, NW, PP, 1, false, false, Q, one, RING>
                                                                                                    : dense_gemv_kernel<T, NW, PP, 0, false, false, Q, one, RING>;
   fn<<<tiles, 64 * NW, lds, st>>>(p, p, q);
@@ -959,7 +960,7 @@ template <typename T, int NW, int PP, int Q = 1>
 void launch_gemv_post(const GemvParams& p, const PostNorm& q, hipStream_t st) {
   if (p.w2) {
     const auto fn = q.branch2 ? dense_gemv_kernel<T, NW, PP, 2, true, false, Q> : q.gain ? dense_gemv_kernel<T, NW, PP, 1, true, false, Q> : dense_gemv_kernel<T, NW, PP, 0, true, false, Q>;
-    fn<<<exo_ceil_div(p.N, 16 / Q), 64 * NW, p.M * (p.ldx * (int)sizeof(T) + 16), st>>>(p, p, q);
+    fn<<<exo_ceil_div(p.N, p.cols), 64 * NW, p.M * (p.ldx * (int)sizeof(T) + 16), st>>>(p, p, q);
   } else if (Q > 1 || gemv_ring_post(p, NW, (int)sizeof(T))) {
     launch_gemv_post_as<T, NW, PP, Q, true>(p, q, st);
   } else if constexpr (Q == 1) {
@@ -968,7 +969,7 @@ void launch_gemv_post(const GemvParams& p, const PostNorm& q, hipStream_t st) {
 }
 template <typename T, int NW>
 void launch_gemv_nw(const GemvParams& p, const GemvParams* p1, const PostNorm* q, hipStream_t st) {
-  const int tiles = exo_ceil_div(p.N, 16);
+  const int tiles = exo_ceil_div(p.N, p.cols);
   const PostNorm none{};
   if (q) {
     const int passes = exo_ceil_div(p.ldx, post_waves_per_row(p.M, NW) * 256);  // (post_fits: at most kPostPasses)
@@ -984,7 +985,7 @@ void launch_gemv_nw(const GemvParams& p, const GemvParams* p1, const PostNorm* q
     const bool ring = gemv_ring(p, p1, NW, (int)sizeof(T));
     const auto fn = p1 ? (ring ? dense_gemv_kernel<T, NW, 0, 0, false, true, 1, kBatch, true> : dense_gemv_kernel<T, NW, 0, 0, false, true>)
                        : (ring ? dense_gemv_kernel<T, NW, 0, 0, false, false, 1, kBatch, true> : dense_gemv_kernel<T, NW, 0, 0, false, false>);
-    fn<<<tiles + (p1 ? exo_ceil_div(p1->N, 16) : 0), 64 * NW, 0, st>>>(p, p1 ? *p1 : p, none);
+    fn<<<tiles + (p1 ? exo_ceil_div(p1->N, p1->cols) : 0), 64 * NW, 0, st>>>(p, p1 ? *p1 : p, none);
   }
 }
 // Parts of K side by side where 16 columns per workgroup leave CUs without work, as many rows of x as the
@@ -1043,7 +1044,7 @@ int post_parts(const GemvParams& p, const PostNorm& q, int elem) {
 }
 template <typename T, bool PAIR, bool DUAL, int Q>
 void launch_gemv_parts(const GemvParams& p, const GemvParams* p1, hipStream_t st) {
-  const int tiles = exo_ceil_div(p.N, 16 / Q) + (DUAL ? exo_ceil_div(p1->N, 16 / Q) : 0);
+  const int tiles = exo_ceil_div(p.N, p.cols) + (DUAL ? exo_ceil_div(p1->N, p1->cols) : 0);
   const PostNorm none{};
   // (half the requests at once where a wave's share of a part is no more: requests past it cost time as well)
   const int ldw = DUAL && p1->ldw > p.ldw ? p1->ldw : p.ldw;
@@ -1052,20 +1053,77 @@ void launch_gemv_parts(const GemvParams& p, const GemvParams* p1, hipStream_t st
   else
     dense_gemv_kernel<T, 8, 0, 0, PAIR, DUAL, Q><<<tiles, 512, 0, st>>>(p, DUAL ? *p1 : p, none);
 }
+// Weight rows of a workgroup and its waves.  All workgroups of a launch of up to about two rounds are resident together, so the CU
+// that got the most rows ends last: 864 workgroups of 8 rows leave some CUs with 32 and the average with 27, 988 of 7 all with 28.  Fewer
+// rows than the product holds cost nothing but its empty lanes.  Fewer waves cost less where every workgroup repeats norms and
+// adds its waves' sums, more of them keep more requests in flight.  gemv_us is a fit to 4873 shapes (64 to 14336 columns of K, 300 to
+// 40000 columns, 1 to 16 rows, with and without norms, bf16 and f32, 12 settings each).  What is fastest by it takes, on average, 0.946 of the time of
+// whole 16 / parts rows and waves by the number of columns (gemv_waves), pairs 0.948, behind norms 0.946 and 0.935 (the best setting of each shape 0.93 to
+// 0.94); slower by more than 3 % are 0.2 to 0.9 %: the 4 % that it has to promise leave most of them out.  us: f32 under 2 rows behind norms, 6432
+// columns of 1024 11.0 -> 9.6, pair of 2560 10.5 -> 9.1; bf16 under 4 rows pair of 6912x2048 13.5 -> 12.6, under 8 15.6 -> 13.9, one row
+// behind a norm 6160x2048 9.8 -> 8.3.
+struct GemvShape {
+  int waves, cols;
+};
+double gemv_us(const GemvParams& p, const GemvParams* p1, const PostNorm* q, int elem, int parts, GemvShape c) {
+  const int mats = p.w2 ? 2 : 1, row = std::max(p.ldw, p1 ? p1->ldw : 0) * elem;
+  const int wgs = exo_ceil_div(p.N, c.cols) + (p1 ? exo_ceil_div(p1->N, c.cols) : 0), held = exo_ceil_div(wgs, 256);  // by the fullest CU
+  const double total = ((double)p.N * p.ldw + (p1 ? (double)p1->N * p1->ldw : 0.0)) * elem * mats;
+  const double cu = (double)c.cols * row * mats / 25e3;  // a workgroup's bytes at 25 GB/s
+  const double fullest = std::max(held * cu, total / 6.4e6), average = wgs * cu / 256;
+  const double x = (double)held * p.M * row / 64e3, waves = c.waves * wgs / 8192.0;  // rows of x read, waves beside one another
+  const int steps = exo_ceil_div(row / 64 / parts, c.waves);
+  const int batch = kBatch / mats / (!q && parts > 1 && steps <= kBatch / mats / 2 ? 2 : 1);
+  const double empty = (double)(exo_ceil_div(steps, batch) * batch - steps) * c.waves * held / 64;  // requests past a wave's range
+  if (!q)
+    return p.w2 ? 2.29 + 0.65 * fullest + 0.41 * average + 1.42 * x + 0.25 * waves + 1.17 * empty + 0.15 * steps
+                : 2.46 + 0.74 * fullest + 0.45 * average + 1.34 * x + 0.83 * empty + (0.002 * p.M + 0.027) * steps;
+  const int passes = exo_ceil_div(p.ldx, post_waves_per_row(p.M, c.waves) * 256);
+  const double norms = (q->branch2 ? 3.2 * waves : 0.0);
+  return norms + (p.w2 ? 0.94 + 0.69 * fullest + 0.34 * average + 4.77 * x + 1.73 * waves + 2.19 * empty + 0.51 * passes + 0.14 * steps + 0.17 * c.waves
+                       : 0.96 + 0.74 * fullest + 0.20 * average + 3.1 * x + 2.52 * waves + 0.51 * empty + 0.66 * passes + 0.083 * steps + 0.21 * c.waves);
+}
+GemvShape gemv_shape(const GemvParams& p, const GemvParams* p1, const PostNorm* q, int elem, int parts) {
+  const int N = p.N + (p1 ? p1->N : 0), most = 16 / parts;
+  auto passes = [&](int waves) { return exo_ceil_div(p.ldx, post_waves_per_row(p.M, waves) * 256); };
+  const GemvShape usual{parts > 1 ? 8 : gemv_waves(N), most};
+  GemvShape best = usual;
+  double least = 0.96 * gemv_us(p, p1, q, elem, parts, usual);
+  for (int waves = 4; waves <= 16; waves *= 2) {
+    if (parts > 1 && waves != 8) continue;
+    if (q && passes(waves) > std::max(2, passes(usual.waves))) continue;  // (beyond, gains are not requested ahead)
+    auto weigh = [&](int cols) {
+      const double us = gemv_us(p, p1, q, elem, parts, {waves, cols});
+      if (us < least) least = us, best = GemvShape{waves, cols};
+    };
+    weigh(most);
+    // one, two ... workgroups a CU (two products: one workgroup more), down to half of the rows that a product holds
+    for (int held = exo_ceil_div(N, 256 * most), cols = most; 2 * cols > most; ++held) {
+      cols = exo_ceil_div(N, 256 * held - (p1 ? 1 : 0));
+      if (cols <= most && 2 * cols >= most) weigh(cols);
+    }
+  }
+  return best;
+}
 template <typename T>
-int launch_gemv(const GemvParams& p, const GemvParams* p1, const PostNorm* q, hipStream_t st) {
-  if (q && post_parts(p, *q, (int)sizeof(T)) == 2) {
-    exo_note_variant("dense_gemv<%s,8,post,%s> M=%d N=%d parts=2", sizeof(T) == 2 ? "bf16" : "f32", p.w2 ? "pair" : "single", p.M, p.N);
+int launch_gemv(GemvParams p, const GemvParams* second, const PostNorm* q, hipStream_t st) {
+  GemvParams other{};
+  const GemvParams* p1 = nullptr;
+  if (second) other = *second, p1 = &other;
+  const int parts = q ? post_parts(p, *q, (int)sizeof(T)) : gemv_parts(p, p1, (int)sizeof(T));
+  const GemvShape shape = gemv_shape(p, p1, q, (int)sizeof(T), parts);
+  p.cols = other.cols = shape.cols;
+  if (q && parts == 2) {
+    exo_note_variant("dense_gemv<%s,8,post,%s> M=%d N=%d parts=2 cols=%d", sizeof(T) == 2 ? "bf16" : "f32", p.w2 ? "pair" : "single", p.M, p.N, p.cols);
     if (p.ldx <= post_waves_per_row(p.M, 8) * 256)
       launch_gemv_post<T, 8, 1, 2>(p, *q, st);
     else
       launch_gemv_post<T, 8, 2, 2>(p, *q, st);
     return EXO_OK;
   }
-  const int parts = q ? 1 : gemv_parts(p, p1, (int)sizeof(T));
   if (parts > 1) {
-    exo_note_variant("dense_gemv<%s,8,plain,%s> M=%d N=%d parts=%d", sizeof(T) == 2 ? "bf16" : "f32",
-                     p1 ? "dual" : p.w2 ? "pair" : "single", p.M, p.N, parts);
+    exo_note_variant("dense_gemv<%s,8,plain,%s> M=%d N=%d parts=%d cols=%d", sizeof(T) == 2 ? "bf16" : "f32",
+                     p1 ? "dual" : p.w2 ? "pair" : "single", p.M, p.N, parts, p.cols);
     const auto launch = parts == 4 ? p1     ? launch_gemv_parts<T, false, true, 4>
                                      : p.w2 ? launch_gemv_parts<T, true, false, 4>
                                             : launch_gemv_parts<T, false, false, 4>
@@ -1075,9 +1133,9 @@ int launch_gemv(const GemvParams& p, const GemvParams* p1, const PostNorm* q, hi
     launch(p, p1, st);
     return EXO_OK;
   }
-  const int nw = gemv_waves(p.N + (p1 ? p1->N : 0));
-  exo_note_variant("dense_gemv<%s,%d,%s,%s> M=%d N=%d", sizeof(T) == 2 ? "bf16" : "f32", nw, q ? "post" : "plain",
-                   p1 ? "dual" : p.w2 ? "pair" : "single", p.M, p.N);
+  const int nw = shape.waves;
+  exo_note_variant("dense_gemv<%s,%d,%s,%s> M=%d N=%d cols=%d", sizeof(T) == 2 ? "bf16" : "f32", nw, q ? "post" : "plain",
+                   p1 ? "dual" : p.w2 ? "pair" : "single", p.M, p.N, p.cols);
   if (nw == 4)
     launch_gemv_nw<T, 4>(p, p1, q, st);
   else if (nw == 8)

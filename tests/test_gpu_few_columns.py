@@ -140,6 +140,45 @@ def test_parts_of_k_behind_norms(device, dtype, M, N, H, two, pair, parts):
     assert bool(((got.double() - a * c / 2).abs() <= bound + 1e-12).all())
 
 
+# workgroups of fewer columns than a product holds, so that CUs get equal shares: one workgroup a CU and two, a last one of one column, the
+# fewest of each number of parts, outputs whose last columns go to another buffer, a pair, two products, 4, 8 and 16 waves
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,N,K,kind", [(1, 2305, 4096, "plain"), (2, 6657, 2048, "plain"), (8, 6700, 2048, "plain"), (16, 2817, 3072, "plain"), (4, 6913, 2048, "pair"),
+                                        (3, 1281, 1024, "pair"), (1, 766, 4096, "plain"), (9, 4353, 512, "pair"), (2, 2600, 2048, "dual"), (5, 6200, 3584, "dual")])
+def test_columns_of_a_workgroup(device, dtype, M, N, K, kind):
+    g = torch.Generator(device=device).manual_seed(M + N + K)
+    x, w = (torch.randn(n, K, device=device, generator=g).to(dtype) for n in (M, N))
+    out = torch.full((M + 1, N + 3), 7.0, dtype=dtype, device=device)
+    if kind == "dual":
+        n0, second = N // 3, torch.full((M + 1, N), 7.0, device=device)
+        D.linear_pair(x, w[:n0], out, x, w[n0:], second, M)
+        check(out[:M, :n0], x, w[:n0])
+        check(second[:M, : N - n0], x, w[n0:])
+        assert bool((out[:, n0:] == 7).all()) and bool((second[M:] == 7).all()) and bool((second[:, N - n0 :] == 7).all())
+    elif kind == "pair":
+
+        class Ones:  # (a gate of 1 and no bend: half the product of the two)
+            limit, alpha, shift, cubic = float("inf"), 0.0, 0.0, 0.0
+
+        u = torch.randn(N, K, device=device, generator=g).to(dtype)
+        D.glu(x, w, u, out, M, Ones)
+        a, c, size_a, size_c = (p.double() @ q.double().T for p, q in ((x, w), (x, u), (x.abs(), w.abs()), (x.abs(), u.abs())))
+        bound = (K + 1) * 2.0**-24 * (size_a * c.abs() + size_c * a.abs()) * 0.51 + (2.0**-8 if dtype == torch.bfloat16 else 2.0**-22) * (a * c / 2).abs()
+        assert bool(((out[:M, :N].double() - a * c / 2).abs() <= bound + 1e-12).all())
+        assert bool((out[M:] == 7).all()) and bool((out[:, N:] == 7).all())
+    else:
+        t = torch.zeros(M, 37, device=device)
+        D.linear(x, w, out, M, tail=(t, 37))
+        check(out[:M, : N - 37], x, w[: N - 37])
+        check(t, x, w[N - 37 :])
+        assert bool((out[M:] == 7).all()) and bool((out[:, N - 37 :] == 7).all())
+    label = native.last_variant()
+    print(label)
+    parts = int(label.split("parts=")[1].split()[0]) if "parts=" in label else 1
+    cols = int(label.split("cols=")[1])
+    assert 8 // parts <= cols < 16 // parts, label
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("M,N,K", [(1, 70, 128), (4, 1530, 896), (8, 2500, 192), (6, 2545, 320)])
 def test_gated_pair_and_two_products(device, dtype, M, N, K):
