@@ -474,6 +474,24 @@ __device__ __forceinline__ void store_tile(const GemmParams& p, floatx16 (&acc)[
     }
     return;
   }
+  // A range of K of a gated pair: the gate's sums, then the up matrix's
+  if (!GROUPED && PAIR && p.ksplit > 1) {
+    const uint32_t row = (uint32_t)p.N * 4;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const __amdgpu_buffer_rsrc_t to = buf_of(p.part + ((size_t)(blockIdx.z * 2 + (j & 1)) * p.M + m0) * p.N, (uint32_t)(m_end - m0) * row);
+      const int n = n0 + wcol * (16 * NJ) + (j >> 1) * 32 + frow;
+      const uint32_t voff = n < p.N ? (uint32_t)(wm + 4 * half) * row + n * 4 : kPastEnd;
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const float v = acc[i][j][e];
+          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), to, voff + (uint32_t)(32 * i + 8 * (e >> 2) + (e & 3)) * row, 0, 0);
+        }
+    }
+    return;
+  }
   // Gated pairs and an expert's rows, in the element type: the same with a row's offset from the list of
   // pairs (four consecutive tile rows at a time).
   if (GROUPED || PAIR) {
@@ -800,6 +818,17 @@ __global__ __launch_bounds__(256) void dense_reduce_kernel(const GemmParams p) {
       p.y2[(size_t)m * p.ldy2 + n + e - p.n1] = v[e];
   }
 }
+// ... of a gated pair, and its unit
+template <typename T>
+__global__ __launch_bounds__(256) void dense_reduce_pair_kernel(const GemmParams p) {
+  const int n = blockIdx.x * 256 + threadIdx.x, m = blockIdx.y;
+  if (n >= p.N) return;
+  const size_t one = (size_t)p.M * p.N;
+  const float* at = p.part + (size_t)m * p.N + n;
+  float g = 0.f, u = 0.f;
+  for (int z = 0; z < p.ksplit; ++z) g += at[2 * z * one], u += at[(2 * z + 1) * one];
+  store_out<T>(p.y, (size_t)m * p.ldy + n, gated<T>(g, u, p.glu), p.y_f32);
+}
 template <typename T>
 void launch_reduce(const GemmParams& p, hipStream_t st) {
   // (from 2 MB of results on; below, one column per thread is as fast or, 130 rows of 2048, 15.9 us of a product against 18.0, faster)
@@ -867,6 +896,25 @@ bool wide_is_faster(int64_t wide, int64_t narrow, int steps, int64_t out_bytes) 
   return tw < tn;
 }
 
+// Ranges of K of a gated pair whose tiles leave CUs without work, or few in flight on each.  us: a step of 128 bytes of K takes 0.6 in bf16 and 1.3 in
+// float, 1.7 times that with two workgroups on a CU, which is a full round; the reduce launch 2.75 and 0.35 a range more, the
+// sums' way through memory 2.5 MB / us.
+// Over 271 shapes (17 to 700 rows, 300 to 9000 columns, K of 128 to 8000) what this gives takes 0.65 of the time of one range on average (the best number
+// 0.644), 1.01 at most.  Pair of 2560x1024 float under 53 rows, 40 workgroups, 40 -> 17 us; of 6912x2048 bf16 under 60 24.3 -> 18.8; of 999x7424 under 206
+// 69 -> 25.
+int pair_ranges(int64_t tiles, int steps, int64_t outputs, bool tall, int elem, int64_t ws_floats) {
+  const double step = (elem == 2 ? 0.6 : 1.3) * (tall ? 1.6 : 1.0);
+  auto rounds = [](int64_t wgs) { return wgs / 512 * 1.7 + (wgs % 512 > 256 ? 1.7 : wgs % 512 ? 1.0 : 0.0); };
+  int best = 1;
+  double least = 0.97 * step * steps * rounds(tiles);
+  for (int ks = 2; ks <= 16 && steps / ks >= 2 && 2 * ks * outputs <= ws_floats; ++ks) {
+    const int range = exo_ceil_div(steps, ks), used = exo_ceil_div(steps, range);
+    const double us = step * range * rounds(tiles * used) + 2.75 + used * (0.35 + 8e-6 / 2.5 * outputs);
+    if (us < least) least = us, best = ks;
+  }
+  return best;
+}
+
 // rows per tile: the tallest that still leaves a workgroup per CU, else the shorter ones
 template <typename T, bool PAIR>
 int launch_plain(GemmParams p, int64_t ws_floats, hipStream_t st) {
@@ -912,13 +960,22 @@ int launch_plain(GemmParams p, int64_t ws_floats, hipStream_t st) {
       p.ksplit = exo_ceil_div(steps, p.ksteps);
     }
   }
+  if (PAIR && p.part) {
+    const int ks = pair_ranges(tall ? t2 : t1, steps, (int64_t)p.M * p.N, tall, (int)sizeof(T), ws_floats);
+    if (ks > 1) {
+      p.ksteps = exo_ceil_div(steps, ks);
+      p.ksplit = exo_ceil_div(steps, p.ksteps);
+    }
+  }
   int rc;
   if (tall)
     rc = launch_gemm<T, 2, 2, false, PAIR>(p, exo_ceil_div(p.M, 128), st);
   else
     rc = launch_gemm<T, 1, 2, false, PAIR>(p, exo_ceil_div(p.M, 64), st);
   if (rc) return rc;
-  if (p.ksplit > 1)
+  if (p.ksplit > 1 && PAIR)
+    dense_reduce_pair_kernel<T><<<dim3(exo_ceil_div(p.N, 256), p.M), 256, 0, st>>>(p);
+  else if (p.ksplit > 1)
     launch_reduce<T>(p, st);
   return EXO_OK;
 }
@@ -1262,11 +1319,11 @@ extern "C" int exo_linear_gemm(const exo_linear* a, float* workspace, int64_t wo
   p.M = a->M, p.N = a->N, p.n1 = a->n1, p.ldx = a->ldx, p.ldw = a->ldw, p.ldy = a->ldy, p.ldy2 = a->ldy2, p.y_f32 = a->y_f32;
   p.glu = GluConst{a->limit, a->alpha, a->shift, a->cubic};
   p.ep = Epilogue{a->act, a->mul, a->mul_rows, a->ldmul, a->cap};
-  p.part = a->w_up ? nullptr : workspace;
+  p.part = workspace;
   EXO_REQUIRE(!a->w_up || a->y_f32 == (a->dtype == 1), "exo_linear_gemm: a gated pair leaves in the element type");
   if (a->w_up)
-    rc = EXO_BY_TYPE(a->dtype, (launch_plain<bf16_t, true>(p, 0, (hipStream_t)stream)),
-                     (launch_plain<float, true>(p, 0, (hipStream_t)stream)));
+    rc = EXO_BY_TYPE(a->dtype, (launch_plain<bf16_t, true>(p, workspace_floats, (hipStream_t)stream)),
+                     (launch_plain<float, true>(p, workspace_floats, (hipStream_t)stream)));
   else
     rc = EXO_BY_TYPE(a->dtype, (launch_plain<bf16_t, false>(p, workspace_floats, (hipStream_t)stream)),
                      (launch_plain<float, false>(p, workspace_floats, (hipStream_t)stream)));

@@ -328,3 +328,28 @@ def test_norm_of_few_rows(device, dtype, n, H, center, at):
     tol = (H / 4 + 20) * 2.0**-24
     assert bool(((out[:n, :H].double() - want).abs() <= (tol + (2.0**-8 if dtype == torch.bfloat16 else 0)) * want.abs() + 5 * tol).all())
     assert bool((out[n:] == 7).all()) and bool((out[:, H:] == 7).all())
+
+
+# gated pairs of few tiles: ranges of K and their sums in a launch of its own; a last range that is shorter, rows and columns that do not
+# fill a tile, the most ranges, tall tiles, and pairs that stay whole
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,N,K,split", [(17, 65, 1152, True), (53, 2560, 1024, None), (100, 333, 4800, True), (64, 6912, 2048, True), (129, 1990, 5952, True), (700, 1100, 6016, None),
+                                         (20, 400, 64, False), (300, 7000, 256, False)])
+def test_gated_pair_in_ranges_of_k(device, dtype, M, N, K, split):
+    g = torch.Generator(device=device).manual_seed(M + N + K)
+    x, gate, up = (torch.randn(n, K, device=device, generator=g).to(dtype) * (1 if n == M else K**-0.5) for n in (M, N, N))
+
+    class Spec:
+        limit, alpha, shift, cubic = 1.5, 1.702, 1.0, 0.0
+
+    out = torch.full((M + 1, N + 5), 7.0, dtype=dtype, device=device)
+    D.glu_gemm(x, gate, up, out, M, Spec)
+    label = native.last_variant()
+    assert "pair" in label and (split is None or label.endswith("x1") != split), label
+    a, c = x.double() @ gate.double().T, x.double() @ up.double().T
+    want = a.clamp(max=1.5) * torch.sigmoid(1.702 * a.clamp(max=1.5)) * (c.clamp(-1.5, 1.5) + 1)
+    # (the unit's slope stays below 1.1 and it below |a|; the two sums' errors as above, the unit's own work 2^-20, in bf16 2^-18, and a rounding)
+    size_a, size_c = x.double().abs() @ gate.double().abs().T, x.double().abs() @ up.double().abs().T
+    bound = (K + 1) * 2.0**-24 * (1.1 * size_a * 2.5 + size_c * 1.5) + (2.0**-20 if dtype == torch.float32 else 2.0**-8 + 2.0**-18) * want.abs()
+    assert bool(((out[:M, :N].double() - want).abs() <= bound + 1e-12).all())
+    assert bool((out[M:] == 7).all()) and bool((out[:, N:] == 7).all())
