@@ -26,7 +26,8 @@ constexpr int rows_lds(int K) {
   return K / 64 * kPlaneGroup * (TOK / 4) + TOK * (K / 64 + 4) * (int)sizeof(GroupSum) + 2 * kRowsTiles<TOK> * kRowsWaves * TOK * 16 * 4;
 }
 
-// K = 2048 * XS; p.slots: tiles of 16 rows (a pair: 8 of each matrix)
+// K = 2048 * XS; p.slots: tiles of 16 rows (a pair: 8 of each matrix), 8 bits: of p.tile_rows, where the product's other columns repeat the
+// last one
 template <int BITS, int NMAT, int XS, int TOK>
 __global__ __launch_bounds__(64 * kRowsWaves) void qmv_planes_rows_kernel(const QmvParams p) {
   extern __shared__ uint4 smem[];
@@ -47,7 +48,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void qmv_planes_rows_kernel(const 
   __shared__ float s_ss[kRowsWaves];
   __shared__ int s_bad[kRowsWaves];
 
-  const int tiles = p.slots;
+  const int tiles = p.slots, rows = BITS == 8 ? p.tile_rows : RPT;
   const int base = tiles / (int)gridDim.x, rem = tiles - base * (int)gridDim.x;
   const int t0 = (int)blockIdx.x * base + min((int)blockIdx.x, rem);
   const int t1 = t0 + base + ((int)blockIdx.x < rem ? 1 : 0);
@@ -65,7 +66,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void qmv_planes_rows_kernel(const 
     }
   }
 
-  const int mat = NMAT == 2 ? n >> 3 : 0, r_of = n % RPT;
+  const int mat = NMAT == 2 ? n >> 3 : 0, r_in = BITS == 8 ? min(n % RPT, p.tile_rows - 1) : n % RPT;
   const size_t row_bytes = (size_t)p.wpr * 4;
   const char* const wm = reinterpret_cast<const char*>(mat ? p.w[NMAT - 1] : p.w[0]) + wave * (GW * 8 * BITS) + q * 16;
   const bf16_t* const sm = (mat ? p.s[NMAT - 1] : p.s[0]) + wave * GW;
@@ -86,7 +87,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void qmv_planes_rows_kernel(const 
   const int nb = (t1 - t0) * ITERS;
   int it = t0, ib = 0;  // tile and batch that are requested next
   auto issue = [&](Batch& b) {
-    const int row = min(min(it, t1 - 1) * RPT + r_of, p.N - 1);  // (rows and tiles past the end: the last one's, dropped)
+    const int row = min(min(it, t1 - 1) * rows + r_in, p.N - 1);  // (rows and tiles past the end: the last one's, dropped)
     const char* w = wm + (size_t)row * row_bytes + ib * (UB * 64);
 #pragma unroll
     for (int u = 0; u < UB; ++u) b.w[u] = *reinterpret_cast<const uint4*>(w + u * 64);
@@ -160,8 +161,8 @@ __global__ __launch_bounds__(64 * kRowsWaves) void qmv_planes_rows_kernel(const 
     const auto& from = red[(first - t0) / C & 1];
     lds_barrier();
     for (int e = threadIdx.x; e < C * TOK * RPT; e += 64 * kRowsWaves) {
-      const int c = e / (TOK * RPT), t = e / RPT % TOK, r = e % RPT, row = (first + c) * RPT + r;
-      if (first + c >= end || t >= p.M || row >= p.N) continue;
+      const int c = e / (TOK * RPT), t = e / RPT % TOK, r = e % RPT, row = (first + c) * rows + r;
+      if (r >= rows || first + c >= end || t >= p.M || row >= p.N) continue;
       const int at = t * 16 + r;
       auto sum = [&](int at) {
         float v = from[c][0][at];

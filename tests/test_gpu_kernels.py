@@ -300,6 +300,35 @@ def test_qmv_planes_rows(device, bits, M, N, K, pair, norm):
     assert bool(other[M - 1].isnan().all()) and torch.equal(other[: M - 1], got[: M - 1])
 
 
+@pytest.mark.parametrize("M,N,K,pair,grid", [
+    (4, 976, 8192, False, 122), (3, 4464, 8192, False, 256), (8, 4112, 4096, False, 256), (2, 2053, 2048, True, 256), (5, 509, 4096, True, 128), (6, 521, 2048, False, 66), (3, 4096, 4096, False, 256),
+])
+def test_planes_rows_tiles_of_fewer_rows(device, M, N, K, pair, grid):
+    """8 bits, fewer tiles than CUs or unequal shares of them: tiles of fewer than 16 rows (a pair: 8 of each matrix), a last tile of a part of those, and equal shares."""
+    g = torch.Generator(device=device).manual_seed(N + K + M)
+    ws = [ops.QuantizedWeight(torch.randint(-2**31, 2**31 - 1, (N, K // 4), dtype=torch.int32, device=device, generator=g),
+                              *((torch.randn(N, K // 64, device=device, generator=g) * f).bfloat16() for f in (0.002, 0.1)), 8) for _ in range(1 + pair)]
+    x, nw = torch.randn(M, K, device=device, generator=g).bfloat16(), torch.ones(K, dtype=torch.bfloat16, device=device)
+    if pair:
+        got = ops.qmv_swiglu(x, *ws)
+    else:
+        got = ops.quantized_matmul(x, ws[0], norm_weight=nw if M in (3, 4) else None, eps=1e-5)
+    assert native.last_variant() == f"qmv_planes_rows<8,{1 + pair},{K // 2048},{4 if M <= 4 else 8}> grid={grid}", native.last_variant()
+    xn = ops.rms_norm(x, nw, 1e-5).double() if not pair and M in (3, 4) else x.double()
+    sums = []
+    for q in ws:
+        codes, s, b = ops.unpack_codes(q.weight, 8).double().view(N, -1, 64), q.scales.double()[..., None], q.biases.double()[..., None]
+        size = xn.abs() @ ((codes + 128) * s.abs() + b.abs()).view(N, K).T
+        # (a sum of K / 64 groups in float32, elements to 2^-30 of their group's largest, the norm's rounding of an element, one to bf16)
+        y = xn @ (codes * s + b).view(N, K).T
+        sums.append((y, ((4 + K // 64) * 2.0**-24 + 2.0**-26) * size + (2.0**-7 * y.pow(2).mean(1, keepdim=True).sqrt() if not pair else 0) + 2.0**-8 * y.abs()))
+    y, slack = sums[0]
+    if pair:
+        (yu, slack_u), unit = sums[1], y * torch.sigmoid(y)
+        y, slack = unit * yu, 1.1 * slack * (yu.abs() + slack_u) + unit.abs() * slack_u + 2.0**-8 * ((unit * yu).abs() + unit.abs() * yu.abs())
+    assert bool(((got.double() - y).abs() <= slack + 1e-30).all()), float(((got.double() - y).abs() - slack).max())
+
+
 @pytest.mark.parametrize("bits,M,N,K,down", [(4, 1, 8600, 2048, 0), (4, 1, 1960, 8192, 0), (8, 1, 4300, 2048, 0), (8, 1, 1400, 6144, 0), (8, 3, 1600, 2048, 0),
                                              (8, 8, 4100, 4096, 0), (4, 3, 28700, 8192, 0), (4, 1, 77, 1536, 8), (8, 2, 50, 768, 2)])
 @pytest.mark.parametrize("far", [2.0**40, 2.0**-90])
