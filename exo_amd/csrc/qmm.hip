@@ -173,6 +173,16 @@ __device__ __forceinline__ void tile_of_block(int& x, int& y) {
   tile_at<GM>(xcd_run(y * gx + x, n), gx, gy, x, y);
 }
 
+// Experts: the column tiles of a row tile go to one XCD, eight row tiles at a time, so that its activations come out of that L2
+// (in launch order each XCD reads those of nearly all experts: 4 MB of 1023 tokens, more than its L2 has room for beside the weights; down products of
+// 2048x768 under 1023 tokens 56 -> 51 us, 512 columns 46 -> 38)
+__device__ __forceinline__ void expert_tile_of_block(int& x, int& y) {
+  const int gx = gridDim.x, gy = gridDim.y, l = blockIdx.y * gx + blockIdx.x;
+  const int g = l / (8 * gx), in = l - g * (8 * gx), rows = min(8, gy - g * 8);
+  x = in / rows;
+  y = g * 8 + (in - x * rows);
+}
+
 // The 256 x 256 tile, one workgroup per CU: whole tiles first, and where the last round would leave half
 // of the CUs idle, its tiles as two halves of 128 rows each.
 constexpr int kCUs = 256;
@@ -224,7 +234,9 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
   int tile_x = blockIdx.x, tile_y = blockIdx.y, half = -1;
   if (MI == 8 && WIDE)
     big_tile_of_block(p, BN, tile_x, tile_y, half);
-  else if (!GROUPED)
+  else if (GROUPED)
+    expert_tile_of_block(tile_x, tile_y);
+  else
     tile_of_block<BM >= 256 ? 4 : 8>(tile_x, tile_y);
   const int n0 = tile_x * BN;
   const int wm = WIDE ? 0 : (wave >> 1) * (32 * MI), wn = WIDE ? wave * WN : (wave & 1) * WN;
@@ -239,7 +251,7 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
   size_t w_off = 0, s_off = 0;
   int* const row_pair = reinterpret_cast<int*>(lds + XS_BYTES);  // grouped: pair index of every row of the tile
   if (GROUPED) {
-    const int32_t* ti = p.tiles + 3 * (size_t)blockIdx.y;
+    const int32_t* ti = p.tiles + 3 * (size_t)tile_y;
     const int e = ti[0];
     if (e < 0) return;  // whole workgroup: tile slot not in use
     m0 = 0;
@@ -608,6 +620,63 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);  // the repeats requested past the end: landed before
   };                                     // the staging below reuses this memory
+  // Experts: the same loop with the codes of a 128-byte line of a weight row requested together.  Requested a K step apart, every step
+  // asked the L2 for the line again, and of 64 workgroups' lines and rows beside one another it had lost half by then: 545 MB moved for the 230 of a
+  // pair of 128 experts of 768x2048 (now 370).  us, with the order of expert_tile_of_block:
+  // gate/up of 128 experts of 1536x4096 under 1023 tokens 499 -> 380, 8 bits 547 -> 507, of 768x2048 under 300 | 1023 | 4096 85 | 112 | 287 -> 80 | 108 | 248, of
+  // 32 experts of 2048x4096 under 700 161 -> 142.  Down products of 96 rows and fewer, and of 8 bits, are 1 to 5 % slower so and keep the other loop; of more
+  // rows 2048x768 under 4096 tokens 145 -> 136.  What bounds it: vector instructions and products, 45 % of the time each, which two workgroups a CU
+  // do not overlap, and the requests' way (a wave's 1 KB of codes is 64 accesses to the L1; by adjacent lanes and turned in registers 32, at no gain).
+  auto ring_lines = [&](auto ni) {
+    constexpr int NI = decltype(ni)::value;
+    constexpr int G = BITS == 8 || NI > 3 ? 2 : 4;    // steps whose codes are requested together (8 bits: a line; 4 bits: half of one, where there are no more registers)
+    constexpr int S = 2 * G, R = 2 * G * (BITS / 4);  // register stages; requests at a time
+    WStage wq[S];
+    SBlock sbc, sbn;
+    const int last = ke - BK;
+    load_sb(sbn, kb >> 8);
+#pragma unroll
+    for (int r = 0; r < R; ++r) load_w1(wq[r / (BITS / 4) % G], min(kb + r / (BITS / 4) % G * BK, last), r / (R / 2), r % (BITS / 4));
+#pragma unroll
+    for (int u = 0; u < 3; ++u) load_x(u, min(kb + u * BK, last), NI);
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    __syncthreads();
+    read_first(ni, wq[0], 0, sbn, 0);
+    for (int k0 = kb; k0 < ke; k0 += 4 * BK) {
+      sbc = sbn;
+      load_sb(sbn, min((k0 >> 8) + 1, (ke >> 8) - 1));
+      auto step = [&](auto at) {
+        constexpr int u = decltype(at)::value, s = u % S;
+        constexpr auto codes = [](int v) { return v % G == 0 ? R : 0; };  // requested in step v
+        const int kx = min(k0 + (u + 3) * BK, last);
+        multiply_on(ni, wq[s], wq[(s + 1) % S], u, (u + 1) & 3, u < 3 ? sbc : sbn, (u + 1) & 3, [&](int slot) {
+          // activations first: the wait at the step's end is for those of the step before, and leaves codes in flight
+#pragma unroll
+          for (int r = 0; r < NI; ++r)
+            if (slot == r) load_x1((u + 3) & 3, kx, r);
+#pragma unroll
+          for (int r = 0; r < codes(u); ++r)
+            if (slot == NI + r * (7 * NI) / R) {
+              const int q = r / (BITS / 4) % G;
+              load_w1(wq[(s + G + q) % S], min(k0 + (u + G + q) * BK, last), r / (R / 2), r % (BITS / 4));
+            }
+        });
+        // Tile k+2 is in LDS behind the barrier; still out may be what was requested behind it
+        wait_vm(std::integral_constant<int, codes((u + 3) & 3) + (u == 0 ? 4 : 0) + NI + codes(u)>{});
+        asm volatile("s_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      step(std::integral_constant<int, 0>{});
+      step(std::integral_constant<int, 1>{});
+      step(std::integral_constant<int, 2>{});
+      step(std::integral_constant<int, 3>{});
+      if (S == 8) {  // (a loop of two blocks, left after either, holds the sums twice)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) wq[u] = wq[S / 2 + u];
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // the repeats requested past the end: landed before
+  };                                     // the staging below reuses this memory
   if constexpr (RING) {
     // a tile with fewer rows multiplies only the row blocks that it has
     const int rows = m_end - m0;
@@ -617,10 +686,16 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
       else if (rows > 64) ring(std::integral_constant<int, 4>{});
       else ring(std::integral_constant<int, 2>{});
     } else if constexpr (GROUPED) {
-      if (rows > 96) ring(std::integral_constant<int, 4>{});
-      else if (rows > 64) ring(std::integral_constant<int, 3>{});
-      else if (rows > 32) ring(std::integral_constant<int, 2>{});
-      else ring(std::integral_constant<int, 1>{});
+      auto run = [&](auto ni) {
+        if constexpr (PAIR || (BITS == 4 && decltype(ni)::value == 4))
+          ring_lines(ni);
+        else
+          ring(ni);
+      };
+      if (rows > 96) run(std::integral_constant<int, 4>{});
+      else if (rows > 64) run(std::integral_constant<int, 3>{});
+      else if (rows > 32) run(std::integral_constant<int, 2>{});
+      else run(std::integral_constant<int, 1>{});
     } else {
       ring(std::integral_constant<int, MI>{});
     }

@@ -117,6 +117,27 @@ def test_grouped_gemm_multiplies_the_rows_of_its_tile(device, rows, K, bits):
         check(y[sel, 0], x[sel, 0], weights64(qs[e]), what=f"expert {e} of {len(sel)} rows")
 
 
+@pytest.mark.parametrize("K,bits", [(256, 4), (512, 4), (768, 4), (1280, 4), (256, 8), (768, 8)])
+def test_grouped_pair_has_the_bits_of_two_products(device, K, bits):
+    """Gate and up products of experts of 1 to 300 rows in one launch, whose loop requests its codes in another order (one block of four steps of K, an
+    odd and an even number of them), more row tiles than XCDs and no multiple of their number, against the two products."""
+    counts, N = [1, 300, 31, 0, 33, 64, 65, 128, 96, 97, 129], 264
+    E = len(counts)
+    gate, up = (QuantizedWeight(*(torch.stack(t) for t in zip(*((q.weight, q.scales, q.biases) for q in (packed(N, K, bits, 100 * s + e, device) for e in range(E))))), bits) for s in (1, 2))
+    idx = torch.cat([torch.full((n,), e) for e, n in enumerate(counts)]).to(torch.int32)
+    idx = idx[torch.randperm(len(idx), generator=torch.Generator().manual_seed(K))].to(device)[:, None].contiguous()
+    x = torch.randn(len(idx), 1, K, device=device, generator=torch.Generator(device=device).manual_seed(K)).bfloat16()
+    ws = ops.moe_group(idx, E)
+    y = ops.grouped_qmm_swiglu(x, gate, up, ws, 1)
+    a, b = ops.grouped_qmm(x, gate, ws, 1), ops.grouped_qmm(x, up, ws, 1)
+    assert torch.equal(y.view(torch.int16), ops.swiglu(a, b).view(torch.int16))
+    for e in range(E):
+        sel = (idx[:, 0] == e).nonzero()[:, 0]
+        one = QuantizedWeight(gate.weight[e], gate.scales[e], gate.biases[e], bits)
+        if len(sel):
+            check(a[sel, 0], x[sel, 0], weights64(one), what=f"expert {e} of {len(sel)} rows")
+
+
 # prompts whose last key tile ends with the cache or inside it, queries that see none of a workgroup's later
 # tiles (300 behind 40: the second half of a split starts past the first queries), one and several heads
 # per kv head, both head sizes, a scale of either sign, scores that reach far above the first tile's
