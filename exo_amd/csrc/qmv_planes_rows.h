@@ -26,7 +26,7 @@ constexpr int rows_lds(int K) {
   return K / 64 * kPlaneGroup * (TOK / 4) + TOK * (K / 64 + 4) * (int)sizeof(GroupSum) + 2 * kRowsTiles<TOK> * kRowsWaves * TOK * 16 * 4;
 }
 
-// K = 2048 * XS; p.slots: tiles of 16 rows (a pair: 8 of each matrix), 8 bits: of p.tile_rows, where the product's other columns repeat the
+// K = 2048 * XS; p.slots: tiles of 16 rows (a pair: 8 of each matrix), 8 bits: of p.spw, where the product's other columns repeat the
 // last one
 template <int BITS, int NMAT, int XS, int TOK>
 __global__ __launch_bounds__(64 * kRowsWaves) void qmv_planes_rows_kernel(const QmvParams p) {
@@ -48,7 +48,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void qmv_planes_rows_kernel(const 
   __shared__ float s_ss[kRowsWaves];
   __shared__ int s_bad[kRowsWaves];
 
-  const int tiles = p.slots, rows = BITS == 8 ? p.tile_rows : RPT;
+  const int tiles = p.slots, rows = BITS == 8 ? p.spw : RPT;
   const int base = tiles / (int)gridDim.x, rem = tiles - base * (int)gridDim.x;
   const int t0 = (int)blockIdx.x * base + min((int)blockIdx.x, rem);
   const int t1 = t0 + base + ((int)blockIdx.x < rem ? 1 : 0);
@@ -66,7 +66,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void qmv_planes_rows_kernel(const 
     }
   }
 
-  const int mat = NMAT == 2 ? n >> 3 : 0, r_in = BITS == 8 ? min(n % RPT, p.tile_rows - 1) : n % RPT;
+  const int mat = NMAT == 2 ? n >> 3 : 0, r_in = BITS == 8 ? min(n % RPT, p.spw - 1) : n % RPT;
   const size_t row_bytes = (size_t)p.wpr * 4;
   const char* const wm = reinterpret_cast<const char*>(mat ? p.w[NMAT - 1] : p.w[0]) + wave * (GW * 8 * BITS) + q * 16;
   const bf16_t* const sm = (mat ? p.s[NMAT - 1] : p.s[0]) + wave * GW;
