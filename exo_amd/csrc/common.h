@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 typedef uint16_t bf16_t;  // raw bfloat16 bit pattern
 
 typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2_t;
@@ -83,6 +85,53 @@ __device__ __forceinline__ float wave_sum(float v) {
   v += dpp_get<0xB1, 0xf>(v);   // quad_perm [1,0,3,2]
   return v;
 }
+// ---- exchanges between lanes whose numbers differ in one bit, without the LDS crossbar (the same values, and for two lanes' sum the same
+// bits, as with __shfl_xor, which is one or two hundred cycles to the result where these are ten)
+template <int BIT>
+__device__ __forceinline__ uint32_t lane_xor_bits(uint32_t v) {
+  static_assert(BIT == 1 || BIT == 2 || BIT == 4 || BIT == 8 || BIT == 16 || BIT == 32, "one bit of the lane's number");
+  auto dpp = [](uint32_t x, auto ctrl) __attribute__((always_inline)) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, decltype(ctrl)::value, 0xf, 0xf, false);
+  };
+  if constexpr (BIT == 1) return dpp(v, std::integral_constant<int, 0xB1>{});
+  if constexpr (BIT == 2) return dpp(v, std::integral_constant<int, 0x4E>{});
+  if constexpr (BIT == 4) return dpp(dpp(v, std::integral_constant<int, 0x141>{}), std::integral_constant<int, 0x1B>{});  // 7 - i, then i ^ 3
+  if constexpr (BIT == 8) return dpp(v, std::integral_constant<int, 0x128>{});                                             // row_ror:8
+  if constexpr (BIT >= 16) {
+    const auto t = BIT == 16 ? __builtin_amdgcn_permlane16_swap(v, v, false, false) : __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    const uint32_t low = t[0], high = t[1];  // of the lanes with the bit clear, and set, in both
+    return threadIdx.x & BIT ? low : high;
+  }
+}
+template <int BIT>
+__device__ __forceinline__ float lane_xor(float v) {
+  return __builtin_bit_cast(float, lane_xor_bits<BIT>(__builtin_bit_cast(uint32_t, v)));
+}
+// a lane's value and the other's: {with the bit clear, with it set}, or the other way round
+template <int BIT>
+__device__ __forceinline__ void lane_pair(float v, float& a, float& b) {
+  if constexpr (BIT >= 16) {
+    const uint32_t u = __builtin_bit_cast(uint32_t, v);
+    const auto t = BIT == 16 ? __builtin_amdgcn_permlane16_swap(u, u, false, false) : __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    const uint32_t low = t[0], high = t[1];
+    a = __builtin_bit_cast(float, low), b = __builtin_bit_cast(float, high);
+  } else {
+    a = v, b = lane_xor<BIT>(v);
+  }
+}
+template <int BIT>
+__device__ __forceinline__ float add_across(float v) {
+  float a, b;
+  lane_pair<BIT>(v, a, b);
+  return a + b;
+}
+template <int BIT>
+__device__ __forceinline__ float max_across(float v) {
+  float a, b;
+  lane_pair<BIT>(v, a, b);
+  return fmaxf(a, b);
+}
+
 // sum over the wave; the total lands in lane 63
 __device__ __forceinline__ float wave_sum_to_lane63(float v) {
   v += dpp_get<0xB1, 0xf>(v);   // quad_perm [1,0,3,2]

@@ -382,6 +382,18 @@ __global__ __launch_bounds__(256) void moe_combine_vec_kernel(const bf16_t* __re
 // Stage 2: one wave per row merges the blocks.
 constexpr int kArgBlocks = 64;
 
+// the wave's largest value and, of equal ones, the first index, in every lane
+template <int BIT = 32>
+__device__ __forceinline__ void first_of_largest(float& mx, int& mi) {
+  const float ov = lane_xor<BIT>(mx);
+  const int oi = (int)lane_xor_bits<BIT>((uint32_t)mi);
+  if (ov > mx || (ov == mx && oi < mi)) {
+    mx = ov;
+    mi = oi;
+  }
+  if constexpr (BIT > 1) first_of_largest<BIT / 2>(mx, mi);
+}
+
 __global__ __launch_bounds__(256) void argmax_stage1(const bf16_t* __restrict__ logits,
                                                      float* __restrict__ ws, int V) {
   __shared__ float smax[4], ssum[4];
@@ -424,15 +436,7 @@ __global__ __launch_bounds__(256) void argmax_stage1(const bf16_t* __restrict__ 
       }
     }
   }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const float ov = __shfl_xor(mx, o, 64);
-    const int oi = __shfl_xor(mi, o, 64);
-    if (ov > mx || (ov == mx && oi < mi)) {
-      mx = ov;
-      mi = oi;
-    }
-  }
+  first_of_largest(mx, mi);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (lane == 0) {
     smax[wave] = mx;
@@ -477,15 +481,7 @@ __global__ __launch_bounds__(64) void argmax_stage2(const float* __restrict__ ws
   float mx = s[0];
   int mi = __float_as_int(s[1]);
   const float bm = mx, bs = s[2];
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const float ov = __shfl_xor(mx, o, 64);
-    const int oi = __shfl_xor(mi, o, 64);
-    if (ov > mx || (ov == mx && oi < mi)) {
-      mx = ov;
-      mi = oi;
-    }
-  }
+  first_of_largest(mx, mi);
   float se = (bm > -INFINITY) ? bs * expf(bm - mx) : 0.f;
   se = wave_sum(se);
   if (lane == 0) {

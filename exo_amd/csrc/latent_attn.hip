@@ -231,8 +231,7 @@ __global__ __launch_bounds__(kRowThreads) void latent_rows_kernel(const Params p
         x[e] = j * KT + wave * 16 + 4 * g + e <= pos ? (s0[e] + s1[e]) * sc : -INFINITY;
         mx = fmaxf(mx, x[e]);
       }
-      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      mx = max_across<32>(max_across<16>(mx));
     }
     if (wave < SW && g == 0) wm[wave][r] = mx;
     __syncthreads();
@@ -248,8 +247,7 @@ __global__ __launch_bounds__(kRowThreads) void latent_rows_kernel(const Params p
         x[e] = __builtin_amdgcn_exp2f(x[e] - mn);
         sum += x[e];
       }
-      sum += __shfl_xor(sum, 16, 64);
-      sum += __shfl_xor(sum, 32, 64);
+      sum = add_across<32>(add_across<16>(sum));
       char* dst = pw + r * kPRow + (wave * 16 + 4 * g) * ES;
       if (ES == 2) {
         float b[4];

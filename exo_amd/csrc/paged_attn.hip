@@ -801,8 +801,7 @@ __global__ __launch_bounds__(64 * kRowWaves) void paged_rows_kernel(const Params
     }
     float a = 1.f;
     if (!SIGMOID) {
-      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      mx = max_across<32>(max_across<16>(mx));
       const float mn = fmaxf(m, mx);  // finite: a dealt tile holds a visible key
       a = __builtin_amdgcn_exp2f(m - mn);
       float sum = 0.f;
@@ -812,8 +811,7 @@ __global__ __launch_bounds__(64 * kRowWaves) void paged_rows_kernel(const Params
         x1[e] = __builtin_amdgcn_exp2f(x1[e] - mn);
         sum += x0[e] + x1[e];
       }
-      sum += __shfl_xor(sum, 16, 64);
-      sum += __shfl_xor(sum, 32, 64);
+      sum = add_across<32>(add_across<16>(sum));
       l = l * a + sum;
       m = mn;
     }
@@ -1005,7 +1003,7 @@ __global__ __launch_bounds__(256, DK > 128 ? 1 : 2) void paged_prompt_kernel(con
 #pragma unroll
       for (int i = 0; i < 4; ++i) ss += bf_lo(w[i]) * bf_lo(w[i]) + bf_hi(w[i]) * bf_hi(w[i]);
     }
-    ss += __shfl_xor(ss, 32, 64);
+    ss = add_across<32>(ss);
     if (p.unit) {
       const float inv = 1.f / sqrtf(ss / p.D + p.eps);
 #pragma unroll
@@ -1134,7 +1132,7 @@ __global__ __launch_bounds__(256, DK > 128 ? 1 : 2) void paged_prompt_kernel(con
       }
     float mr = 0.f, mn = 0.f, al = 1.f;
     if (!SIGMOID) {
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      mx = max_across<32>(mx);
       mn = fmaxf(m, mx), mr = mn == -INFINITY ? 0.f : mn;  // (a query may see none of the tile)
       al = __builtin_amdgcn_exp2f(m - mr);
     }
@@ -1161,7 +1159,7 @@ __global__ __launch_bounds__(256, DK > 128 ? 1 : 2) void paged_prompt_kernel(con
         pl[ks][st] = uint4{pack_bf2(b[0], b[1]), pack_bf2(b[2], b[3]), pack_bf2(b[4], b[5]), pack_bf2(b[6], b[7])};
       }
     if (!SIGMOID) {
-      sum += __shfl_xor(sum, 32, 64);
+      sum = add_across<32>(sum);
       l = l * al + sum;
       m = mn;
     }

@@ -262,8 +262,7 @@ __global__ __launch_bounds__(MSETS == 4 ? 512 : 1024) void qmv_quad_kernel(const
 #pragma unroll
         for (int t = 0; t < 4; ++t) ss += sumsq_word<BITS>(xraw[set][t]);
         ss = sum_blocks_row16(ss);
-        ss += __shfl_xor(ss, 16, 64);
-        ss += __shfl_xor(ss, 32, 64);
+        ss = add_across<32>(add_across<16>(ss));
         if (lane < 4) s_part[wave][set * 4 + lane] = ss;
       }
       __syncthreads();

@@ -991,10 +991,21 @@ __global__ __launch_bounds__(256) void recur_step_kernel(const Rec p, int cols) 
     if (d0 + kAhead * rpp < D) load_state(d0 + kAhead * rpp);
   }
   // over the wave's rows (lanes with the same columns), then over the waves
-  for (int step = lpr; step < 64; step *= 2) {
+  auto rows = [&](auto step) __attribute__((always_inline)) {
+    constexpr int S = decltype(step)::value;
+    if (lpr > S) return;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] += __shfl_xor(o[e], step, 64);
-  }
+    for (int e = 0; e < 4; ++e) {
+      const float v = o[e];
+      o[e] = add_across<S>(v);
+    }
+  };
+  rows(std::integral_constant<int, 1>{});
+  rows(std::integral_constant<int, 2>{});
+  rows(std::integral_constant<int, 4>{});
+  rows(std::integral_constant<int, 8>{});
+  rows(std::integral_constant<int, 16>{});
+  rows(std::integral_constant<int, 32>{});
   if ((tid & 63) < lpr) *reinterpret_cast<floatx4*>(red + (tid >> 6) * cols + cq) = o;
   __syncthreads();
   if (tid < cols && e0 + tid < p.vdim) {

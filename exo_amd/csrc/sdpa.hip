@@ -102,15 +102,28 @@ __device__ __forceinline__ float group_sum_lpk(float d) {
     d += dpp_f<0x140>(d);  // row_mirror
     return d;
   }
-#pragma unroll
-  for (int off = LPK >> 1; off > 0; off >>= 1) d += __shfl_xor(d, off, 64);
-  return d;
+  static_assert(LPK == 16 || LPK == 8, "heads of 128 or 64");
+  return add_across<1>(add_across<2>(add_across<4>(d)));
+}
+// Over the lane groups of a wave, in every one of them.  A call's chain is one of latencies (a wave has a few tiles): through the crossbar
+// (__shfl_xor, about 100 cycles a round) the maximum and the sums of 64-wide heads were six dependent rounds, and the launch 5.94 us
+// where it is 5.68; a pass of 16 layers of 64-wide heads 3380 -> 3354 us, of 32 layers of 128-wide ones 3532 -> 3520 (each the mean over five
+// offsets of the kernels in memory).
+template <int LPK>
+__device__ __forceinline__ float groups_sum(float x, float scale) {  // of x * scale; a lane's own product is not rounded
+  float v = fmaf(x, scale, lane_xor<LPK>(x * scale));
+  if (LPK == 8) v = add_across<16>(v);
+  return add_across<32>(v);
+}
+template <int LPK>
+__device__ __forceinline__ float groups_max(float v) {
+  if (LPK == 8) v = max_across<8>(v);
+  return max_across<32>(max_across<16>(v));
 }
 // value of the lane LPK/2 away inside the lane group (the RoPE partner)
 template <int LPK>
 __device__ __forceinline__ float partner_lpk(float v) {
-  if (LPK == 16) return dpp_f<0x128>(v);  // row_ror:8
-  return __shfl_xor(v, LPK / 2, 64);
+  return lane_xor<LPK / 2>(v);
 }
 
 // one float, or two in one request
@@ -460,20 +473,11 @@ __global__ __launch_bounds__(kThreads) void sdpa_kernel(const SdpaParams p) {
   // merge the KPI lane groups of the wave
 #pragma unroll
   for (int g = 0; g < G; ++g) {
-    float mw = m[g];
-#pragma unroll
-    for (int off = LPK; off < 64; off <<= 1) mw = fmaxf(mw, __shfl_xor(mw, off, 64));
+    const float mw = groups_max<LPK>(m[g]);
     const float sc = (m[g] == -INFINITY) ? 0.f : __expf(m[g] - mw);
-    float lw = l[g] * sc;
+    const float lw = groups_sum<LPK>(l[g], sc);
 #pragma unroll
-    for (int off = LPK; off < 64; off <<= 1) lw += __shfl_xor(lw, off, 64);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      float ov = o[g][e] * sc;
-#pragma unroll
-      for (int off = LPK; off < 64; off <<= 1) ov += __shfl_xor(ov, off, 64);
-      o[g][e] = ov;
-    }
+    for (int e = 0; e < 8; ++e) o[g][e] = groups_sum<LPK>(o[g][e], sc);
     if (sub == 0) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) red[wave][g][sl * 8 + e] = o[g][e];
@@ -718,20 +722,11 @@ __global__ __launch_bounds__(64 * NW) void sdpa_tiles_kernel(const SdpaParams p)
   // merge the KPI lane groups of the wave
 #pragma unroll
   for (int g = 0; g < G; ++g) {
-    float mw = m[g];
-#pragma unroll
-    for (int off = LPK; off < 64; off <<= 1) mw = fmaxf(mw, __shfl_xor(mw, off, 64));
+    const float mw = groups_max<LPK>(m[g]);
     const float sc = (m[g] == -INFINITY) ? 0.f : __expf(m[g] - mw);
-    float lw = l[g] * sc;
+    const float lw = groups_sum<LPK>(l[g], sc);
 #pragma unroll
-    for (int off = LPK; off < 64; off <<= 1) lw += __shfl_xor(lw, off, 64);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      float ov = o[g][e] * sc;
-#pragma unroll
-      for (int off = LPK; off < 64; off <<= 1) ov += __shfl_xor(ov, off, 64);
-      o[g][e] = ov;
-    }
+    for (int e = 0; e < 8; ++e) o[g][e] = groups_sum<LPK>(o[g][e], sc);
     if (sub == 0) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) red[wave][g][sl * 8 + e] = o[g][e];
@@ -951,7 +946,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves<G>) void sdpa_decode_mfma_kernel(co
       sc[e] = x;
       mx = fmaxf(mx, x);
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = max_across<32>(mx);
     const float m_new = fmaxf(m_run, mx);  // finite: key 0 of the tile is real
     const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
     float sum = 0.f;
@@ -971,7 +966,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves<G>) void sdpa_decode_mfma_kernel(co
         pb[st].w = pack_bf2(pr[8 * st + 6], pr[8 * st + 7]);
       }
     }
-    sum += __shfl_xor(sum, 32, 64);
+    sum = add_across<32>(sum);
     l_run = l_run * alpha + sum;
     m_run = m_new;
 #pragma unroll
@@ -1007,7 +1002,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves<G>) void sdpa_decode_mfma_kernel(co
       part = dot2_bf16(qv.z, kn4.z, part);
       part = dot2_bf16(qv.w, kn4.w, part);
     }
-    const float sv = (part + __shfl_xor(part, 32, 64)) * scale_log2e;
+    const float sv = add_across<32>(part) * scale_log2e;
     const float m_new = fmaxf(m_run, sv);
     const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
     const float pn = __builtin_amdgcn_exp2f(sv - m_new);
@@ -1107,11 +1102,14 @@ int launch_sdpa(const SdpaParams& p0, hipStream_t st) {
     switch (G) {
       case 1:
         // few splits (many kv-head groups): eight waves per workgroup halve a wave's tiles
-        // (64 query / 4 kv heads at 4100 keys: 13.4 -> 12.4 us; with 8 splits four waves win)
-        if (p.splits <= 4 && kTileWaves == 4)
-          sdpa_tiles_kernel<D, 1, FUSED, 8><<<grid, 512, 0, st>>>(p);
-        else
+        // (64 query / 4 kv heads at 4100 keys: 13.4 -> 12.4 us; with 8 splits four waves win).
+        // The order of the two calls is the order of the kernels in memory: a layer's kernels are nearly as large as the instruction cache, and the
+        // one of four waves here begins where it displaces the fewest of the products' lines (a pass of 32 layers of 4096 columns in 4 bits 3505 us,
+        // at the other offsets to 16 KB 3503 to 3560).
+        if (p.splits > 4 || kTileWaves != 4)
           sdpa_tiles_kernel<D, 1, FUSED, kTileWaves><<<grid, 64 * kTileWaves, 0, st>>>(p);
+        else
+          sdpa_tiles_kernel<D, 1, FUSED, 8><<<grid, 512, 0, st>>>(p);
         break;
       case 2: sdpa_tiles_kernel<D, 2, FUSED, kTileWaves><<<grid, 64 * kTileWaves, 0, st>>>(p); break;
       case 4: sdpa_tiles_kernel<D, 4, FUSED, kTileWaves><<<grid, 64 * kTileWaves, 0, st>>>(p); break;

@@ -204,7 +204,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, SPLIT ? 1 : 2) void fa_prefill_k
   // error 2.2e-3 -> 2.35e-3 under scores of unit width, 1.9e-3 -> 2.4e-3 under twice that.)
   auto settle = [&](float mx) {
     if (__builtin_amdgcn_ballot_w64(mx > m_run) == 0) return;  // (at the first tile: -infinity)
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = max_across<32>(mx);
     const float m_new = fmaxf(m_run, mx);
     // (a query that has seen no key yet keeps -infinity as its maximum and 0 as its reference)
     const float ref = m_new == -INFINITY ? 0.f : m_new * p.scale_log2e;
@@ -363,7 +363,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, SPLIT ? 1 : 2) void fa_prefill_k
   }
   if (SPLIT) __builtin_amdgcn_s_waitcnt(0x0F70);  // the repeats requested past the end
   float l_run = l0 + l1;
-  l_run += __shfl_xor(l_run, 32, 64);
+  l_run = add_across<32>(l_run);
   if (SPLIT) {
     // the second team's sums: through LDS (lane-contiguous floats per register), merged into
     // the first team's, which goes on alone
