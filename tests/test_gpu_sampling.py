@@ -207,6 +207,30 @@ def test_sample_modes_and_reuse(device):
     np.testing.assert_allclose(ds.lse.cpu().numpy()[:rows], lse.cpu().numpy(), rtol=1e-6)
 
 
+@pytest.mark.parametrize("V", [19, 4099, 131072, 131080])
+def test_rows_finish_by_their_last_slice_or_by_one(device, V):
+    """Drawn rows (finished by the slice that arrives last) between greedy ones (by one workgroup), without the top list, and greedy
+    rows by themselves: each against the oracle, several steps over one workspace."""
+    settings = [SamplerSettings(temperature=0.0), SamplerSettings(temperature=0.8, top_p=0.9, min_p=0.0, seed=5),
+                SamplerSettings(temperature=0.0), SamplerSettings(temperature=1.1, min_p=0.0, seed=6),
+                SamplerSettings(temperature=0.7, min_p=0.1, top_k=12, seed=7)]
+    rows = len(settings)
+    ds = DeviceSampler(rows, V, device)
+    for i, s in enumerate(settings):
+        ds.set_row(i, s, [])
+    for step in range(4):
+        logits = rand_bf16((rows, V), seed=V + step, scale=2.0)
+        before = ds.draws.cpu().numpy().astype(np.uint32).tolist()
+        ds.sample(t_bf16(logits, device), rows, MODE_DRAW | MODE_TABLE)
+        torch.cuda.synchronize()
+        _check_rows(ds, logits, settings, [[]] * rows, before, want_top=False)
+        ds.sample(t_bf16(logits[:1], device), 1, 0)
+        torch.cuda.synchronize()
+        _check_rows(ds, logits[:1], settings[:1], [[]], before, want_top=False)
+    after = ds.draws.cpu().numpy().tolist()
+    assert after == [0 if s.temperature == 0 else 4 for s in settings]
+
+
 def test_top_logprobs_of_flat_and_tied_rows(device):
     """Rows with thousands of tokens at the 20th largest value: an all-equal row (a zeroed or
     saturated head), a row of three distinct values, a row with 12 tokens above a plateau that
