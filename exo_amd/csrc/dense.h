@@ -113,6 +113,7 @@ __device__ __forceinline__ float finish(float v, size_t m, int n, const Epilogue
 
 // 16 bytes as one vector value (a struct copy of a uint4 may end up in scratch memory)
 typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4_t;
+typedef __attribute__((__vector_size__(2 * sizeof(uint32_t)))) uint32_t u32x2_t;
 __device__ __forceinline__ uint4 load16(const void* p) {
   return __builtin_bit_cast(uint4, *reinterpret_cast<const u32x4_t*>(p));
 }

@@ -26,6 +26,11 @@
 //   tiles that hold a visible key are dealt (kept first tokens, then the window).  Splits meet
 //   through device-scope partials and an arrival counter.  FUSE: the launch also normalises and
 //   stores the row's own key and value (the workgroup that owns the last tile does).
+//   What bounds a launch of short contexts is a chain of ways through memory by a few waves: the arguments, position and slot, the page, the
+//   tile, the partials, their counter and the partials again.  So the arguments come in one way, a row's channels with its position (plain
+//   ones 16 bytes a thread, not element by element), the page of a wave's first tile behind that, a value column's eight keys in one
+//   request, and partials in requests of up to 16 bytes, a thread to every run of columns.  Four rows of 32 / 4 heads of 128, up to 700 keys: 15.9 -> 12.9 us
+//   (48 keys of 64 in float32, one split: 8.8 -> 9.0).
 // paged_prepare_kernel: norm over whole projections, rotation and value mixing of all rows of a step
 //   ahead of the other two (queries in place, keys and values into the pool); a step of single tokens
 //   does the same inside paged_rows_kernel.  Convolved queries go to a buffer of their own, since other rows
@@ -74,7 +79,7 @@ struct Params {
   float* ws;
   int* counters;
   float scale, eps, cap, mix;  // cap 0: none
-  int n, H, G, D, E, ldq, ldk, ldv, ldo, ldg, ldmix, max_pages, size, keep, unit, whole, rot, nsplit, gsz, hgroups;
+  int n, H, G, D, E, ldq, ldk, ldv, ldo, ldg, ldmix, max_pages, size, keep, unit, whole, rot, nsplit, gsz, hgroups, group;  // (the last four: of the rows' launch)
   int ldog, ldqo, mpages, pool, one, half, taps, vkeys;  // pool 0, taps 0: none; vkeys: values are keys
   float amp;
 };
@@ -100,27 +105,29 @@ __device__ __forceinline__ Params only(Params p) {
   return p;
 }
 
-__device__ __forceinline__ void st_dev(float* p, float v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// W floats at a multiple of four bytes, written and read at device scope in one request
+constexpr int kDeviceScope = 16;  // (the sc1 bit)
+template <int W>
+struct alignas(W * 4) Run {
+  float v[W];
+};
+template <int W>
+__device__ __forceinline__ void st_dev(__amdgpu_buffer_rsrc_t to, uint32_t voff, uint32_t soff, const Run<W>& r) {
+  if constexpr (W == 4)
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, r), to, voff, soff, kDeviceScope);
+  else if constexpr (W == 2)
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2_t, r), to, voff, soff, kDeviceScope);
+  else
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, r), to, voff, soff, kDeviceScope);
 }
-// two floats, where they lie at a multiple of eight bytes in one request
-template <bool EIGHT>
-__device__ __forceinline__ void st_dev2(float* p, float a, float b) {
-  if (EIGHT) {
-    __hip_atomic_store(reinterpret_cast<uint64_t*>(p), __builtin_bit_cast(uint64_t, make_float2(a, b)), __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
-  } else {
-    st_dev(p, a);
-    st_dev(p + 1, b);
-  }
-}
-template <bool EIGHT>
-__device__ __forceinline__ float2 ld_dev2(const float* p) {
-  if (EIGHT)
-    return __builtin_bit_cast(float2, __hip_atomic_load(reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED,
-                                                        __HIP_MEMORY_SCOPE_AGENT));
-  return make_float2(__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
-                     __hip_atomic_load(p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+template <int W>
+__device__ __forceinline__ Run<W> ld_dev(__amdgpu_buffer_rsrc_t from, uint32_t voff, uint32_t soff) {
+  if constexpr (W == 4)
+    return __builtin_bit_cast(Run<W>, __builtin_amdgcn_raw_buffer_load_b128(from, voff, soff, kDeviceScope));
+  else if constexpr (W == 2)
+    return __builtin_bit_cast(Run<W>, __builtin_amdgcn_raw_buffer_load_b64(from, voff, soff, kDeviceScope));
+  else
+    return __builtin_bit_cast(Run<W>, __builtin_amdgcn_raw_buffer_load_b32(from, voff, soff, kDeviceScope));
 }
 
 // whole blocks that lie before the window of a query at pos
@@ -156,18 +163,30 @@ __device__ __forceinline__ float column_gate(const Params& p, int row, int c) {
   return p.ogate ? 1.f / (1.f + expf(-Elem<T>::load(reinterpret_cast<const T*>(p.ogate)[(size_t)row * p.ldog + c]))) : 1.f;
 }
 
-// one wave: src[0..D) / rms * gain -> dst (element type T, float32 arithmetic)
-template <typename T>
-__device__ __forceinline__ void unit_row(const T* __restrict__ src, T* dst, int D, int unit, float eps,
-                                         const float* __restrict__ gain, int lane) {
-  float ss = 0.f;
-  for (int d = lane; d < D; d += 64) {
-    const float v = Elem<T>::load(src[d]);
-    ss += v * v;
+// one wave: src[0..D) / rms * gain -> dst (element type T, float32 arithmetic), in two steps: what it needs is requested, and much later
+// turned into the row
+template <typename T, int DMAX>
+struct UnitRow {
+  T x[DMAX / 64];
+  __device__ __forceinline__ void request(const T* __restrict__ src, int D, int lane) {
+#pragma unroll
+    for (int i = 0; i < DMAX / 64; ++i)
+      if (lane + 64 * i < D) x[i] = src[lane + 64 * i];
   }
-  const float inv = unit ? 1.f / sqrtf(wave_total(ss) / D + eps) : 1.f;
-  for (int d = lane; d < D; d += 64) dst[d] = Elem<T>::make(Elem<T>::load(src[d]) * inv * (gain ? gain[d] : 1.f));
-}
+  __device__ __forceinline__ void put(T* dst, int D, int unit, float eps, const float* __restrict__ gain, int lane) const {
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < DMAX / 64; ++i)
+      if (lane + 64 * i < D) {
+        const float v = Elem<T>::load(x[i]);
+        ss += v * v;
+      }
+    const float inv = unit ? 1.f / sqrtf(wave_total(ss) / D + eps) : 1.f;
+#pragma unroll
+    for (int i = 0; i < DMAX / 64; ++i)
+      if (lane + 64 * i < D) dst[lane + 64 * i] = Elem<T>::make(Elem<T>::load(x[i]) * inv * (gain ? gain[lane + 64 * i] : 1.f));
+  }
+};
 
 // this thread's share (of `threads`) of the sum of squares of src[0..n); vec: in vectors
 template <typename T>
@@ -290,21 +309,15 @@ __device__ __forceinline__ T mixed_value(const Params& p, T v, int row, int c) {
   return Elem<T>::make((1.f - p.mix) * Elem<T>::load(v) + p.mix * o);
 }
 
-// key and value of one (row, kv head) into the pool, by one wave each
+// key (turned) and value of one (row, kv head) to their places in the pool, by one wave each
 template <typename T>
-__device__ __forceinline__ void put_key(const Params& p, const Channels<T>& x, int row, int g, int page, int at, int lane, float inv,
-                                        const float2* cs) {
+__device__ __forceinline__ void put_key(const Params& p, const Channels<T>& x, int g, T* dst, int lane, float inv, const float2* cs) {
   const int c0 = (p.H + g) * p.D;
-  T* dst = reinterpret_cast<T*>(p.kpool) + (((size_t)page * p.G + g) * kPage + at) * p.ldk;
-  if (p.whole || p.rot || p.taps)
-    turn_row<T>(p, x, c0, dst, inv, p.kgain ? p.kgain + g * p.D : nullptr, cs, lane);
-  else
-    unit_row<T>(x.raw + c0, dst, p.D, p.unit, p.eps, p.kgain, lane);
+  turn_row<T>(p, x, c0, dst, inv, p.kgain ? p.kgain + g * p.D : nullptr, cs, lane);
   if (p.taps) keep_channels<T>(x, c0, p.D, lane, 64);
 }
 template <typename T>
-__device__ __forceinline__ void put_value(const Params& p, const Channels<T>& x, int row, int g, int page, int at, int lane) {
-  T* dst = reinterpret_cast<T*>(p.vpool) + ((size_t)page * p.G + g) * p.ldv * kPage + at;
+__device__ __forceinline__ void put_value(const Params& p, const Channels<T>& x, int row, int g, T* dst, int lane) {
   if (p.vkeys) {
     for (int d = lane; d < p.E; d += 64) dst[(size_t)d * kPage] = Elem<T>::make(x.at((p.H + g) * p.D + d));
     return;
@@ -624,23 +637,23 @@ struct PTerms<float> {
     lo = __builtin_bit_cast(uint4, floatx4{b[0], b[1], b[2], b[3]});
   }
 };
-// a value column's entries of this lane's keys: 4g.. and 16 + 4g.. of the 32-key tile at v
+// The keys of a 32-key tile at the rows of its two 16-key operands: row i holds key ROWS * (i / 4) + i % 4, in the other OTHER keys on.  A lane's
+// weights are those of rows 4g .. 4g + 3 of both, and with it a value column's entries: in bf16 eight consecutive ones, 16 bytes of the column
+// (with rows in order two halves of 8, twice the requests at half the bytes), in float32 two runs of 16 bytes.
 template <typename T>
 struct VTerms;
 template <>
 struct VTerms<bf16_t> {
-  uint2 a, b;
-  __device__ __forceinline__ void load(const bf16_t* v, int g) {
-    a = *reinterpret_cast<const uint2*>(v + 4 * g);
-    b = *reinterpret_cast<const uint2*>(v + 16 + 4 * g);
-  }
+  static constexpr int ROWS = 8, OTHER = 4;
+  uint4 x;
+  __device__ __forceinline__ void load(const bf16_t* v, int g) { x = load16(v + 8 * g); }
   __device__ __forceinline__ floatx4 mma(const PTerms<bf16_t>& p, floatx4 c) const {
-    const uint4 x{a.x, a.y, b.x, b.y};
     return Elem<bf16_t>::mma16(x, p.lo, Elem<bf16_t>::mma16(x, p.hi, c));
   }
 };
 template <>
 struct VTerms<float> {
+  static constexpr int ROWS = 4, OTHER = 16;
   uint4 a, b;
   __device__ __forceinline__ void load(const float* v, int g) {
     a = *reinterpret_cast<const uint4*>(v + 4 * g);
@@ -656,6 +669,7 @@ constexpr int kRowWaves = 4;
 template <typename T, int DMAX, bool FUSE, int MODE>
 __global__ __launch_bounds__(64 * kRowWaves) void paged_rows_kernel(const Params all) {
   constexpr bool SIGMOID = MODE == kSigmoid;
+  if (MODE == kPlain) request_arguments(all);  // (the other modes' registers do not hold what it makes the compiler keep)
   const Params p = only<MODE>(all);
   constexpr int KST = DMAX * (int)sizeof(T) / 64;  // 64-byte steps over a key
   constexpr int VT = DMAX / 16;                    // 16-row tiles of O^T
@@ -668,12 +682,35 @@ __global__ __launch_bounds__(64 * kRowWaves) void paged_rows_kernel(const Params
   __shared__ int s_last;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int r = lane & 15, g = lane >> 4;
-  const int split = blockIdx.x, kvh = blockIdx.y / p.hgroups, hg = blockIdx.y % p.hgroups;
+  const int split = blockIdx.x, kvh = p.hgroups == 1 ? (int)blockIdx.y : (int)blockIdx.y / p.hgroups, hg = blockIdx.y - kvh * p.hgroups;
   const int row = p.list ? p.list[blockIdx.z] : (int)blockIdx.z;
-  const int group = p.H / p.G;
+  const int group = p.group;
   const int h0 = kvh * group + hg * p.gsz, gs = min(p.gsz, (kvh + 1) * group - h0);
-  const int pos = p.pos[row];
-  const int32_t* table = p.table + (size_t)p.slot[row] * p.max_pages;
+  // The row's channels are requested before its position is known, so that they come with it (each is a way through memory): as they are
+  // (plain: 16 bytes per thread), or to be divided by their RMS.
+  const bool turned = p.whole || p.rot || p.taps;
+  const T* const raw = reinterpret_cast<const T*>(p.qkv) + (size_t)row * p.ldq;
+  constexpr int EPV = 16 / (int)sizeof(T), VPR = DMAX / EPV, NQ = (16 * VPR + 64 * kRowWaves - 1) / (64 * kRowWaves);
+  const bool plain = !turned && !p.unit && p.D % EPV == 0 && ((uintptr_t)raw & 15) == 0;
+  u32x4_t qv[NQ], kv = {0, 0, 0, 0};
+  UnitRow<T, DMAX> qin[16 / kRowWaves], kvin;
+  if (plain) {
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {
+      const int at = threadIdx.x + 64 * kRowWaves * i, h = at / VPR, c = at % VPR * EPV;
+      qv[i] = u32x4_t{0, 0, 0, 0};
+      if (h < gs && c < p.D) qv[i] = *reinterpret_cast<const u32x4_t*>(raw + (h0 + h) * p.D + c);
+    }
+    if (FUSE && wave == kRowWaves - 1 && lane * EPV < p.D) kv = *reinterpret_cast<const u32x4_t*>(raw + (p.H + kvh) * p.D + lane * EPV);
+  } else if (!turned) {
+#pragma unroll
+    for (int i = 0; i < 16 / kRowWaves; ++i)
+      if (wave + kRowWaves * i < gs) qin[i].request(raw + (h0 + wave + kRowWaves * i) * p.D, p.D, lane);
+    if (FUSE && wave == kRowWaves - 1) kvin.request(raw + (p.H + kvh) * p.D, p.D, lane);
+  }
+  if (FUSE && !turned && wave == kRowWaves - 2 && !p.vkeys) kvin.request(raw + (p.H + p.G) * p.D + kvh * p.E, p.E, lane);
+  const int pos = p.pos[row], slot = p.slot[row];
+  const int32_t* table = p.table + (size_t)slot * p.max_pages;
   const Tiles tl = tiles_of(p, pos, pos, 32);
   const int seen = blocks_seen(p, pos);
   // The launch is laid out for the longest context that the host allows for: splits without a tile leave at
@@ -687,37 +724,38 @@ __global__ __launch_bounds__(64 * kRowWaves) void paged_rows_kernel(const Params
     uint4 ka[KST], kb[KST];
     VTerms<T> v[VT];
   };
-  auto load_tile = [&](Tile& t, int j) {
+  auto page_of = [&](int j) { return (tl.mean(j) ? p.mtable + (size_t)slot * p.mpages : table)[tl.at(j) * 32 / kPage]; };
+  auto load_tile = [&](Tile& t, int j, int page) {
     const bool mean = tl.mean(j);
     const int key0 = tl.at(j) * 32;
-    const size_t head = (size_t)(mean ? p.mtable + (size_t)p.slot[row] * p.mpages : table)[key0 / kPage] * p.G + kvh;
+    const size_t head = (size_t)page * p.G + kvh;
     const char* kp = reinterpret_cast<const char*>(reinterpret_cast<const T*>(mean ? p.mkpool : p.kpool) +
-                                                   (head * kPage + (key0 % kPage) + r) * p.ldk) + g * 16;
+                                                   (head * kPage + (key0 % kPage) + VTerms<T>::ROWS * (r / 4) + r % 4) * p.ldk) + g * 16;
     const T* vp = reinterpret_cast<const T*>(mean ? p.mvpool : p.vpool) + (head * p.ldv + r) * kPage + (key0 % kPage);
 #pragma unroll
     for (int s = 0; s < KST; ++s)
       if (s < ksteps) {
         t.ka[s] = *reinterpret_cast<const uint4*>(kp + s * 64);
-        t.kb[s] = *reinterpret_cast<const uint4*>(kp + (size_t)16 * p.ldk * sizeof(T) + s * 64);
+        t.kb[s] = *reinterpret_cast<const uint4*>(kp + (size_t)VTerms<T>::OTHER * p.ldk * sizeof(T) + s * 64);
       }
 #pragma unroll
     for (int i = 0; i < VT; ++i)
       if (i < vtiles) t.v[i].load(vp + (size_t)i * 16 * kPage, g);
   };
-  // A wave's first tile is requested before the queries are normalised - unless it is the one
-  // that the row's own key goes into below.
+  // The page of a wave's first tile is on its way while the queries are normalised, and the tile while the row's key is stored - unless it
+  // is the one that this key goes into.
   const int stride = p.nsplit * kRowWaves;
   int j = split * kRowWaves + wave;
   Tile tile;
   const bool early = j < tl.n && !(FUSE && j == tl.n - 1);
-  if (early) load_tile(tile, j);
+  const bool owner = FUSE && split == ((tl.n - 1) % stride) / kRowWaves;
+  const int page0 = j < tl.n ? page_of(j) : 0, own_page = owner ? table[pos / kPage] : 0;
 
   // ---- queries (and the row's own key and value) through float32 norms
   float iq = 1.f, ik = 1.f;
-  const bool turned = p.whole || p.rot || p.taps;
-  const Channels<T> x(p, row, pos, p.slot[row], 0);
+  const Channels<T> x(p, row, pos, slot, 0);
   if (turned) {  // angles, and the RMS of the whole projections, once per workgroup
-    const T* src = reinterpret_cast<const T*>(p.qkv) + (size_t)row * p.ldq;
+    const T* src = raw;
     for (int i = threadIdx.x; 2 * i < p.rot; i += 64 * kRowWaves) cs[i] = turn_at(p, pos, i);
     if (p.whole) {
       const bool vec = p.D % Elem<T>::kVec == 0 && p.ldq % Elem<T>::kVec == 0;
@@ -734,23 +772,54 @@ __global__ __launch_bounds__(64 * kRowWaves) void paged_rows_kernel(const Params
       iq = 1.f / sqrtf(sq / (p.H * p.D) + p.eps), ik = 1.f / sqrtf(sk / (p.G * p.D) + p.eps);
     }
   }
-  for (int h = wave; h < 16; h += kRowWaves) {
-    T* dst = qs + h * QS;
-    if (h < gs && turned)
-      turn_row<T>(p, x, (h0 + h) * p.D, dst, iq, p.qgain ? p.qgain + (h0 + h) * p.D : nullptr, cs, lane);
-    else if (h < gs) unit_row<T>(reinterpret_cast<const T*>(p.qkv) + (size_t)row * p.ldq + (h0 + h) * p.D, dst, p.D, p.unit, p.eps, p.qgain, lane);
-    for (int d = (h < gs ? p.D : 0) + lane; d < QS; d += 64) dst[d] = Elem<T>::make(0.f);
+  if (plain) {
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {
+      const int at = threadIdx.x + 64 * kRowWaves * i, h = at / VPR, c = at % VPR * EPV;
+      if (16 * VPR % (64 * kRowWaves) == 0 || h < 16) *reinterpret_cast<u32x4_t*>(qs + h * QS + c) = qv[i];
+    }
+  } else if (turned) {
+    for (int h = wave; h < 16; h += kRowWaves) {
+      T* dst = qs + h * QS;
+      if (h < gs) turn_row<T>(p, x, (h0 + h) * p.D, dst, iq, p.qgain ? p.qgain + (h0 + h) * p.D : nullptr, cs, lane);
+      for (int d = (h < gs ? p.D : 0) + lane; d < QS; d += 64) dst[d] = Elem<T>::make(0.f);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 16 / kRowWaves; ++i) {
+      const int h = wave + kRowWaves * i;
+      T* dst = qs + h * QS;
+      if (h < gs) qin[i].put(dst, p.D, p.unit, p.eps, p.qgain, lane);
+      for (int d = (h < gs ? p.D : 0) + lane; d < QS; d += 64) dst[d] = Elem<T>::make(0.f);
+    }
   }
-  const bool owner = FUSE && split == ((tl.n - 1) % stride) / kRowWaves;
+  if (early) load_tile(tile, j, page0);
   if (owner) {
-    const int page = table[pos / kPage];
-    if (wave == kRowWaves - 1) put_key<T>(p, x, row, kvh, page, pos % kPage, lane, ik, cs);
-    if (wave == kRowWaves - 2) put_value<T>(p, x, row, kvh, page, pos % kPage, lane);
+    const size_t head = (size_t)own_page * p.G + kvh;
+    if (wave == kRowWaves - 1) {
+      T* const dst = reinterpret_cast<T*>(p.kpool) + (head * kPage + pos % kPage) * p.ldk;
+      if (plain) {
+        if (lane * EPV < p.D) *reinterpret_cast<u32x4_t*>(dst + lane * EPV) = kv;
+      } else if (turned) {
+        put_key<T>(p, x, kvh, dst, lane, ik, cs);
+      } else {
+        kvin.put(dst, p.D, p.unit, p.eps, p.kgain, lane);
+      }
+    } else if (wave == kRowWaves - 2) {
+      T* const dst = reinterpret_cast<T*>(p.vpool) + head * p.ldv * kPage + pos % kPage;
+      if (turned || p.vkeys) {
+        put_value<T>(p, x, row, kvh, dst, lane);
+      } else {
+#pragma unroll
+        for (int i = 0; i < DMAX / 64; ++i)
+          if (lane + 64 * i < p.E) dst[(size_t)(lane + 64 * i) * kPage] = mixed_value<T>(p, kvin.x[i], row, kvh * p.E + lane + 64 * i);
+      }
+    }
     wait_own_stores_done();
   }
   if (FUSE && p.taps && split == 0) keep_channels<T>(x, h0 * p.D, gs * p.D, threadIdx.x, 64 * kRowWaves);
   __syncthreads();
-  if (!early && j < tl.n) load_tile(tile, j);
+  if (!early && j < tl.n) load_tile(tile, j, page0);
   uint4 q[KST];
 #pragma unroll
   for (int s = 0; s < KST; ++s)
@@ -787,7 +856,7 @@ __global__ __launch_bounds__(64 * kRowWaves) void paged_rows_kernel(const Params
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int ja = key0 + 4 * g + e, jb = ja + 16;
+      const int ja = key0 + VTerms<T>::ROWS * g + e, jb = ja + VTerms<T>::OTHER;
       const bool va = ja <= lim && (pos - ja < size || ja < p.keep);
       const bool vb = jb <= lim && (pos - jb < size || jb < p.keep);
       if (SIGMOID) {
@@ -826,10 +895,10 @@ __global__ __launch_bounds__(64 * kRowWaves) void paged_rows_kernel(const Params
         o[t] = tile.v[t].mma(pt, o[t]);
       }
     j += stride;
-    if (j < tl.n) load_tile(tile, j);
+    if (j < tl.n) load_tile(tile, j, page_of(j));
   }
 
-  if (owner && p.pool && hg == 0 && (pos + 1) % p.pool == 0) put_means<T>(p, p.slot[row], pos / p.pool, kvh, threadIdx.x, 64 * kRowWaves);
+  if (owner && p.pool && hg == 0 && (pos + 1) % p.pool == 0) put_means<T>(p, slot, pos / p.pool, kvh, threadIdx.x, 64 * kRowWaves);
 
   // ---- the waves of the workgroup
   if (SIGMOID) m = 0.f, l = split == 0 && wave == 0 ? 1.f : 0.f;  // (factors of 1 from here on)
@@ -853,40 +922,65 @@ __global__ __launch_bounds__(64 * kRowWaves) void paged_rows_kernel(const Params
   __syncthreads();
   T* out = reinterpret_cast<T*>(p.out) + (size_t)row * p.ldo;
   const size_t wsrow = (size_t)blockIdx.z * p.H;
-  // two neighbouring columns per thread (an odd number of them: the last one beside nothing that is stored)
-  const int per = (p.E + 1) / 2, stride_ws = p.E + 2;
-  // every pair of floats of the partials at a multiple of 8 bytes
-  const bool eight = (((uint32_t)(uintptr_t)p.ws >> 2 | (uint32_t)p.E) & 1) == 0;
-  auto finished = [&](int h, int d, float a, float b) {
+  const int stride_ws = p.E + 2;
+  const auto ws = buf_of(p.ws + (wsrow + h0) * p.nsplit * stride_ws, used > 1 ? (uint32_t)(gs * p.nsplit * stride_ws) * 4 : 0);
+  const uint32_t head_ws = (uint32_t)(p.nsplit * stride_ws) * 4;
+  // W neighbouring columns per thread, as many as give every column a thread
+  const int columns = p.E % 4 == 0 && gs * p.E > 2 * 64 * kRowWaves ? 4 : p.E % 2 == 0 && gs * p.E > 64 * kRowWaves ? 2 : 1;
+  auto finished = [&](int h, int d, auto& a, float l) __attribute__((always_inline)) {
+    constexpr int W = sizeof(a.v) / 4;
     const float hgate = head_gate(p, row, h0 + h);
-    out[(h0 + h) * p.E + d] = Elem<T>::make(a * hgate * column_gate<T>(p, row, (h0 + h) * p.E + d));
-    if (d + 1 < p.E) out[(h0 + h) * p.E + d + 1] = Elem<T>::make(b * hgate * column_gate<T>(p, row, (h0 + h) * p.E + d + 1));
-  };
-  for (int i = threadIdx.x; i < gs * per; i += 64 * kRowWaves) {
-    const int h = i / per, d = (i - h * per) * 2;
-    float a0 = 0.f, a1 = 0.f, lw = 0.f, mm = -INFINITY;
+    T* const to = out + (h0 + h) * p.E + d;
+    float f[W];
 #pragma unroll
-    for (int w = 0; w < kRowWaves; ++w) mm = fmaxf(mm, ms[w][h]);
+    for (int c = 0; c < W; ++c) f[c] = a.v[c] / l * hgate;
+    if (p.ogate) {
 #pragma unroll
-    for (int w = 0; w < kRowWaves; ++w) {
-      const float2 v = *reinterpret_cast<const float2*>(&os[(w * p.gsz + h) * osl + d]);
-      a0 += v.x, a1 += v.y;
-      lw += ms[w][h] == -INFINITY ? 0.f : ls[w][h] * __builtin_amdgcn_exp2f(ms[w][h] - mm);
+      for (int c = 0; c < W; ++c) f[c] *= column_gate<T>(p, row, (h0 + h) * p.E + d + c);
     }
-    if (used == 1) {
-      finished(h, d, a0 / lw, a1 / lw);
+    struct alignas(W * sizeof(T)) {
+      T v[W];
+    } t;
+#pragma unroll
+    for (int c = 0; c < W; ++c) t.v[c] = Elem<T>::make(f[c]);
+    if (((uintptr_t)to & (W * sizeof(T) - 1)) == 0) {
+      *reinterpret_cast<decltype(t)*>(to) = t;
     } else {
-      float* dst = p.ws + ((wsrow + h0 + h) * p.nsplit + split) * stride_ws;
-      if (__builtin_expect(eight, 1)) {
-        st_dev2<true>(dst + d, a0, a1);
-        if (d == 0) st_dev2<true>(dst + p.E, mm, lw);
+#pragma unroll
+      for (int c = 0; c < W; ++c) to[c] = t.v[c];
+    }
+  };
+  auto combine = [&](auto run) __attribute__((always_inline)) {
+    constexpr int W = decltype(run)::value;
+    const int per = p.E / W;
+    for (int i = threadIdx.x; i < gs * per; i += 64 * kRowWaves) {
+      const int h = i / per, d = (i - h * per) * W;
+      Run<W> a = {};
+      float lw = 0.f, mm = -INFINITY;
+#pragma unroll
+      for (int w = 0; w < kRowWaves; ++w) mm = fmaxf(mm, ms[w][h]);
+#pragma unroll
+      for (int w = 0; w < kRowWaves; ++w) {
+        const Run<W> v = *reinterpret_cast<const Run<W>*>(&os[(w * p.gsz + h) * osl + d]);
+#pragma unroll
+        for (int c = 0; c < W; ++c) a.v[c] += v.v[c];
+        lw += ms[w][h] == -INFINITY ? 0.f : ls[w][h] * __builtin_amdgcn_exp2f(ms[w][h] - mm);
+      }
+      if (used == 1) {
+        finished(h, d, a, lw);
       } else {
-        st_dev(dst + d, a0);
-        if (d + 1 < p.E) st_dev(dst + d + 1, a1);
-        if (d == 0) st_dev2<false>(dst + p.E, mm, lw);
+        const uint32_t at = h * head_ws, part = (uint32_t)(split * stride_ws) * 4;
+        st_dev<W>(ws, at + d * 4, part, a);
+        if (d == 0) st_dev<2>(ws, at + p.E * 4, part, Run<2>{{mm, lw}});
       }
     }
-  }
+  };
+  if (columns == 4)
+    combine(std::integral_constant<int, 4>());
+  else if (columns == 2)
+    combine(std::integral_constant<int, 2>());
+  else
+    combine(std::integral_constant<int, 1>());
   if (used == 1) return;
 
   // ---- the splits: the last workgroup to arrive merges them (values at device scope, every
@@ -903,41 +997,49 @@ __global__ __launch_bounds__(64 * kRowWaves) void paged_rows_kernel(const Params
   if (!s_last) return;
   // A batch of splits at a time, all its requests ahead of their use, in a running (maximum, sum, weighted sum).  (First every
   // split's factor, then sixteen values of one column at a time whatever the number of splits, the waves one column at a
-  // time through conflicting banks: 4 rows of 32 / 4 heads, 700 keys 19.8 us against 16.3.)
-  auto merge = [&](auto pairs) __attribute__((always_inline)) {
-    constexpr bool EIGHT = decltype(pairs)::value;
-    constexpr int MS = 8;
+  // time through conflicting banks: 4 rows of 32 / 4 heads, 700 keys 19.8 us against 16.3, then.)
+  auto merge = [&](auto run) __attribute__((always_inline)) {
+    constexpr int MS = 8, W = decltype(run)::value;
+    const int per = p.E / W;
     for (int i = threadIdx.x; i < gs * per; i += 64 * kRowWaves) {
-      const int h = i / per, d = (i - h * per) * 2;
-      const float* src = p.ws + (wsrow + h0 + h) * p.nsplit * stride_ws;
-      float a0 = 0.f, a1 = 0.f, lsum = 0.f, mw = -INFINITY;
+      const int h = i / per, d = (i - h * per) * W;
+      const uint32_t at = h * head_ws;
+      Run<W> a = {};
+      float lsum = 0.f, mw = -INFINITY;
       for (int s0 = 0; s0 < used; s0 += MS) {
-        float2 ml[MS], v[MS];
+        Run<2> ml[MS];
+        Run<W> v[MS];
 #pragma unroll
         for (int s = 0; s < MS; ++s) {
-          const float* at = src + (size_t)min(s0 + s, used - 1) * stride_ws;
-          ml[s] = ld_dev2<EIGHT>(at + p.E);
-          v[s] = ld_dev2<EIGHT>(at + d);
+          const uint32_t part = (uint32_t)(min(s0 + s, used - 1) * stride_ws) * 4;
+          ml[s] = ld_dev<2>(ws, at + p.E * 4, part);
+          v[s] = ld_dev<W>(ws, at + d * 4, part);
         }
         float mc = mw;
 #pragma unroll
-        for (int s = 0; s < MS; ++s) mc = s0 + s < used ? fmaxf(mc, ml[s].x) : mc;
+        for (int s = 0; s < MS; ++s) mc = s0 + s < used ? fmaxf(mc, ml[s].v[0]) : mc;
         const float back = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw - mc);
-        a0 *= back, a1 *= back, lsum *= back;
+#pragma unroll
+        for (int c = 0; c < W; ++c) a.v[c] *= back;
+        lsum *= back;
 #pragma unroll
         for (int s = 0; s < MS; ++s) {
-          const float w1 = s0 + s >= used || ml[s].x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml[s].x - mc);
-          a0 += v[s].x * w1, a1 += v[s].y * w1, lsum += ml[s].y * w1;
+          const float w1 = s0 + s >= used || ml[s].v[0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml[s].v[0] - mc);
+#pragma unroll
+          for (int c = 0; c < W; ++c) a.v[c] += v[s].v[c] * w1;
+          lsum += ml[s].v[1] * w1;
         }
         mw = mc;
       }
-      finished(h, d, a0 / lsum, a1 / lsum);
+      finished(h, d, a, lsum);
     }
   };
-  if (__builtin_expect(eight, 1))
-    merge(std::true_type());
+  if (columns == 4)
+    merge(std::integral_constant<int, 4>());
+  else if (columns == 2)
+    merge(std::integral_constant<int, 2>());
   else
-    merge(std::false_type());
+    merge(std::integral_constant<int, 1>());
 }
 
 // ------------------------------------------------------------------------------ prompts
@@ -1397,7 +1499,7 @@ extern "C" int exo_paged_attn_rows(const exo_paged_attn* a, int nsplit, int appe
   p.hgroups = (group + 15) / 16;
   while (nsplit > 1 && p.hgroups < group && p.hgroups < 16 && (int64_t)a->n * p.G * p.hgroups * nsplit * 2 <= 256) p.hgroups *= 2;
   if (p.hgroups > group) p.hgroups = group;
-  p.gsz = (group + p.hgroups - 1) / p.hgroups;
+  p.gsz = (group + p.hgroups - 1) / p.hgroups, p.group = group;
   p.hgroups = (group + p.gsz - 1) / p.gsz;  // (none without a head)
   p.counters = reinterpret_cast<int*>(workspace);
   p.ws = nsplit > 1 ? reinterpret_cast<float*>(workspace) + kCounters : nullptr;

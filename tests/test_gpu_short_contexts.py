@@ -122,3 +122,18 @@ def test_paged_rows_merge_partials_at_any_float(device, monkeypatch, dtype, vdim
         assert "splits=1 " not in native.last_variant(), native.last_variant()
         close(host(out[:, : 8 * vdim]).reshape(len(last), 8, vdim), want[last], 3 * TOL[dtype], f"values of {vdim}")
         assert bool((out[:, 8 * vdim] == 7).all())
+
+
+# single steps of queries and keys without norm or rotation: rows copied in 16 bytes (or element by element where the width is no multiple of
+# that), one, two or four columns of the result to a thread, keys at either end of a tile and of a page, one workgroup and several
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("shape", [(8, 1, 128, 128), (4, 1, 64, 66), (2, 2, 64, 64), (6, 2, 36, 20), (1, 1, 16, 3), (16, 1, 256, 32)])
+def test_paged_rows_of_plain_queries(device, dtype, shape):
+    from tests import test_gpu_gekazen as G
+    from tests.stack_util import TOL, close
+
+    spec = G.make_spec(*shape, None, 0, slopes=False, unit=False)
+    cuts = [30, 1, 1, 1, 1, 29, 1, 1, 1, 61, 1, 1, 1, 126, 1, 1, 1, 1]
+    rows, qkv = G.attn_case(spec, sum(cuts), seed=shape[2])
+    want = G.attn_oracle(spec, qkv, 1e-6)
+    close(G.run_portions(spec, rows, cuts, dtype, 1e-6), want, 3 * TOL[dtype], str(shape))
