@@ -892,6 +892,7 @@ enum Kind { kSteps = 0, kChannel = 1, kGates = 2 };  // what the decay comes fro
 
 template <typename T, int KIND>
 __global__ __launch_bounds__(256) void recur_step_kernel(const Rec p, int cols) {
+  request_arguments(p);  // (64 heads under 4 rows 8.4 -> 8.1 us, in float32 32 heads under 2 rows 7.9 -> 7.4)
   constexpr bool CHANNEL = KIND == kChannel;
   extern __shared__ __attribute__((aligned(16))) float lds[];  // q, k, decay [dim]; values [64]; partials [4][cols]
   const int tid = threadIdx.x, D = p.dim, h = blockIdx.y, e0 = blockIdx.x * cols;
