@@ -28,9 +28,9 @@
 //   stores the row's own key and value (the workgroup that owns the last tile does).
 //   What bounds a launch of short contexts is a chain of ways through memory by a few waves: the arguments, position and slot, the page, the
 //   tile, the partials, their counter and the partials again.  So the arguments come in one way, a row's channels with its position (plain
-//   ones 16 bytes a thread, not element by element), the page of a wave's first tile behind that, a value column's eight keys in one
-//   request, and partials in requests of up to 16 bytes, a thread to every run of columns.  Four rows of 32 / 4 heads of 128, up to 700 keys: 15.9 -> 12.9 us
-//   (48 keys of 64 in float32, one split: 8.8 -> 9.0).
+//   ones 16 bytes a thread, not element by element), the page of a wave's first tile behind that, and partials in requests of up to
+//   16 bytes, a thread to every run of columns.  Launches of a graph, four rows of 32 / 4 heads of 128 with normed queries: 17 | 150 | 700 keys 8.1 | 10.8 | 11.7 ->
+//   6.9 | 10.1 | 11.2 us (48 keys of 64 in float32, one split: 6.5 -> 6.65).
 // paged_prepare_kernel: norm over whole projections, rotation and value mixing of all rows of a step
 //   ahead of the other two (queries in place, keys and values into the pool); a step of single tokens
 //   does the same inside paged_rows_kernel.  Convolved queries go to a buffer of their own, since other rows
@@ -637,23 +637,25 @@ struct PTerms<float> {
     lo = __builtin_bit_cast(uint4, floatx4{b[0], b[1], b[2], b[3]});
   }
 };
-// The keys of a 32-key tile at the rows of its two 16-key operands: row i holds key ROWS * (i / 4) + i % 4, in the other OTHER keys on.  A lane's
-// weights are those of rows 4g .. 4g + 3 of both, and with it a value column's entries: in bf16 eight consecutive ones, 16 bytes of the column
-// (with rows in order two halves of 8, twice the requests at half the bytes), in float32 two runs of 16 bytes.
+// a value column's entries of this lane's keys: 4g.. and 16 + 4g.. of the 32-key tile at v.  (Keys dealt to the two operands in runs
+// of four, so that the eight of a bf16 column are one request of 16 bytes, meet in other sums, and a decoder's outputs change: four rows of 32 / 4 heads of 128,
+// 700 keys 10.6 us for 11.2.)
 template <typename T>
 struct VTerms;
 template <>
 struct VTerms<bf16_t> {
-  static constexpr int ROWS = 8, OTHER = 4;
-  uint4 x;
-  __device__ __forceinline__ void load(const bf16_t* v, int g) { x = load16(v + 8 * g); }
+  uint2 a, b;
+  __device__ __forceinline__ void load(const bf16_t* v, int g) {
+    a = *reinterpret_cast<const uint2*>(v + 4 * g);
+    b = *reinterpret_cast<const uint2*>(v + 16 + 4 * g);
+  }
   __device__ __forceinline__ floatx4 mma(const PTerms<bf16_t>& p, floatx4 c) const {
+    const uint4 x{a.x, a.y, b.x, b.y};
     return Elem<bf16_t>::mma16(x, p.lo, Elem<bf16_t>::mma16(x, p.hi, c));
   }
 };
 template <>
 struct VTerms<float> {
-  static constexpr int ROWS = 4, OTHER = 16;
   uint4 a, b;
   __device__ __forceinline__ void load(const float* v, int g) {
     a = *reinterpret_cast<const uint4*>(v + 4 * g);
@@ -730,13 +732,13 @@ __global__ __launch_bounds__(64 * kRowWaves) void paged_rows_kernel(const Params
     const int key0 = tl.at(j) * 32;
     const size_t head = (size_t)page * p.G + kvh;
     const char* kp = reinterpret_cast<const char*>(reinterpret_cast<const T*>(mean ? p.mkpool : p.kpool) +
-                                                   (head * kPage + (key0 % kPage) + VTerms<T>::ROWS * (r / 4) + r % 4) * p.ldk) + g * 16;
+                                                   (head * kPage + (key0 % kPage) + r) * p.ldk) + g * 16;
     const T* vp = reinterpret_cast<const T*>(mean ? p.mvpool : p.vpool) + (head * p.ldv + r) * kPage + (key0 % kPage);
 #pragma unroll
     for (int s = 0; s < KST; ++s)
       if (s < ksteps) {
         t.ka[s] = *reinterpret_cast<const uint4*>(kp + s * 64);
-        t.kb[s] = *reinterpret_cast<const uint4*>(kp + (size_t)VTerms<T>::OTHER * p.ldk * sizeof(T) + s * 64);
+        t.kb[s] = *reinterpret_cast<const uint4*>(kp + (size_t)16 * p.ldk * sizeof(T) + s * 64);
       }
 #pragma unroll
     for (int i = 0; i < VT; ++i)
@@ -856,7 +858,7 @@ __global__ __launch_bounds__(64 * kRowWaves) void paged_rows_kernel(const Params
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int ja = key0 + VTerms<T>::ROWS * g + e, jb = ja + VTerms<T>::OTHER;
+      const int ja = key0 + 4 * g + e, jb = ja + 16;
       const bool va = ja <= lim && (pos - ja < size || ja < p.keep);
       const bool vb = jb <= lim && (pos - jb < size || jb < p.keep);
       if (SIGMOID) {

@@ -137,3 +137,28 @@ def test_paged_rows_of_plain_queries(device, dtype, shape):
     rows, qkv = G.attn_case(spec, sum(cuts), seed=shape[2])
     want = G.attn_oracle(spec, qkv, 1e-6)
     close(G.run_portions(spec, rows, cuts, dtype, 1e-6), want, 3 * TOL[dtype], str(shape))
+
+
+# bits of the outputs, recorded on the card: the keys of a tile meet in the sums in their order, and a change of it, which no tolerance shows, changes
+# them (and with them what a decoder gives for the same request)
+@pytest.mark.parametrize("heads,kv_heads,dim,keys,scale,digest", [
+    (32, 4, 128, 700, 0.02, "e79732b5ac35948f"), (16, 8, 64, 48, 0.5, "ec73869fddee6247"), (8, 2, 64, 2000, 0.5, "96b7dfdbd97c0ac2")])
+def test_paged_rows_keep_the_order_of_keys(device, heads, kv_heads, dim, keys, scale, digest):
+    import hashlib
+
+    from exo_amd import dense_ops as D
+    from exo_amd.paged_cache import PagedKVCache
+    from tests import test_gpu_gekazen as G
+
+    spec = G.make_spec(heads, kv_heads, dim, dim, None, 0, scale=scale, slopes=False)
+    cache = PagedKVCache([(kv_heads, dim, dim)], 2, keys + 64, "cuda", torch.bfloat16)
+    att = D.PagedAttention(spec, None, 0, cache, 1e-6)
+    qkv = torch.randn(keys, (heads + 2 * kv_heads) * dim, generator=torch.Generator().manual_seed(keys)).to(device).bfloat16()
+    i32 = dict(dtype=torch.int32, device=device)
+    cache.reserve([1], keys)
+    att.append(qkv, torch.full((keys,), 1, **i32), torch.arange(keys, **i32), keys)
+    last = torch.tensor([keys - 1, keys // 2], **i32)
+    out = torch.zeros(2, heads * dim, dtype=torch.bfloat16, device=device)
+    att.rows(qkv[last.long()].contiguous(), out, torch.full((2,), 1, **i32), last, 2, keys, append=False)
+    got = hashlib.sha256(out.view(torch.int16).cpu().numpy().tobytes()).hexdigest()[:16]
+    assert got == digest, got
