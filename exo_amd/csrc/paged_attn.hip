@@ -30,7 +30,7 @@
 //   tile, the partials, their counter and the partials again.  So the arguments come in one way, a row's channels with its position (plain
 //   ones 16 bytes a thread, not element by element), the page of a wave's first tile behind that, and partials in requests of up to
 //   16 bytes, a thread to every run of columns.  Launches of a graph, four rows of 32 / 4 heads of 128 with normed queries: 17 | 150 | 700 keys 8.1 | 10.8 | 11.7 ->
-//   6.9 | 10.1 | 11.2 us (48 keys of 64 in float32, one split: 6.5 -> 6.65).
+//   6.9 | 10.1 | 11.2 us (48 keys of 64 in float32, one split: 6.55 -> 6.45).
 // paged_prepare_kernel: norm over whole projections, rotation and value mixing of all rows of a step
 //   ahead of the other two (queries in place, keys and values into the pool); a step of single tokens
 //   does the same inside paged_rows_kernel.  Convolved queries go to a buffer of their own, since other rows
@@ -745,7 +745,9 @@ __global__ __launch_bounds__(64 * kRowWaves) void paged_rows_kernel(const Params
       if (i < vtiles) t.v[i].load(vp + (size_t)i * 16 * kPage, g);
   };
   // The page of a wave's first tile is on its way while the queries are normalised, and the tile while the row's key is stored - unless it
-  // is the one that this key goes into.
+  // is the one that this key goes into.  Where one split holds all tiles the tile goes out ahead of the queries' arithmetic (us, normed
+  // queries, 48 keys: 16 / 8 heads of 64 float 6.60 -> 6.40, bf16 5.64 -> 5.55, 32 / 4 of 128 bf16 7.40 -> 7.14); with several it is the slower order (4 rows of
+  // 32 / 4 of 128, 3000 keys 17.1 -> 17.7, 150 10.1 -> 10.5).
   const int stride = p.nsplit * kRowWaves;
   int j = split * kRowWaves + wave;
   Tile tile;
@@ -755,6 +757,7 @@ __global__ __launch_bounds__(64 * kRowWaves) void paged_rows_kernel(const Params
 
   // ---- queries (and the row's own key and value) through float32 norms
   float iq = 1.f, ik = 1.f;
+  if (early && used == 1) load_tile(tile, j, page0);
   const Channels<T> x(p, row, pos, slot, 0);
   if (turned) {  // angles, and the RMS of the whole projections, once per workgroup
     const T* src = raw;
@@ -795,7 +798,7 @@ __global__ __launch_bounds__(64 * kRowWaves) void paged_rows_kernel(const Params
       for (int d = (h < gs ? p.D : 0) + lane; d < QS; d += 64) dst[d] = Elem<T>::make(0.f);
     }
   }
-  if (early) load_tile(tile, j, page0);
+  if (early && used > 1) load_tile(tile, j, page0);
   if (owner) {
     const size_t head = (size_t)own_page * p.G + kvh;
     if (wave == kRowWaves - 1) {
