@@ -896,6 +896,7 @@ bool wide_is_faster(int64_t wide, int64_t narrow, int steps, int64_t out_bytes) 
   return tw < tn;
 }
 
+constexpr int64_t kPairWorkspace = 1 << 24;  // floats: as much as a device's single products share
 // Ranges of K of a gated pair whose tiles leave CUs without work, or few in flight on each.  us: a step of 128 bytes of K takes 0.6 in bf16 and 1.3 in
 // float, 1.7 times that with two workgroups on a CU, which is a full round; the reduce launch 2.75 and 0.35 a range more, the
 // sums' way through memory 2.5 MB / us.
@@ -915,18 +916,40 @@ int pair_ranges(int64_t tiles, int steps, int64_t outputs, bool tall, int elem, 
   return best;
 }
 
-// rows per tile: the tallest that still leaves a workgroup per CU, else the shorter ones
+// Tiles of a product: 256 rows high (wide), or 128 where those still leave most CUs a workgroup (tall), else 64
+struct PlainTiles {
+  int64_t t1, t2, w;
+  int steps;
+  bool tall, wide;
+};
+template <typename T, bool PAIR>
+PlainTiles tiles_of(const GemmParams& p) {
+  PlainTiles t;
+  const int64_t cols = exo_ceil_div(p.N, PAIR ? 64 : 128);
+  t.steps = (int)((int64_t)p.ldw * sizeof(T) / 128);
+  t.t2 = cols * exo_ceil_div(p.M, 128), t.t1 = cols * exo_ceil_div(p.M, 64);
+  t.w = (int64_t)exo_ceil_div(p.N, PAIR ? 128 : 256) * exo_ceil_div(p.M, 256);
+  t.tall = p.M > 64 && t.t2 >= 192;
+  t.wide = sizeof(T) == 2 && p.M > 128 && wide_fits(p) && wide_is_faster(t.w, t.t2, t.steps, (int64_t)p.M * p.N * (p.y_f32 ? 4 : 2));
+  return t;
+}
+template <typename T>
+int pair_ranges_of(const GemmParams& p, int64_t ws_floats) {
+  const PlainTiles t = tiles_of<T, true>(p);
+  return t.wide ? 1 : pair_ranges(t.tall ? t.t2 : t.t1, t.steps, (int64_t)p.M * p.N, t.tall, (int)sizeof(T), ws_floats);
+}
+
 template <typename T, bool PAIR>
 int launch_plain(GemmParams p, int64_t ws_floats, hipStream_t st) {
-  const int cols = exo_ceil_div(p.N, PAIR ? 64 : 128);
-  const int steps = (int)((int64_t)p.ldw * sizeof(T) / 128);
+  const PlainTiles plan = tiles_of<T, PAIR>(p);
+  const int64_t t1 = plan.t1, t2 = plan.t2;
+  const int steps = plan.steps;
+  const bool tall = plan.tall;
   p.ksplit = 1;
   p.ksteps = steps;
-  const int64_t t2 = (int64_t)cols * exo_ceil_div(p.M, 128), t1 = (int64_t)cols * exo_ceil_div(p.M, 64);
-  const bool tall = p.M > 64 && t2 >= 192;
   if constexpr (sizeof(T) == 2) {
-    const int64_t wide = (int64_t)exo_ceil_div(p.N, PAIR ? 128 : 256) * exo_ceil_div(p.M, 256);
-    if (p.M > 128 && wide_fits(p) && wide_is_faster(wide, t2, steps, (int64_t)p.M * p.N * (p.y_f32 ? 4 : 2))) return launch_wide<PAIR>(p, st);
+    const int64_t wide = plan.w;
+    if (plan.wide) return launch_wide<PAIR>(p, st);
     // ... or of ranges of K, while they are long against the partial sums' way through memory (columns x K, rows, us before | now:
     // 4096x13824, 300 88 | 66, 700 150 | 105, 2000 271 | 222; 4096x8192, 1004 93 | 85; 3072x6144, 700 65 | 54; 2048x6912, 1500 77 | 66; but
     // in ranges of 864, 1004 rows 54 | 58, and 4096x4096, 1004 rows 51 | 59)
@@ -961,7 +984,7 @@ int launch_plain(GemmParams p, int64_t ws_floats, hipStream_t st) {
     }
   }
   if (PAIR && p.part) {
-    const int ks = pair_ranges(tall ? t2 : t1, steps, (int64_t)p.M * p.N, tall, (int)sizeof(T), ws_floats);
+    const int ks = pair_ranges_of<T>(p, ws_floats);
     if (ks > 1) {
       p.ksteps = exo_ceil_div(steps, ks);
       p.ksplit = exo_ceil_div(steps, p.ksteps);
@@ -1310,15 +1333,27 @@ extern "C" int exo_post_linear(const exo_post_norm* q, const exo_linear* a, exo_
   return EXO_OK;
 }
 
-extern "C" int exo_linear_gemm(const exo_linear* a, float* workspace, int64_t workspace_floats, exo_stream_t stream) {
-  int rc = linear_check(a, "exo_linear_gemm");
-  if (rc) return rc;
-  EXO_REQUIRE(a->x && a->M <= 65535 * 64, "exo_linear_gemm: null x or bad M=%d", a->M);
+static GemmParams gemm_of(const exo_linear* a) {
   GemmParams p{};
   p.x = a->x, p.w = a->w, p.w2 = a->w_up, p.bias = a->bias, p.y = a->y, p.y2 = a->y2;
   p.M = a->M, p.N = a->N, p.n1 = a->n1, p.ldx = a->ldx, p.ldw = a->ldw, p.ldy = a->ldy, p.ldy2 = a->ldy2, p.y_f32 = a->y_f32;
   p.glu = GluConst{a->limit, a->alpha, a->shift, a->cubic};
   p.ep = Epilogue{a->act, a->mul, a->mul_rows, a->ldmul, a->cap};
+  return p;
+}
+
+extern "C" int64_t exo_linear_pair_workspace(const exo_linear* a) {
+  if (linear_check(a, "exo_linear_pair_workspace") || !a->w_up) return 0;
+  const GemmParams p = gemm_of(a);
+  const int ks = EXO_BY_TYPE(a->dtype, pair_ranges_of<bf16_t>(p, kPairWorkspace), pair_ranges_of<float>(p, kPairWorkspace));
+  return ks > 1 ? 2 * (int64_t)ks * p.M * p.N : 0;
+}
+
+extern "C" int exo_linear_gemm(const exo_linear* a, float* workspace, int64_t workspace_floats, exo_stream_t stream) {
+  int rc = linear_check(a, "exo_linear_gemm");
+  if (rc) return rc;
+  EXO_REQUIRE(a->x && a->M <= 65535 * 64, "exo_linear_gemm: null x or bad M=%d", a->M);
+  GemmParams p = gemm_of(a);
   p.part = workspace;
   EXO_REQUIRE(!a->w_up || a->y_f32 == (a->dtype == 1), "exo_linear_gemm: a gated pair leaves in the element type");
   if (a->w_up)

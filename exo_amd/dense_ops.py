@@ -101,11 +101,17 @@ GEMM_WS_FLOATS = 1 << 24
 
 
 def gemm_workspace(device) -> torch.Tensor:
-    """Float32 partial tiles of GEMMs that split K; one per device (work is in stream order)."""
+    """Float32 partial tiles of single products that split K; one per device (work is in stream order)."""
     key = torch.device(device).index or 0
     if key not in _GEMM_WS:
         _GEMM_WS[key] = torch.empty(GEMM_WS_FLOATS, dtype=torch.float32, device=device)
     return _GEMM_WS[key]
+
+
+def pair_workspace(a, device):
+    """... of a gated pair, for this launch alone: pairs on two streams may run side by side."""
+    need = native.load().exo_linear_pair_workspace(C.byref(a))
+    return torch.empty(need, dtype=torch.float32, device=device) if need else None
 
 
 ACTS = {None: 0, "relu2": 1, "gelu_tanh": 2, "cap": 3}
@@ -144,8 +150,8 @@ def _launch_linear(a, n: int, device, force_gemm: bool = False) -> None:
     if n <= GEMV_MAX_ROWS and not force_gemm:
         check(native.load().exo_linear_rows(C.byref(a), None, _stream()), "linear")
     else:
-        ws = gemm_workspace(device)
-        check(native.load().exo_linear_gemm(C.byref(a), _ptr(ws), ws.numel(), _stream()), "linear(gemm)")
+        ws = pair_workspace(a, device) if a.w_up else gemm_workspace(device)
+        check(native.load().exo_linear_gemm(C.byref(a), _ptr(ws), 0 if ws is None else ws.numel(), _stream()), "linear(gemm)")
 
 
 def linear_pair(x0, w0, out0, x1, w1, out1, n: int) -> None:
@@ -190,7 +196,8 @@ def norm_linear(x, gain, eps: float, operand, w, out, n: int) -> None:
 
 
 def glu(x, gate, up, out, n: int, spec, force_gemm: bool = False) -> None:
-    """out[:n] = clamped gated unit of x[:n]."""
+    """out[:n] = clamped gated unit of x[:n].  (Pairs of few tiles take a buffer of partial sums from torch's allocator, on its
+    current stream.)"""
     _launch_linear(_linear(x, gate, out, n, up=up, spec=spec), n, x.device, force_gemm)
 
 

@@ -153,6 +153,7 @@ SIGNATURES: dict[str, tuple] = {
     "exo_moe_sum_post_norm": (_i, [_vp] * 5 + [_i] * 6 + [C.POINTER(PostNorm), _i, _i, _i, _vp]),
     "exo_moe_route": (_i, [_vp] * 4 + [_i] * 4 + [_f, _i, _vp]),
     "exo_linear_rows": (_i, [C.POINTER(Linear), C.POINTER(Linear), _vp]),
+    "exo_linear_pair_workspace": (_i64, [C.POINTER(Linear)]),
     "exo_linear_gemm": (_i, [C.POINTER(Linear), _vp, _i64, _vp]),
     "exo_post_linear_fits": (_i, [_i] * 5),
     "exo_post_linear": (_i, [C.POINTER(PostNorm), C.POINTER(Linear), _vp]),

@@ -499,6 +499,10 @@ typedef struct {
 } exo_linear;
 /* up to 16 rows; b non-null: a second product over the same number of rows in the same launch */
 int exo_linear_rows(const exo_linear* a, const exo_linear* b, exo_stream_t stream);
+/* any rows; workspace: partial sums of products that split K over workgroups (null or smaller: fewer of them).  Launches that
+ * share a workspace must be ordered on one stream.  exo_linear_pair_workspace: floats that a gated pair takes (0: none, or
+ * not a pair, or arguments that exo_linear_gemm refuses). */
+int64_t exo_linear_pair_workspace(const exo_linear* a);
 int exo_linear_gemm(const exo_linear* a, float* workspace, int64_t workspace_floats,
                     exo_stream_t stream);
 /* exo_post_norm_add and the product in one launch (few rows: exo_post_linear_fits): a->x is not

@@ -353,3 +353,34 @@ def test_gated_pair_in_ranges_of_k(device, dtype, M, N, K, split):
     bound = (K + 1) * 2.0**-24 * (1.1 * size_a * 2.5 + size_c * 1.5) + (2.0**-20 if dtype == torch.float32 else 2.0**-8 + 2.0**-18) * want.abs()
     assert bool(((out[:M, :N].double() - want).abs() <= bound + 1e-12).all())
     assert bool((out[M:] == 7).all()) and bool((out[:, N:] == 7).all())
+
+
+def test_gated_pairs_on_two_streams(device):
+    """Pairs whose ranges of K meet in memory, on two streams side by side: each has the bits that it has alone."""
+    M, N, K = 53, 2560, 1024
+    g = torch.Generator(device=device).manual_seed(5)
+
+    class Spec:
+        limit, alpha, shift, cubic = 7.0, 1.702, 1.0, 0.0
+
+    sets = [[torch.randn(n, K, device=device, generator=g) * K**-0.25 for n in (M, N, N)] for _ in range(2)]
+    alone = [torch.empty(M, N, device=device) for _ in sets]
+    for (x, gate, up), out in zip(sets, alone):
+        D.glu(x, gate, up, out, M, Spec)
+    assert "pair" in native.last_variant() and not native.last_variant().endswith("x1"), native.last_variant()
+    outs = [[torch.empty(M, N, device=device) for _ in range(40)] for _ in sets]
+    streams = [torch.cuda.Stream() for _ in sets]
+    big = torch.randn(4096, 4096, device=device)
+    for _ in range(6):  # (both queues fill up behind this)
+        big = big @ big / 64
+    behind = torch.cuda.Event()
+    behind.record()
+    for s in streams:
+        s.wait_event(behind)
+    for i in range(40):
+        for (x, gate, up), out, s in zip(sets, outs, streams):
+            with torch.cuda.stream(s):
+                D.glu(x, gate, up, out[i], M, Spec)
+    torch.cuda.synchronize()
+    for want, out in zip(alone, outs):
+        assert all(torch.equal(o, want) for o in out)

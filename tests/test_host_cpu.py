@@ -96,6 +96,25 @@ def test_argument_errors_without_gpu():
         native.check(-1, "x")
 
 
+def test_workspace_of_gated_pairs():
+    """Float gated pairs of few tiles add ranges of K in memory, whole ones take none."""
+    import ctypes as C
+
+    from exo_amd import native
+
+    lib = native.load()
+
+    def floats(M, N, K, dtype, **more):
+        return lib.exo_linear_pair_workspace(C.byref(native.Linear(**{**dict(x=4096, w=4096, w_up=4096, y=4096, M=M, N=N, n1=N, ldx=K, ldw=K, ldy=N, y_f32=dtype, dtype=dtype), **more})))
+
+    for M, N, K, t in ((53, 2560, 1024, 1), (53, 2560, 1024, 0), (150, 6912, 2048, 1)):  # (the last: tiles of 128 rows)
+        assert floats(M, N, K, t) >= 2 * 2 * M * N and floats(M, N, K, t) % (2 * M * N) == 0
+    assert floats(2000, 6912, 2048, 0) == 0 and floats(20, 400, 64, 1) == 0
+    assert floats(53, 2560, 1024, 1, w_up=None) == 0 and floats(53, 2560, 1000, 1) == 0  # no pair; rows that are refused
+    assert all(0 <= floats(M, N, K, t) <= 1 << 24 for M in (17, 700, 70000) for N in (1, 300, 9000) for K in (64, 1024, 8192) for t in (0, 1))
+
+
+
 def test_bench_reads_the_committed_counter_summary():
     """roofline.traffic of the bench line comes from the committed rocprofv3 --pmc summary:
     the launch names bench.py asks for must be the ones that file lists."""
