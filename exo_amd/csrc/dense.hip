@@ -936,7 +936,8 @@ PlainTiles tiles_of(const GemmParams& p) {
 template <typename T>
 int pair_ranges_of(const GemmParams& p, int64_t ws_floats) {
   const PlainTiles t = tiles_of<T, true>(p);
-  return t.wide ? 1 : pair_ranges(t.tall ? t.t2 : t.t1, t.steps, (int64_t)p.M * p.N, t.tall, (int)sizeof(T), ws_floats);
+  if (t.wide || p.M > 65535) return 1;  // (the launch that adds them has a row per block of y)
+  return pair_ranges(t.tall ? t.t2 : t.t1, t.steps, (int64_t)p.M * p.N, t.tall, (int)sizeof(T), ws_floats);
 }
 
 template <typename T, bool PAIR>

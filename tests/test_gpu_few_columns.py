@@ -384,3 +384,22 @@ def test_gated_pairs_on_two_streams(device):
     torch.cuda.synchronize()
     for want, out in zip(alone, outs):
         assert all(torch.equal(o, want) for o in out)
+
+
+def test_gated_pair_of_more_rows_than_a_grid_holds(device):
+    """A narrow pair of 65600 rows, whose sums' launch would be that many blocks high: whole, and in range at both ends."""
+    M, N, K = 65600, 8, 1024
+    g = torch.Generator(device=device).manual_seed(3)
+    x, gate, up = (torch.randn(n, K, device=device, generator=g) * K**-0.25 for n in (M, N, N))
+
+    class Spec:
+        limit, alpha, shift, cubic = float("inf"), 0.0, 0.0, 0.0
+
+    out = torch.full((M + 1, N), 7.0, device=device)
+    D.glu(x, gate, up, out, M, Spec)
+    assert native.last_variant().endswith("x1"), native.last_variant()
+    for rows in (slice(0, 300), slice(M - 300, M)):  # (a gate of 1 and no bend: half the product of the two)
+        a, c, size_a, size_c = (p.double() @ q.double().T for p, q in ((x[rows], gate), (x[rows], up), (x[rows].abs(), gate.abs()), (x[rows].abs(), up.abs())))
+        bound = (K + 1) * 2.0**-24 * (size_a * c.abs() + size_c * a.abs()) * 0.51 + 2.0**-22 * (a * c / 2).abs()
+        assert bool(((out[rows].double() - a * c / 2).abs() <= bound + 1e-12).all())
+    assert bool((out[M:] == 7).all())

@@ -109,6 +109,8 @@ def test_workspace_of_gated_pairs():
 
     for M, N, K, t in ((53, 2560, 1024, 1), (53, 2560, 1024, 0), (150, 6912, 2048, 1)):  # (the last: tiles of 128 rows)
         assert floats(M, N, K, t) >= 2 * 2 * M * N and floats(M, N, K, t) % (2 * M * N) == 0
+    assert floats(40000, 8, 4096, 1) > 0  # many rows, and more than the launch that adds the ranges takes
+    assert not any(floats(M, N, K, t) for M in (65536, 65600, 1 << 20) for N in (1, 8, 40) for K in (1024, 4096) for t in (0, 1))
     assert floats(2000, 6912, 2048, 0) == 0 and floats(20, 400, 64, 1) == 0
     assert floats(53, 2560, 1024, 1, w_up=None) == 0 and floats(53, 2560, 1000, 1) == 0  # no pair; rows that are refused
     assert all(0 <= floats(M, N, K, t) <= 1 << 24 for M in (17, 700, 70000) for N in (1, 300, 9000) for K in (64, 1024, 8192) for t in (0, 1))
