@@ -107,8 +107,7 @@ __device__ __forceinline__ float group_sum_lpk(float d) {
 }
 // Over the lane groups of a wave, in every one of them.  A call's chain is one of latencies (a wave has a few tiles): through the crossbar
 // (__shfl_xor, about 100 cycles a round) the maximum and the sums of 64-wide heads were six dependent rounds, and the launch 5.94 us
-// where it is 5.68; a pass of 16 layers of 64-wide heads 3380 -> 3354 us, of 32 layers of 128-wide ones 3532 -> 3520 (each the mean over five
-// offsets of the kernels in memory).
+// where it is 5.68.
 template <int LPK>
 __device__ __forceinline__ float groups_sum(float x, float scale) {  // of x * scale; a lane's own product is not rounded
   float v = fmaf(x, scale, lane_xor<LPK>(x * scale));
@@ -1102,14 +1101,11 @@ int launch_sdpa(const SdpaParams& p0, hipStream_t st) {
     switch (G) {
       case 1:
         // few splits (many kv-head groups): eight waves per workgroup halve a wave's tiles
-        // (64 query / 4 kv heads at 4100 keys: 13.4 -> 12.4 us; with 8 splits four waves win).
-        // The order of the two calls is the order of the kernels in memory: a layer's kernels are nearly as large as the instruction cache, and the
-        // one of four waves here begins where it displaces the fewest of the products' lines (a pass of 32 layers of 4096 columns in 4 bits 3505 us,
-        // at the other offsets to 16 KB 3503 to 3560).
-        if (p.splits > 4 || kTileWaves != 4)
-          sdpa_tiles_kernel<D, 1, FUSED, kTileWaves><<<grid, 64 * kTileWaves, 0, st>>>(p);
-        else
+        // (64 query / 4 kv heads at 4100 keys: 13.4 -> 12.4 us; with 8 splits four waves win)
+        if (p.splits <= 4 && kTileWaves == 4)
           sdpa_tiles_kernel<D, 1, FUSED, 8><<<grid, 512, 0, st>>>(p);
+        else
+          sdpa_tiles_kernel<D, 1, FUSED, kTileWaves><<<grid, 64 * kTileWaves, 0, st>>>(p);
         break;
       case 2: sdpa_tiles_kernel<D, 2, FUSED, kTileWaves><<<grid, 64 * kTileWaves, 0, st>>>(p); break;
       case 4: sdpa_tiles_kernel<D, 4, FUSED, kTileWaves><<<grid, 64 * kTileWaves, 0, st>>>(p); break;
