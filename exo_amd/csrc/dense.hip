@@ -1135,7 +1135,7 @@ void launch_gemv_parts(const GemvParams& p, const GemvParams* p1, hipStream_t st
     dense_gemv_kernel<T, 8, 0, 0, PAIR, DUAL, Q><<<tiles, 512, 0, st>>>(p, DUAL ? *p1 : p, none);
 }
 // Weight rows of a workgroup and its waves.  All workgroups of a launch of up to about two rounds are resident together, so the CU
-// that got the most rows ends last: 864 workgroups of 8 rows leave some CUs with 32 and the average with 27, 988 of 7 all with 28.  Fewer
+// that got the most rows ends last: 864 workgroups of 8 rows leave 96 CUs with 32 (27 on average), 988 of 7 none with more than 28.  Fewer
 // rows than the product holds cost nothing but its empty lanes.  Fewer waves cost less where every workgroup repeats norms and
 // adds its waves' sums, more of them keep more requests in flight.  gemv_us is a fit to 4873 shapes (64 to 14336 columns of K, 300 to
 // 40000 columns, 1 to 16 rows, with and without norms, bf16 and f32, 12 settings each).  What is fastest by it takes, on average, 0.946 of the time of
@@ -1154,7 +1154,8 @@ double gemv_us(const GemvParams& p, const GemvParams* p1, const PostNorm* q, int
   const double fullest = std::max(held * cu, total / 6.4e6), average = wgs * cu / 256;
   const double x = (double)held * p.M * row / 64e3, waves = c.waves * wgs / 8192.0;  // rows of x read, waves beside one another
   const int steps = exo_ceil_div(row / 64 / parts, c.waves);
-  const int batch = kBatch / mats / (!q && parts > 1 && steps <= kBatch / mats / 2 ? 2 : 1);
+  const bool half = parts > 1 && (q ? !p.w2 : steps <= kBatch / mats / 2);  // (the instances of launch_gemv_post_as and launch_gemv_parts)
+  const int batch = kBatch / mats / (half ? 2 : 1);
   const double empty = (double)(exo_ceil_div(steps, batch) * batch - steps) * c.waves * held / 64;  // requests past a wave's range
   if (!q)
     return p.w2 ? 2.29 + 0.65 * fullest + 0.41 * average + 1.42 * x + 0.25 * waves + 1.17 * empty + 0.15 * steps
@@ -1172,7 +1173,9 @@ GemvShape gemv_shape(const GemvParams& p, const GemvParams* p1, const PostNorm* 
   double least = 0.96 * gemv_us(p, p1, q, elem, parts, usual);
   for (int waves = 4; waves <= 16; waves *= 2) {
     if (parts > 1 && waves != 8) continue;
-    if (q && passes(waves) > std::max(2, passes(usual.waves))) continue;  // (beyond, gains are not requested ahead)
+    // (More are another instance, which the cost is no fit to.  Behind two branches the second pass already takes its gains where they are used and not
+    // ahead; one pass for those gives 1.10 of the time over the 212 shapes of the sweep that it would change, 0.86 to 1.33.)
+    if (q && passes(waves) > std::max(2, passes(usual.waves))) continue;
     auto weigh = [&](int cols) {
       const double us = gemv_us(p, p1, q, elem, parts, {waves, cols});
       if (us < least) least = us, best = GemvShape{waves, cols};
