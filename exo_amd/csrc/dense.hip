@@ -900,14 +900,15 @@ constexpr int64_t kPairWorkspace = 1 << 24;  // floats: as much as a device's si
 // Ranges of K of a gated pair whose tiles leave CUs without work, or few in flight on each.  us: a step of 128 bytes of K takes 0.6 in bf16 and 1.3 in
 // float, 1.7 times that with two workgroups on a CU, which is a full round; the reduce launch 2.75 and 0.35 a range more, the
 // sums' way through memory 2.5 MB / us.
-// Over 271 shapes (17 to 700 rows, 300 to 9000 columns, K of 128 to 8000) what this gives takes 0.65 of the time of one range on average (the best number
-// 0.644), 1.01 at most.  Pair of 2560x1024 float under 53 rows, 40 workgroups, 40 -> 17 us; of 6912x2048 bf16 under 60 24.3 -> 18.8; of 999x7424 under 206
-// 69 -> 25.
+// It has to promise 12 % of tiles that leave CUs idle, 18 % of more: of 710 shapes (17 to 700 rows, 300 to 40000 columns, K of 256 to 8192) that it would split for 3 %
+// 5 of 475 and 36 of 235 took more than 1.02 of the time of one range, up to 1.11 (f32 194x11240x960 119 | 132 us, bf16 39x36830x6912 203 | 218), and with this line none;
+// of idle CUs 0.64 of the time on average (0.63 without the line), of more tiles 0.91 (0.88).
+// Pair of 2560x1024 float under 53 rows, 40 workgroups, 40 -> 17 us; of 6912x2048 bf16 under 60 24.3 -> 18.8; of 999x7424 under 206 69 -> 25.
 int pair_ranges(int64_t tiles, int steps, int64_t outputs, bool tall, int elem, int64_t ws_floats) {
   const double step = (elem == 2 ? 0.6 : 1.3) * (tall ? 1.6 : 1.0);
   auto rounds = [](int64_t wgs) { return wgs / 512 * 1.7 + (wgs % 512 > 256 ? 1.7 : wgs % 512 ? 1.0 : 0.0); };
   int best = 1;
-  double least = 0.97 * step * steps * rounds(tiles);
+  double least = (tiles <= 256 ? 0.88 : 0.82) * step * steps * rounds(tiles);
   for (int ks = 2; ks <= 16 && steps / ks >= 2 && 2 * ks * outputs <= ws_floats; ++ks) {
     const int range = exo_ceil_div(steps, ks), used = exo_ceil_div(steps, range);
     const double us = step * range * rounds(tiles * used) + 2.75 + used * (0.35 + 8e-6 / 2.5 * outputs);
