@@ -333,11 +333,13 @@ def test_norm_of_few_rows(device, dtype, n, H, center, at):
 
 
 # gated pairs of few tiles: ranges of K and their sums in a launch of its own; a last range that is shorter, rows and columns that do not
-# fill a tile, the most ranges, tall tiles, and pairs that stay whole
+# fill a tile, the most ranges (16), tiles of 64 rows and of 128, and pairs that stay whole.  split: in bf16, in float32
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("M,N,K,split", [(17, 65, 1152, True), (53, 2560, 1024, None), (100, 333, 4800, True), (64, 6912, 2048, True), (129, 1990, 5952, True), (700, 1100, 6016, None),
-                                         (20, 400, 64, False), (300, 7000, 256, False)])
-def test_gated_pair_in_ranges_of_k(device, dtype, M, N, K, split):
+@pytest.mark.parametrize("M,N,K,split,tall", [
+    (17, 65, 1152, (True, True), False), (53, 2560, 1024, (True, True), False), (100, 333, 4800, (True, True), False), (64, 6912, 2048, (True, True), False),
+    (129, 1990, 5952, (True, True), False), (700, 1100, 6016, (False, True), False), (17, 40, 8192, (True, True), False), (66, 16448, 8192, (True, True), True),
+    (150, 8300, 4096, (False, True), True), (20, 400, 64, (False, False), False), (300, 7000, 256, (False, False), True)])
+def test_gated_pair_in_ranges_of_k(device, dtype, M, N, K, split, tall):
     g = torch.Generator(device=device).manual_seed(M + N + K)
     x, gate, up = (torch.randn(n, K, device=device, generator=g).to(dtype) * (1 if n == M else K**-0.5) for n in (M, N, N))
 
@@ -347,7 +349,9 @@ def test_gated_pair_in_ranges_of_k(device, dtype, M, N, K, split):
     out = torch.full((M + 1, N + 5), 7.0, dtype=dtype, device=device)
     D.glu_gemm(x, gate, up, out, M, Spec)
     label = native.last_variant()
-    assert "pair" in label and (split is None or label.endswith("x1") != split), label
+    assert "pair" in label and label.endswith("x1") != split[dtype == torch.float32], label
+    assert "wide" in label or (",2,2,plain" in label) == tall, label
+    assert K != 8192 or N > 40 or label.endswith("x16"), label
     a, c = x.double() @ gate.double().T, x.double() @ up.double().T
     want = a.clamp(max=1.5) * torch.sigmoid(1.702 * a.clamp(max=1.5)) * (c.clamp(-1.5, 1.5) + 1)
     # (the unit's slope stays below 1.1 and it below |a|; the two sums' errors as above, the unit's own work 2^-20, in bf16 2^-18, and a rounding)
