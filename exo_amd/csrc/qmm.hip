@@ -581,9 +581,9 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
     // under 520 rows 115.7 | 121.5 us, 1500 205 | 211, 6144x4096 under 1023 60.9 | 61.5)
     constexpr bool X_FIRST = KH && BITS == 8;
     constexpr int XAHEAD = X_FIRST ? 2 : 3;
-    // Experts: activations behind the last wait for weights, which does not count them; of up to 64 rows, where the step is too short
-    // for what is requested at its end, right behind the first weights (at the end | so, gate/up of 1536x4096, 128 experts, 8 bits: 80
-    // tokens 468 | 455 us, 600 514 | 503; 768x2048 level; 2048x768 47.6 | 48.5 under 400; of more rows 2047 tokens 885 | 897)
+    // Experts (their single products; pairs have a loop of their own): activations behind the last wait for weights, which does not count them; of up
+    // to 64 rows, where the step is too short for what is requested at its end, right behind the first weights (at the end | so, 128 experts of 4096x1536, 8
+    // bits: 150 tokens 209 | 206 us, 300 213 | 210, 400 215 | 213.5; 2048x768 and 4 bits level)
     constexpr bool LATE = NI > 2;
 #pragma unroll
     for (int u = 0; u < AHEAD; ++u) load_w(wq[u], min(kb + u * BK, last));
