@@ -25,16 +25,17 @@
 //            the nucleus edge, the 20th largest value.  (A flat 65536-entry table took 85 us to
 //            fill with 2 atomics per logit and 115 us to scan and clear; the two levels take four
 //            microseconds each.)
-//   finish   per slice the sum of exp((x - max) / T) over the kept tokens (x >= threshold); tokens at or above the
-//            20th largest key are appended to a candidate list.  The row's last slice to arrive (an atomic counter, no
-//            spinning) finishes it: uniform from Philox-4x32-10 (key = request seed,
+//   weights  per slice the sum of exp((x - max) / T) over the kept tokens (x >= threshold);
+//            tokens at or above the 20th largest key are appended to a candidate list;
+//   select   one workgroup per row: uniform from Philox-4x32-10 (key = request seed,
 //            counter = draws so far), the slice in which the running sum crosses u * total,
 //            then the token inside it (inverse CDF in vocabulary order); ranks the
 //            candidates; appends the token to the history ring; advances the cache position.
-//   greedy   in its place where no row is drawn or listed.
-// What bounds a step is latency: four dependent launches of 64 workgroups per row, each the way of its operands from
-// memory and then a chain of reductions.  (The draw in a launch of its own: 5.2 us for the sums and 6.9 for it, where both are 10.6 - what the slices
-// hand over costs three ways through memory, nearly a launch; of four rows of 151936 a token 1.9 us less.)  One row of 128256, top-p, min-p and top-logprobs: 30.8 -> 19.9 us (four rows
+//   greedy   in place of both where no row is drawn or listed: a wave per row (greedy steps 0.95 of the time, 1 to 64 rows).
+// (Weights and select in one launch, whose last slice of a row to arrive finishes it: what the slices hand over costs as much as a launch; one to
+// sixteen rows 0.97 to 1.07 of the time, and the 4096 workgroups of 64 rows wait for their stores where others could run, drawn rows 19.8 -> 26 us.)
+// What bounds a step is latency: up to five dependent launches of 64 workgroups per row, each the way of its operands from
+// memory and then a chain of reductions.  One row of 128256, top-p, min-p and top-logprobs: 30.8 -> 19.9 us (four rows
 // of 151936: 35.3 -> 23.6) with everything requested up front, reductions through lane permutes, one word per table
 // entry and only the values counted that matter; no filter but top-logprobs 44.4 -> 19.5 (an LDS maximum that all kept tokens
 // took one by one), penalties over 64 tokens 76.3 -> 29.4 (edits found by position, not by a walk over the list).
@@ -68,34 +69,24 @@ constexpr int kMassShift = 14;
 __device__ __forceinline__ int mass_shift(float mx) { return fabsf(mx) < 0x1p23f ? 0 : kMassShift; }
 
 struct RowWs {
-  float part[kBlocks][4];  // max, argmax (int bits), sum exp(x - max)
+  float part[kBlocks][4];  // max, argmax (int bits), sum exp(x - max), kept weight
   int n_edit;
+  float thr;    // value threshold from top-p / top-k (-inf: none)
+  int key_top;  // key of the 20th largest value
+  int cand_n;
   // per target: the bucket in which the running count / mass from the top crosses it (-1:
   // never), and the count and mass of the buckets above it
   int bkt[4];
   u64 above[4];
   int edit_idx[kMaxEdits];
   float edit_val[kMaxEdits];
-  // What the slices of the last launch hand to the one that finishes the row, in lines of their own: written and read at device scope
-  // (the counters: zero before it).
-  __attribute__((aligned(128))) int arrived;  // slices that have
-  int cand_n;
-  u64 cand[kMaxCand];    // key << 32 | index, values strictly above the 20th largest
-  float kept[kBlocks];   // weight
+  u64 cand[kMaxCand];  // key << 32 | index, values strictly above the 20th largest
   // tokens whose value EQUALS the 20th largest, per slice: the first kTop of them in
   // vocabulary order (a flat row has thousands; which of them make the list must not depend
   // on the order in which workgroups arrive)
   int tie_n[kBlocks];
   int tie_idx[kBlocks][kTop];
 };
-template <typename T>
-__device__ __forceinline__ void hand_over(T* p, T v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <typename T>
-__device__ __forceinline__ T handed(const T* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 constexpr size_t kRowWsBytes = (sizeof(RowWs) + 255) / 256 * 256;
 
 // count and mass per bucket, and per low key of each target's bucket; zero between steps
@@ -324,7 +315,11 @@ __global__ __launch_bounds__(256) void sample_stats_kernel(const bf16_t* __restr
   Share<NU> sh;
   request_share(logits + (size_t)row * V, g, sh);
   const int n_edit = has_edits ? w->n_edit : 0;
-  if (blockIdx.x == 0 && threadIdx.x == 0) w->arrived = w->cand_n = 0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {  // per-step fields of the row
+    w->thr = -INFINITY;
+    w->key_top = 0;
+    w->cand_n = 0;
+  }
   stage_edits(w, g, n_edit, ed);
   float xv[8 * NU];
   expand_share(sh, g, n_edit, ed, xv);
@@ -648,7 +643,131 @@ __device__ __forceinline__ void fine_keys(const FineRequest& r, const Wanted& q,
   if ((threadIdx.x & 63) == 0) keys[j] = r.bkt >= 0 && at >= 0 ? (r.bkt << 7) | at : -1;
 }
 
-// ---- finish -------------------------------------------------------------------
+// ---- weights ------------------------------------------------------------------
+template <int NU>
+__global__ __launch_bounds__(256) void sample_weights_kernel(
+    const bf16_t* __restrict__ logits, const exo_sampler_params* __restrict__ params, void* ws,
+    int V, int has_edits, int has_tables, int want_top) {
+  __shared__ EditLds ed;
+  __shared__ float ssum[4];
+  __shared__ int s_keys[kTargets], s_ties[4];
+  const int row = blockIdx.y;
+  RowWs* w = row_ws(ws, row);
+  Tables* T = row_tables(ws, row);
+  const SliceGeom g = slice_geom(logits, V, blockIdx.x);
+  FineRequest fine = {};
+  if (has_tables) fine = request_fine(w, T);
+  Share<NU> sh;
+  request_share(logits + (size_t)row * V, g, sh);
+  const Partial part = request_partial(w);
+  const int n_edit = has_edits ? w->n_edit : 0;
+  const exo_sampler_params p = params[row];
+  const bool sampling = p.temperature != 0.f;
+  if (!sampling && !want_top) return;
+  // the exact keys of this step from the fine tables; the first workgroup leaves them for the select
+  // launch and clears the bucket table, whose last reader was the previous launch
+  float table_thr = -INFINITY;
+  int kt = 0;
+  const bool table = has_tables && row_needs_table(p, want_top != 0);  // (uniform over the workgroup)
+  float mx, lse;
+  int mi;
+  merge_stats(part, mx, mi, lse);
+  if (table) {
+    fine_keys(fine, wanted_of(p, want_top != 0, mx), s_keys);
+    if (blockIdx.x == 0)
+      for (int b = threadIdx.x; b < kBuckets; b += 256) T->coarse[b] = 0;
+  }
+  stage_edits(w, g, n_edit, ed);
+  float xv[8 * NU];
+  expand_share(sh, g, n_edit, ed, xv);
+  if (table) {
+    __syncthreads();
+    if (s_keys[0] >= 0) table_thr = value_of(s_keys[0]);
+    if (s_keys[1] >= 0) table_thr = fmaxf(table_thr, value_of(s_keys[1]));
+    if (s_keys[2] >= 0) kt = s_keys[2];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      w->thr = table_thr;
+      w->key_top = kt;
+    }
+  }
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int mine[NU];  // of this thread's chunks, the values equal to the 20th largest
+  if (want_top) {
+    // strictly above the 20th largest value: at most 19 tokens in the whole row, any order
+    // (the select launch ranks them)
+    int all = 0;
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      mine[u] = 0;
+      if (u < sh.chunks) {
+        uint32_t larger = 0;  // (a bit per value: without branches, since hardly any thread has one)
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          const int key = sh.i0[u] + k < g.hi ? key_of(xv[8 * u + k]) : -1;
+          larger |= key > kt ? 1u << k : 0u;
+          mine[u] += key == kt ? 1 : 0;
+        }
+        if (larger) {
+#pragma unroll
+          for (int k = 0; k < 8; ++k)
+            if (larger & (1u << k)) {
+              const int slot = atomicAdd(&w->cand_n, 1);
+              if (slot < kMaxCand) w->cand[slot] = ((u64)key_of(xv[8 * u + k]) << 32) | (unsigned int)(sh.i0[u] + k);
+            }
+        }
+      }
+      all += mine[u];
+    }
+    const u64 any = __ballot(all > 0);
+    if (lane == 0) s_ties[wave] = any != 0;
+  }
+  if (sampling) {
+    const float thr = keep_threshold(p, table_thr, mx);
+    const float inv_t = 1.f / p.temperature;
+    float s = 0.f;
+#pragma unroll
+    for (int u = 0; u < NU; ++u)
+      if (u < sh.chunks) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+          if (xv[8 * u + k] >= thr) s += expf((xv[8 * u + k] - mx) * inv_t);
+      }
+    s = wave_sum(s);
+    if (lane == 0) ssum[wave] = s;
+  }
+  __syncthreads();
+  if (sampling && threadIdx.x == 0) w->part[blockIdx.x][3] = ssum[0] + ssum[1] + ssum[2] + ssum[3];
+  if (!want_top) return;
+  if (!(s_ties[0] | s_ties[1] | s_ties[2] | s_ties[3])) {  // (most slices; uniform over the workgroup)
+    if (threadIdx.x == 0) w->tie_n[blockIdx.x] = 0;
+    return;
+  }
+  // equal to the 20th largest: this slice's first kTop in vocabulary order, by a scan over the
+  // threads (chunk 0 of every thread precedes chunk 1 of any)
+  int base = 0;
+#pragma unroll
+  for (int u = 0; u < NU; ++u) {
+    const int inc = wave_scan_i32(mine[u]);
+    __syncthreads();  // (the words are read above and in the round before)
+    if (lane == 63) s_ties[wave] = inc;
+    __syncthreads();
+    int before = base;
+    for (int q = 0; q < wave; ++q) before += s_ties[q];
+    int at = before + inc - mine[u];  // ties of this slice in front of this thread's chunk
+    if (mine[u] > 0 && at < kTop) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        if (sh.i0[u] + k < g.hi && key_of(xv[8 * u + k]) == kt) {
+          if (at < kTop) w->tie_idx[blockIdx.x][at] = sh.i0[u] + k;
+          ++at;
+        }
+    }
+    base += s_ties[0] + s_ties[1] + s_ties[2] + s_ties[3];
+  }
+  if (threadIdx.x == 0) w->tie_n[blockIdx.x] = min(base, kTop);
+}
+
+// ---- select -------------------------------------------------------------------
 __device__ __forceinline__ void philox4x32_10(uint32_t (&c)[4], uint32_t k0, uint32_t k1) {
 #pragma unroll
   for (int r = 0; r < 10; ++r) {
@@ -708,156 +827,62 @@ __global__ __launch_bounds__(64) void sample_greedy_kernel(const StepOut o, cons
 }
 
 template <int NU>
-__global__ __launch_bounds__(256) void sample_finish_kernel(
-    const bf16_t* __restrict__ logits, const exo_sampler_params* __restrict__ params, const StepOut o, void* ws,
-    int V, int has_edits, int has_tables, int want_top) {
+__global__ __launch_bounds__(256) void sample_select_kernel(
+    const bf16_t* __restrict__ logits, const exo_sampler_params* __restrict__ params, const StepOut out, void* ws, int V,
+    int has_edits, int has_tables, int want_top) {
   __shared__ EditLds ed;
-  __shared__ float ssum[4], s_wsum[4], s_x;
-  __shared__ int s_keys[kTargets], s_ties[4], s_last, s_tok, s_kept[4];
-  const int row = blockIdx.y, tid = threadIdx.x;
+  __shared__ float s_wsum[4], s_rem;
+  __shared__ int s_block, s_tok, s_last[4];
+  __shared__ float s_x;
+  const int row = blockIdx.x, tid = threadIdx.x;
+  const int lane = tid & 63, wave = tid >> 6;
   RowWs* w = row_ws(ws, row);
-  Tables* T = row_tables(ws, row);
-  const SliceGeom g = slice_geom(logits, V, blockIdx.x);
-  FineRequest fine = {};
-  if (has_tables) fine = request_fine(w, T);
-  Share<NU> sh;
-  request_share(logits + (size_t)row * V, g, sh);
-  const Partial part = request_partial(w);
+  // everything that does not depend on the slice of the draw is requested here
+  const float4 stat = *reinterpret_cast<const float4*>(&w->part[lane][0]);
   const int n_edit = has_edits ? w->n_edit : 0;
+  const float table_thr = w->thr;
+  const int key_top = w->key_top, cand_n = w->cand_n;
+  const u64 my_cand = lane < kMaxCand ? w->cand[lane] : 0ull;
+  const int my_ties = w->tie_n[lane];
+  const Sequence seq = request_sequence(out, row);
   const exo_sampler_params p = params[row];
-  const Sequence seq = request_sequence(o, row);
-  const bool sampling = p.temperature != 0.f;
-  const bool one = !sampling && !want_top;  // its largest value is all that the row is asked for: a matter of one workgroup
-  if (one && blockIdx.x) return;
-  // the exact keys of this step from the fine tables; the first workgroup clears the bucket table, whose last reader was the
-  // previous launch
-  float table_thr = -INFINITY;
-  int kt = 0;
-  const bool table = has_tables && row_needs_table(p, want_top != 0);  // (uniform over the workgroup)
+  if (has_tables && row_needs_table(p, want_top != 0)) {  // the weights launch was the fine tables' last reader
+    Tables* T = row_tables(ws, row);
+    for (int i = tid; i < kTargets * kFine; i += 256) (&T->fine[0][0])[i] = 0;
+  }
   float mx, lse;
   int mi;
-  merge_stats(part, mx, mi, lse);
-  if (table) {
-    fine_keys(fine, wanted_of(p, want_top != 0, mx), s_keys);
-    if (blockIdx.x == 0)
-      for (int b = threadIdx.x; b < kBuckets; b += 256) T->coarse[b] = 0;
-  }
-  stage_edits(w, g, n_edit, ed);
-  float xv[8 * NU];
-  expand_share(sh, g, n_edit, ed, xv);
-  if (table) {
-    __syncthreads();
-    if (s_keys[0] >= 0) table_thr = value_of(s_keys[0]);
-    if (s_keys[1] >= 0) table_thr = fmaxf(table_thr, value_of(s_keys[1]));
-    if (s_keys[2] >= 0) kt = s_keys[2];
-  }
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  int mine[NU];  // of this thread's chunks, the values equal to the 20th largest
-  if (want_top) {
-    // strictly above the 20th largest value: at most 19 tokens in the whole row, any order
-    // (the workgroup that finishes ranks them)
-    int all = 0;
+  merge_stats({stat.x, stat.z, __float_as_int(stat.y)}, mx, mi, lse);
+  const bool draw = p.temperature != 0.f;
+  SliceGeom g = {};
+  Share<NU> sh;
+  if (draw) {
+    if (wave == 0) {
+      // the slice in which the running sum of kept weights crosses u * total (slices in order, sums in float32,
+      // the same order every time): a lane holds its slice's sum and what runs up to it
+      const float wb = stat.w;
+      float total = 0.f, run = 0.f;
 #pragma unroll
-    for (int u = 0; u < NU; ++u) {
-      mine[u] = 0;
-      if (u < sh.chunks) {
-        uint32_t larger = 0;  // (a bit per value: without branches, since hardly any thread has one)
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          const int key = sh.i0[u] + k < g.hi ? key_of(xv[8 * u + k]) : -1;
-          larger |= key > kt ? 1u << k : 0u;
-          mine[u] += key == kt ? 1 : 0;
-        }
-        if (larger) {
-#pragma unroll
-          for (int k = 0; k < 8; ++k)
-            if (larger & (1u << k)) {
-              const int slot = atomicAdd(&w->cand_n, 1);
-              if (slot < kMaxCand) hand_over(&w->cand[slot], ((u64)key_of(xv[8 * u + k]) << 32) | (unsigned int)(sh.i0[u] + k));
-            }
-        }
+      for (int b = 0; b < kBlocks; ++b) {
+        if (lane == b) run = total;
+        total += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wb), b));
       }
-      all += mine[u];
-    }
-    const u64 any = __ballot(all > 0);
-    if (lane == 0) s_ties[wave] = any != 0;
-  }
-  const float thr = keep_threshold(p, table_thr, mx), inv_t = 1.f / p.temperature;
-  if (sampling) {
-    float s = 0.f;
-#pragma unroll
-    for (int u = 0; u < NU; ++u)
-      if (u < sh.chunks) {
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-          if (xv[8 * u + k] >= thr) s += expf((xv[8 * u + k] - mx) * inv_t);
+      uint32_t c[4] = {seq.drawn, 0u, 0u, 0u};
+      philox4x32_10(c, p.seed_lo, p.seed_hi);
+      const float u = (float)(c[0] >> 8) * 0x1p-24f;
+      const float target = u * total;
+      const u64 kept = __ballot(wb > 0.f), hit = __ballot(wb > 0.f && run + wb > target);
+      // (no slice: rounding at the very end of the distribution)
+      const int blk = hit ? __ffsll((long long)hit) - 1 : kept ? 63 - __clzll((long long)kept) : 0;
+      if (lane == blk) {
+        s_block = blk;
+        s_rem = hit ? target - run : INFINITY;
+        s_tok = -1;
       }
-    s = wave_sum(s);
-    if (lane == 0) ssum[wave] = s;
-  }
-  __syncthreads();
-  if (sampling && tid == 0) hand_over(&w->kept[blockIdx.x], ssum[0] + ssum[1] + ssum[2] + ssum[3]);
-  int base = 0;  // this slice's ties
-  if (want_top && (s_ties[0] | s_ties[1] | s_ties[2] | s_ties[3])) {  // (in few slices; uniform over the workgroup)
-    // equal to the 20th largest: this slice's first kTop in vocabulary order, by a scan over the
-    // threads (chunk 0 of every thread precedes chunk 1 of any)
-#pragma unroll
-    for (int u = 0; u < NU; ++u) {
-      const int inc = wave_scan_i32(mine[u]);
-      __syncthreads();  // (the words are read above and in the round before)
-      if (lane == 63) s_ties[wave] = inc;
-      __syncthreads();
-      int before = base;
-      for (int q = 0; q < wave; ++q) before += s_ties[q];
-      int at = before + inc - mine[u];  // ties of this slice in front of this thread's chunk
-      if (mine[u] > 0 && at < kTop) {
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-          if (sh.i0[u] + k < g.hi && key_of(xv[8 * u + k]) == kt) {
-            if (at < kTop) hand_over(&w->tie_idx[blockIdx.x][at], sh.i0[u] + k);
-            ++at;
-          }
-      }
-      base += s_ties[0] + s_ties[1] + s_ties[2] + s_ties[3];
     }
-  }
-  if (want_top && tid == 0) hand_over(&w->tie_n[blockIdx.x], min(base, kTop));
-  uint32_t c[4] = {seq.drawn, 0u, 0u, 0u};
-  if (!one) {  // the last of the row's workgroups finishes it
-    wait_own_stores_done();
     __syncthreads();
-    int before = 0;
-    if (tid == 0) before = __hip_atomic_fetch_add(&w->arrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    philox4x32_10(c, p.seed_lo, p.seed_hi);  // (meanwhile)
-    if (tid == 0) s_last = before == kBlocks - 1;
-    __syncthreads();
-    if (!s_last) return;
-  }
-
-  const float wb = handed(&w->kept[lane]);
-  const int cand_n = handed(&w->cand_n), my_ties = handed(&w->tie_n[lane]), first_tie = handed(&w->tie_idx[lane][0]);
-  const u64 my_cand = lane < kMaxCand ? handed(&w->cand[lane]) : 0ull;
-  if (table)  // all have read the fine tables
-    for (int i = tid; i < kTargets * kFine; i += 256) (&T->fine[0][0])[i] = 0;
-  SliceGeom at = {};
-  float rem = 0.f;
-  if (sampling) {
-    // the slice in which the running sum of kept weights crosses u * total (slices in order, sums in float32,
-    // the same order every time): a lane holds its slice's sum and what runs up to it.  Every wave finds it for itself.
-    float total = 0.f, run = 0.f;
-#pragma unroll 16
-    for (int b = 0; b < kBlocks; ++b) {
-      if (lane == b) run = total;
-      total += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wb), b));
-    }
-    const float u = (float)(c[0] >> 8) * 0x1p-24f, target = u * total, left = target - run;
-    const u64 kept = __ballot(wb > 0.f), hit = __ballot(wb > 0.f && run + wb > target);
-    // (no slice: rounding at the very end of the distribution)
-    const int blk = hit ? __ffsll((long long)hit) - 1 : kept ? 63 - __clzll((long long)kept) : 0;
-    at = slice_geom(logits, V, blk);
-    request_share(logits + (size_t)row * V, at, sh);
-    rem = hit ? __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, left), blk)) : INFINITY;
-    if (tid == 0) s_tok = -1;  // (set behind the barrier below)
+    g = slice_geom(logits, V, s_block);
+    request_share(logits + (size_t)row * V, g, sh);
   }
   if (want_top) {
     // (while the slice is on its way) the tokens strictly above the 20th largest value, ranked: higher key first,
@@ -868,37 +893,41 @@ __global__ __launch_bounds__(256) void sample_finish_kernel(
       const unsigned int mk = (unsigned int)(me >> 32), mi2 = (unsigned int)me;
       int rank = 0;
 #pragma unroll
-      for (int t = 0; t < kTop - 1; ++t) {
-        const unsigned int ok = (unsigned int)__builtin_amdgcn_readlane((int)mk, t);
-        const unsigned int oi = (unsigned int)__builtin_amdgcn_readlane((int)mi2, t);
-        rank += t < n && (ok > mk || (ok == mk && oi < mi2)) ? 1 : 0;
+      for (int o = 0; o < kTop - 1; ++o) {
+        const unsigned int ok = (unsigned int)__builtin_amdgcn_readlane((int)mk, o);
+        const unsigned int oi = (unsigned int)__builtin_amdgcn_readlane((int)mi2, o);
+        rank += o < n && (ok > mk || (ok == mk && oi < mi2)) ? 1 : 0;
       }
       if (lane < n) {
-        o.top_idx[(size_t)row * kTop + rank] = (int)mi2;
-        o.top_val[(size_t)row * kTop + rank] = value_of((int)mk) - lse;
+        out.top_idx[(size_t)row * kTop + rank] = (int)mi2;
+        out.top_val[(size_t)row * kTop + rank] = value_of((int)mk) - lse;
       }
     }
     if (wave == 3) {  // a lane per slice: its ties go behind those of the slices before it
       const int inc = wave_scan_i32(my_ties);
-      const float tv = value_of(kt) - lse;
+      const float tv = value_of(key_top) - lse;
       const int first = n + inc - my_ties;
       for (int j = 0; j < my_ties && first + j < kTop; ++j) {
-        o.top_idx[(size_t)row * kTop + first + j] = j ? handed(&w->tie_idx[lane][j]) : first_tie;
-        o.top_val[(size_t)row * kTop + first + j] = tv;
+        out.top_idx[(size_t)row * kTop + first + j] = w->tie_idx[lane][j];
+        out.top_val[(size_t)row * kTop + first + j] = tv;
       }
       // vocabularies of fewer than 20 tokens
       const int all = n + __builtin_amdgcn_readlane(inc, 63);
       if (lane >= all && lane < kTop) {
-        o.top_idx[(size_t)row * kTop + lane] = -1;
-        o.top_val[(size_t)row * kTop + lane] = -INFINITY;
+        out.top_idx[(size_t)row * kTop + lane] = -1;
+        out.top_val[(size_t)row * kTop + lane] = -INFINITY;
       }
     }
   }
   int tok = mi;
   float x_tok = mx;
-  if (sampling) {
-    stage_edits(w, at, n_edit, ed);
-    expand_share(sh, at, n_edit, ed, xv);
+  if (draw) {
+    stage_edits(w, g, n_edit, ed);
+    float xv[8 * NU];
+    expand_share(sh, g, n_edit, ed, xv);
+    const float thr = keep_threshold(p, table_thr, mx);
+    const float inv_t = 1.f / p.temperature;
+    float rem = s_rem;
     int last_kept = -1;  // of this thread's tokens
 #pragma unroll
     for (int u = 0; u < NU; ++u) {
@@ -914,9 +943,9 @@ __global__ __launch_bounds__(256) void sample_finish_kernel(
       // consecutive threads tile the line exactly (excl is the neighbour's incl, bit for bit)
       float inc = local;
 #pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        const float up = __shfl_up(inc, d, 64);
-        if (lane >= d) inc += up;
+      for (int o = 1; o < 64; o <<= 1) {
+        const float up = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += up;
       }
       const float prev = __shfl_up(inc, 1, 64);
       if (lane == 63) s_wsum[wave] = inc;
@@ -953,9 +982,9 @@ __global__ __launch_bounds__(256) void sample_finish_kernel(
     }
     if (s_tok < 0) {  // float32 rounding put the target past the last kept token (uniform over the workgroup)
       const int last = (int)wave_max_u32((uint32_t)(last_kept + 1)) - 1;
-      if (lane == 0) s_kept[wave] = last;
+      if (lane == 0) s_last[wave] = last;
       __syncthreads();
-      const int lk = max(max(s_kept[0], s_kept[1]), max(s_kept[2], s_kept[3]));
+      const int lk = max(max(s_last[0], s_last[1]), max(s_last[2], s_last[3]));
 #pragma unroll
       for (int u = 0; u < NU; ++u)
 #pragma unroll
@@ -966,13 +995,14 @@ __global__ __launch_bounds__(256) void sample_finish_kernel(
           }
       __syncthreads();
     }
-    const float x_drawn = s_x;
-    if (s_tok >= 0 && s_tok < V) {  // (else no token was kept: min_p above 1, logits that are not numbers)
-      tok = s_tok;
-      x_tok = x_drawn;
+    tok = s_tok;
+    x_tok = s_x;
+    if (tok < 0 || tok >= V) {  // no token was kept (min_p above 1, logits that are not numbers)
+      tok = mi;
+      x_tok = mx;
     }
   }
-  if (tid == 0) write_step(o, seq, row, min(max(tok, 0), V - 1), x_tok, lse, sampling);
+  if (tid == 0) write_step(out, seq, row, min(max(tok, 0), V - 1), x_tok, lse, draw);
 }
 
 // The launches of a step, for slices of one or two chunks a thread.
@@ -987,9 +1017,13 @@ void launch_sample(const bf16_t* lg, const exo_sampler_params* params, const Ste
     sample_coarse_kernel<NU><<<slices, 256, 0, st>>>(lg, params, ws, V, edits, top);
     sample_fine_kernel<NU><<<slices, 256, 0, st>>>(lg, params, ws, V, edits, top);
   }
-  // (the last launch also resolves and clears the tables)
-  if (tables || (mode & EXO_SAMPLE_DRAW)) sample_finish_kernel<NU><<<slices, 256, 0, st>>>(lg, params, out, ws, V, edits, tables, top);
-  else sample_greedy_kernel<<<dim3(rows), 64, 0, st>>>(out, ws, V);
+  // (the weights launch also resolves and clears the tables: it runs whenever they were filled)
+  if (tables || (mode & EXO_SAMPLE_DRAW)) {
+    sample_weights_kernel<NU><<<slices, 256, 0, st>>>(lg, params, ws, V, edits, tables, top);
+    sample_select_kernel<NU><<<dim3(rows), 256, 0, st>>>(lg, params, out, ws, V, edits, tables, top);
+  } else {
+    sample_greedy_kernel<<<dim3(rows), 64, 0, st>>>(out, ws, V);
+  }
 }
 
 }  // namespace
