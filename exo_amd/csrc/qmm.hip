@@ -44,6 +44,7 @@
 #include "qmm_short.h"
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 namespace {
@@ -75,6 +76,7 @@ struct QmmParams {
   int ksplit, kc;
   float* part;  // [ksplit][M][N]
   bool wide = false;  // host only: launch the (32*MI) x 256 tile (up to 128 rows)
+  bool by_expert = false;  // grouped wide tile: expert_tile_of_block
   // pair mode (Llama MLP, prefill): w/s/b is the gate matrix, w2/s2/b2 the up matrix, both
   // [N, K]; y[M,N] = silu(x gate^T) * (x up^T) with both projections rounded to bf16 first
   const uint32_t* w2 = nullptr;
@@ -202,7 +204,7 @@ __device__ __forceinline__ void big_tile_of_block(const QmmParams& p, int bn, in
 }
 
 template <int BITS, int MI, bool GROUPED = false, bool SB4 = false, bool PAIR = false,
-          bool WIDE = false, bool DEEP = false, bool KH = false>
+          bool WIDE = false, bool DEEP = false, bool KH = false, bool LINES = false>
 __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_kernel(const QmmParams p) {
   static_assert(!WIDE || GROUPED || !PAIR || MI >= 4, "the wide pair tile has 128 or 256 rows");
   static_assert(!DEEP || (SB4 && ((MI == 2 && !WIDE) || (WIDE && MI < 4))),
@@ -211,6 +213,7 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
   static_assert(!KH || (MI == 4 && SB4 && !GROUPED && !DEEP && !(WIDE && PAIR)),
                 "two K halves per workgroup: the 256-row tile of the plain and the pair GEMM, "
                 "the wide tile of the plain GEMM");
+  static_assert(!LINES || (GROUPED && WIDE && MI == 4), "codes by lines: the wide tile of the experts");
   constexpr int kThreads = 256;  // of a team
   constexpr int BM = WIDE ? 32 * MI : 64 * MI;
   constexpr int WN = PAIR ? 32 : 64;              // output columns per wave
@@ -234,9 +237,9 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
   int tile_x = blockIdx.x, tile_y = blockIdx.y, half = -1;
   if (MI == 8 && WIDE)
     big_tile_of_block(p, BN, tile_x, tile_y, half);
-  else if (GROUPED)
-    expert_tile_of_block(tile_x, tile_y);
-  else
+  else if (GROUPED && WIDE) {
+    if (p.by_expert) expert_tile_of_block(tile_x, tile_y);
+  } else if (!GROUPED)
     tile_of_block<BM >= 256 ? 4 : 8>(tile_x, tile_y);
   const int n0 = tile_x * BN;
   const int wm = WIDE ? 0 : (wave >> 1) * (32 * MI), wn = WIDE ? wave * WN : (wave & 1) * WN;
@@ -581,9 +584,9 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
     // under 520 rows 115.7 | 121.5 us, 1500 205 | 211, 6144x4096 under 1023 60.9 | 61.5)
     constexpr bool X_FIRST = KH && BITS == 8;
     constexpr int XAHEAD = X_FIRST ? 2 : 3;
-    // Experts (their single products; pairs have a loop of their own): activations behind the last wait for weights, which does not count them; of up
-    // to 64 rows, where the step is too short for what is requested at its end, right behind the first weights (at the end | so, 128 experts of 4096x1536, 8
-    // bits: 150 tokens 209 | 206 us, 300 213 | 210, 400 215 | 213.5; 2048x768 and 4 bits level)
+    // Experts: activations behind the last wait for weights, which does not count them; of up to 64 rows, where the step is too short for what is
+    // requested at its end, right behind the first weights (at the end | so, single products of 128 experts of 4096x1536, 8 bits: 150 tokens 209 | 206 us, 300
+    // 213 | 210, 400 215 | 213.5; 2048x768 and 4 bits level)
     constexpr bool LATE = NI > 2;
 #pragma unroll
     for (int u = 0; u < AHEAD; ++u) load_w(wq[u], min(kb + u * BK, last));
@@ -687,7 +690,7 @@ __global__ __launch_bounds__(KH ? 512 : 256, KH || MI == 8 ? 1 : 2) void qmm_ker
       else ring(std::integral_constant<int, 2>{});
     } else if constexpr (GROUPED) {
       auto run = [&](auto ni) {
-        if constexpr (PAIR || (BITS == 4 && decltype(ni)::value == 4))
+        if constexpr (LINES && (PAIR || (BITS == 4 && decltype(ni)::value == 4)))
           ring_lines(ni);
         else
           ring(ni);
@@ -1190,8 +1193,29 @@ void launch_qmm(const QmmParams& p, hipStream_t st) {
   }
 }
 
+// Whether an expert's column tiles go to one XCD (order), and its codes are requested by lines: where the chip is full.  Below a round of workgroups
+// nothing is lost from the L2 between two steps, and requests in bursts only come later; and an expert of several row tiles has its weights
+// read by each XCD in that order, where the launch's own leaves a part of them to each.  By even routing.  Of the time of the launch's own order and a step's requests,
+// 480 shapes (8 to 128 experts of 256x512 to 1536x4096, 17 to 5000 tokens): pairs of 4 bits 0.969 (both everywhere 0.997), of 8 bits 0.989 (1.029), single products
+// 0.982 and 0.992; slower by more than 3 % 13 of 960 launches, by 1.07 at most (both everywhere 247, by up to 1.78: pair of 8 experts of 1536x4096, 8 bits, 1031 tokens 75 | 133 us).
+// us, 4 bits: pairs of 16 experts of 1536x4096 under 250 tokens with order and lines 54 -> 61, 8 of 2048x2048 under 90 rows each 28.9 -> 31.4, 16 of 1536x4096 under 800 rows each by order
+// alone 337 -> 398; 128 of 1536x4096 under 62 rows each with both 505 -> 382, of 768x2048 72.4 -> 66.9.
+struct GroupedPlan {
+  bool by_expert, lines;
+};
 template <int BITS>
-void launch_grouped(const QmmParams& p, int row_tiles, hipStream_t st) {
+GroupedPlan grouped_plan(const QmmParams& p, int experts, bool pair) {
+  const double rows = (double)p.M / experts;  // of an expert
+  const double tiles = experts * (rows > 64 ? rows / 128 + 0.5 : 1 - std::exp(-rows));
+  const double wgs = tiles * exo_ceil_div(p.N, pair ? 128 : 256);
+  GroupedPlan plan;
+  plan.by_expert = wgs >= 448 && rows >= 4 && rows <= (pair ? 200 : 100);
+  plan.lines = pair ? (BITS == 4 && wgs >= 448) || (p.K >= 4096 && wgs >= (BITS == 4 ? 256 : 384)) : BITS == 4 && plan.by_expert;
+  return plan;
+}
+
+template <int BITS>
+void launch_grouped(QmmParams p, int experts, int row_tiles, hipStream_t st) {
   const bool sb4 = p.K % 256 == 0 &&
                    (((uintptr_t)p.s | (uintptr_t)p.b | (uintptr_t)p.s2 | (uintptr_t)p.b2) & 7) == 0;
   const bool pair = p.w2 != nullptr;  // (gate, up) with the SwiGLU in the epilogue
@@ -1200,10 +1224,16 @@ void launch_grouped(const QmmParams& p, int row_tiles, hipStream_t st) {
   // a wave of the 2 x 2 layout dequantises the same 64 weight rows as its neighbour.
   if (sb4 && kGroupedWide) {
     const dim3 grid(exo_ceil_div(p.N, pair ? 128 : 256), row_tiles);
-    if (pair)
-      exo_note_variant("qmm_kernel<%d, 4, true, true, true, true>", BITS), qmm_kernel<BITS, 4, true, true, true, true><<<grid, 256, 0, st>>>(p);
+    const GroupedPlan plan = grouped_plan<BITS>(p, experts, pair);
+    p.by_expert = plan.by_expert;
+    if (pair && plan.lines)
+      exo_note_variant("qmm_kernel<%d, 4, true, true, true, true>", BITS), qmm_kernel<BITS, 4, true, true, true, true, false, false, true><<<grid, 256, 0, st>>>(p);
+    else if (pair)
+      exo_note_variant("qmm_kernel<%d, 4, true, true, true, true> by steps", BITS), qmm_kernel<BITS, 4, true, true, true, true><<<grid, 256, 0, st>>>(p);
+    else if (BITS == 4 && plan.lines)
+      exo_note_variant("qmm_kernel<%d, 4, true, true, false, true>", BITS), qmm_kernel<BITS, 4, true, true, false, true, false, false, BITS == 4><<<grid, 256, 0, st>>>(p);
     else
-      exo_note_variant("qmm_kernel<%d, 4, true, true, false, true>", BITS), qmm_kernel<BITS, 4, true, true, false, true><<<grid, 256, 0, st>>>(p);
+      exo_note_variant("qmm_kernel<%d, 4, true, true, false, true>%s", BITS, BITS == 4 ? " by steps" : ""), qmm_kernel<BITS, 4, true, true, false, true><<<grid, 256, 0, st>>>(p);
     return;
   }
   const dim3 grid(exo_ceil_div(p.N, pair ? 64 : 128), row_tiles);
@@ -1356,9 +1386,9 @@ static int gather_qmm_impl(const uint16_t* x, const uint32_t* w, const uint16_t*
   p.s2 = s2;
   p.b2 = b2;
   if (bits == 4)
-    launch_grouped<4>(p, max_tiles, (hipStream_t)stream);
+    launch_grouped<4>(p, E, max_tiles, (hipStream_t)stream);
   else
-    launch_grouped<8>(p, max_tiles, (hipStream_t)stream);
+    launch_grouped<8>(p, E, max_tiles, (hipStream_t)stream);
   EXO_CHECK_LAUNCH("exo_gather_qmm");
   return EXO_OK;
 }

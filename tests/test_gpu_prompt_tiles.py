@@ -117,11 +117,14 @@ def test_grouped_gemm_multiplies_the_rows_of_its_tile(device, rows, K, bits):
         check(y[sel, 0], x[sel, 0], weights64(qs[e]), what=f"expert {e} of {len(sel)} rows")
 
 
-@pytest.mark.parametrize("K,bits", [(256, 4), (512, 4), (768, 4), (1280, 4), (256, 8), (768, 8)])
-def test_grouped_pair_has_the_bits_of_two_products(device, K, bits):
-    """Gate and up products of experts of 1 to 300 rows in one launch, whose loop requests its codes in another order (one block of four steps of K, an
-    odd and an even number of them), more row tiles than XCDs and no multiple of their number, against the two products."""
-    counts, N = [1, 300, 31, 0, 33, 64, 65, 128, 96, 97, 129], 264
+@pytest.mark.parametrize("N,K,bits,lines", [
+    (264, 256, 4, False), (264, 512, 4, False), (264, 768, 4, False), (264, 1280, 4, False), (264, 256, 8, False), (264, 768, 8, False),
+    (5128, 256, 4, True), (5128, 512, 4, True), (9000, 768, 4, True), (3208, 4096, 4, True), (5128, 768, 8, False), (5128, 4096, 8, True)])
+def test_grouped_pair_has_the_bits_of_two_products(device, N, K, bits, lines):
+    """Gate and up products of experts of 1 to 300 rows in one launch, whose loop requests its codes step by step or, where the chip is full, by lines and in
+    another order of tiles (one block of four steps of K, an odd and an even number of them), more row tiles than XCDs and no multiple of their number,
+    against the two products."""
+    counts = [1, 300, 31, 0, 33, 64, 65, 128, 96, 97, 129]
     E = len(counts)
     gate, up = (QuantizedWeight(*(torch.stack(t) for t in zip(*((q.weight, q.scales, q.biases) for q in (packed(N, K, bits, 100 * s + e, device) for e in range(E))))), bits) for s in (1, 2))
     idx = torch.cat([torch.full((n,), e) for e, n in enumerate(counts)]).to(torch.int32)
@@ -129,7 +132,9 @@ def test_grouped_pair_has_the_bits_of_two_products(device, K, bits):
     x = torch.randn(len(idx), 1, K, device=device, generator=torch.Generator(device=device).manual_seed(K)).bfloat16()
     ws = ops.moe_group(idx, E)
     y = ops.grouped_qmm_swiglu(x, gate, up, ws, 1)
+    assert native.last_variant().endswith("by steps") != lines, native.last_variant()
     a, b = ops.grouped_qmm(x, gate, ws, 1), ops.grouped_qmm(x, up, ws, 1)
+    assert bits == 8 or native.last_variant().endswith("by steps") == (N < 9000), native.last_variant()
     assert torch.equal(y.view(torch.int16), ops.swiglu(a, b).view(torch.int16))
     for e in range(E):
         sel = (idx[:, 0] == e).nonzero()[:, 0]
