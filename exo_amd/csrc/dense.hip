@@ -43,11 +43,14 @@ struct GemvParams {
   const float* bias;
   void* y;
   float* y2;       // columns from n1 on
-  int M, N, n1, ldx, ldw, ldy, ldy2, y_f32;
-  int cols;        // weight rows of a workgroup, at most 16 / Q
+  int M, N, n1, ldx, ldw, ldy, ldy2;
+  int y_f32 : 2, cols : 6, tiles : 24;  // weight rows of a workgroup, at most 16 / Q; workgroups: ceil(N / cols)
   GluConst glu;
   Epilogue ep;
 };
+// Two products and a norm's arguments go to one kernel, each line of 64 bytes another 0.2 to 0.3 us of a small launch's way to its first request: four bytes
+// more were 5 % of two products of 520x960 in float32 under one row (3.44 | 3.65 us), a division by cols in the kernel one more.
+static_assert(sizeof(GemvParams) == 128, "whole lines");
 
 template <typename T>
 __device__ __forceinline__ void store_out(void* y, size_t i, float v, int y_f32) {
@@ -125,7 +128,7 @@ __global__ __launch_bounds__(64 * NW) void dense_gemv_kernel(const GemvParams p0
   extern __shared__ __attribute__((aligned(16))) char xs[];  // POST: [M][ldx * sizeof(T) + 16]
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int r = lane & 15, g = lane >> 4;
-  const int tiles0 = (p0.N + p0.cols - 1) / p0.cols;
+  const int tiles0 = p0.tiles;
   const bool second = DUAL && (int)blockIdx.x >= tiles0;
   const GemvParams& p = second ? p1 : p0;
   const int n0 = ((int)blockIdx.x - (second ? tiles0 : 0)) * p.cols, rows = min(p.cols, p.N - n0);
@@ -1197,7 +1200,7 @@ int launch_gemv(GemvParams p, const GemvParams* second, const PostNorm* q, hipSt
   if (second) other = *second, p1 = &other;
   const int parts = q ? post_parts(p, *q, (int)sizeof(T)) : gemv_parts(p, p1, (int)sizeof(T));
   const GemvShape shape = gemv_shape(p, p1, q, (int)sizeof(T), parts);
-  p.cols = other.cols = shape.cols;
+  p.cols = other.cols = shape.cols, p.tiles = exo_ceil_div(p.N, p.cols);
   if (q && parts == 2) {
     exo_note_variant("dense_gemv<%s,8,post,%s> M=%d N=%d parts=2 cols=%d", sizeof(T) == 2 ? "bf16" : "f32", p.w2 ? "pair" : "single", p.M, p.N, p.cols);
     if (p.ldx <= post_waves_per_row(p.M, 8) * 256)
@@ -1260,7 +1263,7 @@ static int linear_check(const exo_linear* a, const char* what) {
 static GemvParams gemv_of(const exo_linear* a) {
   GemvParams p{};
   p.x = a->x, p.w = a->w, p.w2 = a->w_up, p.bias = a->bias, p.y = a->y, p.y2 = a->y2;
-  p.M = a->M, p.N = a->N, p.n1 = a->n1, p.ldx = a->ldx, p.ldw = a->ldw, p.ldy = a->ldy, p.ldy2 = a->ldy2, p.y_f32 = a->y_f32;
+  p.M = a->M, p.N = a->N, p.n1 = a->n1, p.ldx = a->ldx, p.ldw = a->ldw, p.ldy = a->ldy, p.ldy2 = a->ldy2, p.y_f32 = a->y_f32 != 0;
   p.glu = GluConst{a->limit, a->alpha, a->shift, a->cubic};
   p.ep = Epilogue{a->act, a->mul, a->mul_rows, a->ldmul, a->cap};
   return p;
