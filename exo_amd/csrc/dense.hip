@@ -1144,7 +1144,7 @@ void launch_gemv_parts(const GemvParams& p, const GemvParams* p1, hipStream_t st
 // adds its waves' sums, more of them keep more requests in flight.  gemv_us is a fit to 4873 shapes (64 to 14336 columns of K, 300 to
 // 40000 columns, 1 to 16 rows, with and without norms, bf16 and f32, 12 settings each).  What is fastest by it takes, on average, 0.946 of the time of
 // whole 16 / parts rows and waves by the number of columns (gemv_waves), pairs 0.948, behind norms 0.946 and 0.935 (the best setting of each shape 0.93 to
-// 0.94); slower by more than 3 % are 0.2 to 0.9 %: the 4 % that it has to promise leave most of them out.  us: f32 under 2 rows behind norms, 6432
+// 0.94); slower by more than 2 % are 0.2 to 0.9 %: the 4 % that it has to promise leave most of them out.  us: f32 under 2 rows behind norms, 6432
 // columns of 1024 11.0 -> 9.6, pair of 2560 10.5 -> 9.1; bf16 under 4 rows pair of 6912x2048 13.5 -> 12.6, under 8 15.6 -> 13.9, one row
 // behind a norm 6160x2048 9.8 -> 8.3.
 struct GemvShape {
@@ -1152,7 +1152,7 @@ struct GemvShape {
 };
 double gemv_us(const GemvParams& p, const GemvParams* p1, const PostNorm* q, int elem, int parts, GemvShape c) {
   const int mats = p.w2 ? 2 : 1, row = std::max(p.ldw, p1 ? p1->ldw : 0) * elem;
-  const int wgs = exo_ceil_div(p.N, c.cols) + (p1 ? exo_ceil_div(p1->N, c.cols) : 0), held = exo_ceil_div(wgs, 256);  // by the fullest CU
+  const int wgs = exo_ceil_div(p.N, c.cols) + (p1 ? exo_ceil_div(p1->N, c.cols) : 0), held = std::max(1, exo_ceil_div(wgs - 2, 256));  // by the fullest CU (one or two more make no round)
   const double total = ((double)p.N * p.ldw + (p1 ? (double)p1->N * p1->ldw : 0.0)) * elem * mats;
   const double cu = (double)c.cols * row * mats / 25e3;  // a workgroup's bytes at 25 GB/s
   const double fullest = std::max(held * cu, total / 6.4e6), average = wgs * cu / 256;
@@ -1181,7 +1181,8 @@ GemvShape gemv_shape(const GemvParams& p, const GemvParams* p1, const PostNorm* 
     // ahead; one pass for those gives 1.10 of the time over the 212 shapes of the sweep that it would change, 0.86 to 1.33.)
     if (q && passes(waves) > std::max(2, passes(usual.waves))) continue;
     auto weigh = [&](int cols) {
-      const double us = gemv_us(p, p1, q, elem, parts, {waves, cols});
+      // (more waves than usual: 8 %, which leaves out f32 57806x1856 under two rows 87 | 98 us, two products of 10756x2048 20.5 | 22.1)
+      const double us = gemv_us(p, p1, q, elem, parts, {waves, cols}) * (waves > usual.waves ? 0.96 / 0.92 : 1.0);
       if (us < least) least = us, best = GemvShape{waves, cols};
     };
     weigh(most);
