@@ -105,6 +105,7 @@ def test_steps_of_a_wave(device, dtype, M, N, steps):
     ("f32", 2, 3001, 1000, True, False, 2), ("f32", 2, 3001, 1000, False, True, 1), ("f32", 4, 3001, 1000, False, False, 1), ("bf16", 5, 2501, 320, False, False, 1),
     ("bf16", 2, 5001, 2048, False, False, 2), ("bf16", 1, 5001, 2048, True, False, 1), ("bf16", 1, 5700, 2048, False, False, 1), ("f32", 2, 9001, 1021, False, True, 2),
     ("bf16", 1, 2384, 2048, False, False, 2), ("f32", 2, 2273, 1000, False, False, 2),  # steps that fill half a batch: fewer columns than the product holds
+    ("f32", 2, 4000, 4096, False, True, 1), ("f32", 2, 5000, 4096, False, True, 1), ("f32", 2, 6900, 4096, False, True, 1),  # 16 waves' sums and the rows: more than 64 KB of LDS
     # one batch of a wave, one and a part, two whole ones (requests in a ring) and more
     ("f32", 1, 9001, 1024, True, False, 1), ("f32", 1, 9001, 1500, False, False, 1), ("f32", 1, 9001, 2048, True, False, 1), ("bf16", 1, 16385, 2048, False, False, 1), ("f32", 1, 20001, 1030, True, False, 1),
 ])
