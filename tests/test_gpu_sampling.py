@@ -208,8 +208,8 @@ def test_sample_modes_and_reuse(device):
 
 
 @pytest.mark.parametrize("V", [19, 4099, 131072, 131080])
-def test_rows_finish_by_their_last_slice_or_by_one(device, V):
-    """Drawn rows (finished by the slice that arrives last) between greedy ones (by one workgroup), without the top list, and greedy
+def test_drawn_and_greedy_rows_finish(device, V):
+    """Drawn rows (finished behind the weights of their slices) between greedy ones (by one workgroup), without the top list, and greedy
     rows by themselves: each against the oracle, several steps over one workspace."""
     settings = [SamplerSettings(temperature=0.0), SamplerSettings(temperature=0.8, top_p=0.9, min_p=0.0, seed=5),
                 SamplerSettings(temperature=0.0), SamplerSettings(temperature=1.1, min_p=0.0, seed=6),
